@@ -1,115 +1,260 @@
-// Plain tiled matrix product for gfx950: C[M,N] = A[M,K] * W[N,K]^T with 32-bit
+// Plain matrix product for gfx950: C[M,N] = A[M,K] * W[N,K]^T with 32-bit products and 32-bit
 // accumulation, for any M, N, K and any mix of float / bf16 operands.
 //
-// (a kernel of its own takes up to 16 rows of A: decode steps).
-//
-// This is the true 32-bit path of the linear layers (ordinary fused multiply-adds, no
-// reduced-precision matrix mode) and the fallback for sizes the MFMA kernels refuse.
+// This is the true 32-bit path of the linear layers and the fallback for sizes the bfloat16 kernels
+// refuse.  It runs on the matrix cores' 32-bit instructions (v_mfma_f32_*: operands and sums are whole
+// floats, nothing is narrowed), which do twice the multiply-adds a clock of the vector units.
 // Weights are row-major [out, in] and used as y = W x, as in the reference
 // (src/backend/backend.zig:474, 481).
+//
+// Two kernels: with few rows (decode steps, short prompts) the weights' way from memory bounds the
+// product, with more the multiply-adds do.
 #include "common_impl.h"
 
-#define TM 64
-#define TN 64
-#define TK 16
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-template <typename TA, typename TW, typename TC>
-__global__ __launch_bounds__(256) void gemm_tn_kernel(const TA* __restrict__ A, long lda,
-                                                      const TW* __restrict__ W, long ldw,
-                                                      TC* __restrict__ C, long ldc, int M, int N, int K) {
-    __shared__ float As[TK][TM + 4];
-    __shared__ float Ws[TK][TN + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
-    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    // loader: thread -> (row, 4 consecutive k)
-    const int lr = tid >> 2, lk = (tid & 3) * 4;
-    float acc[4][4];
+// Four neighbouring elements of a row, k .. k+3, as floats; what lies at or behind K is 0.  VEC: K is a
+// multiple of 4 and every row is aligned to four elements, so the four are there or not together.
+template <bool VEC, typename T> __device__ __forceinline__ f32x4_t ld4(const T* row, int k, int K);
+template <> __device__ __forceinline__ f32x4_t ld4<true, float>(const float* row, int k, int K) {
+    return k < K ? *(const f32x4_t*)(row + k) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+}
+template <> __device__ __forceinline__ f32x4_t ld4<true, bf16>(const bf16* row, int k, int K) {
+    if (k >= K) return f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const uint2 u = *(const uint2*)(row + k);
+    return f32x4_t{__builtin_bit_cast(float, u.x << 16), __builtin_bit_cast(float, u.x & 0xffff0000u),
+                   __builtin_bit_cast(float, u.y << 16), __builtin_bit_cast(float, u.y & 0xffff0000u)};
+}
+template <> __device__ __forceinline__ f32x4_t ld4<false, float>(const float* row, int k, int K) {
+    f32x4_t v;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? row[k + e] : 0.f;
+    return v;
+}
+template <> __device__ __forceinline__ f32x4_t ld4<false, bf16>(const bf16* row, int k, int K) {
+    f32x4_t v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? bf16_to_f32(row[k + e]) : 0.f;
+    return v;
+}
 
-    for (int k0 = 0; k0 < K; k0 += TK) {
+// ---------------------------------------------------------------- few rows
+// A workgroup makes 16 columns of C for up to 64 rows (MT tiles of 16; more rows are cut into groups of
+// 64, blockIdx.y); its NW waves share K and add their sums through LDS.  Per k-step of 16 a lane brings
+// 16 bytes of a weight row and 16 of each A tile's row, straight from memory into the registers of
+// v_mfma_f32_16x16x4_f32: that takes k in any order as long as both operands agree, so lane group g holds
+// k = 4g .. 4g+3 and element e of the four goes into the e-th of four instructions.  U steps are asked
+// for together, 256 bytes of every weight row.
+// Bound by the weights' way from memory: NW is chosen so that about 2,048 waves stand in flight (see
+// launch_skinny).  Measured in 32 bits, N x K = 10,752 x 2,048: 3 rows 21.6 us (4.1 TB/s), 16 rows 29 us;
+// 2,048 x 5,376: 3 rows 19 us, 64 rows 64 us.  A wave per column with lanes along K took 82, 256, 89 us,
+// vector tiles with 64 rows 646 us.
+// A sum of K products in 32 bits loses more the longer its one running sum is.  One tile of rows keeps a
+// running sum per step and element (16 a lane, of which each takes K / (16 NW) products), added in pairs
+// at the end; with more tiles there is one per tile.
+template <typename TA, typename TW, typename TC, int MT, int NW, bool VEC>
+__global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw,
+                                                                  TC* __restrict__ C, long ldc, int M, int N, int K) {
+    constexpr int U = MT > 2 ? 2 : 4;
+    constexpr int S = MT == 1 ? 4 * U : 1;                        // running sums
+    __shared__ float part[NW][MT * 256];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16, m0 = blockIdx.y * 64;
+    const TW* w = W + (size_t)min(n0 + r, N - 1) * ldw;           // (rows and columns outside are computed from the last one and not stored)
+    const TA* a[MT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int kk = k0 + lk + i;
-            const int am = m0 + lr, wn = n0 + lr;
-            As[lk + i][lr] = (am < M && kk < K) ? ld(A + (size_t)am * lda + kk) : 0.f;
-            Ws[lk + i][lr] = (wn < N && kk < K) ? ld(W + (size_t)wn * ldw + kk) : 0.f;
+    for (int t = 0; t < MT; ++t) a[t] = A + (size_t)min(m0 + 16 * t + r, M - 1) * lda;
+    f32x4_t acc[S][MT] = {};
+    for (int k0 = wave * U * 16; k0 < K; k0 += NW * U * 16) {
+        f32x4_t wv[U], av[U][MT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + 16 * u + 4 * g;
+            wv[u] = ld4<VEC>(w, k, K);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) av[u][t] = ld4<VEC>(a[t], k, K);
         }
-        __syncthreads();
 #pragma unroll
-        for (int kk = 0; kk < TK; ++kk) {
-            float a[4], w[4];
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-        }
-        __syncthreads();
+                for (int t = 0; t < MT; ++t) {
+                    f32x4_t& sum = acc[(4 * u + e) % S][t];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u][t][e], wv[u][e], sum, 0, 0, 0);
+                }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
+    for (int s = S / 2; s > 0; s /= 2)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n < N) st(C + (size_t)m * ldc + n, acc[i][j]);
-        }
+        for (int i = 0; i < s; ++i)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[i][t] += acc[i + s][t];
+    // acc[0][t][e] is row 16 t + 4 g + e, column r
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[wave][t * 256 + (4 * g + e) * 16 + r] = acc[0][t][e];
+    __syncthreads();
+    for (int i = threadIdx.x; i < MT * 256; i += NW * 64) {
+        const int m = m0 + (i >> 4), n = n0 + (i & 15);
+        if (m >= M || n >= N) continue;
+        float sums[NW];
+#pragma unroll
+        for (int v = 0; v < NW; ++v) sums[v] = part[v][i];
+#pragma unroll
+        for (int s = NW / 2; s > 0; s /= 2)
+#pragma unroll
+            for (int v = 0; v < s; ++v) sums[v] += sums[v + s];
+        st(C + (size_t)m * ldc + n, sums[0]);
     }
 }
 
-// Up to FEW_ROWS rows of A (a decode step's tokens): a wave per column of C, the lanes along K, so a
-// weight row is read once, in whole lines, and the few rows of A come from the cache; the tiled kernel
-// above would fill a sixteenth of its tile and wait at two barriers per 16 columns of K.
-#define FEW_ROWS 16
-template <typename TA, typename TW, typename TC>
-__global__ __launch_bounds__(256) void gemm_few_rows_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W,
-                                                            long ldw, TC* __restrict__ C, long ldc, int M, int N, int K) {
-    const int lane = threadIdx.x & 63;
-    const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (n >= N) return;
-    const TW* w = W + (size_t)n * ldw;
-    float acc[FEW_ROWS];
+// ---------------------------------------------------------------- more rows
+// A workgroup of 4 waves makes BM x 64 of C.  Stages of 32 k go through LDS in two buffers: while a
+// stage is multiplied the next one's loads are in flight into registers.  v_mfma_f32_32x32x2_f32 takes
+// k in any order as long as both operands agree: a lane reads 16 bytes of a row (k = 8 j + 4 h .. + 3 for
+// half h of the wave) and the four elements go into four instructions.  Rows of 36 floats keep the
+// 16-byte reads of neighbouring rows on different banks.
+// Bound by the multiply-adds: 4 waves keep the CU's matrix units busy from 37 KB of LDS a workgroup, so
+// that others stand by for the barriers.  BM = 64: a wave per quarter of the tile.  BM = 32, where the
+// larger tiles would leave compute units without one: two waves side by side, two sharing every
+// stage's k, added at the end.  Tiles one below the other follow each other on an XCD (workgroups go
+// to the 8 XCDs in turn), so that a panel of weights is read into one L2.
+// Measured in 32 bits: 777 rows by 10,752 x 2,048 352 us (97 TFLOP/s), by 2,048 x 5,376 213 us; 2,048 rows
+// by 10,752 x 2,048 840 us (107 TFLOP/s).  Vector multiply-adds from 64 x 64 tiles took 1,280, 837 and 2,471 us.
+#define TN 64
+#define TK 32
+#define TS (TK + 4)
+template <typename TA, typename TW, typename TC, int BM, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw,
+                                                             TC* __restrict__ C, long ldc, int M, int N, int K, int m_tiles, int tiles) {
+    constexpr int AR = BM / 32;                                   // rows of A a thread brings per stage
+    __shared__ float As[2][BM * TS], Ws[2][TN * TS];
+    const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int m0 = tile % m_tiles * BM, n0 = tile / m_tiles * TN;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wn = wave & 1;                                      // which 32 columns
+    const int wm = BM == 64 ? wave >> 1 : 0;                      // which 32 rows
+    const int wk = BM == 64 ? 0 : wave >> 1;                      // which half of a stage's k
+    const int lr = threadIdx.x >> 3, lk = (threadIdx.x & 7) * 4;  // loader: a row, 4 neighbouring k
+    const TA* a[AR];
+    const TW* w[2];
 #pragma unroll
-    for (int m = 0; m < FEW_ROWS; ++m) acc[m] = 0.f;
-    for (int k = lane; k < K; k += 64) {
-        const float wk = ld(w + k);
+    for (int i = 0; i < AR; ++i) a[i] = A + (size_t)min(m0 + lr + 32 * i, M - 1) * lda;
 #pragma unroll
-        for (int m = 0; m < FEW_ROWS; ++m)
-            if (m < M) acc[m] = fmaf(ld(A + (size_t)m * lda + k), wk, acc[m]);
-    }
+    for (int i = 0; i < 2; ++i) w[i] = W + (size_t)min(n0 + lr + 32 * i, N - 1) * ldw;
+    f32x4_t ra[AR], rw[2];
+    auto fetch = [&](int k0) {
 #pragma unroll
-    for (int m = 0; m < FEW_ROWS; ++m) {
-        if (m < M) {                                        // (M is the same for every lane)
-            const float sum = wave_sum(acc[m]);
-            if (lane == 0) st(C + (size_t)m * ldc + n, sum);
+        for (int i = 0; i < AR; ++i) ra[i] = ld4<VEC>(a[i], k0 + lk, K);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) rw[i] = ld4<VEC>(w[i], k0 + lk, K);
+    };
+    auto put = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < AR; ++i) *(f32x4_t*)&As[b][(lr + 32 * i) * TS + lk] = ra[i];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *(f32x4_t*)&Ws[b][(lr + 32 * i) * TS + lk] = rw[i];
+    };
+    f32x16_t acc = {};
+    fetch(0);
+    put(0);
+    __syncthreads();
+    const int row = (lane & 31) * TS + (lane >> 5) * 4;
+    for (int k0 = 0, b = 0; k0 < K; k0 += TK, b ^= 1) {
+        if (k0 + TK < K) fetch(k0 + TK);
+        const float* pa = &As[b][wm * 32 * TS + row];
+        const float* pw = &Ws[b][wn * 32 * TS + row];
+#pragma unroll
+        for (int j = 0; j < (BM == 64 ? 4 : 2); ++j) {
+            const int o = 8 * j + (BM == 64 ? 0 : 16 * wk);
+            const f32x4_t va = *(const f32x4_t*)(pa + o), vw = *(const f32x4_t*)(pw + o);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va[e], vw[e], acc, 0, 0, 0);
         }
+        if (k0 + TK < K) put(b ^ 1);                              // (the other buffer was last read before the barrier below)
+        __syncthreads();
     }
+    if (BM == 32) {                                               // the second pair's sums, 32 x 64 floats, through the first buffer
+        static_assert(64 * 17 * 2 <= 2 * 32 * TS, "a wave's sums, padded by one float a lane, fit");
+        float* half = &As[0][0] + wn * 64 * 17;
+        if (wk == 1)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) half[lane * 17 + e] = acc[e];
+        __syncthreads();
+        if (wk == 1) return;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] += half[lane * 17 + e];
+    }
+    // acc[e] is row 8 (e/4) + 4 (lane/32) + e%4, column lane%32
+    const int n = n0 + wn * 32 + (lane & 31);
+    if (n >= N) return;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wm * 32 + 8 * (e / 4) + 4 * (lane >> 5) + e % 4;
+        if (m < M) st(C + (size_t)m * ldc + n, acc[e]);
+    }
+}
+
+// ---------------------------------------------------------------- launch
+#define SKINNY_M 64
+#define COMPUTE_UNITS 256
+
+template <typename TA, typename TW, typename TC, int MT, bool VEC>
+static void launch_skinny(const TA* A, long lda, const TW* W, long ldw, TC* C, long ldc, int M, int N, int K, hipStream_t stream) {
+    const dim3 groups((N + 15) / 16, (M + 63) / 64);
+    // waves a workgroup: enough for 2,048 in all, as far as K has a stretch for each
+    const int want = (2048 + groups.x - 1) / groups.x, most = (K + 63) / 64;
+    const int waves = want < most ? want : most;
+    if (waves > 8 && MT <= 2)
+        gemm_f32_skinny_kernel<TA, TW, TC, MT <= 2 ? MT : 1, 16, VEC><<<groups, 1024, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    else if (waves > 4)
+        gemm_f32_skinny_kernel<TA, TW, TC, MT, 8, VEC><<<groups, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    else
+        gemm_f32_skinny_kernel<TA, TW, TC, MT, 4, VEC><<<groups, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+}
+
+template <typename TA, typename TW, typename TC, bool VEC>
+static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long ldc, int M, int N, int K, hipStream_t stream) {
+    if (M <= 16) return launch_skinny<TA, TW, TC, 1, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+    if (M <= 32) return launch_skinny<TA, TW, TC, 2, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+    // from 65 rows on: tiles as soon as the smaller ones give every compute unit one (80 rows by 2,048 x 2,048, 96 of
+    // them: 47 us tiled, 24 us in groups of 64 rows; 200 rows, 224: 47 us in groups, 300 rows, 320: 52 us tiled)
+    const int n_tiles = (N + TN - 1) / TN;
+    const long small_tiles = (long)n_tiles * ((M + 31) / 32);
+    if (M <= SKINNY_M || small_tiles < COMPUTE_UNITS) return launch_skinny<TA, TW, TC, 4, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+    const bool large = (long)n_tiles * ((M + 63) / 64) >= COMPUTE_UNITS;
+    const int bm = large ? 64 : 32, m_tiles = (M + bm - 1) / bm, tiles = m_tiles * n_tiles;
+    const int grid = (tiles + 7) / 8 * 8;
+    if (large)
+        gemm_f32_tiled_kernel<TA, TW, TC, 64, VEC><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
+    else
+        gemm_f32_tiled_kernel<TA, TW, TC, 32, VEC><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
+}
+
+template <typename T> static bool rows_of_fours(const void* p, long ld) {
+    return ld % 4 == 0 && (uintptr_t)p % (4 * sizeof(T)) == 0;
 }
 
 template <typename TA, typename TW, typename TC>
 static void launch_gemm(const void* A, long lda, const void* W, long ldw, void* C, long ldc, int M, int N, int K,
                         hipStream_t stream) {
-    if (M <= FEW_ROWS) {
-        gemm_few_rows_kernel<TA, TW, TC><<<(N + 3) / 4, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, ldw, (TC*)C, ldc, M, N, K);
-        return;
-    }
-    dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
-    gemm_tn_kernel<TA, TW, TC><<<grid, 256, 0, stream>>>((const TA*)A, lda, (const TW*)W, ldw, (TC*)C, ldc, M, N, K);
+    if (K % 4 == 0 && rows_of_fours<TA>(A, lda) && rows_of_fours<TW>(W, ldw))
+        launch_vec<TA, TW, TC, true>((const TA*)A, lda, (const TW*)W, ldw, (TC*)C, ldc, M, N, K, stream);
+    else
+        launch_vec<TA, TW, TC, false>((const TA*)A, lda, (const TW*)W, ldw, (TC*)C, ldc, M, N, K, stream);
 }
 
 extern "C" int agave_gemm_plain(int dt_a, const void* A, long lda, int dt_w, const void* W, long ldw, int dt_c,
                                 void* C, long ldc, int M, int N, int K, hipStream_t stream) {
     AGAVE_CHECK(M >= 0 && N > 0 && K > 0, "gemm_plain: bad sizes M=%d N=%d K=%d", M, N, K);
     AGAVE_CHECK(lda >= K && ldw >= K && ldc >= N, "gemm_plain: a row stride is too small (lda=%ld ldw=%ld ldc=%ld)", lda, ldw, ldc);
-    AGAVE_CHECK((M + TM - 1) / TM <= 65535, "gemm_plain: M=%d exceeds the grid limit", M);
+    AGAVE_CHECK((M + 63) / 64 <= 65535, "gemm_plain: M=%d exceeds the grid limit", M);
+    AGAVE_CHECK((long)((M + 31) / 32) * ((N + TN - 1) / TN) < (1L << 30), "gemm_plain: M=%d x N=%d exceeds the grid limit", M, N);
     if (M == 0) return 0;
     const int code = dt_a * 4 + dt_w * 2 + dt_c;
     switch (code) {

@@ -68,7 +68,7 @@ class Engine:
         reach plus one piece per sequence, so their share of the cache does not grow with
         the context.
         ``keep_stored_precision``: in a bfloat16 engine a matrix that the checkpoint stores in
-        32-bit stays in 32-bit (its products then run on the plain multiply-add kernel, far from
+        32-bit stays in 32-bit (its products then run on the plain 32-bit kernel, far from
         the matrix cores' speed; a line on standard error says how many do); False casts such
         matrices to bfloat16 at load.  Half precision is always cast to the engine's type.
         ``will_sample`` False: the sampling kernels are not built with the others at construction (a
@@ -102,7 +102,7 @@ class Engine:
         if self.env.kept_32bit:
             kept = self.env.kept_32bit
             library._log(f"{len(kept)} weight matrices are stored in 32-bit and stay so ({', '.join(sorted(set(kept)))}): "
-                         f"their products run on the plain multiply-add kernel, not on the matrix cores; "
+                         f"their products run on the plain 32-bit kernel, not in bfloat16; "
                          f"keep_stored_precision=False (--cast-weights) casts them to bfloat16")
         if max_context is None:
             self.max_context = min(int(spec.max_context), DEFAULT_CONTEXT)

@@ -411,7 +411,7 @@ def cast(src: torch.Tensor, dst: torch.Tensor) -> None:
 
 
 def gemm_plain(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor) -> None:
-    """c[M,N] = a[M,K] @ w[N,K]^T with 32-bit accumulation (ordinary multiply-adds)."""
+    """c[M,N] = a[M,K] @ w[N,K]^T with 32-bit products and accumulation."""
     _dev(a, w, c)
     lda, ldw, ldc = _rows(a, "a"), _rows(w, "w"), _rows(c, "c")
     m, k = a.shape

@@ -3,7 +3,7 @@
 The weight's element type is the build environment's choice (``BuildEnv.weight_dtype``): a
 32-bit engine widens everything (exactly); a bfloat16 engine keeps bfloat16, casts half
 precision to bfloat16, and keeps a matrix that was stored in 32-bit as it is unless told to cast
-it.  The kernel is chosen by the types: 32-bit anything goes through the plain multiply-add
+it.  The kernel is chosen by the types: 32-bit anything goes through the plain 32-bit
 kernel; bfloat16 activations with bfloat16 weights go through the matrix-core kernels, which
 fall back to the plain kernel for shapes they refuse.
 """

@@ -279,6 +279,35 @@ def test_gemm_plain(K, ta, tw, tc, m, n, k):
     assert torch.allclose(c.cpu().double(), wide[:, 5:5 + k].cpu().double() @ w.double().T, **tol)
 
 
+@pytest.mark.parametrize("ta,tw", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 64, 65, 96, 300])
+@pytest.mark.parametrize("n,k", [(1, 4), (16, 64), (17, 1028), (63, 36), (130, 515), (2100, 260)])
+def test_gemm_plain_tiles(K, ta, tw, m, n, k):
+    """Edges of the tiles of rows, columns and k, whole and broken stretches of four, and rows that are not aligned.
+    Sums of K products in 32-bit are off by at most K 2^-24 of the sum of their sizes."""
+    g = torch.Generator().manual_seed(m * 7 + n)
+    a, w = torch.randn(m, k + 3, generator=g).to(ta).to(DEV), torch.randn(n, k, generator=g).to(tw).to(DEV)
+    for x in (a[:, :k].contiguous(), a[:, 3:]):
+        c = torch.full((m + 1, n + 2), 7.0, device=DEV)
+        K.gemm_plain(x, w, c[:m, :n])
+        bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        assert bool(((c[:m, :n].double() - x.double() @ w.double().T).abs() <= bound).all())
+        assert bool((c[m] == 7.0).all()) and bool((c[:, n:] == 7.0).all())       # nothing outside is written
+
+
+def test_gemm_plain_special_values(K):
+    """A NaN or an infinity stays in its row and column, and zeros behind the last k meet zeros only."""
+    for m in (3, 70):
+        a, w = torch.ones(m, 18, device=DEV), torch.ones(40, 18, device=DEV)
+        a[1, 17], w[5, 2] = float("nan"), float("inf")
+        c = torch.empty(m, 40, device=DEV)
+        K.gemm_plain(a, w, c)
+        want = torch.full((m, 40), 18.0, device=DEV)
+        want[:, 5] = float("inf")
+        want[1] = float("nan")
+        assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c[~c.isnan()], want[~want.isnan()])
+
+
 def _attn_case(K, dtype, nh, nkv, hd, lens, window, scale, seed=0, boost=None):
     """Sequences of the given lengths in scattered pages; every position is a query."""
     g = torch.Generator().manual_seed(seed)
