@@ -17,7 +17,7 @@
 //
 // A (token, slot) pair p = t * top + slot names one chosen output.  The plain kernels take the pairs
 // as they come (a wave per pair and output column).  The matrix-core kernels take them sorted by
-// expert, in tiles of 16 or 64 pairs that never span two experts (`route_sort` makes the list and the
+// expert, in tiles of 16, 64 or 128 pairs that never span two experts (`route_sort` makes the list and the
 // tiles' table on the device, so a step's launches never depend on the choice).
 #include "common_impl.h"
 #include "mfma.h"
@@ -400,19 +400,45 @@ __global__ __launch_bounds__(256) void routed_down_plain_kernel(const T* __restr
 
 // out[t] = sum over the token's pairs of weight * (expert row, or the input row for an identity expert) + shared[t].
 // `place` (may be null): where pair p's row lies in y (a sorted list); null: at p.
-template <typename T>
+// A thread makes V neighbours of a row: 4 where rows and sizes allow accesses of four elements (bound by memory: 3,001
+// tokens of 4 pairs and 2,048 columns, 135 MB, 24.8 us; one element a thread took 39.7), 1 otherwise.
+template <int V, typename T> __device__ __forceinline__ void load_few(const T* p, float* v);
+template <> __device__ __forceinline__ void load_few<1, float>(const float* p, float* v) { v[0] = *p; }
+template <> __device__ __forceinline__ void load_few<1, bf16>(const bf16* p, float* v) { v[0] = bf16_to_f32(*p); }
+template <> __device__ __forceinline__ void load_few<4, float>(const float* p, float* v) {
+    const float4 u = *reinterpret_cast<const float4*>(p);
+    v[0] = u.x; v[1] = u.y; v[2] = u.z; v[3] = u.w;
+}
+template <> __device__ __forceinline__ void load_few<4, bf16>(const bf16* p, float* v) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
+    v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
+}
+template <int V, typename T> __device__ __forceinline__ void store_few(T* p, const float* v);
+template <> __device__ __forceinline__ void store_few<1, float>(float* p, const float* v) { *p = v[0]; }
+template <> __device__ __forceinline__ void store_few<1, bf16>(bf16* p, const float* v) { *p = f32_to_bf16(v[0]); }
+template <> __device__ __forceinline__ void store_few<4, float>(float* p, const float* v) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+template <> __device__ __forceinline__ void store_few<4, bf16>(bf16* p, const float* v) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
+}
+
+template <typename T, int V>
 __global__ void routed_combine_kernel(const float* __restrict__ y, const int* __restrict__ place, const int* __restrict__ choice,
                                       const float* __restrict__ weight, const T* __restrict__ x, long ldx,
                                       const T* __restrict__ shared, long lds, const float* __restrict__ shared_gate,
                                       T* __restrict__ out, long ldo, int N, int top, int E, int hidden) {
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long idx = ((long)blockIdx.x * blockDim.x + threadIdx.x) * V;
     if (idx >= (long)N * hidden) return;
     const int t = (int)(idx / hidden), c = (int)(idx % hidden);
     // (no load under a per-lane condition: the input row's element is read once, an expert row's from a row that exists
     // whatever the choice, and what does not count is left out afterwards)
-    const float xv = ld(x + (size_t)t * ldx + c);
-    const float sv = ld((shared ? shared : x) + (size_t)t * (shared ? lds : ldx) + c);
-    float acc = 0.f;
+    float xv[V], sv[V], acc[V];
+    load_few<V>(x + (size_t)t * ldx + c, xv);
+    load_few<V>((shared ? shared : x) + (size_t)t * (shared ? lds : ldx) + c, sv);
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
 #pragma unroll 4
     for (int r = 0; r < top; ++r) {
         const int p = t * top + r;
@@ -421,12 +447,16 @@ __global__ void routed_combine_kernel(const float* __restrict__ y, const int* __
         const bool expert = e >= 0 && e < E;
         int row = place ? place[p] : p;
         row = (expert && row >= 0) ? row : 0;
-        const float yv = y ? y[(size_t)row * hidden + c] : 0.f;
-        acc = fmaf(w, e >= E ? xv : (expert ? yv : 0.f), acc);
+        float yv[V] = {};
+        if (y) load_few<V>(y + (size_t)row * hidden + c, yv);
+#pragma unroll
+        for (int i = 0; i < V; ++i) acc[i] = fmaf(w, e >= E ? xv[i] : (expert ? yv[i] : 0.f), acc[i]);
     }
     // (the shared expert's row, times the sigmoid of a logit per token where it has a gate)
-    if (shared) acc = shared_gate ? fmaf(1.0f / (1.0f + expf(-shared_gate[t])), sv, acc) : acc + sv;
-    st(out + (size_t)t * ldo + c, acc);
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+        if (shared) acc[i] = shared_gate ? fmaf(1.0f / (1.0f + expf(-shared_gate[t])), sv[i], acc[i]) : acc[i] + sv[i];
+    store_few<V>(out + (size_t)t * ldo + c, acc);
 }
 
 extern "C" int agave_routed_experts_plain(int dtype, const void* x, long ldx, const int* choice, const void* wg, const void* wu,
@@ -459,16 +489,19 @@ extern "C" int agave_routed_combine(int dtype, const float* y, const int* place,
     AGAVE_CHECK(choice && weight && x && out && (E == 0 || y) && ldx >= hidden && ldo >= hidden && (!shared || lds >= hidden),
                 "routed_combine: bad buffers");
     if (N == 0) return 0;
-    const long total = (long)N * hidden;
-    const int blocks = (int)((total + 255) / 256);
-    if (dtype == AGAVE_F32)
-        routed_combine_kernel<float><<<blocks, 256, 0, stream>>>(y, place, choice, weight, (const float*)x, ldx, (const float*)shared,
-                                                                 lds, shared_gate, (float*)out, ldo, N, top, E, hidden);
-    else if (dtype == AGAVE_BF16)
-        routed_combine_kernel<bf16><<<blocks, 256, 0, stream>>>(y, place, choice, weight, (const bf16*)x, ldx, (const bf16*)shared,
-                                                                lds, shared_gate, (bf16*)out, ldo, N, top, E, hidden);
-    else
-        AGAVE_CHECK(false, "routed_combine: unknown dtype %d", dtype);
+    AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "routed_combine: unknown dtype %d", dtype);
+    const uintptr_t wide = 4 * (dtype == AGAVE_F32 ? 4 : 2);           // bytes of four neighbours in a row
+    const bool fours = hidden % 4 == 0 && ldx % 4 == 0 && ldo % 4 == 0 && (!shared || lds % 4 == 0) && (uintptr_t)x % wide == 0 &&
+                       (uintptr_t)out % wide == 0 && (uintptr_t)shared % wide == 0 && (uintptr_t)y % 16 == 0;
+    const long blocks = ((long)N * hidden / (fours ? 4 : 1) + 255) / 256;
+#define COMBINE_GO(T_, V_) routed_combine_kernel<T_, V_><<<(unsigned)blocks, 256, 0, stream>>>(y, place, choice, weight, (const T_*)x, ldx, \
+        (const T_*)shared, lds, shared_gate, (T_*)out, ldo, N, top, E, hidden)
+    if (dtype == AGAVE_F32) {
+        if (fours) COMBINE_GO(float, 4); else COMBINE_GO(float, 1);
+    } else {
+        if (fours) COMBINE_GO(bf16, 4); else COMBINE_GO(bf16, 1);
+    }
+#undef COMBINE_GO
     AGAVE_LAUNCH_CHECK("routed_combine");
     return 0;
 }
@@ -521,7 +554,7 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const int* __restrict_
 
 extern "C" int agave_route_sort(const int* choice, int P, int E, int TM, int cap, int max_tiles, int* place, int* sorted_pair,
                                 int* tile_expert, hipStream_t stream) {
-    AGAVE_CHECK(P >= 0 && E > 0 && E <= ROUTE_MAX && (TM == 16 || TM == 64), "route_sort: bad sizes P=%d E=%d TM=%d", P, E, TM);
+    AGAVE_CHECK(P >= 0 && E > 0 && E <= ROUTE_MAX && (TM == 16 || TM == 64 || TM == 128), "route_sort: bad sizes P=%d E=%d TM=%d", P, E, TM);
     AGAVE_CHECK(max_tiles >= (P + TM - 1) / TM + E && cap >= max_tiles * TM, "route_sort: %d tiles of %d rows do not hold %d pairs of %d experts",
                 max_tiles, TM, P, E);
     AGAVE_CHECK(choice && place && sorted_pair && tile_expert, "route_sort: null buffer");
@@ -682,17 +715,203 @@ __global__ __launch_bounds__(256) void routed_product_mfma_kernel(const bf16* __
         }
 }
 
+// Many pairs an expert, weights in tile order: a workgroup takes a tile of TT sorted rows and 2 TT columns of weights
+// (GATED: TT columns of the gate and the same of the up matrix), TT/16 waves of 64 weight columns by TT/2 rows each.
+// Bound by the multiply-adds once both operands come through LDS: a wave that loads its own operands asks the compute
+// unit's cache for 96 bytes a clock where it delivers 64.  Both operands go straight from memory into LDS (a kilobyte a
+// load), stages of 32 columns in a ring of NS buffers, the loads of NS - 1 stages in flight while one is multiplied; 72 KB
+// (TT 128), so that two workgroups share a compute unit and one multiplies while the other waits at its barrier.
+// The rows' 16-byte pieces are permuted by the row so that the rows an operand reads lie in different banks.
+// Workgroups go to the 8 XCDs in turn: each XCD takes an eighth of the tiles there are (neighbours, so mostly one expert's)
+// and walks them column block by column block, which keeps an expert's block of weights in that XCD's L2 while its tiles
+// pass over it.
+// Measured, both products, 16 experts of 2,048 by 2,048: 12,004 pairs in tiles of 128 445 us (679 TFLOP/s), of 64 572 us;
+// 3,200 pairs 138 and 209 us; 64 pairs in tiles of 64 84 us (4.8 TB/s of weights).  With every wave loading its own operands
+// (as below, tiles of 64) 987 us, 334 us; tiles of 16 109 us at 64 pairs.
+template <int TT, bool GATED>
+__global__ __launch_bounds__(TT * 4, 4) void routed_product_tiled_kernel(const bf16* __restrict__ x, long ldx, const int* __restrict__ sorted_pair,
+                                                                         const int* __restrict__ tile_expert, int max_tiles,
+                                                                         const uint4* __restrict__ w0, const uint4* __restrict__ w1,
+                                                                         void* __restrict__ out_, int top, int n_out, int K, int act, float p0,
+                                                                         float p1) {
+    constexpr int NWV = TT / 16, WSLOTS = TT / 8;                 // waves; weight tiles of 16 columns a stage
+    constexpr int NS = TT == 128 ? 3 : 4;
+    constexpr int X_BYTES = TT * 64, STAGE = X_BYTES + WSLOTS * 1024;
+    constexpr int XB = TT / 32;                                   // 16-row tiles of a wave
+    constexpr int COLS = GATED ? TT : 2 * TT;                     // columns of the result
+    constexpr int LOADS = 3;                                      // a wave's loads per stage: 1 of rows, 2 of weights
+    extern __shared__ __attribute__((aligned(16))) unsigned char rt_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int wn = wave >> 1, wm = wave & 1;
+    const int c = lane & 15, g = lane >> 4;
+    // this XCD's share of the tiles that hold rows (they are the first ones of the table)
+    int count = 0;
+    for (int t0 = 0; t0 < max_tiles; t0 += 64) {
+        const int t = t0 + lane;
+        count += __popcll(__ballot(tile_expert[t < max_tiles ? t : max_tiles - 1] >= 0 && t < max_tiles));
+    }
+    const int share = (count + 7) / 8;
+    if (share == 0) return;
+    const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
+    const int tile = xcd * share + turn % share, col0 = turn / share * COLS;
+    if (tile >= count || col0 >= n_out) return;
+    const int e = tile_expert[tile];
+    const int row0 = tile * TT;
+    const int KB = K / 32, NBK = n_out / 16;
+
+    // staging: one 16-byte piece of a row and two weight tiles a wave and stage
+    const unsigned char* xsrc;
+    {
+        const int o = wave * 64 + lane, row = o >> 2, piece = (o & 3) ^ ((row >> 2) & 3);
+        long r = row0 + row;
+        if (GATED) {
+            const int p = sorted_pair[r];
+            r = p >= 0 ? p / top : 0;                             // (a padding row computes on row 0 and is never read)
+        }
+        xsrc = (const unsigned char*)(x + (size_t)r * ldx) + piece * 16;
+    }
+    const unsigned char* wsrc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int slot = wave * 2 + i;
+        const uint4* w = GATED && slot >= WSLOTS / 2 ? w1 : w0;
+        int nb = col0 / 16 + (GATED ? slot % (WSLOTS / 2) : slot);
+        if (nb >= NBK) nb = NBK - 1;                              // (columns past the end: never stored)
+        wsrc[i] = (const unsigned char*)(w + ((size_t)e * NBK + nb) * KB * 64) + lane * 16;
+    }
+    auto fetch_one = [&](int st, int buf, int i) {                // load i of stage st (past the end: the last one again, never used)
+        const size_t ste = st < KB ? st : KB - 1;
+        unsigned char* dst = rt_lds + buf * STAGE + (i == 0 ? wave * 1024 : X_BYTES + (wave * 2 + i - 1) * 1024);
+        const unsigned char* src = i == 0 ? xsrc + ste * 64 : wsrc[i - 1] + ste * 1024;
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    };
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)rt_lds;
+    // operand a of a wave: 16 weight columns.  GATED: a = 0, 1 the gate's, 2, 3 the up matrix's of the same 32 columns
+    const unsigned w_lane = lds0 + X_BYTES + (GATED ? wn * 2 : wn * 4) * 1024 + lane * 16;
+    constexpr int UP_AT = GATED ? (WSLOTS / 2 - 2) * 1024 : 0;    // from slot a = 2 on: the up matrix's half
+    const unsigned x_lane = lds0 + (wm * (TT / 2) + c) * 64 + ((g ^ ((c >> 2) & 3)) * 16);
+
+    f32x4_t acc[4][XB];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < XB; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < NS - 1; ++st)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) fetch_one(st, st, i);
+    constexpr int IN_FLIGHT = LOADS * (NS - 2);
+    int buf = 0, fill = NS - 1;
+    for (int st = 0; st < KB; ++st) {
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (IN_FLIGHT & 15) | ((IN_FLIGHT >> 4) << 14));
+        __builtin_amdgcn_s_barrier();                             // stage st has landed; stage st - 1 has been read by all
+        frag16 fw[4], fx[XB];
+        const unsigned wa = w_lane + buf * STAGE, xa = x_lane + buf * STAGE;
+        static_for<0, 4>([&](auto a) { lds_read16<a.value * 1024 + (a.value >= 2 ? UP_AT : 0)>(fw[a.value], wa); });
+        static_for<0, XB>([&](auto b) { lds_read16<b.value * 1024>(fx[b.value], xa); });
+        lds_settle();
+#pragma unroll
+        for (int a = 0; a < 4; ++a) lds_use(fw[a]);
+#pragma unroll
+        for (int b = 0; b < XB; ++b) lds_use(fx[b]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < XB; ++b) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a) acc[a][b] = mfma_16x16x32(fw[a], fx[b], acc[a][b]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (b < LOADS) fetch_one(st + NS - 1, fill, b);       // a load at a time, between the multiplications
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int b = XB; b < LOADS; ++b) fetch_one(st + NS - 1, fill, b);
+        buf = buf + 1 == NS ? 0 : buf + 1;
+        fill = fill + 1 == NS ? 0 : fill + 1;
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);                           // loads past the last stage must have landed before LDS is used again
+
+    // acc[a][b]: row 16 b + c of the wave's rows, columns 4 g .. 4 g + 3 of operand a.  Half of the tile's rows at a time go
+    // through LDS and leave it row by row, 16 bytes a lane in whole lines.
+    constexpr int ES = GATED ? 2 : 4, ROW_BYTES = COLS * ES, CH = ROW_BYTES / 16, SWZ = (CH < 32 ? CH : 32) - 1;
+    static_assert((TT / 2) * ROW_BYTES <= NS * STAGE, "half of the finished tile fits the LDS");
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        __syncthreads();
+        if (wm == half) {
+#pragma unroll
+            for (int b = 0; b < XB; ++b) {
+                const int t = 16 * b + c;
+#pragma unroll
+                for (int a = 0; a < (GATED ? 2 : 4); ++a) {
+                    const int off = (GATED ? wn * 32 + a * 16 + 4 * g : wn * 64 + a * 16 + 4 * g) * ES;
+                    unsigned char* dst = rt_lds + t * ROW_BYTES + (((off >> 4) ^ (t & SWZ)) << 4) + (off & 15);
+                    if constexpr (GATED) {
+                        float v[4];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)               // (gate and up are rounded to the rows' type before the activation, as the plain kernel does)
+                            v[k] = expert_gated(bf16_to_f32(f32_to_bf16(acc[a][b][k])), bf16_to_f32(f32_to_bf16(acc[a + 2][b][k])), act, p0, p1);
+                        *reinterpret_cast<uint2*>(dst) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
+                    } else {
+                        *reinterpret_cast<f32x4_t*>(dst) = acc[a][b];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        constexpr int ROWS_PER = 64 / CH > 0 ? 64 / CH : 1;       // rows of one store
+        const int piece = lane % CH;
+        for (int t = wave * ROWS_PER + lane / CH; t < TT / 2; t += NWV * ROWS_PER) {
+            const int col = col0 + piece * (16 / ES);
+            if (col >= n_out) continue;                           // (n_out is a multiple of 16: a piece is inside or outside)
+            const uint4 v = *reinterpret_cast<const uint4*>(rt_lds + t * ROW_BYTES + ((piece ^ (t & SWZ)) << 4));
+            *reinterpret_cast<uint4*>((unsigned char*)out_ + ((size_t)(row0 + half * (TT / 2) + t) * n_out + col) * ES) = v;
+        }
+    }
+}
+
+template <int TT, bool GATED>
+static int launch_routed_tiled(const void* x, long ldx, const int* sorted_pair, const int* tile_expert, int max_tiles, const void* w0,
+                               const void* w1, void* out, int top, int n_out, int K, int act, float p0, float p1, hipStream_t stream) {
+    constexpr int COLS = GATED ? TT : 2 * TT;
+    constexpr size_t lds = (size_t)(TT == 128 ? 3 : 4) * (TT * 64 + TT / 8 * 1024);
+    const long wgs = 8L * ((max_tiles + 7) / 8) * ((n_out + COLS - 1) / COLS);
+    AGAVE_CHECK(wgs < (1L << 31), "routed_experts_mfma: too many tiles for the grid");
+    static bool raised = false;
+    if (!raised) {
+        hipError_t e = hipFuncSetAttribute((const void*)routed_product_tiled_kernel<TT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        AGAVE_CHECK(e == hipSuccess, "routed_experts_mfma: cannot raise the LDS allowance");
+        raised = true;
+    }
+    routed_product_tiled_kernel<TT, GATED><<<(unsigned)wgs, TT * 4, lds, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, max_tiles,
+                                                                                   (const uint4*)w0, (const uint4*)w1, out, top, n_out, K, act, p0, p1);
+    return 0;
+}
+
 // act_rows [cap, ff] bfloat16 and y [cap, hidden] float32 hold sorted rows (see route_sort)
 extern "C" int agave_routed_experts_mfma(const void* x, long ldx, const int* sorted_pair, const int* tile_expert, const void* wg,
                                          const void* wu, const void* wd, void* act_rows, float* y, int TM, int max_tiles, int top,
                                          int E, int ff, int hidden, int act, int wpacked, float p0, float p1, hipStream_t stream) {
     AGAVE_CHECK(!wpacked || (ff % 32 == 0 && hidden % 32 == 0), "routed_experts_mfma: weights in tile order need sizes that are multiples of 32");
-    AGAVE_CHECK(max_tiles > 0 && top > 0 && E > 0 && ff > 0 && hidden > 0 && (TM == 16 || TM == 64), "routed_experts_mfma: bad sizes");
+    AGAVE_CHECK(max_tiles > 0 && top > 0 && E > 0 && ff > 0 && hidden > 0 && (TM == 16 || TM == 64 || (TM == 128 && wpacked)), "routed_experts_mfma: bad sizes");
     AGAVE_CHECK((act >= 0 && act < 4) || act == 6, "routed_experts_mfma: unknown activation %d", act);
     AGAVE_CHECK(hidden % 8 == 0 && ff % 8 == 0 && ldx % 8 == 0, "routed_experts_mfma: sizes must be multiples of 8 (hidden %d, ff %d)", hidden, ff);
     AGAVE_CHECK(x && sorted_pair && tile_expert && wg && wu && wd && act_rows && y, "routed_experts_mfma: null buffer");
     AGAVE_CHECK(((uintptr_t)x % 16) == 0 && ((uintptr_t)wg % 16) == 0 && ((uintptr_t)wu % 16) == 0 && ((uintptr_t)wd % 16) == 0 &&
                 ((uintptr_t)act_rows % 16) == 0, "routed_experts_mfma: buffers must be aligned to 16 bytes");
+    if (wpacked && TM >= 64) {
+        int rc;
+        if (TM == 128) {
+            rc = launch_routed_tiled<128, true>(x, ldx, sorted_pair, tile_expert, max_tiles, wg, wu, act_rows, top, ff, hidden, act, p0, p1, stream);
+            if (rc == 0) rc = launch_routed_tiled<128, false>(act_rows, ff, sorted_pair, tile_expert, max_tiles, wd, nullptr, y, top, hidden, ff, act, p0, p1, stream);
+        } else {
+            rc = launch_routed_tiled<64, true>(x, ldx, sorted_pair, tile_expert, max_tiles, wg, wu, act_rows, top, ff, hidden, act, p0, p1, stream);
+            if (rc == 0) rc = launch_routed_tiled<64, false>(act_rows, ff, sorted_pair, tile_expert, max_tiles, wd, nullptr, y, top, hidden, ff, act, p0, p1, stream);
+        }
+        if (rc != 0) return rc;
+        AGAVE_LAUNCH_CHECK("routed_experts_mfma");
+        return 0;
+    }
     // tiles of 64 rows take 64 columns a wave (an operand that was loaded serves more multiplications); a tile of
     // 16 rows, which streams its weights once, takes 16 columns a workgroup, whose waves share K
     const int cols = TM == 64 ? 256 : 16;

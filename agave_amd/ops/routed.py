@@ -91,11 +91,23 @@ def combine(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: to
                  lds, ptr(shared_gate) if shared is not None else None, ptr(out), ldo, n, top, n_experts, hidden, stream())
 
 
-def tile_plan(n_pairs: int, n_experts: int):
-    """(rows a tile, tiles at most, sorted rows at most) of the sorted list of ``n_pairs`` pairs: tiles of 64 rows
-    where an expert gets some 32 pairs or more on average, of 16 otherwise; every expert's run of rows is padded to
-    whole tiles, so there are at most ``ceil(pairs / rows) + experts`` tiles."""
+def tile_plan(n_pairs: int, n_experts: int, tile_order: bool = False, ff: int = 0, hidden: int = 0):
+    """(rows a tile, tiles at most, sorted rows at most) of the sorted list of ``n_pairs`` pairs; every expert's run of rows
+    is padded to whole tiles, so there are at most ``ceil(pairs / rows) + experts`` tiles.
+
+    Weights row by row: tiles of 64 rows where an expert gets some 32 pairs or more on average, of 16 otherwise.
+    Weights in tile order (``tile_order``, experts of ``ff`` inner rows and ``hidden`` columns): 128 from 128 pairs an expert
+    on; 64 from two pairs an expert on where their workgroups (64 inner rows, 128 columns each) about fill the chip; below
+    that 16.  Measured with 16 experts of 2,048 by 2,048, both products: 16 pairs 66 us in tiles of 16 and 69 in tiles of 64,
+    32 pairs 101 and 82, 256 pairs 156 and 86; 1,600 pairs 124 us in tiles of 64 and 125 in tiles of 128, 2,400 pairs 162
+    and 137."""
     tm = 64 if n_pairs >= 32 * n_experts else 16
+    if tile_order:
+        live = min(n_pairs, n_experts)
+        if n_pairs >= 128 * n_experts:
+            tm = 128
+        elif n_pairs >= 2 * n_experts and live * (ff // 64) >= 256 and live * (hidden // 128) >= 128:
+            tm = 64
     tiles = (n_pairs + tm - 1) // tm + n_experts
     return tm, tiles, tiles * tm
 

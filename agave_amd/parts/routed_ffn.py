@@ -109,7 +109,7 @@ class RoutedFfn:
             raise ValueError("routed feed-forward: its experts are kept in tile order, which takes aligned bfloat16 rows")
         if s.n_experts and self.w_gate.dtype == torch.bfloat16 and routed.mfma_ok(x, s.intermediate):
             # the pairs sorted by expert on the device, then the experts' products tile by tile on the matrix cores
-            tm, tiles, cap = routed.tile_plan(n * top, s.n_experts)
+            tm, tiles, cap = routed.tile_plan(n * top, s.n_experts, self.tile_order, s.intermediate, s.hidden)
             place = ws.get("expert_place", n * top, 1, torch.int32).view(-1)
             sorted_pair = ws.get(f"expert_sorted{tm}", cap, 1, torch.int32).view(-1)
             tile_expert = ws.get(f"expert_tiles{tm}", tiles, 1, torch.int32).view(-1)

@@ -484,3 +484,37 @@ def test_experts_and_their_weighted_sum(dtype, E, I, top, ff, hidden, n):
                                     routed.pack_expert_weights(d(wd)), act_rows, y3, tm, tiles, top, 1, tile_order=True)
                 real = (sorted_pair >= 0)
                 assert torch.equal(y3[real], y2[real]), "weights in tile order give other sums"
+
+
+@pytest.mark.parametrize("tm", [64, 128])
+@pytest.mark.parametrize("n,E,top,ff,hidden", [(1, 3, 2, 32, 32), (70, 2, 1, 96, 160), (129, 5, 3, 64, 288), (300, 1, 1, 320, 64), (520, 9, 2, 160, 128)])
+def test_routed_tiles_in_tile_order(n, E, top, ff, hidden, tm):
+    """Tiles that go through LDS: tiles with one row, full ones, more tiles than an XCD's share, columns that break a block of
+    columns, experts without a pair, one stage of columns.  The sums are those of the kernel without LDS, in the same order
+    (it takes rows in tiles of 64 at most, so rows are compared pair by pair)."""
+    from agave_amd.ops import routed
+    g = torch.Generator().manual_seed(n + tm)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * s[-1] ** -0.5).bfloat16().to(DEV)
+    x, wg, wu, wd = torch.randn(n, hidden, generator=g).bfloat16().to(DEV), rnd(E, ff, hidden), rnd(E, ff, hidden), rnd(E, hidden, ff)
+    # (the last expert gets no pair where there are several; one identity choice)
+    choice = torch.stack([torch.randperm(max(E - 1, top), generator=g)[:top] for _ in range(n)]).int()
+    choice[n // 2, 0] = E
+    choice = choice.view(-1).to(DEV)
+    rows = []
+    for rows_a_tile, packed in ((64, False), (tm, True)):
+        tiles = (n * top + rows_a_tile - 1) // rows_a_tile + E
+        place, sorted_pair, tile_expert = (torch.full((k,), -7, dtype=torch.int32, device=DEV) for k in (n * top, tiles * rows_a_tile, tiles))
+        routed.route_sort(choice, E, rows_a_tile, tiles, place, sorted_pair, tile_expert)
+        act_rows = torch.empty(tiles * rows_a_tile, ff, dtype=torch.bfloat16, device=DEV)
+        y = torch.full((tiles * rows_a_tile, hidden), float("nan"), device=DEV)
+        w = [routed.pack_expert_weights(v) if packed else v for v in (wg, wu, wd)]
+        routed.experts_mfma(x, sorted_pair, tile_expert, *w, act_rows, y, rows_a_tile, tiles, top, 1, tile_order=packed)
+        real = place >= 0
+        assert int(real.sum()) == n * top - 1
+        rows.append(y[place[real].long()])
+    assert torch.equal(rows[0], rows[1])
+    out = [torch.empty(n, hidden + 8, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    weight, shared = torch.rand(n * top, generator=g).to(DEV), torch.randn(n, hidden, generator=g).bfloat16().to(DEV)
+    for o, at in zip(out, (0, 1)):                  # rows aligned to four elements, and one element off
+        routed.combine(y, place, choice, weight, x, shared, o[:, at:at + hidden], top, E)
+    assert torch.equal(out[0][:, :hidden], out[1][:, 1:hidden + 1])
