@@ -14,6 +14,7 @@
 // here: projections arrive as float rows, state is float, angles are made in double.  T is the
 // element type of the cache pages and of the rows handed to the output product.
 #include "common_impl.h"
+#include "mfma.h"
 #include <math.h>
 
 #define CONV_MAX_TAPS 8
@@ -983,6 +984,280 @@ extern "C" int agave_gated_recurrence(int mode, const float* q, long ldq, const 
     }
     if (mode == REC_SSD) return launch_recurrence<REC_SSD>(A, n_seqs, stream);
     return mode == REC_DELTA ? launch_recurrence<REC_DELTA>(A, n_seqs, stream) : launch_recurrence<REC_FORGET>(A, n_seqs, stream);
+}
+
+// ------------------------------------------------------------------ the state-space form, 64 tokens at a time
+// Within a chunk of 64 tokens that starts from S0, with D_i the sum of the tokens' log decays up to i (inclusive),
+//     y_i = exp(D_i) S0^T C_i + sum_(j <= i) exp(D_i - D_j) d_j (C_i . B_j) v_j + skip v_i
+//     S   = exp(D_n) S0 + sum_j exp(D_n - D_j) d_j B_j v_j^T
+// so a chunk is three products for the matrix cores' 32-bit instructions and the chain from token to token becomes one from
+// chunk to chunk.  The sums D are held and subtracted in double: exp of a difference of rounded sums would lose what a
+// product of the tokens' decays keeps.
+//
+// First kernel: what does not depend on the state, for all chunks at once.  blockIdx.y < groups: C_i . B_j of a chunk (a wave per
+// 16 tokens i, tiles of 16 tokens j up to them) into cb[token][group][64]; the others: four heads each (a wave a head, a
+// lane a token): D and, per head and token, what the second kernel would otherwise make in every workgroup and wave:
+//     d;  exp(D_i);  d_j exp(D_n - D_j);  d_j exp(D_e - D_j) with e the last token of j's sixteen
+#define SSD_CHUNK 64
+#define SSD_SUMS 8              // running sums of a product: a sum in 32 bits loses more the longer it runs
+struct SsdScratch {
+    float* cb;                  // [tokens][groups][64]
+    double* cum;                // [heads][tokens]: D
+    float* made;                // [4][heads][tokens]: d, from the start, to the chunk's end, to the end of the sixteen
+    long n;                     // tokens
+    long heads_n;               // heads * tokens
+};
+__device__ __forceinline__ f32x4_t ssd_total(const f32x4_t (&a)[SSD_SUMS]) {
+    return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+__global__ __launch_bounds__(256) void ssd_prepare_kernel(RecurrenceArgs A, SsdScratch X) {
+    const int s = blockIdx.z, r0 = A.cu[s], r1 = A.cu[s + 1], t0 = r0 + blockIdx.x * SSD_CHUNK;
+    if (t0 >= r1) return;
+    const int n = min(SSD_CHUNK, r1 - t0);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if ((int)blockIdx.y < A.nkv) {
+        const int grp = blockIdx.y, r = lane & 15, g = lane >> 4;
+        if (16 * w >= n) return;
+        const float* c = A.q + (size_t)min(t0 + 16 * w + r, r1 - 1) * A.ldq + (size_t)grp * A.dk + 4 * g;
+        for (int jt = 0; jt <= w; ++jt) {
+            const float* b = A.k + (size_t)min(t0 + 16 * jt + r, r1 - 1) * A.ldk + (size_t)grp * A.dk + 4 * g;
+            f32x4_t acc[SSD_SUMS] = {};
+#pragma unroll 2
+            for (int k = 0; k < A.dk; k += 32)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const f32x4_t x = *reinterpret_cast<const f32x4_t*>(c + k + 16 * i), y = *reinterpret_cast<const f32x4_t*>(b + k + 16 * i);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[4 * i + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], acc[4 * i + e], 0, 0, 0);
+                }
+            const f32x4_t sum = ssd_total(acc);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = 16 * w + 4 * g + e;
+                if (i < n) X.cb[((size_t)(t0 + i) * A.nkv + grp) * SSD_CHUNK + 16 * jt + r] = sum[e];
+            }
+        }
+        return;
+    }
+    const int h = (blockIdx.y - A.nkv) * 4 + w;
+    if (h >= A.nh) return;
+    const float d = softplus_exact(A.dt[(size_t)(t0 + min(lane, n - 1)) * A.lddt + h] + A.dt_bias[h]);
+    // (exp(-1000) is 0 in 32 bits: a token that forgets everything stays finite here, so that differences of sums do)
+    double x = -(double)expf(A.a_log[h]) * (double)d;
+    x = x < -1000.0 ? -1000.0 : x;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+        const double y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    const double end = __shfl(x, n - 1), end16 = __shfl(x, min(lane | 15, n - 1));
+    if (lane < n) {
+        const long at = (long)h * X.n + t0 + lane;
+        X.cum[at] = x;
+        X.made[at] = d;
+        X.made[X.heads_n + at] = expf((float)x);
+        X.made[2 * X.heads_n + at] = d * expf((float)(end - x));
+        X.made[3 * X.heads_n + at] = d * expf((float)(end16 - x));
+    }
+}
+
+// Second kernel: a workgroup takes 16 value columns of one head through a sequence's chunks with eight waves, two on every SIMD,
+// so that one multiplies while the other waits.  Waves 0 to 3 make the read-outs of 16 tokens each from the state that the
+// chunk started with; waves 4 to 7 hold a quarter of the key channels of the state in registers, advance it and leave it in
+// LDS for the next chunk (two buffers, one barrier a chunk).  The next chunk's rows are asked for before this one's products.
+// Products take tokens and channels in whatever order suits the loads, as long as both operands agree: a lane's four
+// neighbours go into four instructions.
+// exp(D_i - D_j): within the sixteen of i from the difference itself, before that as exp(D_i - D_e) exp(D_e - D_j), neither
+// of which can overflow (an exponential per pair of tokens is no closer to 64 bits and 14 % slower).
+// A value that is not finite must not reach tokens before it, which a product with a zero weight would do: a chunk with one is
+// summed token by token.
+// Bound by the chain of chunks, some 3.5 us each.  Measured with the kernel before it, 64 heads of 64 x 128: 3,001 tokens 166 us
+// (token by token 600 us), 500 tokens 42 (110), 64 tokens 17 (21), 32 tokens 17 (15); six sequences of 40 tokens 38 (49).
+// Errors against 64 bits are those of the tokens one by one (1.1 to 1.2e-7 of the read-outs); with one running sum a product,
+// 2.2e-7.
+template <int DK>
+__global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScratch X) {
+    constexpr int KW = DK / 4, KF = KW / 16, CF = DK / 16;      // key channels of a state wave, of those a lane's neighbours; operands of a row of C
+    __shared__ __attribute__((aligned(16))) float Ss[2][16][DK + 4];
+    __shared__ __attribute__((aligned(16))) float Vt[2][16][SSD_CHUNK + 4];
+    __shared__ __attribute__((aligned(16))) double Dc[2][SSD_CHUNK];
+    __shared__ __attribute__((aligned(16))) float made[2][4][SSD_CHUNK];
+    __shared__ int odd[3];                                      // chunk ch % 3 holds a value that is not finite
+    const int h = blockIdx.y, s = blockIdx.z, col0 = blockIdx.x * 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3, r = lane & 15, g = lane >> 4;
+    const bool reads = wave < 4;
+    const int r0 = A.cu[s], r1 = A.cu[s + 1], grp = h / (A.nh / A.nkv);
+    const int n_chunks = (r1 - r0 + SSD_CHUNK - 1) / SSD_CHUNK;
+    if (n_chunks <= 0) return;
+    const int last = r1 - 1;
+    if (tid < 3) odd[tid] = 0;
+    lds_barrier();
+    if (reads) {
+        struct Rows {
+            f32x4_t v, c[CF], cb[4];
+            double cum;
+        };
+        const float skip = A.skip[h];
+        const int vt = tid >> 2, vc = (tid & 3) * 4;            // the four values of one token that a thread brings
+        auto ask = [&](Rows& x, int t0) {
+            x.v = *reinterpret_cast<const f32x4_t*>(A.v + (size_t)min(t0 + vt, last) * A.ldv + (size_t)h * A.dv + col0 + vc);
+            const int mine = min(t0 + 16 * w + r, last);
+#pragma unroll
+            for (int k = 0; k < CF; ++k) x.c[k] = *reinterpret_cast<const f32x4_t*>(A.q + (size_t)mine * A.ldq + (size_t)grp * DK + 16 * k + 4 * g);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                x.cb[j] = *reinterpret_cast<const f32x4_t*>(X.cb + ((size_t)mine * A.nkv + grp) * SSD_CHUNK + 16 * min(j, w) + 4 * g);
+            x.cum = X.cum[(long)h * X.n + min(t0 + lane, last)];
+        };
+        Rows cur, next;
+        ask(cur, r0);
+        for (int ch = 0; ch < n_chunks; ++ch) {
+            const int t0 = r0 + ch * SSD_CHUNK, n = min(SSD_CHUNK, r1 - t0), buf = ch & 1;
+            bool finite = true;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                Vt[buf][vc + e][vt] = cur.v[e];
+                finite = finite && fabsf(cur.v[e]) < INFINITY;
+            }
+            if (!finite && vt < n) odd[ch % 3] = 1;
+            if (tid == 0) odd[(ch + 1) % 3] = 0;                // (last read two chunks ago, written next behind the barrier below)
+            if (w == 0) Dc[buf][lane] = cur.cum;
+            lds_barrier();
+            if (ch + 1 < n_chunks) ask(next, t0 + SSD_CHUNK);
+            const bool by_token = odd[ch % 3] != 0;
+            // what the state says
+            f32x4_t acc[SSD_SUMS] = {};
+#pragma unroll
+            for (int k = 0; k < CF; ++k) {
+                const f32x4_t sv = *reinterpret_cast<const f32x4_t*>(&Ss[buf][r][16 * k + 4 * g]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    f32x4_t& sum = acc[(4 * k + e) % SSD_SUMS];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.c[k][e], sv[e], sum, 0, 0, 0);
+                }
+            }
+            f32x4_t y = ssd_total(acc) * *reinterpret_cast<const f32x4_t*>(&made[buf][1][16 * w + 4 * g]);
+            // the chunk's own tokens, up to each
+            const double here = Dc[buf][16 * w + r];
+            if (!by_token) {
+                f32x4_t own[4] = {};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (j > w) continue;
+                    const f32x4_t vf = *reinterpret_cast<const f32x4_t*>(&Vt[buf][r][16 * j + 4 * g]);      // tokens 16 j + 4 g + e, column r
+                    f32x4_t m;
+                    if (j < w) {
+                        m = *reinterpret_cast<const f32x4_t*>(&made[buf][3][16 * j + 4 * g]) * expf((float)(here - Dc[buf][16 * j + 15]));
+                    } else {
+                        const f32x4_t d = *reinterpret_cast<const f32x4_t*>(&made[buf][0][16 * j + 4 * g]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int t = 4 * g + e;
+                            m[e] = t <= r ? expf((float)(here - Dc[buf][16 * j + t])) * d[e] : 0.f;
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float x = 16 * j + 4 * g + e <= 16 * w + r ? cur.cb[j][e] * m[e] : 0.f;
+                        own[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, vf[e], own[e], 0, 0, 0);
+                    }
+                }
+                y += (own[0] + own[1]) + (own[2] + own[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 16 * w + 4 * g + e;
+                    const float* row = X.cb + ((size_t)min(t0 + i, last) * A.nkv + grp) * SSD_CHUNK;
+                    for (int j = 0; j <= i && j < n; ++j)
+                        y[e] = fmaf(row[j] * (expf((float)(Dc[buf][i] - Dc[buf][j])) * made[buf][0][j]), Vt[buf][r][j], y[e]);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = 16 * w + 4 * g + e;
+                if (i < n) A.o[(size_t)(t0 + i) * A.ldo + (size_t)h * A.dv + col0 + r] = fmaf(skip, Vt[buf][r][i], y[e]);
+            }
+            cur = next;
+        }
+    } else {
+        // the state: st[f][e] is channel w KW + KF (4 g + e) + f, column r
+        float* S_g = A.state + (((size_t)A.slots[s] * A.nh + h) * A.dv + col0 + r) * DK + w * KW + KF * 4 * g;
+        f32x4_t st[KF];
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st[f][e] = S_g[KF * e + f];
+        struct Rows {
+            float b[16][KF], made;
+        };
+        auto ask = [&](Rows& x, int t0) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float* b = A.k + (size_t)min(t0 + 16 * j + 4 * g + e, last) * A.ldk + (size_t)grp * DK + w * KW + KF * r;
+#pragma unroll
+                    for (int f = 0; f < KF; ++f) x.b[4 * j + e][f] = b[f];
+                }
+            x.made = X.made[w * X.heads_n + (long)h * X.n + min(t0 + lane, last)];
+        };
+        Rows cur, next;
+        ask(cur, r0);
+        for (int ch = 0; ch < n_chunks; ++ch) {
+            const int t0 = r0 + ch * SSD_CHUNK, n = min(SSD_CHUNK, r1 - t0), buf = ch & 1;
+            // (rows behind the sequence's end repeat its last one and count nothing)
+            made[buf][w][lane] = lane < n ? cur.made : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int f = 0; f < KF; ++f) Ss[buf][r][w * KW + KF * (4 * g + e) + f] = st[f][e];
+            lds_barrier();
+            if (ch + 1 < n_chunks) ask(next, t0 + SSD_CHUNK);
+            const float left = made[buf][1][n - 1];
+#pragma unroll
+            for (int f = 0; f < KF; ++f) st[f] *= left;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4_t vf = *reinterpret_cast<const f32x4_t*>(&Vt[buf][r][16 * j + 4 * g]) *
+                                   *reinterpret_cast<const f32x4_t*>(&made[buf][2][16 * j + 4 * g]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int f = 0; f < KF; ++f) st[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[4 * j + e][f], vf[e], st[f], 0, 0, 0);
+            }
+            cur = next;
+        }
+#pragma unroll
+        for (int f = 0; f < KF; ++f)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S_g[KF * e + f] = st[f][e];
+    }
+}
+
+// The state-space form in chunks, for a step in which some sequence brings many tokens (max_new: the longest).  Takes key
+// channels of 64 or 128 and values in blocks of 16, rows aligned to 16 bytes; agave_gated_recurrence takes the others.
+// cb: float [n_tokens][nkv][64]; cum: double [nh][n_tokens]; made: float [4][nh][n_tokens].
+extern "C" int agave_ssd_chunks(const float* q, long ldq, const float* k, long ldk, const float* v, long ldv, const float* dt, long lddt,
+                                const float* a_log, const float* dt_bias, const float* skip, float* o, long ldo, float* state,
+                                const int* cu, const int* slots, int n_seqs, int nh, int nkv, int dk, int dv, int max_new, long n_tokens,
+                                float* cb, double* cum, float* made, hipStream_t stream) {
+    AGAVE_CHECK(n_seqs >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0 && max_new >= 0 && n_tokens >= 0, "ssd_chunks: bad sizes B=%d nh=%d nkv=%d", n_seqs, nh, nkv);
+    AGAVE_CHECK((dk == 64 || dk == 128) && dv > 0 && dv % 16 == 0, "ssd_chunks: %d key channels and %d values a head (64 or 128, and a multiple of 16)", dk, dv);
+    AGAVE_CHECK(q && k && v && dt && a_log && dt_bias && skip && o && state && cu && slots && cb && cum && made, "ssd_chunks: null buffer");
+    AGAVE_CHECK(ldq >= (long)nkv * dk && ldk >= (long)nkv * dk && ldv >= (long)nh * dv && lddt >= nh && ldo >= (long)nh * dv, "ssd_chunks: a row stride is too small");
+    AGAVE_CHECK(ldq % 4 == 0 && ldk % 4 == 0 && ldv % 4 == 0 && (uintptr_t)q % 16 == 0 && (uintptr_t)k % 16 == 0 && (uintptr_t)v % 16 == 0 &&
+                (uintptr_t)cb % 16 == 0 && (uintptr_t)cum % 8 == 0, "ssd_chunks: rows must be aligned to 16 bytes");
+    AGAVE_CHECK(n_seqs < 65536 && nh < 65536 && nkv + (nh + 3) / 4 < 65536, "ssd_chunks: too many sequences or heads");
+    if (n_seqs == 0 || max_new == 0) return 0;
+    RecurrenceArgs A{q, ldq, k, ldk, v, ldv, dt, lddt, nullptr, 0, a_log, dt_bias, skip, nullptr, nullptr, o, ldo, state, cu, slots, nh, nkv, dk, dv, 0.f};
+    const dim3 first((max_new + SSD_CHUNK - 1) / SSD_CHUNK, nkv + (nh + 3) / 4, n_seqs), second(dv / 16, nh, n_seqs);
+    const SsdScratch X{cb, cum, made, n_tokens, (long)nh * n_tokens};
+    ssd_prepare_kernel<<<first, 256, 0, stream>>>(A, X);
+    AGAVE_LAUNCH_CHECK("ssd_prepare");
+    if (dk == 64) ssd_chunk_kernel<64><<<second, 512, 0, stream>>>(A, X);
+    else ssd_chunk_kernel<128><<<second, 512, 0, stream>>>(A, X);
+    AGAVE_LAUNCH_CHECK("ssd_chunks");
+    return 0;
 }
 
 // ------------------------------------------------------------------ read-out norm with a gate

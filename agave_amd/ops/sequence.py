@@ -23,6 +23,7 @@ kernels.register_signatures(LIBRARY, {
                                   _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "agave_talk_attention": [_I, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I,
                              _F, _I, _F, _P, _I, _P],
+    "agave_ssd_chunks": [_P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _P, _P, _P, _P],
     "agave_gated_recurrence": [_I, _P, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _L, _P, _P, _P,
                                _I, _I, _I, _I, _I, _F, _I, _P],
     "agave_gated_group_norm": [_I, _P, _L, _P, _L, _P, _P, _L, _I, _I, _I, _F, _P],
@@ -151,6 +152,29 @@ def talk_attention(q: torch.Tensor, gate: Optional[torch.Tensor], out: torch.Ten
                  n, n_heads, n_kv, dk, dv, float(scale), int(chunk or 0), float(out_scale), ptr(parts), tiles, stream())
 
 
+SSD_CHUNK = 64
+# A sequence that brings this many tokens: chunks of 64 from here on, token by token below (64 heads of 64 x 128: 32 tokens
+# take 15 us token by token and 17 in chunks, 48 tokens 17 and 16, 64 tokens 21 and 17).
+SSD_CHUNKS_FROM = 48
+
+
+def ssd_chunks_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step, dk: int, dv: int) -> bool:
+    """Whether the state-space form runs in chunks of tokens: a sequence of the step is long enough and the chunk kernel
+    takes the sizes and the rows' alignment."""
+    return (step.max_new >= SSD_CHUNKS_FROM and getattr(step, "workspace", None) is not None and dk in (64, 128) and dv % 16 == 0
+            and all(t.data_ptr() % 16 == 0 and t.stride(0) % 4 == 0 for t in (q, k, v)))
+
+
+def _ssd_chunks(q, ldq, k, ldk, v, ldv, dt_in, lddt, a_log, dt_bias, skip, out, ldo, state, step, n_heads, n_kv, dk, dv) -> None:
+    n, ws = step.n_tokens, step.workspace
+    cb = ws.get("ssd_cb", n, n_kv * SSD_CHUNK, torch.float32)
+    cum = ws.get("ssd_cum", n, n_heads, torch.float64)
+    made = ws.get("ssd_made", 4 * n, n_heads, torch.float32)
+    library.call(_lib(), "agave_ssd_chunks", ptr(q), ldq, ptr(k), ldk, ptr(v), ldv, ptr(dt_in), lddt, ptr(a_log), ptr(dt_bias), ptr(skip),
+                 ptr(out), ldo, ptr(state), ptr(step.cu_dev), ptr(step.slots_dev), step.n_seqs, n_heads, n_kv, dk, dv, step.max_new, n,
+                 ptr(cb), ptr(cum), ptr(made), stream())
+
+
 def gated_recurrence(mode: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tensor,
                      state: torch.Tensor, step, n_heads: int, n_kv: int, dk: int, dv: int, *,
                      dt_in: Optional[torch.Tensor] = None, beta: Optional[torch.Tensor] = None,
@@ -190,6 +214,9 @@ def gated_recurrence(mode: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
         _f32vec(skip, "skip", n_heads)
         if a_log is None or dt_bias is None or skip is None:
             raise ValueError("gated_recurrence: the state-space form needs a_log, dt_bias and skip")
+        if ssd_chunks_ok(q, k, v, step, dk, dv):
+            _ssd_chunks(q, ldq, k, ldk, v, ldv, dt_in, lddt, a_log, dt_bias, skip, out, ldo, state, step, n_heads, n_kv, dk, dv)
+            return
     elif mode == FORGET:
         _f32vec(lower, "lower", n_heads * dk)
         _f32vec(f_bias, "f_bias", n_heads * dk)

@@ -167,6 +167,58 @@ def test_state_space_whole_pieces_and_tokens(H, G, N, dv):
         assert torch.allclose(S_got, S_ref, atol=3e-5, rtol=1e-4), plan[:2]
 
 
+def chunked(T, cuts_, H, G, N, dv, seed=3, change=None):
+    """One sequence through the chunked kernels in the given pieces: (read-outs, last state, the 64-bit ones)."""
+    from agave_amd.cache import StateNeed
+    from agave_amd.ops import sequence as S
+    from agave_amd.parts import Workspace
+    cache, planner = planner_for(state={0: StateNeed((H, dv, N))})
+    planner.workspace = Workspace(torch.device(DEV))
+    cache.alloc_slot()
+    slot = cache.alloc_slot()
+    t, vec = state_space_inputs(H, G, N, dv, T, seed)
+    if change is not None:
+        change(t, vec)
+    out = torch.zeros(T, H * dv, device=DEV)
+    for lo, hi in cuts_:
+        step = feed(cache, planner, [slot], [hi - lo])
+        d = {n: x[lo:hi].to(DEV).contiguous() for n, x in t.items()}
+        assert S.ssd_chunks_ok(d["C"], d["B"], d["xs"], step, N, dv) == (hi - lo >= S.SSD_CHUNKS_FROM)
+        S.gated_recurrence(S.SSD, d["C"], d["B"], d["xs"], out[lo:hi], cache.state[0], step, H, G, N, dv, dt_in=d["dt"],
+                           **{n: x.to(DEV) for n, x in vec.items()})
+        planner.commit(step)
+    return out.cpu().to(F64), cache.state[0][slot].cpu().to(F64).transpose(1, 2), plain_state_space(t, vec, H, G, N, dv)
+
+
+@pytest.mark.parametrize("H, G, N, dv", [(4, 2, 64, 16), (3, 1, 128, 48), (1, 1, 64, 32), (2, 2, 128, 16)])
+@pytest.mark.parametrize("T", [64, 65, 127, 209])
+def test_state_space_in_chunks(H, G, N, dv, T):
+    """Whole and broken chunks, a state that goes on from a step before, tokens behind it one by one."""
+    for plan in ([(0, T)], [(0, T - 13), (T - 13, T)], [(0, 3), (3, T - 1), (T - 1, T)]):
+        got, S_got, (ref, S_ref) = chunked(T, plan, H, G, N, dv)
+        assert torch.allclose(got, ref.reshape(T, -1), atol=3e-5, rtol=1e-4), plan
+        assert torch.allclose(S_got, S_ref, atol=3e-5, rtol=1e-4), plan
+
+
+def test_state_space_in_chunks_at_its_ends():
+    """Tokens that forget everything (also with an infinite rate), step sizes of almost nothing, and a value that is not finite:
+    it reaches its own column from its token on, and nothing before it."""
+    def forget(t, vec):
+        vec["a_log"][0], vec["a_log"][1] = 30.0, 100.0
+        t["dt"][::5] = 40.0
+        t["dt"][2::5] = -60.0
+    got, S_got, (ref, S_ref) = chunked(150, [(0, 150)], 3, 1, 64, 16, change=forget)
+    assert torch.allclose(got, ref.reshape(150, -1), atol=1e-4, rtol=1e-4) and torch.allclose(S_got, S_ref, atol=1e-4, rtol=1e-4)
+    for odd in (float("nan"), float("inf")):
+        def spoil(t, vec):
+            t["xs"][70, 5] = odd
+        got, _, (ref, _) = chunked(150, [(0, 150)], 3, 1, 128, 16, change=spoil)
+        bad = ~torch.isfinite(got)
+        assert bool(bad[70:, 5].all()) and int(bad.sum()) == 80
+        ref = ref.reshape(150, -1)
+        assert torch.allclose(got[~bad], ref[~bad], atol=3e-5, rtol=1e-4)
+
+
 def test_state_space_step_sizes_without_a_clamp_and_a_write_far_back():
     """Step sizes from almost nothing to dozens (softplus of -20 to 40, neither clamped); and with a decay rate of
     almost nothing what token 3 wrote is read 600 tokens later among small writes, while a fast rate forgets it."""
