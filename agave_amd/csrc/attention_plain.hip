@@ -1,7 +1,7 @@
-// Plain attention over the paged cache for gfx950, for any even head size and either
-// element type: one workgroup per (token, query head), scores and probabilities in 32-bit,
-// exact expf, no skipping of small probabilities.  It is the true 32-bit path and the
-// fallback for head sizes the MFMA kernels refuse.
+// Plain attention over the paged cache for gfx950, for any head size up to 512 and either
+// element type: scores, probabilities and sums in 32-bit, exact expf, no skipping of small
+// probabilities.  It is the true 32-bit path and the fallback for head sizes the bfloat16 kernels
+// refuse.
 //
 // Reference: src/backend/kernels/cpu/sdpa.zig:34-88 (scores * scale, softmax, weighted sum
 // of V), window bounds as src/ops/attention.zig:92-93 with the callers' convention of
@@ -10,118 +10,307 @@
 // Cache pages: K [page][kv head][64 rows][hd]; V transposed [page][kv head][hd][64 rows].
 // Position j of sequence b lies in page table[b][j/64 - base[b]], row j % 64.
 #include "common_impl.h"
+#include "fours.h"
 #include <math.h>
 
-#define CHUNK 256            // keys per pass = 4 pages
-#define ACC_MAX 2            // head_dim <= 512
+#define ROWS 16              // query rows a workgroup: tokens next to each other times the heads of a key head
+#define COMPUTE_UNITS 256
+#define MOST_SPLITS 16
 
-template <typename T>
+// The largest / the sum over a row of 16 lanes, in each of them.
+__device__ __forceinline__ float lanes16_max(float v) {
+    v = fmaxf(v, dpp_get<0xB1, 0xF>(v, v));
+    v = fmaxf(v, dpp_get<0x4E, 0xF>(v, v));
+    v = fmaxf(v, dpp_get<0x141, 0xF>(v, v));
+    return fmaxf(v, dpp_get<0x140, 0xF>(v, v));
+}
+__device__ __forceinline__ float lanes16_sum(float v) {
+    v += dpp_get<0xB1, 0xF>(0.f, v);
+    v += dpp_get<0x4E, 0xF>(0.f, v);
+    v += dpp_get<0x141, 0xF>(0.f, v);
+    return v + dpp_get<0x140, 0xF>(0.f, v);
+}
+
+// A workgroup of 4 waves takes 16 query rows (`run` neighbouring tokens of one key head's query heads) through the pages they
+// see, a page of 64 keys at a time: every wave the scores of 16 keys, then, with the page's probabilities in LDS, the sums over
+// the page for a quarter of the value elements.  Both are products for v_mfma_f32_16x16x4_f32, whose operands K and V come
+// straight from memory in 16-byte pieces (it takes the summed index in any order as long as both operands agree).  Tokens of
+// several sequences in one workgroup (any tok_seq is taken) go one sequence after another.
+// gridDim.y workgroups share a row's pages and leave (sum, maximum, unnormalised result) for attn_plain_merge_kernel: with a
+// token per sequence there are few rows and the pages one after another bound the time.
+// NT: tiles of 64 value elements (16 a wave).  A probability of 0 must not meet a value that is not finite (a key behind a
+// token's position may hold anything): such pages are summed element by element.
+// Bound by the 32-bit products (half of them for a token of 4 rows' padding) and, with few tokens, by the loads' way from memory.
+// Measured, 16 heads on 4 key heads of 128 in 32 bits: prompts of 97, 259 and 421 tokens 63 us (a workgroup per token and head, a
+// key a thread: 943 us), 2,000 tokens 0.45 ms (16.8 ms); a token each behind as many keys 15 us (59 us), behind 4,000 keys
+// 33 us (562 us).  Errors against 64 bits are half as large (2.0 to 2.8e-7 after 4.2 to 5.5e-7).
+template <typename T, int NT, bool VEC>
 __global__ __launch_bounds__(256) void attn_plain_kernel(
     const T* __restrict__ q, long ldq, T* __restrict__ out, long ldo, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ table, int width, const int* __restrict__ base,
-    int n_pages, const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, int nh, int nkv, int hd,
-    float scale, int window) {
-    __shared__ float qs[512];
-    __shared__ float sc[CHUNK];
-    __shared__ long page_of[CHUNK / AGAVE_PAGE];
-    __shared__ float red[16];
+    int n_pages, const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, int N, int nh, int nkv, int hd,
+    float scale, int window, int run, float* __restrict__ part_o, float* __restrict__ part_ml) {
+    constexpr int HDP = NT * 64;
+    constexpr bool V_AHEAD = NT <= 4;                        // a page's values are asked for before its scores are made
+    __shared__ __attribute__((aligned(16))) float Qs[ROWS][HDP + 4];
+    __shared__ __attribute__((aligned(16))) float P[ROWS][AGAVE_PAGE + 4];
+    __shared__ __attribute__((aligned(16))) float wmax[4][ROWS], wsum[4][ROWS];
+    __shared__ __attribute__((aligned(16))) int row_pos[ROWS], row_lo[ROWS], row_seq[ROWS];
 
-    const int tid = threadIdx.x;
-    const int t = blockIdx.x / nh, h = blockIdx.x % nh;
-    const int kvh = h / (nh / nkv);
-    const int b = tok_seq[t];
-    const int p = tok_pos[t];
-    const int lo = window > 0 ? (p - window + 1 > 0 ? p - window + 1 : 0) : 0;
-    const int pbase = base[b];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const int G = nh / nkv, chunks = (G + ROWS - 1) / ROWS;
+    const int chunk = blockIdx.x % chunks, kvh = blockIdx.x / chunks % nkv, t0 = blockIdx.x / chunks / nkv * run;
+    const int heads = min(G - chunk * ROWS, ROWS), head0 = kvh * G + chunk * ROWS;
+    const int rows = min(min(run, N - t0) * heads, ROWS);
+    const int split = blockIdx.y, splits = gridDim.y;
 
-    for (int d = tid; d < hd; d += blockDim.x) qs[d] = ld(q + (size_t)t * ldq + (size_t)h * hd + d);
+    if (tid < ROWS) {
+        const int t = t0 + tid / heads;
+        const bool real = tid < rows;
+        const int p = real ? tok_pos[t] : -1;
+        row_pos[tid] = p;
+        row_lo[tid] = real && window > 0 && p - window + 1 > 0 ? p - window + 1 : 0;
+        row_seq[tid] = real ? tok_seq[t] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {                           // four elements a thread and turn
+        const int row = (tid + 256 * i) / (HDP / 4), d = (tid + 256 * i) % (HDP / 4) * 4, real = min(row, rows - 1);
+        const f32x4_t x = ld4<VEC>(q + (size_t)(t0 + real / heads) * ldq + (size_t)(head0 + real % heads) * hd, d, hd);
+        *reinterpret_cast<f32x4_t*>(&Qs[row][d]) = row < rows ? x : f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
     __syncthreads();
 
-    float m = -INFINITY, l = 0.f;
-    float acc[ACC_MAX] = {0.f, 0.f};
-
-    for (int c0 = (lo / AGAVE_PAGE) * AGAVE_PAGE; c0 <= p; c0 += CHUNK) {
-        // pages of this chunk
-        if (tid < CHUNK / AGAVE_PAGE) {
-            const int first = c0 + tid * AGAVE_PAGE;
-            long pg = -1;
-            const int col = first / AGAVE_PAGE - pbase;
-            if (first <= p && col >= 0 && col < width) pg = table[(size_t)b * width + col];
-            if (pg >= n_pages) pg = -1;
-            page_of[tid] = pg;
-        }
-        __syncthreads();
-        // scores: one key per thread
-        const int j = c0 + tid;
-        const long pg = page_of[tid / AGAVE_PAGE];
-        const bool valid = j >= lo && j <= p && pg >= 0;
-        float s = -INFINITY;
-        if (valid) {
-            const T* kr = k_pages + (((size_t)pg * nkv + kvh) * AGAVE_PAGE + (j % AGAVE_PAGE)) * hd;
-            float dot = 0.f;
-            for (int d = 0; d < hd; ++d) dot = fmaf(qs[d], ld(kr + d), dot);
-            s = dot * scale;
-        }
-        const float cmax = block_max(s, red);
-        const float m_new = fmaxf(m, cmax);
-        // m_new is finite whenever any key of this or an earlier chunk was valid
-        const float alpha = (m == -INFINITY) ? 0.f : expf(m - m_new);
-        const float pr = valid ? expf(s - m_new) : 0.f;
-        sc[tid] = pr;
-        const float csum = block_sum(pr, red);      // has barriers: sc[] is visible afterwards
-        l = l * alpha + csum;
-        m = m_new;
-        // weighted sum of V: one output element per thread
+    // rows 4 g + e; value element (4 nt + w) 16 + r
+    float m[4], l[4];
+    f32x4_t o[NT];
 #pragma unroll
-        for (int a = 0; a < ACC_MAX; ++a) {
-            const int d = tid + a * 256;
-            if (d < hd) {
-                float sum = 0.f;
-                for (int pi = 0; pi < CHUNK / AGAVE_PAGE; ++pi) {
-                    const long vp = page_of[pi];
-                    if (vp < 0) continue;
-                    const T* vr = v_pages + (((size_t)vp * nkv + kvh) * hd + d) * AGAVE_PAGE;
-                    for (int r = 0; r < AGAVE_PAGE; ++r) {
-                        const float w = sc[pi * AGAVE_PAGE + r];
-                        if (w != 0.f) sum = fmaf(w, ld(vr + r), sum);   // rows outside the range hold w == 0 and may hold anything
+    for (int e = 0; e < 4; ++e) {
+        m[e] = -INFINITY;
+        l[e] = 0.f;
+    }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) o[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int4 pos4 = *reinterpret_cast<const int4*>(&row_pos[4 * g]), lo4 = *reinterpret_cast<const int4*>(&row_lo[4 * g]);
+    const int pos[4] = {pos4.x, pos4.y, pos4.z, pos4.w}, low[4] = {lo4.x, lo4.y, lo4.z, lo4.w};
+
+    for (int s0 = 0, s1; s0 < rows; s0 = s1) {               // a run of rows of one sequence
+        const int seq = row_seq[s0];
+        int lo = row_lo[s0], hi = row_pos[s0];
+        for (s1 = s0 + 1; s1 < rows && row_seq[s1] == seq; ++s1) {
+            lo = min(lo, row_lo[s1]);
+            hi = max(hi, row_pos[s1]);
+        }
+        if (hi < 0) continue;
+        const int first = lo / AGAVE_PAGE, count = hi / AGAVE_PAGE - first + 1, share = (count + splits - 1) / splits;
+        const int from = first + split * share, to = min(from + share, first + count), pbase = base[seq];
+        for (int page = from; page < to; ++page) {
+            const int col = page - pbase;
+            const long pg = col >= 0 && col < width ? table[(size_t)seq * width + col] : -1;
+            if (pg < 0 || pg >= n_pages) continue;
+            const T* kr = k_pages + ((size_t)(pg * nkv + kvh) * AGAVE_PAGE + 16 * w + r) * hd;
+            const T* vr = v_pages + (size_t)(pg * nkv + kvh) * hd * AGAVE_PAGE;
+            const int key0 = page * AGAVE_PAGE;
+            f32x4_t vv[V_AHEAD ? NT : 1][4];
+            auto values = [&](f32x4_t (&v)[4], int nt) {
+                const T* row = vr + (size_t)min((4 * nt + w) * 16 + r, hd - 1) * AGAVE_PAGE;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = ld4<true>(row, 16 * j + 4 * g, AGAVE_PAGE);
+            };
+            if constexpr (V_AHEAD)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) values(vv[nt], nt);
+            // scores of keys 16 w + r
+            f32x4_t sum[4] = {};
+#pragma unroll 8
+            for (int d = 0; d < hd; d += 16) {
+                const f32x4_t kv = ld4<VEC>(kr, d + 4 * g, hd), qv = *reinterpret_cast<const f32x4_t*>(&Qs[r][d + 4 * g]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[e], kv[e], sum[e], 0, 0, 0);
+            }
+            f32x4_t s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            const int key = key0 + 16 * w + r;
+            bool seen[4];
+            f32x4_t most;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                seen[e] = 4 * g + e >= s0 && 4 * g + e < s1 && key >= low[e] && key <= pos[e];
+                s[e] = seen[e] ? s[e] * scale : -INFINITY;
+                most[e] = lanes16_max(s[e]);
+            }
+            if (r == 0) *reinterpret_cast<f32x4_t*>(&wmax[w][4 * g]) = most;
+            __syncthreads();
+            f32x4_t total;
+            float alpha[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = 4 * g + e;
+                const float m_new = fmaxf(m[e], fmaxf(fmaxf(wmax[0][row], wmax[1][row]), fmaxf(wmax[2][row], wmax[3][row])));
+                // m_new is finite whenever any key of this or an earlier page was seen
+                alpha[e] = m[e] == -INFINITY ? 0.f : expf(m[e] - m_new);
+                const float pr = seen[e] ? expf(s[e] - m_new) : 0.f;
+                m[e] = m_new;
+                P[row][16 * w + r] = pr;
+                total[e] = lanes16_sum(pr);
+            }
+            if (r == 0) *reinterpret_cast<f32x4_t*>(&wsum[w][4 * g]) = total;
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = 4 * g + e;
+                l[e] = l[e] * alpha[e] + ((wsum[0][row] + wsum[1][row]) + (wsum[2][row] + wsum[3][row]));
+            }
+            f32x4_t pf[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) pf[j] = *reinterpret_cast<const f32x4_t*>(&P[r][16 * j + 4 * g]);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                if ((4 * nt + w) * 16 >= hd) continue;
+                f32x4_t late[4];
+                if constexpr (!V_AHEAD) values(late, nt);
+                f32x4_t (&v)[4] = V_AHEAD ? vv[V_AHEAD ? nt : 0] : late;
+                f32x4_t add = {};
+                bool finite = true;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int at = key0 + 16 * j + 4 * g + e;
+                        if (at < lo || at > hi) v[j][e] = 0.f;         // (no row sees it: it may hold anything)
+                        finite = finite && fabsf(v[j][e]) < INFINITY;
+                    }
+                if (__all(finite)) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) add = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[j][e], v[j][e], add, 0, 0, 0);
+                } else {
+                    const T* row = vr + (size_t)min((4 * nt + w) * 16 + r, hd - 1) * AGAVE_PAGE;
+                    for (int k = 0; k < AGAVE_PAGE; ++k) {
+                        const float x = ld(row + k);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float pr = P[4 * g + e][k];
+                            if (pr != 0.f) add[e] = fmaf(pr, x, add[e]);
+                        }
                     }
                 }
-                acc[a] = acc[a] * alpha + sum;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[nt][e] = o[nt][e] * alpha[e] + add[e];
             }
         }
-        __syncthreads();     // sc[] and page_of[] are rewritten by the next chunk
     }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
 #pragma unroll
-    for (int a = 0; a < ACC_MAX; ++a) {
-        const int d = tid + a * 256;
-        if (d < hd) st(out + (size_t)t * ldo + (size_t)h * hd + d, acc[a] * inv);
+    for (int e = 0; e < 4; ++e) {
+        const int row = 4 * g + e;
+        if (row >= rows) continue;
+        const size_t t = t0 + row / heads;
+        const int h = head0 + row % heads;
+        const float inv = l[e] > 0.f ? 1.0f / l[e] : 0.f;
+        const size_t part = (t * nh + h) * splits + split;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int d = (4 * nt + w) * 16 + r;
+            if (d >= hd) continue;
+            if (splits > 1) part_o[part * hd + d] = o[nt][e];
+            else st(out + t * ldo + (size_t)h * hd + d, o[nt][e] * inv);
+        }
+        if (splits > 1 && w == 0 && r == 0) {
+            part_ml[2 * part] = m[e];
+            part_ml[2 * part + 1] = l[e];
+        }
     }
 }
 
+// The results that a row's workgroups left: a workgroup per (token, head).
+template <typename T>
+__global__ __launch_bounds__(128) void attn_plain_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                               T* __restrict__ out, long ldo, int nh, int hd, int splits) {
+    const size_t row = blockIdx.x;
+    const float* ml = part_ml + 2 * row * splits;
+    float m = -INFINITY, l = 0.f, f[MOST_SPLITS];
+    for (int s = 0; s < splits; ++s) m = fmaxf(m, ml[2 * s]);
+#pragma unroll
+    for (int s = 0; s < MOST_SPLITS; ++s) {
+        f[s] = s < splits && ml[2 * s] != -INFINITY ? expf(ml[2 * s] - m) : 0.f;
+        if (s < splits) l = fmaf(ml[2 * s + 1], f[s], l);
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    for (int d = threadIdx.x; d < hd; d += 128) {
+        float sum = 0.f;
+#pragma unroll
+        for (int s = 0; s < MOST_SPLITS; ++s)
+            if (s < splits && f[s] != 0.f) sum = fmaf(part_o[(row * splits + s) * hd + d], f[s], sum);
+        st(out + (row / nh) * ldo + (row % nh) * hd + d, sum * inv);
+    }
+}
+
+template <typename T, int NT>
+static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages, const T* v_pages, const int* table, int width,
+                        const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
+                        int window, int run, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+    const int chunks = (nh / nkv + ROWS - 1) / ROWS;
+    const dim3 grid((N + run - 1) / run * nkv * chunks, splits);
+    const bool vec = hd % 4 == 0 && ldq % 4 == 0 && (uintptr_t)k_pages % (4 * sizeof(T)) == 0 && (uintptr_t)q % (4 * sizeof(T)) == 0;
+    if (vec)
+        attn_plain_kernel<T, NT, true><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq,
+                                                                 tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml);
+    else
+        attn_plain_kernel<T, NT, false><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq,
+                                                                  tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml);
+    if (splits > 1) attn_plain_merge_kernel<T><<<N * nh, 128, 0, stream>>>(part_o, part_ml, out, ldo, nh, hd, splits);
+}
+
+template <typename T>
+static void launch_type(const void* q, long ldq, void* out, long ldo, const void* k_pages, const void* v_pages, const int* table, int width,
+                        const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
+                        int window, int run, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+#define ROWS_GO(NT_) launch_rows<T, NT_>((const T*)q, ldq, (T*)out, ldo, (const T*)k_pages, (const T*)v_pages, table, width, base, n_pages, \
+                                         tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, splits, part_o, part_ml, stream)
+    if (hd <= 64) ROWS_GO(1);
+    else if (hd <= 128) ROWS_GO(2);
+    else if (hd <= 256) ROWS_GO(4);
+    else ROWS_GO(8);
+#undef ROWS_GO
+}
+
+// How many workgroups share a row's pages when every sequence brings one token and spans at most `span` pages: a page each at
+// least, and no more workgroups in all than fill the compute units once.
+extern "C" int agave_attn_plain_splits(int N, int nh, int nkv, int span) {
+    if (N <= 0 || nh <= 0 || nkv <= 0 || nh % nkv != 0) return 1;
+    const long wgs = (long)N * nkv * ((nh / nkv + ROWS - 1) / ROWS);
+    long z = COMPUTE_UNITS / wgs;
+    if (z > span) z = span;
+    if (z > MOST_SPLITS) z = MOST_SPLITS;
+    return z < 1 ? 1 : (int)z;
+}
+
+// one_token_each: neighbouring tokens are of different sequences (a decode step), so a workgroup takes one.  splits > 1: part_o
+// [N][nh][splits][hd] and part_ml [N][nh][splits][2] receive what a row's workgroups leave.
 extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, long ldo, const void* k_pages,
                                 const void* v_pages, const int* table, int width, const int* base, int n_pages,
                                 const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                                int window, hipStream_t stream) {
+                                int window, int one_token_each, int splits, float* part_o, float* part_ml, hipStream_t stream) {
     AGAVE_CHECK(N >= 0 && nh > 0 && nkv > 0 && hd > 0, "attn_plain: bad sizes N=%d nh=%d nkv=%d hd=%d", N, nh, nkv, hd);
     AGAVE_CHECK(nh % nkv == 0, "attn_plain: %d query heads are not a multiple of %d kv heads", nh, nkv);
-    AGAVE_CHECK(hd <= 256 * ACC_MAX, "attn_plain: head_dim %d exceeds the supported maximum %d", hd, 256 * ACC_MAX);
+    AGAVE_CHECK(hd <= 512, "attn_plain: head_dim %d exceeds the supported maximum %d", hd, 512);
     AGAVE_CHECK(ldq >= (long)nh * hd && ldo >= (long)nh * hd, "attn_plain: a row stride is below nh*hd");
     AGAVE_CHECK(window >= 0, "attn_plain: negative window");
     AGAVE_CHECK(q && out && k_pages && v_pages && table && base && tok_seq && tok_pos && width > 0 && n_pages > 0,
                 "attn_plain: null buffer or empty table");
+    AGAVE_CHECK((uintptr_t)v_pages % 16 == 0, "attn_plain: value pages must be aligned to 16 bytes");
     AGAVE_CHECK((long)N * nh < 2147483647L, "attn_plain: too many (token, head) pairs");
+    AGAVE_CHECK(splits >= 1 && splits <= MOST_SPLITS && (splits == 1 || (part_o && part_ml)), "attn_plain: %d splits (1 to %d, with buffers for what they leave)",
+                splits, MOST_SPLITS);
+    AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "attn_plain: unknown dtype %d", dtype);
     if (N == 0) return 0;
+    // neighbouring tokens share a page's keys where there are enough of them to fill the compute units without
+    const int G = nh / nkv, run = one_token_each || G >= ROWS || (long)N * nkv <= COMPUTE_UNITS ? 1 : ROWS / G;
     if (dtype == AGAVE_F32)
-        attn_plain_kernel<float><<<N * nh, 256, 0, stream>>>((const float*)q, ldq, (float*)out, ldo, (const float*)k_pages,
-                                                             (const float*)v_pages, table, width, base, n_pages, tok_seq,
-                                                             tok_pos, nh, nkv, hd, scale, window);
-    else if (dtype == AGAVE_BF16)
-        attn_plain_kernel<bf16><<<N * nh, 256, 0, stream>>>((const bf16*)q, ldq, (bf16*)out, ldo, (const bf16*)k_pages,
-                                                            (const bf16*)v_pages, table, width, base, n_pages, tok_seq,
-                                                            tok_pos, nh, nkv, hd, scale, window);
+        launch_type<float>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
+                           run, splits, part_o, part_ml, stream);
     else
-        AGAVE_CHECK(false, "attn_plain: unknown dtype %d", dtype);
+        launch_type<bf16>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
+                          run, splits, part_o, part_ml, stream);
     AGAVE_LAUNCH_CHECK("attn_plain");
     return 0;
 }

@@ -17,8 +17,9 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages
     if packed:
         attention_mfma.attention(q, out, k_pages, v_pages, table, base, step, n_heads, n_kv, head_dim, scale, window)
         return
-    kernels.attn_plain(q, out, k_pages, v_pages, table, base, step.tok_seq, step.tok_pos,
-                       n_heads, n_kv, head_dim, scale, window)
+    one_each = step.is_decode and step.n_tokens == step.n_seqs
+    kernels.attn_plain(q, out, k_pages, v_pages, table, base, step.tok_seq, step.tok_pos, n_heads, n_kv, head_dim, scale, window,
+                       one_token_each=one_each, span=step.page_span(window) if one_each else 1, workspace=step.workspace)
 
 
 def qk_attention(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.Tensor], q_rot: torch.Tensor,

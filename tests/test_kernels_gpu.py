@@ -352,6 +352,60 @@ def test_attn_plain(K, dtype, nh, nkv, hd, window):
     assert torch.allclose(got, ref, **tol)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh,nkv,hd,window", [(16, 4, 128, None), (20, 1, 6, 70), (32, 2, 34, None), (3, 1, 512, 130), (1, 1, 2, 1), (17, 1, 130, None)])
+def test_attn_plain_rows(K, dtype, nh, nkv, hd, window):
+    """Rows of several heads and tokens a workgroup: sequences that change within one, more heads on a key head than it takes,
+    head sizes at the edges of its tiles and not a multiple of four; and one token a sequence, alone and with several
+    workgroups to a row's pages."""
+    from agave_amd.parts import Workspace
+    lens = [1, 2, 1, 5, 130, 64, 65, 1, 300]
+    scale = hd ** -0.5
+    got, ref, _ = _attn_case(K, dtype, nh, nkv, hd, lens, window, scale)
+    tol = dict(atol=2e-6 + 1e-7 * hd, rtol=2e-5) if dtype == torch.float32 else dict(atol=2e-2, rtol=2e-2)
+    assert torch.allclose(got, ref, **tol)
+    real, asked = K.attn_plain, {}
+
+    def last_tokens(q, out, kp, vp, table, base, tok_seq, tok_pos, *rest):
+        """The same call for every sequence's last token."""
+        ends = torch.tensor([sum(lens[:i + 1]) - 1 for i in range(len(lens))], device=DEV)
+        for name, more in (("alone", {}), ("shared", {"span": 5, "workspace": Workspace(torch.device(DEV))})):
+            o = torch.empty(len(lens), nh * hd, dtype=q.dtype, device=DEV)
+            real(q[ends].contiguous(), o, kp, vp, table, base, tok_seq[ends].contiguous(), tok_pos[ends].contiguous(), *rest,
+                 one_token_each=True, **more)
+            asked[name] = o.cpu().double().view(-1, nh, hd)
+        real(q, out, kp, vp, table, base, tok_seq, tok_pos, *rest)
+    K.attn_plain = last_tokens
+    try:
+        _, ref, _ = _attn_case(K, dtype, nh, nkv, hd, lens, window, scale)
+    finally:
+        K.attn_plain = real
+    ends = [sum(lens[:i + 1]) - 1 for i in range(len(lens))]
+    for o in asked.values():
+        assert torch.allclose(o, ref[ends], **tol)
+
+
+def test_attn_plain_values_that_are_not_finite(K):
+    """What lies behind a token's position reaches no result, also where a later token of the same workgroup sees it."""
+    nh, nkv, hd, n = 4, 2, 32, 90
+    kp, vp = _pages(2, nkv, hd, torch.float32)
+    kp.normal_()
+    vp.normal_()
+    q, out = torch.randn(n, nh * hd, device=DEV), torch.empty(n, nh * hd, device=DEV)
+    args = (torch.tensor([[0, 1]], dtype=torch.int32, device=DEV), _i32([0]), _i32([0] * n), _i32(list(range(n))), nh, nkv, hd, 0.2, None)
+    K.attn_plain(q, out, kp, vp, *args)
+    want = out.clone()
+    vp[1, 0, 3, 6] = float("inf")                                        # position 70, element 3 of key head 0
+    vp[1, :, :, 26:] = float("nan")                                       # positions that no token has
+    kp[1, :, 26:] = float("nan")
+    K.attn_plain(q, out, kp, vp, *args)
+    bad = ~torch.isfinite(out)
+    hit = torch.zeros(n, nh, hd, dtype=torch.bool, device=DEV)
+    hit[70:, :2, 3] = True
+    assert torch.equal(bad.view(n, nh, hd), hit)
+    assert torch.allclose(out[~bad], want[~bad], atol=1e-6, rtol=1e-5)
+
+
 def test_attn_plain_far_key_wins(K):
     # among 700 keys, key 3 is made to dominate the last query's softmax: the output must be its value
     got, ref, vs = _attn_case(K, torch.float32, 2, 1, 32, [700], None, 0.5, seed=1, boost=3)
