@@ -715,6 +715,120 @@ __global__ __launch_bounds__(256) void routed_product_mfma_kernel(const bf16* __
         }
 }
 
+// Few pairs, weights in tile order, K a multiple of 1,024 (KQ = K / 128 steps of 32 a wave): bound by the weights' way from
+// memory.  A workgroup takes a tile of 16 sorted rows through `blocks` blocks of columns (GATED: 16 columns of the gate and the
+// up matrix, otherwise 32), its four waves a quarter of K each.  A wave keeps its quarter of the rows in registers for all
+// blocks (loaded again for every block, the rows were a third and a half of what the kernel above asks for) and streams its
+// weights, two tiles of a kilobyte a step, through a ring of NS steps in LDS of its own: it waits for nobody but its own loads,
+// and the loads of the next block's first steps are on their way while this one's sums meet in LDS.
+// Measured, both products, 16 experts of 2,048 by 2,048, 4 a row: 2 rows 47 us, 4 rows 60 us, 6 rows 70 us (330 MB, 4.7 TB/s);
+// with the kernel above 69, 81 and 89 us.
+template <int KQ, bool GATED>
+__global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* __restrict__ x, long ldx, const int* __restrict__ sorted_pair,
+                                                                    const int* __restrict__ tile_expert, const uint4* __restrict__ w0,
+                                                                    const uint4* __restrict__ w1, void* __restrict__ out_, int top, int n_out,
+                                                                    int act, int blocks, float p0, float p1) {
+    constexpr int K = KQ * 128, KB = K / 32, NS = 8;
+    static_assert(KQ % NS == 0, "a step's place in the ring is known where it is written");
+    constexpr int COLS = GATED ? 16 : 32;
+    __shared__ __attribute__((aligned(16))) unsigned char ring[4][NS][2048];
+    __shared__ float part[2][4][2][256];
+    const int e = tile_expert[blockIdx.x];
+    if (e < 0) return;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.x * 16, NBK = n_out / 16;
+    const int b0 = blockIdx.y * blocks, b1 = min(b0 + blocks, (n_out + COLS - 1) / COLS);
+    if (b0 >= b1) return;
+    long r = row0 + c;
+    if (GATED) {
+        const int p = sorted_pair[r];
+        r = p >= 0 ? p / top : 0;                                 // (a padding row computes on row 0 and is never read)
+    }
+    const bf16* arow = x + (size_t)r * ldx + w * (K / 4) + 8 * g;
+    frag16 a[KQ];
+#pragma unroll
+    for (int k = 0; k < KQ; ++k) a[k].u = *reinterpret_cast<const uint4*>(arow + 32 * k);
+    // the two tiles of step k of block b
+    auto fetch = [&](int b, int k, int slot) {
+        b = b < b1 ? b : b1 - 1;                                  // (past the end: loaded, never used)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            int nb = GATED ? b : 2 * b + i;
+            nb = nb < NBK ? nb : NBK - 1;                         // (columns past the end: never stored)
+            const uint4* src = (GATED && i ? w1 : w0) + (((size_t)e * NBK + nb) * KB + w * KQ + k) * 64 + lane;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                             (__attribute__((address_space(3))) void*)&ring[w][slot][i * 1024], 16, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < NS - 1; ++k) fetch(b0, k, k);
+    const unsigned at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&ring[w][0][0] + lane * 16;
+    constexpr int IN_FLIGHT = 2 * (NS - 2);
+    for (int b = b0; b < b1; ++b) {
+        f32x4_t acc[2] = {};
+        static_for<0, KQ>([&](auto kc) {
+            constexpr int k = kc.value, slot = k % NS;
+            __builtin_amdgcn_s_waitcnt(0x0F70 | (IN_FLIGHT & 15) | ((IN_FLIGHT >> 4) << 14));
+            frag16 f0, f1;
+            lds_read16<slot * 2048>(f0, at);
+            lds_read16<slot * 2048 + 1024>(f1, at);
+            lds_settle();
+            lds_use(f0);
+            lds_use(f1);
+            // (the step before this one has been read: its place is free)
+            fetch(k + NS - 1 < KQ ? b : b + 1, (k + NS - 1) % KQ, (slot + NS - 1) % NS);
+            acc[0] = mfma_16x16x32(a[k], f0, acc[0]);
+            acc[1] = mfma_16x16x32(a[k], f1, acc[1]);
+        });
+        // D: lane holds rows 4 g + e4, column c; wave w adds up and stores rows 4 g + w
+        float (&sums)[4][2][256] = part[b & 1];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) sums[w][i][e4 * 64 + lane] = acc[i][e4];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                             // (a bare barrier: the next block's weights stay on their way)
+        asm volatile("" ::: "memory");
+        float v[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) v[i] = ((sums[0][i][w * 64 + lane] + sums[1][i][w * 64 + lane]) + sums[2][i][w * 64 + lane]) + sums[3][i][w * 64 + lane];
+        const size_t row = (size_t)row0 + 4 * g + w;
+        if constexpr (GATED) {
+            // (gate and up are rounded to the rows' type before the activation, as the plain kernel does)
+            ((bf16*)out_)[row * n_out + b * 16 + c] = f32_to_bf16(expert_gated(bf16_to_f32(f32_to_bf16(v[0])), bf16_to_f32(f32_to_bf16(v[1])), act, p0, p1));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int col = b * 32 + 16 * i + c;
+                if (col < n_out) ((float*)out_)[row * n_out + col] = v[i];
+            }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);                           // loads past the last step land before the LDS goes to another workgroup
+}
+
+template <bool GATED>
+static bool launch_routed_few(const void* x, long ldx, const int* sorted_pair, const int* tile_expert, int max_tiles, const void* w0,
+                              const void* w1, void* out, int top, int live, int n_out, int K, int act, float p0, float p1, hipStream_t stream) {
+    if (K != 1024 && K != 2048 && K != 4096) return false;
+    const int all = (n_out + (GATED ? 15 : 31)) / (GATED ? 16 : 32);
+    // Blocks a workgroup: the fewest with which all workgroups run at once, two to a compute unit at most (some 450 where 512
+    // have a place: `live` is an expectation).  Both products, 4 rows: 75.8, 63.0, 66.7 us with 2, 4, 5 blocks of the gate;
+    // 6 rows 78.8, 68.3, 70.7; 16 rows 93.5, 93.0, 89.1; 1 row 32.5 and 42.3 with 2 and 4.
+    int blocks = (int)(((long)live * all + 447) / 448);
+    blocks = blocks < 1 ? 1 : blocks > 16 ? 16 : blocks;
+    const dim3 grid(max_tiles, (all + blocks - 1) / blocks);
+    if (grid.y > 65535) return false;
+#define FEW_GO(KQ_) routed_product_few_kernel<KQ_, GATED><<<grid, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const uint4*)w0, \
+                                                                                    (const uint4*)w1, out, top, n_out, act, blocks, p0, p1)
+    if (K == 1024) FEW_GO(8);
+    else if (K == 2048) FEW_GO(16);
+    else FEW_GO(32);
+#undef FEW_GO
+    return true;
+}
+
 // Many pairs an expert, weights in tile order: a workgroup takes a tile of TT sorted rows and 2 TT columns of weights
 // (GATED: TT columns of the gate and the same of the up matrix), TT/16 waves of 64 weight columns by TT/2 rows each.
 // Bound by the multiply-adds once both operands come through LDS: a wave that loads its own operands asks the compute
@@ -890,10 +1004,10 @@ static int launch_routed_tiled(const void* x, long ldx, const int* sorted_pair, 
 
 // act_rows [cap, ff] bfloat16 and y [cap, hidden] float32 hold sorted rows (see route_sort)
 extern "C" int agave_routed_experts_mfma(const void* x, long ldx, const int* sorted_pair, const int* tile_expert, const void* wg,
-                                         const void* wu, const void* wd, void* act_rows, float* y, int TM, int max_tiles, int top,
+                                         const void* wu, const void* wd, void* act_rows, float* y, int TM, int max_tiles, int n_rows, int top,
                                          int E, int ff, int hidden, int act, int wpacked, float p0, float p1, hipStream_t stream) {
     AGAVE_CHECK(!wpacked || (ff % 32 == 0 && hidden % 32 == 0), "routed_experts_mfma: weights in tile order need sizes that are multiples of 32");
-    AGAVE_CHECK(max_tiles > 0 && top > 0 && E > 0 && ff > 0 && hidden > 0 && (TM == 16 || TM == 64 || (TM == 128 && wpacked)), "routed_experts_mfma: bad sizes");
+    AGAVE_CHECK(max_tiles > 0 && n_rows >= 0 && top > 0 && E > 0 && ff > 0 && hidden > 0 && (TM == 16 || TM == 64 || (TM == 128 && wpacked)), "routed_experts_mfma: bad sizes");
     AGAVE_CHECK((act >= 0 && act < 4) || act == 6, "routed_experts_mfma: unknown activation %d", act);
     AGAVE_CHECK(hidden % 8 == 0 && ff % 8 == 0 && ldx % 8 == 0, "routed_experts_mfma: sizes must be multiples of 8 (hidden %d, ff %d)", hidden, ff);
     AGAVE_CHECK(x && sorted_pair && tile_expert && wg && wu && wd && act_rows && y, "routed_experts_mfma: null buffer");
@@ -923,9 +1037,15 @@ extern "C" int agave_routed_experts_mfma(const void* x, long ldx, const int* sor
         routed_product_mfma_kernel<4, 4, false><<<g2, 256, 0, stream>>>((const bf16*)act_rows, ff, sorted_pair, tile_expert, (const bf16*)wd,
                                                                      nullptr, y, top, hidden, ff, act, wpacked, p0, p1);
     } else {
-        routed_product_mfma_kernel<1, 1, true><<<g1, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const bf16*)wg,
+        // experts that have rows, if the rows choose evenly
+        const int live = top >= E ? E : (int)ceil(E * (1.0 - pow(1.0 - (double)top / E, (double)n_rows)));
+        const bool few1 = wpacked && launch_routed_few<true>(x, ldx, sorted_pair, tile_expert, max_tiles, wg, wu, act_rows, top, live, ff, hidden, act, p0, p1, stream);
+        if (!few1)
+            routed_product_mfma_kernel<1, 1, true><<<g1, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const bf16*)wg,
                                                                     (const bf16*)wu, act_rows, top, ff, hidden, act, wpacked, p0, p1);
-        routed_product_mfma_kernel<1, 1, false><<<g2, 256, 0, stream>>>((const bf16*)act_rows, ff, sorted_pair, tile_expert, (const bf16*)wd,
+        const bool few2 = wpacked && launch_routed_few<false>(act_rows, ff, nullptr, tile_expert, max_tiles, wd, nullptr, y, top, live, hidden, ff, act, p0, p1, stream);
+        if (!few2)
+            routed_product_mfma_kernel<1, 1, false><<<g2, 256, 0, stream>>>((const bf16*)act_rows, ff, sorted_pair, tile_expert, (const bf16*)wd,
                                                                      nullptr, y, top, hidden, ff, act, wpacked, p0, p1);
     }
     AGAVE_LAUNCH_CHECK("routed_experts_mfma");

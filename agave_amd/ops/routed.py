@@ -16,7 +16,7 @@ kernels.register_signatures(LIBRARY, {
     "agave_routed_experts_plain": [_I, _P, _L, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "agave_route_rows": [_I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _P, _I, _I, _P],
     "agave_route_sort": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P],
-    "agave_routed_experts_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
+    "agave_routed_experts_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "agave_routed_combine": [_I, _P, _P, _P, _P, _P, _L, _P, _L, _P, _P, _L, _I, _I, _I, _I, _P],
 })
 
@@ -97,16 +97,16 @@ def tile_plan(n_pairs: int, n_experts: int, tile_order: bool = False, ff: int = 
 
     Weights row by row: tiles of 64 rows where an expert gets some 32 pairs or more on average, of 16 otherwise.
     Weights in tile order (``tile_order``, experts of ``ff`` inner rows and ``hidden`` columns): 128 from 128 pairs an expert
-    on; 64 from two pairs an expert on where their workgroups (64 inner rows, 128 columns each) about fill the chip; below
-    that 16.  Measured with 16 experts of 2,048 by 2,048, both products: 16 pairs 66 us in tiles of 16 and 69 in tiles of 64,
-    32 pairs 101 and 82, 256 pairs 156 and 86; 1,600 pairs 124 us in tiles of 64 and 125 in tiles of 128, 2,400 pairs 162
+    on; 64 from four pairs an expert on (two where tiles of 16 have no kernel that streams the sizes) where their workgroups (64 inner rows, 128 columns each) about fill the chip; below
+    that 16.  Measured with 16 experts of 2,048 by 2,048, both products: 16 pairs 60 us in tiles of 16 and 73 in tiles of 64,
+    32 pairs 82 and 83, 64 pairs 85 and 87, 128 pairs 95 and 89; 1,600 pairs 124 us in tiles of 64 and 125 in tiles of 128, 2,400 pairs 162
     and 137."""
     tm = 64 if n_pairs >= 32 * n_experts else 16
     if tile_order:
         live = min(n_pairs, n_experts)
         if n_pairs >= 128 * n_experts:
             tm = 128
-        elif n_pairs >= 2 * n_experts and live * (ff // 64) >= 256 and live * (hidden // 128) >= 128:
+        elif n_pairs >= (4 if ff in (1024, 2048, 4096) and hidden in (1024, 2048, 4096) else 2) * n_experts and live * (ff // 64) >= 256 and live * (hidden // 128) >= 128:
             tm = 64
     tiles = (n_pairs + tm - 1) // tm + n_experts
     return tm, tiles, tiles * tm
@@ -156,7 +156,7 @@ def experts_mfma(x: torch.Tensor, sorted_pair: torch.Tensor, tile_expert: torch.
     _i32(sorted_pair, "sorted_pair", cap)
     _i32(tile_expert, "tile_expert", tiles)
     library.call(_lib(), "agave_routed_experts_mfma", ptr(x), x.stride(0), ptr(sorted_pair), ptr(tile_expert), ptr(w_gate),
-                 ptr(w_up), ptr(w_down), ptr(act_rows), ptr(y), tm, tiles, top, e, ff, hidden, activation,
+                 ptr(w_up), ptr(w_down), ptr(act_rows), ptr(y), tm, tiles, n, top, e, ff, hidden, activation,
                  1 if tile_order else 0, float(p0), float(p1), stream())
 
 

@@ -518,3 +518,26 @@ def test_routed_tiles_in_tile_order(n, E, top, ff, hidden, tm):
     for o, at in zip(out, (0, 1)):                  # rows aligned to four elements, and one element off
         routed.combine(y, place, choice, weight, x, shared, o[:, at:at + hidden], top, E)
     assert torch.equal(out[0][:, :hidden], out[1][:, 1:hidden + 1])
+
+
+@pytest.mark.parametrize("n,E,top,ff,hidden", [(1, 5, 2, 1024, 2048), (6, 16, 4, 2048, 1056), (40, 3, 2, 1024, 1024), (3, 4, 4, 4096, 1024)])
+def test_routed_few_pairs_in_tile_order(n, E, top, ff, hidden):
+    """Tiles of 16 rows whose weights stream through a ring in LDS (columns summed over 1,024, 2,048 or 4,096; with others the kernel
+    without one): one block of columns a workgroup and several, a block that breaks off, experts without a pair.  The sums are
+    those of the kernel that takes weights row by row, in the same order."""
+    from agave_amd.ops import routed
+    g = torch.Generator().manual_seed(n + ff)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * s[-1] ** -0.5).bfloat16().to(DEV)
+    x, wg, wu, wd = torch.randn(n, hidden, generator=g).bfloat16().to(DEV), rnd(E, ff, hidden), rnd(E, ff, hidden), rnd(E, hidden, ff)
+    choice = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(n)]).int().view(-1).to(DEV)
+    tiles = (n * top + 15) // 16 + E
+    place, sorted_pair, tile_expert = (torch.full((k,), -7, dtype=torch.int32, device=DEV) for k in (n * top, tiles * 16, tiles))
+    routed.route_sort(choice, E, 16, tiles, place, sorted_pair, tile_expert)
+    rows = []
+    for packed in (False, True):
+        act_rows = torch.empty(tiles * 16, ff, dtype=torch.bfloat16, device=DEV)
+        y = torch.full((tiles * 16, hidden), float("nan"), device=DEV)
+        w = [routed.pack_expert_weights(v) if packed else v for v in (wg, wu, wd)]
+        routed.experts_mfma(x, sorted_pair, tile_expert, *w, act_rows, y, 16, tiles, top, 1, tile_order=packed)
+        rows.append(y[place.long()])
+    assert bool(torch.isfinite(rows[0]).all()) and torch.equal(rows[0], rows[1])
