@@ -1094,21 +1094,24 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
 __global__ __launch_bounds__(256) void attn_biased_merge_kernel(const float* __restrict__ parts, int splits, int nh, int vd,
                                                                 bf16* __restrict__ out, long ldo, const bf16* __restrict__ gate,
                                                                 long ldg) {
-    const int t = blockIdx.x / nh, h = blockIdx.x % nh;
+    // a lane per share (at most 64): all references and sums in one round trip, the shares' weights through LDS
+    __shared__ float weight[4][64];
+    const int t = blockIdx.x / nh, h = blockIdx.x % nh, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const float* mine = parts + (size_t)blockIdx.x * splits * (vd + 2);
-    float mx = -INFINITY;
-    for (int s = 0; s < splits; ++s) mx = fmaxf(mx, mine[(size_t)s * (vd + 2)]);
-    float total = 0.f;
-    for (int s = 0; s < splits; ++s) {
-        const float ms = mine[(size_t)s * (vd + 2)];
-        if (ms != -INFINITY) total += mine[(size_t)s * (vd + 2) + 1] * __builtin_amdgcn_exp2f(ms - mx);
-    }
+    const float* ml = mine + (size_t)(lane < splits ? lane : 0) * (vd + 2);
+    const float m0 = ml[0], l0 = ml[1];
+    const float ms = lane < splits ? m0 : -INFINITY, mx = wave_max(ms);
+    const float f = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+    const float total = wave_sum(f == 0.f ? 0.f : l0 * f);
     const float inv = total > 0.f ? 1.0f / total : 0.f;
+    weight[w][lane] = ms == -INFINITY ? -1.f : f;              // (a share without a key is left out whatever it holds)
+    __builtin_amdgcn_wave_barrier();                           // (a wave's LDS accesses happen in the order they were issued)
     for (int d = threadIdx.x; d < vd; d += blockDim.x) {
         float acc = 0.f;
+#pragma unroll 8
         for (int s = 0; s < splits; ++s) {
-            const float ms = mine[(size_t)s * (vd + 2)];
-            if (ms != -INFINITY) acc = fmaf(mine[(size_t)s * (vd + 2) + 2 + d], __builtin_amdgcn_exp2f(ms - mx), acc);
+            const float x = mine[(size_t)s * (vd + 2) + 2 + d], fs = weight[w][s];
+            acc = fs != -1.f ? fmaf(x, fs, acc) : acc;
         }
         float y = acc * inv;
         if (gate) y *= 1.0f / (1.0f + __expf(-bf16_to_f32(gate[(size_t)t * ldg + (size_t)h * vd + d])));

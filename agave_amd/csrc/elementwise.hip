@@ -18,7 +18,21 @@ __global__ void embed_scale_kernel(const int* __restrict__ tokens, const T* __re
     tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);   // the host rejects such ids; never read outside
     const T* row = table + (size_t)tok * e;
     float* o = out + (size_t)t * e;
-    for (int i = threadIdx.x; i < e; i += blockDim.x) o[i] = ld(row + i) * scale;
+    // (eight elements of a thread at a time are asked for together: the row is one round trip to memory and not eight)
+    constexpr int U = 8;
+    for (int i0 = threadIdx.x; i0 < e; i0 += U * blockDim.x) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + u * blockDim.x;
+            v[u] = ld(row + (i < e ? i : 0));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = i0 + u * blockDim.x;
+            if (i < e) o[i] = v[u] * scale;
+        }
+    }
 }
 
 extern "C" int agave_embed_scale(int dtype, const int* tokens, const void* table, float scale,

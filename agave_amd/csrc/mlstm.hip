@@ -163,16 +163,24 @@ __global__ __launch_bounds__(256) void mlstm_readout_kernel(MlstmArgs A, const f
     const float* x = num + row * ((long)A.nh * dv) + (long)h * dv;
     const float* g = A.gate + row * A.ld + (long)h * dv;
     const float* w = A.weight + (long)h * dv;
+    // (the rows, the gate and the weights are asked for before anything waits: one round trip to memory)
+    float o[KEEP], gv[KEEP], wv[KEEP], ss = 0.f;
+#pragma unroll
+    for (int u = 0; u < KEEP; ++u) {
+        if (u * nt >= dv) break;
+        const int e = (int)threadIdx.x + u * nt < dv ? (int)threadIdx.x + u * nt : 0;
+        o[u] = x[e];
+        gv[u] = g[e];
+        wv[u] = w[e];
+    }
     float i, f;
     log_gates(A, row, h, i, f);
     const float m1 = (float)fmax((double)f + (double)A.m[sh], (double)i);
     const float inv_den = 1.0f / (fmaxf(fabsf(nq[row * A.nh + h]), expf(-m1)) + A.floor_eps);
-    float o[KEEP], ss = 0.f;
 #pragma unroll
     for (int u = 0; u < KEEP; ++u) {
-        const int e = (int)threadIdx.x + u * nt;
         if (u * nt >= dv) break;
-        o[u] = e < dv ? x[e] * inv_den : 0.f;
+        o[u] = (int)threadIdx.x + u * nt < dv ? o[u] * inv_den : 0.f;
         ss = fmaf(o[u], o[u], ss);
     }
     ss = block_sum(ss, red);                        // (its barriers: every thread has read m)
@@ -182,7 +190,7 @@ __global__ __launch_bounds__(256) void mlstm_readout_kernel(MlstmArgs A, const f
     for (int u = 0; u < KEEP; ++u) {
         const int e = (int)threadIdx.x + u * nt;
         if (u * nt >= dv) break;
-        if (e < dv) st(out + row * ldo + (long)h * dv + e, o[u] * inv * w[e] * sigmoid_of(g[e]));
+        if (e < dv) st(out + row * ldo + (long)h * dv + e, o[u] * inv * wv[u] * sigmoid_of(gv[u]));
     }
 }
 
