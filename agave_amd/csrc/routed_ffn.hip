@@ -134,39 +134,52 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
     for (int e = threadIdx.x; e < R; e += blockDim.x) corr[e] = correction ? correction[e] : 0.f;
     const int t0 = blockIdx.x * RR;
     const int rows = min(RR, N - t0);
-    for (int r = w; r < Rt; r += nw) {
+    // Two outputs a wave at a time, w and w + nw (a wave without a second one reads its first again): with a few more outputs than
+    // waves the rows of both are one round trip to memory (17 outputs of 2,048, 6 tokens: 8.2 us one after the other, 7.3 us so; 3,001 tokens 37.6 and 31.8).
+    for (int r = w; r < Rt; r += 2 * nw) {
+        const bool second = r + nw < Rt;
         const float* wr = router + (size_t)r * K;
-        float acc[RR];
+        const float* wr2 = second ? wr + (size_t)nw * K : wr;
+        float acc[RR], acc2[RR];
 #pragma unroll
-        for (int i = 0; i < RR; ++i) acc[i] = 0.f;
+        for (int i = 0; i < RR; ++i) acc[i] = acc2[i] = 0.f;
         if (WIDE) {
-#pragma unroll(RR == 1 ? 4 : 2)
+#pragma unroll(RR == 1 ? 4 : 1)
             for (int k = 8 * lane; k < K; k += 512) {
-                float wk[8];
+                float wk[8], wk2[8];
                 load8(wr + k, wk);
+                load8(wr2 + k, wk2);
 #pragma unroll
                 for (int i = 0; i < RR; ++i) {
                     const int t = t0 + (i < rows ? i : 0);
                     float xv[8];
                     load8(x + (size_t)t * ldx + k, xv);
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) acc[i] = fmaf(xv[j], wk[j], acc[i]);
+                    for (int j = 0; j < 8; ++j) {
+                        acc[i] = fmaf(xv[j], wk[j], acc[i]);
+                        acc2[i] = fmaf(xv[j], wk2[j], acc2[i]);
+                    }
                 }
             }
         } else {
             for (int k = lane; k < K; k += 64) {
-                const float wk = wr[k];
+                const float wk = wr[k], wk2 = wr2[k];
 #pragma unroll
                 for (int i = 0; i < RR; ++i) {
                     const int t = t0 + (i < rows ? i : 0);
-                    acc[i] = fmaf(ld(x + (size_t)t * ldx + k), wk, acc[i]);
+                    const float xv = ld(x + (size_t)t * ldx + k);
+                    acc[i] = fmaf(xv, wk, acc[i]);
+                    acc2[i] = fmaf(xv, wk2, acc2[i]);
                 }
             }
         }
 #pragma unroll
         for (int i = 0; i < RR; ++i) {
-            const float sum = wave_sum(acc[i]);
-            if (lane == 0) zs[i * Rt + r] = sum;
+            const float sum = wave_sum(acc[i]), sum2 = wave_sum(acc2[i]);
+            if (lane == 0) {
+                zs[i * Rt + r] = sum;
+                if (second) zs[i * Rt + r + nw] = sum2;
+            }
         }
     }
     __syncthreads();
@@ -552,6 +565,44 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const int* __restrict_
     }
 }
 
+// Up to 64 pairs and 64 experts (a decode step of few tokens): one wave, a lane per pair.  A pair's rank within its expert is a
+// count of the lanes below it, so nothing meets in LDS and no thread walks the experts alone.  24 pairs of 16 experts: 4.7 us,
+// with the kernel above 5.3.
+#define FEW_CAP (65 * 64)      // sorted rows: 64 experts and a tile more, in tiles of up to 64
+__global__ __launch_bounds__(64) void route_sort_few_kernel(const int* __restrict__ choice, int P, int E, int TM, int cap, int max_tiles,
+                                                            int* __restrict__ place, int* __restrict__ sorted_pair,
+                                                            int* __restrict__ tile_expert) {
+    const int lane = threadIdx.x;
+    const int mine = lane < P ? choice[lane] : -1;
+    const unsigned long long below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+    __shared__ int sorted[FEW_CAP];
+    for (int r = lane; r < cap; r += 64) sorted[r] = -1;
+    int row = -1, count = 0;                               // this lane's pair's row; pairs of expert `lane`
+    int tile = 0;
+    for (int e = 0; e < E; ++e) {
+        const unsigned long long who = __ballot(mine == e);
+        const int n = __popcll(who);
+        if (mine == e) row = tile * TM + __popcll(who & below);
+        if (lane == e) count = tile;                        // (its first tile, for the table below)
+        tile += (n + TM - 1) / TM;
+    }
+    // expert of a tile: the last one that starts at or before it and has a tile
+    for (int t = lane; t < max_tiles; t += 64) {
+        int ex = -1;
+        for (int e = 0; e < E; ++e) {
+            const int first = __builtin_amdgcn_readlane(count, e), next = e + 1 < E ? __builtin_amdgcn_readlane(count, e + 1) : tile;
+            if (t >= first && t < next) ex = e;
+        }
+        tile_expert[t] = ex;
+    }
+    // (a wave's LDS accesses happen in the order they were issued)
+    __builtin_amdgcn_wave_barrier();
+    if (row >= 0 && row < cap) sorted[row] = lane;
+    __builtin_amdgcn_wave_barrier();
+    for (int r = lane; r < cap; r += 64) sorted_pair[r] = sorted[r];
+    if (lane < P) place[lane] = row < cap ? row : -1;
+}
+
 extern "C" int agave_route_sort(const int* choice, int P, int E, int TM, int cap, int max_tiles, int* place, int* sorted_pair,
                                 int* tile_expert, hipStream_t stream) {
     AGAVE_CHECK(P >= 0 && E > 0 && E <= ROUTE_MAX && (TM == 16 || TM == 64 || TM == 128), "route_sort: bad sizes P=%d E=%d TM=%d", P, E, TM);
@@ -559,6 +610,11 @@ extern "C" int agave_route_sort(const int* choice, int P, int E, int TM, int cap
                 max_tiles, TM, P, E);
     AGAVE_CHECK(choice && place && sorted_pair && tile_expert, "route_sort: null buffer");
     if (P == 0) return 0;
+    if (P <= 64 && E <= 64 && cap <= FEW_CAP) {
+        route_sort_few_kernel<<<1, 64, 0, stream>>>(choice, P, E, TM, cap, max_tiles, place, sorted_pair, tile_expert);
+        AGAVE_LAUNCH_CHECK("route_sort");
+        return 0;
+    }
     route_sort_kernel<<<1, 1024, 0, stream>>>(choice, P, E, TM, cap, max_tiles, place, sorted_pair, tile_expert);
     AGAVE_LAUNCH_CHECK("route_sort");
     return 0;

@@ -541,3 +541,23 @@ def test_routed_few_pairs_in_tile_order(n, E, top, ff, hidden):
         routed.experts_mfma(x, sorted_pair, tile_expert, *w, act_rows, y, 16, tiles, top, 1, tile_order=packed)
         rows.append(y[place.long()])
     assert bool(torch.isfinite(rows[0]).all()) and torch.equal(rows[0], rows[1])
+
+
+@pytest.mark.parametrize("tm", [16, 64])
+@pytest.mark.parametrize("P,E,chosen", [(1, 1, 1), (1, 64, 70), (64, 64, 64), (63, 7, 9), (40, 3, 2), (64, 1, 1), (65, 64, 66), (64, 65, 65)])
+def test_route_sort_of_few_pairs(P, E, chosen, tm):
+    """Every pair in a row of one of its expert's tiles, every row's pair, every tile's expert, all others empty; with identity
+    choices, experts without a pair, and the sizes at which another kernel takes over."""
+    from agave_amd.ops import routed
+    g = torch.Generator().manual_seed(P + E)
+    choice = torch.randint(0, chosen, (P,), generator=g).int()
+    tiles = (P + tm - 1) // tm + E
+    place, sorted_pair, tile_expert = (torch.full((k,), -7, dtype=torch.int32, device=DEV) for k in (P, tiles * tm, tiles))
+    routed.route_sort(choice.to(DEV), E, tm, tiles, place, sorted_pair, tile_expert)
+    place, sorted_pair, tile_expert = place.tolist(), sorted_pair.tolist(), tile_expert.tolist()
+    for p, e in enumerate(choice.tolist()):
+        assert (place[p] == -1) if e >= E else (sorted_pair[place[p]] == p and tile_expert[place[p] // tm] == e)
+    real = [e for e in choice.tolist() if e < E]
+    assert sum(r >= 0 for r in sorted_pair) == len(real) and set(sorted_pair) <= set(range(P)) | {-1}
+    want = [e for e in range(E) for _ in range((real.count(e) + tm - 1) // tm)]
+    assert tile_expert == want + [-1] * (tiles - len(want))
