@@ -64,6 +64,31 @@ def test_short_conv_whole_pieces_and_tokens(taps, silu):
         assert torch.allclose(got.to(F64), ref, atol=2e-5, rtol=1e-5), (first, piece)
 
 
+@pytest.mark.parametrize("taps", [2, 3, 4])
+def test_short_conv_many_rows(taps):
+    """The kernel that slides along neighbouring rows against the one with a thread per row (which takes the same channels a few at
+    a time): sequences shorter than the taps, beginning and ending inside its stretches of rows, with states that go on."""
+    from agave_amd.cache import StateNeed
+    from agave_amd.ops import sequence as S
+    g = torch.Generator().manual_seed(taps)
+    C, part = 1000, 250
+    w, bias, ib = (torch.randn(*k, generator=g).to(DEV) for k in ((C, taps), (C,), (C,)))
+    cols = [slice(i, i + part) for i in range(0, C, part)]
+    whole, parts = planner_for(state={0: StateNeed((taps - 1, C))}, slots=6, context=4096), [planner_for(state={0: StateNeed((taps - 1, part))}, slots=6, context=4096) for _ in cols]
+    slots = [[cache.alloc_slot() for _ in range(6)] for cache, _ in [whole] + parts][0]
+    for lens in ([3, 1, 2, 5], [700, 1, 17, 1400], [1, 2, 2200, 16]):
+        x = torch.randn(sum(lens), C, generator=g).to(DEV)
+        ys = []
+        for (cache, planner), at in zip([whole] + parts, [slice(0, C)] + cols):
+            step = feed(cache, planner, slots[1:5], lens)
+            y = torch.empty(sum(lens), at.stop - at.start, device=DEV)
+            S.short_conv(x[:, at].contiguous(), w[at].contiguous(), y, cache.state[0], step, True, bias[at].contiguous(), ib[at].contiguous())
+            planner.commit(step)
+            ys.append(y)
+        assert torch.equal(ys[0], torch.cat(ys[1:], 1)), lens
+        assert torch.equal(whole[0].state[0], torch.cat([cache.state[0] for cache, _ in parts], -1)), lens
+
+
 def test_short_conv_batch_of_unequal_sequences_and_a_slot_used_again():
     from agave_amd.cache import StateNeed
     from agave_amd.ops import sequence as S
