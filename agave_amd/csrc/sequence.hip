@@ -1055,7 +1055,7 @@ extern "C" int agave_gated_recurrence(int mode, const float* q, long ldq, const 
 // lane a token): D and, per head and token, what the second kernel would otherwise make in every workgroup and wave:
 //     d;  exp(D_i);  d_j exp(D_n - D_j);  d_j exp(D_e - D_j) with e the last token of j's sixteen
 #define SSD_CHUNK 64
-#define SSD_SUMS 8              // running sums of a product: a sum in 32 bits loses more the longer it runs
+#define SSD_SUMS 16             // running sums of a product: a sum in 32 bits loses more the longer it runs
 struct SsdScratch {
     float* cb;                  // [tokens][groups][64]
     double* cum;                // [heads][tokens]: D
@@ -1063,8 +1063,20 @@ struct SsdScratch {
     long n;                     // tokens
     long heads_n;               // heads * tokens
 };
+// exp of a number held in double: the argument's rounding to 32 bits would be an error of its size in units of the last place
+__device__ __forceinline__ float exp_of(double x) {
+    const float h = (float)x, e = expf(h);
+    return fmaf(e, (float)(x - (double)h), e);
+}
 __device__ __forceinline__ f32x4_t ssd_total(const f32x4_t (&a)[SSD_SUMS]) {
-    return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+    f32x4_t t[SSD_SUMS / 2];
+#pragma unroll
+    for (int i = 0; i < SSD_SUMS / 2; ++i) t[i] = a[2 * i] + a[2 * i + 1];
+#pragma unroll
+    for (int n = SSD_SUMS / 4; n > 0; n /= 2)
+#pragma unroll
+        for (int i = 0; i < n; ++i) t[i] = t[2 * i] + t[2 * i + 1];
+    return t[0];
 }
 __global__ __launch_bounds__(256) void ssd_prepare_kernel(RecurrenceArgs A, SsdScratch X) {
     const int s = blockIdx.z, r0 = A.cu[s], r1 = A.cu[s + 1], t0 = r0 + blockIdx.x * SSD_CHUNK;
@@ -1078,10 +1090,9 @@ __global__ __launch_bounds__(256) void ssd_prepare_kernel(RecurrenceArgs A, SsdS
         for (int jt = 0; jt <= w; ++jt) {
             const float* b = A.k + (size_t)min(t0 + 16 * jt + r, r1 - 1) * A.ldk + (size_t)grp * A.dk + 4 * g;
             f32x4_t acc[SSD_SUMS] = {};
-#pragma unroll 2
-            for (int k = 0; k < A.dk; k += 32)
+            for (int k = 0; k < A.dk; k += 64)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
+                for (int i = 0; i < 4; ++i) {
                     const f32x4_t x = *reinterpret_cast<const f32x4_t*>(c + k + 16 * i), y = *reinterpret_cast<const f32x4_t*>(b + k + 16 * i);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) acc[4 * i + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], acc[4 * i + e], 0, 0, 0);
@@ -1097,9 +1108,11 @@ __global__ __launch_bounds__(256) void ssd_prepare_kernel(RecurrenceArgs A, SsdS
     }
     const int h = (blockIdx.y - A.nkv) * 4 + w;
     if (h >= A.nh) return;
-    const float d = softplus_exact(A.dt[(size_t)(t0 + min(lane, n - 1)) * A.lddt + h] + A.dt_bias[h]);
+    // (softplus, rate and exponentials in double: all that follows multiplies by them, and here they are made once)
+    const double u = (double)A.dt[(size_t)(t0 + min(lane, n - 1)) * A.lddt + h] + (double)A.dt_bias[h];
+    const double d = u > 40.0 ? u : log1p(exp(u));
     // (exp(-1000) is 0 in 32 bits: a token that forgets everything stays finite here, so that differences of sums do)
-    double x = -(double)expf(A.a_log[h]) * (double)d;
+    double x = -exp((double)A.a_log[h]) * d;
     x = x < -1000.0 ? -1000.0 : x;
 #pragma unroll
     for (int o = 1; o < 64; o *= 2) {
@@ -1110,10 +1123,10 @@ __global__ __launch_bounds__(256) void ssd_prepare_kernel(RecurrenceArgs A, SsdS
     if (lane < n) {
         const long at = (long)h * X.n + t0 + lane;
         X.cum[at] = x;
-        X.made[at] = d;
-        X.made[X.heads_n + at] = expf((float)x);
-        X.made[2 * X.heads_n + at] = d * expf((float)(end - x));
-        X.made[3 * X.heads_n + at] = d * expf((float)(end16 - x));
+        X.made[at] = (float)d;
+        X.made[X.heads_n + at] = (float)exp(x);
+        X.made[2 * X.heads_n + at] = (float)(d * exp(end - x));
+        X.made[3 * X.heads_n + at] = (float)(d * exp(end16 - x));
     }
 }
 
@@ -1127,10 +1140,11 @@ __global__ __launch_bounds__(256) void ssd_prepare_kernel(RecurrenceArgs A, SsdS
 // of which can overflow (an exponential per pair of tokens is no closer to 64 bits and 14 % slower).
 // A value that is not finite must not reach tokens before it, which a product with a zero weight would do: a chunk with one is
 // summed token by token.
-// Bound by the chain of chunks, some 3.5 us each.  Measured with the kernel before it, 64 heads of 64 x 128: 3,001 tokens 166 us
-// (token by token 600 us), 500 tokens 42 (110), 64 tokens 17 (21), 32 tokens 17 (15); six sequences of 40 tokens 38 (49).
-// Errors against 64 bits are those of the tokens one by one (1.1 to 1.2e-7 of the read-outs); with one running sum a product,
-// 2.2e-7.
+// Bound by the chain of chunks, some 3.6 us each.  Measured with the kernel before it, 64 heads of 64 x 128: 3,001 tokens 176 us
+// (token by token 600 us), 500 tokens 45 (109), 64 tokens 17 (19), 48 tokens 16 (17), 32 tokens 17 (15); six sequences of 40
+// tokens 41 (49).  Errors against 64 bits, here and token by token, in units of 1e-7: read-outs 1.04 to 1.09 and 1.08 to 1.23,
+// states 0.5 to 0.7 and 0.6 to 1.1, at 48 to 3,001 tokens.  Read-outs with one running sum a product 2.2; with eight, and step sizes
+// and exponentials in 32 bits, 1.12 to 1.25.
 template <int DK>
 __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScratch X) {
     constexpr int KW = DK / 4, KF = KW / 16, CF = DK / 16;      // key channels of a state wave, of those a lane's neighbours; operands of a row of C
@@ -1203,13 +1217,13 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
                     const f32x4_t vf = *reinterpret_cast<const f32x4_t*>(&Vt[buf][r][16 * j + 4 * g]);      // tokens 16 j + 4 g + e, column r
                     f32x4_t m;
                     if (j < w) {
-                        m = *reinterpret_cast<const f32x4_t*>(&made[buf][3][16 * j + 4 * g]) * expf((float)(here - Dc[buf][16 * j + 15]));
+                        m = *reinterpret_cast<const f32x4_t*>(&made[buf][3][16 * j + 4 * g]) * exp_of(here - Dc[buf][16 * j + 15]);
                     } else {
                         const f32x4_t d = *reinterpret_cast<const f32x4_t*>(&made[buf][0][16 * j + 4 * g]);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const int t = 4 * g + e;
-                            m[e] = t <= r ? expf((float)(here - Dc[buf][16 * j + t])) * d[e] : 0.f;
+                            m[e] = t <= r ? exp_of(here - Dc[buf][16 * j + t]) * d[e] : 0.f;
                         }
                     }
 #pragma unroll
@@ -1225,7 +1239,7 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
                     const int i = 16 * w + 4 * g + e;
                     const float* row = X.cb + ((size_t)min(t0 + i, last) * A.nkv + grp) * SSD_CHUNK;
                     for (int j = 0; j <= i && j < n; ++j)
-                        y[e] = fmaf(row[j] * (expf((float)(Dc[buf][i] - Dc[buf][j])) * made[buf][0][j]), Vt[buf][r][j], y[e]);
+                        y[e] = fmaf(row[j] * (exp_of(Dc[buf][i] - Dc[buf][j]) * made[buf][0][j]), Vt[buf][r][j], y[e]);
                 }
             }
 #pragma unroll
@@ -1270,8 +1284,7 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
             lds_barrier();
             if (ch + 1 < n_chunks) ask(next, t0 + SSD_CHUNK);
             const float left = made[buf][1][n - 1];
-#pragma unroll
-            for (int f = 0; f < KF; ++f) st[f] *= left;
+            f32x4_t sum[2][KF] = {};                            // (sums of their own: each rounds as its own size asks, not as the state's)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const f32x4_t vf = *reinterpret_cast<const f32x4_t*>(&Vt[buf][r][16 * j + 4 * g]) *
@@ -1279,8 +1292,12 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int f = 0; f < KF; ++f) st[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[4 * j + e][f], vf[e], st[f], 0, 0, 0);
+                    for (int f = 0; f < KF; ++f) sum[e & 1][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[4 * j + e][f], vf[e], sum[e & 1][f], 0, 0, 0);
             }
+#pragma unroll
+            for (int f = 0; f < KF; ++f)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) st[f][e] = fmaf(st[f][e], left, sum[0][f][e] + sum[1][f][e]);
             cur = next;
         }
 #pragma unroll

@@ -154,7 +154,7 @@ def talk_attention(q: torch.Tensor, gate: Optional[torch.Tensor], out: torch.Ten
 
 SSD_CHUNK = 64
 # A sequence that brings this many tokens: chunks of 64 from here on, token by token below (64 heads of 64 x 128: 32 tokens
-# take 15 us token by token and 17 in chunks, 48 tokens 17 and 16, 64 tokens 21 and 17).
+# take 15 us token by token and 17 in chunks, 48 tokens 17 and 16, 64 tokens 19 and 17).
 SSD_CHUNKS_FROM = 48
 
 
