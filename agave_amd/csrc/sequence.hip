@@ -154,8 +154,10 @@ extern "C" int agave_short_conv(const float* u, long ldu, const float* w, const 
     const dim3 grid((C + threads - 1) / threads, n_tokens), rows((C + threads - 1) / threads, (n_tokens + CONV_ROWS - 1) / CONV_ROWS);
 #define CONV_GO(SILU_, TAPS_) short_conv_rows_kernel<SILU_, TAPS_><<<rows, threads, 0, stream>>>(u, ldu, w, bias, y, ldy, state, tok_seq, tok_pos, \
                                                                                               pos0, slots, n_tokens, C, in_bias)
-    // (from some 1,000 workgroups of the kernel for many rows on; below that its rows one after another cost more than they save)
-    if (!one_token_each && taps >= 2 && taps <= 4 && (long)rows.x * rows.y >= 512) {
+    // (With fewer workgroups of the kernel for many rows, its rows one after another take longer than they save.  us, a row a
+    // thread and many, four taps: 4,352 channels 128 rows, 136 workgroups, 7.8 and 8.1, 256 rows, 272, 10.5 and 8.6; 12,288
+    // channels 64 rows, 192, 8.7 and 8.2; 512 channels 1,000 rows, 126, 7.2 and 8.0, 3,001 rows, 376, 12.1 and 8.9.)
+    if (!one_token_each && taps >= 2 && taps <= 4 && (long)rows.x * rows.y >= 192) {
         if (silu) {
             if (taps == 2) CONV_GO(true, 2); else if (taps == 3) CONV_GO(true, 3); else CONV_GO(true, 4);
         } else {
