@@ -1432,7 +1432,12 @@ __global__ __launch_bounds__(1024) void gated_group_norm_kernel(const float* __r
             ss = fmaf(a[v], a[v], ss);
         }
     }
-    ss = blockDim.x > 64 ? block_sum(ss, red) : wave_sum(ss);
+    ss = wave_sum(ss);
+    if (blockDim.x > 64) {                              // (the waves' sums in pairs as well: sixteen one after another lose more)
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = wave_sum((threadIdx.x & 63) < blockDim.x / 64 ? red[threadIdx.x & 63] : 0.f);
+    }
     const float inv = 1.0f / sqrtf(ss / (float)size + eps);
     T* o = out + (size_t)t * ldo + (size_t)g * size;
 #pragma unroll
@@ -1464,9 +1469,11 @@ extern "C" int agave_gated_group_norm(int dtype, const float* y, long ldy, const
     const uintptr_t wide = dtype == AGAVE_F32 ? 16 : 8;                // bytes of four neighbours of a row of out
     const bool fours = size % 4 == 0 && ldy % 4 == 0 && ldz % 4 == 0 && ldo % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)z % 16 == 0 &&
                        (uintptr_t)w % 16 == 0 && (uintptr_t)out % wide == 0;
-    // few rows: four elements a thread, as far as a workgroup has threads (nothing else fills the chip); many: sixteen
+    // Few rows: four elements a thread, as far as a workgroup has threads (nothing else fills the chip); many: sixteen.  us, four
+    // and sixteen: rows of 4,096 256 of them 4.3 and 5.2, 512 6.8 and 6.5; of 2,048 256 3.4 and 3.8, 1,024 6.2 and 5.9; of 8,192
+    // 512 12.8 and 13.4, 1,024 21.6 and 20.9; of 20,000 512 26.4 and 31.8.
     int threads = size <= 256 ? 64 : size <= 1024 ? 128 : 256;
-    if (fours && (long)N * parts <= 512 && size > 1024) threads = size >= 4096 ? 1024 : (size / 4 + 63) / 64 * 64;
+    if (fours && (long)N * parts <= (size >= 8192 ? 512 : 256) && size > 1024) threads = size >= 4096 ? 1024 : (size / 4 + 63) / 64 * 64;
 #define GROUP_NORM_GO(T_, V_) gated_group_norm_kernel<T_, V_><<<N * parts, threads, 0, stream>>>(y, ldy, z, ldz, w, (T_*)out, ldo, parts, size, eps)
     if (dtype == AGAVE_F32) {
         if (fours) GROUP_NORM_GO(float, 4); else GROUP_NORM_GO(float, 1);

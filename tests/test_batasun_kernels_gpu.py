@@ -468,3 +468,21 @@ def test_a_model_of_one_layer(name, dtype):
     for piece in (2, 3):
         eng.prefill_chunk = piece
         near(U.run_whole(eng, toks[:67]), ref[:67], f"pieces of {piece}")
+
+
+@pytest.mark.parametrize("n,parts,size", [(256, 1, 4096), (257, 1, 4096), (1, 1, 4100), (128, 2, 1028), (3, 1, 1030), (512, 1, 8196),
+                                          (513, 1, 8192), (2, 1, 20000), (2, 3, 64)])
+def test_group_norm_of_few_and_of_many_rows(n, parts, size):
+    """Either side of the line between a workgroup of many threads and one of few, rows longer than a workgroup keeps, rows whose
+    sizes are no multiple of four."""
+    from agave_amd.ops import sequence as S
+    g = torch.Generator().manual_seed(n + size)
+    y, z = (torch.randn(n, parts * size, generator=g).to(DEV) for _ in range(2))
+    w = (torch.rand(parts * size, generator=g) + 0.5).to(DEV)
+    out = torch.full_like(y, float("nan"))
+    S.gated_group_norm(y, z, w, out, parts, 1e-5)
+    gated = (y.double() * z.double() * torch.sigmoid(z.double())).view(n, parts, size)
+    ref = (gated / (gated.square().mean(-1, keepdim=True) + 1e-5).sqrt()).view(n, -1) * w.double()
+    # every output: some 12 roundings of its own, and half the relative error of a sum of positive numbers in which none passes
+    # through more than 100 additions (80 in a thread, 16 at most across them)
+    assert float(((out.double() - ref).abs() / ref.abs().clamp_min(1e-30)).max()) <= (12 + 50) * 2.0 ** -24
