@@ -303,7 +303,10 @@ extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, l
                 splits, MOST_SPLITS);
     AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "attn_plain: unknown dtype %d", dtype);
     if (N == 0) return 0;
-    // neighbouring tokens share a page's keys where there are enough of them to fill the compute units without
+    // Neighbouring tokens share a page's keys where there are enough of them to fill the compute units without.  us, a token a
+    // workgroup and several, 32-bit: 16 heads of 128 over 4, 64 tokens (256 workgroups) 10.5 and 11.2, 96 tokens 18.1 and 16.2, 421
+    // tokens 99 and 47; 8 heads of 256 over 4, 64 tokens 14.1 and 15.8, 96 tokens 27.3 and 24.5; 4 heads of 64 over one, 256
+    // tokens 17.6 and 18.1, 300 tokens 22.4 and 20.9; 8 heads of 64 over 8, 64 tokens (512 workgroups) 8.4 and 8.8, 96 tokens 13.2 and 11.9.
     const int G = nh / nkv, run = one_token_each || G >= ROWS || (long)N * nkv <= COMPUTE_UNITS ? 1 : ROWS / G;
     if (dtype == AGAVE_F32)
         launch_type<float>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
