@@ -91,22 +91,28 @@ def combine(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: to
                  lds, ptr(shared_gate) if shared is not None else None, ptr(out), ldo, n, top, n_experts, hidden, stream())
 
 
+STREAMED = (1024, 2048, 4096)        # columns for which the kernel of few pairs is built
+
+
 def tile_plan(n_pairs: int, n_experts: int, tile_order: bool = False, ff: int = 0, hidden: int = 0):
     """(rows a tile, tiles at most, sorted rows at most) of the sorted list of ``n_pairs`` pairs; every expert's run of rows
     is padded to whole tiles, so there are at most ``ceil(pairs / rows) + experts`` tiles.
 
     Weights row by row: tiles of 64 rows where an expert gets some 32 pairs or more on average, of 16 otherwise.
     Weights in tile order (``tile_order``, experts of ``ff`` inner rows and ``hidden`` columns): 128 from 128 pairs an expert
-    on; 64 from four pairs an expert on (two where tiles of 16 have no kernel that streams the sizes) where their workgroups (64 inner rows, 128 columns each) about fill the chip; below
-    that 16.  Measured with 16 experts of 2,048 by 2,048, both products: 16 pairs 60 us in tiles of 16 and 73 in tiles of 64,
-    32 pairs 82 and 83, 64 pairs 85 and 87, 128 pairs 95 and 89; 1,600 pairs 124 us in tiles of 64 and 125 in tiles of 128, 2,400 pairs 162
-    and 137."""
+    on; 64 from 16 pairs an expert on where their workgroups (64 inner rows, 128 columns each) about fill the chip; below that
+    16.  Where neither product has the columns that the kernel of few pairs streams, 64 from two pairs an expert on.  us, both
+    products in tiles of 16 and of 64: 16 experts of 2,048 by 2,048 4 pairs an expert 85 and 89, 8 87 and 88, 12 90 and 89, 16 114
+    and 91; 64 of 512 by 2,048 4 88 and 101, 12 100 and 104, 16 112 and 106; 32 of 1,024 by 1,024 8 49 and 53, 16 63 and 54; 16 of
+    1,536 by 1,536 2 63 and 57, 16 91 and 60.  With workgroups for a part of the chip: 8 of 512 by 512 16 12 and 20, 4 of 2,048 by 1,024
+    16 23 and 34.  In tiles of 64 and of 128, 16 experts of 2,048 by 2,048: 100 pairs an expert 124 and 125, 150 162 and 137."""
     tm = 64 if n_pairs >= 32 * n_experts else 16
     if tile_order:
         live = min(n_pairs, n_experts)
         if n_pairs >= 128 * n_experts:
             tm = 128
-        elif n_pairs >= (4 if ff in (1024, 2048, 4096) and hidden in (1024, 2048, 4096) else 2) * n_experts and live * (ff // 64) >= 256 and live * (hidden // 128) >= 128:
+        elif (n_pairs >= (16 if ff in STREAMED or hidden in STREAMED else 2) * n_experts
+              and live * (ff // 64) >= 256 and live * (hidden // 128) >= 128):
             tm = 64
     tiles = (n_pairs + tm - 1) // tm + n_experts
     return tm, tiles, tiles * tm
