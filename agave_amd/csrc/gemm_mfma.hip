@@ -1027,29 +1027,26 @@ extern "C" int agave_gemm_oproj_combine(const float* part_o, const float* part_m
 typedef __attribute__((address_space(3))) u32x4_t tl_lds_u32x4;
 
 
-template <int WT, int KT, int NS, int EPI, typename TC, int NWV, int TT, bool TURNS, int WNV>
+template <int WT, int KT, int NS, int EPI, typename TC, int NWV, int TT, bool TURNS>
 __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __restrict__ X, long ldx,
                                                          const uint4* __restrict__ Wp, TC* __restrict__ Y, long ldy,
                                                          int M, int N, int K, int KB, int NB, int NBS, long part_stride, GateForm F) {
     // NBS: row blocks of the whole packed matrix (Wp may point at a later row block of it)
     constexpr int CPR = KT * 4;                       // 16-byte pieces per staged token row
     constexpr int RP = 16 / CPR;                      // token rows per 256 bytes of LDS
-    constexpr int WTILES = 2 * WNV * WT;              // packed 16-row weight tiles per workgroup (WNV waves side by side, 32 WT rows each)
+    constexpr int WTILES = 4 * WT;                    // packed 16-row weight tiles per workgroup
     constexpr int X_BYTES = TT * KT * 64, W_BYTES = WTILES * KT * 1024;      // TT tokens per workgroup
     constexpr int STAGE_BYTES = X_BYTES + W_BYTES;
-    constexpr int XB = (TT / 32) / (NWV / WNV);       // 32-token tiles per wave
-    static_assert(XB >= 1 && XB * (NWV / WNV) * 32 == TT, "the waves' token tiles must cover the workgroup's tokens");
-    constexpr int X_CHUNKS = X_BYTES / 1024;
-    constexpr int X_LOADS = (X_CHUNKS + NWV - 1) / NWV, W_LOADS = W_BYTES / 1024 / NWV;   // per wave and stage
+    constexpr int XB = (TT / 32) / (NWV / 2);         // 32-token tiles per wave
+    static_assert(XB >= 1 && XB * (NWV / 2) * 32 == TT, "the waves' token tiles must cover the workgroup's tokens");
+    constexpr int X_LOADS = X_BYTES / 1024 / NWV, W_LOADS = W_BYTES / 1024 / NWV;     // per wave and stage
     static_assert(NWV == 4 || NWV == 8, "four or eight waves");
-    // (192 tokens are one load and a half a wave: the last waves load the first ones' pieces a second time, the same bytes to the
-    // same place, so that every wave has as many loads on their way)
-    static_assert(X_CHUNKS * 1024 == X_BYTES && W_LOADS * NWV * 1024 == W_BYTES, "whole loads per wave");
+    static_assert(X_LOADS * NWV * 1024 == X_BYTES && W_LOADS * NWV * 1024 == W_BYTES, "whole loads per wave");
     constexpr int LOADS = X_LOADS + W_LOADS;
     static_assert(NS >= 2, "a stage is loaded while another is multiplied");
     extern __shared__ __attribute__((aligned(16))) unsigned char tl_lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int wn = wave % WNV, wm = wave / WNV;
+    const int wn = wave & 1, wm = wave >> 1;
     const int nbw = blockIdx.x * WTILES;                  // first packed weight tile of this workgroup
     const int m0 = blockIdx.y * TT;                       // first token of this workgroup
     // gridDim.z workgroups share a tile's columns: each takes a run of stages and leaves its sum
@@ -1076,7 +1073,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
     const int st_last = n_stage_all - 1;                               // the stage that may hold columns past K
 #pragma unroll
     for (int i = 0; i < X_LOADS; ++i) {
-        const int o = (((wave * X_LOADS + i) % X_CHUNKS) * 64 + lane); // 16-byte slot in the stage
+        const int o = ((wave * X_LOADS + i) * 64 + lane);              // 16-byte slot in the stage
         const int row = o / CPR, pos = o % CPR;                        // LDS row and position this lane's piece lands in
         const int piece = pos ^ ((row / RP) % CPR);                    // which 8 columns of that row it holds
         int mrow = row;
@@ -1095,7 +1092,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
             const unsigned char* src = xbase + (size_t)ste * (KT * 64);
             const unsigned off = ste == st_last ? xoff_last[i] : xoff[i];
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + off),
-                                             (__attribute__((address_space(3))) void*)(buf + ((wave * X_LOADS + i) % X_CHUNKS) * 1024), 16, 0, 0);
+                                             (__attribute__((address_space(3))) void*)(buf + (wave * X_LOADS + i) * 1024), 16, 0, 0);
         } else {
             const int tt = wave * W_LOADS + (i - X_LOADS);             // tile: row tile tt / KT, k-step tt % KT
             int nb = nbw + tt / KT, kb = ste * KT + tt % KT;
@@ -1242,7 +1239,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
     // now, and leaves it row by row: 16 bytes a lane, whole lines.  The 16-byte pieces of a row are
     // permuted by the token so that the 32 tokens of a store into LDS fall into different banks.
     constexpr int ES = (int)sizeof(TC);
-    constexpr int OUT_COLS = EPI == 0 ? WTILES * 16 : WTILES * 8;     // columns of Y this workgroup computes
+    constexpr int OUT_COLS = EPI == 0 ? WT * 64 : WT * 32;            // columns of Y this workgroup computes
     constexpr int ROW_BYTES = OUT_COLS * ES, CH = ROW_BYTES / 16;     // 16-byte pieces per row
     constexpr bool VIA_LDS = TT * ROW_BYTES <= NS * STAGE_BYTES && CH >= 1 && CH <= 64;
     const int n_base = EPI == 0 ? nbw * 16 : nbw * 8;
@@ -1323,21 +1320,21 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
     }
 }
 
-template <int WT, int KT, int NS, int EPI, typename TC, int NWV, int TT, bool TURNS, int WNV = 2>
+template <int WT, int KT, int NS, int EPI, typename TC, int NWV, int TT, bool TURNS>
 static int launch_tiled(const void* X, long ldx, const void* Wp, void* Y, long ldy, int M, int N, int K, int KB, int NB,
                         const GateForm& F, hipStream_t stream, int splits = 1, long part_stride = 0, int NBS = 0) {
-    constexpr int WTILES = 2 * WNV * WT;
+    constexpr int WTILES = 4 * WT;
     const size_t lds = (size_t)NS * (TT * KT * 64 + WTILES * KT * 1024);
     dim3 grid((NB + WTILES - 1) / WTILES, (M + TT - 1) / TT, splits);
     AGAVE_CHECK(grid.y <= 65535, "gemm_tiled: M=%d exceeds the grid limit", M);
     static bool raised = false;
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiled_kernel<WT, KT, NS, EPI, TC, NWV, TT, TURNS, WNV>,
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiled_kernel<WT, KT, NS, EPI, TC, NWV, TT, TURNS>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         AGAVE_CHECK(e == hipSuccess, "gemm_tiled: cannot raise the LDS allowance");
         raised = true;
     }
-    gemm_tiled_kernel<WT, KT, NS, EPI, TC, NWV, TT, TURNS, WNV><<<grid, NWV * 64, lds, stream>>>((const bf16*)X, ldx, (const uint4*)Wp, (TC*)Y, ldy,
+    gemm_tiled_kernel<WT, KT, NS, EPI, TC, NWV, TT, TURNS><<<grid, NWV * 64, lds, stream>>>((const bf16*)X, ldx, (const uint4*)Wp, (TC*)Y, ldy,
                                                                       M, N, K, KB, NB, NBS > 0 ? NBS : NB, part_stride, F);
     return 0;
 }
@@ -1359,7 +1356,7 @@ static int dispatch_tiled(const void* X, long ldx, const void* Wp, void* Y, long
     // The largest tile that still gives some 160 workgroups (a larger tile reads a third less from
     // L2 per flop, which outweighs idle compute units down to about that number); with few tokens
     // or few rows none does, and the tile with the most workgroups is taken.
-    //   256 x 256, 128 x 256, 128 x 128, 64 x 128 (weight rows x tokens); 256 x 192 below
+    //   256 x 256, 128 x 256, 128 x 128, 64 x 128 (weight rows x tokens)
     const long rows16 = (NB + 15) / 16, rows8 = (NB + 7) / 8, rows4 = (NB + 3) / 4;
     const long t256 = (M + 255) / 256, t128 = (M + 127) / 128;
     const long wgs[4] = {rows16 * t256, rows8 * t256, rows8 * t128, rows4 * t128};
@@ -1371,15 +1368,6 @@ static int dispatch_tiled(const void* X, long ldx, const void* Wp, void* Y, long
         for (int i = 1; i < 4; ++i)
             if (wgs[i] > wgs[pick]) pick = i;
     }
-    // 256 x 192 tiles where they come to one round of the 256 compute units with a third more workgroups than 256 x 256 tiles, so
-    // that next to none of the chip is idle (the two tilings' sums are the same bits).  us, 256-token tiles and these: gate/up of
-    // 10,240 x 2,560 400 rows 69.5 and 59.6, 509 72.5 and 64.7; 8,192 x 2,560 1,345 rows 62.8 and 59.1, 1,536
-    // 69.2 and 67.5.  With fewer workgroups than that it is now this side, now the other (1,300 rows of 8,192 63.1 and 65.4; 900 of
-    // gate/up 5,376 x 2,048 51.3 and 46.7; 2,100 of 5,000 x 1,544 42.8 and 51.2), with more than one round these lose (gate/up of
-    // 10,240: 600 rows 72.6 and 97.5, 1,024 107 and 120).
-    const long wide = rows16 * ((M + 191) / 192);
-    if (pick == 0 && wide <= 256 && 3 * wide >= 4 * wgs[0])
-        return launch_tiled<2, 1, 5, EPI, TC, 8, 192, true, 4>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
     // up to 128 tokens would leave half of a 256-token tile empty: tiles of 128 tokens (a step of 65
     // to 128 tokens 3 to 5 % faster)
     if (pick <= 1 && M <= 128) pick = 2;
@@ -1575,14 +1563,13 @@ static int launch_tile_shape(int tile, const void* X, long ldx, const void* Wp, 
         case 0: return launch_tiled<4, 1, 4, EPI, TC, 8, 256, true>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
         case 1: return launch_tiled<2, 2, 3, EPI, TC, 8, 256, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
         case 2: return launch_tiled<2, 2, 3, EPI, TC, 8, 128, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-        case 4: return launch_tiled<2, 1, 5, EPI, TC, 8, 192, true, 4>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
         default: return launch_tiled<1, 2, 4, EPI, TC, 8, 128, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
     }
 }
 
 extern "C" int agave_gemm_tiled_as(const void* X, long ldx, const void* Wp, int dt_y, void* Y, long ldy, int M, int N,
                                    int K, int epilogue, float act_a, float act_b, float act_limit, float act_shift, const float* gate_b, const float* up_b, int tile, hipStream_t stream) {
-    AGAVE_CHECK(M > 0 && N > 0 && K > 0 && tile >= 0 && tile <= 4, "gemm_tiled_as: bad sizes M=%d N=%d K=%d or tile %d", M, N, K, tile);
+    AGAVE_CHECK(M > 0 && N > 0 && K > 0 && tile >= 0 && tile <= 3, "gemm_tiled_as: bad sizes M=%d N=%d K=%d or tile %d", M, N, K, tile);
     AGAVE_CHECK(K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)X % 16) == 0,
                 "gemm_tiled_as: X must be 16-byte aligned with K and its row stride multiples of 8 (K=%d ldx=%ld)", K, ldx);
     AGAVE_CHECK(ldx >= K && ldy >= N && ldx < (1L << 22), "gemm_tiled_as: bad row strides");

@@ -1083,30 +1083,6 @@ def test_gemm_tiled_every_tile_shape_in_slices(G, tile, m, n, k, z):
     assert float((whole.double().cpu() - ref).abs().max()) <= 6e-3 * float(ref.abs().max())
 
 
-@pytest.mark.parametrize("m,n,k,epilogue", [
-    (1153, 8185, 200, 0),       # 224 tiles of 256 x 192, one row in the last of them; ragged weight rows and columns
-    (1536, 8192, 40, 0),        # 256 of them, all full, two stages
-    (385, 10233, 72, 1),        # 240, gate and up
-    (512, 10240, 32, 1),        # 240, a single stage
-    (576, 10240, 32, 1),        # 240, all full, but as many of 256 x 256
-    (1300, 8192, 64, 0),        # 224, but not a third more than the 192 of 256 x 256: those are taken
-    (193, 200, 1000, 0)])       # next to none: small tiles
-def test_gemm_tiled_of_192_tokens(G, m, n, k, epilogue):
-    """Tiles of 256 weight rows and 192 tokens add up in the order of the others: the same bits as tiles of 256 x 256, whichever
-    the library takes by itself."""
-    g = torch.Generator().manual_seed(m + n + k)
-    x = torch.randn(m, k, generator=g).bfloat16().to(DEV)
-    w = (torch.randn(n * (1 + epilogue), k, generator=g) * 0.1).bfloat16().to(DEV)
-    packed = G.pack_weight(w, interleave_ff=n if epilogue else 0)
-    own, wide, square = (torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(3))
-    G.product(x, packed, own, n, epilogue=epilogue)
-    G.tiled_as(x, packed, wide, n, 4, epilogue=epilogue)
-    G.tiled_as(x, packed, square, n, 0, epilogue=epilogue)
-    assert torch.equal(wide, square) and not bool(wide.isnan().any())
-    assert torch.equal(own, square) or (n == 200 and float((own.float() - square.float()).abs().max())
-                                        <= 2.0 ** -7 * float(square.float().abs().max()))     # (slices of columns may round the other way)
-
-
 @pytest.mark.parametrize("m,ff,k", [(70, 192, 64), (513, 1000, 96), (256, 20, 40), (1024, 5120, 1000), (2048, 10236, 64),
                                     (1024, 10236, 64)])
 def test_gemm_tiled_geglu(G, m, ff, k):
