@@ -221,7 +221,9 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
     }
 }
 
-// The results that a row's workgroups left: a workgroup per (token, head).
+// The results that a row's workgroups left: a workgroup per (token, head).  A share without a key holds zeros and counts as
+// such.  One whose scores are all not a number has no maximum either, but a sum and results that are not numbers: it goes into
+// the row's as any other, so that a row comes out as it does from one workgroup.
 template <typename T>
 __global__ __launch_bounds__(128) void attn_plain_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                                T* __restrict__ out, long ldo, int nh, int hd, int splits) {
@@ -239,7 +241,7 @@ __global__ __launch_bounds__(128) void attn_plain_merge_kernel(const float* __re
         float sum = 0.f;
 #pragma unroll
         for (int s = 0; s < MOST_SPLITS; ++s)
-            if (s < splits && f[s] != 0.f) sum = fmaf(part_o[(row * splits + s) * hd + d], f[s], sum);
+            if (s < splits) sum = fmaf(part_o[(row * splits + s) * hd + d], f[s], sum);
         st(out + (row / nh) * ldo + (row % nh) * hd + d, sum * inv);
     }
 }

@@ -406,6 +406,51 @@ def test_attn_plain_values_that_are_not_finite(K):
     assert torch.allclose(out[~bad], want[~bad], atol=1e-6, rtol=1e-5)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("spoil", ["query", "page", "key of no weight", "value"])
+def test_attn_plain_rows_that_are_not_a_number(K, dtype, spoil):
+    """A token whose query, or a key or value that it sees, is not a number: its heads' results say so, with one workgroup to a
+    row and with several, also where a share of its pages has no other score or no weight; all other rows stay as they are."""
+    from agave_amd.parts import Workspace
+    nh, nkv, hd, B, ctx = 4, 2, 40, 2, 330
+    g = torch.Generator().manual_seed(5)
+    kp, vp = (torch.randn(6 * B, nkv, *shape, generator=g).to(dtype).to(DEV) for shape in ((64, hd), (hd, 64)))
+    q = torch.randn(B, nh * hd, generator=g).to(dtype).to(DEV)
+    table = torch.arange(6 * B, dtype=torch.int32, device=DEV).view(B, 6)
+    hit = torch.zeros(B, nh, hd, dtype=torch.bool, device=DEV)
+
+    def both():
+        outs = []
+        for more in ({}, {"span": 6, "workspace": Workspace(torch.device(DEV))}):
+            out = torch.empty_like(q)
+            K.attn_plain(q, out, kp, vp, table, _i32([0] * B), _i32(list(range(B))), _i32([ctx - 1] * B), nh, nkv, hd, 0.2, None,
+                         one_token_each=True, **more)
+            outs.append(out.view(B, nh, hd))
+        return outs
+    if spoil == "key of no weight":           # (page 4's scores exceed all others by some 300: nothing else has a weight)
+        kp[4, 0] = 0.0
+        kp[4, 0, :, 0] = 300.0 / 0.2
+        q.view(B, nh, hd)[0, :2, 0] = 1.0
+    want = both()
+    if spoil == "query":
+        q.view(B, nh, hd)[0, 1] = float("nan")
+        hit[0, 1] = True
+    elif spoil == "page":                     # (every score of one share)
+        kp[2, 0] = float("nan")
+        hit[0, :2] = True
+    elif spoil == "key of no weight":
+        kp[1, 0, 7] = float("nan")
+        hit[0, :2] = True
+    else:
+        vp[1, 1, 3, 7] = float("nan")
+        hit[0, 2:, 3] = True
+    for got, ref in zip(both(), want):
+        assert torch.equal(got.isnan(), hit)
+        # (values that are not finite are summed element by element, in another order than the matrix cores')
+        tol = dict(atol=1e-6, rtol=1e-5) if dtype == torch.float32 else dict(atol=1e-2, rtol=1e-2)
+        assert torch.allclose(got[~hit], ref[~hit], **tol)
+
+
 def test_attn_plain_far_key_wins(K):
     # among 700 keys, key 3 is made to dominate the last query's softmax: the output must be its value
     got, ref, vs = _attn_case(K, torch.float32, 2, 1, 32, [700], None, 0.5, seed=1, boost=3)
