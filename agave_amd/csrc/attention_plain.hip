@@ -38,13 +38,13 @@ __device__ __forceinline__ float lanes16_sum(float v) {
 // several sequences in one workgroup (any tok_seq is taken) go one sequence after another.
 // gridDim.y workgroups share a row's pages and leave (sum, maximum, unnormalised result) for attn_plain_merge_kernel: with a
 // token per sequence there are few rows and the pages one after another bound the time.
-// NT: tiles of 64 value elements (16 a wave).  A probability of 0 must not meet a value that is not finite (a key behind a
+// NT: tiles of 64 value elements (16 a wave).  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of 0 must not meet a value that is not finite (a key behind a
 // token's position may hold anything): such pages are summed element by element.
 // Bound by the 32-bit products (half of them for a token of 4 rows' padding) and, with few tokens, by the loads' way from memory.
 // Measured, 16 heads on 4 key heads of 128 in 32 bits: prompts of 97, 259 and 421 tokens 63 us (a workgroup per token and head, a
 // key a thread: 943 us), 2,000 tokens 0.45 ms (16.8 ms); a token each behind as many keys 15 us (59 us), behind 4,000 keys
 // 33 us (562 us).  Errors against 64 bits are half as large (2.0 to 2.8e-7 after 4.2 to 5.5e-7).
-template <typename T, int NT, bool VEC>
+template <typename T, int NT, bool VEC, bool VEC_V>
 __global__ __launch_bounds__(256) void attn_plain_kernel(
     const T* __restrict__ q, long ldq, T* __restrict__ out, long ldo, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ table, int width, const int* __restrict__ base,
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
             auto values = [&](f32x4_t (&v)[4], int nt) {
                 const T* row = vr + (size_t)min((4 * nt + w) * 16 + r, hd - 1) * AGAVE_PAGE;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = ld4<true>(row, 16 * j + 4 * g, AGAVE_PAGE);
+                for (int j = 0; j < 4; ++j) v[j] = ld4<VEC_V>(row, 16 * j + 4 * g, AGAVE_PAGE);
             };
             if constexpr (V_AHEAD)
 #pragma unroll
@@ -252,13 +252,14 @@ static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages
                         int window, int run, int splits, float* part_o, float* part_ml, hipStream_t stream) {
     const int chunks = (nh / nkv + ROWS - 1) / ROWS;
     const dim3 grid((N + run - 1) / run * nkv * chunks, splits);
-    const bool vec = hd % 4 == 0 && ldq % 4 == 0 && (uintptr_t)k_pages % (4 * sizeof(T)) == 0 && (uintptr_t)q % (4 * sizeof(T)) == 0;
-    if (vec)
-        attn_plain_kernel<T, NT, true><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq,
-                                                                 tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml);
-    else
-        attn_plain_kernel<T, NT, false><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq,
-                                                                  tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml);
+    // four elements at a time where rows are aligned to as many (a value row is a page long, so its pages' start decides)
+    const uintptr_t wide = 4 * sizeof(T);
+    const bool vec_v = (uintptr_t)v_pages % wide == 0;
+    const bool vec = vec_v && hd % 4 == 0 && ldq % 4 == 0 && (uintptr_t)k_pages % wide == 0 && (uintptr_t)q % wide == 0;
+#define PLAIN_GO(VEC_, VEC_V_) attn_plain_kernel<T, NT, VEC_, VEC_V_><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, width, \
+        base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml)
+    if (vec) PLAIN_GO(true, true); else if (vec_v) PLAIN_GO(false, true); else PLAIN_GO(false, false);
+#undef PLAIN_GO
     if (splits > 1) attn_plain_merge_kernel<T><<<N * nh, 128, 0, stream>>>(part_o, part_ml, out, ldo, nh, hd, splits);
 }
 
@@ -299,7 +300,6 @@ extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, l
     AGAVE_CHECK(window >= 0, "attn_plain: negative window");
     AGAVE_CHECK(q && out && k_pages && v_pages && table && base && tok_seq && tok_pos && width > 0 && n_pages > 0,
                 "attn_plain: null buffer or empty table");
-    AGAVE_CHECK((uintptr_t)v_pages % 16 == 0, "attn_plain: value pages must be aligned to 16 bytes");
     AGAVE_CHECK((long)N * nh < 2147483647L, "attn_plain: too many (token, head) pairs");
     AGAVE_CHECK(splits >= 1 && splits <= MOST_SPLITS && (splits == 1 || (part_o && part_ml)), "attn_plain: %d splits (1 to %d, with buffers for what they leave)",
                 splits, MOST_SPLITS);

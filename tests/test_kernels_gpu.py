@@ -451,6 +451,30 @@ def test_attn_plain_rows_that_are_not_a_number(K, dtype, spoil):
         assert torch.allclose(got[~hit], ref[~hit], **tol)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hd,k_at,v_at", [(40, 0, 1), (40, 0, 4), (40, 1, 0), (34, 0, 2), (300, 3, 3)])
+def test_attn_plain_pages_at_any_element(K, dtype, hd, k_at, v_at):
+    """Pages that begin at any element of a buffer give the results of aligned ones, in prompts and decode steps."""
+    from agave_amd.parts import Workspace
+    nh, nkv, n = 4, 2, 150
+    g = torch.Generator().manual_seed(hd + k_at)
+    kp, vp = (torch.randn(3, nkv, *shape, generator=g).to(dtype).to(DEV) for shape in ((64, hd), (hd, 64)))
+    q = torch.randn(n, nh * hd, generator=g).to(dtype).to(DEV)
+
+    def moved(x, at):
+        return torch.zeros(x.numel() + at, dtype=dtype, device=DEV)[at:].view(x.shape).copy_(x)
+    table = _i32([[0, 1, 2]])
+    outs = []
+    for k, v in ((kp, vp), (moved(kp, k_at), moved(vp, v_at))):
+        out = torch.empty_like(q)
+        K.attn_plain(q, out, k, v, table, _i32([0]), _i32([0] * n), _i32(list(range(n))), nh, nkv, hd, 0.2, None)
+        last = torch.empty_like(q[-1:])
+        K.attn_plain(q[-1:], last, k, v, table, _i32([0]), _i32([0]), _i32([n - 1]), nh, nkv, hd, 0.2, None, one_token_each=True,
+                     span=3, workspace=Workspace(torch.device(DEV)))
+        outs.append(torch.cat([out, last]))
+    assert bool(outs[0].isfinite().all()) and torch.equal(outs[0], outs[1])
+
+
 def test_attn_plain_far_key_wins(K):
     # among 700 keys, key 3 is made to dominate the last query's softmax: the output must be its value
     got, ref, vs = _attn_case(K, torch.float32, 2, 1, 32, [700], None, 0.5, seed=1, boost=3)
