@@ -1002,7 +1002,9 @@ __global__ __launch_bounds__(TT * 4, 4) void routed_product_tiled_kernel(const b
     __builtin_amdgcn_s_waitcnt(0x0F70);                           // loads past the last stage must have landed before LDS is used again
 
     // acc[a][b]: row 16 b + c of the wave's rows, columns 4 g .. 4 g + 3 of operand a.  Half of the tile's rows at a time go
-    // through LDS and leave it row by row, 16 bytes a lane in whole lines.
+    // through LDS and leave it row by row, 16 bytes a lane in whole lines (the 32-bit rows may begin at any element: in
+    // single ones where that is off 16 bytes; the inner rows are aligned, the host has seen to it).
+    const bool whole = ((uintptr_t)out_ & 15) == 0;
     constexpr int ES = GATED ? 2 : 4, ROW_BYTES = COLS * ES, CH = ROW_BYTES / 16, SWZ = (CH < 32 ? CH : 32) - 1;
     static_assert((TT / 2) * ROW_BYTES <= NS * STAGE, "half of the finished tile fits the LDS");
 #pragma unroll
@@ -1035,7 +1037,13 @@ __global__ __launch_bounds__(TT * 4, 4) void routed_product_tiled_kernel(const b
             const int col = col0 + piece * (16 / ES);
             if (col >= n_out) continue;                           // (n_out is a multiple of 16: a piece is inside or outside)
             const uint4 v = *reinterpret_cast<const uint4*>(rt_lds + t * ROW_BYTES + ((piece ^ (t & SWZ)) << 4));
-            *reinterpret_cast<uint4*>((unsigned char*)out_ + ((size_t)(row0 + half * (TT / 2) + t) * n_out + col) * ES) = v;
+            unsigned char* dst = (unsigned char*)out_ + ((size_t)(row0 + half * (TT / 2) + t) * n_out + col) * ES;
+            if (GATED || whole) {
+                *reinterpret_cast<uint4*>(dst) = v;
+            } else {
+                unsigned* one = reinterpret_cast<unsigned*>(dst);
+                one[0] = v.x; one[1] = v.y; one[2] = v.z; one[3] = v.w;
+            }
         }
     }
 }

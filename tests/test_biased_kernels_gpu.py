@@ -561,3 +561,26 @@ def test_route_sort_of_few_pairs(P, E, chosen, tm):
     assert sum(r >= 0 for r in sorted_pair) == len(real) and set(sorted_pair) <= set(range(P)) | {-1}
     want = [e for e in range(E) for _ in range((real.count(e) + tm - 1) // tm)]
     assert tile_expert == want + [-1] * (tiles - len(want))
+
+
+@pytest.mark.parametrize("tm", [16, 64, 128])
+def test_routed_rows_at_any_element(tm):
+    """The experts' 32-bit rows may begin at any element of a buffer: the same rows, and nothing beside them is written."""
+    from agave_amd.ops import routed
+    n, E, top, ff, hidden = 150, 3, 2, 128, 160
+    g = torch.Generator().manual_seed(tm)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * s[-1] ** -0.5).bfloat16().to(DEV)
+    x, w = torch.randn(n, hidden, generator=g).bfloat16().to(DEV), [routed.pack_expert_weights(rnd(*s)) for s in ((E, ff, hidden), (E, ff, hidden), (E, hidden, ff))]
+    choice = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(n)]).int().view(-1).to(DEV)
+    tiles = (n * top + tm - 1) // tm + E
+    place, sorted_pair, tile_expert = (torch.full((k,), -7, dtype=torch.int32, device=DEV) for k in (n * top, tiles * tm, tiles))
+    routed.route_sort(choice, E, tm, tiles, place, sorted_pair, tile_expert)
+    rows = []
+    for at in range(4):
+        held = torch.full((tiles * tm * hidden + 8,), 7.0, device=DEV)
+        y = held[at:at + tiles * tm * hidden].view(tiles * tm, hidden)
+        routed.experts_mfma(x, sorted_pair, tile_expert, *w, torch.empty(tiles * tm, ff, dtype=torch.bfloat16, device=DEV), y, tm, tiles, top, 1,
+                            tile_order=True)
+        assert bool((held[:at] == 7.0).all()) and bool((held[at + y.numel():] == 7.0).all())
+        rows.append(y[place.long()])
+    assert all(torch.equal(r, rows[0]) for r in rows) and bool(torch.isfinite(rows[0]).all())
