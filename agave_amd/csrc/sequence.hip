@@ -1188,10 +1188,11 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
             bool finite = true;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                Vt[buf][vc + e][vt] = cur.v[e];
-                finite = finite && fabsf(cur.v[e]) < INFINITY;
+                const float v = vt < n ? cur.v[e] : 0.f;        // (behind the sequence's end: nothing, also where its last value is infinite)
+                Vt[buf][vc + e][vt] = v;
+                finite = finite && fabsf(v) < INFINITY;
             }
-            if (!finite && vt < n) odd[ch % 3] = 1;
+            if (!finite) odd[ch % 3] = 1;
             if (tid == 0) odd[(ch + 1) % 3] = 0;                // (last read two chunks ago, written next behind the barrier below)
             if (w == 0) Dc[buf][lane] = cur.cum;
             lds_barrier();
@@ -1277,8 +1278,13 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
         ask(cur, r0);
         for (int ch = 0; ch < n_chunks; ++ch) {
             const int t0 = r0 + ch * SSD_CHUNK, n = min(SSD_CHUNK, r1 - t0), buf = ch & 1;
-            // (rows behind the sequence's end repeat its last one and count nothing)
+            // (rows behind the sequence's end repeat its last one: they count nothing, whatever it holds)
             made[buf][w][lane] = lane < n ? cur.made : 0.f;
+            if (n < SSD_CHUNK)
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+#pragma unroll
+                    for (int f = 0; f < KF; ++f) cur.b[j][f] = 16 * (j >> 2) + 4 * g + (j & 3) < n ? cur.b[j][f] : 0.f;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll

@@ -219,6 +219,22 @@ def test_state_space_in_chunks_at_its_ends():
         assert torch.allclose(got[~bad], ref[~bad], atol=3e-5, rtol=1e-4)
 
 
+@pytest.mark.parametrize("T", [50, 64, 150])
+@pytest.mark.parametrize("which", ["value", "key"])
+def test_state_space_in_chunks_ends_with_an_infinity(T, which):
+    """An infinite value, or an infinite element of B, in a sequence's last token: the state holds what the token wrote, an
+    infinity of the right sign in that column or key channel, also where rows behind the end fill up the chunk."""
+    def spoil(t, vec):
+        t["xs" if which == "value" else "B"][T - 1, 5] = float("inf")
+    got, S_got, (ref, S_ref) = chunked(T, [(0, T)], 2, 1, 64, 16, change=spoil)
+    odd = ~torch.isfinite(S_ref)
+    assert int(odd.sum()) == (64 if which == "value" else 32) and bool(torch.isinf(S_ref[odd]).all())
+    assert torch.equal(S_got[odd], S_ref[odd])
+    assert torch.allclose(S_got[~odd], S_ref[~odd], atol=3e-5, rtol=1e-4)
+    ref = ref.reshape(T, -1)
+    assert torch.allclose(got[:-1], ref[:-1], atol=3e-5, rtol=1e-4)
+
+
 def test_state_space_step_sizes_without_a_clamp_and_a_write_far_back():
     """Step sizes from almost nothing to dozens (softplus of -20 to 40, neither clamped); and with a decay rate of
     almost nothing what token 3 wrote is read 600 tokens later among small writes, while a fast rate forgets it."""
