@@ -15,6 +15,7 @@
 // element type of the cache pages and of the rows handed to the output product.
 #include "common_impl.h"
 #include "mfma.h"
+#include <limits.h>
 #include <math.h>
 
 #define CONV_MAX_TAPS 8
@@ -619,6 +620,7 @@ struct RecurrenceArgs {
     const int* cu; const int* slots;
     int nh, nkv, dk, dv;
     float unit_eps;                    // delta: inside the root of the unit vectors
+    int most;                          // a sequence that brings more tokens than this is another kernel's
 };
 
 // softplus by the exact functions, for the one step size a head and token has (the state-space form): what it
@@ -691,6 +693,7 @@ __global__ __launch_bounds__(512) void gated_recurrence_kernel(RecurrenceArgs A)
     const int h = blockIdx.y, s = blockIdx.z, col0 = blockIdx.x * CB;
     const int dk = A.dk, dv = A.dv;
     const int r0 = A.cu[s], r1 = A.cu[s + 1];
+    if (r1 - r0 > A.most) return;
     const int n_blocks = (r1 - r0 + TB - 1) / TB;
 
     // ---- consumers: their share of the state
@@ -1012,11 +1015,12 @@ static int launch_recurrence(const RecurrenceArgs& A, int n_seqs, hipStream_t st
     return 0;
 }
 
+// most: sequences that bring more tokens than this are left alone (agave_ssd_chunks takes them in the same step).
 extern "C" int agave_gated_recurrence(int mode, const float* q, long ldq, const float* k, long ldk, const float* v, long ldv,
                                       const float* dt, long lddt, const float* b, long ldb, const float* a_log,
                                       const float* dt_bias, const float* low, const float* f_bias, const float* skip, float* o, long ldo,
                                       float* state, const int* cu, const int* slots, int n_seqs, int nh, int nkv, int dk,
-                                      int dv, float unit_eps, int one_token_each, hipStream_t stream) {
+                                      int dv, float unit_eps, int one_token_each, int most, hipStream_t stream) {
     AGAVE_CHECK(mode == REC_DELTA || mode == REC_FORGET || mode == REC_SSD, "gated_recurrence: unknown mode %d", mode);
     AGAVE_CHECK(n_seqs >= 0 && nh > 0 && nkv > 0 && dk > 0 && dv > 0, "gated_recurrence: bad sizes B=%d nh=%d nkv=%d dk=%d dv=%d", n_seqs, nh, nkv, dk, dv);
     AGAVE_CHECK(dk <= 256, "gated_recurrence: %d key channels a head (up to 256 are supported)", dk);
@@ -1024,6 +1028,7 @@ extern "C" int agave_gated_recurrence(int mode, const float* q, long ldq, const 
     AGAVE_CHECK(q && k && v && o && state && cu && slots, "gated_recurrence: null buffer");
     AGAVE_CHECK(ldv >= (long)nh * dv && ldo >= (long)nh * dv, "gated_recurrence: a row stride is too small");
     AGAVE_CHECK(n_seqs < 65536 && nh < 65536, "gated_recurrence: too many sequences or heads");
+    AGAVE_CHECK(most >= 1, "gated_recurrence: sequences of at most %d tokens", most);
     if (mode == REC_DELTA) {
         AGAVE_CHECK(dt && b && a_log && dt_bias, "gated_recurrence: the delta rule needs dt, b, A_log and dt_bias");
         AGAVE_CHECK(ldq >= (long)nkv * dk && ldk >= (long)nkv * dk && lddt >= (long)nh * dk && ldb >= nh, "gated_recurrence: a row stride is too small");
@@ -1035,7 +1040,7 @@ extern "C" int agave_gated_recurrence(int mode, const float* q, long ldq, const 
         AGAVE_CHECK(nkv == nh && ldq >= (long)nh * dk && ldk >= (long)nh * dk, "gated_recurrence: the forget-gate form has a gate per head");
     }
     if (n_seqs == 0) return 0;
-    RecurrenceArgs A{q, ldq, k, ldk, v, ldv, dt, lddt, b, ldb, a_log, dt_bias, skip, low, f_bias, o, ldo, state, cu, slots, nh, nkv, dk, dv, unit_eps};
+    RecurrenceArgs A{q, ldq, k, ldk, v, ldv, dt, lddt, b, ldb, a_log, dt_bias, skip, low, f_bias, o, ldo, state, cu, slots, nh, nkv, dk, dv, unit_eps, most};
     if (one_token_each) {                                   // the host vouches that every sequence brings one token
         if (mode == REC_SSD) return launch_recurrence_step<REC_SSD>(A, n_seqs, stream);
         return mode == REC_DELTA ? launch_recurrence_step<REC_DELTA>(A, n_seqs, stream) : launch_recurrence_step<REC_FORGET>(A, n_seqs, stream);
@@ -1064,6 +1069,7 @@ struct SsdScratch {
     float* made;                // [4][heads][tokens]: d, from the start, to the chunk's end, to the end of the sixteen
     long n;                     // tokens
     long heads_n;               // heads * tokens
+    int least;                  // a sequence that brings fewer tokens is another kernel's
 };
 // exp of a number held in double: the argument's rounding to 32 bits would be an error of its size in units of the last place
 __device__ __forceinline__ float exp_of(double x) {
@@ -1082,7 +1088,7 @@ __device__ __forceinline__ f32x4_t ssd_total(const f32x4_t (&a)[SSD_SUMS]) {
 }
 __global__ __launch_bounds__(256) void ssd_prepare_kernel(RecurrenceArgs A, SsdScratch X) {
     const int s = blockIdx.z, r0 = A.cu[s], r1 = A.cu[s + 1], t0 = r0 + blockIdx.x * SSD_CHUNK;
-    if (t0 >= r1) return;
+    if (t0 >= r1 || r1 - r0 < X.least) return;
     const int n = min(SSD_CHUNK, r1 - t0);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if ((int)blockIdx.y < A.nkv) {
@@ -1160,7 +1166,7 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
     const bool reads = wave < 4;
     const int r0 = A.cu[s], r1 = A.cu[s + 1], grp = h / (A.nh / A.nkv);
     const int n_chunks = (r1 - r0 + SSD_CHUNK - 1) / SSD_CHUNK;
-    if (n_chunks <= 0) return;
+    if (n_chunks <= 0 || r1 - r0 < X.least) return;
     const int last = r1 - 1;
     if (tid < 3) odd[tid] = 0;
     lds_barrier();
@@ -1315,12 +1321,13 @@ __global__ __launch_bounds__(512) void ssd_chunk_kernel(RecurrenceArgs A, SsdScr
     }
 }
 
-// The state-space form in chunks, for a step in which some sequence brings many tokens (max_new: the longest).  Takes key
+// The state-space form in chunks, for a step in which some sequence brings many tokens (max_new: the longest).  Sequences of
+// fewer than `least` are left alone (agave_gated_recurrence takes them in the same step, `most` = least - 1).  Takes key
 // channels of 64 or 128 and values in blocks of 16, rows aligned to 16 bytes; agave_gated_recurrence takes the others.
 // cb: float [n_tokens][nkv][64]; cum: double [nh][n_tokens]; made: float [4][nh][n_tokens].
 extern "C" int agave_ssd_chunks(const float* q, long ldq, const float* k, long ldk, const float* v, long ldv, const float* dt, long lddt,
                                 const float* a_log, const float* dt_bias, const float* skip, float* o, long ldo, float* state,
-                                const int* cu, const int* slots, int n_seqs, int nh, int nkv, int dk, int dv, int max_new, long n_tokens,
+                                const int* cu, const int* slots, int n_seqs, int nh, int nkv, int dk, int dv, int max_new, int least, long n_tokens,
                                 float* cb, double* cum, float* made, hipStream_t stream) {
     AGAVE_CHECK(n_seqs >= 0 && nh > 0 && nkv > 0 && nh % nkv == 0 && max_new >= 0 && n_tokens >= 0, "ssd_chunks: bad sizes B=%d nh=%d nkv=%d", n_seqs, nh, nkv);
     AGAVE_CHECK((dk == 64 || dk == 128) && dv > 0 && dv % 16 == 0, "ssd_chunks: %d key channels and %d values a head (64 or 128, and a multiple of 16)", dk, dv);
@@ -1330,9 +1337,9 @@ extern "C" int agave_ssd_chunks(const float* q, long ldq, const float* k, long l
                 (uintptr_t)cb % 16 == 0 && (uintptr_t)cum % 8 == 0, "ssd_chunks: rows must be aligned to 16 bytes");
     AGAVE_CHECK(n_seqs < 65536 && nh < 65536 && nkv + (nh + 3) / 4 < 65536, "ssd_chunks: too many sequences or heads");
     if (n_seqs == 0 || max_new == 0) return 0;
-    RecurrenceArgs A{q, ldq, k, ldk, v, ldv, dt, lddt, nullptr, 0, a_log, dt_bias, skip, nullptr, nullptr, o, ldo, state, cu, slots, nh, nkv, dk, dv, 0.f};
+    RecurrenceArgs A{q, ldq, k, ldk, v, ldv, dt, lddt, nullptr, 0, a_log, dt_bias, skip, nullptr, nullptr, o, ldo, state, cu, slots, nh, nkv, dk, dv, 0.f, INT_MAX};
     const dim3 first((max_new + SSD_CHUNK - 1) / SSD_CHUNK, nkv + (nh + 3) / 4, n_seqs), second(dv / 16, nh, n_seqs);
-    const SsdScratch X{cb, cum, made, n_tokens, (long)nh * n_tokens};
+    const SsdScratch X{cb, cum, made, n_tokens, (long)nh * n_tokens, least};
     ssd_prepare_kernel<<<first, 256, 0, stream>>>(A, X);
     AGAVE_LAUNCH_CHECK("ssd_prepare");
     if (dk == 64) ssd_chunk_kernel<64><<<second, 512, 0, stream>>>(A, X);

@@ -8,6 +8,7 @@ pages and the rows handed to the output product have the engine's element type.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -23,9 +24,9 @@ kernels.register_signatures(LIBRARY, {
                                   _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "agave_talk_attention": [_I, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I,
                              _F, _I, _F, _P, _I, _P],
-    "agave_ssd_chunks": [_P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _L, _P, _P, _P, _P],
+    "agave_ssd_chunks": [_P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _L, _P, _P, _P, _P],
     "agave_gated_recurrence": [_I, _P, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _P, _P, _P, _P, _L, _P, _P, _P,
-                               _I, _I, _I, _I, _I, _F, _I, _P],
+                               _I, _I, _I, _I, _I, _F, _I, _I, _P],
     "agave_gated_group_norm": [_I, _P, _L, _P, _L, _P, _P, _L, _I, _I, _I, _F, _P],
     "agave_head_norm_gate": [_I, _P, _L, _P, _P, _L, _P, _L, _I, _I, _I, _F, _F, _P],
     "agave_scaled_sum": [_I, _P, _L, _F, _P, _L, _F, _P, _L, _I, _I, _P],
@@ -152,9 +153,10 @@ def talk_attention(q: torch.Tensor, gate: Optional[torch.Tensor], out: torch.Ten
                  n, n_heads, n_kv, dk, dv, float(scale), int(chunk or 0), float(out_scale), ptr(parts), tiles, stream())
 
 
+WHOLE_STEP = 2 ** 31 - 1
 SSD_CHUNK = 64
-# A sequence that brings this many tokens: chunks of 64 from here on, token by token below (64 heads of 64 x 128: 32 tokens
-# take 15 us token by token and 17 in chunks, 48 tokens 17 and 16, 64 tokens 19 and 17).
+# A sequence that brings fewer tokens than this is faster token by token, if it is alone (64 heads of 64 x 128: 32 tokens take
+# 14 us token by token and 17 in chunks, 48 tokens 17 and 16, 64 tokens 20 and 18).
 SSD_CHUNKS_FROM = 48
 
 
@@ -165,13 +167,46 @@ def ssd_chunks_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step, dk: i
             and all(t.data_ptr() % 16 == 0 and t.stride(0) % 4 == 0 for t in (q, k, v)))
 
 
-def _ssd_chunks(q, ldq, k, ldk, v, ldv, dt_in, lddt, a_log, dt_bias, skip, out, ldo, state, step, n_heads, n_kv, dk, dv) -> None:
+@functools.lru_cache(maxsize=256)
+def ssd_chunked_from(n_new: tuple, blocks: int, dk: int) -> int:
+    """Sequences of a step that bring at least this many tokens go through the state-space form in chunks, the others token by
+    token: 0 all of them, ``WHOLE_STEP`` none, ``SSD_CHUNKS_FROM`` the long ones in a kernel of their own.  ``n_new``: the
+    sequences' tokens; ``blocks``: blocks of 16 value columns of all heads, a workgroup each per sequence; ``dk``: key channels.
+
+    The least of three estimates in us.  Either kernel takes as long as its longest sequence, and what its workgroups take
+    beyond one to a compute unit comes on top; a workgroup of the chunks is long also for a single token.  With 128
+    channels a lone sequence of n tokens was measured at 6.5 + 0.19 n token by token and at 14.5 + 3.3 a chunk, and 256
+    workgroups beyond the first at 0.6 + 0.15 n (1.15 at least, the state's bytes) and at 4.4 + 0.024 n + 3.3 for each further chunk.
+    us, token by token, all in chunks, long ones in chunks: 64 heads of 64 x 128, 64 tokens beside 30 sequences of one
+    51, 155 and 67; 500 beside 30 of one 109, 182 and 92; 500 beside 20 of forty 209, 150 and 187; eight of 100 and eight of
+    30 169, 122 and 135; one of 65 20 and 22.  Over 175 mixtures of 2 to 128 heads the choice is at most 6 % slower than token by
+    token, over 300 batches of equal sequences at most 8 %, just behind a whole chunk."""
+    pace, wait = (1.0, 1.0) if dk > 64 else (0.62, 0.78)
+    share = pace * blocks / 256
+
+    def tokens(ns):
+        each = [max(1.15, 0.6 + 0.15 * n) for n in ns]
+        return (6.5 + 0.19 * max(ns) if dk > 64 else 5.2 + 0.165 * max(ns)) + max(0.0, share * sum(each) - pace * max(each))
+
+    def chunks(ns):
+        each = [4.4 + 0.024 * min(n, SSD_CHUNK) + 3.3 * ((n - 1) // SSD_CHUNK) for n in ns]
+        longest = max(ns)
+        alone = 14.5 + 3.3 * ((longest + SSD_CHUNK - 1) // SSD_CHUNK) - 0.17 * max(0, SSD_CHUNK - longest)
+        return wait * alone + max(0.0, share * sum(each) - pace * max(each))
+    plans = [(tokens(n_new), WHOLE_STEP), (chunks(n_new), 0)]
+    short, long = [n for n in n_new if n < SSD_CHUNKS_FROM], [n for n in n_new if n >= SSD_CHUNKS_FROM]
+    if short and long:
+        plans.append((1.2 * tokens(short) + chunks(long) + 3.0, SSD_CHUNKS_FROM))       # (one kernel behind the other)
+    return min(plans)[1]
+
+
+def _ssd_chunks(q, ldq, k, ldk, v, ldv, dt_in, lddt, a_log, dt_bias, skip, out, ldo, state, step, least, n_heads, n_kv, dk, dv) -> None:
     n, ws = step.n_tokens, step.workspace
     cb = ws.get("ssd_cb", n, n_kv * SSD_CHUNK, torch.float32)
     cum = ws.get("ssd_cum", n, n_heads, torch.float64)
     made = ws.get("ssd_made", 4 * n, n_heads, torch.float32)
     library.call(_lib(), "agave_ssd_chunks", ptr(q), ldq, ptr(k), ldk, ptr(v), ldv, ptr(dt_in), lddt, ptr(a_log), ptr(dt_bias), ptr(skip),
-                 ptr(out), ldo, ptr(state), ptr(step.cu_dev), ptr(step.slots_dev), step.n_seqs, n_heads, n_kv, dk, dv, step.max_new, n,
+                 ptr(out), ldo, ptr(state), ptr(step.cu_dev), ptr(step.slots_dev), step.n_seqs, n_heads, n_kv, dk, dv, step.max_new, least, n,
                  ptr(cb), ptr(cum), ptr(made), stream())
 
 
@@ -201,6 +236,7 @@ def gated_recurrence(mode: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     if max(step.slots) >= state.shape[0]:
         raise ValueError("gated_recurrence: a slot lies outside the state")
     lddt = ldb = 0
+    most = WHOLE_STEP
     if mode == DELTA:
         lddt, ldb = _f32rows(dt_in, "dt", n, n_heads * dk), _f32rows(beta, "beta", n, n_heads)
         _f32vec(a_log, "a_log", n_heads)
@@ -215,8 +251,12 @@ def gated_recurrence(mode: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
         if a_log is None or dt_bias is None or skip is None:
             raise ValueError("gated_recurrence: the state-space form needs a_log, dt_bias and skip")
         if ssd_chunks_ok(q, k, v, step, dk, dv):
-            _ssd_chunks(q, ldq, k, ldk, v, ldv, dt_in, lddt, a_log, dt_bias, skip, out, ldo, state, step, n_heads, n_kv, dk, dv)
-            return
+            least = ssd_chunked_from(tuple(step.n_new), n_heads * dv // 16, dk)
+            if least <= step.max_new:
+                _ssd_chunks(q, ldq, k, ldk, v, ldv, dt_in, lddt, a_log, dt_bias, skip, out, ldo, state, step, least, n_heads, n_kv, dk, dv)
+                if least <= 1:
+                    return
+                most = least - 1
     elif mode == FORGET:
         _f32vec(lower, "lower", n_heads * dk)
         _f32vec(f_bias, "f_bias", n_heads * dk)
@@ -227,7 +267,7 @@ def gated_recurrence(mode: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
     library.call(_lib(), "agave_gated_recurrence", mode, ptr(q), ldq, ptr(k), ldk, ptr(v), ldv, ptr(dt_in), lddt, ptr(beta),
                  ldb, ptr(a_log), ptr(dt_bias), ptr(lower), ptr(f_bias), ptr(skip), ptr(out), ldo, ptr(state), ptr(step.cu_dev),
                  ptr(step.slots_dev), step.n_seqs, n_heads, n_heads if mode == FORGET else n_kv, dk, dv, float(unit_eps),
-                 1 if (step.is_decode and step.n_tokens == step.n_seqs) else 0, stream())
+                 1 if (step.is_decode and step.n_tokens == step.n_seqs) else 0, most, stream())
 
 
 def head_norm_gate(o: torch.Tensor, weight: torch.Tensor, gate: Optional[torch.Tensor], out: torch.Tensor,

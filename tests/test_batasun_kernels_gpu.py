@@ -235,6 +235,63 @@ def test_state_space_in_chunks_ends_with_an_infinity(T, which):
     assert torch.allclose(got[:-1], ref[:-1], atol=3e-5, rtol=1e-4)
 
 
+def state_space_batch(H, G, N, dv, steps, least, seed=7):
+    """Sequences through steps that bring each of them ``steps[k][i]`` tokens (0: not in the step), those of at least ``least``
+    in chunks: (read-outs, states) of every sequence and the 64-bit ones."""
+    from agave_amd.cache import StateNeed
+    from agave_amd.ops import sequence as S
+    from agave_amd.parts import Workspace
+    n_seqs = len(steps[0])
+    cache, planner = planner_for(state={0: StateNeed((H, dv, N))}, slots=n_seqs + 2, context=4096)
+    planner.workspace = Workspace(torch.device(DEV))
+    got_slots = [cache.alloc_slot() for _ in range(n_seqs + 2)]
+    slots = [got_slots[(5 * i + 3) % (n_seqs + 2)] for i in range(n_seqs)] if (n_seqs + 2) % 5 else got_slots[2:][::-1]
+    made = [state_space_inputs(H, G, N, dv, sum(n[i] for n in steps), seed + i)[0] for i in range(n_seqs)]
+    vec = state_space_inputs(H, G, N, dv, 1, seed)[1]
+    outs, at = [[] for _ in range(n_seqs)], [0] * n_seqs
+    real = S.ssd_chunked_from
+    if least is not None:
+        S.ssd_chunked_from = lambda *_: least
+    try:
+        for counts in steps:
+            live = [i for i, n in enumerate(counts) if n]
+            step = feed(cache, planner, [slots[i] for i in live], [counts[i] for i in live])
+            cat = {n: torch.cat([made[i][n][at[i]:at[i] + counts[i]] for i in live]).to(DEV) for n in ("xs", "B", "C", "dt")}
+            out = torch.full((sum(counts), H * dv), float("nan"), device=DEV)
+            S.gated_recurrence(S.SSD, cat["C"], cat["B"], cat["xs"], out, cache.state[0], step, H, G, N, dv, dt_in=cat["dt"],
+                               **{n: x.to(DEV) for n, x in vec.items()})
+            planner.commit(step)
+            for i, o in zip(live, out.split([counts[i] for i in live])):
+                outs[i].append(o.cpu())
+                at[i] += counts[i]
+    finally:
+        S.ssd_chunked_from = real
+    refs = [plain_state_space(t, vec, H, G, N, dv) for t in made]
+    return ([torch.cat(o).to(F64) for o in outs], [cache.state[0][s].cpu().to(F64).transpose(1, 2) for s in slots],
+            [r.reshape(len(r), -1) for r, _ in refs], [S_ref for _, S_ref in refs])
+
+
+@pytest.mark.parametrize("H, G, N, dv", [(4, 2, 64, 32), (3, 1, 128, 16)])
+@pytest.mark.parametrize("least", [0, 48, 66, 2 ** 31 - 1, None])
+def test_state_space_chunks_of_a_batch(H, G, N, dv, least):
+    """Sequences of one token to several chunks in one step, in slots out of order and with states that go on: all in chunks,
+    the long ones alone, none, and as the rule has it.  A sequence that the step leaves out keeps its state."""
+    outs, states, refs, S_refs = state_space_batch(H, G, N, dv, [[1, 130, 17, 64, 65, 47], [48, 1, 0, 129, 3, 0], [1, 70, 200, 1, 1, 1]], least)
+    for got, ref, S_got, S_ref in zip(outs, refs, states, S_refs):
+        # (a read-out's or a state's error is some 1e-7 of their size, and sums of a few hundred numbers leave no more than 3e-7)
+        assert float((got - ref).norm() / ref.norm()) < 3e-7 and float((S_got - S_ref).norm() / S_ref.norm()) < 3e-7
+
+
+def test_state_space_chunks_are_as_close_as_tokens():
+    """Against 64 bits, chunks lose no more than the same sequences token by token."""
+    errs = []
+    for least in (0, 2 ** 31 - 1):
+        outs, states, refs, S_refs = state_space_batch(24, 1, 128, 64, [[300, 64]], least)
+        errs.append([float((torch.cat([a.flatten() for a in x]) - torch.cat([a.flatten() for a in y])).norm() / torch.cat([a.flatten() for a in y]).norm())
+                     for x, y in ((outs, refs), (states, S_refs))])
+    assert errs[0][0] <= errs[1][0] and errs[0][1] <= errs[1][1], errs
+
+
 def test_state_space_step_sizes_without_a_clamp_and_a_write_far_back():
     """Step sizes from almost nothing to dozens (softplus of -20 to 40, neither clamped); and with a decay rate of
     almost nothing what token 3 wrote is read 600 tokens later among small writes, while a fast rate forgets it."""
