@@ -35,7 +35,8 @@ __device__ __forceinline__ float lanes16_sum(float v) {
 // see, a page of 64 keys at a time: every wave the scores of 16 keys, then, with the page's probabilities in LDS, the sums over
 // the page for a quarter of the value elements.  Both are products for v_mfma_f32_16x16x4_f32, whose operands K and V come
 // straight from memory in 16-byte pieces (it takes the summed index in any order as long as both operands agree).  Tokens of
-// several sequences in one workgroup (any tok_seq is taken) go one sequence after another.
+// several sequences in one workgroup (any tok_seq is taken) go one sequence after another, or, with gridDim.z turns, the
+// z-th of them in a workgroup of its own.
 // gridDim.y workgroups share a row's pages and leave (sum, maximum, unnormalised result) for attn_plain_merge_kernel: with a
 // token per sequence there are few rows and the pages one after another bound the time.
 // NT: tiles of 64 value elements (16 a wave).  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of 0 must not meet a value that is not finite (a key behind a
@@ -59,9 +60,20 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
 
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const int G = nh / nkv, chunks = (G + ROWS - 1) / ROWS;
-    const int chunk = blockIdx.x % chunks, kvh = blockIdx.x / chunks % nkv, t0 = blockIdx.x / chunks / nkv * run;
+    const int chunk = blockIdx.x % chunks, kvh = blockIdx.x / chunks % nkv;
+    int t0 = blockIdx.x / chunks / nkv * run, tokens = min(run, N - t0);
+    if (gridDim.z > 1) {                                     // this workgroup's turn of the sequences among its tokens
+        const int t = t0 + (lane < tokens ? lane : 0);
+        unsigned long long left = __ballot(lane < tokens && (lane == 0 || tok_seq[t] != tok_seq[t > 0 ? t - 1 : 0]));
+        for (int i = blockIdx.z; i > 0; --i) left &= left - 1;
+        if (left == 0) return;
+        const int a = __builtin_ctzll(left);
+        left &= left - 1;
+        tokens = (left == 0 || blockIdx.z + 1 == gridDim.z ? tokens : __builtin_ctzll(left)) - a;       // (the last turn takes all that are left)
+        t0 += a;
+    }
     const int heads = min(G - chunk * ROWS, ROWS), head0 = kvh * G + chunk * ROWS;
-    const int rows = min(min(run, N - t0) * heads, ROWS);
+    const int rows = min(tokens * heads, ROWS);
     const int split = blockIdx.y, splits = gridDim.y;
 
     if (tid < ROWS) {
@@ -249,9 +261,9 @@ __global__ __launch_bounds__(128) void attn_plain_merge_kernel(const float* __re
 template <typename T, int NT>
 static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages, const T* v_pages, const int* table, int width,
                         const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                        int window, int run, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                        int window, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
     const int chunks = (nh / nkv + ROWS - 1) / ROWS;
-    const dim3 grid((N + run - 1) / run * nkv * chunks, splits);
+    const dim3 grid((N + run - 1) / run * nkv * chunks, splits, turns);
     // four elements at a time where rows are aligned to as many (a value row is a page long, so its pages' start decides)
     const uintptr_t wide = 4 * sizeof(T);
     const bool vec_v = (uintptr_t)v_pages % wide == 0;
@@ -266,9 +278,9 @@ static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages
 template <typename T>
 static void launch_type(const void* q, long ldq, void* out, long ldo, const void* k_pages, const void* v_pages, const int* table, int width,
                         const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                        int window, int run, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                        int window, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
 #define ROWS_GO(NT_) launch_rows<T, NT_>((const T*)q, ldq, (T*)out, ldo, (const T*)k_pages, (const T*)v_pages, table, width, base, n_pages, \
-                                         tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, splits, part_o, part_ml, stream)
+                                         tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, turns, splits, part_o, part_ml, stream)
     if (hd <= 64) ROWS_GO(1);
     else if (hd <= 128) ROWS_GO(2);
     else if (hd <= 256) ROWS_GO(4);
@@ -287,12 +299,24 @@ extern "C" int agave_attn_plain_splits(int N, int nh, int nkv, int span) {
     return z < 1 ? 1 : (int)z;
 }
 
-// one_token_each: neighbouring tokens are of different sequences (a decode step), so a workgroup takes one.  splits > 1: part_o
+// How many neighbouring tokens a workgroup takes.
+// Neighbouring tokens share a page's keys where there are enough of them to fill the compute units without.  us, a token a
+// workgroup and several, 32-bit: 16 heads of 128 over 4, 64 tokens (256 workgroups) 10.5 and 11.2, 96 tokens 18.1 and 16.2, 421
+// tokens 99 and 47; 8 heads of 256 over 4, 64 tokens 14.1 and 15.8, 96 tokens 27.3 and 24.5; 4 heads of 64 over one, 256
+// tokens 17.6 and 18.1, 300 tokens 22.4 and 20.9; 8 heads of 64 over 8, 64 tokens (512 workgroups) 8.4 and 8.8, 96 tokens 13.2 and 11.9.
+extern "C" int agave_attn_plain_run(int N, int nh, int nkv) {
+    if (N <= 0 || nh <= 0 || nkv <= 0 || nh % nkv != 0) return 1;
+    const int G = nh / nkv;
+    return G >= ROWS || (long)N * nkv <= COMPUTE_UNITS ? 1 : ROWS / G;
+}
+
+// one_token_each: neighbouring tokens are of different sequences (a decode step), so a workgroup takes one.  most_seqs: of as
+// many sequences at most are any `agave_attn_plain_run` tokens from a multiple of it on (no result depends on it).  splits > 1: part_o
 // [N][nh][splits][hd] and part_ml [N][nh][splits][2] receive what a row's workgroups leave.
 extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, long ldo, const void* k_pages,
                                 const void* v_pages, const int* table, int width, const int* base, int n_pages,
                                 const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                                int window, int one_token_each, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                                int window, int one_token_each, int most_seqs, int splits, float* part_o, float* part_ml, hipStream_t stream) {
     AGAVE_CHECK(N >= 0 && nh > 0 && nkv > 0 && hd > 0, "attn_plain: bad sizes N=%d nh=%d nkv=%d hd=%d", N, nh, nkv, hd);
     AGAVE_CHECK(nh % nkv == 0, "attn_plain: %d query heads are not a multiple of %d kv heads", nh, nkv);
     AGAVE_CHECK(hd <= 512, "attn_plain: head_dim %d exceeds the supported maximum %d", hd, 512);
@@ -304,18 +328,19 @@ extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, l
     AGAVE_CHECK(splits >= 1 && splits <= MOST_SPLITS && (splits == 1 || (part_o && part_ml)), "attn_plain: %d splits (1 to %d, with buffers for what they leave)",
                 splits, MOST_SPLITS);
     AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "attn_plain: unknown dtype %d", dtype);
+    AGAVE_CHECK(most_seqs >= 1, "attn_plain: %d sequences a workgroup", most_seqs);
     if (N == 0) return 0;
-    // Neighbouring tokens share a page's keys where there are enough of them to fill the compute units without.  us, a token a
-    // workgroup and several, 32-bit: 16 heads of 128 over 4, 64 tokens (256 workgroups) 10.5 and 11.2, 96 tokens 18.1 and 16.2, 421
-    // tokens 99 and 47; 8 heads of 256 over 4, 64 tokens 14.1 and 15.8, 96 tokens 27.3 and 24.5; 4 heads of 64 over one, 256
-    // tokens 17.6 and 18.1, 300 tokens 22.4 and 20.9; 8 heads of 64 over 8, 64 tokens (512 workgroups) 8.4 and 8.8, 96 tokens 13.2 and 11.9.
-    const int G = nh / nkv, run = one_token_each || G >= ROWS || (long)N * nkv <= COMPUTE_UNITS ? 1 : ROWS / G;
+    const int run = one_token_each ? 1 : agave_attn_plain_run(N, nh, nkv);
+    // A workgroup for each of a run's sequences from three on (of two, one waits for the other).  40 tokens behind 1,000 keys
+    // each and a prompt of 64 tokens, 32 bits, us, one after another and so: 8 heads of 64 over 8 885 and 75, 8 of 256 over 4 1,548
+    // and 260 (a workgroup per token and head 148 and 400).
+    const int most_turns = most_seqs < run ? most_seqs : run, turns = most_turns > 2 ? most_turns : 1;
     if (dtype == AGAVE_F32)
         launch_type<float>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
-                           run, splits, part_o, part_ml, stream);
+                           run, turns, splits, part_o, part_ml, stream);
     else
         launch_type<bf16>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
-                          run, splits, part_o, part_ml, stream);
+                          run, turns, splits, part_o, part_ml, stream);
     AGAVE_LAUNCH_CHECK("attn_plain");
     return 0;
 }

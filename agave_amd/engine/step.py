@@ -16,8 +16,9 @@ stands for.
 """
 from __future__ import annotations
 
+from collections import Counter
 from dataclasses import dataclass, field
-from typing import List, Optional, Sequence, Tuple, Union
+from typing import Dict, List, Optional, Sequence, Tuple, Union
 
 import numpy as np
 import torch
@@ -58,6 +59,7 @@ class Step:
     carry_dev: Optional[torch.Tensor] = None    # int32 [B]: rows of the previous step's sample that these tokens are
     floats_dev: Optional[torch.Tensor] = None   # float32 payload that travelled with the step (sampling parameters)
     n_pad: int = 0                               # rows behind the last sequence's tokens that belong to no request (see plan)
+    seqs_a_run: Dict[int, int] = field(default_factory=dict)    # what ``most_seqs`` has counted
 
     def page_span(self, window: Optional[int]) -> int:
         """Most pages any sequence's last token of this step reaches back over."""
@@ -72,6 +74,14 @@ class Step:
             lo = max(0, p - window + 1) if window is not None else 0
             span = max(span, p // PAGE - lo // PAGE + 1)
         return span
+
+    def most_seqs(self, run: int) -> int:
+        """Of how many sequences at most any ``run`` rows of this step are, from a multiple of ``run`` on."""
+        got = self.seqs_a_run.get(run)
+        if got is None:
+            inside = Counter(c // run for c in self.cu[1:-1] if c % run)       # (sequences that begin within such rows)
+            got = self.seqs_a_run[run] = 1 + max(inside.values(), default=0)
+        return got
 
     @property
     def is_decode(self) -> bool:

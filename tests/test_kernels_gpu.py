@@ -475,6 +475,31 @@ def test_attn_plain_pages_at_any_element(K, dtype, hd, k_at, v_at):
     assert bool(outs[0].isfinite().all()) and torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh,nkv,hd", [(4, 4, 32), (6, 2, 40), (8, 2, 300)])
+def test_attn_plain_steps_of_many_sequences(K, dtype, nh, nkv, hd):
+    """Tokens of several sequences among those that a workgroup would take, in any order: each has the result it has alone,
+    whether the sequences get a workgroup each, share a few, or go one after another in one."""
+    g = torch.Generator().manual_seed(hd)
+    seqs, ctx = 5, 150
+    kp, vp = (torch.randn(3 * seqs, nkv, *shape, generator=g).to(dtype).to(DEV) for shape in ((64, hd), (hd, 64)))
+    table = torch.randperm(3 * seqs, generator=g).view(seqs, 3).int().to(DEV)
+    tok_seq = [0] * 90 + [1, 2, 3, 4, 0, 2] + [3] * 20 + torch.randint(0, seqs, (200,), generator=g).tolist()
+    tok_pos = torch.randint(0, ctx, (len(tok_seq),), generator=g).tolist()
+    n = len(tok_seq)
+    q = torch.randn(n, nh * hd, generator=g).to(dtype).to(DEV)
+
+    def go(rows, **more):
+        out = torch.empty(len(rows), nh * hd, dtype=dtype, device=DEV)
+        K.attn_plain(q[rows].contiguous(), out, kp, vp, table, _i32([0] * seqs), _i32([tok_seq[r] for r in rows]), _i32([tok_pos[r] for r in rows]),
+                     nh, nkv, hd, 0.2, 70, **more)
+        return out
+    rows = list(range(n))
+    want = go(rows, one_token_each=True)
+    for most in (lambda run: 1, lambda run: 3, lambda run: run, None):
+        assert torch.equal(go(rows, most_seqs=most), want)
+
+
 def test_attn_plain_far_key_wins(K):
     # among 700 keys, key 3 is made to dominate the last query's softmax: the output must be its value
     got, ref, vs = _attn_case(K, torch.float32, 2, 1, 32, [700], None, 0.5, seed=1, boost=3)

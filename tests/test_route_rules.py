@@ -13,3 +13,13 @@ from agave_amd.ops import sequence as S
 def test_which_sequences_go_through_the_state_space_form_in_chunks(n_new, heads, dk, dv, least):
     """A step of a prompt beside sequences of one token does not pay for a chunk per sequence."""
     assert S.ssd_chunked_from(tuple(n_new), heads * dv // 16, dk) == least
+
+
+@pytest.mark.parametrize("n_new", [[1], [5, 1, 1, 1, 7], [1] * 20, [16, 16, 1, 15, 3], [40, 2, 2, 2, 2, 2, 90]])
+@pytest.mark.parametrize("run", [2, 4, 5, 16])
+def test_sequences_among_neighbouring_rows(n_new, run):
+    from agave_amd.engine.step import Step
+    cu = [sum(n_new[:i]) for i in range(len(n_new) + 1)]
+    step = Step(**{**dict.fromkeys(Step.__dataclass_fields__), "cu": cu, "n_new": n_new, "seqs_a_run": {}})
+    seq = [i for i, n in enumerate(n_new) for _ in range(n)]
+    assert step.most_seqs(run) == step.most_seqs(run) == max(len(set(seq[a:a + run])) for a in range(0, len(seq), run))
