@@ -258,16 +258,112 @@ __global__ __launch_bounds__(128) void attn_plain_merge_kernel(const float* __re
     }
 }
 
+// Few keys: a workgroup per token and head, four lanes a key, then a thread per value element (two from 257 elements on).  Bound by
+// its chain of trips to memory; the kernel above brings whole pages and multiplies tiles that are mostly empty.  A key's product
+// has sixteen running sums.  Takes any number of keys, a page at a time.
+// Measured in 32 bits, us, tiles of rows and so: a prompt of 5 tokens, 8 heads of 256 over 4, 13.7 and 5.7 (an element at a time a key
+// and a thread, the kernel before both, 9.9), of 512 over one 21.9 and 7.7 (16.2); of 33 tokens 13.7 and 7.8, 22.1 and 11.5; eight
+// tokens behind 64 keys 13.8 and 7.8, 22.0 and 11.3.  Errors against 64 bits 0.6 to 1.3e-7 after 0.8 to 1.9e-7.
+template <typename T, bool VEC, bool VEC_V>
+__global__ __launch_bounds__(256) void attn_plain_few_keys_kernel(
+    const T* __restrict__ q, long ldq, T* __restrict__ out, long ldo, const T* __restrict__ k_pages,
+    const T* __restrict__ v_pages, const int* __restrict__ table, int width, const int* __restrict__ base,
+    int n_pages, const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, int nh, int nkv, int hd, float scale, int window) {
+    __shared__ __attribute__((aligned(16))) float qs[512], P[AGAVE_PAGE];
+    __shared__ float wmax[4], wsum[4];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int t = blockIdx.x / nh, h = blockIdx.x % nh, kvh = h / (nh / nkv);
+    const int seq = tok_seq[t], hi = tok_pos[t], lo = window > 0 && hi - window + 1 > 0 ? hi - window + 1 : 0;
+    const int pbase = base[seq];
+    for (int d = tid; d < (hd + 3) / 4 * 4; d += 256) qs[d] = d < hd ? ld(q + (size_t)t * ldq + (size_t)h * hd + d) : 0.f;
+    __syncthreads();
+    float m = -INFINITY, l = 0.f, o[2] = {0.f, 0.f};
+    for (int page = lo / AGAVE_PAGE; page * AGAVE_PAGE <= hi; ++page) {
+        const int col = page - pbase;
+        const long pg = col >= 0 && col < width ? table[(size_t)seq * width + col] : -1;
+        if (pg < 0 || pg >= n_pages) continue;               // (the same for the whole workgroup)
+        const T* v[2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) v[a] = v_pages + ((size_t)(pg * nkv + kvh) * hd + min(tid + 256 * a, hd - 1)) * AGAVE_PAGE;
+        const int j0 = max(lo - page * AGAVE_PAGE, 0), j1 = min(hi - page * AGAVE_PAGE, AGAVE_PAGE - 1);      // the keys that are seen
+        f32x4_t vv[2][4];
+        auto values = [&](int j) {                           // of the sixteen keys from j on
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+                if (256 * a < hd)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) vv[a][i] = ld4<VEC_V>(v[a], j + 4 * i, AGAVE_PAGE);
+        };
+        values(j0 & ~15);
+        const int key = tid >> 2;
+        const bool seen = key >= j0 && key <= j1;
+        f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+        if (seen) {
+            const T* kr = k_pages + ((size_t)(pg * nkv + kvh) * AGAVE_PAGE + key) * hd;
+#pragma unroll 8
+            for (int d = 4 * (tid & 3); d < hd; d += 16) {
+                const f32x4_t kv = ld4<VEC>(kr, d, hd), qv = *reinterpret_cast<const f32x4_t*>(&qs[d]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] = fmaf(kv[e], qv[e], sum[e]);
+            }
+        }
+        float s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+        s += dpp_get<0xB1, 0xF>(0.f, s);
+        s += dpp_get<0x4E, 0xF>(0.f, s);
+        s = seen ? s * scale : -INFINITY;
+        const float most = wave_max(s);
+        if (lane == 0) wmax[w] = most;
+        __syncthreads();
+        const float m_new = fmaxf(m, fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])));
+        const float alpha = m == -INFINITY ? 0.f : expf(m - m_new), pr = seen ? expf(s - m_new) : 0.f;
+        m = m_new;
+        if ((tid & 3) == 0) P[key] = pr;
+        const float total = wave_sum((tid & 3) == 0 ? pr : 0.f);
+        if (lane == 0) wsum[w] = total;
+        __syncthreads();
+        l = l * alpha + ((wsum[0] + wsum[1]) + (wsum[2] + wsum[3]));
+        o[0] *= alpha;
+        o[1] *= alpha;
+        float add[2] = {0.f, 0.f};
+        for (int j = j0 & ~15; j <= j1; j += 16) {
+            if (j != (j0 & ~15)) values(j);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const f32x4_t pv = *reinterpret_cast<const f32x4_t*>(&P[j + 4 * i]);
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+                    if (256 * a < hd)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) add[a] = pv[e] != 0.f ? fmaf(pv[e], vv[a][i][e], add[a]) : add[a];    // (a key that is not seen may hold anything)
+            }
+        }
+        o[0] += add[0];
+        o[1] += add[1];
+        __syncthreads();                                     // P, wmax and wsum are written again
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+        if (tid + 256 * a < hd) st(out + (size_t)t * ldo + (size_t)h * hd + tid + 256 * a, o[a] * inv);
+}
+
 template <typename T, int NT>
 static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages, const T* v_pages, const int* table, int width,
                         const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                        int window, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                        int window, bool few_keys, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
     const int chunks = (nh / nkv + ROWS - 1) / ROWS;
     const dim3 grid((N + run - 1) / run * nkv * chunks, splits, turns);
     // four elements at a time where rows are aligned to as many (a value row is a page long, so its pages' start decides)
     const uintptr_t wide = 4 * sizeof(T);
     const bool vec_v = (uintptr_t)v_pages % wide == 0;
     const bool vec = vec_v && hd % 4 == 0 && ldq % 4 == 0 && (uintptr_t)k_pages % wide == 0 && (uintptr_t)q % wide == 0;
+    if (few_keys) {
+#define FEW_GO(VEC_, VEC_V_) attn_plain_few_keys_kernel<T, VEC_, VEC_V_><<<N * nh, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, \
+        width, base, n_pages, tok_seq, tok_pos, nh, nkv, hd, scale, window)
+        if (vec) FEW_GO(true, true); else if (vec_v) FEW_GO(false, true); else FEW_GO(false, false);
+#undef FEW_GO
+        return;
+    }
 #define PLAIN_GO(VEC_, VEC_V_) attn_plain_kernel<T, NT, VEC_, VEC_V_><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, width, \
         base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml)
     if (vec) PLAIN_GO(true, true); else if (vec_v) PLAIN_GO(false, true); else PLAIN_GO(false, false);
@@ -278,9 +374,9 @@ static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages
 template <typename T>
 static void launch_type(const void* q, long ldq, void* out, long ldo, const void* k_pages, const void* v_pages, const int* table, int width,
                         const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                        int window, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                        int window, bool few_keys, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
 #define ROWS_GO(NT_) launch_rows<T, NT_>((const T*)q, ldq, (T*)out, ldo, (const T*)k_pages, (const T*)v_pages, table, width, base, n_pages, \
-                                         tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, turns, splits, part_o, part_ml, stream)
+                                         tok_seq, tok_pos, N, nh, nkv, hd, scale, window, few_keys, run, turns, splits, part_o, part_ml, stream)
     if (hd <= 64) ROWS_GO(1);
     else if (hd <= 128) ROWS_GO(2);
     else if (hd <= 256) ROWS_GO(4);
@@ -311,12 +407,13 @@ extern "C" int agave_attn_plain_run(int N, int nh, int nkv) {
 }
 
 // one_token_each: neighbouring tokens are of different sequences (a decode step), so a workgroup takes one.  most_seqs: of as
-// many sequences at most are any `agave_attn_plain_run` tokens from a multiple of it on (no result depends on it).  splits > 1: part_o
+// many sequences at most are any `agave_attn_plain_run` tokens from a multiple of it on (no result depends on it).  most_keys: no token
+// sees more keys than this, 0 where that is not known (nor on it).  splits > 1: part_o
 // [N][nh][splits][hd] and part_ml [N][nh][splits][2] receive what a row's workgroups leave.
 extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, long ldo, const void* k_pages,
                                 const void* v_pages, const int* table, int width, const int* base, int n_pages,
                                 const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                                int window, int one_token_each, int most_seqs, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                                int window, int one_token_each, int most_seqs, int most_keys, int splits, float* part_o, float* part_ml, hipStream_t stream) {
     AGAVE_CHECK(N >= 0 && nh > 0 && nkv > 0 && hd > 0, "attn_plain: bad sizes N=%d nh=%d nkv=%d hd=%d", N, nh, nkv, hd);
     AGAVE_CHECK(nh % nkv == 0, "attn_plain: %d query heads are not a multiple of %d kv heads", nh, nkv);
     AGAVE_CHECK(hd <= 512, "attn_plain: head_dim %d exceeds the supported maximum %d", hd, 512);
@@ -330,6 +427,9 @@ extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, l
     AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "attn_plain: unknown dtype %d", dtype);
     AGAVE_CHECK(most_seqs >= 1, "attn_plain: %d sequences a workgroup", most_seqs);
     if (N == 0) return 0;
+    // Few keys and few rows: beyond, tiles of rows share what they load (the longest times of the few-key kernel over those of the
+    // tiles, over 16 head shapes and types: 16 keys and 1,024 rows 1.01, 2,048 rows 2.9; 48 and 512 1.01, 1,024 1.4; 64 and 256 1.03, 512 1.13).
+    const bool few_keys = splits == 1 && most_keys > 0 && most_keys <= 64 && (long)N * nh <= (most_keys <= 16 ? 1024 : most_keys <= 48 ? 512 : 256);
     const int run = one_token_each ? 1 : agave_attn_plain_run(N, nh, nkv);
     // A workgroup for each of a run's sequences from three on (of two, one waits for the other).  40 tokens behind 1,000 keys
     // each and a prompt of 64 tokens, 32 bits, us, one after another and so: 8 heads of 64 over 8 885 and 75, 8 of 256 over 4 1,548
@@ -337,10 +437,10 @@ extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, l
     const int most_turns = most_seqs < run ? most_seqs : run, turns = most_turns > 2 ? most_turns : 1;
     if (dtype == AGAVE_F32)
         launch_type<float>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
-                           run, turns, splits, part_o, part_ml, stream);
+                           few_keys, run, turns, splits, part_o, part_ml, stream);
     else
         launch_type<bf16>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
-                          run, turns, splits, part_o, part_ml, stream);
+                          few_keys, run, turns, splits, part_o, part_ml, stream);
     AGAVE_LAUNCH_CHECK("attn_plain");
     return 0;
 }

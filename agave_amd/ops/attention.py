@@ -5,6 +5,7 @@ from typing import Optional
 
 import torch
 
+from ..cache import PAGE
 from . import attention_mfma, kernels
 
 
@@ -19,7 +20,8 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages
         return
     one_each = step.is_decode and step.n_tokens == step.n_seqs
     kernels.attn_plain(q, out, k_pages, v_pages, table, base, step.tok_seq, step.tok_pos, n_heads, n_kv, head_dim, scale, window,
-                       one_token_each=one_each, span=step.page_span(window) if one_each else 1, workspace=step.workspace, most_seqs=step.most_seqs)
+                       one_token_each=one_each, span=step.page_span(window) if one_each else 1, workspace=step.workspace, most_seqs=step.most_seqs,
+                       most_keys=step.max_len if step.fixed_span is None else PAGE * step.fixed_span)
 
 
 def qk_attention(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.Tensor], q_rot: torch.Tensor,

@@ -38,7 +38,7 @@ _SIGNATURES = {
         "agave_gemm_plain": [_I, _P, _L, _I, _P, _L, _I, _P, _L, _I, _I, _I, _P],
     },
     "attention_plain": {
-        "agave_attn_plain": [_I, _P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _F, _I, _I, _I, _I, _P, _P, _P],
+        "agave_attn_plain": [_I, _P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _F, _I, _I, _I, _I, _I, _P, _P, _P],
         "agave_attn_plain_splits": [_I, _I, _I, _I],
         "agave_attn_plain_run": [_I, _I, _I],
     },
@@ -427,12 +427,13 @@ def gemm_plain(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor) -> None:
 def attn_plain(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                table: torch.Tensor, base: torch.Tensor, tok_seq: torch.Tensor, tok_pos: torch.Tensor,
                n_heads: int, n_kv: int, head_dim: int, scale: float, window: Optional[int],
-               one_token_each: bool = False, span: int = 1, workspace=None, most_seqs=None) -> None:
+               one_token_each: bool = False, span: int = 1, workspace=None, most_seqs=None, most_keys: int = 0) -> None:
     """Attention of every token over its sequence's cache pages (keys up to its own position,
     and not older than ``window`` - 1 positions back if a window is given).  ``one_token_each``: a step in which
     every sequence brings one token, which sees at most ``span`` pages; with a ``workspace`` for their partial results
     several workgroups then share a row's pages.  ``most_seqs(run)``: of how many sequences at most any ``run`` tokens of
-    the step are, from a multiple of ``run`` on (None: as many as the table has)."""
+    the step are, from a multiple of ``run`` on (None: as many as the table has).
+    ``most_keys``: no token sees more keys than this (0: as many as the table's pages hold; the results do not depend on it)."""
     _dev(q, out, k_pages, v_pages, table, base, tok_seq, tok_pos)
     n = tok_pos.numel()
     _i32(tok_pos, "tok_pos")
@@ -454,4 +455,4 @@ def attn_plain(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_page
             part_ml = workspace.get("attn_part_ml", n * n_heads * splits, 2, torch.float32)
     library.call(lib("attention_plain"), "agave_attn_plain", dt(q), ptr(q), ldq, ptr(out), ldo, ptr(k_pages),
                  ptr(v_pages), ptr(table), width, ptr(base), n_pages, ptr(tok_seq), ptr(tok_pos), n, n_heads, n_kv,
-                 head_dim, scale, int(window or 0), 1 if one_token_each else 0, int(seqs), splits, ptr(part_o), ptr(part_ml), stream())
+                 head_dim, scale, int(window or 0), 1 if one_token_each else 0, int(seqs), int(most_keys) or 64 * width, splits, ptr(part_o), ptr(part_ml), stream())

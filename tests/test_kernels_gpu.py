@@ -500,6 +500,64 @@ def test_attn_plain_steps_of_many_sequences(K, dtype, nh, nkv, hd):
         assert torch.equal(go(rows, most_seqs=most), want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh,nkv,hd,window", [(4, 2, 40, None), (3, 1, 512, 9), (5, 5, 2, None), (6, 2, 130, 20), (2, 2, 256, 70)])
+@pytest.mark.parametrize("most_keys", [5, 16, 64])
+def test_attn_plain_few_keys(K, dtype, nh, nkv, hd, window, most_keys):
+    """Steps of few keys and rows, against the plain implementation; a sequence that sees more keys than it was said to is right
+    all the same, also where what it does not see is not a number."""
+    lens = [1, 2, min(most_keys, 40), 90 if most_keys == 64 else 70]
+    real, rows = K.attn_plain, {}
+
+    def few(q, out, kp, vp, table, base, tok_seq, tok_pos, *rest):
+        n = 256 // nh                                             # (few rows: the first ones, and the last ones)
+        for at in (slice(0, n), slice(q.shape[0] - n if q.shape[0] > n else 0, q.shape[0])):
+            for junk in (False, True):
+                if junk:
+                    for b, L in enumerate(lens):
+                        page = int(table[b, (L - 1) // 64])
+                        if L % 64:
+                            kp[page, :, L % 64:] = float("nan")
+                            vp[page, :, :, L % 64:] = float("nan")
+                o = torch.empty_like(q[at])
+                real(q[at].contiguous(), o, kp, vp, table, base, tok_seq[at].contiguous(), tok_pos[at].contiguous(), *rest, most_keys=most_keys)
+                rows[at.start, junk] = (at, o.cpu().double().view(-1, nh, hd))
+        real(q, out, kp, vp, table, base, tok_seq, tok_pos, *rest)
+    K.attn_plain = few
+    try:
+        _, ref, _ = _attn_case(K, dtype, nh, nkv, hd, lens, window, hd ** -0.5)
+    finally:
+        K.attn_plain = real
+    tol = dict(atol=2e-6 + 1e-7 * hd, rtol=2e-5) if dtype == torch.float32 else dict(atol=2e-2, rtol=2e-2)
+    for at, got in rows.values():
+        assert torch.allclose(got, ref[at], **tol)
+
+
+@pytest.mark.parametrize("what", ["query", "key", "value"])
+def test_attn_plain_few_keys_that_are_not_finite(K, what):
+    """A NaN reaches the rows that see it, all of a head's elements or a value's own, and nothing else."""
+    nh, nkv, hd, n = 4, 2, 24, 30
+    g = torch.Generator().manual_seed(1)
+    kp, vp = (torch.randn(1, nkv, *shape, generator=g).to(DEV) for shape in ((64, hd), (hd, 64)))
+    q = torch.randn(n, nh * hd, generator=g).to(DEV)
+    args = (_i32([[0]]), _i32([0]), _i32([0] * n), _i32(list(range(n))), nh, nkv, hd, 0.2, None)
+    want, out = torch.empty_like(q), torch.empty_like(q)
+    K.attn_plain(q, want, kp, vp, *args, most_keys=n)
+    hit = torch.zeros(n, nh, hd, dtype=torch.bool, device=DEV)
+    if what == "query":
+        q.view(n, nh, hd)[7, 1, 3] = float("nan")
+        hit[7, 1] = True
+    elif what == "key":
+        kp[0, 1, 17, 5] = float("nan")
+        hit[17:, 2:] = True
+    else:
+        vp[0, 0, 9, 17] = float("inf")
+        hit[17:, :2, 9] = True
+    K.attn_plain(q, out, kp, vp, *args, most_keys=n)
+    assert torch.equal(~torch.isfinite(out.view(n, nh, hd)), hit)
+    assert torch.equal(out.view(n, nh, hd)[~hit], want.view(n, nh, hd)[~hit])
+
+
 def test_attn_plain_far_key_wins(K):
     # among 700 keys, key 3 is made to dominate the last query's softmax: the output must be its value
     got, ref, vs = _attn_case(K, torch.float32, 2, 1, 32, [700], None, 0.5, seed=1, boost=3)
