@@ -121,7 +121,9 @@ __device__ __forceinline__ void load8(const float* p, float* v) {
 // where few tokens leave the chip idle) take the outputs in turn.
 // RR tokens a workgroup: eight where there are many, one where few tokens would leave the chip idle (a wave then holds
 // a whole row's share of loads in flight at once).
-template <typename T, bool WIDE, int RR>
+// OUT outputs a wave at a time: one, or two, w and w + nw, whose rows are one round trip to memory (a wave without a second
+// one reads its first again).
+template <typename T, bool WIDE, int RR, int OUT>
 __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ x, long ldx, const float* __restrict__ router,
                                                           const float* __restrict__ correction, int N, int K, int R, int groups,
                                                           int keep, int top, float scale, int* __restrict__ choice,
@@ -134,21 +136,19 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
     for (int e = threadIdx.x; e < R; e += blockDim.x) corr[e] = correction ? correction[e] : 0.f;
     const int t0 = blockIdx.x * RR;
     const int rows = min(RR, N - t0);
-    // Two outputs a wave at a time, w and w + nw (a wave without a second one reads its first again): with a few more outputs than
-    // waves the rows of both are one round trip to memory (17 outputs of 2,048, 6 tokens: 8.2 us one after the other, 7.3 us so; 3,001 tokens 37.6 and 31.8).
-    for (int r = w; r < Rt; r += 2 * nw) {
-        const bool second = r + nw < Rt;
+    for (int r = w; r < Rt; r += OUT * nw) {
+        const bool second = OUT == 2 && r + nw < Rt;
         const float* wr = router + (size_t)r * K;
         const float* wr2 = second ? wr + (size_t)nw * K : wr;
         float acc[RR], acc2[RR];
 #pragma unroll
         for (int i = 0; i < RR; ++i) acc[i] = acc2[i] = 0.f;
         if (WIDE) {
-#pragma unroll(RR == 1 ? 4 : 1)
+#pragma unroll(RR == 1 ? 4 : 3 - OUT)
             for (int k = 8 * lane; k < K; k += 512) {
-                float wk[8], wk2[8];
+                float wk[8], wk2[8] = {};
                 load8(wr + k, wk);
-                load8(wr2 + k, wk2);
+                if (OUT == 2) load8(wr2 + k, wk2);
 #pragma unroll
                 for (int i = 0; i < RR; ++i) {
                     const int t = t0 + (i < rows ? i : 0);
@@ -157,25 +157,25 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
                         acc[i] = fmaf(xv[j], wk[j], acc[i]);
-                        acc2[i] = fmaf(xv[j], wk2[j], acc2[i]);
+                        if (OUT == 2) acc2[i] = fmaf(xv[j], wk2[j], acc2[i]);
                     }
                 }
             }
         } else {
             for (int k = lane; k < K; k += 64) {
-                const float wk = wr[k], wk2 = wr2[k];
+                const float wk = wr[k], wk2 = OUT == 2 ? wr2[k] : 0.f;
 #pragma unroll
                 for (int i = 0; i < RR; ++i) {
                     const int t = t0 + (i < rows ? i : 0);
                     const float xv = ld(x + (size_t)t * ldx + k);
                     acc[i] = fmaf(xv, wk, acc[i]);
-                    acc2[i] = fmaf(xv, wk2, acc2[i]);
+                    if (OUT == 2) acc2[i] = fmaf(xv, wk2, acc2[i]);
                 }
             }
         }
 #pragma unroll
         for (int i = 0; i < RR; ++i) {
-            const float sum = wave_sum(acc[i]), sum2 = wave_sum(acc2[i]);
+            const float sum = wave_sum(acc[i]), sum2 = OUT == 2 ? wave_sum(acc2[i]) : 0.f;
             if (lane == 0) {
                 zs[i * Rt + r] = sum;
                 if (second) zs[i * Rt + r + nw] = sum2;
@@ -321,19 +321,24 @@ extern "C" int agave_route_rows(int dtype, const void* x, long ldx, const float*
     const bool wide = K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 32) == 0 && ((uintptr_t)router % 32) == 0;
     AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "route_rows: unknown dtype %d", dtype);
     const bool f32 = dtype == AGAVE_F32;
-    if (N <= 64) {
-        const size_t lds = (size_t)(2 * R + extra) * sizeof(float);
-#define ROUTE_GO(T_, W_) route_rows_kernel<T_, W_, 1><<<N, 1024, lds, stream>>>((const T_*)x, ldx, router, correction, N, K, R, groups, keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise)
-        if (f32 && wide) ROUTE_GO(float, true); else if (f32) ROUTE_GO(float, false); else if (wide) ROUTE_GO(bf16, true); else ROUTE_GO(bf16, false);
+    const int rows = N <= 64 ? 1 : 8, blocks = (N + rows - 1) / rows;
+    const int threads = blocks <= 512 ? 1024 : 256;            // (more waves to share the outputs while they all fit the chip at once)
+    const size_t lds = (size_t)(rows * (R + extra) + R) * sizeof(float);
+    // Two outputs a wave at a time where there are more than one for each wave.  With a token a workgroup not where the last two
+    // turns would be one for most waves, and of one or two tokens only where they are little more than one turn: a wave's second
+    // row is then work for nothing, or more than one compute unit takes from memory at once.  us, one and two, routers from memory, rows
+    // of 2,048: 16 outputs, 6 tokens 5.2 and 6.1, 3,001 tokens 18.6 and 22.0; 17 outputs 6.5 and 6.1, 26.3 and 22.2; 32 outputs, one
+    // token 8.7 and 9.0, 64 tokens 8.5 and 8.1; 48 outputs, 6 tokens 11.1 and 11.9, 3,001 tokens 41.1 and 37.6; 128 outputs, one
+    // token 24.3 and 25.1, 12 tokens 22.8 and 21.1.
+    const int waves = threads / 64, outputs = R + extra, last = outputs % (2 * waves);
+    const bool two = outputs > waves && (rows == 8 || (N > 2 ? last == 0 || last <= waves / 2 || last > waves : last > waves && last <= waves * 3 / 2));
+#define ROUTE_GO(T_, W_, RR_, OUT_) route_rows_kernel<T_, W_, RR_, OUT_><<<blocks, threads, lds, stream>>>((const T_*)x, ldx, router, correction, N, K, R, groups, \
+        keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise)
+#define ROUTE_ROWS(T_, W_) do { if (rows == 1 && two) ROUTE_GO(T_, W_, 1, 2); else if (rows == 1) ROUTE_GO(T_, W_, 1, 1); \
+        else if (two) ROUTE_GO(T_, W_, 8, 2); else ROUTE_GO(T_, W_, 8, 1); } while (0)
+    if (f32 && wide) ROUTE_ROWS(float, true); else if (f32) ROUTE_ROWS(float, false); else if (wide) ROUTE_ROWS(bf16, true); else ROUTE_ROWS(bf16, false);
+#undef ROUTE_ROWS
 #undef ROUTE_GO
-    } else {
-        const int blocks = (N + 7) / 8;
-        const size_t lds = (size_t)(9 * R + 8 * extra) * sizeof(float);
-        const int threads = blocks <= 512 ? 1024 : 256;        // (more waves to share the outputs while they all fit the chip at once)
-#define ROUTE_GO(T_, W_) route_rows_kernel<T_, W_, 8><<<blocks, threads, lds, stream>>>((const T_*)x, ldx, router, correction, N, K, R, groups, keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise)
-        if (f32 && wide) ROUTE_GO(float, true); else if (f32) ROUTE_GO(float, false); else if (wide) ROUTE_GO(bf16, true); else ROUTE_GO(bf16, false);
-#undef ROUTE_GO
-    }
     AGAVE_LAUNCH_CHECK("route_rows");
     return 0;
 }

@@ -584,3 +584,22 @@ def test_routed_rows_at_any_element(tm):
         assert bool((held[:at] == 7.0).all()) and bool((held[at + y.numel():] == 7.0).all())
         rows.append(y[place.long()])
     assert all(torch.equal(r, rows[0]) for r in rows) and bool(torch.isfinite(rows[0]).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("outputs", [2, 15, 16, 17, 24, 25, 32, 33, 40, 41, 48, 49, 64])
+def test_router_products(dtype, outputs):
+    """Every output's product, whether a wave makes one or two of them at a time: fewer outputs than waves, some more, whole and broken
+    turns; a token a workgroup and eight, whole and broken stretches of a row."""
+    from agave_amd.ops import routed
+    g = torch.Generator().manual_seed(outputs)
+    for k in (24, 100, 1032):
+        for n in (1, 2, 3, 64, 65, 70):
+            x, router = torch.randn(n, k, generator=g).to(dtype).to(DEV), torch.randn(outputs, k, generator=g).to(DEV)
+            choice, weight = torch.full((n, 1), -1, dtype=torch.int32, device=DEV), torch.zeros(n, 1, device=DEV)
+            rest = torch.full((n, outputs - 1), float("nan"), device=DEV)
+            routed.route_rows(x, router, None, 1, 1, 1, 2.0, choice, weight, softmax_top=True, extra_out=rest)
+            assert bool((choice == 0).all()) and bool((weight == 2.0).all())
+            # (sums of k products in 32-bit are off by at most k 2^-24 of the sum of their sizes)
+            bound = k * 2.0 ** -24 * (x.double().abs() @ router[1:].double().abs().T)
+            assert bool(((rest.double() - x.double() @ router[1:].double().T).abs() <= bound).all()), (k, n)
