@@ -570,42 +570,37 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(const int* __restrict_
     }
 }
 
-// Up to 64 pairs and 64 experts (a decode step of few tokens): one wave, a lane per pair.  A pair's rank within its expert is a
-// count of the lanes below it, so nothing meets in LDS and no thread walks the experts alone.  24 pairs of 16 experts: 4.7 us,
-// with the kernel above 5.3.
+// Up to 64 pairs and 64 experts (a decode step of few tokens): one wave, a lane per pair and per expert, the experts' tiles counted
+// up across the lanes, so that no thread walks the experts alone.  us, with the kernel above and so, tiles
+// of 16: 8 pairs of 8 experts 3.2 and 2.2, 24 of 16 4.4 and 2.4, 32 of 64 9.1 and 3.1.
 #define FEW_CAP (65 * 64)      // sorted rows: 64 experts and a tile more, in tiles of up to 64
 __global__ __launch_bounds__(64) void route_sort_few_kernel(const int* __restrict__ choice, int P, int E, int TM, int cap, int max_tiles,
                                                             int* __restrict__ place, int* __restrict__ sorted_pair,
                                                             int* __restrict__ tile_expert) {
+    __shared__ int count[64], first[64], sorted[FEW_CAP];
     const int lane = threadIdx.x;
-    const int mine = lane < P ? choice[lane] : -1;
-    const unsigned long long below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
-    __shared__ int sorted[FEW_CAP];
+    const int chosen = lane < P ? choice[lane] : -1, mine = chosen < E ? chosen : -1;
+    count[lane] = 0;
     for (int r = lane; r < cap; r += 64) sorted[r] = -1;
-    int row = -1, count = 0;                               // this lane's pair's row; pairs of expert `lane`
-    int tile = 0;
-    for (int e = 0; e < E; ++e) {
-        const unsigned long long who = __ballot(mine == e);
-        const int n = __popcll(who);
-        if (mine == e) row = tile * TM + __popcll(who & below);
-        if (lane == e) count = tile;                        // (its first tile, for the table below)
-        tile += (n + TM - 1) / TM;
+    __syncthreads();
+    const int rank = mine >= 0 ? atomicAdd(&count[mine], 1) : 0;
+    __syncthreads();
+    const int tiles = (count[lane] + TM - 1) / TM;           // of expert `lane`
+    int upto = tiles;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+        const int below = __shfl_up(upto, o);
+        if (lane >= o) upto += below;
     }
-    // expert of a tile: the last one that starts at or before it and has a tile
-    for (int t = lane; t < max_tiles; t += 64) {
-        int ex = -1;
-        for (int e = 0; e < E; ++e) {
-            const int first = __builtin_amdgcn_readlane(count, e), next = e + 1 < E ? __builtin_amdgcn_readlane(count, e + 1) : tile;
-            if (t >= first && t < next) ex = e;
-        }
-        tile_expert[t] = ex;
-    }
-    // (a wave's LDS accesses happen in the order they were issued)
-    __builtin_amdgcn_wave_barrier();
-    if (row >= 0 && row < cap) sorted[row] = lane;
-    __builtin_amdgcn_wave_barrier();
+    first[lane] = (upto - tiles) * TM;
+    for (int t = upto - tiles; t < upto; ++t) tile_expert[t] = lane;
+    for (int t = __shfl(upto, 63) + lane; t < max_tiles; t += 64) tile_expert[t] = -1;
+    __syncthreads();
+    const int row = mine >= 0 ? first[mine] + rank : -1;
+    if (row >= 0) sorted[row] = lane;                        // (cap holds every pair and every expert's padding)
+    __syncthreads();
     for (int r = lane; r < cap; r += 64) sorted_pair[r] = sorted[r];
-    if (lane < P) place[lane] = row < cap ? row : -1;
+    if (lane < P) place[lane] = row;
 }
 
 extern "C" int agave_route_sort(const int* choice, int P, int E, int TM, int cap, int max_tiles, int* place, int* sorted_pair,
