@@ -418,8 +418,8 @@ __global__ __launch_bounds__(256) void routed_down_plain_kernel(const T* __restr
 
 // out[t] = sum over the token's pairs of weight * (expert row, or the input row for an identity expert) + shared[t].
 // `place` (may be null): where pair p's row lies in y (a sorted list); null: at p.
-// A thread makes V neighbours of a row: 4 where rows and sizes allow accesses of four elements (bound by memory: 3,001
-// tokens of 4 pairs and 2,048 columns, 135 MB, 24.8 us; one element a thread took 39.7), 1 otherwise.
+// A thread makes V neighbours of a row: 4 in steps of many tokens where rows and sizes allow accesses of four elements (bound by
+// memory: 3,001 tokens of 4 pairs and 2,048 columns, 135 MB, 21.6 us; one element a thread 35.8), 1 otherwise.
 template <int V, typename T> __device__ __forceinline__ void load_few(const T* p, float* v);
 template <> __device__ __forceinline__ void load_few<1, float>(const float* p, float* v) { v[0] = *p; }
 template <> __device__ __forceinline__ void load_few<1, bf16>(const bf16* p, float* v) { v[0] = bf16_to_f32(*p); }
@@ -509,7 +509,9 @@ extern "C" int agave_routed_combine(int dtype, const float* y, const int* place,
     if (N == 0) return 0;
     AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "routed_combine: unknown dtype %d", dtype);
     const uintptr_t wide = 4 * (dtype == AGAVE_F32 ? 4 : 2);           // bytes of four neighbours in a row
-    const bool fours = hidden % 4 == 0 && ldx % 4 == 0 && ldo % 4 == 0 && (!shared || lds % 4 == 0) && (uintptr_t)x % wide == 0 &&
+    // (Few elements leave most of the chip without a thread when each takes four.  us, 1 and 4, bfloat16, 2,048 columns of 4 pairs: 6
+    // tokens 2.8 and 3.1, 64 3.0 and 3.2, 100 3.24 and 3.16, 300 4.8 and 3.5; 4,096 columns of 2 pairs, 32 2.84 and 2.96, 48 2.95 and 2.89.)
+    const bool fours = (long)N * hidden >= 3 << 16 && hidden % 4 == 0 && ldx % 4 == 0 && ldo % 4 == 0 && (!shared || lds % 4 == 0) && (uintptr_t)x % wide == 0 &&
                        (uintptr_t)out % wide == 0 && (uintptr_t)shared % wide == 0 && (uintptr_t)y % 16 == 0;
     const long blocks = ((long)N * hidden / (fours ? 4 : 1) + 255) / 256;
 #define COMBINE_GO(T_, V_) routed_combine_kernel<T_, V_><<<(unsigned)blocks, 256, 0, stream>>>(y, place, choice, weight, (const T_*)x, ldx, \
