@@ -100,16 +100,19 @@ def tile_plan(n_pairs: int, n_experts: int, tile_order: bool = False, ff: int = 
 
     Weights row by row: tiles of 64 rows where an expert gets some 32 pairs or more on average, of 16 otherwise.
     Weights in tile order (``tile_order``, experts of ``ff`` inner rows and ``hidden`` columns): 128 from 128 pairs an expert
-    on; 64 from 16 pairs an expert on where their workgroups (64 inner rows, 128 columns each) about fill the chip; below that
-    16.  Where neither product has the columns that the kernel of few pairs streams, 64 from two pairs an expert on.  us, both
-    products in tiles of 16 and of 64: 16 experts of 2,048 by 2,048 4 pairs an expert 85 and 89, 8 87 and 88, 12 90 and 89, 16 114
-    and 91; 64 of 512 by 2,048 4 88 and 101, 12 100 and 104, 16 112 and 106; 32 of 1,024 by 1,024 8 49 and 53, 16 63 and 54; 16 of
-    1,536 by 1,536 2 63 and 57, 16 91 and 60.  With workgroups for a part of the chip: 8 of 512 by 512 16 12 and 20, 4 of 2,048 by 1,024
-    16 23 and 34.  In tiles of 64 and of 128, 16 experts of 2,048 by 2,048: 100 pairs an expert 124 and 125, 150 162 and 137."""
+    on where their workgroups (128 inner rows, 256 columns each) fill the chip; else 64 from 32 pairs an expert on, and from
+    16 on where their workgroups (64 inner rows, 128 columns each) about fill the chip; below that 16.  Where neither product
+    has the columns that the kernel of few pairs streams, 64 from two pairs an expert on.  us, both products in tiles of 16 and
+    of 64: 16 experts of 2,048 by 2,048 4 pairs an expert 85 and 89, 8 87 and 88, 12 90 and 89, 16 114 and 91; 64 of 512 by
+    2,048 4 88 and 101, 12 100 and 104, 16 112 and 106; 32 of 1,024 by 1,024 8 49 and 53, 16 63 and 54; 16 of 1,536 by 1,536
+    2 63 and 57, 16 91 and 60.  With workgroups for a part of the chip: 8 of 512 by 512 16 12 and 20, 4 of 2,048 by 1,024 16 23
+    and 34.  In tiles of 64 and of 128: 16 experts of 2,048 by 2,048 64 pairs an expert 124 and 128, 128 162 and 150, 750 532
+    and 408; 64 of 512 by 2,048 128 169 and 172, 375 349 and 285; 4 of 2,048 by 1,024 512 72 and 82, 1,500 126 and 124; 8 of
+    512 by 512 128 25 and 44, 750 45 and 53; 16 of 32 by 32 375 15 and 24 (without LDS 16)."""
     tm = 64 if n_pairs >= 32 * n_experts else 16
     if tile_order:
-        live = min(n_pairs, n_experts)
-        if n_pairs >= 128 * n_experts:
+        live, full = min(n_pairs, n_experts), n_pairs // 128
+        if n_pairs >= 128 * n_experts and full * (ff // 128) >= 256 and full * (hidden // 256) >= 128:
             tm = 128
         elif (n_pairs >= (16 if ff in STREAMED or hidden in STREAMED else 2) * n_experts
               and live * (ff // 64) >= 256 and live * (hidden // 128) >= 128):

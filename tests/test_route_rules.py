@@ -23,3 +23,15 @@ def test_sequences_among_neighbouring_rows(n_new, run):
     step = Step(**{**dict.fromkeys(Step.__dataclass_fields__), "cu": cu, "n_new": n_new, "seqs_a_run": {}})
     seq = [i for i, n in enumerate(n_new) for _ in range(n)]
     assert step.most_seqs(run) == step.most_seqs(run) == max(len(set(seq[a:a + run])) for a in range(0, len(seq), run))
+
+
+@pytest.mark.parametrize("pairs,experts,ff,hidden,rows", [
+    (8192, 16, 2048, 2048, 128), (2048, 16, 2048, 2048, 128), (2047, 16, 2048, 2048, 64), (256, 16, 2048, 2048, 64), (255, 16, 2048, 2048, 16),
+    (6002, 16, 32, 32, 64), (9003, 12, 96, 64, 64), (6002, 8, 512, 512, 64), (2048, 4, 2048, 1024, 64), (8192, 64, 512, 2048, 128),
+    (31, 1, 512, 512, 16), (32, 1, 512, 512, 64)])
+def test_rows_of_a_tile_of_sorted_pairs(pairs, experts, ff, hidden, rows):
+    """The largest tiles only where their workgroups fill the chip: small experts' tiles would be mostly empty."""
+    from agave_amd.ops import routed
+    tm, tiles, cap = routed.tile_plan(pairs, experts, True, ff, hidden)
+    assert tm == rows and cap == tiles * tm and tiles >= -(-pairs // tm) + experts
+    assert routed.tile_plan(pairs, experts)[0] == (64 if pairs >= 32 * experts else 16)
