@@ -779,8 +779,9 @@ __global__ __launch_bounds__(256) void routed_product_mfma_kernel(const bf16* __
 // blocks (loaded again for every block, the rows were a third and a half of what the kernel above asks for) and streams its
 // weights, two tiles of a kilobyte a step, through a ring of NS steps in LDS of its own: it waits for nobody but its own loads,
 // and the loads of the next block's first steps are on their way while this one's sums meet in LDS.
-// Measured, both products, 16 experts of 2,048 by 2,048, 4 a row: 2 rows 47 us, 4 rows 60 us, 6 rows 70 us (330 MB, 4.7 TB/s);
-// with the kernel above 69, 81 and 89 us.
+// Measured, us, both products, with the kernel above and so, 1, 2, 4 and 16 rows: 16 experts of 2,048 by 2,048, 4 a row, 34 44 78 117
+// and 30 43 57 87; 32 of 1,024 by 1,024, 4 a row, 18 21 27 49 and 15 20 24 38; 8 of 4,096 by 4,096, 2 a row, 44 118 116 185 and 48
+// 96 107 153; 8 of 4,096 inner rows by 1,024, 2 a row, 25 33 40 49 and 21 27 39 46.
 template <int KQ, bool GATED>
 __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* __restrict__ x, long ldx, const int* __restrict__ sorted_pair,
                                                                     const int* __restrict__ tile_expert, const uint4* __restrict__ w0,
@@ -866,10 +867,13 @@ __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* 
     __builtin_amdgcn_s_waitcnt(0x0F70);                           // loads past the last step land before the LDS goes to another workgroup
 }
 
+// The columns that the kernel above is built for (its rows take K / 32 registers a lane, and the ring's places have to come out even).
+extern "C" int agave_routed_few_takes(int K) { return K == 1024 || K == 2048 || K == 4096; }
+
 template <bool GATED>
 static bool launch_routed_few(const void* x, long ldx, const int* sorted_pair, const int* tile_expert, int max_tiles, const void* w0,
                               const void* w1, void* out, int top, int live, int n_out, int K, int act, float p0, float p1, hipStream_t stream) {
-    if (K != 1024 && K != 2048 && K != 4096) return false;
+    if (!agave_routed_few_takes(K)) return false;
     const int all = (n_out + (GATED ? 15 : 31)) / (GATED ? 16 : 32);
     // Blocks a workgroup: the fewest with which all workgroups run at once, two to a compute unit at most (some 450 where 512
     // have a place: `live` is an expectation).  Both products, 4 rows: 75.8, 63.0, 66.7 us with 2, 4, 5 blocks of the gate;

@@ -15,6 +15,7 @@ kernels.register_signatures(LIBRARY, {
     "agave_route_topk": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P, _P],
     "agave_routed_experts_plain": [_I, _P, _L, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "agave_route_rows": [_I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _P, _I, _I, _P],
+    "agave_routed_few_takes": [_I],
     "agave_route_sort": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     "agave_routed_experts_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "agave_routed_combine": [_I, _P, _P, _P, _P, _P, _L, _P, _L, _P, _P, _L, _I, _I, _I, _I, _P],
@@ -91,7 +92,7 @@ def combine(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: to
                  lds, ptr(shared_gate) if shared is not None else None, ptr(out), ldo, n, top, n_experts, hidden, stream())
 
 
-STREAMED = (1024, 2048, 4096)        # columns for which the kernel of few pairs is built
+STREAMED = (1024, 2048, 4096)        # columns for which the kernel of few pairs is built (agave_routed_few_takes)
 
 
 def tile_plan(n_pairs: int, n_experts: int, tile_order: bool = False, ff: int = 0, hidden: int = 0):

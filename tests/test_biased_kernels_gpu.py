@@ -603,3 +603,9 @@ def test_router_products(dtype, outputs):
             # (sums of k products in 32-bit are off by at most k 2^-24 of the sum of their sizes)
             bound = k * 2.0 ** -24 * (x.double().abs() @ router[1:].double().abs().T)
             assert bool(((rest.double() - x.double() @ router[1:].double().T).abs() <= bound).all()), (k, n)
+
+
+def test_columns_that_the_kernel_of_few_pairs_takes():
+    """The rule for the tiles of sorted pairs and the kernel's launch name the same columns."""
+    from agave_amd.ops import routed
+    assert tuple(k for k in range(32, 16385, 32) if routed._lib().agave_routed_few_takes(k)) == routed.STREAMED
