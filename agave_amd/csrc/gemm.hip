@@ -14,6 +14,34 @@
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
+// ---------------------------------------------------------------- one or two rows that fours do not fit
+// A wave per column of C, the lanes along K.  Bound by its trips to memory: a lane's loads are single elements, and a wave's 64 lie
+// next to each other, where the kernel below asks for sixteen rows' lines with each.  The sums are held in double, which costs
+// nothing here: in 32 bits they would be a lane's few products added across 64 lanes, and up to a third less exact than below.
+// Measured, us, with the kernel below and so: 1 row by 130 x 2,049 in 32 bits 12.7 and 7.4, in bfloat16 by 30,000 x 515 40 and 25; 2 rows
+// by 16 x 4,097 30 and 16.  Errors against 64 bits 0.25 to 0.3e-7 after 0.7 to 1.1e-7.
+#define FEW_ROWS 2
+template <typename TA, typename TW, typename TC>
+__global__ __launch_bounds__(256) void gemm_f32_few_rows_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw,
+                                                                TC* __restrict__ C, long ldc, int M, int N, int K) {
+    const int lane = threadIdx.x & 63, n = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (n >= N) return;
+    const TW* w = W + (size_t)n * ldw;
+    const TA* a[FEW_ROWS] = {A, A + (size_t)(M - 1) * lda};   // (a single row is made twice)
+    double acc[FEW_ROWS] = {};
+#pragma unroll 8
+    for (int k = lane; k < K; k += 64) {
+        const double wk = ld(w + k);
+#pragma unroll
+        for (int m = 0; m < FEW_ROWS; ++m) acc[m] = fma((double)ld(a[m] + k), wk, acc[m]);
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2)
+#pragma unroll
+        for (int m = 0; m < FEW_ROWS; ++m) acc[m] += __shfl_xor(acc[m], o);
+    if (lane < M) st(C + (size_t)lane * ldc + n, (float)acc[lane == 0 ? 0 : 1]);
+}
+
 // ---------------------------------------------------------------- few rows
 // A workgroup makes 16 columns of C for up to 64 rows (MT tiles of 16; more rows are cut into groups of
 // 64, blockIdx.y); its NW waves share K and add their sums through LDS.  Per k-step of 16 a lane brings
@@ -103,7 +131,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const TA* __re
 #define TN 64
 #define TK 32
 #define TS (TK + 4)
-template <typename TA, typename TW, typename TC, int BM, bool VEC>
+// S: running sums of an element; four where few rows come here that groups of rows, with as many, would otherwise take.
+template <typename TA, typename TW, typename TC, int BM, bool VEC, int S>
 __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw,
                                                              TC* __restrict__ C, long ldc, int M, int N, int K, int m_tiles, int tiles) {
     constexpr int AR = BM / 32;                                   // rows of A a thread brings per stage
@@ -135,7 +164,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const TA* __restric
 #pragma unroll
         for (int i = 0; i < 2; ++i) *(f32x4_t*)&Ws[b][(lr + 32 * i) * TS + lk] = rw[i];
     };
-    f32x16_t acc = {};
+    f32x16_t sums[S] = {};
     fetch(0);
     put(0);
     __syncthreads();
@@ -149,11 +178,13 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const TA* __restric
             const int o = 8 * j + (BM == 64 ? 0 : 16 * wk);
             const f32x4_t va = *(const f32x4_t*)(pa + o), vw = *(const f32x4_t*)(pw + o);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va[e], vw[e], acc, 0, 0, 0);
+            for (int e = 0; e < 4; ++e) sums[e % S] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[e], vw[e], sums[e % S], 0, 0, 0);
         }
         if (k0 + TK < K) put(b ^ 1);                              // (the other buffer was last read before the barrier below)
         __syncthreads();
     }
+    f32x16_t acc = sums[0];
+    if (S == 4) acc = (sums[0] + sums[1]) + (sums[2] + sums[3]);
     if (BM == 32) {                                               // the second pair's sums, 32 x 64 floats, through the first buffer
         static_assert(64 * 17 * 2 <= 2 * 32 * TS, "a wave's sums, padded by one float a lane, fit");
         float* half = &As[0][0] + wn * 64 * 17;
@@ -195,20 +226,29 @@ static void launch_skinny(const TA* A, long lda, const TW* W, long ldw, TC* C, l
 
 template <typename TA, typename TW, typename TC, bool VEC>
 static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long ldc, int M, int N, int K, hipStream_t stream) {
+    if (!VEC && M <= FEW_ROWS) {
+        gemm_f32_few_rows_kernel<TA, TW, TC><<<(N + 3) / 4, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+        return;
+    }
     if (M <= 16) return launch_skinny<TA, TW, TC, 1, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
-    if (M <= 32) return launch_skinny<TA, TW, TC, 2, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
-    // from 65 rows on: tiles as soon as the smaller ones give every compute unit one (80 rows by 2,048 x 2,048, 96 of
-    // them: 47 us tiled, 24 us in groups of 64 rows; 200 rows, 224: 47 us in groups, 300 rows, 320: 52 us tiled)
+    // from 65 rows on (17 where fours do not fit and K is not short): tiles as soon as the smaller ones give every compute unit one (80 rows by
+    // 2,048 x 2,048, 96 of them: 47 us tiled, 24 us in groups of 64 rows; 200 rows, 224: 47 us in groups, 300 rows, 320: 52 us tiled;
+    // 30,000 x 515, 469 a row of tiles: 17 rows 54.7 in groups and 25.3 tiled, 64 rows 108 and 39)
     const int n_tiles = (N + TN - 1) / TN;
     const long small_tiles = (long)n_tiles * ((M + 31) / 32);
-    if (M <= SKINNY_M || small_tiles < COMPUTE_UNITS) return launch_skinny<TA, TW, TC, 4, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
-    const bool large = (long)n_tiles * ((M + 63) / 64) >= COMPUTE_UNITS;
+    if ((M <= SKINNY_M && (VEC || K < 256)) || small_tiles < COMPUTE_UNITS) {
+        if (M <= 32) return launch_skinny<TA, TW, TC, 2, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+        return launch_skinny<TA, TW, TC, 4, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+    }
+    const bool few = M <= SKINNY_M, large = !few && (long)n_tiles * ((M + 63) / 64) >= COMPUTE_UNITS;
     const int bm = large ? 64 : 32, m_tiles = (M + bm - 1) / bm, tiles = m_tiles * n_tiles;
     const int grid = (tiles + 7) / 8 * 8;
-    if (large)
-        gemm_f32_tiled_kernel<TA, TW, TC, 64, VEC><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
+    if (few)
+        gemm_f32_tiled_kernel<TA, TW, TC, 32, VEC, VEC ? 1 : 4><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
+    else if (large)
+        gemm_f32_tiled_kernel<TA, TW, TC, 64, VEC, 1><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
     else
-        gemm_f32_tiled_kernel<TA, TW, TC, 32, VEC><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
+        gemm_f32_tiled_kernel<TA, TW, TC, 32, VEC, 1><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
 }
 
 template <typename T> static bool rows_of_fours(const void* p, long ld) {

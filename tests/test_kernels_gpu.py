@@ -295,6 +295,38 @@ def test_gemm_plain_tiles(K, ta, tw, m, n, k):
         assert bool((c[m] == 7.0).all()) and bool((c[:, n:] == 7.0).all())       # nothing outside is written
 
 
+@pytest.mark.parametrize("ta,tw", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16),
+                                   (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("m,n,k", [(257, 3300, 36), (300, 3300, 515), (320, 4161, 260), (1100, 960, 129),           # tiles of 64 rows
+                                   (97, 5500, 68), (200, 2400, 131),                                                 # of 32
+                                   (17, 16400, 257), (64, 8200, 259), (33, 8200, 515),                               # of 32 for few rows that fours do not fit
+                                   (2, 70, 33), (2, 515, 1027), (1, 33, 4097)])                                      # a wave a column
+def test_gemm_plain_large_tiles_and_odd_rows(K, ta, tw, m, n, k):
+    """Enough tiles to fill the chip, their last rows and columns broken, whole and broken stretches of k; and rows that four
+    elements do not fit, few and many.  Every output is within K 2^-24 of the sum of its products' sizes."""
+    g = torch.Generator().manual_seed(m * 7 + n)
+    a, w = torch.randn(m, k + 3, generator=g).to(ta).to(DEV), torch.randn(n, k, generator=g).to(tw).to(DEV)
+    for x in (a[:, :k].contiguous(), a[:, 3:]):
+        c = torch.full((m + 1, n + 2), 7.0, device=DEV)
+        K.gemm_plain(x, w, c[:m, :n])
+        bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        assert bool(((c[:m, :n].double() - x.double() @ w.double().T).abs() <= bound).all())
+        assert bool((c[m] == 7.0).all()) and bool((c[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(2, 40, 17), (70, 40, 18), (300, 3300, 20), (290, 3300, 18), (97, 5500, 20), (17, 16400, 258), (40, 8200, 257)])
+def test_gemm_plain_special_values_in_every_kernel(K, m, n, k):
+    """A NaN or an infinity stays in its row and column, and zeros behind the last k meet zeros only."""
+    a, w = torch.ones(m, k, device=DEV), torch.ones(n, k, device=DEV)
+    a[1, k - 1], w[5, 2] = float("nan"), float("inf")
+    c = torch.empty(m, n, device=DEV)
+    K.gemm_plain(a, w, c)
+    want = torch.full((m, n), float(k), device=DEV)
+    want[:, 5] = float("inf")
+    want[1] = float("nan")
+    assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c[~c.isnan()], want[~want.isnan()])
+
+
 def test_gemm_plain_special_values(K):
     """A NaN or an infinity stays in its row and column, and zeros behind the last k meet zeros only."""
     for m in (3, 70):
