@@ -70,12 +70,13 @@ __global__ void short_conv_kernel(const float* __restrict__ u, long ldu, const f
     }
 }
 
-// Steps of many tokens: a thread takes CONV_ROWS neighbouring rows of one channel, whose inputs it asks for together, and slides
-// the taps' window along them; where a row starts another sequence than the row before it the window is filled as above.  Bound
-// by memory (every input read once, every output written once; a thread per row and channel reads each input TAPS times and
-// finds out its row's place for itself): 3,001 rows of 4,352 channels 96 us so, 27 us here.
+// Steps of many tokens: a thread takes CONV_ROWS neighbouring rows of one channel, whose inputs it asks for together, and slides the
+// taps' window along them.  Where a row is the first of its sequence the window comes from the sequence's state: asked for with
+// the rows where several sequences may begin among them (MANY), since one after another they are trips to memory, and on the way
+// otherwise, since it would cost registers.  Bound by memory (every input read once, every output written once; a thread per row and
+// channel reads each input TAPS times and finds out its row's place for itself): 3,001 rows of 4,352 channels 97 us so, 27 us here.
 #define CONV_ROWS 16
-template <bool SILU, int TAPS>
+template <bool SILU, int TAPS, bool MANY>
 __global__ __launch_bounds__(256) void short_conv_rows_kernel(const float* __restrict__ u, long ldu, const float* __restrict__ w,
                                                               const float* __restrict__ bias, float* __restrict__ y, long ldy,
                                                               const float* __restrict__ state, const int* __restrict__ tok_seq,
@@ -90,22 +91,43 @@ __global__ __launch_bounds__(256) void short_conv_rows_kernel(const float* __res
     for (int i = 0; i < CONV_ROWS; ++i) x[i] = u[(size_t)min(t0 + i, n_tokens - 1) * ldu + c];
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) wt[j] = w[(size_t)c * TAPS + j];
+    // (everything about a row is the same for the whole workgroup; rows behind the last repeat it)
+    int seq[MANY ? CONV_ROWS : 1];
+    float held[MANY ? CONV_ROWS : 1][TAPS - 1];
+    if constexpr (MANY) {
+#pragma unroll
+        for (int i = 0; i < CONV_ROWS; ++i) seq[i] = tok_seq[min(t0 + i, n_tokens - 1)];
+        int slot[CONV_ROWS];
+#pragma unroll
+        for (int i = 0; i < CONV_ROWS; ++i) slot[i] = slots[seq[i]];
+#pragma unroll
+        for (int i = 1; i < CONV_ROWS; ++i)
+            if (seq[i] != seq[i - 1])                           // (a sequence's rows follow one another, so this is its first)
+#pragma unroll
+                for (int j = 0; j < TAPS - 1; ++j) held[i][j] = state[((size_t)slot[i] * (TAPS - 1) + j) * C + c];
+    }
     int before = -1;
 #pragma unroll
     for (int i = 0; i < CONV_ROWS; ++i) {
         const int t = t0 + i;
-        if (t >= n_tokens) break;                               // (the same for the whole workgroup, as is everything about the row)
-        const int s = tok_seq[t];
-        if (s != before) {
-            const int p = tok_pos[t], p0 = pos0[s];
-            const float* st_c = state + ((size_t)slots[s] * (TAPS - 1)) * C + c;
+        if (t >= n_tokens) break;
+        if (MANY && i > 0) {
+            if (seq[i] != seq[i - 1])
 #pragma unroll
-            for (int j = 1; j < TAPS; ++j) {
-                const int r = p - TAPS + j;                     // the inputs that the row before this one would have left, oldest first
-                if (r >= p0) in[j] = u[(size_t)(t - (p - r)) * ldu + c] + ib;
-                else in[j] = st_c[(size_t)(r - (p0 - (TAPS - 1))) * C];
+                for (int j = 1; j < TAPS; ++j) in[j] = held[i][j - 1];
+        } else {
+            const int s = tok_seq[t];
+            if (s != before) {
+                const int p = tok_pos[t], p0 = pos0[s];
+                const float* st_c = state + ((size_t)slots[s] * (TAPS - 1)) * C + c;
+#pragma unroll
+                for (int j = 1; j < TAPS; ++j) {
+                    const int r = p - TAPS + j;                 // the inputs that the row before this one would have left, oldest first
+                    if (r >= p0) in[j] = u[(size_t)(t - (p - r)) * ldu + c] + ib;
+                    else in[j] = st_c[(size_t)(r - (p0 - (TAPS - 1))) * C];
+                }
+                before = s;
             }
-            before = s;
         }
 #pragma unroll
         for (int j = 1; j < TAPS; ++j) in[j - 1] = in[j];
@@ -140,10 +162,11 @@ __global__ void conv_state_kernel(const float* __restrict__ u, long ldu, float* 
         if (i < taps - 1) st_c[(size_t)i * C] = keep[i];
 }
 
+// most_seqs: of how many sequences at most any 16 rows are, from a multiple of 16 on (the results do not depend on it).
 extern "C" int agave_short_conv(const float* u, long ldu, const float* w, const float* bias, float* y, long ldy, float* state,
                                 const int* tok_seq, const int* tok_pos, const int* cu, const int* pos0,
                                 const int* slots, int n_tokens, int n_seqs, int C, int taps, int silu,
-                                int one_token_each, const float* in_bias, hipStream_t stream) {
+                                int one_token_each, int most_seqs, const float* in_bias, hipStream_t stream) {
     AGAVE_CHECK(n_tokens >= 0 && n_seqs >= 0 && C > 0, "short_conv: bad sizes N=%d B=%d C=%d", n_tokens, n_seqs, C);
     AGAVE_CHECK(taps >= 1 && taps <= CONV_MAX_TAPS, "short_conv: %d taps (1 to %d are supported)", taps, CONV_MAX_TAPS);
     AGAVE_CHECK(ldu >= C && ldy >= C, "short_conv: a row stride is below %d", C);
@@ -153,12 +176,17 @@ extern "C" int agave_short_conv(const float* u, long ldu, const float* w, const 
     if (n_tokens == 0) return 0;
     const int threads = C >= 256 ? 256 : 64;
     const dim3 grid((C + threads - 1) / threads, n_tokens), rows((C + threads - 1) / threads, (n_tokens + CONV_ROWS - 1) / CONV_ROWS);
-#define CONV_GO(SILU_, TAPS_) short_conv_rows_kernel<SILU_, TAPS_><<<rows, threads, 0, stream>>>(u, ldu, w, bias, y, ldy, state, tok_seq, tok_pos, \
-                                                                                              pos0, slots, n_tokens, C, in_bias)
+#define CONV_ROWS_GO(SILU_, TAPS_, MANY_) short_conv_rows_kernel<SILU_, TAPS_, MANY_><<<rows, threads, 0, stream>>>(u, ldu, w, bias, y, ldy, state, tok_seq, \
+                                                                                                    tok_pos, pos0, slots, n_tokens, C, in_bias)
+#define CONV_GO(SILU_, TAPS_) do { if (many) CONV_ROWS_GO(SILU_, TAPS_, true); else CONV_ROWS_GO(SILU_, TAPS_, false); } while (0)
     // (With fewer workgroups of the kernel for many rows, its rows one after another take longer than they save.  us, a row a
     // thread and many, four taps: 4,352 channels 128 rows, 136 workgroups, 7.8 and 8.1, 256 rows, 272, 10.5 and 8.6; 12,288
-    // channels 64 rows, 192, 8.7 and 8.2; 512 channels 1,000 rows, 126, 7.2 and 8.0, 3,001 rows, 376, 12.1 and 8.9.)
-    if (!one_token_each && taps >= 2 && taps <= 4 && (long)rows.x * rows.y >= 192) {
+    // channels 64 rows, 192, 8.7 and 8.2; 512 channels 1,000 rows, 126, 7.2 and 8.0, 3,001 rows, 376, 12.1 and 8.9; two taps: 1,000
+    // channels 990 rows, 248, 8.6 and 9.0.  States asked for on the way and ahead, four taps: 60 sequences of one row and one of 1,000,
+    // 1,000 channels, 268 workgroups, 14.0 and 10.4 (a row a thread 10.8); 400 of five rows, 12,288 channels, 6,000, 68.7 and 72.7.)
+    const long wgs = (long)rows.x * rows.y;
+    const bool many = most_seqs > 2 ? wgs <= 3072 : most_seqs == 2 && wgs <= 512;
+    if (!one_token_each && taps >= 2 && taps <= 4 && wgs >= (taps == 2 ? 256 : 192)) {
         if (silu) {
             if (taps == 2) CONV_GO(true, 2); else if (taps == 3) CONV_GO(true, 3); else CONV_GO(true, 4);
         } else {

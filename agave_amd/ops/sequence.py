@@ -19,7 +19,7 @@ from .kernels import _P, _I, _L, _F, _dev, _f32vec, _i32, dt, ptr, stream
 LIBRARY = "sequence"
 
 kernels.register_signatures(LIBRARY, {
-    "agave_short_conv": [_P, _L, _P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P],
+    "agave_short_conv": [_P, _L, _P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _P],
     "agave_head_norm_rope_rows": [_I, _P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _F, _F, _I, _I, _P, _I, _I, _P, _P,
                                   _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
     "agave_talk_attention": [_I, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I,
@@ -33,6 +33,7 @@ kernels.register_signatures(LIBRARY, {
 })
 
 MAX_TAPS = 8
+CONV_ROWS = 16            # neighbouring rows that a thread of the kernel for long steps takes
 DELTA, FORGET, SSD = 0, 1, 2
 
 
@@ -69,7 +70,8 @@ def short_conv(u: torch.Tensor, weight: torch.Tensor, y: torch.Tensor, state: to
         raise ValueError("short_conv: a slot lies outside the state")
     library.call(_lib(), "agave_short_conv", ptr(u), ldu, ptr(weight), ptr(bias), ptr(y), ldy, ptr(state), ptr(step.tok_seq),
                  ptr(step.tok_pos), ptr(step.cu_dev), ptr(step.pos0_dev), ptr(step.slots_dev), n, step.n_seqs, c, taps,
-                 1 if silu else 0, 1 if step.is_decode else 0, ptr(in_bias), stream())
+                 1 if silu else 0, 1 if step.is_decode else 0, 1 if step.n_seqs == 1 or step.is_decode else step.most_seqs(CONV_ROWS),
+                 ptr(in_bias), stream())
 
 
 def head_norm_rope_rows(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Optional[torch.Tensor],

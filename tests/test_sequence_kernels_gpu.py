@@ -65,28 +65,32 @@ def test_short_conv_whole_pieces_and_tokens(taps, silu):
 
 
 @pytest.mark.parametrize("taps", [2, 3, 4])
-def test_short_conv_many_rows(taps):
-    """The kernel that slides along neighbouring rows against the one with a thread per row (which takes the same channels a few at
-    a time): sequences shorter than the taps, beginning and ending inside its stretches of rows, with states that go on."""
+@pytest.mark.parametrize("silu", [False, True])
+def test_short_conv_many_rows(taps, silu):
+    """The kernel that slides along neighbouring rows (steps that fill the chip) against the plain convolution in 64 bits: sequences
+    shorter than the taps, beginning and ending inside its stretches of rows, one and many to a stretch, with states that go on
+    from steps of few rows and of many; biases of the inputs and of the sums; the states it leaves."""
     from agave_amd.cache import StateNeed
     from agave_amd.ops import sequence as S
     g = torch.Generator().manual_seed(taps)
-    C, part = 1000, 250
-    w, bias, ib = (torch.randn(*k, generator=g).to(DEV) for k in ((C, taps), (C,), (C,)))
-    cols = [slice(i, i + part) for i in range(0, C, part)]
-    whole, parts = planner_for(state={0: StateNeed((taps - 1, C))}, slots=6, context=4096), [planner_for(state={0: StateNeed((taps - 1, part))}, slots=6, context=4096) for _ in cols]
-    slots = [[cache.alloc_slot() for _ in range(6)] for cache, _ in [whole] + parts][0]
-    for lens in ([3, 1, 2, 5], [700, 1, 17, 1400], [1, 2, 2200, 16]):
-        x = torch.randn(sum(lens), C, generator=g).to(DEV)
-        ys = []
-        for (cache, planner), at in zip([whole] + parts, [slice(0, C)] + cols):
-            step = feed(cache, planner, slots[1:5], lens)
-            y = torch.empty(sum(lens), at.stop - at.start, device=DEV)
-            S.short_conv(x[:, at].contiguous(), w[at].contiguous(), y, cache.state[0], step, True, bias[at].contiguous(), ib[at].contiguous())
-            planner.commit(step)
-            ys.append(y)
-        assert torch.equal(ys[0], torch.cat(ys[1:], 1)), lens
-        assert torch.equal(whole[0].state[0], torch.cat([cache.state[0] for cache, _ in parts], -1)), lens
+    C, n_seqs = 1000, 40
+    w, bias, ib = (torch.randn(*k, generator=g) for k in ((C, taps), (C,), (C,)))
+    cache, planner = planner_for(state={0: StateNeed((taps - 1, C))}, slots=n_seqs + 1, context=4096)
+    slots = [cache.alloc_slot() for _ in range(n_seqs + 1)][::-1]
+    history = [torch.zeros(0, C) for _ in range(n_seqs)]
+    for lens in ([3, 1, 2, 5], [700, 1, 17, 1400], [1] * (n_seqs - 1) + [900], [1, 2, 2200, 16], [20] * n_seqs, [2000]):
+        x = torch.randn(sum(lens), C, generator=g)
+        step = feed(cache, planner, slots[:len(lens)], lens)
+        y = torch.full((sum(lens), C), float("nan"), device=DEV)
+        S.short_conv(x.to(DEV), w.to(DEV), y, cache.state[0], step, silu, bias.to(DEV), ib.to(DEV))
+        planner.commit(step)
+        for i, (rows, got) in enumerate(zip(x.split(lens), y.cpu().to(F64).split(lens))):
+            history[i] = torch.cat([history[i], rows])
+            seen = history[i].to(F64) + ib.to(F64)
+            ref = P.short_conv(seen, w.to(F64))[-len(rows):] + bias.to(F64)
+            assert torch.allclose(got, P.silu(ref) if silu else ref, atol=2e-5, rtol=1e-5), (lens[:3], i)
+            held = torch.cat([torch.zeros(taps - 1, C, dtype=F64), seen])[-(taps - 1):]
+            assert torch.allclose(cache.state[0][slots[i]].cpu().to(F64), held, atol=1e-6, rtol=1e-6), (lens[:3], i)
 
 
 def test_short_conv_batch_of_unequal_sequences_and_a_slot_used_again():
