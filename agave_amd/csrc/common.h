@@ -8,6 +8,8 @@
 #define AGAVE_WAVE 64
 #define AGAVE_PAGE 64          // positions per cache page
 
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
 // dtype codes shared with the Python side
 #define AGAVE_F32 0
 #define AGAVE_BF16 1

@@ -1,8 +1,6 @@
-// Four neighbouring elements of a row as floats, for the 32-bit kernels.
+// Neighbouring elements of a row as floats.
 #pragma once
 #include "common.h"
-
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // Elements k .. k+3 of a row; what lies at or behind K is 0.  VEC: K is a multiple of 4 and every row is
 // aligned to four elements, so the four are there or not together.
@@ -27,4 +25,23 @@ template <> __device__ __forceinline__ f32x4_t ld4<false, bf16>(const bf16* row,
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = k + e < K ? bf16_to_f32(row[k + e]) : 0.f;
     return v;
+}
+
+// V neighbours, one or four (aligned to as many), from memory and to it.
+template <int V, typename T> __device__ __forceinline__ void load_near(const T* p, float* v) {
+    static_assert(V == 1 || V == 4, "one or four");
+    if constexpr (V == 4) {
+        const f32x4_t u = ld4<true>(p, 0, 4);
+        v[0] = u[0]; v[1] = u[1]; v[2] = u[2]; v[3] = u[3];
+    } else {
+        v[0] = ld(p);
+    }
+}
+template <int V> __device__ __forceinline__ void store_near(float* p, const float* v) {
+    if constexpr (V == 4) *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    else *p = v[0];
+}
+template <int V> __device__ __forceinline__ void store_near(bf16* p, const float* v) {
+    if constexpr (V == 4) *reinterpret_cast<uint2*>(p) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
+    else *p = f32_to_bf16(v[0]);
 }

@@ -15,7 +15,6 @@
 #include "common.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 // Place of tile (row block nb, k-step kb) in a packed matrix of NB row blocks and KB k-steps.

@@ -20,6 +20,7 @@
 // expert, in tiles of 16, 64 or 128 pairs that never span two experts (`route_sort` makes the list and the
 // tiles' table on the device, so a step's launches never depend on the choice).
 #include "common_impl.h"
+#include "fours.h"
 #include "mfma.h"
 #include <math.h>
 
@@ -420,28 +421,6 @@ __global__ __launch_bounds__(256) void routed_down_plain_kernel(const T* __restr
 // `place` (may be null): where pair p's row lies in y (a sorted list); null: at p.
 // A thread makes V neighbours of a row: 4 in steps of many tokens where rows and sizes allow accesses of four elements (bound by
 // memory: 3,001 tokens of 4 pairs and 2,048 columns, 135 MB, 21.6 us; one element a thread 35.8), 1 otherwise.
-template <int V, typename T> __device__ __forceinline__ void load_few(const T* p, float* v);
-template <> __device__ __forceinline__ void load_few<1, float>(const float* p, float* v) { v[0] = *p; }
-template <> __device__ __forceinline__ void load_few<1, bf16>(const bf16* p, float* v) { v[0] = bf16_to_f32(*p); }
-template <> __device__ __forceinline__ void load_few<4, float>(const float* p, float* v) {
-    const float4 u = *reinterpret_cast<const float4*>(p);
-    v[0] = u.x; v[1] = u.y; v[2] = u.z; v[3] = u.w;
-}
-template <> __device__ __forceinline__ void load_few<4, bf16>(const bf16* p, float* v) {
-    const uint2 u = *reinterpret_cast<const uint2*>(p);
-    v[0] = __uint_as_float(u.x << 16); v[1] = __uint_as_float(u.x & 0xffff0000u);
-    v[2] = __uint_as_float(u.y << 16); v[3] = __uint_as_float(u.y & 0xffff0000u);
-}
-template <int V, typename T> __device__ __forceinline__ void store_few(T* p, const float* v);
-template <> __device__ __forceinline__ void store_few<1, float>(float* p, const float* v) { *p = v[0]; }
-template <> __device__ __forceinline__ void store_few<1, bf16>(bf16* p, const float* v) { *p = f32_to_bf16(v[0]); }
-template <> __device__ __forceinline__ void store_few<4, float>(float* p, const float* v) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-}
-template <> __device__ __forceinline__ void store_few<4, bf16>(bf16* p, const float* v) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
-}
-
 template <typename T, int V>
 __global__ void routed_combine_kernel(const float* __restrict__ y, const int* __restrict__ place, const int* __restrict__ choice,
                                       const float* __restrict__ weight, const T* __restrict__ x, long ldx,
@@ -453,8 +432,8 @@ __global__ void routed_combine_kernel(const float* __restrict__ y, const int* __
     // (no load under a per-lane condition: the input row's element is read once, an expert row's from a row that exists
     // whatever the choice, and what does not count is left out afterwards)
     float xv[V], sv[V], acc[V];
-    load_few<V>(x + (size_t)t * ldx + c, xv);
-    load_few<V>((shared ? shared : x) + (size_t)t * (shared ? lds : ldx) + c, sv);
+    load_near<V>(x + (size_t)t * ldx + c, xv);
+    load_near<V>((shared ? shared : x) + (size_t)t * (shared ? lds : ldx) + c, sv);
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[i] = 0.f;
 #pragma unroll 4
@@ -466,7 +445,7 @@ __global__ void routed_combine_kernel(const float* __restrict__ y, const int* __
         int row = place ? place[p] : p;
         row = (expert && row >= 0) ? row : 0;
         float yv[V] = {};
-        if (y) load_few<V>(y + (size_t)row * hidden + c, yv);
+        if (y) load_near<V>(y + (size_t)row * hidden + c, yv);
 #pragma unroll
         for (int i = 0; i < V; ++i) acc[i] = fmaf(w, e >= E ? xv[i] : (expert ? yv[i] : 0.f), acc[i]);
     }
@@ -474,7 +453,7 @@ __global__ void routed_combine_kernel(const float* __restrict__ y, const int* __
 #pragma unroll
     for (int i = 0; i < V; ++i)
         if (shared) acc[i] = shared_gate ? fmaf(1.0f / (1.0f + expf(-shared_gate[t])), sv[i], acc[i]) : acc[i] + sv[i];
-    store_few<V>(out + (size_t)t * ldo + c, acc);
+    store_near<V>(out + (size_t)t * ldo + c, acc);
 }
 
 extern "C" int agave_routed_experts_plain(int dtype, const void* x, long ldx, const int* choice, const void* wg, const void* wu,

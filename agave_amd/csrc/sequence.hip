@@ -14,6 +14,7 @@
 // here: projections arrive as float rows, state is float, angles are made in double.  T is the
 // element type of the cache pages and of the rows handed to the output product.
 #include "common_impl.h"
+#include "fours.h"
 #include "mfma.h"
 #include <limits.h>
 #include <math.h>
@@ -1413,27 +1414,10 @@ extern "C" int agave_head_norm_gate(int dtype, const float* o, long ldo_in, cons
 
 // ------------------------------------------------------------------ a gate, then a norm in equal parts of the row
 //   g = y * silu(z);  out = g / sqrt(mean over the part (g^2) + eps) * w     (w is [parts * size])
-// A workgroup per (token, part), of one to four waves by the part's size; a thread keeps up to sixteen gated values in
-// registers between the sum of squares and the output (longer parts are computed twice).
-// A thread holds up to 16 elements (V neighbours at a time: 4 where sizes and alignment allow), a longer part's rest is read
-// twice.  The weights are asked for with the rows: behind the workgroup's sum they would cost a second round trip.
+// A workgroup per (token, part), of one to four waves by the part's size, in steps of few rows up to sixteen.  A thread holds up to
+// 16 elements between the sum of squares and the output (V neighbours at a time: 4 where sizes and alignment allow), a longer
+// part's rest is read twice.  The weights are asked for with the rows: behind the workgroup's sum they would cost a second round trip.
 // Measured, parts of 4,096: 6 rows 10.6 us with 256 threads and an element at a time, 5.1 us so.
-template <int V> __device__ __forceinline__ void load_floats(const float* p, float* v) {
-    if constexpr (V == 4) {
-        const float4 x = *reinterpret_cast<const float4*>(p);
-        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-    } else {
-        v[0] = *p;
-    }
-}
-template <int V> __device__ __forceinline__ void store_floats(float* p, const float* v) {
-    if constexpr (V == 4) *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-    else *p = v[0];
-}
-template <int V> __device__ __forceinline__ void store_floats(bf16* p, const float* v) {
-    if constexpr (V == 4) *reinterpret_cast<uint2*>(p) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
-    else *p = f32_to_bf16(v[0]);
-}
 template <typename T, int V>
 __global__ __launch_bounds__(1024) void gated_group_norm_kernel(const float* __restrict__ y, long ldy, const float* __restrict__ z,
                                                                 long ldz, const float* __restrict__ w, T* __restrict__ out, long ldo,
@@ -1449,9 +1433,9 @@ __global__ __launch_bounds__(1024) void gated_group_norm_kernel(const float* __r
     for (int i = 0; i < KEEP; ++i) {                    // (loads from inside the part, emptied afterwards)
         if (i * step >= size) break;                    // (the same for the whole workgroup)
         const int e = first + i * step < size ? first + i * step : 0;
-        load_floats<V>(yr + e, yv[i]);
-        load_floats<V>(zr + e, zv[i]);
-        load_floats<V>(wr + e, wv[i]);
+        load_near<V>(yr + e, yv[i]);
+        load_near<V>(zr + e, zv[i]);
+        load_near<V>(wr + e, wv[i]);
     }
     float ss = 0.f;
 #pragma unroll
@@ -1465,8 +1449,8 @@ __global__ __launch_bounds__(1024) void gated_group_norm_kernel(const float* __r
     }
     for (int e = first + KEEP * step; e < size; e += step) {
         float a[V], c[V];
-        load_floats<V>(yr + e, a);
-        load_floats<V>(zr + e, c);
+        load_near<V>(yr + e, a);
+        load_near<V>(zr + e, c);
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             a[v] *= c[v] / (1.0f + expf(-c[v]));
@@ -1487,16 +1471,16 @@ __global__ __launch_bounds__(1024) void gated_group_norm_kernel(const float* __r
         const int e = first + i * step;
 #pragma unroll
         for (int v = 0; v < V; ++v) yv[i][v] = yv[i][v] * inv * wv[i][v];
-        if (e < size) store_floats<V>(o + e, yv[i]);
+        if (e < size) store_near<V>(o + e, yv[i]);
     }
     for (int e = first + KEEP * step; e < size; e += step) {
         float a[V], c[V], x[V];
-        load_floats<V>(yr + e, a);
-        load_floats<V>(zr + e, c);
-        load_floats<V>(wr + e, x);
+        load_near<V>(yr + e, a);
+        load_near<V>(zr + e, c);
+        load_near<V>(wr + e, x);
 #pragma unroll
         for (int v = 0; v < V; ++v) a[v] = a[v] * (c[v] / (1.0f + expf(-c[v]))) * inv * x[v];
-        store_floats<V>(o + e, a);
+        store_near<V>(o + e, a);
     }
 }
 extern "C" int agave_gated_group_norm(int dtype, const float* y, long ldy, const float* z, long ldz, const float* w, void* out,
