@@ -18,8 +18,8 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // A wave per column of C, the lanes along K.  Bound by its trips to memory: a lane's loads are single elements, and a wave's 64 lie
 // next to each other, where the kernel below asks for sixteen rows' lines with each.  The sums are held in double, which costs
 // nothing here: in 32 bits they would be a lane's few products added across 64 lanes, and up to a third less exact than below.
-// Measured, us, with the kernel below and so: 1 row by 130 x 2,049 in 32 bits 12.7 and 7.4, in bfloat16 by 30,000 x 515 40 and 25; 2 rows
-// by 16 x 4,097 30 and 16.  Errors against 64 bits 0.25 to 0.3e-7 after 0.7 to 1.1e-7.
+// Measured, us, with the kernel below and so: 1 row by 130 x 2,049 in 32 bits 12.7 and 4.1, by 30,000 x 515 28.4 and 15.7, in bfloat16 40.0
+// and 14.8, by 1,000 x 33 3.6 and 3.1; 2 rows by 16 x 4,097 29.5 and 5.1.  Errors against 64 bits 0.25 to 0.3e-7 after 0.6 to 1.6e-7.
 #define FEW_ROWS 2
 template <typename TA, typename TW, typename TC>
 __global__ __launch_bounds__(256) void gemm_f32_few_rows_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw,
@@ -131,7 +131,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const TA* __re
 #define TN 64
 #define TK 32
 #define TS (TK + 4)
-// S: running sums of an element; four where few rows come here that groups of rows, with as many, would otherwise take.
+// S: running sums of an element (of each half of k where BM = 32); two where few rows come here that groups of rows, with a running
+// sum per quarter of k, would otherwise take.
 template <typename TA, typename TW, typename TC, int BM, bool VEC, int S>
 __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W, long ldw,
                                                              TC* __restrict__ C, long ldc, int M, int N, int K, int m_tiles, int tiles) {
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const TA* __restric
         __syncthreads();
     }
     f32x16_t acc = sums[0];
-    if (S == 4) acc = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    if (S == 2) acc += sums[S - 1];
     if (BM == 32) {                                               // the second pair's sums, 32 x 64 floats, through the first buffer
         static_assert(64 * 17 * 2 <= 2 * 32 * TS, "a wave's sums, padded by one float a lane, fit");
         float* half = &As[0][0] + wn * 64 * 17;
@@ -233,7 +234,7 @@ static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long
     if (M <= 16) return launch_skinny<TA, TW, TC, 1, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
     // from 65 rows on (17 where fours do not fit and K is not short): tiles as soon as the smaller ones give every compute unit one (80 rows by
     // 2,048 x 2,048, 96 of them: 47 us tiled, 24 us in groups of 64 rows; 200 rows, 224: 47 us in groups, 300 rows, 320: 52 us tiled;
-    // 30,000 x 515, 469 a row of tiles: 17 rows 54.7 in groups and 25.3 tiled, 64 rows 108 and 39)
+    // 30,000 x 515, 469 a row of tiles: 17 rows 54.2 in groups and 25.3 tiled, 64 rows 108 and 47, in bfloat16 132 and 62)
     const int n_tiles = (N + TN - 1) / TN;
     const long small_tiles = (long)n_tiles * ((M + 31) / 32);
     if ((M <= SKINNY_M && (VEC || K < 256)) || small_tiles < COMPUTE_UNITS) {
@@ -244,7 +245,7 @@ static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long
     const int bm = large ? 64 : 32, m_tiles = (M + bm - 1) / bm, tiles = m_tiles * n_tiles;
     const int grid = (tiles + 7) / 8 * 8;
     if (few)
-        gemm_f32_tiled_kernel<TA, TW, TC, 32, VEC, VEC ? 1 : 4><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
+        gemm_f32_tiled_kernel<TA, TW, TC, 32, VEC, VEC ? 1 : 2><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
     else if (large)
         gemm_f32_tiled_kernel<TA, TW, TC, 64, VEC, 1><<<grid, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
     else

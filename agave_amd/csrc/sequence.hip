@@ -184,7 +184,7 @@ extern "C" int agave_short_conv(const float* u, long ldu, const float* w, const 
     // thread and many, four taps: 4,352 channels 128 rows, 136 workgroups, 7.8 and 8.1, 256 rows, 272, 10.5 and 8.6; 12,288
     // channels 64 rows, 192, 8.7 and 8.2; 512 channels 1,000 rows, 126, 7.2 and 8.0, 3,001 rows, 376, 12.1 and 8.9; two taps: 1,000
     // channels 990 rows, 248, 8.6 and 9.0.  States asked for on the way and ahead, four taps: 60 sequences of one row and one of 1,000,
-    // 1,000 channels, 268 workgroups, 14.0 and 10.4 (a row a thread 10.8); 400 of five rows, 12,288 channels, 6,000, 68.7 and 72.7.)
+    // 1,000 channels, 268 workgroups, 14.4 and 9.3 (a row a thread 11.0); 400 of five rows, 12,288 channels, 6,000, 68.7 and 72.7.)
     const long wgs = (long)rows.x * rows.y;
     const bool many = most_seqs > 2 ? wgs <= 3072 : most_seqs == 2 && wgs <= 512;
     if (!one_token_each && taps >= 2 && taps <= 4 && wgs >= (taps == 2 ? 256 : 192)) {
