@@ -39,8 +39,9 @@ __device__ __forceinline__ float lanes16_sum(float v) {
 // z-th of them in a workgroup of its own.
 // gridDim.y workgroups share a row's pages and leave (sum, maximum, unnormalised result) for attn_plain_merge_kernel: with a
 // token per sequence there are few rows and the pages one after another bound the time.
-// NT: tiles of 64 value elements (16 a wave).  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of 0 must not meet a value that is not finite (a key behind a
-// token's position may hold anything): such pages are summed element by element.
+// NT: tiles of 64 value elements (16 a wave).  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of
+// 0 must not meet a value that is not finite (a key behind a token's position may hold anything): such pages are summed element
+// by element.
 // Bound by the 32-bit products (half of them for a token of 4 rows' padding) and, with few tokens, by the loads' way from memory.
 // Measured, 16 heads on 4 key heads of 128 in 32 bits: prompts of 97, 259 and 421 tokens 63 us (a workgroup per token and head, a
 // key a thread: 943 us), 2,000 tokens 0.45 ms (16.8 ms); a token each behind as many keys 15 us (59 us), behind 4,000 keys
@@ -407,9 +408,9 @@ extern "C" int agave_attn_plain_run(int N, int nh, int nkv) {
 }
 
 // one_token_each: neighbouring tokens are of different sequences (a decode step), so a workgroup takes one.  most_seqs: of as
-// many sequences at most are any `agave_attn_plain_run` tokens from a multiple of it on (no result depends on it).  most_keys: no token
-// sees more keys than this, 0 where that is not known (nor on it).  splits > 1: part_o
-// [N][nh][splits][hd] and part_ml [N][nh][splits][2] receive what a row's workgroups leave.
+// many sequences at most are any `agave_attn_plain_run` tokens from a multiple of it on.  most_keys: no token sees more keys than
+// this, 0 where that is not known.  (No result depends on either being right.)  splits > 1: part_o [N][nh][splits][hd] and part_ml
+// [N][nh][splits][2] receive what a row's workgroups leave.
 extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, long ldo, const void* k_pages,
                                 const void* v_pages, const int* table, int width, const int* base, int n_pages,
                                 const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,

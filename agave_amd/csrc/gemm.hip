@@ -8,7 +8,7 @@
 // (src/backend/backend.zig:474, 481).
 //
 // Two kernels: with few rows (decode steps, short prompts) the weights' way from memory bounds the
-// product, with more the multiply-adds do.
+// product, with more the multiply-adds do.  A third takes one or two rows that four elements do not fit.
 #include "common_impl.h"
 #include "fours.h"
 
