@@ -6,7 +6,8 @@
 //  * embed_scale_packed: the embedding gather reading rows out of a packed table (tied head);
 //  * gemm_skinny: M <= 64 tokens (decode): the weight streams through once at memory speed,
 //    K is split over the four waves of a workgroup, partial sums meet in LDS;
-//  * gemm_tiled: large M (prefill): 128x128 tiles per workgroup, X staged through LDS.
+//  * gemm_tiled: large M (prefill): tiles of 64 x 128 to 256 x 256 (weight rows x tokens), both operands
+//    staged through LDS (gemm_tiles.h has the kernel of all tiles but the largest).
 //
 // The reference computes the same products row by row: one workgroup per output row with a
 // block reduction (src/backend/kernels/rocm/gemv_bf16.zig:6-24), looped over tokens for a
@@ -130,14 +131,6 @@ __device__ __forceinline__ float gated_at(float gate, float up, const GateForm& 
 }
 static GateForm gate_form(float a, float b, float limit, float shift, const float* gate_b, const float* up_b) {
     return GateForm{-1.4426950408889634f * a, -1.4426950408889634f * b, limit, shift, gate_b, up_b};
-}
-// the form for a part of the output that starts at column n
-static GateForm from_column(GateForm F, int n) {
-    if (F.gate_b) {
-        F.gate_b += n;
-        F.up_b += n;
-    }
-    return F;
 }
 
 // R: row blocks (of 16 weight rows) per workgroup; MT: tiles of 16 tokens; EPI 0: store, 1: gated;
@@ -1004,34 +997,28 @@ extern "C" int agave_gemm_oproj_combine(const float* part_o, const float* part_m
     return 0;
 }
 
-// ------------------------------------------------------------------ tiled product (prefill)
-// A workgroup computes WT*64 weight rows x TT tokens in tiles of 32 x 32
-// (v_mfma_f32_32x32x16_bf16) with eight waves (2 x 4, a wave WT x TT/128 tiles): two per SIMD,
-// so that one multiplies while the other waits for a stage of loads, at a barrier or for its
-// operands, which a single wave per SIMD cannot hide (a third of its time was waiting); they
-// read a half more from LDS per flop, which the LDS (256 bytes a clock) has to spare.
-// Both operands come into LDS straight from global memory (no registers in between), KT k-steps
-// of 32 columns per stage, in a ring of NS buffers: the loads of NS-1 stages ahead are in flight
-// while a stage is multiplied.  What a compute unit can load is 64 bytes a clock (a load of one
-// kilobyte keeps its address unit busy for 16 cycles), half of which a 256 x 256 tile needs
-// when the matrix cores never wait; smaller tiles need more, which is why the largest tile that
-// still fills the chip is taken.
+// ------------------------------------------------------------------ tiled product (prefill), 256 x 256
+// A workgroup computes 256 weight rows x 256 tokens in tiles of 32 x 32 (v_mfma_f32_32x32x16_bf16)
+// with eight waves (2 x 4, a wave 4 x 2 tiles): two per SIMD, so that one multiplies while the other
+// waits for a stage of loads, at a barrier or for its operands, which a single wave per SIMD cannot
+// hide (a third of its time was waiting); they read a half more from LDS per flop, which the LDS (256
+// bytes a clock) has to spare.  Both operands come into LDS straight from global memory (no registers
+// in between), a k-step of 32 columns per stage, in a ring of four buffers: the loads of three stages
+// ahead are in flight while a stage is multiplied.
 // Weight tiles arrive in their packed order (one kilobyte per wave load; a 32-row operand is
 // read out of two packed 16-row tiles); token rows are stored with their 16-byte pieces
 // permuted so that the rows an MFMA operand reads fall into different banks.
-//   WT 4, KT 1, NS 4:  256 x 256 tiles, 128 KB of LDS, the two waves of a SIMD taking turns
-//   WT 2, KT 2, NS 3:  128 x 256 and 128 x 128 tiles - more workgroups for smaller products
-//   WT 1, KT 2, NS 4:  64 x 128 tiles
 // blockIdx.x walks the weight rows, so that workgroups sharing weight rows (ids a multiple of
 // the number of row tiles apart) tend to land on the same XCD and find them in its L2.
-typedef __attribute__((address_space(3))) u32x4_t tl_lds_u32x4;
+// What bounds it: the matrix cores at 1.6 to 1.9 GHz (a full chip of them runs into the power limit; the
+// clock falls from 2.4) for two thirds of the time; a tile's start and end, 10 of its 73 us at 2,560 columns.
+#include "gemm_tiles.h"
 
-
-template <int WT, int KT, int NS, int EPI, typename TC, int NWV, int TT, bool TURNS>
-__global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __restrict__ X, long ldx,
+template <int EPI, typename TC>
+__global__ __launch_bounds__(512, 2) void gemm_tiled_kernel(const bf16* __restrict__ X, long ldx,
                                                          const uint4* __restrict__ Wp, TC* __restrict__ Y, long ldy,
-                                                         int M, int N, int K, int KB, int NB, int NBS, long part_stride, GateForm F) {
-    // NBS: row blocks of the whole packed matrix (Wp may point at a later row block of it)
+                                                         int M, int N, int K, int KB, int NB, long part_stride, GateForm F) {
+    constexpr int WT = 4, KT = 1, NS = 4, NWV = 8, TT = 256;
     constexpr int CPR = KT * 4;                       // 16-byte pieces per staged token row
     constexpr int RP = 16 / CPR;                      // token rows per 256 bytes of LDS
     constexpr int WTILES = 4 * WT;                    // packed 16-row weight tiles per workgroup
@@ -1098,7 +1085,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
             int nb = nbw + tt / KT, kb = ste * KT + tt % KT;
             if (nb >= NB) nb = NB - 1;                                 // rows past the end: never stored
             if (kb >= KB) kb = KB - 1;                                 // k-steps past the end: never multiplied
-            const unsigned char* src = (const unsigned char*)(Wp + w_tile(nb, kb, NBS, KB) * 64);
+            const unsigned char* src = (const unsigned char*)(Wp + w_tile(nb, kb, NB, KB) * 64);
             __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + woff),
                                              (__attribute__((address_space(3))) void*)(buf + X_BYTES + tt * 1024), 16, 0, 0);
         }
@@ -1147,12 +1134,10 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
     // The stage loop.  Loads run NS-1 stages ahead and are issued one at a time between the
     // multiplications: in their shadow they cost no time, while all at once they queue up at the
     // address unit, which takes 16 cycles for each, and the matrix cores wait.
-    //   TURNS false: every wave reads the operands of a phase from LDS while the phase before it
-    //      multiplies; the first phase's are read after the stage's barrier.
-    //   TURNS true: the two waves of a SIMD take turns (waves 0-3 and 4-7, half a stage apart): one
-    //      reads its operands of a whole stage while the other multiplies, then a barrier, and they
-    //      change places.  The matrix cores then always have a wave that does nothing else.
-    constexpr int IN_FLIGHT = LOADS * (NS - 2 - (TURNS ? 1 : 0));     // loads that may be outstanding at a barrier
+    // The two waves of a SIMD take turns (waves 0-3 and 4-7, half a stage apart): one reads its operands
+    // of a whole stage while the other multiplies, then a barrier, and they change places.  The matrix
+    // cores then always have a wave that does nothing else.
+    constexpr int IN_FLIGHT = LOADS * (NS - 3);     // loads that may be outstanding at a barrier
     static_assert(IN_FLIGHT >= 0 && IN_FLIGHT < 64, "the load counter holds 6 bits");
 #pragma unroll
     for (int s0 = 0; s0 < NS - 1; ++s0)
@@ -1182,8 +1167,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
 #pragma unroll
         for (; li < end_load; ++li) fetch_one(st + NS - 1, li);
     };
-    if constexpr (TURNS) {
-        static_assert(NWV == 8 && NS >= 4, "two waves per SIMD take turns; a stage is in flight behind the awaited one");
+    {
         // Slots between barriers: the first group reads stage i in slot 2i and multiplies in slot
         // 2i+1, the second group one slot later; the loads for stage i+NS-1 are issued while stage
         // i is multiplied.  The first group reads stage i+1 in slot 2i+2, so every wave's loads
@@ -1209,21 +1193,6 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
             __builtin_amdgcn_s_setprio(0);
             __builtin_amdgcn_sched_barrier(0);
             if (!(second && st + 1 == n_stage)) __builtin_amdgcn_s_barrier();
-        }
-    } else {
-        Operands f[2];
-        for (int st = st0; st < n_stage; ++st) {
-            landed();
-            read_operands(f[0], st, IntC<0>{});
-            settle(f[0]);
-            static_for<0, PH>([&](auto phc) {
-                constexpr int ph = decltype(phc)::value;
-                if constexpr (ph + 1 < PH) read_operands(f[(ph + 1) & 1], st, IntC<ph + 1>{});
-                __builtin_amdgcn_sched_barrier(0);
-                multiply(f[ph & 1], st, ph, (ph * LOADS + PH - 1) / PH, ((ph + 1) * LOADS + PH - 1) / PH);
-                __builtin_amdgcn_sched_barrier(0);
-                if constexpr (ph + 1 < PH) settle(f[(ph + 1) & 1]);
-            });
         }
     }
 
@@ -1320,23 +1289,74 @@ __global__ __launch_bounds__(NWV * 64, 2) void gemm_tiled_kernel(const bf16* __r
     }
 }
 
-template <int WT, int KT, int NS, int EPI, typename TC, int NWV, int TT, bool TURNS>
+template <int EPI, typename TC>
 static int launch_tiled(const void* X, long ldx, const void* Wp, void* Y, long ldy, int M, int N, int K, int KB, int NB,
-                        const GateForm& F, hipStream_t stream, int splits = 1, long part_stride = 0, int NBS = 0) {
-    constexpr int WTILES = 4 * WT;
-    const size_t lds = (size_t)NS * (TT * KT * 64 + WTILES * KT * 1024);
-    dim3 grid((NB + WTILES - 1) / WTILES, (M + TT - 1) / TT, splits);
+                        const GateForm& F, hipStream_t stream, int splits, long part_stride) {
+    constexpr size_t lds = 4 * (256 * 64 + 16 * 1024);
+    const dim3 grid((NB + 15) / 16, (M + 255) / 256, splits);
     AGAVE_CHECK(grid.y <= 65535, "gemm_tiled: M=%d exceeds the grid limit", M);
     static bool raised = false;
     if (!raised) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiled_kernel<WT, KT, NS, EPI, TC, NWV, TT, TURNS>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_tiled_kernel<EPI, TC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         AGAVE_CHECK(e == hipSuccess, "gemm_tiled: cannot raise the LDS allowance");
         raised = true;
     }
-    gemm_tiled_kernel<WT, KT, NS, EPI, TC, NWV, TT, TURNS><<<grid, NWV * 64, lds, stream>>>((const bf16*)X, ldx, (const uint4*)Wp, (TC*)Y, ldy,
-                                                                      M, N, K, KB, NB, NBS > 0 ? NBS : NB, part_stride, F);
+    gemm_tiled_kernel<EPI, TC><<<grid, 512, lds, stream>>>((const bf16*)X, ldx, (const uint4*)Wp, (TC*)Y, ldy, M, N, K, KB, NB,
+                                                           part_stride, F);
     return 0;
+}
+
+// The tile shapes, by number: weight rows / 16 x tokens, and what one round of 256 workgroups takes in
+// microseconds: start + per_k * columns (measured with cold weights on random numbers, 2,048 to 10,240 columns;
+// `idle` of it where half of the compute units or fewer have one: the fewer work, the faster each of them runs).
+// Shapes 4 and 5 have no 32-bit output (such a finished tile does not fit the LDS).
+struct TileShape { int rows16, tokens; double start, per_k, idle; };
+static const TileShape TILES[] = {{16, 256, 17.0, 0.0222, 0.88}, {8, 256, 8.5, 0.0134, 0.78}, {8, 128, 4.2, 0.0096, 0.78},
+                                  {4, 128, 4.2, 0.0060, 0.92},   {10, 256, 9.0, 0.0162, 0.78}, {10, 192, 8.5, 0.0128, 0.80},
+                                  {10, 128, 7.0, 0.0099, 0.86}};
+constexpr int N_TILES = 7;
+static bool has_f32(int tile) { return tile != 4 && tile != 5; }
+
+// Microseconds of a product of M tokens and NB row blocks in tiles of a shape, its K columns in z slices.
+static double tile_time(int tile, int M, long NB, int K, int z, bool f32) {
+    const TileShape& t = TILES[tile];
+    const long groups = (NB + t.rows16 - 1) / t.rows16 * ((M + t.tokens - 1) / t.tokens) * z;
+    const double start = t.start + (f32 && tile == 0 ? 12.0 : 0.0);      // (a 32-bit tile of 256 x 256 is not stored by way of the LDS)
+    const double round = start + t.per_k * K / z, fill = (groups % 256) / 256.0;
+    const double last = groups % 256 == 0 ? 0.0 : t.idle + (1.0 - t.idle) * (fill > 0.5 ? 2.0 * fill - 1.0 : 0.0);
+    return 4.0 + (round - 4.0) * (double)(groups / 256) + (round - 4.0) * last;
+}
+static int best_tile(int M, long NB, int K, int z, bool f32) {
+    int best = -1;
+    double least = 0.0;
+    for (int i = 0; i < N_TILES; ++i) {
+        if (f32 && !has_f32(i)) continue;
+        const double t = tile_time(i, M, NB, K, z, f32);
+        if (best < 0 || t < least) {
+            best = i;
+            least = t;
+        }
+    }
+    return best;
+}
+
+template <int EPI, typename TC>
+static int launch_tile_shape(int tile, const void* X, long ldx, const void* Wp, void* Y, long ldy, int M, int N, int K, int KB,
+                             int NB, const GateForm& F, hipStream_t stream, int splits = 1, long part_stride = 0) {
+    switch (tile) {
+        case 0: return launch_tiled<EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, part_stride);
+        case 1: return launch_tile<4, 4, 2, 4, 3, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, part_stride);
+        case 2: return launch_tile<4, 2, 2, 4, 3, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, part_stride);
+        case 3: return launch_tile<2, 2, 2, 4, 4, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, part_stride);
+        case 6: return launch_tile<5, 2, 2, 4, 4, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, part_stride);
+        default: break;
+    }
+    if constexpr (sizeof(TC) == 2) {
+        if (tile == 4) return launch_tile<5, 4, 2, 4, 3, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, part_stride);
+        if (tile == 5) return launch_tile<5, 3, 2, 4, 3, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, part_stride);
+    }
+    AGAVE_CHECK(false, "gemm_tiled: no tile %d for this output", tile);
+    return -1;
 }
 
 // Y[m][n] = sum over the splits' partial sums
@@ -1353,30 +1373,18 @@ __global__ void gemm_sum_parts_kernel(const float* __restrict__ part, int splits
 template <int EPI, typename TC>
 static int dispatch_tiled(const void* X, long ldx, const void* Wp, void* Y, long ldy, int M, int N, int K, int KB,
                           int NB, float* part, long part_elems, const GateForm& F, hipStream_t stream) {
-    // The largest tile that still gives some 160 workgroups (a larger tile reads a third less from
-    // L2 per flop, which outweighs idle compute units down to about that number); with few tokens
-    // or few rows none does, and the tile with the most workgroups is taken.
-    //   256 x 256, 128 x 256, 128 x 128, 64 x 128 (weight rows x tokens)
-    const long rows16 = (NB + 15) / 16, rows8 = (NB + 7) / 8, rows4 = (NB + 3) / 4;
+    // Products of few tiles and many columns: the smallest shapes, by the number of workgroups there are
+    // (128 x 128 from 160 of them on, else 64 x 128).
+    const long rows8 = (NB + 7) / 8, rows4 = (NB + 3) / 4;
     const long t256 = (M + 255) / 256, t128 = (M + 127) / 128;
-    const long wgs[4] = {rows16 * t256, rows8 * t256, rows8 * t128, rows4 * t128};
-    int pick = -1;
-    for (int i = 0; i < 4 && pick < 0; ++i)
-        if (wgs[i] >= 160) pick = i;
-    if (pick < 0) {
-        pick = 0;
-        for (int i = 1; i < 4; ++i)
-            if (wgs[i] > wgs[pick]) pick = i;
-    }
-    // up to 128 tokens would leave half of a 256-token tile empty: tiles of 128 tokens (a step of 65
-    // to 128 tokens 3 to 5 % faster)
-    if (pick <= 1 && M <= 128) pick = 2;
-    // Still few workgroups and many columns: several workgroups share a tile's columns and leave
-    // partial sums (32-bit, in a buffer the caller lends), which a second kernel adds up.
+    const bool many = (NB + 15) / 16 * t256 >= 160 || rows8 * t256 >= 160 || rows8 * t128 >= 160;
+    const long wgs = rows4 * t128;
+    // Several workgroups share a tile's columns and leave partial sums (32-bit, in a buffer the caller lends), which a
+    // second kernel adds up.
     int splits = 1;
-    if (EPI == 0 && part != nullptr && wgs[pick] < 160) {
-        const int n_stage = (KB + 1) / 2;                 // the two small tiles take two k-steps a stage
-        splits = (int)((256 + wgs[pick] - 1) / wgs[pick]);
+    if (EPI == 0 && part != nullptr && !many && wgs < 160) {
+        const int n_stage = (KB + 1) / 2;                 // these tiles take two k-steps a stage
+        splits = (int)((256 + wgs - 1) / wgs);
         if (splits > 8) splits = 8;
         if (splits > K / (4 * M)) splits = K / (4 * M);       // the partial sums' traffic stays well below the weights'
         while (splits > 1 && (n_stage / splits < 8 || (long)splits * M * N > part_elems)) --splits;
@@ -1384,65 +1392,26 @@ static int dispatch_tiled(const void* X, long ldx, const void* Wp, void* Y, long
     }
     if (splits > 1) {
         const long stride = (long)M * N;
-        int rc;
-        if (pick == 2) rc = launch_tiled<2, 2, 3, 0, float, 8, 128, false>(X, ldx, Wp, part, N, M, N, K, KB, NB, GateForm{}, stream, splits, stride);
-        else rc = launch_tiled<1, 2, 4, 0, float, 8, 128, false>(X, ldx, Wp, part, N, M, N, K, KB, NB, GateForm{}, stream, splits, stride);
+        const int rc = launch_tile_shape<0, float>(3, X, ldx, Wp, part, N, M, N, K, KB, NB, GateForm{}, stream, splits, stride);
         if (rc != 0) return rc;
         AGAVE_LAUNCH_CHECK("gemm_tiled (partial sums)");
         const long total = (long)M * N;
         gemm_sum_parts_kernel<TC><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(part, splits, stride, (TC*)Y, ldy, M, N);
         return 0;
     }
-    if (pick == 0) {
-        // 256 compute units take 256 tiles at a time.  When the last round would be at most half
-        // full, the rows of that round are computed in tiles of half the height instead, in a
-        // second launch: all compute units then work for half a round, not half of them for a whole one.
-        const long tiles = wgs[0];
-        long rows_main = 0;                                // 256-row tiles of the first launch
-        if (tiles > 256 && tiles % 256 > 0) {
-            // as many whole rows of tiles as fit the whole rounds; the others, if their tiles of half
-            // the height fit one round
-            rows_main = (tiles / 256) * 256 / t256;
-            if (rows_main <= 0 || (rows16 - rows_main) * 2 * t256 > 256) rows_main = 0;
-        }
-        const long rest = tiles - rows_main * t256;        // 256 x 256 tiles' worth of the second launch
-        if (rows_main > 0) {
-            const int nb_main = (int)rows_main * 16;
-            const int n_main = EPI == 0 ? nb_main * 16 : nb_main * 8;
-            int rc = launch_tiled<4, 1, 4, EPI, TC, 8, 256, true>(X, ldx, Wp, Y, ldy, M, n_main, K, KB, nb_main, F, stream, 1, 0, NB);
-            if (rc != 0) return rc;
-            // (a quarter of a round or less: tiles of a quarter of the size, which again fill the compute units)
-            if (rest <= 64 && (rows16 - rows_main) * 2 * ((M + 127) / 128) <= 256)
-                return launch_tiled<2, 2, 3, EPI, TC, 8, 128, false>(X, ldx, (const uint4*)Wp + w_tile(nb_main, 0, NB, KB) * 64,
-                                                                     (TC*)Y + n_main, ldy, M, N - n_main, K, KB, NB - nb_main,
-                                                                     from_column(F, n_main), stream, 1, 0, NB);
-            return launch_tiled<2, 2, 3, EPI, TC, 8, 256, false>(X, ldx, (const uint4*)Wp + w_tile(nb_main, 0, NB, KB) * 64,
-                                                                 (TC*)Y + n_main, ldy, M, N - n_main, K, KB, NB - nb_main, from_column(F, n_main), stream,
-                                                                 1, 0, NB);
-        }
-    }
-    switch (pick) {
-        case 0: return launch_tiled<4, 1, 4, EPI, TC, 8, 256, true>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-        case 1: return launch_tiled<2, 2, 3, EPI, TC, 8, 256, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-        case 2: return launch_tiled<2, 2, 3, EPI, TC, 8, 128, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-        default: return launch_tiled<1, 2, 4, EPI, TC, 8, 128, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-    }
+    return launch_tile_shape<EPI, TC>(best_tile(M, NB, K, 1, sizeof(TC) == 4), X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
 }
 
 // A product of many tokens whose reader adds 32-bit slices up (the residual kernel does): when
-// its 128 x 256 tiles fill the 256 compute units' rounds badly (160 tiles for 2,048 tokens and
+// its tiles fill the 256 compute units' rounds badly (160 tiles of 128 x 256 for 2,048 tokens and
 // 2,560 rows leave 96 of them idle for the whole product), each tile's columns are shared among
-// z workgroups, each of which leaves its sums in a slice of its own.  In units of one tile's
-// time the product then takes rounds(tiles * z) / z, and every slice beyond the first costs its
-// bytes, written here and read by whoever adds them: some 0.07 of a tile's time at 160 tiles and
-// 10,240 columns (measured: down at 2,048 tokens takes 114 us in three slices instead of 136, and
-// the kernel that adds them 8 us more), in proportion to the tiles and inversely to the columns.
-// Products that run in 256 x 256 tiles are left alone: sliced, they were slower (measured at
-// 4,096 and 8,192 tokens, by 4 %; slices of 256 x 256 tiles by 1 to 2 %, except for 168 tiles, a
-// round two thirds full, where they gained 2 %).  Shorter prompts gain as much: down at 1,024 tokens takes 59 us
-// in three slices of 80 tiles instead of 81 us in 160 tiles of 128 x 128 (a prefill of 384 to
-// 1,024 tokens 2 to 5 % less).
-struct SlicePlan { int tile; int z; };      // tile: 0 256 x 256, 1 128 x 256, 2 128 x 128, 3 64 x 128 (weight rows x tokens)
+// z workgroups, each of which leaves its sums in a slice of its own.  How many slices that is worth is
+// counted in units of one 128 x 256 tile's time: the product takes rounds(tiles * z) / z, and every slice
+// beyond the first costs its bytes, some 0.07 of a tile's time at 160 tiles and 10,240 columns, in
+// proportion to the tiles and inversely to the columns.  Products that run in 256 x 256 tiles are left alone.
+// In which tiles the slices run, and whether the one product is not faster after all, is left to the
+// shapes' times (down of the 4B sizes at 2,048 tokens: 107 us as one product in tiles of 160 x 128, 108 us and 8 more in the
+// kernel that adds them in three slices of 256 x 256; at 1,024 tokens 77 us as one, 53 us in three slices of 128 x 256).
 
 static int cut_tiled_slices(int M, int N, int K) {
     const long NB = (N + 15) / 16;
@@ -1474,7 +1443,7 @@ static int cut_tiled_slices(int M, int N, int K) {
     return z_best;
 }
 
-static SlicePlan plan_tiled_slices(int M, int N, int K) {
+static int plan_tiled_slices(int M, int N, int K) {
     // Short prompts (up to 128 tiles of 64 x 128: some 400 tokens at 2,560 rows): as many slices of
     // those tiles as fit one round of 256 workgroups, each with at least six stages.  Measured at
     // 2,560 rows, 96 to 384 tokens: 10,240 columns take 17 to 36 us so (4 slices of 128 x 256 tiles:
@@ -1488,36 +1457,35 @@ static SlicePlan plan_tiled_slices(int M, int N, int K) {
             int z = (int)(256 / small);
             if (z > 8) z = 8;
             while (z > 1 && n_stage / z < 6) --z;
-            if (z > 1) return SlicePlan{3, z};
+            if (z > 1) return z;
         }
     }
-    const int z = cut_tiled_slices(M, N, K);
-    // 256 x 256 tiles where the slices of those fill the compute units in one round (down of the 4B
-    // sizes at 2,048 tokens: 240 workgroups, 112 us; as 480 of 128 x 256: 119)
-    const long NB = (N + 15) / 16;
-    const long big = (long)((NB + 15) / 16) * ((M + 255) / 256) * z;
-    return SlicePlan{(big > 192 && big <= 256) ? 0 : 1, z};
+    return cut_tiled_slices(M, N, K);
 }
 
 // How many 32-bit slices a product of M > 64 tokens is best computed in by a caller that can
 // add them up (1: as one product).
 extern "C" int agave_gemm_tiled_slices(int M, int N, int K) {
     if (M <= 64 || N <= 0 || K <= 0 || K % 8 != 0) return 1;
-    return plan_tiled_slices(M, N, K).z;
+    return plan_tiled_slices(M, N, K);
 }
 
-// The slices of a product in tiles of a given shape (0: 256 x 256, 1: 128 x 256, 2: 128 x 128,
-// 3: 64 x 128, weight rows x tokens).
+// The same for a caller that has the choice: 1 where one 32-bit slice, the whole product, is the faster way (each slice,
+// written here and read by whoever adds them up, costs a microsecond per million elements).
+extern "C" int agave_gemm_tiled_slices_worth(int M, int N, int K) {
+    const int z = agave_gemm_tiled_slices(M, N, K);
+    if (z == 1) return 1;
+    const long NB = ((long)N + 15) / 16;
+    auto cost = [&](int slices) {
+        return tile_time(best_tile(M, NB, K, slices, true), M, NB, K, slices, true) + 0.96e-6 * slices * (double)M * N;
+    };
+    return cost(z) < cost(1) ? z : 1;
+}
+
+// The slices of a product in tiles of a given shape.
 static int launch_slices(int tile, const void* X, long ldx, const void* Wp, float* Y, int M, int N, int K, int z,
                          hipStream_t stream) {
-    const int KB = (K + 31) / 32, NB = (N + 15) / 16;
-    const long stride = (long)M * N;
-    switch (tile) {
-        case 0: return launch_tiled<4, 1, 4, 0, float, 8, 256, true>(X, ldx, Wp, Y, N, M, N, K, KB, NB, GateForm{}, stream, z, stride);
-        case 1: return launch_tiled<2, 2, 3, 0, float, 8, 256, false>(X, ldx, Wp, Y, N, M, N, K, KB, NB, GateForm{}, stream, z, stride);
-        case 2: return launch_tiled<2, 2, 3, 0, float, 8, 128, false>(X, ldx, Wp, Y, N, M, N, K, KB, NB, GateForm{}, stream, z, stride);
-        default: return launch_tiled<1, 2, 4, 0, float, 8, 128, false>(X, ldx, Wp, Y, N, M, N, K, KB, NB, GateForm{}, stream, z, stride);
-    }
+    return launch_tile_shape<0, float>(tile, X, ldx, Wp, Y, N, M, N, K, (K + 31) / 32, (N + 15) / 16, GateForm{}, stream, z, (long)M * N);
 }
 
 static int check_slices_args(const char* who, const void* X, long ldx, int M, int N, int K) {
@@ -1533,43 +1501,31 @@ static int check_slices_args(const char* who, const void* X, long ldx, int M, in
 extern "C" int agave_gemm_tiled_in_slices(const void* X, long ldx, const void* Wp, float* Y, int M, int N, int K,
                                           int z, hipStream_t stream) {
     if (check_slices_args("gemm_tiled_in_slices", X, ldx, M, N, K)) return -1;
-    const SlicePlan plan = plan_tiled_slices(M, N, K);
-    AGAVE_CHECK(z > 1 && z == plan.z, "gemm_tiled_in_slices: %d slices asked for, %d planned", z, plan.z);
-    if (launch_slices(plan.tile, X, ldx, Wp, Y, M, N, K, z, stream) != 0) return -1;
+    const int plan = plan_tiled_slices(M, N, K);
+    AGAVE_CHECK(z > 1 && z == plan, "gemm_tiled_in_slices: %d slices asked for, %d planned", z, plan);
+    if (launch_slices(best_tile(M, (N + 15) / 16, K, z, true), X, ldx, Wp, Y, M, N, K, z, stream) != 0) return -1;
     AGAVE_LAUNCH_CHECK("gemm_tiled_in_slices");
     return 0;
 }
 
-// The same with the tile shape and the number of slices given by the caller (tile 0: 256 x 256,
-// 1: 128 x 256, 2: 128 x 128, 3: 64 x 128): for tests of every shape and for measurements.  z = 1
-// leaves the whole product in the one slice.
+// The same with the tile shape and the number of slices given by the caller: for tests of every shape and for
+// measurements.  z = 1 leaves the whole product in the one slice.
 extern "C" int agave_gemm_tiled_in_slices_as(const void* X, long ldx, const void* Wp, float* Y, int M, int N, int K,
                                              int tile, int z, hipStream_t stream) {
     if (check_slices_args("gemm_tiled_in_slices_as", X, ldx, M, N, K)) return -1;
     const int n_stage = tile == 0 ? (K + 31) / 32 : (K + 63) / 64;
-    AGAVE_CHECK(tile >= 0 && tile <= 3 && z >= 1 && z <= 16 && z <= n_stage, "gemm_tiled_in_slices_as: tile %d in %d slices of %d stages",
+    AGAVE_CHECK(tile >= 0 && tile < N_TILES && has_f32(tile) && z >= 1 && z <= 16 && z <= n_stage, "gemm_tiled_in_slices_as: tile %d in %d slices of %d stages",
                 tile, z, n_stage);
     if (launch_slices(tile, X, ldx, Wp, Y, M, N, K, z, stream) != 0) return -1;
     AGAVE_LAUNCH_CHECK("gemm_tiled_in_slices_as");
     return 0;
 }
 
-// One product in tiles of a shape the caller names (0: 256 x 256, 1: 128 x 256, 2: 128 x 128,
-// 3: 64 x 128), whatever agave_gemm_tiled would choose: for tests of every shape and for measurements.
-template <int EPI, typename TC>
-static int launch_tile_shape(int tile, const void* X, long ldx, const void* Wp, void* Y, long ldy, int M, int N, int K,
-                             int KB, int NB, const GateForm& F, hipStream_t stream) {
-    switch (tile) {
-        case 0: return launch_tiled<4, 1, 4, EPI, TC, 8, 256, true>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-        case 1: return launch_tiled<2, 2, 3, EPI, TC, 8, 256, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-        case 2: return launch_tiled<2, 2, 3, EPI, TC, 8, 128, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-        default: return launch_tiled<1, 2, 4, EPI, TC, 8, 128, false>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
-    }
-}
-
+// One product in tiles of a shape the caller names, whatever agave_gemm_tiled would choose: for tests of every shape and for
+// measurements.
 extern "C" int agave_gemm_tiled_as(const void* X, long ldx, const void* Wp, int dt_y, void* Y, long ldy, int M, int N,
                                    int K, int epilogue, float act_a, float act_b, float act_limit, float act_shift, const float* gate_b, const float* up_b, int tile, hipStream_t stream) {
-    AGAVE_CHECK(M > 0 && N > 0 && K > 0 && tile >= 0 && tile <= 3, "gemm_tiled_as: bad sizes M=%d N=%d K=%d or tile %d", M, N, K, tile);
+    AGAVE_CHECK(M > 0 && N > 0 && K > 0 && tile >= 0 && tile < N_TILES, "gemm_tiled_as: bad sizes M=%d N=%d K=%d or tile %d", M, N, K, tile);
     AGAVE_CHECK(K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)X % 16) == 0,
                 "gemm_tiled_as: X must be 16-byte aligned with K and its row stride multiples of 8 (K=%d ldx=%ld)", K, ldx);
     AGAVE_CHECK(ldx >= K && ldy >= N && ldx < (1L << 22), "gemm_tiled_as: bad row strides");

@@ -1272,6 +1272,60 @@ def test_gemm_tiled_every_tile_shape_in_slices(G, tile, m, n, k, z):
     assert float((whole.double().cpu() - ref).abs().max()) <= 6e-3 * float(ref.abs().max())
 
 
+# Columns: one stage of 64 and less, a k-step of 32 missing from the last stage, as many stages as the ring has buffers and
+# one more or less, many.  Rows and tokens: a tile of each shape, one more, one less.
+@pytest.mark.parametrize("k", [8, 64, 72, 96, 192, 200, 256, 320, 1000])
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("gated", [False, True])
+def test_gemm_tile_edges(G, tile, gated, k):
+    rows, tokens = G.TILE_SHAPES[tile]
+    g = torch.Generator().manual_seed(tile + k)
+    for m, n in ((tokens, rows), (tokens + 1, rows + 1), (2 * tokens - 1, 2 * rows - 3), (3, 5)):
+        n = (n + 1) // 2 if gated else n
+        x = torch.randn(m, k + 24, generator=g).bfloat16().to(DEV)[:, :k]            # (rows further apart than they are long)
+        w = (torch.randn(2 * n if gated else n, k, generator=g) * 0.2).bfloat16().to(DEV)
+        packed = G.pack_weight(w, interleave_ff=n if gated else 0)
+        ref = x.double() @ w.double().T
+        if gated:
+            ref = P.gelu_tanh(ref[:, :n]) * ref[:, n:]
+        out = torch.full((m, n + 3), float("nan"), dtype=torch.bfloat16, device=DEV)
+        G.tiled_as(x, packed, out[:, :n], n, tile, epilogue=int(gated))
+        # bfloat16 results (half an ulp: 2^-9 of each), of sums in 32 bits whose rounding is far below; gated: of two factors
+        assert float((out[:, :n].double() - ref).abs().max()) <= (8e-3 if gated else 6e-3) * float(ref.abs().max())
+        assert bool(out[:, n:].isnan().all())
+        if gated or tile in G.BF16_ONLY_TILES or m <= 64:            # (slices: more than 64 tokens)
+            continue
+        whole = torch.full((1, m, n), float("nan"), device=DEV)
+        G.tiled_slices_as(x, packed, whole, n, tile)
+        assert float((whole[0].double() - ref).abs().max()) <= 2e-5 * float(ref.abs().max()) * math.sqrt(max(k, 64) / 64)
+
+
+@pytest.mark.parametrize("tile", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("k", [40, 104, 136, 328])
+def test_gemm_tile_infinities_stay_theirs(G, tile, k):
+    """Whatever stands in a row stays that row's, and what is read in the place of missing columns counts nothing: a row with an
+    infinity anywhere gives infinities of the right sign, not NaN."""
+    g = torch.Generator().manual_seed(k)
+    m, n = 140, 170
+    x = torch.randn(m, k, generator=g).bfloat16()
+    w = (torch.rand(n, k, generator=g) + 0.5).bfloat16()
+    for r, c in enumerate(range(0, k, 8)):
+        x[r, c] = math.inf if r % 2 else -math.inf
+    marked = (k + 7) // 8
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    G.tiled_as(x.to(DEV), G.pack_weight(w.to(DEV)), out, n, tile)
+    got = out.cpu().double()
+    assert torch.equal(got[:marked], torch.tensor([[math.inf if r % 2 else -math.inf] * n for r in range(marked)], dtype=torch.float64))
+    ref = x.double()[marked:] @ w.double().T
+    assert float((got[marked:] - ref).abs().max()) <= 6e-3 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 2560, 10240), (1024, 2560, 10240), (300, 2560, 2048), (2048, 2560, 2048)])
+def test_gemm_tiled_slices_are_taken_where_they_pay(G, m, n, k):
+    assert G.tiled_slices_worth(m, n, k) in (1, G.tiled_slices_for(m, n, k))
+    assert G.tiled_slices_worth(2048, 2560, 10240) == 1 and G.tiled_slices_worth(1024, 2560, 10240) == 3
+
+
 @pytest.mark.parametrize("m,ff,k", [(70, 192, 64), (513, 1000, 96), (256, 20, 40), (1024, 5120, 1000), (2048, 10236, 64),
                                     (1024, 10236, 64)])
 def test_gemm_tiled_geglu(G, m, ff, k):
