@@ -707,10 +707,67 @@ extern "C" int agave_gemm_row_normed(const float* h_in, float* h_out, const void
     return 0;
 }
 
+// ------------------------------------------------------------------ tiles of 64 tokens
+#include "gemm_tiles.h"
+
+// From 17 tokens on the waves of gemm_skinny spend more on staging X, each its own columns through registers, than on the
+// weights; a workgroup of the tile kernel (gemm_tiles.h) stages X once for 64 to 128 weight rows, straight into LDS.  It is
+// the faster one where its workgroups fill 256 compute units' rounds by five eighths or more (measured, 4B sizes, us,
+// gemm_skinny and these tiles at 17, 32 and 64 tokens: gate and up 21.5, 22.6, 23.9 and 19.6, 21.1, 22.2 in 214 workgroups of
+// 96 rows; down in slices 14.0, 15.5, 16.9 and 12.0, 13.0, 14.0; the output matrix of 262,208 rows 262, 270, 326 and 256, 258, 279;
+// q/k/v, which make 64 workgroups of 64 rows, 8.3, 9.1, 10.9 and 12.3, 12.6, 14.8: they stay).  With fewer tokens gemm_skinny reads the
+// weights at what the memory gives, but for products of one whole round: 32,768 rows of 2,048, 2 to 12 tokens, 28 to 32 and
+// 24.6 to 25.
+// Returns the tile's row blocks (8, 6, 4), 0: gemm_skinny.
+static double few_fill(long NB, int rows16, int z) {
+    const long groups = (NB + rows16 - 1) / rows16 * z;
+    return (double)groups / (256.0 * ((groups + 255) / 256));
+}
+static int few_tile(int M, long NB, int z) {
+    int best = 0;
+    double most = 0.0;
+    for (int rows16 = 8; rows16 >= 4; rows16 -= 2) {
+        const double f = few_fill(NB, rows16, z);
+        if (f > most) {
+            best = rows16;
+            most = f;
+        }
+    }
+    if (M >= 17) return most >= 0.62 ? best : 0;
+    return z == 1 && most >= 0.98 && (NB + best - 1) / best <= 256 ? best : 0;
+}
+
+template <int EPI, typename TC>
+static int launch_few(int tile, const void* X, long ldx, const void* Wp, void* Y, long ldy, int M, int N, int K, int KB, int NB,
+                      int splits, const GateForm& F, hipStream_t stream) {
+    const long stride = (long)M * ldy;
+    switch (tile) {
+        case 8: return launch_tile<2, 2, 4, 2, 5, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, stride);
+        case 6: return launch_tile<3, 1, 2, 4, 6, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, stride);
+        default: return launch_tile<2, 1, 2, 4, 6, EPI, TC>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream, splits, stride);
+    }
+}
+
 // How many 32-bit slices a product of M <= 64 tokens is best computed in by a caller that can add
 // them up (1: as one product).
 extern "C" int agave_gemm_skinny_slices(int M, int N, int K) {
     if (M <= 0 || M > 64 || N <= 0 || K <= 0) return 1;
+    if (M >= 17) {                              // the slices (of eight stages at least) that fill the rounds best; each costs its bytes
+        const long NB = ((long)N + 15) / 16;
+        const int n_stage = (K + 63) / 64;
+        double best = 0.0;
+        int cut = 0;
+        for (int z = 1; z <= 8 && (z == 1 || n_stage / z >= 8); ++z) {
+            const int tile = few_tile(M, NB, z);
+            if (tile == 0) continue;
+            const double worth = few_fill(NB, tile, z) - 0.04 * (z - 1);
+            if (cut == 0 || worth > best) {
+                best = worth;
+                cut = z;
+            }
+        }
+        if (cut > 0) return cut;
+    }
     return cut_skinny(M, (N + 15) / 16, (K + 31) / 32, 8).z;
 }
 
@@ -732,7 +789,18 @@ extern "C" int agave_gemm_skinny(const void* X, long ldx, const void* Wp, int dt
                 splits, K);
     AGAVE_CHECK(splits == 1 || (epilogue == 0 && dt_y == AGAVE_F32), "gemm_skinny: partial sums are plain 32-bit sums");
     int rc;
-    if (epilogue == 0) {
+    const int tile = ldx < (1L << 22) ? few_tile(M, NB, splits) : 0;       // (the tile kernel's offsets have 32 bits)
+    if (tile > 0) {
+        if (epilogue == 1) {
+            AGAVE_CHECK(dt_y == AGAVE_BF16, "gemm_skinny: the gated epilogue writes bfloat16");
+            rc = launch_few<1, bf16>(tile, X, ldx, Wp, Y, ldy, M, N, K, KB, NB, 1, gate_form(act_a, act_b, act_limit, act_shift, gate_b, up_b), stream);
+        } else if (dt_y == AGAVE_BF16) {
+            rc = launch_few<0, bf16>(tile, X, ldx, Wp, Y, ldy, M, N, K, KB, NB, 1, GateForm{}, stream);
+        } else {
+            AGAVE_CHECK(dt_y == AGAVE_F32, "gemm_skinny: unknown output dtype %d", dt_y);
+            rc = launch_few<0, float>(tile, X, ldx, Wp, Y, ldy, M, N, K, KB, NB, splits, GateForm{}, stream);
+        }
+    } else if (epilogue == 0) {
         if (dt_y == AGAVE_BF16) rc = dispatch_skinny<0, bf16>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, 1, GateForm{}, stream);
         else if (dt_y == AGAVE_F32) rc = dispatch_skinny<0, float>(X, ldx, Wp, Y, ldy, M, N, K, KB, NB, splits, GateForm{}, stream);
         else AGAVE_CHECK(false, "gemm_skinny: unknown output dtype %d", dt_y);
@@ -1012,8 +1080,6 @@ extern "C" int agave_gemm_oproj_combine(const float* part_o, const float* part_m
 // the number of row tiles apart) tend to land on the same XCD and find them in its L2.
 // What bounds it: the matrix cores at 1.6 to 1.9 GHz (a full chip of them runs into the power limit; the
 // clock falls from 2.4) for two thirds of the time; a tile's start and end, 10 of its 73 us at 2,560 columns.
-#include "gemm_tiles.h"
-
 template <int EPI, typename TC>
 __global__ __launch_bounds__(512, 2) void gemm_tiled_kernel(const bf16* __restrict__ X, long ldx,
                                                          const uint4* __restrict__ Wp, TC* __restrict__ Y, long ldy,

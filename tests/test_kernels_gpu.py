@@ -1320,6 +1320,41 @@ def test_gemm_tile_infinities_stay_theirs(G, tile, k):
     assert float((got[marked:] - ref).abs().max()) <= 6e-3 * float(ref.abs().max())
 
 
+# Tiles of 64 tokens by 128, 96 and 64 weight rows (160 to 256 workgroups of each make a round that is filled well enough):
+# rows that end inside a tile, columns that end inside a stage, fewer stages than the ring has buffers, 17 and 64 tokens, and
+# the products of one whole round that fewer tokens take them for.
+@pytest.mark.parametrize("m,n,k", [(17, 32760, 72), (64, 32760, 200), (2, 32760, 328), (1, 32768, 64), (16, 32765, 1000),
+                                   (33, 20530, 104), (64, 24570, 64), (20, 10750, 456), (63, 10300, 8), (64, 16380, 1096)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32, "gated"])
+def test_gemm_tiles_of_64_tokens(G, m, n, k, out_dtype):
+    g = torch.Generator().manual_seed(m + n + k)
+    gated = out_dtype == "gated"
+    n = n // 2 if gated else n
+    x = torch.randn(m, k + 8, generator=g).bfloat16().to(DEV)[:, :k]
+    w = (torch.randn(2 * n if gated else n, k, generator=g) * 0.1).bfloat16().to(DEV)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16 if gated else out_dtype, device=DEV)
+    G.product(x, G.pack_weight(w, interleave_ff=n if gated else 0), out, n, epilogue=int(gated))
+    ref = x.double() @ w.double().T
+    if gated:
+        ref = P.gelu_tanh(ref[:, :n]) * ref[:, n:]
+    scale = float(ref.abs().max())
+    tol = 2e-5 * scale * math.sqrt(max(k, 64) / 64) if out_dtype == torch.float32 else 8e-3 * scale
+    assert float((out.double() - ref).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 2560, 10240), (64, 2552, 10248), (40, 2560, 2048), (33, 2040, 5384), (64, 4304, 5168)])
+def test_gemm_tiles_of_64_tokens_in_slices(G, m, n, k):
+    z = G.slices_for(m, n, k)
+    assert 1 < z <= 8
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(n, k, generator=g) * 0.1).bfloat16().to(DEV)
+    out = torch.full((z, m, n), float("nan"), device=DEV)
+    G.skinny_slices(x, G.pack_weight(w), out, n)
+    ref = x.double() @ w.double().T
+    assert float((out.double().sum(0) - ref).abs().max()) <= 2e-5 * float(ref.abs().max()) * math.sqrt(k / 64)
+
+
 @pytest.mark.parametrize("m,n,k", [(2048, 2560, 10240), (1024, 2560, 10240), (300, 2560, 2048), (2048, 2560, 2048)])
 def test_gemm_tiled_slices_are_taken_where_they_pay(G, m, n, k):
     assert G.tiled_slices_worth(m, n, k) in (1, G.tiled_slices_for(m, n, k))
