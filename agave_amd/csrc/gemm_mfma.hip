@@ -1372,14 +1372,14 @@ static int launch_tiled(const void* X, long ldx, const void* Wp, void* Y, long l
     return 0;
 }
 
-// The tile shapes, by number: weight rows / 16 x tokens, and what one round of 256 workgroups takes in
-// microseconds: start + per_k * columns (measured with cold weights on random numbers, 2,048 to 10,240 columns;
-// `idle` of it where half of the compute units or fewer have one: the fewer work, the faster each of them runs).
+// The tile shapes, by number: weight rows / 16 x tokens, and what a round of 256 workgroups takes in microseconds, ends +
+// per_k * columns (measured with cold weights on random numbers, 2,048 to 10,240 columns, 512 to 8,192 tokens; `idle` of it where half
+// of the compute units or fewer have a workgroup: the fewer work, the faster each of them runs).
 // Shapes 4 and 5 have no 32-bit output (such a finished tile does not fit the LDS).
-struct TileShape { int rows16, tokens; double start, per_k, idle; };
-static const TileShape TILES[] = {{16, 256, 17.0, 0.0222, 0.88}, {8, 256, 8.5, 0.0134, 0.78}, {8, 128, 4.2, 0.0096, 0.78},
-                                  {4, 128, 4.2, 0.0060, 0.92},   {10, 256, 9.0, 0.0162, 0.78}, {10, 192, 8.5, 0.0128, 0.80},
-                                  {10, 128, 7.0, 0.0099, 0.86}};
+struct TileShape { int rows16, tokens; double ends, per_k, idle; };
+static const TileShape TILES[] = {{16, 256, 10.5, 0.0245, 0.86}, {8, 256, 5.5, 0.0125, 0.80}, {8, 128, 3.8, 0.0086, 0.80},
+                                  {4, 128, 2.8, 0.0052, 0.92},   {10, 256, 7.0, 0.0155, 0.80}, {10, 192, 5.5, 0.0124, 0.82},
+                                  {10, 128, 4.5, 0.0098, 0.86}};
 constexpr int N_TILES = 7;
 static bool has_f32(int tile) { return tile != 4 && tile != 5; }
 
@@ -1387,10 +1387,11 @@ static bool has_f32(int tile) { return tile != 4 && tile != 5; }
 static double tile_time(int tile, int M, long NB, int K, int z, bool f32) {
     const TileShape& t = TILES[tile];
     const long groups = (NB + t.rows16 - 1) / t.rows16 * ((M + t.tokens - 1) / t.tokens) * z;
-    const double start = t.start + (f32 && tile == 0 ? 12.0 : 0.0);      // (a 32-bit tile of 256 x 256 is not stored by way of the LDS)
-    const double round = start + t.per_k * K / z, fill = (groups % 256) / 256.0;
+    // (twice the bytes to store; 256 x 256 in 32 bits does not even go by way of the LDS)
+    const double ends = t.ends * (!f32 ? 1.0 : tile == 0 ? 2.0 : 1.4);
+    const double fill = (groups % 256) / 256.0;
     const double last = groups % 256 == 0 ? 0.0 : t.idle + (1.0 - t.idle) * (fill > 0.5 ? 2.0 * fill - 1.0 : 0.0);
-    return 4.0 + (round - 4.0) * (double)(groups / 256) + (round - 4.0) * last;
+    return 3.0 + (ends + t.per_k * K / z) * ((double)(groups / 256) + last);
 }
 static int best_tile(int M, long NB, int K, int z, bool f32) {
     int best = -1;
@@ -1439,22 +1440,28 @@ __global__ void gemm_sum_parts_kernel(const float* __restrict__ part, int splits
 template <int EPI, typename TC>
 static int dispatch_tiled(const void* X, long ldx, const void* Wp, void* Y, long ldy, int M, int N, int K, int KB,
                           int NB, float* part, long part_elems, const GateForm& F, hipStream_t stream) {
-    // Products of few tiles and many columns: the smallest shapes, by the number of workgroups there are
-    // (128 x 128 from 160 of them on, else 64 x 128).
+    // Products of few tiles, even of the smallest shapes, and many columns.
     const long rows8 = (NB + 7) / 8, rows4 = (NB + 3) / 4;
     const long t256 = (M + 255) / 256, t128 = (M + 127) / 128;
     const bool many = (NB + 15) / 16 * t256 >= 160 || rows8 * t256 >= 160 || rows8 * t128 >= 160;
     const long wgs = rows4 * t128;
+    const int tile = best_tile(M, NB, K, 1, sizeof(TC) == 4);
     // Several workgroups share a tile's columns and leave partial sums (32-bit, in a buffer the caller lends), which a
     // second kernel adds up.
     int splits = 1;
     if (EPI == 0 && part != nullptr && !many && wgs < 160) {
         const int n_stage = (KB + 1) / 2;                 // these tiles take two k-steps a stage
-        splits = (int)((256 + wgs - 1) / wgs);
-        if (splits > 8) splits = 8;
-        if (splits > K / (4 * M)) splits = K / (4 * M);       // the partial sums' traffic stays well below the weights'
-        while (splits > 1 && (n_stage / splits < 8 || (long)splits * M * N > part_elems)) --splits;
-        if (splits < 1) splits = 1;
+        // (the second kernel takes its start, 1.5 us of it beside the first one's end, and its bytes: 4,096 rows of 2,560, 128 tokens
+        // 15.4 us in four shares and 20 as one, but 8,512 rows of 2,048, 80 tokens 22 us in two shares and 14.6 as one)
+        double least = tile_time(tile, M, NB, K, 1, sizeof(TC) == 4);
+        // (at most K / 4M of them: the partial sums' traffic stays well below the weights')
+        for (int z = 2; z <= 8 && z <= K / (4 * M) && n_stage / z >= 8 && (long)z * M * N <= part_elems; ++z) {
+            const double t = tile_time(3, M, NB, K, z, true) + 1.5 + 0.2e-6 * (double)M * N * (4 * z + (int)sizeof(TC));
+            if (t < least) {
+                least = t;
+                splits = z;
+            }
+        }
     }
     if (splits > 1) {
         const long stride = (long)M * N;
@@ -1465,7 +1472,7 @@ static int dispatch_tiled(const void* X, long ldx, const void* Wp, void* Y, long
         gemm_sum_parts_kernel<TC><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(part, splits, stride, (TC*)Y, ldy, M, N);
         return 0;
     }
-    return launch_tile_shape<EPI, TC>(best_tile(M, NB, K, 1, sizeof(TC) == 4), X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
+    return launch_tile_shape<EPI, TC>(tile, X, ldx, Wp, Y, ldy, M, N, K, KB, NB, F, stream);
 }
 
 // A product of many tokens whose reader adds 32-bit slices up (the residual kernel does): when
