@@ -7,8 +7,9 @@
 // Weights are row-major [out, in] and used as y = W x, as in the reference
 // (src/backend/backend.zig:474, 481).
 //
-// Two kernels: with few rows (decode steps, short prompts) the weights' way from memory bounds the
-// product, with more the multiply-adds do.  A third takes one or two rows that four elements do not fit.
+// With few rows (decode steps, short prompts) the weights' way from memory bounds the product, with more the
+// multiply-adds do: a kernel for up to eight rows, one for up to 64, one for more, and one for one or two rows that four
+// elements do not fit.
 #include "common_impl.h"
 #include "fours.h"
 
@@ -50,8 +51,8 @@ __global__ __launch_bounds__(256) void gemm_f32_few_rows_kernel(const TA* __rest
 // k = 4g .. 4g+3 and element e of the four goes into the e-th of four instructions.  U steps are asked
 // for together, 256 bytes of every weight row.
 // Bound by the weights' way from memory: NW is chosen so that about 2,048 waves stand in flight (see
-// launch_skinny).  Measured in 32 bits, N x K = 10,752 x 2,048: 3 rows 21.6 us (4.1 TB/s), 16 rows 29 us;
-// 2,048 x 5,376: 3 rows 19 us, 64 rows 64 us.  A wave per column with lanes along K took 82, 256, 89 us,
+// launch_skinny).  Measured in 32 bits, N x K = 10,752 x 2,048: 16 rows 31 us (2.8 TB/s), 64 rows 76 us; 2,048 x 5,376: 16 rows
+// 26 us, 64 rows 64 us.  A wave per column with lanes along K took 82, 256, 89 us,
 // vector tiles with 64 rows 646 us.
 // A sum of K products in 32 bits loses more the longer its one running sum is.  One tile of rows keeps a
 // running sum per step and element (16 a lane, of which each takes K / (16 NW) products), added in pairs
@@ -113,6 +114,125 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const TA* __re
             for (int v = 0; v < s; ++v) sums[v] += sums[v + s];
         st(C + (size_t)m * ldc + n, sums[0]);
     }
+}
+
+// ---------------------------------------------------------------- up to eight rows
+// A workgroup makes 8 columns of C; its NW waves share K.  Eight rows fill half of v_mfma_f32_16x16x4_f32's sixteen, so the other
+// half of rows and columns takes 16 further k: rows i and columns j of the result belong together where both are below 8 or
+// both are not, and those two quarters are added at the end (the other two mean nothing).  A wave's load is then 128
+// bytes, a whole line, of each of 8 weight rows, where sixteen rows took 64 of each; and 2,048 columns make a workgroup for each
+// of the 256 compute units (with 16 a workgroup 128 of them pulled 2.2 TB/s).  Three chunks of 64 k are in flight a wave: a load leaves as
+// soon as the chunk three before it is multiplied, without a condition around it (past the end it repeats the last four
+// elements, which are not used), so that a wait leaves the younger ones in flight.
+// Bound by the weights' way from memory.  Measured in 32 bits, us, three rows, before (sixteen columns a workgroup, four loads at a
+// time) and now: 10,752 x 2,048 23.7 and 20.7 (4.3 TB/s), 2,048 x 5,376 20.3 and 13.0, 3,072 x 2,048 9.8 and 8.9, 2,048 x 2,048 9.0 and 6.2,
+// 32,768 x 2,048 61 and 51 (5.3 TB/s); eight rows 26.8 and 22.5, 22.2 and 15.7, 10.4 and 10.9, 9.5 and 7.3, 67 and 55.
+// A running sum per step and element, eight a lane in each half of k, as many sums of as many products as sixteen rows have.
+template <typename TA, typename TW, typename TC, int NW, int R>
+__global__ __launch_bounds__(NW * 64) void gemm_f32_eight_rows_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W,
+                                                                      long ldw, TC* __restrict__ C, long ldc, int M, int N, int K) {
+    constexpr int U = 2, CHUNK = U * 32, S = 3;
+    __shared__ float part[NW][R * 64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 7, h = (lane >> 3) & 1, g = lane >> 4;
+    const int n0 = blockIdx.x * 8 * R;
+    const TW* w[R];                                               // (rows and columns outside are computed from the last one and not stored)
+#pragma unroll
+    for (int i = 0; i < R; ++i) w[i] = W + (size_t)min(n0 + 8 * i + r, N - 1) * ldw;
+    const TA* a = A + (size_t)min(r, M - 1) * lda;
+    const int lane_k = 16 * h + 4 * g;
+    const int n_chunks = (K + CHUNK - 1) / CHUNK, n_iter = (n_chunks + NW - 1) / NW;
+    f32x4_t acc[4 * U][R] = {};
+    f32x4_t wv[S][U][R], av[S][U];
+    // Chunks are dealt to the waves in turn, from another one on in every workgroup: rows that lie a multiple of 4 KB apart have
+    // their like columns in one channel of the L2, and all workgroups would ask the same few at a time.
+    const int first = (int)(blockIdx.x >> 3) % n_chunks;
+    auto chunk_of = [&](int it) {
+        const int c = min(it * NW + wave, n_chunks - 1) + first;
+        return c < n_chunks ? c : c - n_chunks;
+    };
+    auto load = [&](int st, int it) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(chunk_of(it) * CHUNK + 32 * u + lane_k, K - 4);
+#pragma unroll
+            for (int i = 0; i < R; ++i) wv[st][u][i] = ld4<true>(w[i], k, K);
+            av[st][u] = ld4<true>(a, k, K);
+        }
+    };
+    auto use = [&](int st, int it) {
+        if (it * NW + wave >= n_chunks) return;
+        const int c = chunk_of(it);
+        if ((c + 1) * CHUNK > K) {                                // the last chunk, where columns are missing from it
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (c * CHUNK + 32 * u + lane_k >= K) {
+                    av[st][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int i = 0; i < R; ++i) wv[st][u][i] = av[st][u];
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+                    acc[4 * u + e][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[st][u][e], wv[st][u][i][e], acc[4 * u + e][i], 0, 0, 0);
+    };
+    if (n_iter < S) {                                             // (nothing is asked for twice)
+        load(0, 0);
+        if (n_iter > 1) load(1, 1);
+        use(0, 0);
+        if (n_iter > 1) use(1, 1);
+    } else {
+#pragma unroll
+        for (int st = 0; st < S; ++st) load(st, st);
+        int it = 0;
+        for (; it + 2 * S <= n_iter; it += S)                     // every load is of a chunk that exists
+#pragma unroll
+            for (int st = 0; st < S; ++st) {
+                __builtin_amdgcn_sched_barrier(0);
+                use(st, it + st);
+                __builtin_amdgcn_sched_barrier(0);
+                load(st, it + st + S);
+            }
+#pragma unroll
+        for (int st = 0; st < S; ++st) {                          // the last S to 2 S - 1
+            __builtin_amdgcn_sched_barrier(0);
+            use(st, it + st);
+            __builtin_amdgcn_sched_barrier(0);
+            if (it + st + S < n_iter) load(st, it + st + S);
+        }
+#pragma unroll
+        for (int st = 0; st < S - 1; ++st) use(st, it + st + S);
+    }
+#pragma unroll
+    for (int s = 2 * U; s > 0; s /= 2)
+#pragma unroll
+        for (int i = 0; i < s; ++i)
+#pragma unroll
+            for (int j = 0; j < R; ++j) acc[i][j] += acc[i + s][j];
+    // acc[0][i][e] is row 4 g + e, column lane % 16; the quarters that mean something: rows below 8 in lane groups 0 and 1 with
+    // columns below 8, and what lies 8 rows (two lane groups) and 8 columns further, 40 lanes in all
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float sum = acc[0][i][e] + __shfl_xor(acc[0][i][e], 40, 64);
+            if (h == 0 && g < 2) part[wave][(4 * g + e) * 8 * R + 8 * i + r] = sum;
+        }
+    __syncthreads();
+    const int m = threadIdx.x / (8 * R), n = n0 + threadIdx.x % (8 * R);
+    if (m >= M || n >= N) return;
+    float sums[NW];
+#pragma unroll
+    for (int v = 0; v < NW; ++v) sums[v] = part[v][threadIdx.x];
+#pragma unroll
+    for (int s = NW / 2; s > 0; s /= 2)
+#pragma unroll
+        for (int v = 0; v < s; ++v) sums[v] += sums[v + s];
+    st(C + (size_t)m * ldc + n, sums[0]);
 }
 
 // ---------------------------------------------------------------- more rows
@@ -225,11 +345,24 @@ static void launch_skinny(const TA* A, long lda, const TW* W, long ldw, TC* C, l
         gemm_f32_skinny_kernel<TA, TW, TC, MT, 4, VEC><<<groups, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
 }
 
+// Up to eight rows: 16 waves for each of up to 256 workgroups of one block of columns, 8 for up to 512 (two a compute unit), and beyond
+// that two blocks a workgroup of 4 waves, which take the rows of A once for both.
+template <typename TA, typename TW, typename TC>
+static void launch_eight_rows(const TA* A, long lda, const TW* W, long ldw, TC* C, long ldc, int M, int N, int K, hipStream_t stream) {
+    const int blocks = (N + 7) / 8;
+    if (blocks <= COMPUTE_UNITS) gemm_f32_eight_rows_kernel<TA, TW, TC, 16, 1><<<blocks, 1024, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    else if (blocks <= 2 * COMPUTE_UNITS) gemm_f32_eight_rows_kernel<TA, TW, TC, 8, 1><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    else gemm_f32_eight_rows_kernel<TA, TW, TC, 4, 2><<<(blocks + 1) / 2, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+}
+
 template <typename TA, typename TW, typename TC, bool VEC>
 static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long ldc, int M, int N, int K, hipStream_t stream) {
     if (!VEC && M <= FEW_ROWS) {
         gemm_f32_few_rows_kernel<TA, TW, TC><<<(N + 3) / 4, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
         return;
+    }
+    if constexpr (VEC) {
+        if (M <= 8) return launch_eight_rows<TA, TW, TC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
     }
     if (M <= 16) return launch_skinny<TA, TW, TC, 1, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
     // from 65 rows on (17 where fours do not fit and K is not short): tiles as soon as the smaller ones give every compute unit one (80 rows by

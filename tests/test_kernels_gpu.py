@@ -314,6 +314,29 @@ def test_gemm_plain_large_tiles_and_odd_rows(K, ta, tw, m, n, k):
         assert bool((c[m] == 7.0).all()) and bool((c[:, n:] == 7.0).all())
 
 
+# Up to eight rows whose fours fit: workgroups of 16, 8 and 4 waves (256 and 512 blocks of eight columns are the lines between them), a
+# broken last block, chunks of 64 columns that break off, one chunk in all, and as many chunks a wave as are in flight, more or less.
+@pytest.mark.parametrize("ta,tw", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("n", [7, 2048, 2050, 4096, 4101, 9001])
+@pytest.mark.parametrize("k", [4, 60, 64, 68, 256, 772, 1028, 2052, 3084, 4164])
+def test_gemm_plain_up_to_eight_rows(K, ta, tw, n, k):
+    g = torch.Generator().manual_seed(n + k)
+    w = torch.randn(n, k, generator=g).to(tw).to(DEV)
+    for m in (1, 3, 8):
+        x = torch.randn(m, k + 4, generator=g).to(ta).to(DEV)[:, :k]
+        c = torch.full((m + 1, n + 2), 7.0, device=DEV)
+        K.gemm_plain(x, w, c[:m, :n])
+        bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        assert bool(((c[:m, :n].double() - x.double() @ w.double().T).abs() <= bound).all())
+        assert bool((c[m] == 7.0).all()) and bool((c[:, n:] == 7.0).all())
+    x[1, k - 1], x[2, 0], w[5, 2] = float("nan"), float("inf"), float("-inf")          # they stay in their rows and columns
+    K.gemm_plain(x, w, c[:m, :n])
+    got, plain = c[:m, :n].cpu(), torch.ones(m, n, dtype=torch.bool)
+    plain[1], plain[2], plain[:, 5] = False, False, False
+    assert bool(got[1].isnan().all()) and bool(got[plain].isfinite().all())
+    assert not bool(got[2, :5].isfinite().any()) and not bool(got[0, 5].isfinite())
+
+
 @pytest.mark.parametrize("m,n,k", [(2, 40, 17), (70, 40, 18), (300, 3300, 20), (290, 3300, 18), (97, 5500, 20), (17, 16400, 258), (40, 8200, 257)])
 def test_gemm_plain_special_values_in_every_kernel(K, m, n, k):
     """A NaN or an infinity stays in its row and column, and zeros behind the last k meet zeros only."""
