@@ -12,8 +12,7 @@
 // elements do not fit.
 #include "common_impl.h"
 #include "fours.h"
-
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
+#include "mfma.h"
 
 // ---------------------------------------------------------------- one or two rows that fours do not fit
 // A wave per column of C, the lanes along K.  Bound by its trips to memory: a lane's loads are single elements, and a wave's 64 lie
@@ -327,6 +326,142 @@ __global__ __launch_bounds__(256) void gemm_f32_tiled_kernel(const TA* __restric
     }
 }
 
+// ---------------------------------------------------------------- more rows, 32-bit operands that fours fit
+// WM x WN waves make BM x BN of C, a wave BM/WM x BN/WN in tiles of 32 x 32.  Stages of 32 k come into LDS straight from memory, in a
+// ring of NS buffers: while a stage is multiplied the next NS - 1 are on their way, and no wave spends registers or LDS writes on
+// bringing them (the kernel above does, and waits for a stage's loads with nothing else in flight).  A row's eight 16-byte pieces are
+// permuted by its number, so that the 32 rows of a read lie on different banks.  The waits are for "all but the youngest n": loads
+// and LDS reads come back in the order they were asked for.
+// Bound by the multiply-adds (64 clocks for 32 x 32 x 2).  The ring of 32 x 128 tiles is made so large (80 KB) that two workgroups share a
+// compute unit: a third (64 x 64 tiles in 48 KB) made 624 tiles 16 % slower.  Measured in 32 bits, us, the kernel above and this one:
+// 777 rows by 10,752 x 2,048 370 and 309 (111 TFLOP/s), by 2,048 x 5,376 208 and 174, by 2,048 x 2,048 85 and 72, by 3,072 x 2,048 122 and
+// 108; 300 rows by 10,752 x 2,048 175 and 134; 2,048 rows 870 and 730 (124 TFLOP/s).
+// S running sums of an element, each of every S-th k.
+template <int BM, int BN, int WM, int WN, int S, int NS>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_f32_ring_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W,
+                                                                     long ldw, float* __restrict__ C, long ldc, int M, int N, int K,
+                                                                     int m_tiles, int tiles) {
+    constexpr int NWV = WM * WN, MT = BM / WM / 32, NT = BN / WN / 32;
+    constexpr int LA = BM / 8 / NWV, LW = BN / 8 / NWV, LOADS = LA + LW;      // of a kilobyte, eight rows, a wave and stage
+    static_assert(LA * NWV * 8 == BM && LW * NWV * 8 == BN && MT * WM * 32 == BM && NT * WN * 32 == BN, "whole loads and tiles a wave");
+    constexpr int A_BYTES = BM * 128, STAGE = (BM + BN) * 128;
+    __shared__ __attribute__((aligned(16))) unsigned char ring[NS * STAGE];
+    // (tiles one below the other follow each other on an XCD, as above)
+    const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int m0 = tile % m_tiles * BM, n0 = tile / m_tiles * BN;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = wave % WN, wm = wave / WN, r = lane & 31, h = lane >> 5;
+    const unsigned char* ap = (const unsigned char*)(A + (size_t)m0 * lda);
+    const unsigned char* wp = (const unsigned char*)(W + (size_t)n0 * ldw);
+    unsigned aoff[LA], woff[LW];                                  // (rows outside: the last one again, not stored)
+    const int row0 = wave * 8 + (lane >> 3);                      // this lane's row of load 0; a load further: 8 NWV rows
+    auto piece = [&](int i) { return (lane & 7) ^ (((row0 + i * NWV * 8) >> 1) & 7); };       // the four k it brings
+#pragma unroll
+    for (int i = 0; i < LA; ++i) aoff[i] = (unsigned)min(row0 + i * NWV * 8, M - 1 - m0) * (unsigned)(lda * 4) + piece(i) * 16;
+#pragma unroll
+    for (int i = 0; i < LW; ++i) woff[i] = (unsigned)min(row0 + i * NWV * 8, N - 1 - n0) * (unsigned)(ldw * 4) + piece(i) * 16;
+    auto to_lds = [&](const unsigned char* src, int at) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                         (__attribute__((address_space(3))) void*)(ring + at), 16, 0, 0);
+    };
+    const int n_stage = (K + 31) / 32, rest = K & 31;             // rest: k of a broken last stage
+    auto mend = [&]() {                                           // pieces past the last k: the stage's first one, zeroed when read
+#pragma unroll
+        for (int i = 0; i < LA; ++i) aoff[i] -= piece(i) * 4 >= rest ? piece(i) * 16 : 0;
+#pragma unroll
+        for (int i = 0; i < LW; ++i) woff[i] -= piece(i) * 4 >= rest ? piece(i) * 16 : 0;
+    };
+    auto fetch = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < LA; ++i) to_lds(ap + aoff[i], buf + (i * NWV + wave) * 1024);
+#pragma unroll
+        for (int i = 0; i < LW; ++i) to_lds(wp + woff[i], buf + A_BYTES + (i * NWV + wave) * 1024);
+        ap += 128;
+        wp += 128;
+    };
+    // v_mfma_f32_32x32x2_f32 takes k in any order as long as both operands agree: the four elements of piece 2 j + h go into four
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)ring;
+    unsigned at[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) at[j] = lds0 + r * 128 + (((2 * j + h) ^ ((r >> 1) & 7)) * 16);
+    const unsigned a_wave = wm * MT * 4096, w_wave = A_BYTES + wn * NT * 4096;
+    f32x16_t sums[S][MT][NT] = {};
+    static_for<0, NS - 1>([&](auto p) {
+        if (p.value < n_stage) {
+            if (p.value == n_stage - 1 && rest != 0) mend();
+            fetch(p.value * STAGE);
+        }
+    });
+    int buf = 0, free_buf = (NS - 1) * STAGE;
+    // a stage; FLIGHT: loads of the stages behind it that may still be on their way; ASK: another stage's are asked for; BROKEN:
+    // pieces of it lie past the last k
+    auto stage = [&](auto flight, auto ask, auto broken) {
+        constexpr int n = decltype(flight)::value;
+        static_assert(n < 64, "the counter holds six bits");
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+        __builtin_amdgcn_s_barrier();                             // (all that this stage needs has come, and the one before it is read)
+        frag16 va[4][MT], vw[4][NT];
+        static_for<0, 4>([&](auto j) {
+            static_for<0, MT>([&](auto t) { lds_read16<t.value * 4096>(va[j.value][t.value], at[j.value] + a_wave + buf); });
+            static_for<0, NT>([&](auto t) { lds_read16<t.value * 4096>(vw[j.value][t.value], at[j.value] + w_wave + buf); });
+        });
+        if constexpr (decltype(ask)::value != 0) fetch(free_buf);
+        static_for<0, 4>([&](auto j) {
+            __builtin_amdgcn_sched_barrier(0);                    // (each piece's multiplications as soon as it is here)
+            lds_settle_to<(3 - j.value) * (MT + NT)>();
+#pragma unroll
+            for (int t = 0; t < MT; ++t) lds_use(va[j.value][t]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) lds_use(vw[j.value][t]);
+            if (decltype(broken)::value != 0 && (2 * j.value + h) * 4 >= rest) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) va[j.value][t].u = uint4{0, 0, 0, 0};
+#pragma unroll
+                for (int t = 0; t < NT; ++t) vw[j.value][t].u = uint4{0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int u = 0; u < NT; ++u)
+                        sums[e % S][t][u] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(f32x4_t, va[j.value][t].r)[e],
+                                                                                 __builtin_bit_cast(f32x4_t, vw[j.value][u].r)[e],
+                                                                                 sums[e % S][t][u], 0, 0, 0);
+        });
+        free_buf = buf;
+        buf = buf == (NS - 1) * STAGE ? 0 : buf + STAGE;
+    };
+    for (int st = 0; st + NS < n_stage; ++st) stage(IntC<(NS - 2) * LOADS>{}, IntC<1>{}, IntC<0>{});
+    if (n_stage >= NS) {                                          // the last stage's loads
+        if (rest != 0) mend();
+        stage(IntC<(NS - 2) * LOADS>{}, IntC<1>{}, IntC<0>{});
+    }
+    static_for<0, NS - 2>([&](auto p) {                           // NS - 1 stages are left, or all that there are
+        constexpr int left = NS - 1 - p.value;
+        if (n_stage >= left) stage(IntC<(left - 1) * LOADS>{}, IntC<0>{}, IntC<0>{});
+    });
+    if (rest != 0) stage(IntC<0>{}, IntC<0>{}, IntC<1>{});
+    else stage(IntC<0>{}, IntC<0>{}, IntC<0>{});
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+#pragma unroll
+            for (int s = S / 2; s > 0; s /= 2)
+#pragma unroll
+                for (int i = 0; i < s; ++i) sums[i][t][u] += sums[i + s][t][u];
+            // element e is row 8 (e/4) + 4 (lane/32) + e%4, column lane%32
+            const int n = n0 + (wn * NT + u) * 32 + r;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + (wm * MT + t) * 32 + 8 * (e / 4) + 4 * h + e % 4;
+                if (m < M && n < N) C[(size_t)m * ldc + n] = sums[0][t][u][e];
+            }
+        }
+}
+
 // ---------------------------------------------------------------- launch
 #define SKINNY_M 64
 #define COMPUTE_UNITS 256
@@ -355,6 +490,26 @@ static void launch_eight_rows(const TA* A, long lda, const TW* W, long ldw, TC* 
     else gemm_f32_eight_rows_kernel<TA, TW, TC, 4, 2><<<(blocks + 1) / 2, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
 }
 
+template <int BM, int BN, int WM, int WN, int S, int NS>
+static void launch_ring(const float* A, long lda, const float* W, long ldw, float* C, long ldc, int M, int N, int K, hipStream_t stream) {
+    const int m_tiles = (M + BM - 1) / BM, tiles = m_tiles * ((N + BN - 1) / BN);
+    gemm_f32_ring_kernel<BM, BN, WM, WN, S, NS><<<(tiles + 7) / 8 * 8, WM * WN * 64, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles);
+}
+
+// Rows a tile of gemm_f32_ring_kernel, 0: not that kernel.  Tiles of 32 x 128, two at a time on a compute unit, or, where that is less by
+// the times of so many tiles a compute unit (measured at 2,048 columns, us; what is left over after whole rounds takes as long as if it
+// were alone), of 128 x 128, 130 us each.  The kernel of 32 x 64 tiles keeps products of one round of those (37.5 us), which halve the k
+// between waves.  Up to 64 rows stay in groups of 64 rows where these have eight running sums a product or more (under 8,192 columns), and
+// are added up as in groups with four.
+static int ring_rows(int M, int N) {
+    auto a_unit = [&](int bm) { return (((long)M + bm - 1) / bm * (((long)N + 127) / 128) + COMPUTE_UNITS - 1) / COMPUTE_UNITS; };
+    static const double t32[] = {0, 44, 72, 109, 146, 195};
+    if (M <= SKINNY_M) return N >= (M > 32 ? 8192 : 16384) ? 32 : 0;
+    if ((long)((M + 31) / 32) * ((N + TN - 1) / TN) <= COMPUTE_UNITS) return 0;
+    const long n32 = a_unit(32);
+    return (n32 <= 5 ? t32[n32] : 35.0 * n32) <= 130.0 * a_unit(128) ? 32 : 128;
+}
+
 template <typename TA, typename TW, typename TC, bool VEC>
 static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long ldc, int M, int N, int K, hipStream_t stream) {
     if (!VEC && M <= FEW_ROWS) {
@@ -365,6 +520,12 @@ static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long
         if (M <= 8) return launch_eight_rows<TA, TW, TC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
     }
     if (M <= 16) return launch_skinny<TA, TW, TC, 1, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+    if constexpr (VEC && std::is_same<TA, float>::value && std::is_same<TW, float>::value && std::is_same<TC, float>::value) {
+        const int rows = lda < (1L << 22) && ldw < (1L << 22) ? ring_rows(M, N) : 0;       // (offsets in a tile have 32 bits)
+        if (rows == 32 && M <= SKINNY_M) return launch_ring<32, 128, 1, 4, 4, 4>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+        if (rows == 32) return launch_ring<32, 128, 1, 4, 2, 4>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+        if (rows == 128) return launch_ring<128, 128, 2, 4, 2, 3>(A, lda, W, ldw, C, ldc, M, N, K, stream);
+    }
     // from 65 rows on (17 where fours do not fit and K is not short): tiles as soon as the smaller ones give every compute unit one (80 rows by
     // 2,048 x 2,048, 96 of them: 47 us tiled, 24 us in groups of 64 rows; 200 rows, 224: 47 us in groups, 300 rows, 320: 52 us tiled;
     // 30,000 x 515, 469 a row of tiles: 17 rows 54.2 in groups and 25.3 tiled, 64 rows 108 and 47, in bfloat16 132 and 62)

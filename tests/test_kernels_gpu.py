@@ -337,6 +337,29 @@ def test_gemm_plain_up_to_eight_rows(K, ta, tw, n, k):
     assert not bool(got[2, :5].isfinite().any()) and not bool(got[0, 5].isfinite())
 
 
+# Tiles whose stages of 32 columns come by themselves: 64 x 64 (also for up to 64 rows), 32 x 128 (also for up to 32) and 128 x 128,
+# their last rows and columns broken, one stage, two, three and more, whole and broken.
+@pytest.mark.parametrize("m,n", [(33, 8200), (64, 8250), (17, 16400), (32, 16390),
+                                 (300, 4000), (70, 10700), (65, 8190), (777, 10700), (257, 10700), (300, 10752)])
+@pytest.mark.parametrize("k", [4, 28, 32, 36, 64, 92, 100, 132, 516])
+def test_gemm_plain_rings(K, m, n, k):
+    g = torch.Generator().manual_seed(m + n + k)
+    a, w = torch.randn(m, k + 8, generator=g).to(DEV), torch.randn(n, k + 4, generator=g).to(DEV)[:, :k]
+    x = a[:, 4:4 + k]
+    c = torch.full((m + 1, n + 2), 7.0, device=DEV)
+    K.gemm_plain(x, w, c[:m, :n])
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((c[:m, :n].double() - x.double() @ w.double().T).abs() <= bound).all())
+    assert bool((c[m] == 7.0).all()) and bool((c[:, n:] == 7.0).all())
+    x[1, k - 1], x[m - 1, 0], w[5, 2], w[n - 1, k - 2] = float("nan"), float("inf"), float("-inf"), float("inf")
+    K.gemm_plain(x, w, c[:m, :n])                                  # they stay in their rows and columns
+    plain = torch.ones(m, n, dtype=torch.bool, device=DEV)
+    plain[[1, m - 1]] = False
+    plain[:, [5, n - 1]] = False
+    assert bool(c[1, :n].isnan().all()) and bool(c[:m, :n][plain].isfinite().all())
+    assert not bool(c[:m, :n][~plain].isfinite().any())
+
+
 @pytest.mark.parametrize("m,n,k", [(2, 40, 17), (70, 40, 18), (300, 3300, 20), (290, 3300, 18), (97, 5500, 20), (17, 16400, 258), (40, 8200, 257)])
 def test_gemm_plain_special_values_in_every_kernel(K, m, n, k):
     """A NaN or an infinity stays in its row and column, and zeros behind the last k meet zeros only."""
