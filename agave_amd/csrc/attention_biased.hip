@@ -616,10 +616,12 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
             valid[cb] = false;
         }
     } else {
+        // (along x the heads come first, so that the workgroups of a head share an XCD's L2 where the heads are a multiple
+        // of eight, then the runs of rows, the latest, which see the most keys, in front)
         b = blockIdx.y;
-        const int r0 = M.cu[b] + blockIdx.x * 4 * WROWS, r1 = M.cu[b + 1];
+        const int runs = gridDim.x / nh, r0 = M.cu[b] + (runs - 1 - (int)blockIdx.x / nh) * 4 * WROWS, r1 = M.cu[b + 1];
         if (r0 >= r1) return;                                   // (the whole workgroup: a shorter sequence of the batch)
-        head = blockIdx.z;
+        head = blockIdx.x % nh;
         if (M.table_in_lds) {                                   // (before any wave leaves: all of them meet at the barrier)
             const float* src = A.bias + (size_t)head * A.bias_len;
             for (int i = threadIdx.x; i < A.bias_len; i += blockDim.x) lds[i] = src[i] * 1.4426950408889634f;
@@ -642,6 +644,9 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
     }
     const int kvh = head / per;
     const int ksl = (hd + 31) / 32;                 // steps along the head that the pages hold
+    // steps that the pages hold whatever the head's size (the launch takes the least KS that holds it): only the others
+    // are emptied, four instructions an operand
+    constexpr int KALL = KS <= 2 ? KS : KS == 4 ? 3 : KS <= 8 ? 5 : 1;
     const int W = A.window, keep = A.keep_first, C = A.chunk;
     int lo = W > 0 ? max(0, pmin - W + 1) : 0;
     if (C > 0) lo = max(lo, (pmin / C) * C);           // (the earliest chunk start among the wave's rows)
@@ -707,14 +712,8 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
         const long pg = (col >= 0 && col < A.width) ? A.table[(size_t)b * A.width + col] : -1;
         return pg < A.n_pages ? pg : -1;
     };
-    // One page: kt and vt hold its key and value operands, 64 lanes x 16 bytes each (tile (kb, ks) of the keys at
-    // kb ksl + ks, tile (nb, h) of the values at 2 nb + h), in memory or in LDS.
-    auto page = [&](int pi, auto kt, auto vt) {
-        // What the page needs from memory is asked for before any of it is used (a wave's loads come back in the
-        // order they left): the bias where it is read from memory, the value operands where the registers allow, then
-        // the keys.
-        constexpr bool V_AHEAD = VB <= 8 && NC == 1;
-        float bv[NC][4][4];
+    // the page's bias where it is read from memory
+    auto load_bias = [&](int pi, float (&bv)[NC][4][4]) {
         if (A.bias_mode == 2 && !M.table_in_lds) {
 #pragma unroll
             for (int cb = 0; cb < NC; ++cb)
@@ -726,6 +725,109 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
                         bv[cb][kb][e] = bias_row[dist < 0 ? 0 : (dist < A.bias_len ? dist : A.bias_len - 1)] * LOG2E;
                     }
         }
+    };
+    // Scale, bias, mask and softmax, a column block at a time, in the base-2 domain (scale, slopes, table and
+    // sinks carry the factor log2(e), so an exponential is one instruction).  A page that every row of the wave
+    // sees whole (below the diagonal, inside the window or among the kept positions) needs no mask: most pages
+    // of a long sequence are such, and the mask is most of the arithmetic of a score.
+    auto softmax = [&](int pi, f32x4_t (&s)[NC][4], auto& bv, frag16 (&pf)[NC][2], float (&alpha)[NC]) {
+        const int j_last = pi * AGAVE_PAGE + AGAVE_PAGE - 1;
+        const bool whole = j_last <= pmin && (W == 0 || pmax - pi * AGAVE_PAGE < W || j_last < keep) &&
+                           (C == 0 || pi * AGAVE_PAGE >= cstart_max);
+        auto scores = [&](auto whole_tag, auto kind_tag) {
+            constexpr bool WHOLE = decltype(whole_tag)::value != 0, PLAIN = decltype(kind_tag)::value == 0, TABLE = decltype(kind_tag)::value == 2;
+#pragma unroll
+            for (int cb = 0; cb < NC; ++cb) {
+                float tile_max = -INFINITY;
+                const int d0 = pos[cb] - pi * AGAVE_PAGE - 8 * g;           // distance to the lane group's first key
+                const float t0 = -slope2 * (float)d0;
+#pragma unroll
+                for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int off = 32 * (kb >> 1) + 4 * (kb & 1) + e;  // (a constant once the loops are unrolled)
+                        const int dist = d0 - off;
+                        float v;
+                        if (PLAIN) {
+                            v = fmaf(s[cb][kb][e], scale2, 0.f);          // (a sum, so that the difference below is not taken into one rounding with it)
+                        } else if (cap2 > 0.f) {
+                            // cap tanh(x / cap) with tanh(z) = 1 - 2 / (e^(2z) + 1), which is right at both ends
+                            const float e2 = __builtin_amdgcn_exp2f(s[cb][kb][e] * scale_cap * 2.8853900817779268f);
+                            v = fmaf(cap2, 1.0f - 2.0f * __builtin_amdgcn_rcpf(e2 + 1.0f), fmaf(slope2, (float)off, t0));
+                        } else {
+                            v = fmaf(s[cb][kb][e], scale2, fmaf(slope2, (float)off, t0));
+                        }
+                        bool see = true;
+                        if (!WHOLE) see = valid[cb] && dist >= 0 && (W == 0 || dist < W || pos[cb] - dist < keep) &&
+                                          pos[cb] - dist >= cstart[cb];
+                        if (TABLE) {
+                            int at = dist < A.bias_len ? dist : A.bias_len - 1;
+                            if (!WHOLE) at = see ? at : 0;
+                            if constexpr (LDSP) v += M.table_in_lds ? lds[at] : bias_row[at] * LOG2E;      // (no registers for a page's bias)
+                            else v += M.table_in_lds ? lds[at] : bv[cb][kb][e];
+                        }
+                        if (!WHOLE) v = see ? v : -INFINITY;
+                        s[cb][kb][e] = v;
+                        tile_max = fmaxf(tile_max, v);
+                    }
+                }
+                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16));
+                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+                const float m_new = fmaxf(m[cb], tile_max);
+                // (a column that sees nothing of this page and has seen nothing before keeps m = -inf; its p are 0)
+                const float ref = m_new == -INFINITY ? 0.f : m_new;
+                alpha[cb] = m[cb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[cb] - ref);
+                float sum = 0.f;
+#pragma unroll
+                for (int kb = 0; kb < 4; ++kb) {
+                    float p[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        p[e] = __builtin_amdgcn_exp2f(s[cb][kb][e] - ref);      // 2^(-inf) = 0 for what is not seen
+                        sum += p[e];
+                    }
+                    const uint32_t lo2 = f32x2_to_bf16x2(p[0], p[1]), hi2 = f32x2_to_bf16x2(p[2], p[3]);
+                    if (kb & 1) {
+                        pf[cb][kb >> 1].r[2] = lo2;
+                        pf[cb][kb >> 1].r[3] = hi2;
+                    } else {
+                        pf[cb][kb >> 1].r[0] = lo2;
+                        pf[cb][kb >> 1].r[1] = hi2;
+                    }
+                }
+                l[cb] = l[cb] * alpha[cb] + sum;
+                m[cb] = m_new;
+            }
+        };
+        if (A.bias_mode == 2) {
+            if (whole) scores(IntC<1>{}, IntC<2>{}); else scores(IntC<0>{}, IntC<2>{});
+        } else if (A.bias_mode == 1 || cap2 > 0.f) {
+            if (whole) scores(IntC<1>{}, IntC<1>{}); else scores(IntC<0>{}, IntC<1>{});
+        } else {
+            if (whole) scores(IntC<1>{}, IntC<0>{}); else scores(IntC<0>{}, IntC<0>{});
+        }
+    };
+    auto rescale = [&](const float (&alpha)[NC]) {
+        // (the references move on a few of the first pages and seldom afterwards)
+        bool moved = false;
+#pragma unroll
+        for (int cb = 0; cb < NC; ++cb) moved = moved || alpha[cb] != 1.f;
+        if (__any(moved)) {
+#pragma unroll
+            for (int nb = 0; nb < VB; ++nb)
+#pragma unroll
+                for (int cb = 0; cb < NC; ++cb) o[cb][nb] *= alpha[cb];
+        }
+    };
+    // One page: kt and vt hold its key and value operands, 64 lanes x 16 bytes each (tile (kb, ks) of the keys at
+    // kb ksl + ks, tile (nb, h) of the values at 2 nb + h), in memory or in LDS.
+    auto page = [&](int pi, auto kt, auto vt) {
+        // What the page needs from memory is asked for before any of it is used (a wave's loads come back in the
+        // order they left): the bias where it is read from memory, the value operands where the registers allow, then
+        // the keys.
+        constexpr bool V_AHEAD = VB <= 8 && NC == 1;
+        float bv[NC][4][4];
+        load_bias(pi, bv);
         frag16 va[V_AHEAD ? VB : 1][2];
         if (V_AHEAD) {
 #pragma unroll
@@ -792,8 +894,9 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
 #pragma unroll
                     for (int kk = 0; kk < KCH; ++kk) {
                         const int ks = k0 + kk;
-                        const u32x4_t got = kt[(kb * ksl + (ks < ksl ? ks : 0)) * 64 + lane];
-                        kf[kk].r = ks < ksl ? got : u32x4_t{0u, 0u, 0u, 0u};
+                        const bool held = ks < KALL || ks < ksl;
+                        const u32x4_t got = kt[(kb * ksl + (held ? ks : 0)) * 64 + lane];
+                        kf[kk].r = held ? got : u32x4_t{0u, 0u, 0u, 0u};
                     }
 #pragma unroll
                     for (int cb = 0; cb < NC; ++cb) {
@@ -810,82 +913,9 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
                 }
             }
         }
-        // Scale, bias, mask and softmax, a column block at a time, in the base-2 domain (scale, slopes, table and
-        // sinks carry the factor log2(e), so an exponential is one instruction).  A page that every row of the wave
-        // sees whole (below the diagonal, inside the window or among the kept positions) needs no mask: most pages
-        // of a long sequence are such, and the mask is most of the arithmetic of a score.
         frag16 pf[NC][2];
         float alpha[NC];
-        const int j_last = pi * AGAVE_PAGE + AGAVE_PAGE - 1;
-        const bool whole = j_last <= pmin && (W == 0 || pmax - pi * AGAVE_PAGE < W || j_last < keep) &&
-                           (C == 0 || pi * AGAVE_PAGE >= cstart_max);
-        auto scores = [&](auto whole_tag, auto table_tag) {
-            constexpr bool WHOLE = decltype(whole_tag)::value != 0, TABLE = decltype(table_tag)::value != 0;
-#pragma unroll
-            for (int cb = 0; cb < NC; ++cb) {
-                float tile_max = -INFINITY;
-                const int d0 = pos[cb] - pi * AGAVE_PAGE - 8 * g;           // distance to the lane group's first key
-                const float t0 = -slope2 * (float)d0;
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int off = 32 * (kb >> 1) + 4 * (kb & 1) + e;  // (a constant once the loops are unrolled)
-                        const int dist = d0 - off;
-                        float v;
-                        if (cap2 > 0.f) {
-                            // cap tanh(x / cap) with tanh(z) = 1 - 2 / (e^(2z) + 1), which is right at both ends
-                            const float e2 = __builtin_amdgcn_exp2f(s[cb][kb][e] * scale_cap * 2.8853900817779268f);
-                            v = fmaf(cap2, 1.0f - 2.0f * __builtin_amdgcn_rcpf(e2 + 1.0f), fmaf(slope2, (float)off, t0));
-                        } else {
-                            v = fmaf(s[cb][kb][e], scale2, fmaf(slope2, (float)off, t0));
-                        }
-                        bool see = true;
-                        if (!WHOLE) see = valid[cb] && dist >= 0 && (W == 0 || dist < W || pos[cb] - dist < keep) &&
-                                          pos[cb] - dist >= cstart[cb];
-                        if (TABLE) {
-                            int at = dist < A.bias_len ? dist : A.bias_len - 1;
-                            if (!WHOLE) at = see ? at : 0;
-                            v += M.table_in_lds ? lds[at] : bv[cb][kb][e];
-                        }
-                        if (!WHOLE) v = see ? v : -INFINITY;
-                        s[cb][kb][e] = v;
-                        tile_max = fmaxf(tile_max, v);
-                    }
-                }
-                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16));
-                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-                const float m_new = fmaxf(m[cb], tile_max);
-                // (a column that sees nothing of this page and has seen nothing before keeps m = -inf; its p are 0)
-                const float ref = m_new == -INFINITY ? 0.f : m_new;
-                alpha[cb] = m[cb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[cb] - ref);
-                float sum = 0.f;
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb) {
-                    float p[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        p[e] = __builtin_amdgcn_exp2f(s[cb][kb][e] - ref);      // 2^(-inf) = 0 for what is not seen
-                        sum += p[e];
-                    }
-                    const uint32_t lo2 = f32x2_to_bf16x2(p[0], p[1]), hi2 = f32x2_to_bf16x2(p[2], p[3]);
-                    if (kb & 1) {
-                        pf[cb][kb >> 1].r[2] = lo2;
-                        pf[cb][kb >> 1].r[3] = hi2;
-                    } else {
-                        pf[cb][kb >> 1].r[0] = lo2;
-                        pf[cb][kb >> 1].r[1] = hi2;
-                    }
-                }
-                l[cb] = l[cb] * alpha[cb] + sum;
-                m[cb] = m_new;
-            }
-        };
-        if (A.bias_mode == 2) {
-            if (whole) scores(IntC<1>{}, IntC<1>{}); else scores(IntC<0>{}, IntC<1>{});
-        } else {
-            if (whole) scores(IntC<1>{}, IntC<0>{}); else scores(IntC<0>{}, IntC<0>{});
-        }
+        softmax(pi, s, bv, pf, alpha);
         // O^T = O^T alpha + V^T P^T
         if constexpr (VB > 16 && !QL) {
             // (wide values: two blocks' operands at a time, the next two asked for while these are multiplied)
@@ -919,6 +949,7 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
                 }
             }
         } else {
+        rescale(alpha);
 #pragma unroll
         for (int nb = 0; nb < VB; ++nb) {
             if (16 * nb < vd) {
@@ -932,7 +963,6 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
                 }
 #pragma unroll
                 for (int cb = 0; cb < NC; ++cb) {
-                    o[cb][nb] *= alpha[cb];
                     o[cb][nb] = mfma_16x16x32(vf[0], pf[cb][0], o[cb][nb]);
                     o[cb][nb] = mfma_16x16x32(vf[1], pf[cb][1], o[cb][nb]);
                 }
@@ -942,6 +972,103 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
             }
         }
         }
+    };
+
+    // The same from a page in LDS at `kaddr` (this lane's 16 bytes of its first tile; `vaddr` of its first value tile) while the next
+    // page is on its way there.  The LDS reads are written as instructions (see lds_read16: left to the compiler each waits for
+    // that page): the keys in batches, a batch asked for while the one before it is multiplied, the values' first batch
+    // before the exponentials are computed.
+    // Bound by a wave's own chain of multiplications and exponentials.  Prompt of 3,001 tokens, 16 heads of 192 and 128: 143 us
+    // (159 with reads by the compiler; 200 when the pages' numbers were asked for behind the pages' loads, too).
+    auto page_in_lds = [&](int pi, unsigned kaddr, auto vaddr) {             // (generic: only what calls it has it)
+        constexpr int KB = KS <= 4 ? KS : KS / 2, NBAT = 4 * KS / KB;           // tiles a batch (registers: two batches), batches
+        constexpr int VH = VB <= 4 ? 1 : VB / 4, NVB = VB / VH;                 // value blocks a batch, two tiles each; batches
+        f32x4_t s[NC][4];
+#pragma unroll
+        for (int cb = 0; cb < NC; ++cb)
+#pragma unroll
+            for (int kb = 0; kb < 4; ++kb) s[cb][kb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        frag16 kf[2][KB];
+        auto read_keys = [&](auto bat) {
+            constexpr int kb = bat.value * KB / KS, k0 = bat.value * KB % KS;
+            const unsigned at = kaddr + (unsigned)(kb * ksl) * 1024u;
+            static_for<0, KB>([&](auto i) {
+                constexpr int ks = k0 + i.value;
+                if constexpr (ks < KALL) lds_read16<ks * 1024>(kf[bat.value & 1][i.value], at);
+                else lds_read16<0>(kf[bat.value & 1][i.value], at + (ks < ksl ? ks * 1024u : 0u));
+            });
+        };
+        read_keys(IntC<0>{});
+        static_for<0, NBAT>([&](auto bat) {
+            constexpr int kb = bat.value * KB / KS, k0 = bat.value * KB % KS;
+            if constexpr (bat.value + 1 < NBAT) {
+                read_keys(IntC<bat.value + 1>{});
+                lds_settle_to<KB>();
+            } else {
+                lds_settle();
+            }
+#pragma unroll
+            for (int i = 0; i < KB; ++i) {
+                lds_use(kf[bat.value & 1][i]);
+                if (!(k0 + i < KALL || k0 + i < ksl)) kf[bat.value & 1][i].r = u32x4_t{0u, 0u, 0u, 0u};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < KB; ++i)
+#pragma unroll
+                for (int cb = 0; cb < NC; ++cb) s[cb][kb] = mfma_16x16x32(kf[bat.value & 1][i], qf[cb][QL ? 0 : k0 + i], s[cb][kb]);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        // (the first half of the blocks always exists, see the launch; of the second, one past the value size reads the first
+        // block again and is not used)
+        frag16 vf[2][2 * VH];
+        auto read_values = [&](auto bat) {
+            static_for<0, VH>([&](auto i) {
+                constexpr int nb = bat.value * VH + i.value;
+                frag16 (&to)[2 * VH] = vf[bat.value & 1];
+                if constexpr (nb < (VB + 1) / 2) {
+                    lds_read16<nb * 2048>(to[2 * i.value], vaddr);
+                    lds_read16<nb * 2048 + 1024>(to[2 * i.value + 1], vaddr);
+                } else {
+                    const unsigned at = vaddr + (16 * nb < vd ? nb * 2048u : 0u);
+                    lds_read16<0>(to[2 * i.value], at);
+                    lds_read16<1024>(to[2 * i.value + 1], at);
+                }
+            });
+        };
+        constexpr bool V_FIRST = KS <= 6;                                       // (the longest heads' Q leaves no registers for it)
+        if constexpr (V_FIRST) read_values(IntC<0>{});
+        __builtin_amdgcn_sched_barrier(0);
+        frag16 pf[NC][2];
+        float alpha[NC];
+        softmax(pi, s, o, pf, alpha);                                           // (no bias by key: it is looked up where it is added)
+        rescale(alpha);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!V_FIRST) read_values(IntC<0>{});
+        static_for<0, NVB>([&](auto bat) {
+            if constexpr (bat.value + 1 < NVB) {
+                read_values(IntC<bat.value + 1>{});
+                lds_settle_to<2 * VH>();
+            } else {
+                lds_settle();
+            }
+            frag16 (&now)[2 * VH] = vf[bat.value & 1];
+#pragma unroll
+            for (int i = 0; i < 2 * VH; ++i) lds_use(now[i]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < VH; ++i) {
+                const int nb = bat.value * VH + i;
+                if (nb < (VB + 1) / 2 || 16 * nb < vd) {
+#pragma unroll
+                    for (int cb = 0; cb < NC; ++cb) {
+                        o[cb][nb] = mfma_16x16x32(now[2 * i], pf[cb][0], o[cb][nb]);
+                        o[cb][nb] = mfma_16x16x32(now[2 * i + 1], pf[cb][1], o[cb][nb]);
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
     };
 
     if constexpr (LDSP) {
@@ -962,9 +1089,7 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
             const long pg = (col >= 0 && col < A.width) ? A.table[(size_t)b * A.width + col] : -1;
             return pg < A.n_pages ? pg : -1;
         };
-        auto fetch = [&](int gi, int buf) {
-            int pi;
-            const long pg = page_at(gi, pi);
+        auto fetch = [&](long pg, int buf) {
             if (pg < 0) return;
             const uint4* ksrc = (const uint4*)A.k_pages + ((size_t)pg * nkv + kvh) * (size_t)n_k * 64;
             const uint4* vsrc = (const uint4*)A.v_pages + ((size_t)pg * nkv + kvh) * (size_t)n_v * 64;
@@ -975,21 +1100,28 @@ __global__ __launch_bounds__((KS > 8 || VB > 16) ? 256 : 512) void attn_biased_m
                                                  (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
             }
         };
-        fetch(0, 0);
+        // The pages' numbers are asked for two pages ahead: a number that was asked for behind the next page's loads would
+        // arrive behind them (a wave's loads come back in order), and no page would travel while another is multiplied.
+        int pi, pi_next, pi_after;
+        long pg = page_at(0, pi), pg_next = page_at(1, pi_next);
+        fetch(pg, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         for (int gi = 0; gi < g_n; ++gi) {
             const int buf = gi & 1;
-            if (gi + 1 < g_n) fetch(gi + 1, buf ^ 1);
-            int pi;
-            const long pg = page_at(gi, pi);
+            const long pg_after = page_at(gi + 2, pi_after);
+            if (gi + 1 < g_n) fetch(pg_next, buf ^ 1);
             const bool mine = wave_on && pg >= 0 && pi <= pmax / AGAVE_PAGE && (pi >= first_win || pi * AGAVE_PAGE < keep);
             if (mine) {
-                const lds_u32x4* kl = pages + (size_t)buf * buf_tiles * 64;
-                page(pi, kl, kl + (size_t)n_k * 64);
+                const unsigned kaddr = (unsigned)(uintptr_t)pages + (unsigned)(buf * buf_tiles * 64 + lane) * 16u;
+                page_in_lds(pi, kaddr, kaddr + (unsigned)n_k * 1024u);
             }
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
+            pi = pi_next;
+            pg = pg_next;
+            pi_next = pi_after;
+            pg_next = pg_after;
         }
         if (!wave_on) return;
     } else {
@@ -1213,8 +1345,9 @@ extern "C" int agave_attn_biased_mfma(const void* q, long ldq, void* out, long l
             else
                 nc = 1;
         }
-        grid = dim3((max_rows + 64 * nc - 1) / (64 * nc), n_seqs, nh);
-        AGAVE_CHECK(grid.y <= 65535 && grid.z <= 65535, "attn_biased_mfma: too many sequences or heads for the grid");
+        const long blocks = (long)((max_rows + 64 * nc - 1) / (64 * nc)) * nh;
+        AGAVE_CHECK(n_seqs <= 65535 && nh <= 65535 && blocks <= 0x7fffffffl, "attn_biased_mfma: too many sequences or heads for the grid");
+        grid = dim3((unsigned)blocks, n_seqs, 1);
     }
     if (ks > 12) {                                      // Q in LDS, behind whatever else is there
         M.q_off = (int)(lds_bytes / sizeof(float));

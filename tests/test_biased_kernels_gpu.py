@@ -196,6 +196,23 @@ def test_long_prompts_share_pages_through_lds(shape):
     close(c.run([(0, 230), (230, T)], torch.bfloat16), ref, torch.bfloat16, f"{shape} 230 + 870")
 
 
+@pytest.mark.parametrize("shape", [
+    (16, 2, 136, 112, None, 0, "none", False, True),      # keys of four steps and a fourth, a value block short of the kernel's
+    (16, 4, 192, 128, 300, 70, "slopes", True, False),    # the heads of a latent attention, whole
+    (16, 1, 232, 80, 130, 0, "none", False, False),       # keys of eight steps, the last not whole; five value blocks of eight
+    (17, 17, 256, 32, None, 0, "table", False, False),    # the longest keys beside the shortest values
+    (20, 4, 104, 16, None, 0, "none", False, False),      # keys of four steps, the last not whole; one value block
+])
+def test_long_prompts_of_heads_that_fill_the_kernel_in_part(shape):
+    """Pages through LDS for heads whose last step along the keys, or whose last value blocks, the kernel has and the pages
+    have not; heads that are no multiple of the XCDs.  A step of eight rows' runs, the last one short."""
+    T = 128 * 12 + 5 if shape[2] <= 128 else 128 * 8 + 5
+    c = Case(*shape, T=T, seed=9)
+    c.rounded(torch.bfloat16)
+    ref = c.plain()
+    close(c.run([(0, T)], torch.bfloat16), ref, torch.bfloat16, f"{shape} whole")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_a_batch_against_each_alone_and_slots_and_pages_used_again(dtype):
     from agave_amd.ops import attention_biased as A
