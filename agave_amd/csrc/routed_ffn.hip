@@ -124,7 +124,13 @@ __device__ __forceinline__ void load8(const float* p, float* v) {
 // a whole row's share of loads in flight at once).
 // OUT outputs a wave at a time: one, or two, w and w + nw, whose rows are one round trip to memory (a wave without a second
 // one reads its first again).
-template <typename T, bool WIDE, int RR, int OUT>
+// TILES > 0 (many tokens, RR = 16): the matrix cores' 32-bit instruction makes the product, TILES tiles of 16 outputs by the
+// workgroup's 16 tokens, and plain multiply-adds up to two outputs behind them (a shared expert's gate would else cost a
+// tile).  The sixteen waves take runs of 32 columns in turn, lane i + 16 g columns 8 g .. 8 g + 7 of row i of either
+// operand, which is the same order for both; four running sums a tile, so that none is longer than a lane's of the other way.
+// That one reads every token's row once for each output (pair) and is bound by these reads from the compute unit's cache; here a
+// row is read once.  3,001 tokens of 2,048 by 17 outputs, in a prompt: 30.1 -> 13.7 us.
+template <typename T, bool WIDE, int RR, int OUT, int TILES>
 __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ x, long ldx, const float* __restrict__ router,
                                                           const float* __restrict__ correction, int N, int K, int R, int groups,
                                                           int keep, int top, float scale, int* __restrict__ choice,
@@ -137,7 +143,65 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
     for (int e = threadIdx.x; e < R; e += blockDim.x) corr[e] = correction ? correction[e] : 0.f;
     const int t0 = blockIdx.x * RR;
     const int rows = min(RR, N - t0);
-    for (int r = w; r < Rt; r += OUT * nw) {
+    if constexpr (TILES > 0) {
+        constexpr int NW = 16, REST = 2;
+        float* part = corr + R;                // [NW][RR][Rt]
+        const int i = lane & 15, g = lane >> 4, tiled = min(Rt, 16 * TILES), rest = Rt - tiled;
+        const T* xr = x + (size_t)(t0 + min(i, rows - 1)) * ldx + 8 * g;
+        const float* wt[TILES];
+#pragma unroll
+        for (int j = 0; j < TILES; ++j) wt[j] = router + (size_t)min(16 * j + i, Rt - 1) * K + 8 * g;     // (outputs past the end: never stored)
+        const float* wr[REST];
+#pragma unroll
+        for (int j = 0; j < REST; ++j) wr[j] = router + (size_t)min(tiled + j, Rt - 1) * K + 8 * g;
+        f32x4_t acc[TILES][4] = {};
+        float more[REST][2] = {};
+#pragma unroll(TILES == 1 ? 4 : TILES == 2 ? 2 : 1)
+        for (int k = 32 * w; k < K; k += 32 * NW) {
+            float xv[8], wv[TILES][8], rv[REST][8];
+            load8(xr + k, xv);
+#pragma unroll
+            for (int j = 0; j < TILES; ++j) load8(wt[j] + k, wv[j]);
+#pragma unroll
+            for (int j = 0; j < REST; ++j)
+                if (j < rest) load8(wr[j] + k, rv[j]);
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+#pragma unroll
+                for (int j = 0; j < TILES; ++j) acc[j][m & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[m], wv[j][m], acc[j][m & 3], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < REST; ++j)
+                    if (j < rest) more[j][m & 1] = fmaf(xv[m], rv[j][m], more[j][m & 1]);
+            }
+        }
+        // a tile: lane holds tokens 4 g + e of output 16 j + i; the rest: lane holds a fourth of token i's sum
+        float* mine = part + w * RR * Rt;
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (16 * j + i < tiled) mine[(4 * g + e) * Rt + 16 * j + i] = (acc[j][0][e] + acc[j][1][e]) + (acc[j][2][e] + acc[j][3][e]);
+#pragma unroll
+        for (int j = 0; j < REST; ++j)
+            if (j < rest) {
+                float sum = more[j][0] + more[j][1];
+                sum += __shfl_xor(sum, 16);
+                sum += __shfl_xor(sum, 32);
+                if (g == 0) mine[i * Rt + tiled + j] = sum;
+            }
+        __syncthreads();
+        for (int at = threadIdx.x; at < RR * Rt; at += 64 * NW) {
+            float sum[NW];
+#pragma unroll
+            for (int o = 0; o < NW; ++o) sum[o] = part[o * RR * Rt + at];
+#pragma unroll
+            for (int half = NW / 2; half > 0; half /= 2)
+#pragma unroll
+                for (int o = 0; o < half; ++o) sum[o] += sum[o + half];
+            zs[at] = sum[0];
+        }
+    }
+    for (int r = w; TILES == 0 && r < Rt; r += OUT * nw) {
         const bool second = OUT == 2 && r + nw < Rt;
         const float* wr = router + (size_t)r * K;
         const float* wr2 = second ? wr + (size_t)nw * K : wr;
@@ -322,6 +386,22 @@ extern "C" int agave_route_rows(int dtype, const void* x, long ldx, const float*
     const bool wide = K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 32) == 0 && ((uintptr_t)router % 32) == 0;
     AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "route_rows: unknown dtype %d", dtype);
     const bool f32 = dtype == AGAVE_F32;
+    // Many tokens, more than a few outputs and whole runs of 32 columns: tiles of 16 outputs on the matrix cores, a last tile of one
+    // or two left to plain multiply-adds.  From 2,049 tokens on, where eight a workgroup are more than one round of
+    // workgroups.  us, the other way and this, bfloat16 rows of 2,048: 17 outputs 2,000 tokens 13.6 and 13.3, 3,001 22.4 and 13.3, 12,000
+    // 51.9 and 35.4; 32 outputs 13.5 and 16.2, 22.4 and 16.4, 66.7 and 45.4; 49 outputs 21.6 and 21.6, 37.5 and 22.1, 105 and 63;
+    // 8 outputs 12,000 tokens 27.5 and 27.6, rows of 512 17.5 and 18.2.
+    const int outputs_all = R + extra, tiles = outputs_all < 16 || outputs_all % 16 > 2 ? (outputs_all + 15) / 16 : outputs_all / 16;
+    if (wide && K % 32 == 0 && N > 2048 && outputs_all > 8 && tiles <= 3) {
+        const size_t lds_tiles = ((size_t)17 * 16 * outputs_all + R) * sizeof(float);
+#define ROUTE_TILES(T_, TILES_) route_rows_kernel<T_, true, 16, 1, TILES_><<<(N + 15) / 16, 1024, lds_tiles, stream>>>((const T_*)x, ldx, router, correction, \
+        N, K, R, groups, keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise)
+        if (f32) { if (tiles == 1) ROUTE_TILES(float, 1); else if (tiles == 2) ROUTE_TILES(float, 2); else ROUTE_TILES(float, 3); }
+        else if (tiles == 1) ROUTE_TILES(bf16, 1); else if (tiles == 2) ROUTE_TILES(bf16, 2); else ROUTE_TILES(bf16, 3);
+#undef ROUTE_TILES
+        AGAVE_LAUNCH_CHECK("route_rows");
+        return 0;
+    }
     const int rows = N <= 64 ? 1 : 8, blocks = (N + rows - 1) / rows;
     const int threads = blocks <= 512 ? 1024 : 256;            // (more waves to share the outputs while they all fit the chip at once)
     const size_t lds = (size_t)(rows * (R + extra) + R) * sizeof(float);
@@ -333,7 +413,7 @@ extern "C" int agave_route_rows(int dtype, const void* x, long ldx, const float*
     // token 24.3 and 25.1, 12 tokens 22.8 and 21.1.
     const int waves = threads / 64, outputs = R + extra, last = outputs % (2 * waves);
     const bool two = outputs > waves && (rows == 8 || (N > 2 ? last == 0 || last <= waves / 2 || last > waves : last > waves && last <= waves * 3 / 2));
-#define ROUTE_GO(T_, W_, RR_, OUT_) route_rows_kernel<T_, W_, RR_, OUT_><<<blocks, threads, lds, stream>>>((const T_*)x, ldx, router, correction, N, K, R, groups, \
+#define ROUTE_GO(T_, W_, RR_, OUT_) route_rows_kernel<T_, W_, RR_, OUT_, 0><<<blocks, threads, lds, stream>>>((const T_*)x, ldx, router, correction, N, K, R, groups, \
         keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise)
 #define ROUTE_ROWS(T_, W_) do { if (rows == 1 && two) ROUTE_GO(T_, W_, 1, 2); else if (rows == 1) ROUTE_GO(T_, W_, 1, 1); \
         else if (two) ROUTE_GO(T_, W_, 8, 2); else ROUTE_GO(T_, W_, 8, 1); } while (0)
@@ -512,40 +592,81 @@ extern "C" int agave_routed_combine(int dtype, const float* y, const int* place,
 //   tile_expert[t]  expert of tile t (-1: no such tile)
 // The order of an expert's pairs among themselves is whatever the atomics make it; every row's result is
 // its own, so nothing depends on it.
+// A thread keeps its pairs' choices and ranks in registers (SORT_PER of them; of more pairs the ranks wait in `place`), all loads
+// of choices leave together and the experts' first tiles are counted up across the lanes.  12,004 pairs of 16
+// experts, tiles of 128: 9.1 us, with a load, an atomic and a store at a time and one thread for the tiles 16.1; 32,768 of 64 20.7
+// and 55.0.
+#define SORT_PER 32
 __global__ __launch_bounds__(1024) void route_sort_kernel(const int* __restrict__ choice, int P, int E, int TM, int cap,
                                                           int max_tiles, int* __restrict__ place,
                                                           int* __restrict__ sorted_pair, int* __restrict__ tile_expert) {
     __shared__ int counts[ROUTE_MAX];
     __shared__ int first_row[ROUTE_MAX];
+    __shared__ int wave_tiles[16];
     const int tid = threadIdx.x;
-    for (int e = tid; e < E; e += blockDim.x) counts[e] = 0;
-    for (int r = tid; r < cap; r += blockDim.x) sorted_pair[r] = -1;
-    for (int t = tid; t < max_tiles; t += blockDim.x) tile_expert[t] = -1;
-    __syncthreads();
-    for (int p = tid; p < P; p += blockDim.x) {
-        const int e = choice[p];
-        place[p] = (e >= 0 && e < E) ? atomicAdd(&counts[e], 1) : -1;        // for now: the pair's rank within its expert
+    const bool kept = P <= SORT_PER * 1024;
+    int e[SORT_PER], rank[SORT_PER];
+    if (kept) {
+#pragma unroll
+        for (int u = 0; u < SORT_PER; ++u) {
+            if (u * 1024 >= P) break;
+            e[u] = choice[min(tid + u * 1024, P - 1)];
+        }
     }
+    counts[tid] = 0;                                       // (ROUTE_MAX is the workgroup's size)
+    for (int r = tid; r < cap; r += 1024) sorted_pair[r] = -1;
     __syncthreads();
-    if (tid == 0) {
-        int tile = 0;
-        for (int e = 0; e < E; ++e) {
-            first_row[e] = tile * TM;
-            const int n = (counts[e] + TM - 1) / TM;
-            for (int i = 0; i < n && tile + i < max_tiles; ++i) tile_expert[tile + i] = e;
-            tile += n;
+    if (kept) {
+#pragma unroll
+        for (int u = 0; u < SORT_PER; ++u) {
+            if (u * 1024 >= P) break;
+            if (tid + u * 1024 >= P || e[u] >= E) e[u] = -1;
+            rank[u] = e[u] >= 0 ? atomicAdd(&counts[e[u]], 1) : 0;
+        }
+    } else {
+        for (int p = tid; p < P; p += 1024) {
+            const int ep = choice[p];
+            place[p] = (ep >= 0 && ep < E) ? atomicAdd(&counts[ep], 1) : -1;        // for now: the pair's rank within its expert
         }
     }
     __syncthreads();
-    for (int p = tid; p < P; p += blockDim.x) {
-        const int e = choice[p];
-        if (e >= 0 && e < E) {
-            const int r = first_row[e] + place[p];
-            if (r < cap) {
-                place[p] = r;
-                sorted_pair[r] = p;
-            } else {
-                place[p] = -1;          // (cannot happen: cap holds every pair and every expert's padding)
+    const int lane = tid & 63, w = tid >> 6, tiles = tid < E ? (counts[tid] + TM - 1) / TM : 0;      // of expert `tid`
+    int upto = tiles;
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2) {
+        const int below = __shfl_up(upto, o);
+        if (lane >= o) upto += below;
+    }
+    if (lane == 63) wave_tiles[w] = upto;
+    __syncthreads();
+    int all = 0;
+#pragma unroll
+    for (int o = 0; o < 16; ++o) {
+        if (o == w) upto += all;
+        all += wave_tiles[o];
+    }
+    first_row[tid] = (upto - tiles) * TM;
+    for (int t = upto - tiles; t < upto && t < max_tiles; ++t) tile_expert[t] = tid;
+    for (int t = all + tid; t < max_tiles; t += 1024) tile_expert[t] = -1;
+    __syncthreads();
+    // (a row beyond cap cannot be: cap holds every pair and every expert's padding)
+    if (kept) {
+#pragma unroll
+        for (int u = 0; u < SORT_PER; ++u) {
+            if (u * 1024 >= P) break;
+            const int p = tid + u * 1024;
+            if (p >= P) continue;
+            const int r = e[u] >= 0 ? first_row[e[u]] + rank[u] : -1;
+            place[p] = r < cap ? r : -1;
+            if (r >= 0 && r < cap) sorted_pair[r] = p;
+        }
+    } else {
+        for (int p = tid; p < P; p += 1024) {
+            const int ep = choice[p];
+            if (ep >= 0 && ep < E) {
+                const int r = first_row[ep] + place[p];
+                place[p] = r < cap ? r : -1;
+                if (r < cap) sorted_pair[r] = p;
             }
         }
     }

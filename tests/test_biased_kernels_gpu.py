@@ -622,6 +622,47 @@ def test_router_products(dtype, outputs):
             assert bool(((rest.double() - x.double() @ router[1:].double().T).abs() <= bound).all()), (k, n)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("outputs", [8, 9, 15, 16, 17, 18, 19, 32, 34, 35, 48, 50, 51])
+def test_router_products_of_many_tokens(dtype, outputs):
+    """On either side of the line to the tiles of 16 outputs: tiles whole, broken and with one or two outputs behind them, more than
+    three of them; rows with fewer runs of 32 columns than waves, more, and none; tokens that do not fill the last workgroup."""
+    from agave_amd.ops import routed
+    g = torch.Generator().manual_seed(outputs)
+    for n, k in ((2048, 64), (2049, 64), (2050, 544), (2063, 1056), (2049, 40)):
+        x, router = torch.randn(n, k, generator=g).to(dtype).to(DEV), torch.randn(outputs, k, generator=g).to(DEV)
+        x[5], x[n - 1, 3] = float("inf"), float("nan")                     # (these tokens' own results only)
+        choice, weight = torch.full((n, 1), -1, dtype=torch.int32, device=DEV), torch.zeros(n, 1, device=DEV)
+        rest = torch.full((n, outputs - 1), 7.0, device=DEV)
+        routed.route_rows(x, router, None, 1, 1, 1, 2.0, choice, weight, softmax_top=True, extra_out=rest)
+        want, fine = x.double() @ router[1:].double().T, torch.ones(n, dtype=torch.bool, device=DEV)
+        fine[5] = fine[n - 1] = False
+        assert bool((choice[fine] == 0).all()) and bool((weight[fine] == 2.0).all())
+        assert not bool(torch.isfinite(rest[~fine]).any())
+        # (sums of k products in 32-bit are off by at most k 2^-24 of the sum of their sizes)
+        bound = k * 2.0 ** -24 * (x.double().abs() @ router[1:].double().abs().T)
+        assert bool(((rest.double() - want).abs() <= bound)[fine].all()), (k, n)
+
+
+@pytest.mark.parametrize("P,E,chosen", [(1023, 5, 7), (1025, 1000, 1024), (32768, 16, 16), (32769, 65, 65)])
+def test_route_sort_of_many_pairs(P, E, chosen):
+    """The pairs that a thread keeps in registers and one more, experts without a pair, identity choices, experts past a wave."""
+    from agave_amd.ops import routed
+    tm, g = 64, torch.Generator().manual_seed(P)
+    choice = torch.randint(0, chosen, (P,), generator=g).int()
+    tiles = (P + tm - 1) // tm + E
+    place, sorted_pair, tile_expert = (torch.full((k,), -7, dtype=torch.int32, device=DEV) for k in (P, tiles * tm, tiles))
+    routed.route_sort(choice.to(DEV), E, tm, tiles, place, sorted_pair, tile_expert)
+    place, sorted_pair, tile_expert = place.cpu().long(), sorted_pair.cpu().long(), tile_expert.cpu().long()
+    real = choice < E
+    assert bool((place[~real] == -1).all()) and torch.equal(sorted_pair[place[real]], real.nonzero().view(-1))
+    assert torch.equal(tile_expert[place[real] // tm], choice[real].long())
+    assert int((sorted_pair >= 0).sum()) == int(real.sum()) and int(sorted_pair.min()) >= -1
+    count = torch.bincount(choice[real].long(), minlength=E)
+    want = torch.arange(E).repeat_interleave((count + tm - 1) // tm)
+    assert torch.equal(tile_expert, torch.cat([want, torch.full((tiles - len(want),), -1)]))
+
+
 def test_columns_that_the_kernel_of_few_pairs_takes():
     """The rule for the tiles of sorted pairs and the kernel's launch name the same columns."""
     from agave_amd.ops import routed
