@@ -1482,9 +1482,7 @@ static int dispatch_tiled(const void* X, long ldx, const void* Wp, void* Y, long
 // counted in units of one 128 x 256 tile's time: the product takes rounds(tiles * z) / z, and every slice
 // beyond the first costs its bytes, some 0.07 of a tile's time at 160 tiles and 10,240 columns, in
 // proportion to the tiles and inversely to the columns.  Products that run in 256 x 256 tiles are left alone.
-// In which tiles the slices run, and whether the one product is not faster after all, is left to the
-// shapes' times (down of the 4B sizes at 2,048 tokens: 107 us as one product in tiles of 160 x 128, 108 us and 8 more in the
-// kernel that adds them in three slices of 256 x 256; at 1,024 tokens 77 us as one, 53 us in three slices of 128 x 256).
+// In which tiles the slices run is left to the shapes' times.
 
 static int cut_tiled_slices(int M, int N, int K) {
     const long NB = (N + 15) / 16;
@@ -1541,18 +1539,6 @@ static int plan_tiled_slices(int M, int N, int K) {
 extern "C" int agave_gemm_tiled_slices(int M, int N, int K) {
     if (M <= 64 || N <= 0 || K <= 0 || K % 8 != 0) return 1;
     return plan_tiled_slices(M, N, K);
-}
-
-// The same for a caller that has the choice: 1 where one 32-bit slice, the whole product, is the faster way (each slice,
-// written here and read by whoever adds them up, costs a microsecond per million elements).
-extern "C" int agave_gemm_tiled_slices_worth(int M, int N, int K) {
-    const int z = agave_gemm_tiled_slices(M, N, K);
-    if (z == 1) return 1;
-    const long NB = ((long)N + 15) / 16;
-    auto cost = [&](int slices) {
-        return tile_time(best_tile(M, NB, K, slices, true), M, NB, K, slices, true) + 0.96e-6 * slices * (double)M * N;
-    };
-    return cost(z) < cost(1) ? z : 1;
 }
 
 // The slices of a product in tiles of a given shape.

@@ -17,7 +17,6 @@ kernels.register_signatures("gemm_mfma", {
     "agave_gemm_row_normed_ok": [_I, _I, _I, _I],
     "agave_gemm_row_normed": [_P, _P, _P, _I, _I, _L, _P, _F, _P, _F, _P, _P, _I, _I, _I, _F, _F, _F, _F, _P, _P, _P],
     "agave_gemm_tiled_slices": [_I, _I, _I],
-    "agave_gemm_tiled_slices_worth": [_I, _I, _I],
     "agave_gemm_tiled_in_slices": [_P, _L, _P, _P, _I, _I, _I, _I, _P],
     "agave_gemm_tiled": [_P, _L, _P, _I, _P, _L, _I, _I, _I, _I, _F, _F, _F, _F, _P, _P, _P, _L, _P],
     "agave_gemm_tiled_as": [_P, _L, _P, _I, _P, _L, _I, _I, _I, _I, _F, _F, _F, _F, _P, _P, _I, _P],
@@ -188,24 +187,12 @@ def tiled_slices_for(m: int, n_out: int, k: int) -> int:
     return got
 
 
-def tiled_slices_worth(m: int, n_out: int, k: int) -> int:
-    """:func:`tiled_slices_for`, but 1 where that says more and one float32 slice, the whole product, is faster all the same."""
-    key = ("worth", m, n_out, k)
-    got = _slices.get(key)
-    if got is None:
-        got = tiled_slices_for(m, n_out, k)
-        if got > 1:
-            got = int(kernels.lib("gemm_mfma").agave_gemm_tiled_slices_worth(m, n_out, k))
-        _slices[key] = got
-    return got
-
-
 TILED_SLICES_MAX_BYTES = 512 << 20       # what the slices of one product may take
 
 
 def tiled_slices(x: torch.Tensor, packed: torch.Tensor, out: torch.Tensor, n_out: int) -> None:
     """out[s] = the sums over the s-th run of columns of x[M, K] @ W^T for M > 64; out is float32
-    [tiled_slices_for(M, n_out, K), M, n_out] and its slices add up to the product, or [1, M, n_out] and the product itself."""
+    [tiled_slices_for(M, n_out, K), M, n_out] and its slices add up to the product."""
     if not (x.is_cuda and packed.is_cuda and out.is_cuda):
         raise RuntimeError("agave_amd kernels run on the GPU only; got a CPU tensor")
     if not _x_ok(x):
@@ -215,9 +202,6 @@ def tiled_slices(x: torch.Tensor, packed: torch.Tensor, out: torch.Tensor, n_out
         raise ValueError(f"partial sums must be a contiguous float32 [slices, {m}, {n_out}] tensor")
     if packed.numel() != ((n_out + 15) // 16) * ((k + 31) // 32) * 512:
         raise ValueError("packed product: the packed weight does not fit these sizes")
-    if out.shape[0] == 1:
-        _launch("agave_gemm_tiled", x, packed, out[0], n_out, 0, NO_FORM)
-        return
     library.call(kernels.lib("gemm_mfma"), "agave_gemm_tiled_in_slices", x.data_ptr(), x.stride(0), packed.data_ptr(),
                  out.data_ptr(), m, n_out, k, out.shape[0], kernels.stream())
 

@@ -88,8 +88,6 @@ class Linear:
             many = n > gemm_mfma.SKINNY_MAX_M
             slices = (gemm_mfma.tiled_slices_for if many else gemm_mfma.slices_for)(n, self.out_features, self.in_features)
             if slices > 1 and gemm_mfma._x_ok(x):
-                if many:            # (perhaps one slice: the reader gets 32-bit sums in either case)
-                    slices = gemm_mfma.tiled_slices_worth(n, self.out_features, self.in_features)
                 out = self.env.workspace.get3((tag or self.name) + "_slices", slices, n, self.out_features, torch.float32)
                 library.profile.label = self.name
                 (gemm_mfma.tiled_slices if many else gemm_mfma.skinny_slices)(x, self.packed, out, self.out_features)

@@ -1401,12 +1401,6 @@ def test_gemm_tiles_of_64_tokens_in_slices(G, m, n, k):
     assert float((out.double().sum(0) - ref).abs().max()) <= 2e-5 * float(ref.abs().max()) * math.sqrt(k / 64)
 
 
-@pytest.mark.parametrize("m,n,k", [(2048, 2560, 10240), (1024, 2560, 10240), (300, 2560, 2048), (2048, 2560, 2048)])
-def test_gemm_tiled_slices_are_taken_where_they_pay(G, m, n, k):
-    assert G.tiled_slices_worth(m, n, k) in (1, G.tiled_slices_for(m, n, k))
-    assert G.tiled_slices_worth(2048, 2560, 10240) == 1 and G.tiled_slices_worth(1024, 2560, 10240) == 3
-
-
 @pytest.mark.parametrize("m,ff,k", [(70, 192, 64), (513, 1000, 96), (256, 20, 40), (1024, 5120, 1000), (2048, 10236, 64),
                                     (1024, 10236, 64)])
 def test_gemm_tiled_geglu(G, m, ff, k):
