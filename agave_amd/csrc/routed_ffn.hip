@@ -12,6 +12,8 @@
 //   A third way (mode 2): s = sigmoid(z), each output on its own; choice and groups as with the softmax over all.
 //   `group_top` 2: a group's score is the sum of its two largest c instead of its largest.  `normalise`: the chosen
 //   outputs' weights are divided by their sum + 1e-20 before the factor.
+//   A shared expert, which every token runs through, may be one more expert of the products: the choice then ends every token's
+//   pairs with it, weighted by the sigmoid of its gate's logit.
 //   The router matrix may carry further rows behind its R outputs (`extra`): their products with the token are handed
 //   out as they are (the logit of a gate on the shared expert), so that they cost no kernel of their own.
 //
@@ -135,7 +137,8 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
                                                           const float* __restrict__ correction, int N, int K, int R, int groups,
                                                           int keep, int top, float scale, int* __restrict__ choice,
                                                           float* __restrict__ weight, int mode, int extra,
-                                                          float* __restrict__ extra_out, int group_top, int normalise) {
+                                                          float* __restrict__ extra_out, int group_top, int normalise, int stride,
+                                                          int shared_at) {
     extern __shared__ float zs[];                      // [RR][R + extra], then the corrections [R]
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int Rt = R + extra;
@@ -248,13 +251,41 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < rows * extra; i += blockDim.x)
+    for (int i = threadIdx.x; extra_out && i < rows * extra; i += blockDim.x)
         extra_out[(size_t)(t0 + i / extra) * extra + i % extra] = zs[(i / extra) * Rt + R + i % extra];
     // the choice: a wave per token, the lanes along the outputs
     const int gs = R / groups;
     for (int i = w; i < rows; i += nw) {
         float* sr = zs + (size_t)i * Rt;
         const int t = t0 + i;
+        if (shared_at >= 0 && lane == 0) {          // the shared expert: every token's last pair, weighted by its gate
+            choice[(size_t)t * stride + top] = shared_at;
+            weight[(size_t)t * stride + top] = extra ? 1.0f / (1.0f + expf(-sr[R])) : 1.0f;
+        }
+        if (mode == 1 && R <= 64) {
+            // An output a lane, its place among all counted at once (the loop below is `top` chains of two maxima over the lanes: 6
+            // tokens of 2,048 by 17 outputs, 4 chosen, 7.5 us with it and 6.7 so, under the profiler).  Logits that are not finite keep that loop's order.
+            const float z = lane < R ? sr[lane] + corr[lane] : 0.f;
+            if (!__any(!(fabsf(z) < INFINITY))) {
+                int place = 0;
+                for (int f = 0; f < R; ++f) {
+                    const float zf = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(z), f));
+                    place += (zf > z || (zf == z && f < lane)) ? 1 : 0;
+                }
+                const bool chosen = lane < R && place < top;
+                __builtin_amdgcn_wave_barrier();
+                if (chosen) sr[place] = z;
+                __builtin_amdgcn_wave_barrier();
+                const float first_v = sr[0];
+                float sum = 0.f;
+                for (int r = 0; r < top; ++r) sum += expf(sr[r] - first_v);
+                if (chosen) {
+                    choice[(size_t)t * stride + place] = lane;
+                    weight[(size_t)t * stride + place] = expf(z - first_v) / sum * scale;
+                }
+                continue;
+            }
+        }
         if (mode == 1) {
             // the largest logits (bias added) are chosen, the lower index among equals; a chosen place is marked by
             // -infinity; lane r keeps round r's logit, and the weights are the softmax over those (top <= 64)
@@ -286,8 +317,8 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
                 __builtin_amdgcn_wave_barrier();
             }
             if (lane < top) {
-                choice[(size_t)t * top + lane] = my_choice;
-                weight[(size_t)t * top + lane] = expf(my_logit - first_v) / sum * scale;
+                choice[(size_t)t * stride + lane] = my_choice;
+                weight[(size_t)t * stride + lane] = expf(my_logit - first_v) / sum * scale;
             }
             continue;
         }
@@ -363,8 +394,8 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
             if ((r & 63) == 63 || r == top - 1) {
                 const int at = (r & ~63) + lane;
                 if (at <= r) {
-                    choice[(size_t)t * top + at] = my_choice;
-                    weight[(size_t)t * top + at] = normalise ? my_weight / (chosen_sum + 1e-20f) : my_weight;      // (normalise: top <= 64, one batch)
+                    choice[(size_t)t * stride + at] = my_choice;
+                    weight[(size_t)t * stride + at] = normalise ? my_weight / (chosen_sum + 1e-20f) : my_weight;      // (normalise: top <= 64, one batch)
                 }
             }
         }
@@ -373,10 +404,11 @@ __global__ __launch_bounds__(1024) void route_rows_kernel(const T* __restrict__ 
 
 extern "C" int agave_route_rows(int dtype, const void* x, long ldx, const float* router, const float* correction, int N, int K,
                                 int R, int groups, int keep, int top, float scale, int* choice, float* weight, int mode,
-                                int extra, float* extra_out, int group_top, int normalise, hipStream_t stream) {
+                                int extra, float* extra_out, int group_top, int normalise, int stride, int shared_at, hipStream_t stream) {
+    AGAVE_CHECK(stride >= top + (shared_at >= 0 ? 1 : 0) && (shared_at < 0 || extra <= 1), "route_rows: rows of %d pairs do not hold %d chosen and the shared expert, which has one gate at most", stride, top);
     AGAVE_CHECK(mode == 0 || mode == 2 || (mode == 1 && top <= 64 && groups == 1), "route_rows: the softmax over the chosen logits takes at most 64 of them and no groups");
     AGAVE_CHECK((group_top == 1 || group_top == 2) && (!normalise || (top <= 64 && mode != 1)), "route_rows: a group counts by its largest or its two largest; weights are divided by their sum for at most 64 chosen");
-    AGAVE_CHECK(extra >= 0 && extra <= 64 && (extra == 0 || extra_out), "route_rows: %d further rows of the router (0 to 64, with a place for their products)", extra);
+    AGAVE_CHECK(extra >= 0 && extra <= 64 && (extra == 0 || extra_out || shared_at >= 0), "route_rows: %d further rows of the router (0 to 64, with a place for their products)", extra);
     AGAVE_CHECK(N >= 0 && K > 0 && R > 0 && R <= ROUTE_MAX, "route_rows: %d router outputs (1 to %d)", R, ROUTE_MAX);
     AGAVE_CHECK(groups > 0 && groups <= 64 && R % groups == 0, "route_rows: %d outputs in %d groups (equal groups, at most 64)", R, groups);
     AGAVE_CHECK(keep > 0 && keep <= groups, "route_rows: %d of %d groups kept", keep, groups);
@@ -395,7 +427,7 @@ extern "C" int agave_route_rows(int dtype, const void* x, long ldx, const float*
     if (wide && K % 32 == 0 && N > 2048 && outputs_all > 8 && tiles <= 3) {
         const size_t lds_tiles = ((size_t)17 * 16 * outputs_all + R) * sizeof(float);
 #define ROUTE_TILES(T_, TILES_) route_rows_kernel<T_, true, 16, 1, TILES_><<<(N + 15) / 16, 1024, lds_tiles, stream>>>((const T_*)x, ldx, router, correction, \
-        N, K, R, groups, keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise)
+        N, K, R, groups, keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise, stride, shared_at)
         if (f32) { if (tiles == 1) ROUTE_TILES(float, 1); else if (tiles == 2) ROUTE_TILES(float, 2); else ROUTE_TILES(float, 3); }
         else if (tiles == 1) ROUTE_TILES(bf16, 1); else if (tiles == 2) ROUTE_TILES(bf16, 2); else ROUTE_TILES(bf16, 3);
 #undef ROUTE_TILES
@@ -414,7 +446,7 @@ extern "C" int agave_route_rows(int dtype, const void* x, long ldx, const float*
     const int waves = threads / 64, outputs = R + extra, last = outputs % (2 * waves);
     const bool two = outputs > waves && (rows == 8 || (N > 2 ? last == 0 || last <= waves / 2 || last > waves : last > waves && last <= waves * 3 / 2));
 #define ROUTE_GO(T_, W_, RR_, OUT_) route_rows_kernel<T_, W_, RR_, OUT_, 0><<<blocks, threads, lds, stream>>>((const T_*)x, ldx, router, correction, N, K, R, groups, \
-        keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise)
+        keep, top, scale, choice, weight, mode, extra, extra_out, group_top, normalise, stride, shared_at)
 #define ROUTE_ROWS(T_, W_) do { if (rows == 1 && two) ROUTE_GO(T_, W_, 1, 2); else if (rows == 1) ROUTE_GO(T_, W_, 1, 1); \
         else if (two) ROUTE_GO(T_, W_, 8, 2); else ROUTE_GO(T_, W_, 8, 1); } while (0)
     if (f32 && wide) ROUTE_ROWS(float, true); else if (f32) ROUTE_ROWS(float, false); else if (wide) ROUTE_ROWS(bf16, true); else ROUTE_ROWS(bf16, false);
@@ -975,10 +1007,12 @@ static bool launch_routed_few(const void* x, long ldx, const int* sorted_pair, c
                               const void* w1, void* out, int top, int live, int n_out, int K, int act, float p0, float p1, hipStream_t stream) {
     if (!agave_routed_few_takes(K)) return false;
     const int all = (n_out + (GATED ? 15 : 31)) / (GATED ? 16 : 32);
-    // Blocks a workgroup: the fewest with which all workgroups run at once, two to a compute unit at most (some 450 where 512
-    // have a place: `live` is an expectation).  Both products, 4 rows: 75.8, 63.0, 66.7 us with 2, 4, 5 blocks of the gate;
-    // 6 rows 78.8, 68.3, 70.7; 16 rows 93.5, 93.0, 89.1; 1 row 32.5 and 42.3 with 2 and 4.
-    int blocks = (int)(((long)live * all + 447) / 448);
+    // Blocks a workgroup: the fewest with which all workgroups of the experts that are expected, and of one more, run at once, two to
+    // a compute unit.  Both products, 4 rows: 75.8, 63.0, 66.7 us with 2, 4, 5 blocks of the gate; 6 rows 78.8, 68.3,
+    // 70.7; 16 rows 93.5, 93.0, 89.1; 1 row 32.5 and 42.3 with 2 and 4.  (Sixteen experts and a shared one, 6 rows: 5
+    // and 3 blocks of gate and down 78.3, 4 and 2 73.5.)
+    const int places = 512 / live > 0 ? 512 / live : 1;
+    int blocks = (all + places - 1) / places;
     blocks = blocks < 1 ? 1 : blocks > 16 ? 16 : blocks;
     const dim3 grid(max_tiles, (all + blocks - 1) / blocks);
     if (grid.y > 65535) return false;
@@ -1207,8 +1241,9 @@ extern "C" int agave_routed_experts_mfma(const void* x, long ldx, const int* sor
         routed_product_mfma_kernel<4, 4, false><<<g2, 256, 0, stream>>>((const bf16*)act_rows, ff, sorted_pair, tile_expert, (const bf16*)wd,
                                                                      nullptr, y, top, hidden, ff, act, wpacked, p0, p1);
     } else {
-        // experts that have rows, if the rows choose evenly
-        const int live = top >= E ? E : (int)ceil(E * (1.0 - pow(1.0 - (double)top / E, (double)n_rows)));
+        // experts that have rows, if the rows choose evenly, and one more
+        const int even = top >= E ? E : (int)ceil(E * (1.0 - pow(1.0 - (double)top / E, (double)n_rows)));
+        const int live = even < E ? even + 1 : E;
         const bool few1 = wpacked && launch_routed_few<true>(x, ldx, sorted_pair, tile_expert, max_tiles, wg, wu, act_rows, top, live, ff, hidden, act, p0, p1, stream);
         if (!few1)
             routed_product_mfma_kernel<1, 1, true><<<g1, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const bf16*)wg,

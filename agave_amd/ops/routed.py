@@ -14,7 +14,7 @@ MAX_OUTPUTS = 1024
 kernels.register_signatures(LIBRARY, {
     "agave_route_topk": [_P, _L, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P, _P],
     "agave_routed_experts_plain": [_I, _P, _L, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P],
-    "agave_route_rows": [_I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _P, _I, _I, _P],
+    "agave_route_rows": [_I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _P, _I, _I, _I, _I, _P],
     "agave_routed_few_takes": [_I],
     "agave_route_sort": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     "agave_routed_experts_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
@@ -173,7 +173,7 @@ def experts_mfma(x: torch.Tensor, sorted_pair: torch.Tensor, tile_expert: torch.
 def route_rows(x: torch.Tensor, router: torch.Tensor, correction: Optional[torch.Tensor], groups: int, keep: int, top: int,
                scale: float, choice: torch.Tensor, weight: torch.Tensor, softmax_top: bool = False,
                extra_out: Optional[torch.Tensor] = None, sigmoid: bool = False, group_top: int = 1,
-               normalise: bool = False) -> None:
+               normalise: bool = False, shared_expert: Optional[int] = None, shared_gate: bool = False) -> None:
     """The router's 32-bit product ``x router^T`` and :func:`route_topk`'s choice in one kernel (the logits never
     leave the compute unit).  ``router`` is float32 [R, width]; ``x`` [N, width] in either element type.
     ``softmax_top``: the ``top`` largest logits + ``correction`` are chosen (the lower index among equals) and their
@@ -181,7 +181,9 @@ def route_rows(x: torch.Tensor, router: torch.Tensor, correction: Optional[torch
     (float32 [N, extra]): the router matrix has ``extra`` further rows behind its outputs, whose products with
     the rows are left there as they are.  ``sigmoid``: the scores are the logits' sigmoids instead of their softmax.
     ``group_top`` 2: a group counts by the sum of its two largest scores + correction.  ``normalise``: the chosen
-    weights are divided by their sum + 1e-20 before ``scale`` (``top`` <= 64)."""
+    weights are divided by their sum + 1e-20 before ``scale`` (``top`` <= 64).  ``shared_expert``: ``choice`` and ``weight`` are
+    [N, top + 1], and every token's last pair is this expert with the weight 1 or, with ``shared_gate``, the sigmoid of
+    the product with one further row of the router matrix."""
     _dev(x, router, correction, choice, weight, extra_out)
     n, k = x.shape
     ldx = _rows(x, "x")
@@ -192,6 +194,11 @@ def route_rows(x: torch.Tensor, router: torch.Tensor, correction: Optional[torch
         if extra_out.dtype != torch.float32 or extra_out.dim() != 2 or extra_out.shape[0] != n or not extra_out.is_contiguous():
             raise ValueError(f"route_rows: extra_out must be contiguous float32 [{n}, extra]")
         extra = extra_out.shape[1]
+    if shared_gate:
+        if shared_expert is None or extra:
+            raise ValueError("route_rows: a gate is a shared expert's, and then the only further row")
+        extra = 1
+    pairs = top + (shared_expert is not None)
     r = router.shape[0] - extra
     if r < 1:
         raise ValueError("route_rows: the router has no outputs")
@@ -203,12 +210,12 @@ def route_rows(x: torch.Tensor, router: torch.Tensor, correction: Optional[torch
         raise ValueError("route_rows: a group counts by its largest or its two largest scores; weights are divided by their "
                          "sum for at most 64 chosen")
     _f32vec(correction, "correction", r)
-    _i32(choice, "choice", n * top)
-    if weight.dtype != torch.float32 or not weight.is_contiguous() or weight.numel() < n * top:
-        raise ValueError("route_rows: weight must be contiguous float32 [N, top]")
+    _i32(choice, "choice", n * pairs)
+    if weight.dtype != torch.float32 or not weight.is_contiguous() or weight.numel() < n * pairs:
+        raise ValueError("route_rows: weight must be contiguous float32, a value per pair")
     library.call(_lib(), "agave_route_rows", dt(x), ptr(x), ldx, ptr(router), ptr(correction), n, k, r, groups, keep, top,
                  float(scale), ptr(choice), ptr(weight), 1 if softmax_top else (2 if sigmoid else 0), extra, ptr(extra_out),
-                 int(group_top), 1 if normalise else 0, stream())
+                 int(group_top), 1 if normalise else 0, pairs, -1 if shared_expert is None else int(shared_expert), stream())
 
 
 def pack_expert_weights(w: torch.Tensor) -> torch.Tensor:

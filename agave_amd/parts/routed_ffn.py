@@ -7,7 +7,8 @@ outputs of the best groups, the weights are the plain scores times a factor (see
 weighted by the softmax over the chosen alone.  Outputs past the experts with weights are identity experts:
 their result is the input row.  The chosen experts' rows are summed with their weights, the shared
 expert's row is added, times the sigmoid of a logit per token where it has a gate (the gate's vector rides along
-as one more row of the router matrix, so its product costs no kernel).
+as one more row of the router matrix, so its product costs no kernel).  A shared expert of the experts' own form is one of
+the experts to the products.
 
 Nothing on the host depends on the choice: every launch has the same shape whatever the tokens are, so a
 decode step is recorded into a graph like any other.
@@ -61,10 +62,22 @@ class RoutedFfn:
         if s.shared_gate:
             rows.append(weights.get(s.shared_gate).to(torch.float32).view(1, s.hidden))
         self.router = torch.cat(rows, 0).contiguous().to(dev)
+        # A shared expert of the experts' own form is one more of them (the last), and every token's last pair: two products and
+        # their starts and ends less, and 32-bit rows.  Its matrices are then held with theirs and nowhere else.
+        names = (s.shared.gate_proj, s.shared.up_proj, s.shared.down_proj) if s.shared is not None else ()
+        self.shared_as_expert = bool(
+            s.shared is not None and s.n_experts and not s.n_identity and env.dtype == torch.bfloat16
+            and s.hidden % 32 == 0 and s.intermediate % 32 == 0
+            and (s.shared.hidden, s.shared.intermediate, s.shared.activation) == (s.hidden, s.intermediate, s.activation)
+            and (s.shared.act_limit, s.shared.act_alpha) == (s.act_limit, s.act_alpha)
+            and not (s.shared.gate_bias or s.shared.up_bias or s.shared.down_bias)
+            and all(env.weight_dtype(weights.get(name).dtype) == torch.bfloat16 for name in names))
         self.correction = weights.get(s.correction).to(torch.float32).contiguous().to(dev) if s.correction else None
 
         def stack(which: str) -> torch.Tensor:
             mats = [weights.get(f"{s.expert_prefix}{i}.{which}") for i in range(s.n_experts)]
+            if self.shared_as_expert:
+                mats.append(weights.get(dict(zip((s.gate_name, s.up_name, s.down_name), names))[which]))
             return torch.stack([m.to(env.dtype) for m in mats]).contiguous().to(dev)     # [experts, out, in]
         # bfloat16 experts whose sizes are multiples of 32 are kept in the matrix cores' tile order (only that copy)
         self.tile_order = bool(s.n_experts) and env.dtype == torch.bfloat16 and s.hidden % 32 == 0 and s.intermediate % 32 == 0
@@ -74,7 +87,7 @@ class RoutedFfn:
                 self.w_gate, self.w_up, self.w_down = (routed.pack_expert_weights(w) for w in (self.w_gate, self.w_up, self.w_down))
         else:
             self.w_gate = self.w_up = self.w_down = None
-        self.shared = GatedFfn(s.shared, weights, env) if s.shared is not None else None
+        self.shared = GatedFfn(s.shared, weights, env) if s.shared is not None and not self.shared_as_expert else None
 
     @staticmethod
     def tensor_needs(spec: RoutedFfnSpec) -> List[TensorNeed]:
@@ -97,26 +110,29 @@ class RoutedFfn:
     def forward(self, x: torch.Tensor, step) -> torch.Tensor:
         s, ws = self.spec, self.env.workspace
         n, r, top = x.shape[0], self.n_outputs, s.top
-        choice = ws.get("router_choice", n, top, torch.int32)
-        weight = ws.get("router_weight", n, top, torch.float32)
+        merged = self.shared_as_expert
+        experts, pairs = s.n_experts + merged, top + merged
+        choice = ws.get("router_choice", n, pairs, torch.int32)
+        weight = ws.get("router_weight", n, pairs, torch.float32)
         # the router's 32-bit product and the choice in one kernel
-        shared_gate = ws.get("router_shared_gate", n, 1, torch.float32) if s.shared_gate else None
+        shared_gate = ws.get("router_shared_gate", n, 1, torch.float32) if s.shared_gate and not merged else None
         routed.route_rows(x, self.router, self.correction, s.groups, s.keep_groups, top, s.route_scale, choice, weight,
                           softmax_top=s.score == "softmax_top", extra_out=shared_gate, sigmoid=s.score == "sigmoid",
-                          group_top=s.group_top, normalise=s.normalise)
+                          group_top=s.group_top, normalise=s.normalise, shared_expert=s.n_experts if merged else None,
+                          shared_gate=bool(merged and s.shared_gate))
         y = place = None
         if self.tile_order and not routed.mfma_ok(x, s.intermediate):
             raise ValueError("routed feed-forward: its experts are kept in tile order, which takes aligned bfloat16 rows")
         if s.n_experts and self.w_gate.dtype == torch.bfloat16 and routed.mfma_ok(x, s.intermediate):
             # the pairs sorted by expert on the device, then the experts' products tile by tile on the matrix cores
-            tm, tiles, cap = routed.tile_plan(n * top, s.n_experts, self.tile_order, s.intermediate, s.hidden)
-            place = ws.get("expert_place", n * top, 1, torch.int32).view(-1)
+            tm, tiles, cap = routed.tile_plan(n * pairs, experts, self.tile_order, s.intermediate, s.hidden)
+            place = ws.get("expert_place", n * pairs, 1, torch.int32).view(-1)
             sorted_pair = ws.get(f"expert_sorted{tm}", cap, 1, torch.int32).view(-1)
             tile_expert = ws.get(f"expert_tiles{tm}", tiles, 1, torch.int32).view(-1)
-            routed.route_sort(choice.view(-1), s.n_experts, tm, tiles, place, sorted_pair, tile_expert)
+            routed.route_sort(choice.view(-1), experts, tm, tiles, place, sorted_pair, tile_expert)
             act_rows = ws.get("expert_act", cap, s.intermediate, x.dtype)
             y = ws.get("expert_rows", cap, s.hidden, torch.float32)
-            routed.experts_mfma(x, sorted_pair, tile_expert, self.w_gate, self.w_up, self.w_down, act_rows, y, tm, tiles, top,
+            routed.experts_mfma(x, sorted_pair, tile_expert, self.w_gate, self.w_up, self.w_down, act_rows, y, tm, tiles, pairs,
                                 self.act, tile_order=self.tile_order, p0=s.act_limit, p1=s.act_alpha)
         elif s.n_experts:
             act_rows = ws.get("expert_act", n * top, s.intermediate, x.dtype)
@@ -125,7 +141,7 @@ class RoutedFfn:
                                  s.act_limit, s.act_alpha)
         shared = self.shared.forward(x, step, slices_ok=False, tag="shared_ffn") if self.shared is not None else None
         out = ws.get("routed_out", n, s.hidden, x.dtype)
-        routed.combine(y, place, choice.view(-1), weight.view(-1), x, shared, out, top, s.n_experts,
+        routed.combine(y, place, choice.view(-1), weight.view(-1), x, shared, out, pairs, experts,
                        shared_gate.view(-1) if shared_gate is not None else None)
         return out
 

@@ -426,3 +426,73 @@ def test_block_part(dtype, kind):
     check(h, r, dtype, f"{kind} residual stream")
     check(out, P.rms_norm(r, final_gain, 1e-5), dtype, f"{kind} norm after the block")
     assert h.dtype == torch.float32
+
+
+@pytest.mark.parametrize("gate", [True, False])
+@pytest.mark.parametrize("score", ["softmax_top", "softmax_all"])
+def test_routed_ffn_whose_shared_expert_is_one_of_the_experts(score, gate):
+    """A shared expert of the experts' form runs as the last of them: in the kernel of few pairs, in tiles of 16, 64 and 128
+    rows, with its gate and without; one whose limit is another stays a feed-forward of its own."""
+    from agave_amd.config.spec import GatedFfnSpec, RoutedFfnSpec
+    from agave_amd.parts import RoutedFfn
+    E, top, hidden, ff = 6, 2, 1024, 1024
+    names = ("gate_proj", "up_proj", "down_proj")
+    t = {f"e{i}.{w}": rnd((hidden, ff), 90 + i, 0.03) for i in range(E) for w in ("gate", "up", "down")}
+    t.update({n: rnd((hidden, ff), 80 + k, 0.03) for k, n in enumerate(names)})
+    t.update({"r": rnd((E, hidden), 70, 0.05), "rb": rnd((E,), 71, 0.3), "sg": rnd((1, hidden), 72, 0.05)})
+    t = {k: v.to(torch.bfloat16).double() for k, v in t.items()}
+    for limit in (3.0, 2.0):
+        shared = GatedFfnSpec(kind="gated_dense", hidden=hidden, intermediate=ff, activation="swish_clamped", act_limit=limit, act_alpha=1.5,
+                              gate_proj=names[0], up_proj=names[1], down_proj=names[2])
+        spec = RoutedFfnSpec(kind="routed", hidden=hidden, intermediate=ff, n_experts=E, top=top, activation="swish_clamped", act_limit=3.0,
+                             act_alpha=1.5, router="r", correction="rb", expert_prefix="e", shared=shared, score=score,
+                             shared_gate="sg" if gate else "")
+        needs = RoutedFfn.tensor_needs(spec)
+        b = Bench("bfloat16")
+        part = RoutedFfn(spec, weights_of({n.name: t[n.name] for n in needs}, needs, "bfloat16"), b.env)
+        assert part.shared_as_expert == (limit == 3.0) and (part.shared is None) == (limit == 3.0)
+
+        def expert(x, g, u, d, lim):
+            a, c = torch.clamp((x @ g.T).bfloat16().double(), max=lim), torch.clamp((x @ u.T).bfloat16().double(), -lim, lim)
+            return (a * torch.sigmoid(1.5 * a) * (c + 1)).bfloat16().double() @ d.T
+        for n in (1, 6, 40, 130, 700):
+            x = rnd((n, hidden), n, 1.0).bfloat16().double()
+            z = x @ t["r"].T
+            s = z + t["rb"] if score == "softmax_top" else torch.softmax(z, -1)
+            order = (s if score == "softmax_top" else s + t["rb"]).topk(top, -1).indices
+            w = torch.zeros(n, E, dtype=torch.float64)
+            chosen = s.gather(1, order)
+            w.scatter_(1, order, torch.softmax(chosen, -1) if score == "softmax_top" else chosen)
+            ref = sum(w[:, i:i + 1] * expert(x, t[f"e{i}.gate"], t[f"e{i}.up"], t[f"e{i}.down"], 3.0) for i in range(E))
+            one = expert(x, *(t[k] for k in names), limit)
+            ref = ref + (torch.sigmoid(x @ t["sg"].T) * one if gate else one)
+            check(part.forward(x.bfloat16().to(DEV), None), ref, "bfloat16", f"limit {limit}, {n} rows")
+
+
+@pytest.mark.parametrize("R, top", [(3, 3), (16, 4), (64, 64), (65, 4)])
+def test_choice_among_logits_with_equals_and_without_a_number(R, top):
+    """The largest logits are chosen, the lower index among equals, whether all outputs' places are counted at once (64 outputs) or one
+    maximum is taken after another, as where a logit is minus infinity (never chosen before the others)."""
+    from agave_amd.ops import routed
+    g = torch.Generator().manual_seed(R)
+    n = 40
+    x = torch.randn(n, 64, generator=g).to(DEV)
+    router = torch.randn(R, 64, generator=g).to(DEV)
+    router[1::2] = router[:R // 2]                                      # (equals: the same row twice)
+    bias = torch.zeros(R, device=DEV)
+    for lowest in (0.0, -float("inf")) if top < R else (0.0,):
+        bias[R - 1] = lowest
+        choice, weight = torch.empty(n, top + 1, dtype=torch.int32, device=DEV), torch.empty(n, top + 1, device=DEV)
+        routed.route_rows(x, router, bias, 1, 1, top, 1.0, choice, weight, softmax_top=True, shared_expert=R)
+        # (the kernel's own logits: every output's product, handed out)
+        z = torch.empty(n, R, device=DEV)
+        routed.route_rows(x, torch.cat([torch.ones(1, 64, device=DEV), router]), None, 1, 1, 1, 1.0, choice.new_empty(n, 1), weight.new_empty(n, 1),
+                          softmax_top=True, extra_out=z) if R <= 64 else z.copy_(x @ router.T)
+        z = (z + bias).double()
+        order = torch.sort(z, dim=-1, descending=True, stable=True).indices[:, :top]
+        if R <= 64:
+            assert torch.equal(choice[:, :top].long(), order)
+        got = z.gather(1, choice[:, :top].long())
+        assert bool(((got - z.gather(1, order)).abs().nan_to_num(0.0) <= 1e-4).all())
+        assert bool((choice[:, top] == R).all()) and bool((weight[:, top] == 1.0).all())
+        assert torch.allclose(weight[:, :top].double(), torch.softmax(got, -1), rtol=1e-4, atol=1e-6)
