@@ -8,6 +8,7 @@
 // (position scaled before the angle), src/backend/kernels/cpu/activation.zig:69-113 (tanh GELU).
 #include "common_impl.h"
 #include "qk_rope.h"
+#include "trig.h"
 
 // ------------------------------------------------------------------ embedding
 template <typename T>
@@ -715,6 +716,178 @@ __global__ void qk_norm_rope_kv_kernel(const T* q, long ldq, const T* __restrict
     }
 }
 
+// The same for steps of many tokens over pages in tile order: a wave takes four tokens and up to four of their query heads, four of
+// their key heads, or E runs of 128 of their value elements; sixteen lanes take a head of a token.
+//
+// What bounded the kernel above there: a wave a head is four elements a lane between a wave's sum, a root and a division, sincosf once
+// a head (12 times the same angles at 4B sizes), and stores of single elements to places 16 bytes apart.  Here a lane holds E
+// neighbours of the row's lower half and the E they rotate with (head sizes 128 and 256, all of a head rotated or nothing), so a row
+// comes and leaves in two pieces of 2 E bytes, which is how key tiles are made up, and angles are worked out once for four heads.
+// All of a wave's rows are asked for at its start.  Values: four aligned positions lie side by side in a value tile, so the group's
+// first token stores all four where the step holds them (the next three rows, of the same sequence); a position outside of a whole
+// group is stored alone.
+// Bound by its chain of loads up to some 700 tokens and by memory beyond.  us, above and here, 8 query and 4 key heads of 256, rows from
+// memory: 150 tokens 4.1 and 4.5, 256 4.8 and 4.6, 509 7.2 and 4.9, 2,048 17.5 and 10.0, 8,192 62.3 and 35.9 (134 MB, 3.7 TB/s).
+template <int E> struct QkPiece { uint32_t u[E / 2]; };
+template <int E>
+__global__ __launch_bounds__(256) void qk_norm_rope_kv_tokens_kernel(const bf16* q, long ldq, const bf16* __restrict__ k, long ldk,
+                                                                     const bf16* __restrict__ v, long ldv, bf16* q_out, long ldqo,
+                                                                     const float* __restrict__ q_gain, const float* __restrict__ k_gain,
+                                                                     float eps_q, float eps_k, const float* __restrict__ inv_freq,
+                                                                     float pos_scale, const int* __restrict__ tok_seq,
+                                                                     const int* __restrict__ tok_pos, bf16* __restrict__ k_pages,
+                                                                     bf16* __restrict__ v_pages, const int* __restrict__ table, int width,
+                                                                     const int* __restrict__ base, int n_pages, int N, int nh, int nkv) {
+    constexpr int HD = 32 * E, HALF = HD / 2, KS_N = HD / 32;
+    constexpr int HW = 4;                                   // heads of a wave
+    typedef QkPiece<E> Piece;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int m = lane & 15;                                // this lane's pieces: elements E m .. and HALF + E m ..
+    const int q_roles = (nh + HW - 1) / HW, k_roles = (nkv + HW - 1) / HW, roles = q_roles + 2 * k_roles;
+    // Workgroups go to the 8 XCDs in turn: each XCD takes a run of neighbouring tokens, whose pieces share the pages' cache lines
+    const int unit = ((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) * 4 + wave;
+    const int t0 = unit / roles * 4, role = unit % roles;
+    if (t0 >= N) return;
+    const bool active = t0 + (lane >> 4) < N;               // (lanes past the end go through the last token and store nothing)
+    const int t = active ? t0 + (lane >> 4) : N - 1;
+    const int p = tok_pos[t], b = nkv > 0 ? tok_seq[t] : 0;
+
+    if (role < q_roles + k_roles) {
+        const bool is_q = role < q_roles;
+        const int head0 = (is_q ? role : role - q_roles) * HW, heads = is_q ? nh : nkv;
+        const bf16* src = is_q ? q + (size_t)t * ldq : k + (size_t)t * ldk;
+        const float* gain = is_q ? q_gain : k_gain;
+        Piece lo[HW], hi[HW];
+#pragma unroll
+        for (int h = 0; h < HW; ++h) {                      // (past the last head: the last one again)
+            const bf16* at = src + (size_t)(head0 + h < heads ? head0 + h : heads - 1) * HD + E * m;
+            lo[h] = *reinterpret_cast<const Piece*>(at);
+            hi[h] = *reinterpret_cast<const Piece*>(at + HALF);
+        }
+        const bool rotated = inv_freq != nullptr;
+        float4 g4[E / 2], f4[E / 4];
+        if (gain) {
+#pragma unroll
+            for (int i = 0; i < E / 2; ++i) g4[i] = *reinterpret_cast<const float4*>(gain + E * m + (i < E / 4 ? 4 * i : HALF + 4 * i - E));
+        }
+        if (rotated) {
+#pragma unroll
+            for (int i = 0; i < E / 4; ++i) f4[i] = *reinterpret_cast<const float4*>(inv_freq + E * m + 4 * i);
+        }
+        int pg = -1;
+        if (!is_q) {
+            const int col = p / AGAVE_PAGE - base[b];
+            if (col >= 0 && col < width) pg = table[(size_t)b * width + col];
+            if (pg >= n_pages) pg = -1;                     // (a table the host built wrongly: nothing is written)
+        }
+        float sn[E], cs[E];
+        if (rotated) {
+#pragma unroll
+            for (int i = 0; i < E; ++i) {
+                const float f = i % 4 == 0 ? f4[i / 4].x : i % 4 == 1 ? f4[i / 4].y : i % 4 == 2 ? f4[i / 4].z : f4[i / 4].w;
+                sincos_of_angle((double)((float)p * pos_scale * f), sn[i], cs[i]);
+            }
+        }
+        const int row = p % AGAVE_PAGE;
+        // the lower piece's place in a page's block of keys; the upper one's is HALF / 32 tiles further
+        const size_t k_at = ((size_t)((row >> 4) * KS_N + E * m / 32) * 64 + (row & 15) + 16 * ((E * m & 31) >> 3)) * 8 + (E * m & 7);
+#pragma unroll
+        for (int h = 0; h < HW; ++h) {
+            float x[2 * E];
+#pragma unroll
+            for (int i = 0; i < E / 2; ++i) {
+                x[2 * i] = __builtin_bit_cast(float, lo[h].u[i] << 16);
+                x[2 * i + 1] = __builtin_bit_cast(float, lo[h].u[i] & 0xffff0000u);
+                x[E + 2 * i] = __builtin_bit_cast(float, hi[h].u[i] << 16);
+                x[E + 2 * i + 1] = __builtin_bit_cast(float, hi[h].u[i] & 0xffff0000u);
+            }
+            if (gain) {
+                float ss = 0.f;
+#pragma unroll
+                for (int i = 0; i < 2 * E; ++i) ss += x[i] * x[i];
+                ss += dpp_get<0xB1, 0xF>(0.f, ss);          // the sum of the head's sixteen lanes (see wave_sum)
+                ss += dpp_get<0x4E, 0xF>(0.f, ss);
+                ss += dpp_get<0x141, 0xF>(0.f, ss);
+                ss += dpp_get<0x140, 0xF>(0.f, ss);
+                const float inv = 1.0f / sqrtf(ss / (float)HD + (is_q ? eps_q : eps_k));
+#pragma unroll
+                for (int i = 0; i < E / 2; ++i) {
+                    x[4 * i] = x[4 * i] * inv * g4[i].x;
+                    x[4 * i + 1] = x[4 * i + 1] * inv * g4[i].y;
+                    x[4 * i + 2] = x[4 * i + 2] * inv * g4[i].z;
+                    x[4 * i + 3] = x[4 * i + 3] * inv * g4[i].w;
+                }
+            }
+            if (rotated) {
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    const float a = x[i], b2 = x[i + E];
+                    x[i] = a * cs[i] - b2 * sn[i];
+                    x[i + E] = a * sn[i] + b2 * cs[i];
+                }
+            }
+            Piece out_lo, out_hi;
+#pragma unroll
+            for (int i = 0; i < E / 2; ++i) {
+                out_lo.u[i] = f32x2_to_bf16x2(x[2 * i], x[2 * i + 1]);
+                out_hi.u[i] = f32x2_to_bf16x2(x[E + 2 * i], x[E + 2 * i + 1]);
+            }
+            if (head0 + h >= heads || !active) continue;
+            if (is_q) {
+                bf16* dst = q_out + (size_t)t * ldqo + (size_t)(head0 + h) * HD + E * m;
+                *reinterpret_cast<Piece*>(dst) = out_lo;
+                *reinterpret_cast<Piece*>(dst + HALF) = out_hi;
+            } else if (pg >= 0) {
+                bf16* dst = k_pages + ((size_t)pg * nkv + head0 + h) * (size_t)(AGAVE_PAGE * HD) + k_at;
+                *reinterpret_cast<Piece*>(dst) = out_lo;
+                *reinterpret_cast<Piece*>(dst + (HALF / 32) * 512) = out_hi;
+            }
+        }
+        return;
+    }
+
+    // values, 128 elements of the four tokens at a time
+    const int run0 = (role - q_roles - k_roles) * E, runs = nkv * HD / 128;
+    const int near_row = t0 - 3 + lane, near_in = near_row < 0 ? 0 : (near_row < N ? near_row : N - 1);
+    const int near_pos = tok_pos[near_in], near_seq = tok_seq[near_in];         // rows t0 - 3 .. t0 + 6 (and more, unused)
+    const int col = p / AGAVE_PAGE - base[b];
+    int pg = col >= 0 && col < width ? table[(size_t)b * width + col] : -1;
+    if (pg >= n_pages) pg = -1;
+    auto ahead = [&](int value, int o) { return __shfl(value, (lane + o) & 63); };
+    bool near_ok = near_row >= 0 && near_row + 3 < N && near_pos % 4 == 0;
+#pragma unroll
+    for (int o = 1; o < 4; ++o) near_ok = (ahead(near_pos, o) == near_pos + o) & (ahead(near_seq, o) == near_seq) & near_ok;
+    const unsigned near_leads = (unsigned)__ballot(near_ok) & 0x7f;             // bit i: row t0 - 3 + i leads a whole group of four
+    const unsigned leads = near_leads >> 3, led = (near_leads << 1 | near_leads << 2 | near_leads << 3) >> 3;
+    for (int j = 0; j < 4 && t0 + j < N; ++j) {
+        const bool leading = (leads >> j) & 1;
+        if (!leading && ((led >> j) & 1)) continue;         // the group's first token stores it
+        const int page = __builtin_amdgcn_readlane(pg, 16 * j), rj = __builtin_amdgcn_readlane(p, 16 * j) % AGAVE_PAGE, r32 = rj & 31;
+        if (page < 0) continue;
+        const int in_page = ((rj >> 5) * 64 + 16 * ((r32 & 15) >> 2)) * 8 + (r32 & 3) + ((r32 >> 4) << 2);
+        uint32_t two[E][4];
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const bf16* src = v + (size_t)(t0 + j) * ldv + (run0 + i < runs ? run0 + i : runs - 1) * 128 + lane * 2;
+#pragma unroll
+            for (int o = 0; o < 4; ++o) two[i][o] = *reinterpret_cast<const uint32_t*>(src + (leading ? o : 0) * ldv);
+        }
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            if (run0 + i >= runs) continue;
+            const int at = (run0 + i) * 128 + lane * 2, head = at / HD, d = at % HD;            // this lane's two elements: d, d + 1 of a head
+            bf16* dst = v_pages + ((size_t)page * nkv + head) * (size_t)(HD * AGAVE_PAGE) + ((size_t)(d >> 4) * 128 + (d & 15)) * 8 + in_page;
+            if (leading) {
+                *reinterpret_cast<uint2*>(dst) = make_uint2((two[i][0] & 0xffffu) | (two[i][1] << 16), (two[i][2] & 0xffffu) | (two[i][3] << 16));
+                *reinterpret_cast<uint2*>(dst + 8) = make_uint2((two[i][0] >> 16) | (two[i][1] & 0xffff0000u), (two[i][2] >> 16) | (two[i][3] & 0xffff0000u));
+            } else {
+                dst[0].x = (uint16_t)two[i][0];
+                dst[8].x = (uint16_t)(two[i][0] >> 16);
+            }
+        }
+    }
+}
+
 template <typename T>
 static void launch_qk_norm_rope_kv(int blocks, hipStream_t stream, const void* q, long ldq, const void* k, long ldk,
                                    const void* v, long ldv, void* q_out, long ldqo, const float* q_gain,
@@ -753,6 +926,24 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
     const long units = (long)N * (nh + nkv);
     if (units == 0) return 0;
     AGAVE_CHECK(units < (1L << 31) - 4, "qk_norm_rope_kv: %ld (token, head) pairs exceed what one launch takes", units);
+    // The line lies where both took the same time (256 tokens of 12 heads); below it a wave a head is the shorter chain.
+    const uintptr_t addresses = (nh ? (uintptr_t)q | (uintptr_t)q_out : 0) | (nkv ? (uintptr_t)k | (uintptr_t)v | (uintptr_t)k_pages | (uintptr_t)v_pages : 0) |
+                                (uintptr_t)q_gain | (uintptr_t)k_gain | (uintptr_t)(rot_half ? inv_freq : nullptr);
+    const long strides = (nh ? ldq | ldqo : 0) | (nkv ? ldk | ldv : 0);
+    if (dtype == AGAVE_BF16 && (packed || nkv == 0) && (hd == 128 || hd == 256) && (rot_half == 0 || rot_half == hd / 2) &&
+        units >= 3072 && addresses % 16 == 0 && strides % 8 == 0) {
+        const long waves = (long)((N + 3) / 4) * ((nh + 3) / 4 + 2 * ((nkv + 3) / 4));
+        const int grid = (int)(8 * (((waves + 3) / 4 + 7) / 8));
+#define QK_TOKENS(E_)                                                                                                           \
+    qk_norm_rope_kv_tokens_kernel<E_><<<grid, 256, 0, stream>>>(                                                                \
+        (const bf16*)q, ldq, (const bf16*)k, ldk, (const bf16*)v, ldv, (bf16*)q_out, ldqo, q_gain, k_gain, eps_q, eps_k,          \
+        rot_half ? inv_freq : nullptr, pos_scale, tok_seq, tok_pos, (bf16*)k_pages, (bf16*)v_pages, table, width, base, n_pages, N, nh, nkv)
+        if (hd == 128) QK_TOKENS(4);
+        else QK_TOKENS(8);
+#undef QK_TOKENS
+        AGAVE_LAUNCH_CHECK("qk_norm_rope_kv");
+        return 0;
+    }
     const int blocks = (int)((units + 3) / 4);
     if (dtype == AGAVE_F32)
         launch_qk_norm_rope_kv<float>(blocks, stream, q, ldq, k, ldk, v, ldv, q_out, ldqo, q_gain, k_gain, eps_q, eps_k,

@@ -178,6 +178,60 @@ def test_qk_norm_rope_kv(K, dtype):
     assert float(kp.cpu().float().abs().sum(dim=(1, 3))[mask].sum()) == 0.0
 
 
+@pytest.mark.parametrize("hd,nh,nkv,seqs,gains,rotates", [
+    (256, 8, 4, [(0, 256)], True, True),                             # whole groups of four positions only
+    (256, 8, 4, [(3, 130), (61, 71), (126, 66)], True, True),        # groups that begin and end inside of a wave's four tokens
+    (256, 5, 3, [(62, 3), (1, 381)], False, True),
+    (128, 16, 4, [(5, 1), (2, 2), (63, 190)], True, True),
+    (128, 6, 1, [(1, 439)], True, False),
+    (128, 16, 0, [(7, 193)], True, True),                            # a layer that reads another one's cache
+])
+def test_qk_norm_rope_kv_of_many_tokens(K, hd, nh, nkv, seqs, gains, rotates):
+    """Steps of many tokens over pages in tile order, which take a kernel of their own: against 64-bit rows (bfloat16 rounds to
+    2^-9 of a value; a rotated pair's two 32-bit products are far below that), values as they are, other rows untouched."""
+    g = torch.Generator().manual_seed(hd + nh)
+    tok_seq = [b for b, (_, m) in enumerate(seqs) for _ in range(m)]
+    tok_pos = [p + i for p, m in seqs for i in range(m)]
+    n, width = len(tok_pos), max((p + m + 63) // 64 for p, m in seqs)
+    assert n * (nh + nkv) >= 3072
+    qkv = torch.randn(n, (nh + 2 * nkv) * hd, generator=g).bfloat16()
+    q, k, v = qkv[:, :nh * hd], qkv[:, nh * hd:(nh + nkv) * hd], qkv[:, (nh + nkv) * hd:]
+    qg, kg = ((torch.randn(hd, generator=g) * 0.1 + 1) for _ in range(2)) if gains else (None, None)
+    inv = torch.from_numpy(np.exp(-np.log(1e6) * 2.0 * np.arange(hd // 2) / hd).astype(np.float32)) if rotates else None
+    pages = len(seqs) * width
+    table = torch.randperm(pages, generator=g).to(torch.int32).view(len(seqs), width)
+    kp = torch.zeros(pages, max(nkv, 1), 64, hd, dtype=torch.bfloat16, device=DEV)
+    vp = torch.zeros(pages, max(nkv, 1), hd, 64, dtype=torch.bfloat16, device=DEV)
+    dev = lambda x: x.to(DEV) if x is not None else None
+    on = qkv.to(DEV)
+    q_out = torch.empty(n, nh * hd, dtype=torch.bfloat16, device=DEV)
+    keys = (on[:, nh * hd:(nh + nkv) * hd], on[:, (nh + nkv) * hd:]) if nkv else (None, None)
+    K.qk_norm_rope_kv(on[:, :nh * hd], *keys, q_out, dev(qg), dev(kg), 1e-6, 2e-6, dev(inv), 0.125, _i32(tok_seq), _i32(tok_pos),
+                      kp if nkv else None, vp if nkv else None, table.to(DEV), _i32([0] * len(seqs)), nh, nkv, hd, True)
+    pos = torch.tensor(tok_pos, dtype=torch.float64)
+
+    def want(x, gain, eps, heads):
+        x = x.double().reshape(n, heads, hd)
+        if gain is not None:
+            x = P.rms_norm(x, gain.double(), eps, add_one=False)
+        return P.apply_rope(x, P.rope_angles(pos, hd, 1e6, 8.0)) if rotates else x
+    # (the kernel's angles are 32-bit products: at position 500 they are off by up to 3e-5)
+    tol = dict(atol=2e-4, rtol=2 ** -8)
+    assert torch.allclose(q_out.cpu().double().view(n, nh, hd), want(q, qg, 1e-6, nh), **tol)
+    if not nkv:
+        return
+    # tile order, back to [page, kv head, 64, hd]: keys are tiles of 16 rows by 32 elements, values of 16 elements by 32 rows
+    k_rows = kp.cpu().view(pages, nkv, 4, hd // 32, 4, 16, 8).permute(0, 1, 2, 5, 3, 4, 6).reshape(pages, nkv, 64, hd)
+    v_rows = vp.cpu().view(pages, nkv, hd // 16, 2, 4, 16, 2, 4).permute(0, 1, 3, 6, 4, 7, 2, 5).reshape(pages, nkv, 64, hd)
+    page = torch.tensor([int(table[b, p // 64]) for b, p in zip(tok_seq, tok_pos)])
+    row = torch.tensor([p % 64 for p in tok_pos])
+    assert torch.allclose(k_rows[page, :, row].double(), want(k, kg, 2e-6, nkv), **tol)
+    assert torch.equal(v_rows[page, :, row], v.reshape(n, nkv, hd))
+    written = torch.zeros(pages, 64, dtype=torch.bool)
+    written[page, row] = True
+    assert float(k_rows.float().abs().sum((1, 3))[~written].sum()) == 0 == float(v_rows.float().abs().sum((1, 3))[~written].sum())
+
+
 @pytest.mark.parametrize("pos", [0, 1, 10, 100, 1000])
 def test_rope_golden(K, pos):
     # research/kernels/generate_golden.py:140-155: nh 4, hd 256, theta 1e4, no norm
