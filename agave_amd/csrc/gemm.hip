@@ -484,6 +484,158 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_f32_ring_kernel(const float
         }
 }
 
+// ---------------------------------------------------------------- more rows, on the bfloat16 instructions
+// A float is the sum of three bfloat16 values exactly (24 bits are three times 8: the nearest bfloat16, the nearest of what is left, and
+// the rest), so a product of floats is the sum of nine exact products of pieces.  The six large ones are made here on
+// v_mfma_f32_16x16x32_bf16, whose sums are 32-bit; the three left out are below 2^-24 of the product.  The large pieces' products have a
+// running sum of their own, the five corrections another.  That sum takes 32 products an instruction, the 32-bit
+// instruction two or four, and so rounds a sixteenth as often.
+// Bound by the multiply-adds and, where a stage's tiles are few, by their chain of loads, cuts and barriers.  us, the kernels above and
+// this one with its sums of slices: 777 rows by 10,752 x 2,048 324 and 229 (149 TFLOP/s; the 32-bit instructions reach 153 on the largest
+// products), by 2,048 x 5,376 170 and 108, by 2,048 x 2,048 73 and 52, by 3,072 x 2,048 121 and 77; 2,048 rows by 10,752 x 2,048 722 and
+// 443 (204 TFLOP/s); 64 rows 42 and 34, 59 and 25, 26 and 15, 26 and 18.  Root mean square of the error against 64 bits over that of
+// the result, in 1e-7: 2,048 columns 5.7 (rings) and 2.7 whole, 1.9 in two slices, 1.3 in four; 5,376 9.3 and 4.6, 3.2, 2.2.
+// A piece of an infinity or NaN is none of the two (and the largest floats round to an infinity): an element that comes out neither
+// finite is made again from the floats themselves.
+// WM x WN = 2 x 2 waves make BM rows x BN columns of C.  A stage of 32 k is brought into registers a stage ahead, cut into pieces there
+// and put into LDS in the order the instruction reads its operands; two workgroups share a compute unit, and one cuts while the other
+// multiplies.
+struct Pieces { uint32_t u[3]; };                                 // two floats' pieces, largest first, side by side
+__device__ __forceinline__ Pieces pieces_of(float a, float b) {
+    Pieces p;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        p.u[i] = f32x2_to_bf16x2(a, b);
+        a -= __builtin_bit_cast(float, p.u[i] << 16);
+        b -= __builtin_bit_cast(float, p.u[i] & 0xffff0000u);
+    }
+    return p;
+}
+template <int BM, int BN>
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const float* __restrict__ A, long lda, const float* __restrict__ W,
+                                                                long ldw, float* __restrict__ C, long ldc, int M, int N, int K,
+                                                                int m_tiles, int tiles, long part_stride) {
+    constexpr int ROWS = BM + BN, UNITS = ROWS / 64;              // 8 k of a row: a unit; so many of a stage a thread
+    constexpr int MT = BM / 32, NT = BN / 32;                     // tiles of 16 x 16 of a wave
+    constexpr int PLANE = ROWS * 64;                              // bytes of one piece of all rows
+    static_assert(BM % 64 == 0 && BN % 64 == 0, "a pass of the loads is of rows of A or of W");
+    __shared__ __attribute__((aligned(16))) unsigned char stage[3 * PLANE];
+    const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);      // (one below the other on an XCD, as above)
+    if (tile >= tiles) return;
+    const int m0 = tile % m_tiles * BM, n0 = tile / m_tiles * BN;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave & 1, wn = wave >> 1, j = lane & 15, g = lane >> 4;
+    // gridDim.y workgroups share a tile's k and leave their sums in slices of C
+    const int stages = (K + 31) / 32;
+    const int st0 = (int)((long)blockIdx.y * stages / gridDim.y), st_end = (int)((long)(blockIdx.y + 1) * stages / gridDim.y);
+    C += (size_t)blockIdx.y * part_stride;
+
+    const int ug = threadIdx.x & 3, ur = threadIdx.x >> 2;        // unit u: row ur + 64 u of the stage, k 8 ug .. + 8
+    const float* src[UNITS];
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {                             // (rows outside: the last one again, not stored)
+        const int row = ur + 64 * u;
+        src[u] = row < BM ? A + (size_t)min(m0 + row, M - 1) * lda : W + (size_t)min(n0 + row - BM, N - 1) * ldw;
+    }
+    f32x4_t raw[UNITS][2];
+    auto fetch = [&](int st) {
+        const int k = st * 32 + 8 * ug;                           // (K is a multiple of 4; past it the last four again, cleared below)
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) raw[u][i] = *reinterpret_cast<const f32x4_t*>(src[u] + min(k + 4 * i, K - 4));
+    };
+    // a unit's place: tile of 16 rows, lane row % 16 + 16 ug of the operand, moved so that a store's lanes take different banks
+    const unsigned put = (ur >> 4) * 1024 + ug * 256 + (((ur & 15) ^ (2 * ug)) * 16);
+    const unsigned get = g * 256 + ((j ^ (2 * g)) * 16);
+    f32x4_t high[MT][NT] = {}, low[MT][NT] = {};
+    if (st0 < st_end) fetch(st0);
+    for (int st = st0; st < st_end; ++st) {
+        uint4 cut[UNITS][3];
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            if (st * 32 + 32 > K) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    if (st * 32 + 8 * ug + 4 * i >= K) raw[u][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
+            const Pieces a = pieces_of(raw[u][0][0], raw[u][0][1]), b = pieces_of(raw[u][0][2], raw[u][0][3]);
+            const Pieces c = pieces_of(raw[u][1][0], raw[u][1][1]), d = pieces_of(raw[u][1][2], raw[u][1][3]);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) cut[u][p] = make_uint4(a.u[p], b.u[p], c.u[p], d.u[p]);
+        }
+        __builtin_amdgcn_s_barrier();                             // (every wave has its operands of the stage before this one)
+#pragma unroll
+        for (int u = 0; u < UNITS; ++u)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) *reinterpret_cast<uint4*>(stage + p * PLANE + u * 4096 + put) = cut[u][p];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        fetch(st + 1 < st_end ? st + 1 : st);                     // (the last stage's once more, not used)
+        __builtin_amdgcn_sched_barrier(0);                        // (or the compiler asks when it needs them)
+        frag16 w[NT][3];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                w[t][p].u = *reinterpret_cast<const uint4*>(stage + p * PLANE + (BM / 16 + wn * NT + t) * 1024 + get);
+#pragma unroll
+        for (int r = 0; r < MT; ++r) {
+            frag16 x[3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) x[p].u = *reinterpret_cast<const uint4*>(stage + p * PLANE + (wm * MT + r) * 1024 + get);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) high[r][t] = mfma_16x16x32(w[t][0], x[0], high[r][t]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) low[r][t] = mfma_16x16x32(w[t][2], x[0], low[r][t]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) low[r][t] = mfma_16x16x32(w[t][0], x[2], low[r][t]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) low[r][t] = mfma_16x16x32(w[t][1], x[1], low[r][t]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) low[r][t] = mfma_16x16x32(w[t][1], x[0], low[r][t]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) low[r][t] = mfma_16x16x32(w[t][0], x[1], low[r][t]);
+        }
+    }
+    // high[r][t][e]: row 16 r + j, column 16 t + 4 g + e of the wave's
+    const bool fours = ldc % 4 == 0 && ((uintptr_t)C & 15) == 0;
+#pragma unroll
+    for (int r = 0; r < MT; ++r) {
+        const int m = m0 + (wm * MT + r) * 16 + j;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int n = n0 + (wn * NT + t) * 16 + 4 * g;
+            f32x4_t s = high[r][t] + low[r][t];
+            if (m >= M || n >= N) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (!(__builtin_fabsf(s[e]) < __builtin_inff()) && n + e < N) {
+                    float again = 0.f;
+                    const float *pa = A + (size_t)m * lda, *pw = W + (size_t)(n + e) * ldw;
+                    for (int k = st0 * 32; k < min(st_end * 32, K); ++k) again = fmaf(pa[k], pw[k], again);
+                    s[e] = again;
+                }
+            float* dst = C + (size_t)m * ldc + n;
+            if (fours && n + 4 <= N) {
+                *reinterpret_cast<f32x4_t*>(dst) = s;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) dst[e] = s[e];
+            }
+        }
+    }
+}
+
+template <int BM, int BN>
+static void launch_split(const float* A, long lda, const float* W, long ldw, float* C, long ldc, int M, int N, int K, int slices, long part_stride,
+                         hipStream_t stream) {
+    const int m_tiles = (M + BM - 1) / BM, tiles = m_tiles * ((N + BN - 1) / BN);
+    gemm_f32_split_kernel<BM, BN><<<dim3((tiles + 7) / 8 * 8, slices), 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, m_tiles, tiles, part_stride);
+}
+
 // ---------------------------------------------------------------- launch
 #define SKINNY_M 64
 #define COMPUTE_UNITS 256
@@ -524,16 +676,76 @@ static void launch_ring(const float* A, long lda, const float* W, long ldw, floa
 // were alone), of 128 x 128, 130 us each.  The kernel of 32 x 64 tiles keeps products of one round of those (37.5 us), which halve the k
 // between waves.  Up to 64 rows stay in groups of 64 rows where these have eight running sums a product or more (under 8,192 columns), and
 // are added up as in groups with four.
+static const double RING_32[] = {0, 44, 72, 109, 146, 195};
 static int ring_rows(int M, int N) {
     auto a_unit = [&](int bm) { return (((long)M + bm - 1) / bm * (((long)N + 127) / 128) + COMPUTE_UNITS - 1) / COMPUTE_UNITS; };
-    static const double t32[] = {0, 44, 72, 109, 146, 195};
     if (M <= SKINNY_M) return N >= (M > 32 ? 8192 : 16384) ? 32 : 0;
     if ((long)((M + 31) / 32) * ((N + TN - 1) / TN) <= COMPUTE_UNITS) return 0;
     const long n32 = a_unit(32);
     // three tiles of 32 x 128 a unit, of which two run at a time, take 117 to 133, and three of 64 x 64 in the kernel above 118 (5,376 columns
     // 320 to 338 and 298; 1,500 rows by 2,048 x 2,048 132.8 and 118.3, 512 by 5,376 x 10,752 667 and 591)
     if (n32 == 3 && ((long)M + 63) / 64 * (((long)N + TN - 1) / TN) <= 3 * COMPUTE_UNITS) return 0;
-    return (n32 <= 5 ? t32[n32] : 35.0 * n32) <= 130.0 * a_unit(128) ? 32 : 128;
+    return (n32 <= 5 ? RING_32[n32] : 35.0 * n32) <= 130.0 * a_unit(128) ? 32 : 128;
+}
+
+// Microseconds of a product on a tile shape of gemm_f32_split_kernel, from the time of a stage of 32 k with so many tiles a compute unit
+// (2,048 columns, all operands from memory; two workgroups share a unit, up to four of the smaller tiles) and of a launch.
+struct SplitShape { int bm, bn; double start, stage[12]; };
+static const double SPLIT_TILES[12] = {0.25, 0.5, 1, 1.25, 1.5, 2, 2.5, 3, 4, 5, 6, 8};
+static const SplitShape SPLIT_SHAPES[4] = {
+    {128, 128, 8, {1.66, 1.71, 1.89, 2.32, 2.39, 2.63, 4.16, 4.25, 5.13, 7.15, 7.81, 10.52}},
+    {64, 128, 6, {1.16, 1.18, 1.22, 1.43, 1.44, 1.55, 2.23, 2.36, 3.27, 3.95, 4.75, 6.24}},
+    {128, 64, 6, {1.11, 1.10, 1.15, 1.35, 1.38, 1.50, 2.16, 2.32, 3.24, 3.74, 4.64, 6.02}},
+    {64, 64, 5, {0.76, 0.78, 0.81, 0.93, 0.96, 0.99, 1.39, 1.45, 1.75, 2.21, 2.88, 3.55}}};
+static double split_stage(const SplitShape& s, double tiles_a_unit) {
+    if (tiles_a_unit <= SPLIT_TILES[0]) return s.stage[0];
+    for (int i = 1; i < 12; ++i)
+        if (tiles_a_unit <= SPLIT_TILES[i])
+            return s.stage[i - 1] + (s.stage[i] - s.stage[i - 1]) * (tiles_a_unit - SPLIT_TILES[i - 1]) / (SPLIT_TILES[i] - SPLIT_TILES[i - 1]);
+    return s.stage[11] * tiles_a_unit / SPLIT_TILES[11];
+}
+struct SplitPlan { int shape, slices; double us; };
+// The fastest shape, with k shared out among up to max_slices workgroups where that pays for adding up the slices (4 bytes each of
+// them and the result at 3.5 TB/s, and a launch).
+static SplitPlan plan_split(int M, int N, int K, int max_slices) {
+    SplitPlan best = {0, 1, 1e30};
+    const int stages = (K + 31) / 32;
+    for (int i = 0; i < 4; ++i) {
+        const SplitShape& s = SPLIT_SHAPES[i];
+        const double tiles = (double)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+        for (int z = 1; z <= max_slices && (z == 1 || stages / z >= 8); z *= 2) {
+            double us = s.start + 0.95 * split_stage(s, tiles * z / COMPUTE_UNITS) * ((stages + z - 1) / z);
+            if (z > 1) us += 2.0 + (z + 1.0) * M * N * 4 / 3.5e6;
+            if (us < best.us) best = {i, z, us};
+        }
+    }
+    return best;
+}
+static void launch_split(const SplitPlan& plan, const float* A, long lda, const float* W, long ldw, float* C, long ldc, int M, int N, int K,
+                         long part_stride, hipStream_t stream) {
+    switch (plan.shape) {
+        case 0: return launch_split<128, 128>(A, lda, W, ldw, C, ldc, M, N, K, plan.slices, part_stride, stream);
+        case 1: return launch_split<64, 128>(A, lda, W, ldw, C, ldc, M, N, K, plan.slices, part_stride, stream);
+        case 2: return launch_split<128, 64>(A, lda, W, ldw, C, ldc, M, N, K, plan.slices, part_stride, stream);
+        default: return launch_split<64, 64>(A, lda, W, ldw, C, ldc, M, N, K, plan.slices, part_stride, stream);
+    }
+}
+// The plan of a product in pieces, us 0 where the 32-bit instructions take it.  The rings' times are known (see ring_rows): less than
+// theirs.  Where groups of rows or the tiles above would take it: only in slices, from 1,024 columns and 33 rows (or 4,096 and 17) on.  us, those and
+// slices: 17 rows by 3,072 x 2,048 14.1 and 15.3, 48 rows 23.8 and 17.0; 17 rows by 2,048 x 5,376 31.7 and 23.2; 400 rows by 2,048 x 2,048 42.7
+// and 37.1; 512 by 1,024 x 512 11.9 and 14.3.
+static SplitPlan split_instead(int M, int N, int K, int max_slices) {
+    SplitPlan plan = {0, 1, 0};
+    if (M <= 16 || (M <= 32 && K < 4096)) return plan;
+    const int rows = ring_rows(M, N);
+    plan = plan_split(M, N, K, max_slices);
+    if (rows != 0) {
+        const long n = (((long)M + rows - 1) / rows * (((long)N + 127) / 128) + COMPUTE_UNITS - 1) / COMPUTE_UNITS;
+        if (plan.us >= (rows == 128 ? 130.0 * n : n <= 5 ? RING_32[n] : 35.0 * n) * K / 2048) plan.us = 0;
+    } else if (K < 1024 || plan.slices == 1) {
+        plan.us = 0;
+    }
+    return plan;
 }
 
 template <typename TA, typename TW, typename TC, bool VEC>
@@ -551,6 +763,8 @@ static void launch_vec(const TA* A, long lda, const TW* W, long ldw, TC* C, long
     }
     if (M <= 16) return launch_skinny<TA, TW, TC, 1, VEC>(A, lda, W, ldw, C, ldc, M, N, K, stream);
     if constexpr (VEC && std::is_same<TA, float>::value && std::is_same<TW, float>::value && std::is_same<TC, float>::value) {
+        const SplitPlan plan = split_instead(M, N, K, 1);
+        if (plan.us > 0) return launch_split(plan, A, lda, W, ldw, C, ldc, M, N, K, 0, stream);
         const int rows = lda < (1L << 22) && ldw < (1L << 22) ? ring_rows(M, N) : 0;       // (offsets in a tile have 32 bits)
         if (rows == 32 && M <= SKINNY_M) return launch_ring<32, 128, 1, 4, 4, 4>(A, lda, W, ldw, C, ldc, M, N, K, stream);
         if (rows == 32) return launch_ring<32, 128, 1, 4, 2, 4>(A, lda, W, ldw, C, ldc, M, N, K, stream);
@@ -611,4 +825,66 @@ extern "C" int agave_gemm_plain(int dt_a, const void* A, long lda, int dt_w, con
     }
     AGAVE_LAUNCH_CHECK("gemm_plain");
     return 0;
+}
+
+// ---------------------------------------------------------------- in slices
+// out[i] = the sum of the slices' i-th elements, in their order
+__global__ __launch_bounds__(256) void gemm_f32_add_slices_kernel(const f32x4_t* __restrict__ parts, long n4, int slices, f32x4_t* __restrict__ out) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    f32x4_t s = parts[i];
+#pragma unroll 4
+    for (int z = 1; z < slices; ++z) s += parts[z * n4 + i];
+    out[i] = s;
+}
+
+// Slices in which agave_gemm_slices makes a product of aligned floats faster than agave_gemm_plain does (1: it does not).
+extern "C" int agave_gemm_slices_for(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % 4 != 0 || N % 4 != 0) return 1;
+    const SplitPlan plan = split_instead(M, N, K, 8);
+    return plan.us > 0 ? plan.slices : 1;
+}
+
+extern "C" int agave_add_slices(const float* parts, long n, int slices, float* out, hipStream_t stream) {
+    AGAVE_CHECK(n >= 0 && slices >= 1 && n / 1024 < (1L << 31) - 1, "add_slices: bad sizes n=%ld slices=%d", n, slices);
+    AGAVE_CHECK(n % 4 == 0 && (((uintptr_t)parts | (uintptr_t)out) & 15) == 0, "add_slices: aligned fours only (n=%ld)", n);
+    if (n == 0) return 0;
+    gemm_f32_add_slices_kernel<<<(unsigned)((n / 4 + 255) / 256), 256, 0, stream>>>((const f32x4_t*)parts, n / 4, slices, (f32x4_t*)out);
+    AGAVE_LAUNCH_CHECK("add_slices");
+    return 0;
+}
+
+// parts [slices, M, N] <- 32-bit slices that add up to A W^T
+extern "C" int agave_gemm_slices(const float* A, long lda, const float* W, long ldw, float* parts, int M, int N, int K, int slices,
+                                 hipStream_t stream) {
+    AGAVE_CHECK(M > 0 && N > 0 && K > 0 && lda >= K && ldw >= K, "gemm_slices: bad sizes M=%d N=%d K=%d", M, N, K);
+    AGAVE_CHECK(K % 4 == 0 && N % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)A | (uintptr_t)W | (uintptr_t)parts) & 15) == 0,
+                "gemm_slices: rows of aligned fours");
+    AGAVE_CHECK((long)((M + 63) / 64) * ((N + 63) / 64) < (1L << 30), "gemm_slices: M=%d x N=%d exceeds the grid limit", M, N);
+    AGAVE_CHECK(slices >= 1 && slices <= 8 && slices <= (K + 31) / 32, "gemm_slices: %d slices of %d columns", slices, K);
+    SplitPlan plan = plan_split(M, N, K, 1);
+    for (int z = 2; z <= slices; z *= 2) {                        // (the shape that goes with as many slices)
+        const SplitPlan more = plan_split(M, N, K, z);
+        if (more.slices == z) plan = more;
+    }
+    plan.slices = slices;
+    launch_split(plan, A, lda, W, ldw, parts, N, M, N, K, (long)M * N, stream);
+    AGAVE_LAUNCH_CHECK("gemm_slices");
+    return 0;
+}
+
+// A product in a tile shape and a number of slices that the caller names.
+extern "C" int agave_gemm_slices_as(const float* A, long lda, const float* W, long ldw, float* parts, int M, int N, int K, int bm, int bn, int slices,
+                                    hipStream_t stream) {
+    AGAVE_CHECK(M > 0 && N > 0 && K > 0 && lda >= K && ldw >= K, "gemm_slices_as: bad sizes M=%d N=%d K=%d", M, N, K);
+    AGAVE_CHECK(K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (((uintptr_t)A | (uintptr_t)W) & 15) == 0, "gemm_slices_as: rows of aligned fours");
+    AGAVE_CHECK((long)((M + 63) / 64) * ((N + 63) / 64) < (1L << 30), "gemm_slices_as: M=%d x N=%d exceeds the grid limit", M, N);
+    AGAVE_CHECK(slices >= 1 && slices <= 8 && slices <= (K + 31) / 32, "gemm_slices_as: %d slices of %d columns", slices, K);
+    for (int i = 0; i < 4; ++i)
+        if (SPLIT_SHAPES[i].bm == bm && SPLIT_SHAPES[i].bn == bn) {
+            launch_split({i, slices, 0}, A, lda, W, ldw, parts, N, M, N, K, (long)M * N, stream);
+            AGAVE_LAUNCH_CHECK("gemm_slices_as");
+            return 0;
+        }
+    AGAVE_CHECK(false, "gemm_slices_as: no tiles of %d x %d", bm, bn);
 }

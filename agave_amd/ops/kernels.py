@@ -36,6 +36,10 @@ _SIGNATURES = {
     },
     "gemm": {
         "agave_gemm_plain": [_I, _P, _L, _I, _P, _L, _I, _P, _L, _I, _I, _I, _P],
+        "agave_gemm_slices_for": [_I, _I, _I],
+        "agave_gemm_slices": [_P, _L, _P, _L, _P, _I, _I, _I, _I, _P],
+        "agave_add_slices": [_P, _L, _I, _P, _P],
+        "agave_gemm_slices_as": [_P, _L, _P, _L, _P, _I, _I, _I, _I, _I, _I, _P],
     },
     "attention_plain": {
         "agave_attn_plain": [_I, _P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _F, _I, _I, _I, _I, _I, _P, _P, _P],
@@ -422,6 +426,40 @@ def gemm_plain(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor) -> None:
         raise ValueError(f"gemm: shapes do not fit: a {tuple(a.shape)}, w {tuple(w.shape)}, c {tuple(c.shape)}")
     library.call(lib("gemm"), "agave_gemm_plain", dt(a), ptr(a), lda, dt(w), ptr(w), ldw, dt(c), ptr(c), ldc,
                  m, n, k, stream())
+
+
+def gemm_slices_for(a: torch.Tensor, w: torch.Tensor) -> int:
+    """In how many 32-bit slices ``a @ w^T`` is made faster than by :func:`gemm_plain` (1: it is not, or not of aligned floats)."""
+    if a.dtype != torch.float32 or w.dtype != torch.float32 or a.dim() != 2 or a.stride(1) != 1 or w.stride(1) != 1:
+        return 1
+    if a.stride(0) % 4 or w.stride(0) % 4 or (a.data_ptr() | w.data_ptr()) % 16:
+        return 1
+    return lib("gemm").agave_gemm_slices_for(a.shape[0], w.shape[0], a.shape[1])
+
+
+def gemm_slices(a: torch.Tensor, w: torch.Tensor, parts: torch.Tensor, tile: Optional[tuple] = None) -> None:
+    """``parts`` [slices, M, N] (float32) <- slices that add up to ``a @ w^T``.  ``tile``: rows and columns of the tiles, where
+    the caller names them."""
+    _dev(a, w, parts)
+    lda, ldw = _rows(a, "a"), _rows(w, "w")
+    (m, k), n, z = a.shape, w.shape[0], parts.shape[0]
+    if a.dtype != torch.float32 or w.dtype != torch.float32 or parts.dtype != torch.float32:
+        raise TypeError("gemm_slices: float32 tensors only")
+    if w.shape[1] != k or parts.shape != (z, m, n) or not parts.is_contiguous():
+        raise ValueError(f"gemm_slices: shapes do not fit: a {tuple(a.shape)}, w {tuple(w.shape)}, parts {tuple(parts.shape)}")
+    if tile is not None:
+        library.call(lib("gemm"), "agave_gemm_slices_as", ptr(a), lda, ptr(w), ldw, ptr(parts), m, n, k, tile[0], tile[1], z, stream())
+    else:
+        library.call(lib("gemm"), "agave_gemm_slices", ptr(a), lda, ptr(w), ldw, ptr(parts), m, n, k, z, stream())
+
+
+def add_slices(parts: torch.Tensor, out: torch.Tensor) -> None:
+    """``out`` [M, N] <- the sum of the slices ``parts`` [slices, M, N] (both float32)."""
+    _dev(parts, out)
+    if parts.dtype != torch.float32 or out.dtype != torch.float32 or parts.dim() != 3 or parts.shape[1:] != out.shape \
+            or not parts.is_contiguous() or not out.is_contiguous():
+        raise ValueError(f"add_slices: float32 [slices, rows, columns] and [rows, columns], got {tuple(parts.shape)} and {tuple(out.shape)}")
+    library.call(lib("gemm"), "agave_add_slices", ptr(parts), out.numel(), parts.shape[0], ptr(out), stream())
 
 
 def attn_plain(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,

@@ -95,12 +95,27 @@ class Linear:
                     kernels.add_bias(out[0], self.bias)
                 library.profile.label = None
                 return out
-        if out is None:
+        # a 32-bit product of more than a few rows may be shared out along its columns too; where the caller does not
+        # take its slices they are added up here
+        slices = kernels.gemm_slices_for(x, self.weight) if self.packed is None and n > 16 and out_dtype in (None, torch.float32) else 1
+        handed_on = slices > 1 and slices_ok and out is None
+        if not handed_on and out is None:
             out = self.env.workspace.get(tag or self.name, n, self.out_features, out_dtype or x.dtype)
         if self.interleave_ff:
             raise RuntimeError(f"{self.name}: a weight packed for a gated product only serves forward_gated")
         library.profile.label = self.name
-        gemm.linear(x, self, out)
+        if slices > 1 and (handed_on or (out.dtype == torch.float32 and out.is_contiguous() and out.data_ptr() % 16 == 0)):
+            name = (tag or self.name) + "_slices" if handed_on else "product_slices"
+            parts = self.env.workspace.get3(name, slices, n, self.out_features, torch.float32)
+            kernels.gemm_slices(x, self.weight, parts)
+            if handed_on:
+                if self.bias is not None:
+                    kernels.add_bias(parts[0], self.bias)
+                library.profile.label = None
+                return parts
+            kernels.add_slices(parts, out)
+        else:
+            gemm.linear(x, self, out)
         if self.bias is not None:
             kernels.add_bias(out, self.bias)
         library.profile.label = None

@@ -20,6 +20,7 @@ import torch
 
 from ..cache import GroupKey, StateNeed
 from ..config.spec import ParallelMixerSpec
+from ..ops import kernels
 from ..ops import sequence as seq_ops
 from ..weights.loader import TensorNeed
 from .base import BuildEnv, lookup, mixer_libraries, register
@@ -95,6 +96,14 @@ class ParallelMixer:
             out.update(need)
         return out or None
 
+    def _whole(self, y: torch.Tensor, name: str) -> torch.Tensor:
+        """A branch's rows; those of a 32-bit engine may come as slices that add up to them."""
+        if y.dim() != 3 or self.env.dtype != torch.float32:
+            return y
+        out = self.env.workspace.get(name, y.shape[1], y.shape[2], torch.float32)
+        kernels.add_slices(y, out)
+        return out
+
     def forward(self, x: torch.Tensor, step, memory: int, writes: bool = True) -> torch.Tensor:
         ws, n = self.env.workspace, x.shape[0]
         if self.fused:
@@ -105,7 +114,8 @@ class ParallelMixer:
                 p.context_into(x, step, memory, writes, view, scale, proj=rows)
             return self.o.forward(ctx, tag="parallel_o", slices_ok=True)
         a = self.branches[0].forward(x, step, memory, writes)
-        b = self.branches[1].forward(x, step, memory, writes)
+        a = self._whole(a, "parallel_a")             # (before the other branch runs: its slices may lie in the same buffer)
+        b = self._whole(self.branches[1].forward(x, step, memory, writes), "parallel_b")
         if a.dim() != 2 or b.dim() != 2:
             raise ValueError("a branch of a parallel mixer returns plain rows [N, hidden], not slices that add up")
         out = ws.get("parallel_sum", n, a.shape[1], self.env.dtype)

@@ -1390,6 +1390,51 @@ def test_gemm_tiled_every_tile_shape_in_slices(G, tile, m, n, k, z):
     assert float((whole.double().cpu() - ref).abs().max()) <= 6e-3 * float(ref.abs().max())
 
 
+# 32-bit products in pieces on the bfloat16 instructions: every tile shape, its last rows and columns broken, stages of 32 columns
+# broken, one of them, as many as slices and more; rows that lie apart; values next to the largest float, which round to an infinity.
+@pytest.mark.parametrize("tile", [(128, 128), (64, 128), (128, 64), (64, 64)])
+@pytest.mark.parametrize("m,n", [(17, 5), (64, 64), (129, 65), (200, 258)])
+@pytest.mark.parametrize("k,z", [(4, 1), (36, 2), (64, 1), (260, 8), (1028, 4)])
+def test_gemm_slices(K, tile, m, n, k, z):
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    x = torch.randn(m, k + 8, device=DEV, generator=g)[:, 4:4 + k]
+    w = torch.randn(n, k + 4, device=DEV, generator=g)[:, :k]
+    for scale in (1.0, 2.0 ** -40, 2.0 ** 60):              # (pieces of 2^-40 and less are still whole numbers of the smallest float)
+        parts = torch.full((z, m, n), float("nan"), device=DEV)
+        K.gemm_slices(x * scale if scale != 1.0 else x, w, parts, tile)
+        ref, size = x.double() * scale @ w.double().T, (x.double() * scale).abs() @ w.double().abs().T
+        # a piece's rest is below 2^-23 of a product (three products of the nine are left out), an addition below 2^-24 of the sum
+        assert bool(((parts.double().sum(0) - ref).abs() <= (k + 2) * 2.0 ** -24 * size).all())
+    x[1, k - 1], x[m - 1, 0], w[2, 1], w[n - 1, k - 2] = float("nan"), float("inf"), float("-inf"), 3.4e38
+    x[3] *= 1e-3
+    parts = torch.full((z, m, n), float("nan"), device=DEV)
+    K.gemm_slices(x, w, parts, tile)
+    got, want = parts.double().sum(0), x.double() @ w.double().T
+    plain = torch.ones(m, n, dtype=torch.bool, device=DEV)
+    plain[[1, m - 1]], plain[:, [2, n - 1]] = False, False
+    assert bool(got[plain].isfinite().all()) and bool(got[1].isnan().all())
+    assert not bool(got[m - 1].isfinite().any()) and not bool(got[:, 2].isfinite().any())
+    assert abs(float(got[3, n - 1] / want[3, n - 1]) - 1) <= (k + 2) * 2.0 ** -24       # (the large product outweighs the others)
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 2048, 2048), (64, 10752, 2048), (100, 512, 2048), (200, 2048, 5376), (700, 3072, 2048), (17, 2304, 9216)])
+def test_gemm_in_slices_is_as_exact_as_whole(K, m, n, k):
+    """Where a product is made in slices its error against 64 bits is no larger than that of the kernels of the 32-bit instructions
+    (1.0 to 2.1e-7 of the result over these sizes, 2.9 to 5.7e-7 there)."""
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    x, w = torch.randn(m, k, device=DEV, generator=g), torch.randn(n, k, device=DEV, generator=g)
+    z = K.gemm_slices_for(x, w)
+    assert z > 1 and K.gemm_slices_for(x[:, 1:], w[:, 1:]) == 1 and K.gemm_slices_for(x.bfloat16(), w) == 1
+    parts, out, plain = torch.empty(z, m, n, device=DEV), torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+    K.gemm_slices(x, w, parts)
+    K.add_slices(parts, out)
+    K.gemm_plain(x, w, plain)
+    ref = x.double() @ w.double().T
+    of = lambda c: float((c.double() - ref).pow(2).mean().sqrt() / ref.pow(2).mean().sqrt())
+    print(m, n, k, "slices", z, "error", of(out), "whole", of(plain))
+    assert of(out) <= 1.1 * of(plain)
+
+
 # Between the rings of 32 and of 128 rows: three tiles of either kernel a compute unit, their last rows and columns broken.  Two running
 # sums an element as in the rings (some 5.7e-7 of the result at 2,048 columns, 8.1e-7 with one; the bound lies between).
 @pytest.mark.parametrize("m,n", [(1500, 2050), (510, 5372), (130, 16000), (1536, 2048)])
