@@ -612,6 +612,128 @@ extern "C" int agave_routed_combine(int dtype, const float* y, const int* place,
     return 0;
 }
 
+// ------------------------------------------------------------------ the pairs' sum, straight into the residual stream
+// b = sum over the token's pairs of weight * expert row + shared row (as routed_combine_kernel, no identity experts);
+// h[t] += post_gain ? rmsnorm(b) * post_gain : b;  out[t] = pre_gain ? rmsnorm(h[t]) * pre_gain : h[t].
+// A workgroup a token, its row in registers; everything is asked for before anything is used, the pairs' rows PB at a time.  As a
+// row of its own the sum cost a kernel, its write and its read.
+// Bound by memory with many tokens, by its round trips with few.  us, the two kernels and this one, 2,048 columns, 5 pairs a token: 6 tokens
+// 5.8 and 4.0, 300 9.6 and 6.0, 3,001 50.3 and 37.0 (185 MB); 4,096 columns of 2 pairs, 64 6.4 and 4.4, 2,000 44.3 and 27.8.
+template <typename T, int VPT, int PB>
+__global__ void routed_norm_kernel(float* __restrict__ h, const float* __restrict__ y, const int* __restrict__ place, const int* __restrict__ choice,
+                                   const float* __restrict__ weight, int top, int E, const T* __restrict__ shared, long lds,
+                                   const float* __restrict__ shared_gate, const float* __restrict__ post_gain, float post_eps, T* __restrict__ out,
+                                   long ldo, const float* __restrict__ pre_gain, float pre_eps, int e) {
+    __shared__ float red[2][16];
+    const int t = blockIdx.x;
+    float* hr = h + (size_t)t * e;
+    f32x4_t hv[VPT], g1[VPT], g2[VPT], b[VPT] = {}, yv[PB][VPT];
+    float sv[VPT][4];
+    int col[VPT];
+    bool in[VPT];
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) {
+        const int c = (threadIdx.x + v * blockDim.x) * 4;
+        in[v] = c < e;
+        col[v] = in[v] ? c : 0;                              // (a lane past the row's end reads its start and uses nothing of it)
+        hv[v] = *reinterpret_cast<const f32x4_t*>(hr + col[v]);
+        g1[v] = *reinterpret_cast<const f32x4_t*>((post_gain ? post_gain : hr) + col[v]);       // (a gain that is not there: the row, not used)
+        g2[v] = *reinterpret_cast<const f32x4_t*>((pre_gain ? pre_gain : hr) + col[v]);
+        if (shared) load_near<4>(shared + (size_t)t * lds + col[v], sv[v]);
+    }
+    for (int r0 = 0; r0 < top; r0 += PB) {
+        float w[PB];
+        bool live[PB];
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {                       // (a pair past the last: the last one again, not added)
+            const int p = t * top + min(r0 + u, top - 1), ex = choice[p];
+            live[u] = ex >= 0 && ex < E && r0 + u < top;
+            int row = place ? place[p] : p;
+            row = live[u] && row >= 0 ? row : 0;
+            w[u] = weight[p];
+#pragma unroll
+            for (int v = 0; v < VPT; ++v) yv[u][v] = *reinterpret_cast<const f32x4_t*>(y + (size_t)row * e + col[v]);
+        }
+#pragma unroll
+        for (int u = 0; u < PB; ++u)
+#pragma unroll
+            for (int v = 0; v < VPT; ++v)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) b[v][i] = live[u] ? fmaf(w[u], yv[u][v][i], b[v][i]) : b[v][i];
+    }
+    if (shared) {
+        const float sg = shared_gate ? 1.0f / (1.0f + expf(-shared_gate[t])) : 1.0f;
+#pragma unroll
+        for (int v = 0; v < VPT; ++v)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[v][i] = fmaf(sg, sv[v][i], b[v][i]);
+    }
+    // (rounded as the row that routed_combine leaves, so that a step's results do not depend on which of the two it takes)
+#pragma unroll
+    for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            T rounded;
+            st(&rounded, b[v][i]);
+            b[v][i] = ld(&rounded);
+        }
+    auto squares = [&](const f32x4_t& x) { return x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3]; };
+    if (post_gain) {
+        float ss = 0.f;
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) ss += in[v] ? squares(b[v]) : 0.f;
+        const float inv = 1.0f / sqrtf(block_sum(ss, red[0]) / (float)e + post_eps);
+#pragma unroll
+        for (int v = 0; v < VPT; ++v) b[v] = b[v] * inv * g1[v];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) {
+        hv[v] += b[v];
+        if (in[v]) {
+            *reinterpret_cast<f32x4_t*>(hr + col[v]) = hv[v];
+            ss += squares(hv[v]);
+        }
+    }
+    float inv = 1.0f;
+    if (pre_gain) inv = 1.0f / sqrtf(block_sum(ss, red[1]) / (float)e + pre_eps);
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) {
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = pre_gain ? hv[v][i] * inv * g2[v][i] : hv[v][i];
+        if (in[v]) store_near<4>(out + (size_t)t * ldo + col[v], o);
+    }
+}
+
+extern "C" int agave_routed_norm(int dtype, float* h, const float* y, const int* place, const int* choice, const float* weight, int top, int E,
+                                 const void* shared, long lds, const float* shared_gate, const float* post_gain, float post_eps, void* out, long ldo,
+                                 const float* pre_gain, float pre_eps, int N, int e, hipStream_t stream) {
+    AGAVE_CHECK(N >= 0 && top > 0 && E > 0 && e > 0 && e % 4 == 0 && e <= 16384, "routed_norm: bad sizes N=%d top=%d E=%d e=%d", N, top, E, e);
+    AGAVE_CHECK(h && y && choice && weight && out && ldo >= e && ldo % 4 == 0 && (!shared || (lds >= e && lds % 4 == 0)), "routed_norm: bad buffers");
+    AGAVE_CHECK((((uintptr_t)h | (uintptr_t)y | (uintptr_t)shared | (uintptr_t)post_gain | (uintptr_t)out | (uintptr_t)pre_gain) & 15) == 0,
+                "routed_norm: rows must be aligned to 16 bytes");
+    AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "routed_norm: unknown dtype %d", dtype);
+    if (N == 0) return 0;
+    // threads as residual_norm takes them: one float4 each in steps of few tokens, two (four) in steps of many
+    int threads;
+    if (e <= 1024 || (N <= 64 && e <= 4096)) threads = 64 * ((e / 4 + 63) / 64);
+    else {
+        const int per = e / 4 <= 2048 ? 2 : 4;
+        threads = 64 * ((e / 4 + per * 64 - 1) / (per * 64));
+    }
+    const int vpt = (e / 4 + threads - 1) / threads;
+#define NORM_GO(T_, V_, P_) routed_norm_kernel<T_, V_, P_><<<N, threads, 0, stream>>>(h, y, place, choice, weight, top, E, (const T_*)shared, lds, shared_gate, \
+        post_gain, post_eps, (T_*)out, ldo, pre_gain, pre_eps, e)
+#define NORM_T(T_) do { if (vpt <= 1) { if (top > 4) NORM_GO(T_, 1, 8); else NORM_GO(T_, 1, 4); } else if (vpt <= 2) { if (top > 4) NORM_GO(T_, 2, 5); else NORM_GO(T_, 2, 4); } \
+        else NORM_GO(T_, 4, 2); } while (0)
+    if (dtype == AGAVE_F32) NORM_T(float); else NORM_T(bf16);
+#undef NORM_T
+#undef NORM_GO
+    AGAVE_LAUNCH_CHECK("routed_norm");
+    return 0;
+}
+
 // ------------------------------------------------------------------ the pairs sorted by expert
 // One workgroup.  Every expert's pairs get a run of whole tiles of TM sorted rows (the last one padded):
 //   place[p]        sorted row of pair p (-1: the pair's choice is an identity expert)

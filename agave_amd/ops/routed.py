@@ -18,6 +18,7 @@ kernels.register_signatures(LIBRARY, {
     "agave_routed_few_takes": [_I],
     "agave_route_sort": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P],
     "agave_routed_experts_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
+    "agave_routed_norm": [_I, _P, _P, _P, _P, _P, _I, _I, _P, _L, _P, _P, _F, _P, _L, _P, _F, _I, _I, _P],
     "agave_routed_combine": [_I, _P, _P, _P, _P, _P, _L, _P, _L, _P, _P, _L, _I, _I, _I, _I, _P],
 })
 
@@ -90,6 +91,47 @@ def combine(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: to
     _i32(place, "place", n * top)
     library.call(_lib(), "agave_routed_combine", dt(x), ptr(y), ptr(place), ptr(choice), ptr(weight), ptr(x), ldx, ptr(shared),
                  lds, ptr(shared_gate) if shared is not None else None, ptr(out), ldo, n, top, n_experts, hidden, stream())
+
+
+class RoutedRows:
+    """A routed feed-forward's result that is still its pairs' rows: the arguments of :func:`combine`.  The norm that takes it
+    adds the pairs up itself (:meth:`norm_into`) where it can; whoever cannot asks for the rows (:meth:`rows`)."""
+
+    def __init__(self, y, place, choice, weight, x, shared, out, top, n_experts, shared_gate):
+        self.arguments = (y, place, choice, weight, x, shared, out, top, n_experts, shared_gate)
+        self._rows: Optional[torch.Tensor] = None
+
+    def rows(self) -> torch.Tensor:
+        if self._rows is None:
+            combine(*self.arguments)
+            self._rows = self.arguments[6]
+        return self._rows
+
+    def norm_into(self, h: torch.Tensor, post_gain: Optional[torch.Tensor], post_eps: float, out: torch.Tensor,
+                  pre_gain: Optional[torch.Tensor], pre_eps: float) -> bool:
+        """``h += post(rows)`` and ``out = rmsnorm(h) * pre_gain`` (or the rows of ``h`` without a gain) in one kernel, if it takes
+        these sizes and nothing was added up yet."""
+        y, place, choice, weight, x, shared, _, top, n_experts, shared_gate = self.arguments
+        n, e = h.shape
+        if self._rows is not None or e % 4 or e > 16384 or out.dtype != x.dtype or h.shape != x.shape:
+            return False
+        for t in (h, y, shared, post_gain, out, pre_gain):
+            if t is not None and (t.data_ptr() % 16 or (t.dim() == 2 and (t.stride(1) != 1 or t.stride(0) % 4))):
+                return False
+        if not h.is_contiguous() or h.dtype != torch.float32 or out.shape != x.shape:
+            return False
+        _dev(h, y, place, choice, weight, shared, shared_gate, post_gain, out, pre_gain)
+        _f32vec(post_gain, "post_gain", e)
+        _f32vec(pre_gain, "pre_gain", e)
+        _f32vec(shared_gate, "shared_gate", n)
+        if y.dtype != torch.float32 or not y.is_contiguous() or y.shape[1] != e or (place is None and y.shape[0] < n * top):
+            raise ValueError("routed rows: y must be float32 [>= N * top, hidden]")
+        _i32(choice, "choice", n * top)
+        _i32(place, "place", n * top)
+        library.call(_lib(), "agave_routed_norm", dt(out), ptr(h), ptr(y), ptr(place), ptr(choice), ptr(weight), top, n_experts, ptr(shared),
+                     _rows(shared, "shared") if shared is not None else 0, ptr(shared_gate) if shared is not None else None, ptr(post_gain),
+                     float(post_eps), ptr(out), out.stride(0), ptr(pre_gain), float(pre_eps), n, e, stream())
+        return True
 
 
 STREAMED = (1024, 2048, 4096)        # columns for which the kernel of few pairs is built (agave_routed_few_takes)

@@ -92,7 +92,7 @@ class SandwichBlock:
         if self.ffn is None:
             return pending
         self.pre_ffn.add_and_norm(h, pending, x)
-        f = self.ffn.forward(x, step)
+        f = getattr(self.ffn, "forward_pending", self.ffn.forward)(x, step)
         return (f, self.post_ffn)
 
     def _forward_few_rows(self, h: torch.Tensor, pending: Pending, step, memory: int, writes: bool) -> Pending:
@@ -153,7 +153,7 @@ class PostNormBlock(SandwichBlock):
         if self.ffn is None:
             return pending
         rows_as_they_are(h, pending, x)
-        return (self.ffn.forward(x, step), self.post_ffn)
+        return (getattr(self.ffn, "forward_pending", self.ffn.forward)(x, step), self.post_ffn)
 
 
 class PostNormSumBlock(PostNormBlock):

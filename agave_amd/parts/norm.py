@@ -20,11 +20,12 @@ from typing import List, Optional, Tuple
 import torch
 
 from ..config.spec import NormSpec
-from ..ops import kernels
+from ..ops import kernels, routed
 from ..weights.loader import TensorNeed
 from .base import BuildEnv, register
 
-# (branch, the norm after its sublayer | None[, base]).  ``base``: the tensor that holds the residual
+# (branch, the norm after its sublayer | None[, base]).  The branch may be a routed feed-forward's rows that are not added up
+# yet (agave_amd.ops.routed.RoutedRows): unpack_pending adds them up.  ``base``: the tensor that holds the residual
 # stream at this moment if that is not ``h`` (a product that made its own normalised rows summed the
 # stream up in other memory, see NormedRows); whoever adds the branch reads the rows there and
 # writes them to ``h``.
@@ -32,12 +33,22 @@ Pending = Optional[Tuple]
 
 
 def unpack_pending(pending: Pending):
-    """(branch, post norm, base), each None where there is none."""
+    """(branch, post norm, base), each None where there is none; a routed feed-forward's rows are added up for it."""
     if pending is None:
         return None, None, None
-    if len(pending) == 2:
-        return pending[0], pending[1], None
-    return pending
+    branch, post, base = pending if len(pending) == 3 else (*pending, None)
+    return branch.rows() if isinstance(branch, routed.RoutedRows) else branch, post, base
+
+
+def _routed_rows_into(h: torch.Tensor, pending: Pending, out: torch.Tensor, gain: Optional[torch.Tensor], eps: float) -> bool:
+    """h += post(branch), out = rms(h) * gain (``gain`` None: h as it is) where the branch is a routed feed-forward's rows that
+    are not added up yet and one kernel does all of it."""
+    if pending is None or len(pending) != 2 or not isinstance(pending[0], routed.RoutedRows):
+        return False
+    branch, post = pending
+    if post is not None and not isinstance(post, RmsNorm):
+        return False
+    return branch.norm_into(h, post.gain if post is not None else None, post.eps if post is not None else 0.0, out, gain, eps)
 
 
 def add_branch(h: torch.Tensor, pending: Pending) -> None:
@@ -113,6 +124,8 @@ def rows_as_they_are(h: torch.Tensor, pending: Pending, out: torch.Tensor, rows:
     """What stands where a norm would for a model without one: the pending branch is added and
     the (chosen) rows of ``h`` are handed on, rounded to ``out``'s element type.  One kernel where the
     branch's norm is an RMS norm (or none) and all rows are wanted, as with a norm in front."""
+    if rows is None and _routed_rows_into(h, pending, out, None, 0.0):
+        return
     branch, post, base = unpack_pending(pending)
     if isinstance(post, NormOfSum) and base is None and rows is None and (branch.dim() == 3 or branch.dtype == out.dtype):
         kernels.norm_of_sum(h, branch, post.alpha, post.bias, post.gain, post.eps, out)
@@ -173,6 +186,8 @@ class RmsNorm(Norm):
     def add_and_norm(self, h, pending, out, rows=None) -> None:
         """One kernel adds the branch (through the RMS norm after its sublayer, if it has one) and
         computes this norm, reading and writing ``h`` once."""
+        if rows is None and out is not None and _routed_rows_into(h, pending, out, self.gain, self.eps):
+            return
         branch, post, base = unpack_pending(pending)
         if isinstance(post, NormOfSum) and out is not None and rows is None and base is None \
                 and (branch.dim() == 3 or branch.dtype == out.dtype):

@@ -143,6 +143,12 @@ class RoutedFfn:
         return needs
 
     def forward(self, x: torch.Tensor, step) -> torch.Tensor:
+        y = self.forward_pending(x, step)
+        return y.rows() if isinstance(y, routed.RoutedRows) else y
+
+    def forward_pending(self, x: torch.Tensor, step):
+        """The result with its pairs' rows not added up yet (:class:`agave_amd.ops.routed.RoutedRows`), for a block whose next norm
+        may do that; plain rows where some of the experts are identity experts, whose result is ``x``."""
         s, ws = self.spec, self.env.workspace
         n, r, top = x.shape[0], self.n_outputs, s.top
         merged = self.shared_as_expert and (self.shared is None or merges(n, s.n_experts, top, s.intermediate, s.hidden))
@@ -176,9 +182,9 @@ class RoutedFfn:
                                  s.act_limit, s.act_alpha)
         shared = self.shared.forward(x, step, slices_ok=False, tag="shared_ffn") if self.shared is not None and not merged else None
         out = ws.get("routed_out", n, s.hidden, x.dtype)
-        routed.combine(y, place, choice.view(-1), weight.view(-1), x, shared, out, pairs, experts,
-                       shared_gate.view(-1) if shared_gate is not None else None)
-        return out
+        pending = routed.RoutedRows(y, place, choice.view(-1), weight.view(-1), x, shared, out, pairs, experts,
+                                    shared_gate.view(-1) if shared_gate is not None else None)
+        return pending.rows() if s.n_identity or y is None else pending
 
 
 register("ffn", "routed", RoutedFfn)

@@ -545,6 +545,54 @@ def test_routed_tiles_in_tile_order(n, E, top, ff, hidden, tm):
     assert torch.equal(out[0][:, :hidden], out[1][:, 1:hidden + 1])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,E,top,hidden", [(1, 3, 1, 4), (6, 17, 5, 2048), (65, 4, 4, 2052), (3, 9, 9, 4100), (130, 8, 2, 1024), (2, 6, 3, 12292)])
+@pytest.mark.parametrize("post,pre_norm,shared,gated,sorted_rows", [(False, True, False, False, True), (True, False, True, True, True),
+                                                                  (True, True, False, False, False), (False, False, True, False, True)])
+def test_routed_rows_into_the_norm(n, E, top, hidden, dtype, post, pre_norm, shared, gated, sorted_rows):
+    """The pairs' sum, the residual sum and the norm in one kernel, against 64 bits: one float4 a thread and several, pairs that
+    fill a batch of loads and do not, rows by pair and through places, a choice that is no expert.  A row's sums are of `top` + 2
+    products in 32 bits, rounded to the activations' type as a row of its own would be, and so is the result."""
+    from agave_amd.ops import routed
+    g = torch.Generator().manual_seed(n + hidden)
+    cap = n * top + 3
+    y = torch.randn(cap, hidden, generator=g)
+    place = torch.randperm(cap, generator=g)[:n * top].int() if sorted_rows else None
+    choice = torch.randint(0, E, (n * top,), generator=g, dtype=torch.int32)
+    if top > 1:
+        choice[top - 1] = -1
+    weight, gate = torch.rand(n * top, generator=g), torch.randn(n, generator=g)
+    x, sh = torch.randn(n, hidden, generator=g).to(dtype), torch.randn(n, hidden, generator=g).to(dtype)
+    h, gain, pre = torch.randn(n, hidden, generator=g), torch.rand(hidden, generator=g) + 0.5, torch.rand(hidden, generator=g) + 0.5
+    rows = y[place.long()] if sorted_rows else y[:n * top]
+    b = (rows.double() * (weight * (choice >= 0)).double()[:, None]).view(n, top, hidden).sum(1)
+    if shared:
+        b = b + sh.double() * (gate.double().sigmoid()[:, None] if gated else 1.0)
+    b = b.float().to(dtype).double()                # (an element next to the middle of two may come out as the other)
+    norm = lambda v, w, eps: v / (v.pow(2).mean(-1, keepdim=True) + eps).sqrt() * w.double()
+    want_h = h.double() + (norm(b, gain, 1e-5) if post else b)
+    want = norm(want_h, pre, 1e-6) if pre_norm else want_h
+    d = lambda v: v.to(DEV) if v is not None else None
+    out, hd, spare = torch.empty(n, hidden, dtype=dtype, device=DEV), h.to(DEV), torch.empty(n, hidden, dtype=dtype, device=DEV)
+    r = routed.RoutedRows(d(y), d(place), d(choice), d(weight), d(x), d(sh) if shared else None, spare, top, E, d(gate) if shared and gated else None)
+    assert r.norm_into(hd, d(gain) if post else None, 1e-5, out, d(pre) if pre_norm else None, 1e-6)
+    step = 4e-6 if dtype == torch.float32 else 2.0 ** -8
+    size = float((want_h - h.double()).abs().max())
+    assert float((hd.cpu().double() - want_h).abs().max()) <= step * size + 4e-6 * float(want_h.abs().max())
+    assert bool(((out.cpu().double() - want).abs() <= 1.5 * step * (want.abs() + float(want.abs().max()))).all())
+    plain_h, plain = h.to(DEV), torch.empty_like(out)
+    if hidden >= 64:                                # (as the two kernels in a row)
+        from agave_amd.ops import kernels
+        summed = torch.empty_like(spare)
+        routed.combine(d(y), d(place), d(choice), d(weight), d(x), d(sh) if shared else None, summed, top, E, d(gate) if shared and gated else None)
+        kernels.residual_norm(plain_h, summed, d(gain) if post else None, 1e-5, plain, d(pre) if pre_norm else None, 1e-6)
+        assert float((plain_h - hd).abs().max()) <= 4e-6 * float(want_h.abs().max())
+    assert not r.norm_into(hd[:, :hidden - 1], None, 0.0, out, d(pre), 1e-6)
+    got = r.rows().cpu().double()                   # whoever cannot take the pairs' rows gets them added up, once
+    assert r.rows() is spare and float((got - b).abs().max()) <= (2.0 ** -8 if dtype == torch.bfloat16 else 4e-6) * float(b.abs().max())
+    assert not r.norm_into(hd, None, 0.0, out, d(pre), 1e-6)
+
+
 @pytest.mark.parametrize("n,E,top,ff,hidden", [(1, 5, 2, 1024, 2048), (6, 16, 4, 2048, 1056), (40, 3, 2, 1024, 1024), (3, 4, 4, 4096, 1024)])
 def test_routed_few_pairs_in_tile_order(n, E, top, ff, hidden):
     """Tiles of 16 rows whose weights stream through a ring in LDS (columns summed over 1,024, 2,048 or 4,096; with others the kernel
