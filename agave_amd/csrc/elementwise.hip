@@ -7,6 +7,7 @@
 // src/backend/kernels/cpu/rope.zig:11-48 (split-half pairs), src/models/gemma3.zig:884-902
 // (position scaled before the angle), src/backend/kernels/cpu/activation.zig:69-113 (tanh GELU).
 #include "common_impl.h"
+#include "gate_act.h"
 #include "qk_rope.h"
 #include "trig.h"
 
@@ -960,39 +961,13 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
 }
 
 // ------------------------------------------------------------------ GeGLU
-__device__ __forceinline__ float gelu_tanh(float x) {
-    const float c = 0.7978845608028654f;
-    return 0.5f * x * (1.0f + tanhf(c * (x + 0.044715f * x * x * x)));
-}
-
-// The gate's activation, by number (the feed-forward part knows the names): 0 gelu, tanh form;
-// 1 silu, x / (1 + exp(-x)); 2 gelu with the error function; 3 relu.  Another one is another case
-// here; only the tanh form also ends the matrix-core products (gemm_mfma.hip).
-#define AGAVE_GATE_ACTS 4
-#define AGAVE_GATE_SWISH_CLAMPED 6     // a gated form with two numbers of its own, known to gated_act only
-__device__ __forceinline__ float gate_act(float x, int act) {
-    switch (act) {
-        case 0: return gelu_tanh(x);
-        case 1: return x / (1.0f + expf(-x));
-        case 2: return 0.5f * x * (1.0f + erff(x * 0.7071067811865476f));
-        default: return x > 0.f ? x : 0.f;
-    }
-}
-
 template <typename T>
 __global__ void gated_act_kernel(const T* __restrict__ gate, long ldg, const T* __restrict__ up, long ldu,
                                  T* __restrict__ out, long ldo, long total, int ff, int act, float p0, float p1) {
     for (long idx = (long)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
         const long r = idx / ff;
         const int c = (int)(idx % ff);
-        const float g = ld(gate + r * ldg + c), u = ld(up + r * ldu + c);
-        if (act == AGAVE_GATE_SWISH_CLAMPED) {
-            // g' = min(g, p0), u' = clamp(u, -p0, p0);  g' sigmoid(p1 g') (u' + 1)
-            const float gc = fminf(g, p0), uc = fminf(fmaxf(u, -p0), p0);
-            st(out + r * ldo + c, gc / (1.0f + expf(-p1 * gc)) * (uc + 1.0f));
-        } else {
-            st(out + r * ldo + c, gate_act(g, act) * u);
-        }
+        st(out + r * ldo + c, gate_form(ld(gate + r * ldg + c), ld(up + r * ldu + c), act, p0, p1));
     }
 }
 

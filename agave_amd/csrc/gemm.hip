@@ -12,6 +12,7 @@
 // elements do not fit.
 #include "common_impl.h"
 #include "fours.h"
+#include "gate_act.h"
 #include "mfma.h"
 
 // ---------------------------------------------------------------- one or two rows that fours do not fit
@@ -131,17 +132,21 @@ __global__ __launch_bounds__(NW * 64) void gemm_f32_skinny_kernel(const TA* __re
 // the waves there.  Root mean square of the error against 64 bits over that of the result, in 1e-7, groups of sixteen, as one run and so:
 // 3,072 x 2,048 0.94, 1.03, 0.94; 2,304 x 5,376 1.14, 1.38, 1.14; 5,376 x 2,048 1.03, 1.23, 1.03; 8,176 x 5,376 1.37, 1.78, 1.38; 32,768 x
 // 5,376 1.78, 1.78, 1.38, in the same time.
-template <typename TA, typename TW, typename TC, int NW, int R>
+// GATED (R = 2): W holds N rows of the gate matrix and behind them N of the up matrix; a workgroup makes 8 columns of either and leaves
+// act(gate) * up.  The activation as a kernel of its own cost its start, its end and a round trip to memory, 2.8 us of some 21 (2 x 5,376
+// columns of 2,048, three rows): 12 decode steps of 8 layers 7.37 -> 7.10 ms.
+template <typename TA, typename TW, typename TC, int NW, int R, bool GATED>
 __global__ __launch_bounds__(NW * 64, R == 2 ? 3 : 4) void gemm_f32_eight_rows_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W,
-                                                                      long ldw, TC* __restrict__ C, long ldc, int M, int N, int K) {
+                                                                      long ldw, TC* __restrict__ C, long ldc, int M, int N, int K, int act, float p0, float p1) {
+    static_assert(!GATED || R == 2, "a block of the gate's columns and one of the up matrix's");
     constexpr int U = 2, CHUNK = U * 32, S = 3;
     __shared__ float part[NW][R * 64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 7, h = (lane >> 3) & 1, g = lane >> 4;
-    const int n0 = blockIdx.x * 8 * R;
+    const int n0 = blockIdx.x * 8 * (GATED ? 1 : R);
     const TW* w[R];                                               // (rows and columns outside are computed from the last one and not stored)
 #pragma unroll
-    for (int i = 0; i < R; ++i) w[i] = W + (size_t)min(n0 + 8 * i + r, N - 1) * ldw;
+    for (int i = 0; i < R; ++i) w[i] = W + (GATED ? (size_t)i * N + min(n0 + r, N - 1) : (size_t)min(n0 + 8 * i + r, N - 1)) * ldw;
     const TA* a = A + (size_t)min(r, M - 1) * lda;
     const int lane_k = 16 * h + 4 * g;
     const int n_chunks = (K + CHUNK - 1) / CHUNK, n_iter = (n_chunks + NW - 1) / NW;
@@ -243,8 +248,8 @@ __global__ __launch_bounds__(NW * 64, R == 2 ? 3 : 4) void gemm_f32_eight_rows_k
             if (h == 0 && g < 2) part[wave][(4 * g + e) * 8 * R + 8 * i + r] = sum;
         }
     __syncthreads();
-    const int m = threadIdx.x / (8 * R), n = n0 + threadIdx.x % (8 * R);
-    if (m >= M || n >= N) return;
+    const int m = threadIdx.x / (8 * R), n = n0 + threadIdx.x % (GATED ? 8 : 8 * R);
+    if (m >= M || (!GATED && n >= N)) return;                     // (GATED: all sixteen lanes of a row stay for the exchange)
     float sums[NW];
 #pragma unroll
     for (int v = 0; v < NW; ++v) sums[v] = part[v][threadIdx.x];
@@ -252,7 +257,12 @@ __global__ __launch_bounds__(NW * 64, R == 2 ? 3 : 4) void gemm_f32_eight_rows_k
     for (int s = NW / 2; s > 0; s /= 2)
 #pragma unroll
         for (int v = 0; v < s; ++v) sums[v] += sums[v + s];
-    st(C + (size_t)m * ldc + n, sums[0]);
+    if (GATED) {
+        const float up = __shfl_xor(sums[0], 8);                  // column n of the up matrix lies eight lanes further
+        if ((threadIdx.x & 8) == 0 && n < N) st(C + (size_t)m * ldc + n, gate_form(sums[0], up, act, p0, p1));
+    } else {
+        st(C + (size_t)m * ldc + n, sums[0]);
+    }
 }
 
 // ---------------------------------------------------------------- more rows
@@ -660,9 +670,9 @@ static void launch_skinny(const TA* A, long lda, const TW* W, long ldw, TC* C, l
 template <typename TA, typename TW, typename TC>
 static void launch_eight_rows(const TA* A, long lda, const TW* W, long ldw, TC* C, long ldc, int M, int N, int K, hipStream_t stream) {
     const int blocks = (N + 7) / 8;
-    if (blocks <= COMPUTE_UNITS) gemm_f32_eight_rows_kernel<TA, TW, TC, 16, 1><<<blocks, 1024, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
-    else if (blocks <= (K > 512 ? 2 : 3) * COMPUTE_UNITS) gemm_f32_eight_rows_kernel<TA, TW, TC, 8, 1><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
-    else gemm_f32_eight_rows_kernel<TA, TW, TC, 4, 2><<<(blocks + 1) / 2, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    if (blocks <= COMPUTE_UNITS) gemm_f32_eight_rows_kernel<TA, TW, TC, 16, 1, false><<<blocks, 1024, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, 0, 0.f, 0.f);
+    else if (blocks <= (K > 512 ? 2 : 3) * COMPUTE_UNITS) gemm_f32_eight_rows_kernel<TA, TW, TC, 8, 1, false><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, 0, 0.f, 0.f);
+    else gemm_f32_eight_rows_kernel<TA, TW, TC, 4, 2, false><<<(blocks + 1) / 2, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, 0, 0.f, 0.f);
 }
 
 template <int BM, int BN, int WM, int WN, int S, int NS>
@@ -887,4 +897,21 @@ extern "C" int agave_gemm_slices_as(const float* A, long lda, const float* W, lo
             return 0;
         }
     AGAVE_CHECK(false, "gemm_slices_as: no tiles of %d x %d", bm, bn);
+}
+
+// ---------------------------------------------------------------- gate and up of few rows, with their activation
+// Whether agave_gemm_gated takes M rows by a gate and an up matrix of ff rows: up to eight, where the product of both takes two blocks of
+// columns a workgroup (launch_eight_rows), so that a workgroup has a block of either.
+extern "C" int agave_gemm_gated_takes(int M, int ff, int K) {
+    return M > 0 && M <= 8 && K > 0 && K % 4 == 0 && ff > 0 && (2L * ff + 7) / 8 > (K > 512 ? 2 : 3) * COMPUTE_UNITS;
+}
+// C [M, ff] <- act(A Wg^T) * (A Wu^T) for W = [Wg; Wu], all 32-bit
+extern "C" int agave_gemm_gated(const float* A, long lda, const float* W, long ldw, float* C, long ldc, int M, int ff, int K, int act, float p0,
+                                float p1, hipStream_t stream) {
+    AGAVE_CHECK(agave_gemm_gated_takes(M, ff, K), "gemm_gated: M=%d ff=%d K=%d", M, ff, K);
+    AGAVE_CHECK(lda >= K && ldw >= K && ldc >= ff && rows_of_fours<float>(A, lda) && rows_of_fours<float>(W, ldw), "gemm_gated: rows of aligned fours");
+    AGAVE_CHECK((act >= 0 && act < AGAVE_GATE_ACTS) || act == AGAVE_GATE_SWISH_CLAMPED, "gemm_gated: unknown activation %d", act);
+    gemm_f32_eight_rows_kernel<float, float, float, 4, 2, true><<<(ff + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, ff, K, act, p0, p1);
+    AGAVE_LAUNCH_CHECK("gemm_gated");
+    return 0;
 }

@@ -36,6 +36,8 @@ _SIGNATURES = {
     },
     "gemm": {
         "agave_gemm_plain": [_I, _P, _L, _I, _P, _L, _I, _P, _L, _I, _I, _I, _P],
+        "agave_gemm_gated_takes": [_I, _I, _I],
+        "agave_gemm_gated": [_P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _F, _F, _P],
         "agave_gemm_slices_for": [_I, _I, _I],
         "agave_gemm_slices": [_P, _L, _P, _L, _P, _I, _I, _I, _I, _P],
         "agave_add_slices": [_P, _L, _I, _P, _P],
@@ -350,6 +352,21 @@ def gated_act(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor, activatio
     n, ff = gate.shape
     library.call(lib("elementwise"), "agave_gated_act", dt(gate), act, float(p0), float(p1), ptr(gate), ldg, ptr(up), ldu, ptr(out), ldo, n, ff,
                  stream())
+
+
+def gemm_gated(x: torch.Tensor, w: Optional[torch.Tensor], out: torch.Tensor, activation: str = "gelu_tanh", p0: float = 0.0, p1: float = 1.0) -> bool:
+    """out = act(x Wg^T) * (x Wu^T) for ``w`` = [Wg; Wu], in one 32-bit kernel that takes a few rows; False: it does not take these."""
+    if w is None or x.dtype != torch.float32 or w.dtype != torch.float32 or out.dtype != torch.float32 or w.shape[0] % 2:
+        return False
+    (m, k), ff = x.shape, w.shape[0] // 2
+    if w.shape[1] != k or out.shape != (m, ff):
+        raise ValueError(f"gemm_gated: shapes do not fit: x {tuple(x.shape)}, w {tuple(w.shape)}, out {tuple(out.shape)}")
+    if (x.data_ptr() | w.data_ptr()) % 16 or x.stride(0) % 4 or w.stride(0) % 4 or not lib("gemm").agave_gemm_gated_takes(m, ff, k):
+        return False
+    _dev(x, w, out)
+    library.call(lib("gemm"), "agave_gemm_gated", ptr(x), _rows(x, "x"), ptr(w), _rows(w, "w"), ptr(out), _rows(out, "out"), m, ff, k,
+                 GATE_ACTIVATIONS[activation], float(p0), float(p1), stream())
+    return True
 
 
 # The activations of a feed-forward without a gate: the gate's, xIELU with two learned numbers, and the square of ReLU.

@@ -22,7 +22,7 @@ import time
 from typing import Dict, Iterable, List, Optional
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
-HEADERS = ("common.h", "common_impl.h", "mfma.h", "qk_rope.h", "noalloc.h", "trig.h", "row_pages.h", "fours.h", "gemm_tiles.h")
+HEADERS = ("common.h", "common_impl.h", "mfma.h", "qk_rope.h", "noalloc.h", "trig.h", "row_pages.h", "fours.h", "gemm_tiles.h", "gate_act.h")
 ARCH = "gfx950"
 # Packed 32-bit float instructions are switched off for all device code.
 FLAGS = ["-O3", "-std=c++17", "-shared", "-fPIC", f"--offload-arch={ARCH}",

@@ -6,8 +6,9 @@ product); the activation is the tanh form of GELU
 
 The activation is the spec's (``GatedFfnSpec.activation``, one of
 ``agave_amd.ops.kernels.GATE_ACTIVATIONS``).  On the matrix cores the product itself ends in the tanh form of
-GELU, SiLU and the clamped swish (one form with four numbers, ``agave_amd.ops.gemm_mfma.GateForm``); with any other, and
-in 32-bit, the stacked product is followed by the elementwise kernel, which takes the activation as a parameter.
+GELU, SiLU and the clamped swish (one form with four numbers, ``agave_amd.ops.gemm_mfma.GateForm``), and so does a 32-bit
+product of up to eight rows, in any activation; otherwise the stacked product is followed by the elementwise kernel, which
+takes the activation as a parameter.
 """
 from __future__ import annotations
 
@@ -18,10 +19,11 @@ import torch
 import math
 
 from ..config.spec import DenseFfnSpec, GatedFfnSpec
-from ..ops import gemm_mfma, kernels
+from ..ops import gemm_mfma, kernels, library
 from ..weights.loader import TensorNeed
 from .base import BuildEnv, register
 from .linear import Linear
+from .norm import NormedRows
 
 
 class GatedFfn:
@@ -62,13 +64,24 @@ class GatedFfn:
         without it."""
         return self.down.hand_over_bias()
 
+    def _gated_few_rows(self, x, act: torch.Tensor) -> bool:
+        """The 32-bit product of a few rows that ends in the activation."""
+        if self.gate_up.packed is not None or self.gate_up.bias is not None or act.dtype != torch.float32 or act.shape[0] > 8:
+            return False
+        if isinstance(x, NormedRows):
+            x = x.rows()
+        library.profile.label = self.gate_up.name
+        made = kernels.gemm_gated(x, self.gate_up.weight, act, self.spec.activation, self.spec.act_limit, self.spec.act_alpha)
+        library.profile.label = None
+        return made
+
     def forward(self, x: torch.Tensor, step, slices_ok: bool = True, tag: str = "ffn") -> torch.Tensor:
         """``slices_ok`` False: the result is wanted as rows of the activations' type (a caller that is no
         block and adds something to it); ``tag`` keeps the buffers of two feed-forwards of one layer apart."""
         ff = self.spec.intermediate
         n = x.shape[0]
         act = self.env.workspace.get(tag + "_act", n, ff, x.dtype)
-        if not self.gate_up.forward_gated(x, act):
+        if not self.gate_up.forward_gated(x, act) and not self._gated_few_rows(x, act):
             gu = self.gate_up.forward(x, tag="gate_up" if tag == "ffn" else tag + "_gate_up")
             kernels.gated_act(gu[:, :ff], gu[:, ff:], act, self.spec.activation, self.spec.act_limit, self.spec.act_alpha)
         return self.down.forward(act, tag=tag + "_down", slices_ok=slices_ok)    # the block adds it to the residual stream

@@ -391,6 +391,31 @@ def test_gemm_plain_up_to_eight_rows(K, ta, tw, n, k):
     assert not bool(got[2, :5].isfinite().any()) and not bool(got[0, 5].isfinite())
 
 
+@pytest.mark.parametrize("ff,k", [(2049, 516), (3080, 512), (3073, 4), (5376, 2048), (2056, 772)])
+@pytest.mark.parametrize("activation", ["gelu_tanh", "silu", "swish_clamped"])
+def test_gemm_gated_few_rows(K, ff, k, activation):
+    """Gate and up of up to eight rows with their activation in one kernel, against the product and the activation in a row (their
+    sums begin at another chunk of columns for another block, so they differ by rounding: either is within k 2^-24 of its
+    products' sizes, which the forms here pass on at most 1.2-fold): a broken last block of columns, rows that lie apart; what
+    it does not take is refused."""
+    g = torch.Generator(device=DEV).manual_seed(ff + k)
+    w = torch.randn(2 * ff, k, device=DEV, generator=g) * k ** -0.5
+    for m in (1, 3, 8):
+        x = torch.randn(m, k + 4, device=DEV, generator=g)[:, :k]
+        out, gu, want = torch.full((m + 1, ff + 2), 7.0, device=DEV), torch.empty(m, 2 * ff, device=DEV), torch.empty(m, ff, device=DEV)
+        assert K.gemm_gated(x, w, out[:m, :ff], activation, 1.5, 0.7)
+        K.gemm_plain(x, w, gu)
+        K.gated_act(gu[:, :ff], gu[:, ff:], want, activation, 1.5, 0.7)
+        size = x.abs() @ w.abs().T
+        off = 1.2 * 2 * k * 2.0 ** -24 * (size[:, :ff] * (gu[:, ff:].abs() + 1.0) + size[:, ff:] * gu[:, :ff].abs()) + 1e-6 * want.abs()
+        assert bool(((out[:m, :ff] - want).abs() <= off).all()) and float((out[:m, :ff] - want).norm()) <= 1e-6 * float(want.norm())
+        assert bool((out[m] == 7.0).all()) and bool((out[:, ff:] == 7.0).all())
+    x = torch.randn(9, k + 4, device=DEV, generator=g)
+    out = torch.empty(9, ff, device=DEV)
+    assert not K.gemm_gated(x[:, :k], w, out) and not K.gemm_gated(x[:3, 1:k + 1], w, out[:3])
+    assert not K.gemm_gated(x[:3, :k].bfloat16(), w, out[:3]) and not K.gemm_gated(x[:3, :k].contiguous(), w[:2048], out[:3, :1024])
+
+
 def test_gemm_plain_up_to_eight_rows_rounds_alike(K):
     """Sums are no longer on one side of the lines between the kernels than on the other: 16 waves share K up to 2,048 columns, 8 up to
     4,096 (the same products a sum, so the same error but for chance, some 1 % over 16,000 results) and 4 beyond (twice as
