@@ -20,7 +20,8 @@
 // A (token, slot) pair p = t * top + slot names one chosen output.  The plain kernels take the pairs
 // as they come (a wave per pair and output column).  The matrix-core kernels take them sorted by
 // expert, in tiles of 16, 64 or 128 pairs that never span two experts (`route_sort` makes the list and the
-// tiles' table on the device, so a step's launches never depend on the choice).
+// tiles' table on the device, so a step's launches never depend on the choice), or, of few pairs, find an expert's from the
+// choices themselves.
 #include "common_impl.h"
 #include "fours.h"
 #include "mfma.h"
@@ -1029,17 +1030,93 @@ __global__ __launch_bounds__(256) void routed_product_mfma_kernel(const bf16* __
 // Measured, us, both products, with the kernel above and so, 1, 2, 4 and 16 rows: 16 experts of 2,048 by 2,048, 4 a row, 34 44 78 117
 // and 30 43 57 87; 32 of 1,024 by 1,024, 4 a row, 18 21 27 49 and 15 20 24 38; 8 of 4,096 by 4,096, 2 a row, 44 118 116 185 and 48
 // 96 107 153; 8 of 4,096 inner rows by 1,024, 2 a row, 25 33 40 49 and 21 27 39 46.
-template <int KQ, bool GATED>
+// Of up to FEW_PAIRS pairs a workgroup finds its own rows from the pairs' choices (CHOSEN): which of them chose the same expert
+// as it takes a vote a bit of the expert's number, and a tile is then led by every sixteenth pair of an expert, tiles counted in the
+// pairs' order.  The rows of either product are the pairs themselves, and there is no sorted list to wait for, neither its kernel nor
+// two loads one after the other at the start of both products.  us, sorting and both products, and so: 17 experts of 2,048 by
+// 2,048, 5 a row, 1 row 37.1 and 35.4, 6 rows 80.2 and 72.9, 16 rows 89.6 and 82.4, 48 rows 115.9 and 109.2; 32 of 1,024 by 2,048, 4 a row,
+// 23.9 and 16.0, 54.3 and 52.9, 72.6 and 66.1, 84.8 and 79.2; 8 of 4,096 by 4,096, 2 a row, 60.1 and 44.8, 141 and 134, 150 and 141, 177 and 169;
+// 256 of 1,024 by 1,024, 8 a row, 26.2 and 18.2, 58.2 and 59.5, 141 and 126, 32 rows 228 and 200.  A thread looks at one pair, which is the
+// limit; more pairs are sorted as before, in a time that is little of theirs.
+#define FEW_PAIRS 256
+// The expert of tile `tile` (-1: no such tile) and in mine[16], of this wave, the pairs of its rows (-1: no such row).  LDS, 16-byte
+// pieces nobody else uses until all waves are back: `counts` 4 E + 6 words, `mine` the waves' rows `stride` words apart.
+__device__ __forceinline__ int few_tile(const int* __restrict__ choice, int P, int E, int tile, int* counts, int* mine, int stride) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool alone = P <= 64;                                   // (every wave looks at all pairs and needs no other)
+    const int pair = alone ? lane : (int)threadIdx.x;
+    const int chosen = choice[min(pair, P - 1)];
+    const bool valid = pair < P && (unsigned)chosen < (unsigned)E;
+    if (lane < 16) mine[w * stride + lane] = -1;
+    if (!alone)
+        for (int i = threadIdx.x; i < 4 * E; i += 256) counts[i] = 0;
+    unsigned long long same = __ballot(valid);
+    for (int b = 0; (E - 1) >> b; ++b) {
+        const bool bit = (chosen >> b) & 1;
+        const unsigned long long ones = __ballot(bit);
+        same &= bit ? ones : ~ones;
+    }
+    const unsigned long long below = (1ull << lane) - 1;
+    int rank = __popcll(same & below);                            // of the pair among its expert's
+    if (!alone) {
+        __syncthreads();
+        if (valid && (same >> lane) == 1) counts[w * E + chosen] = rank + 1;       // (its expert's last of the wave)
+        __syncthreads();
+        for (int o = 0; o < w; ++o)
+            if (valid) rank += counts[o * E + chosen];
+    }
+    const unsigned long long leaders = __ballot(valid && (rank & 15) == 0);
+    int first = 0, e = -1, base = 0;
+    if (!alone) {
+        if (lane == 0) counts[4 * E + w] = __popcll(leaders);
+        __syncthreads();
+        int all = 0;
+        for (int o = 0; o < 4; ++o) {
+            if (o == w) first = all;
+            all += counts[4 * E + o];
+        }
+        if (tile >= all) return -1;
+    } else if (tile >= __popcll(leaders)) {
+        return -1;
+    }
+    const unsigned long long leads = __ballot(((leaders >> lane) & 1) && first + __popcll(leaders & below) == tile);
+    if (leads) {
+        const int at = __ffsll(leads) - 1;
+        e = __builtin_amdgcn_readlane(chosen, at);
+        base = __builtin_amdgcn_readlane(rank, at);
+    }
+    if (alone) {
+        if (valid && chosen == e && rank >= base && rank < base + 16) mine[w * stride + rank - base] = pair;
+    } else {
+        if (leads && lane == 0) {
+            counts[4 * E + 4] = e;
+            counts[4 * E + 5] = base;
+        }
+        __syncthreads();
+        e = counts[4 * E + 4];
+        base = counts[4 * E + 5];
+        if (valid && chosen == e && rank >= base && rank < base + 16)
+            for (int o = 0; o < 4; ++o) mine[o * stride + rank - base] = pair;
+        __syncthreads();
+    }
+    __builtin_amdgcn_wave_barrier();                              // (a wave's LDS accesses happen in the order they were issued)
+    return __builtin_amdgcn_readfirstlane(e);
+}
+
+template <int KQ, bool GATED, bool CHOSEN>
 __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* __restrict__ x, long ldx, const int* __restrict__ sorted_pair,
                                                                     const int* __restrict__ tile_expert, const uint4* __restrict__ w0,
                                                                     const uint4* __restrict__ w1, void* __restrict__ out_, int top, int n_out,
-                                                                    int act, int blocks, float p0, float p1) {
+                                                                    int act, int blocks, float p0, float p1, int P, int E) {
     constexpr int K = KQ * 128, KB = K / 32, NS = 8;
     static_assert(KQ % NS == 0, "a step's place in the ring is known where it is written");
     constexpr int COLS = GATED ? 16 : 32;
     __shared__ __attribute__((aligned(16))) unsigned char ring[4][NS][2048];
     __shared__ float part[2][4][2][256];
-    const int e = tile_expert[blockIdx.x];
+    static_assert(sizeof(ring) >= (4 * ROUTE_MAX + 6) * sizeof(int), "the experts' counts fit the ring");
+    // (CHOSEN: sorted_pair holds the choices; part's first half keeps the rows' pairs until its first sums)
+    int* mine = reinterpret_cast<int*>(&part[0][0][0][0]);
+    const int e = CHOSEN ? few_tile(sorted_pair, P, E, blockIdx.x, reinterpret_cast<int*>(&ring[0][0][0]), mine, 512) : tile_expert[blockIdx.x];
     if (e < 0) return;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
@@ -1047,7 +1124,12 @@ __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* 
     const int b0 = blockIdx.y * blocks, b1 = min(b0 + blocks, (n_out + COLS - 1) / COLS);
     if (b0 >= b1) return;
     long r = row0 + c;
-    if (GATED) {
+    int out_row = row0 + 4 * g + w;                               // -1: not stored
+    if (CHOSEN) {
+        const int p = mine[w * 512 + c];
+        out_row = mine[w * 512 + 4 * g + w];
+        r = p >= 0 ? (GATED ? p / top : p) : 0;
+    } else if (GATED) {
         const int p = sorted_pair[r];
         r = p >= 0 ? p / top : 0;                                 // (a padding row computes on row 0 and is never read)
     }
@@ -1099,7 +1181,8 @@ __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* 
         float v[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) v[i] = ((sums[0][i][w * 64 + lane] + sums[1][i][w * 64 + lane]) + sums[2][i][w * 64 + lane]) + sums[3][i][w * 64 + lane];
-        const size_t row = (size_t)row0 + 4 * g + w;
+        if (CHOSEN && out_row < 0) continue;
+        const size_t row = (size_t)out_row;
         if constexpr (GATED) {
             ((bf16*)out_)[row * n_out + b * 16 + c] = f32_to_bf16(expert_gated(v[0], v[1], act, p0, p1));
         } else {
@@ -1116,9 +1199,9 @@ __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* 
 // The columns that the kernel above is built for (its rows take K / 32 registers a lane, and the ring's places have to come out even).
 extern "C" int agave_routed_few_takes(int K) { return K == 1024 || K == 2048 || K == 4096; }
 
-template <bool GATED>
+template <bool GATED, bool CHOSEN>
 static bool launch_routed_few(const void* x, long ldx, const int* sorted_pair, const int* tile_expert, int max_tiles, const void* w0,
-                              const void* w1, void* out, int top, int live, int n_out, int K, int act, float p0, float p1, hipStream_t stream) {
+                              const void* w1, void* out, int top, int live, int n_out, int K, int act, float p0, float p1, int P, int E, hipStream_t stream) {
     if (!agave_routed_few_takes(K)) return false;
     const int all = (n_out + (GATED ? 15 : 31)) / (GATED ? 16 : 32);
     // Blocks a workgroup: the fewest with which all workgroups of the experts that are expected run at once, two to a compute unit, with a
@@ -1130,13 +1213,40 @@ static bool launch_routed_few(const void* x, long ldx, const int* sorted_pair, c
     blocks = blocks < 1 ? 1 : blocks > 16 ? 16 : blocks;
     const dim3 grid(max_tiles, (all + blocks - 1) / blocks);
     if (grid.y > 65535) return false;
-#define FEW_GO(KQ_) routed_product_few_kernel<KQ_, GATED><<<grid, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const uint4*)w0, \
-                                                                                    (const uint4*)w1, out, top, n_out, act, blocks, p0, p1)
+#define FEW_GO(KQ_) routed_product_few_kernel<KQ_, GATED, CHOSEN><<<grid, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const uint4*)w0, \
+                                                                                            (const uint4*)w1, out, top, n_out, act, blocks, p0, p1, P, E)
     if (K == 1024) FEW_GO(8);
     else if (K == 2048) FEW_GO(16);
     else FEW_GO(32);
 #undef FEW_GO
     return true;
+}
+
+// experts that have rows, if the rows choose evenly
+static int live_experts(int n_rows, int top, int E) { return top >= E ? E : (int)ceil(E * (1.0 - pow(1.0 - (double)top / E, (double)n_rows))); }
+
+// Whether agave_routed_experts_chosen takes a feed-forward: few pairs, columns of both products that the kernel above streams.
+extern "C" int agave_routed_chosen_takes(int P, int E, int ff, int hidden) {
+    return P > 0 && P <= FEW_PAIRS && E > 0 && E <= ROUTE_MAX && agave_routed_few_takes(ff) && agave_routed_few_takes(hidden);
+}
+
+// The experts' products of few pairs, weights in tile order, without a sorted list: act_rows [n top, ff] bfloat16 and
+// y [n top, hidden] float32 hold a row a pair (nothing for a pair whose choice is no expert).
+extern "C" int agave_routed_experts_chosen(const void* x, long ldx, const int* choice, const void* wg, const void* wu, const void* wd, void* act_rows, float* y,
+                                           int n_rows, int top, int E, int ff, int hidden, int act, float p0, float p1, hipStream_t stream) {
+    AGAVE_CHECK(n_rows >= 0 && top > 0 && ldx >= hidden && ldx % 8 == 0, "routed_experts_chosen: bad sizes");
+    if (n_rows == 0) return 0;
+    AGAVE_CHECK((long)n_rows * top <= FEW_PAIRS && agave_routed_chosen_takes(n_rows * top, E, ff, hidden), "routed_experts_chosen: %d rows of %d pairs, %d experts of %d by %d",
+                n_rows, top, E, ff, hidden);
+    AGAVE_CHECK((act >= 0 && act < 4) || act == 6, "routed_experts_chosen: unknown activation %d", act);
+    AGAVE_CHECK(x && choice && wg && wu && wd && act_rows && y, "routed_experts_chosen: null buffer");
+    AGAVE_CHECK((((uintptr_t)x | (uintptr_t)wg | (uintptr_t)wu | (uintptr_t)wd | (uintptr_t)act_rows) & 15) == 0, "routed_experts_chosen: buffers must be aligned to 16 bytes");
+    const int P = n_rows * top, live = live_experts(n_rows, top, E), tiles = min(P, (P + 15) / 16 + E);
+    const bool done = launch_routed_few<true, true>(x, ldx, choice, nullptr, tiles, wg, wu, act_rows, top, live, ff, hidden, act, p0, p1, P, E, stream)
+                   && launch_routed_few<false, true>(act_rows, ff, choice, nullptr, tiles, wd, nullptr, y, top, live, hidden, ff, act, p0, p1, P, E, stream);
+    AGAVE_CHECK(done, "routed_experts_chosen: sizes the kernel is not built for");
+    AGAVE_LAUNCH_CHECK("routed_experts_chosen");
+    return 0;
 }
 
 // Many pairs an expert, weights in tile order: a workgroup takes a tile of TT sorted rows and 2 TT columns of weights
@@ -1354,13 +1464,12 @@ extern "C" int agave_routed_experts_mfma(const void* x, long ldx, const int* sor
         routed_product_mfma_kernel<4, 4, false><<<g2, 256, 0, stream>>>((const bf16*)act_rows, ff, sorted_pair, tile_expert, (const bf16*)wd,
                                                                      nullptr, y, top, hidden, ff, act, wpacked, p0, p1);
     } else {
-        // experts that have rows, if the rows choose evenly
-        const int live = top >= E ? E : (int)ceil(E * (1.0 - pow(1.0 - (double)top / E, (double)n_rows)));
-        const bool few1 = wpacked && launch_routed_few<true>(x, ldx, sorted_pair, tile_expert, max_tiles, wg, wu, act_rows, top, live, ff, hidden, act, p0, p1, stream);
+        const int live = live_experts(n_rows, top, E);
+        const bool few1 = wpacked && launch_routed_few<true, false>(x, ldx, sorted_pair, tile_expert, max_tiles, wg, wu, act_rows, top, live, ff, hidden, act, p0, p1, 0, 0, stream);
         if (!few1)
             routed_product_mfma_kernel<1, 1, true><<<g1, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const bf16*)wg,
                                                                     (const bf16*)wu, act_rows, top, ff, hidden, act, wpacked, p0, p1);
-        const bool few2 = wpacked && launch_routed_few<false>(act_rows, ff, nullptr, tile_expert, max_tiles, wd, nullptr, y, top, live, hidden, ff, act, p0, p1, stream);
+        const bool few2 = wpacked && launch_routed_few<false, false>(act_rows, ff, nullptr, tile_expert, max_tiles, wd, nullptr, y, top, live, hidden, ff, act, p0, p1, 0, 0, stream);
         if (!few2)
             routed_product_mfma_kernel<1, 1, false><<<g2, 256, 0, stream>>>((const bf16*)act_rows, ff, sorted_pair, tile_expert, (const bf16*)wd,
                                                                      nullptr, y, top, hidden, ff, act, wpacked, p0, p1);

@@ -17,6 +17,8 @@ kernels.register_signatures(LIBRARY, {
     "agave_route_rows": [_I, _P, _L, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _P, _I, _I, _P, _I, _I, _I, _I, _P],
     "agave_routed_few_takes": [_I],
     "agave_route_sort": [_P, _I, _I, _I, _I, _I, _P, _P, _P, _P],
+    "agave_routed_chosen_takes": [_I, _I, _I, _I],
+    "agave_routed_experts_chosen": [_P, _L, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "agave_routed_experts_mfma": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _P],
     "agave_routed_norm": [_I, _P, _P, _P, _P, _P, _I, _I, _P, _L, _P, _P, _F, _P, _L, _P, _F, _I, _I, _P],
     "agave_routed_combine": [_I, _P, _P, _P, _P, _P, _L, _P, _L, _P, _P, _L, _I, _I, _I, _I, _P],
@@ -210,6 +212,35 @@ def experts_mfma(x: torch.Tensor, sorted_pair: torch.Tensor, tile_expert: torch.
     library.call(_lib(), "agave_routed_experts_mfma", ptr(x), x.stride(0), ptr(sorted_pair), ptr(tile_expert), ptr(w_gate),
                  ptr(w_up), ptr(w_down), ptr(act_rows), ptr(y), tm, tiles, n, top, e, ff, hidden, activation,
                  1 if tile_order else 0, float(p0), float(p1), stream())
+
+
+def chosen_takes(n_pairs: int, n_experts: int, ff: int, hidden: int) -> bool:
+    """Whether :func:`experts_chosen` takes this many pairs of experts of these sizes (held in tile order)."""
+    return bool(_lib().agave_routed_chosen_takes(n_pairs, n_experts, ff, hidden))
+
+
+def experts_chosen(x: torch.Tensor, choice: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
+                   act_rows: torch.Tensor, y: torch.Tensor, top: int, activation: int, p0: float = 0.0, p1: float = 1.0) -> None:
+    """The experts' products of few pairs, straight from the pairs' choices: ``act_rows`` [N * top, ff] bfloat16 and ``y``
+    [N * top, hidden] float32 receive a row a pair (nothing where the choice is no expert).  The weights were rearranged by
+    :func:`pack_expert_weights`."""
+    _dev(x, choice, w_gate, w_up, w_down, act_rows, y)
+    n, hidden = x.shape
+    e, ff, k = w_gate.shape
+    if k != hidden or w_up.shape != w_gate.shape or w_down.shape != (e, hidden, ff):
+        raise ValueError("experts: weights must be [E, ff, hidden], [E, ff, hidden] and [E, hidden, ff]")
+    for w in (w_gate, w_up, w_down):
+        if w.dtype != torch.bfloat16 or not w.is_contiguous():
+            raise TypeError("experts: the matrix-core kernels take contiguous bfloat16 weights")
+    if not mfma_ok(x, ff) or x.stride(1) != 1 or not chosen_takes(n * top, e, ff, hidden):
+        raise ValueError("experts: rows or sizes that the kernel of few pairs does not take")
+    if act_rows.dtype != torch.bfloat16 or not act_rows.is_contiguous() or act_rows.shape != (n * top, ff):
+        raise ValueError(f"experts: inner rows must be bfloat16 [{n * top}, {ff}]")
+    if y.dtype != torch.float32 or not y.is_contiguous() or y.shape != (n * top, hidden):
+        raise ValueError(f"experts: y must be float32 [{n * top}, {hidden}]")
+    _i32(choice, "choice", n * top)
+    library.call(_lib(), "agave_routed_experts_chosen", ptr(x), x.stride(0), ptr(choice), ptr(w_gate), ptr(w_up), ptr(w_down),
+                 ptr(act_rows), ptr(y), n, top, e, ff, hidden, activation, float(p0), float(p1), stream())
 
 
 def route_rows(x: torch.Tensor, router: torch.Tensor, correction: Optional[torch.Tensor], groups: int, keep: int, top: int,

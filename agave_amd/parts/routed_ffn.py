@@ -165,16 +165,23 @@ class RoutedFfn:
         if self.tile_order and not routed.mfma_ok(x, s.intermediate):
             raise ValueError("routed feed-forward: its experts are kept in tile order, which takes aligned bfloat16 rows")
         if s.n_experts and self.w_gate.dtype == torch.bfloat16 and routed.mfma_ok(x, s.intermediate):
-            # the pairs sorted by expert on the device, then the experts' products tile by tile on the matrix cores
             tm, tiles, cap = routed.tile_plan(n * pairs, experts, self.tile_order, s.intermediate, s.hidden)
-            place = ws.get("expert_place", n * pairs, 1, torch.int32).view(-1)
-            sorted_pair = ws.get(f"expert_sorted{tm}", cap, 1, torch.int32).view(-1)
-            tile_expert = ws.get(f"expert_tiles{tm}", tiles, 1, torch.int32).view(-1)
-            routed.route_sort(choice.view(-1), experts, tm, tiles, place, sorted_pair, tile_expert)
-            act_rows = ws.get("expert_act", cap, s.intermediate, x.dtype)
-            y = ws.get("expert_rows", cap, s.hidden, torch.float32)
-            routed.experts_mfma(x, sorted_pair, tile_expert, self.w_gate, self.w_up, self.w_down, act_rows, y, tm, tiles, pairs,
-                                self.act, tile_order=self.tile_order, p0=s.act_limit, p1=s.act_alpha)
+            if self.tile_order and tm == 16 and routed.chosen_takes(n * pairs, experts, s.intermediate, s.hidden):
+                # few pairs: the products find their rows from the choices themselves
+                act_rows = ws.get("expert_act", n * pairs, s.intermediate, x.dtype)
+                y = ws.get("expert_rows", n * pairs, s.hidden, torch.float32)
+                routed.experts_chosen(x, choice.view(-1), self.w_gate, self.w_up, self.w_down, act_rows, y, pairs, self.act,
+                                      s.act_limit, s.act_alpha)
+            else:
+                # the pairs sorted by expert on the device, then the experts' products tile by tile on the matrix cores
+                place = ws.get("expert_place", n * pairs, 1, torch.int32).view(-1)
+                sorted_pair = ws.get(f"expert_sorted{tm}", cap, 1, torch.int32).view(-1)
+                tile_expert = ws.get(f"expert_tiles{tm}", tiles, 1, torch.int32).view(-1)
+                routed.route_sort(choice.view(-1), experts, tm, tiles, place, sorted_pair, tile_expert)
+                act_rows = ws.get("expert_act", cap, s.intermediate, x.dtype)
+                y = ws.get("expert_rows", cap, s.hidden, torch.float32)
+                routed.experts_mfma(x, sorted_pair, tile_expert, self.w_gate, self.w_up, self.w_down, act_rows, y, tm, tiles, pairs,
+                                    self.act, tile_order=self.tile_order, p0=s.act_limit, p1=s.act_alpha)
         elif s.n_experts:
             act_rows = ws.get("expert_act", n * top, s.intermediate, x.dtype)
             y = ws.get("expert_rows", n * top, s.hidden, torch.float32)

@@ -616,6 +616,29 @@ def test_routed_few_pairs_in_tile_order(n, E, top, ff, hidden):
     assert bool(torch.isfinite(rows[0]).all()) and torch.equal(rows[0], rows[1])
 
 
+@pytest.mark.parametrize("n,top,E,chosen", [(1, 1, 1, 1), (1, 64, 64, 64), (6, 5, 17, 17), (63, 1, 3, 5), (64, 1, 1, 1), (65, 1, 1, 1), (16, 4, 65, 70), (16, 5, 17, 17),
+                                            (85, 3, 4, 6), (256, 1, 1, 1), (32, 8, 130, 140)])
+def test_few_pairs_find_their_rows_from_the_choices(n, top, E, chosen):
+    """Without a sorted list the same rows as with one, to the bit: pairs of one wave and of four, experts of none, one, 16, 17 and all
+    pairs, choices that are no expert's (negative or past the last), whose rows stay as they are."""
+    from agave_amd.ops import routed
+    ff, hidden, P = 1024, 2048, n * top
+    g = torch.Generator().manual_seed(P + E)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * s[-1] ** -0.5).bfloat16().to(DEV)
+    x, w = torch.randn(n, hidden, generator=g).bfloat16().to(DEV), [routed.pack_expert_weights(rnd(*s)) for s in ((E, ff, hidden), (E, ff, hidden), (E, hidden, ff))]
+    choice = torch.randint(-1 if chosen > E else 0, chosen, (P,), generator=g).int().to(DEV)
+    tiles = (P + 15) // 16 + E
+    place, sorted_pair, tile_expert = (torch.full((k,), -7, dtype=torch.int32, device=DEV) for k in (P, tiles * 16, tiles))
+    routed.route_sort(choice, E, 16, tiles, place, sorted_pair, tile_expert)
+    want = torch.empty(tiles * 16, hidden, device=DEV)
+    routed.experts_mfma(x, sorted_pair, tile_expert, *w, torch.empty(tiles * 16, ff, dtype=torch.bfloat16, device=DEV), want, 16, tiles, top, 1, tile_order=True)
+    assert routed.chosen_takes(P, E, ff, hidden) and not routed.chosen_takes(257, E, ff, hidden) and not routed.chosen_takes(P, E, ff, 1056)
+    y = torch.full((P, hidden), 7.0, device=DEV)
+    routed.experts_chosen(x, choice, *w, torch.empty(P, ff, dtype=torch.bfloat16, device=DEV), y, top, 1)
+    expert = (choice >= 0) & (choice < E)
+    assert torch.equal(y[expert], want[place[expert].long()]) and bool((y[~expert] == 7.0).all()) and bool(torch.isfinite(y).all())
+
+
 @pytest.mark.parametrize("tm", [16, 64])
 @pytest.mark.parametrize("P,E,chosen", [(1, 1, 1), (1, 64, 70), (64, 64, 64), (63, 7, 9), (40, 3, 2), (64, 1, 1), (65, 64, 66), (64, 65, 65)])
 def test_route_sort_of_few_pairs(P, E, chosen, tm):
