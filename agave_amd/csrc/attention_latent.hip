@@ -214,18 +214,37 @@ struct LatentValuesArgs {
     int heads, vd, out;
 };
 
-// A workgroup per (row, head), eight waves.  The merge: four groups of 128 threads take the shares in turn, a thread four
+// One workgroup or a few per (row, head), eight waves.  The merge: four groups of 128 threads take the shares in turn, a thread four
 // neighbouring elements.  The product: a wave per block of 16 outputs, the merged row as all sixteen columns of the
-// operand.  VK: steps of 32 elements along the row.
-template <int VK>
+// operand.  VK: steps of 32 elements along the row.  SR: shares of a group at most.
+// Bound by the ways to memory, one after the other: everything that is read (the shares' sums, then their rows, the first block's
+// matrix and gate) is asked for before anything is waited for, and in the order in which it is needed, and every wave has all shares'
+// weights in its lanes.  us, with the shares' sums waited for first and a workgroup a (row, head), and so, 16 heads of 512 by 128: 1 row
+// of 64 shares 7.1 and 4.3, 4 rows 7.2 and 4.8, 6 rows of 42 7.9 and 6.3, 16 rows of 16 7.6 and 7.3, 64 rows of 4 25.0 and 23.6; 128 heads,
+// 8 rows of 4 23.0 and 22.8.
+template <int VK, int SR>
 __global__ __launch_bounds__(512) void latent_values_kernel(LatentValuesArgs A) {
     __shared__ f32x4_t part[4][LATENT_MAX_VALUE / 4];
-    __shared__ float wt[LATENT_MAX_SPLITS];
     __shared__ __attribute__((aligned(16))) bf16 row[LATENT_MAX_VALUE + 32];
     const int r = blockIdx.x / A.heads, h = blockIdx.x % A.heads, tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
-    const int vd = A.vd, out = A.out, n_ob = (out + 15) / 16;
+    const int vd = A.vd, out = A.out, splits = A.splits;
+    // this workgroup's blocks of outputs
+    const int all = (out + 15) / 16, per = (all + gridDim.y - 1) / gridDim.y, ob0 = blockIdx.y * per, n_ob = min(ob0 + per, all);
     const bf16* w = A.w + (size_t)h * out * vd;
+    const size_t first = (size_t)blockIdx.x * splits;
+    const float* ml = A.part_ml + (first + (lane < splits ? lane : 0)) * 2;
+    const float share_m = ml[0], share_l = ml[1];
+    const int grp = wv >> 1, d = (tid & 127) * 4;
+    f32x4_t x[SR];
+    {
+        const float* src = A.part_o + first * vd + (d < vd ? d : 0);
+#pragma unroll
+        for (int j = 0; j < SR; ++j) {
+            const int s = grp + 4 * j;                       // (past the last share: the last one again, of weight 0)
+            x[j] = *reinterpret_cast<const f32x4_t*>(src + (size_t)(s < splits ? s : splits - 1) * vd);
+        }
+    }
     // the first block's share of the matrix travels while the shares are merged
     frag16 f[VK];
     auto ask = [&](int ob) {
@@ -237,34 +256,33 @@ __global__ __launch_bounds__(512) void latent_values_kernel(LatentValuesArgs A) 
             f[k].u = *reinterpret_cast<const uint4*>(wr + (e < vd ? e : 0));       // (the row is empty there)
         }
     };
-    ask(wv < n_ob ? wv : 0);
-    const size_t first = (size_t)blockIdx.x * A.splits;
-    // every wave makes the shares' weights; the first leaves them in LDS
-    {
-        const int s = lane < A.splits ? lane : 0;
-        const float ms = A.part_ml[(first + s) * 2], ls = A.part_ml[(first + s) * 2 + 1];
-        const float m = lane < A.splits ? ms : -INFINITY, top = wave_max(m);
-        const float e = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - top);
-        const float total = wave_sum(e * ls);
-        if (wv == 0) wt[lane] = total > 0.f ? e / total : 0.f;
+    float gate[4];
+    auto ask_gate = [&](int ob) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int n = 16 * ob + 4 * g + e;
+            gate[e] = A.gate ? A.gate[(size_t)r * A.ldg + (size_t)h * out + (n < out ? n : out - 1)] : 0.f;
+        }
+    };
+    if (ob0 + wv < n_ob) {
+        ask(ob0 + wv);
+        ask_gate(ob0 + wv);
     }
-    __syncthreads();
-    const int grp = tid >> 7, d = (tid & 127) * 4;
-    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    if (d < vd) {
-        const float* src = A.part_o + first * vd + d;
-        for (int s0 = grp; s0 < A.splits; s0 += 16) {
-            f32x4_t x[4];
+    __builtin_amdgcn_sched_barrier(0);
+    float weight;                                            // of share `lane`
+    {
+        const float m = lane < splits ? share_m : -INFINITY, top = wave_max(m);
+        const float e = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - top);
+        const float total = wave_sum(e * share_l);
+        weight = total > 0.f ? e / total : 0.f;
+    }
+    {
+        f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int s = s0 + 4 * j;
-                x[j] = *reinterpret_cast<const f32x4_t*>(src + (size_t)(s < A.splits ? s : s0) * vd);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int s = s0 + 4 * j;
-                acc += x[j] * (s < A.splits ? wt[s] : 0.f);
-            }
+        for (int j = 0; j < SR; ++j) {
+            const int s = grp + 4 * j;
+            const float ws = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s));      // (SR <= 16: s < 64)
+            acc += x[j] * (s < splits ? ws : 0.f);
         }
         part[grp][tid & 127] = acc;
     }
@@ -272,20 +290,23 @@ __global__ __launch_bounds__(512) void latent_values_kernel(LatentValuesArgs A) 
     if (tid < 128) {
         uint2 p = make_uint2(0, 0);
         if (d < vd) {
-            const f32x4_t x = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
-            p = make_uint2(f32x2_to_bf16x2(x[0], x[1]), f32x2_to_bf16x2(x[2], x[3]));
+            const f32x4_t sum = part[0][tid] + part[1][tid] + part[2][tid] + part[3][tid];
+            p = make_uint2(f32x2_to_bf16x2(sum[0], sum[1]), f32x2_to_bf16x2(sum[2], sum[3]));
         }
         *reinterpret_cast<uint2*>(row + d) = p;              // (elements past the row's end are zeros)
     }
     __syncthreads();
-    for (int ob = wv; ob < n_ob; ob += 8) {
-        if (ob != wv) ask(ob);
+    for (int ob = ob0 + wv; ob < n_ob; ob += 8) {
+        if (ob != ob0 + wv) {
+            ask(ob);
+            ask_gate(ob);
+        }
         f32x4_t y = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int k = 0; k < VK; ++k) {
-            frag16 x;
-            x.u = *reinterpret_cast<const uint4*>(row + 32 * k + 8 * g);
-            y = mfma_16x16x32(f[k], x, y);
+            frag16 in;
+            in.u = *reinterpret_cast<const uint4*>(row + 32 * k + 8 * g);
+            y = mfma_16x16x32(f[k], in, y);
         }
         if (c == 0) {                                        // all columns are the same row: outputs 16 ob + 4 g + e
 #pragma unroll
@@ -293,11 +314,28 @@ __global__ __launch_bounds__(512) void latent_values_kernel(LatentValuesArgs A) 
                 const int n = 16 * ob + 4 * g + e;
                 if (n >= out) continue;
                 float v = y[e];
-                if (A.gate) v *= 1.0f / (1.0f + expf(-A.gate[(size_t)r * A.ldg + (size_t)h * out + n]));
+                if (A.gate) v *= 1.0f / (1.0f + expf(-gate[e]));
                 A.y[(size_t)r * A.ldy + (size_t)h * out + n] = f32_to_bf16(v);
             }
         }
     }
+}
+
+template <int VK>
+static void launch_latent_values(const LatentValuesArgs& A, unsigned wgs, hipStream_t stream) {
+    // As many workgroups a (row, head) as leave one a compute unit: what a compute unit takes from memory bounds them, and each merges the
+    // shares for itself.  us, 1, 2, 4 and 8 of them (16 heads of 512 by 128): 1 row of 64 shares 7.0 5.5 4.6 4.2, 4 rows 7.2 5.7 4.9
+    // 7.4, 6 rows of 42 shares 7.6 6.3 8.4 10.3, 16 rows of 16 shares 7.3 9.8 13.6 21.2.
+    const int blocks = (A.out + 15) / 16;
+    unsigned parts = 1;
+    while (2 * parts * wgs <= 256 && 2 * parts <= (unsigned)blocks) parts *= 2;
+    const dim3 grid(wgs, parts);
+    if (A.splits <= 4) latent_values_kernel<VK, 1><<<grid, 512, 0, stream>>>(A);
+    else if (A.splits <= 8) latent_values_kernel<VK, 2><<<grid, 512, 0, stream>>>(A);
+    else if (A.splits <= 16) latent_values_kernel<VK, 4><<<grid, 512, 0, stream>>>(A);
+    else if (A.splits <= 32) latent_values_kernel<VK, 8><<<grid, 512, 0, stream>>>(A);
+    else if (A.splits <= 48) latent_values_kernel<VK, 12><<<grid, 512, 0, stream>>>(A);
+    else latent_values_kernel<VK, 16><<<grid, 512, 0, stream>>>(A);
 }
 
 extern "C" int agave_latent_values(const float* part_o, const float* part_ml, int splits, const void* w, void* y, long ldy,
@@ -309,9 +347,9 @@ extern "C" int agave_latent_values(const float* part_o, const float* part_ml, in
     AGAVE_CHECK((long)rows * heads < 2147483647L, "latent_values: too many (row, head) pairs");
     if (rows == 0) return 0;
     LatentValuesArgs A{part_o, part_ml, splits, (const bf16*)w, (bf16*)y, ldy, gate, ldg, heads, vd, out};
-    if (vd <= 128) latent_values_kernel<4><<<rows * heads, 512, 0, stream>>>(A);
-    else if (vd <= 256) latent_values_kernel<8><<<rows * heads, 512, 0, stream>>>(A);
-    else latent_values_kernel<16><<<rows * heads, 512, 0, stream>>>(A);
+    if (vd <= 128) launch_latent_values<4>(A, rows * heads, stream);
+    else if (vd <= 256) launch_latent_values<8>(A, rows * heads, stream);
+    else launch_latent_values<16>(A, rows * heads, stream);
     AGAVE_LAUNCH_CHECK("latent_values");
     return 0;
 }

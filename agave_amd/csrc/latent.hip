@@ -263,9 +263,10 @@ __device__ __forceinline__ frag16 eight(const float* p) {
 // output columns (or, in a step of up to 16 tokens, those tokens and 256 columns); each of its four waves 16 tokens
 // against 64 columns, both operands straight from memory in the order v_mfma_f32_16x16x32_bf16 reads them (a lane's
 // eight neighbours along K are 16 bytes of a row; a 32-bit row is rounded on the way in).  The head's weights are small
-// and stay in the caches; what the kernel moves is the rows.  The trailing elements are copied, turned, by the
-// workgroups of the first column block, a thread a pair.
-template <typename XT>
+// and stay in the caches; what the kernel moves is the rows.  The trailing elements are copied, turned, a thread a pair, by the
+// workgroups of the first column block, and in a step of up to 16 tokens, which is bound by its ways to memory one after the
+// other, by workgroups of their own behind the last column block (16 heads, 6 tokens: 5.76 us before, 5.44 so).
+template <typename XT, int J>
 __device__ __forceinline__ void heads_product_tile(const HeadsProductArgs& A, int bx, int h, int bz) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
@@ -273,7 +274,7 @@ __device__ __forceinline__ void heads_product_tile(const HeadsProductArgs& A, in
     const bool few = A.n_tokens <= 16;
     const int wg_row0 = few ? 0 : bx * 64, wg_rows = few ? 16 : 64;
     const int row0 = few ? 0 : wg_row0 + wv * 16;
-    const int col0 = few ? (bz * 4 + wv) * 64 : bz * 64;
+    const int col0 = few ? (bz * 4 + wv) * 16 * J : bz * 64;
     const int K = A.K, n_out = A.n_out;
     const XT* x = (const XT*)A.x;
     const bf16* w = (const bf16*)A.w + (size_t)h * n_out * K;
@@ -282,39 +283,39 @@ __device__ __forceinline__ void heads_product_tile(const HeadsProductArgs& A, in
         int trow = row0 + c;
         trow = trow < A.n_tokens ? trow : A.n_tokens - 1;
         const XT* arow = x + (size_t)trow * A.ldx + (size_t)h * A.xs + 8 * g;
-        const bf16* brow[4];
+        const bf16* brow[J];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < J; ++j) {
             int col = col0 + 16 * j + c;
             col = col < n_out ? col : n_out - 1;
             brow[j] = w + (size_t)col * K + 8 * g;
         }
-        f32x4_t acc[4];
+        f32x4_t acc[J];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < J; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         // four steps along K at a time: their loads leave together (without conditions, from inside the row; a lane past the
         // row's end reads its start and is emptied), so a product is a few round trips to memory and not one per step
         for (int k0 = 0; k0 < K; k0 += 128) {
-            frag16 a[4], b[4][4];
+            frag16 a[4], b[4][J];
             bool in[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 in[u] = k0 + 32 * u + 8 * g < K;
                 const int at = in[u] ? k0 + 32 * u : -8 * g;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) b[u][j].u = *reinterpret_cast<const uint4*>(brow[j] + at);
+                for (int j = 0; j < J; ++j) b[u][j].u = *reinterpret_cast<const uint4*>(brow[j] + at);
                 a[u] = eight(arow + at);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 if (!in[u]) a[u].u = make_uint4(0, 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[j] = mfma_16x16x32(a[u], b[u][j], acc[j]);
+                for (int j = 0; j < J; ++j) acc[j] = mfma_16x16x32(a[u], b[u][j], acc[j]);
             }
         }
         // D[j]: the lane holds tokens row0 + 4 g + e4, column col0 + 16 j + c
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < J; ++j) {
             const int col = col0 + 16 * j + c;
             if (col >= n_out) continue;
 #pragma unroll
@@ -327,7 +328,7 @@ __device__ __forceinline__ void heads_product_tile(const HeadsProductArgs& A, in
             }
         }
     }
-    if (A.tail && bz == 0) {
+    if (A.tail && bz == (few ? (n_out + 64 * J - 1) / (64 * J) : 0)) {
         const Turn R = A.turn;
         const int rows = min(wg_rows, A.n_tokens - wg_row0), rest = A.tail - 2 * R.half;
         for (int i = threadIdx.x; i < rows * R.half; i += 256) {
@@ -350,24 +351,30 @@ __device__ __forceinline__ void heads_product_tile(const HeadsProductArgs& A, in
     }
 }
 
-template <typename XT>
+template <typename XT, int J>
 __global__ __launch_bounds__(256) void heads_product_mfma_kernel(HeadsProductArgs A) {
-    heads_product_tile<XT>(A, blockIdx.x, blockIdx.y, blockIdx.z);
+    heads_product_tile<XT, J>(A, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // A decode step of up to 16 tokens: grid (1, heads + tokens, column blocks).  The first `heads` rows of workgroups fold
 // the queries, the others (first column block) make the tokens' key/value rows.
-template <typename XT>
+template <typename XT, int J>
 __global__ __launch_bounds__(256) void latent_decode_rows_kernel(HeadsProductArgs A, LatentKv K, Turn R, float eps) {
     __shared__ float red[16];
     __shared__ float cs[2][MAX_TURNED];
     if ((int)blockIdx.y < A.heads) {
-        heads_product_tile<XT>(A, 0, blockIdx.y, blockIdx.z);
+        heads_product_tile<XT, J>(A, 0, blockIdx.y, blockIdx.z);
     } else if (blockIdx.z == 0) {
         const int t = blockIdx.y - A.heads;
         latent_kv_row<bf16>(K, R, t, A.tok_pos[t], eps, red, cs);
     }
 }
+
+// In a step of up to 16 tokens: whether a wave takes 16 columns instead of 64, so that a head's weights are spread over four times as
+// many compute units, whose ways to memory bound the kernel: up to two workgroups on each.  us, 64 columns and 16, K 128, 512 columns:
+// 16 heads 1 token 4.74 and 2.96, 6 tokens 5.34 and 3.36, 16 tokens 5.75 and 3.75; 8 tokens of 40 heads 5.60 and 4.56, 64 (512 workgroups)
+// 5.71 and 4.70, 128 7.29 and 7.50.
+static bool narrow_columns(int heads, int n_out) { return (long)heads * ((n_out + 63) / 64) <= 512; }
 
 static int check_heads_product(const HeadsProductArgs& A) {
     AGAVE_CHECK(A.n_tokens >= 0 && A.heads > 0 && A.n_out > 0 && A.K > 0 && A.tail >= 0, "heads_product: bad sizes N=%d heads=%d out=%d K=%d", A.n_tokens, A.heads, A.n_out, A.K);
@@ -393,10 +400,14 @@ extern "C" int agave_heads_product(int dtype, int x_f32, const void* x, long ldx
     if (check_heads_product(A)) return -1;
     if (n_tokens == 0) return 0;
     if (!plain && heads_product_on_matrix_cores(dtype, x_f32, A)) {
-        const dim3 grid = n_tokens <= 16 ? dim3(1, heads, (n_out + 255) / 256) : dim3((n_tokens + 63) / 64, heads, (n_out + 63) / 64);
+        const bool few = n_tokens <= 16, narrow = few && narrow_columns(heads, n_out);
+        const int cols = few && !narrow ? 256 : 64;
+        const dim3 grid(few ? 1 : (n_tokens + 63) / 64, heads, (n_out + cols - 1) / cols + (few && tail > 0));
         AGAVE_CHECK(grid.z <= 65535, "heads_product: too many columns");
-        if (x_f32) heads_product_mfma_kernel<float><<<grid, 256, 0, stream>>>(A);
-        else heads_product_mfma_kernel<bf16><<<grid, 256, 0, stream>>>(A);
+        if (x_f32 && narrow) heads_product_mfma_kernel<float, 1><<<grid, 256, 0, stream>>>(A);
+        else if (x_f32) heads_product_mfma_kernel<float, 4><<<grid, 256, 0, stream>>>(A);
+        else if (narrow) heads_product_mfma_kernel<bf16, 1><<<grid, 256, 0, stream>>>(A);
+        else heads_product_mfma_kernel<bf16, 4><<<grid, 256, 0, stream>>>(A);
     } else {
         const dim3 grid(n_tokens, heads);
         const size_t lds = (size_t)(K + tail) * sizeof(float);
@@ -427,9 +438,12 @@ extern "C" int agave_latent_decode_rows(const float* q, long ldq, const void* fo
     if (check_heads_product(A) || check_turn("latent_decode_rows", R, rot_dim) || check_kv("latent_decode_rows", K, AGAVE_BF16)) return -1;
     AGAVE_CHECK(agave_latent_decode_rows_ok(n_tokens, dim, rot_dim, (int)(ldq % 4)) && heads_product_on_matrix_cores(AGAVE_BF16, 1, A) && kvraw && tok_pos,
                 "latent_decode_rows: sizes or alignment that it does not take");
-    const dim3 grid(1, heads + n_tokens, (kv_rank + 255) / 256);
+    const bool narrow = narrow_columns(heads, kv_rank);
+    const int cols = narrow ? 64 : 256;
+    const dim3 grid(1, heads + n_tokens, (kv_rank + cols - 1) / cols + (rot_dim > 0));
     AGAVE_CHECK(grid.y <= 65535, "latent_decode_rows: too many heads");
-    latent_decode_rows_kernel<float><<<grid, 256, 0, stream>>>(A, K, R, eps);
+    if (narrow) latent_decode_rows_kernel<float, 1><<<grid, 256, 0, stream>>>(A, K, R, eps);
+    else latent_decode_rows_kernel<float, 4><<<grid, 256, 0, stream>>>(A, K, R, eps);
     AGAVE_LAUNCH_CHECK("latent_decode_rows");
     return 0;
 }

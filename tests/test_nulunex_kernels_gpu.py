@@ -276,6 +276,57 @@ def test_decode_attention_over_latent_rows(heads, kd, kv_rank, out, window, with
         assert rel(y[i], want[i]) < 1.5e-2, (before[i], rel(y[i], want[i]))
 
 
+@pytest.mark.parametrize("splits", [1, 4, 5, 8, 9, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("rows, heads, vd, out", [(1, 2, 48, 10), (3, 20, 256, 40), (9, 16, 512, 128), (17, 16, 272, 200)])
+def test_latent_shares_merged_and_multiplied(rows, heads, vd, out, splits):
+    """One to eight workgroups a (row, head), every number of shares a group of threads keeps, shares without a key.  The merged row is
+    rounded to bfloat16, the product's result too: half a unit in the last of eight places each."""
+    from agave_amd.ops import latent as L
+    from agave_amd.ops import library
+    from agave_amd.ops.kernels import ptr, stream
+    g = torch.Generator().manual_seed(splits + out)
+    part = torch.randn(rows, heads, splits, vd, generator=g)
+    ml = torch.stack([torch.randn(rows, heads, splits, generator=g) * 3, torch.rand(rows, heads, splits, generator=g) + 0.5], -1)
+    empty = torch.rand(rows, heads, splits, generator=g) < 0.3
+    empty[..., 0] = False
+    ml[..., 0][empty], ml[..., 1][empty], part[empty] = float("-inf"), 0.0, 0.0
+    w, gate = (torch.randn(heads, out, vd, generator=g) * vd ** -0.5).to(BF), torch.randn(rows, heads * out, generator=g)
+    y = torch.full((rows, heads * out + 3), 9.0, dtype=BF, device=DEV)
+    d = [t.to(DEV) for t in (part, ml, w, gate)]
+    library.call(L._attn(), "agave_latent_values", ptr(d[0]), ptr(d[1]), splits, ptr(d[2]), ptr(y), y.stride(0), ptr(d[3]), heads * out, rows, heads,
+                 vd, out, stream())
+    f = torch.exp2(ml[..., 0].to(F64) - ml[..., 0].to(F64).amax(-1, keepdim=True))
+    merged = (part.to(F64) * f[..., None]).sum(2) / (f * ml[..., 1].to(F64)).sum(-1)[..., None]
+    turned, opened = torch.einsum("rhd,hod->rho", merged, w.to(F64)), torch.sigmoid(gate.to(F64)).view(rows, heads, out)
+    most = torch.einsum("rhd,hod->rho", merged.abs(), w.to(F64).abs()) * opened
+    want = turned * opened
+    got = y[:, :heads * out].cpu().to(F64).view(rows, heads, out)
+    assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + (2.0 ** -9 + 2.0 ** -16) * most).all())
+    assert bool((y[:, heads * out:] == 9.0).all())
+
+
+@pytest.mark.parametrize("n", [1, 16, 17])
+@pytest.mark.parametrize("heads", [1, 64, 65])
+def test_folds_of_few_tokens(n, heads):
+    """16 or 64 columns a wave, turned elements from workgroups of their own: up to 512 workgroups and beyond, the largest step of few
+    tokens and the next.  Queries are rounded to bfloat16 on the way in, the result too."""
+    from agave_amd.ops import latent as L
+    K, n_out, rot = 40, 500, 8
+    g = torch.Generator().manual_seed(n + heads)
+    x, w = torch.randn(n, heads * (K + rot), generator=g), (torch.randn(heads, n_out, K, generator=g) * K ** -0.5).to(BF)
+    freq = torch.rand(rot // 2, generator=g).to(F64)
+    pos = torch.arange(n, dtype=torch.int32) * 7
+    y = torch.full((n, heads * (n_out + rot)), float("nan"), dtype=BF, device=DEV)
+    L.heads_product(x.to(DEV), w.to(DEV), y, heads, K + rot, n_out + rot, tail=rot, turn=L.Turn(freq.to(DEV)), tok_pos=pos.to(DEV))
+    got, x = y.cpu().to(F64).view(n, heads, -1), x.to(F64).view(n, heads, -1)
+    want, most = (torch.einsum("nhk,hok->nho", v, u) for v, u in ((x[..., :K], w.to(F64)), (x[..., :K].abs(), w.to(F64).abs())))
+    assert bool(((got[..., :n_out] - want).abs() <= 2.0 ** -8 * want.abs() + (2.0 ** -9 + 2.0 ** -16) * most).all())
+    angle = pos.to(F64)[:, None, None] * freq
+    a, b = x[..., K:K + rot // 2], x[..., K + rot // 2:]
+    turned = torch.cat([a * angle.cos() - b * angle.sin(), b * angle.cos() + a * angle.sin()], -1)
+    assert bool(((got[..., n_out:] - turned).abs() <= 2.0 ** -8 * turned.abs() + 2.0 ** -20 * (a.abs() + b.abs()).repeat(1, 1, 2)).all())
+
+
 @pytest.mark.parametrize("window", [5, 64, 65, 200])
 def test_a_key_at_the_windows_edge_of_the_decode_attention(window):
     """One row stands out by thirty in the score, just inside and just outside the window, at page borders and at the
