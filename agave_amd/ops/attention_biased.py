@@ -11,6 +11,7 @@ from typing import NamedTuple, Optional
 import torch
 
 from . import kernels, library
+from ..cache import PAGE
 from .kernels import _P, _I, _L, _F, _dev, _f32vec, _i32, _rows, dt, ptr, stream
 
 LIBRARY = "attention_biased"
@@ -138,7 +139,8 @@ def attention(q: torch.Tensor, out: torch.Tensor, gate: Optional[torch.Tensor], 
         if not one_row or workspace is None:
             splits = 1
         elif splits is None:
-            splits = decode_splits(n, n_kv, n_heads // n_kv, v_head_dim, width)
+            # (never more shares than pages that a token of this step, or of the recorded one's kind, may see)
+            splits = min(decode_splits(n, n_kv, n_heads // n_kv, v_head_dim, width), step.page_span(window) + -(-keep_first // PAGE))
         if not 1 <= splits <= 64:
             raise ValueError(f"attention: {splits} shares of a row (1 to 64)")
         if splits > 1:

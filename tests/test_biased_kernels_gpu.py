@@ -166,6 +166,20 @@ def test_a_rows_pages_shared_among_workgroups(shape, splits):
     assert 1 <= A.decode_splits(8, 1, 16, 512, 64) <= A.MAX_SPLITS and A.decode_splits(300, 4, 4, 128, 64) == 1
 
 
+@pytest.mark.parametrize("splits", [17, 33, 64])
+@pytest.mark.parametrize("heads, kv, hd, vd", [(8, 2, 64, 128), (4, 1, 96, 272)])
+def test_a_rows_pages_shared_among_many_workgroups(heads, kv, hd, vd, splits):
+    """More shares than the merging kernel asks for ahead, a value row longer than its workgroup: most shares without a page, and a
+    page of its own for every one of 17."""
+    from agave_amd.parts import Workspace
+    T = 1090
+    c = Case(heads, kv, hd, vd, None, 0, "none", True, True, T=T, seed=9)
+    c.rounded(torch.bfloat16)
+    ref = c.plain()
+    c.workspace, c.splits = Workspace(torch.device(DEV)), splits
+    close(c.run([(0, 70)] + [(t, t + 1) for t in range(70, 74)] + [(74, T - 4)] + cuts(T, T - 4, 1)[1:], torch.bfloat16), ref, torch.bfloat16, f"{splits} shares")
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_a_table_too_long_for_lds_is_read_from_memory(dtype):
     """A bias over distances up to 20,000: the table's row of a head does not fit the kernel's LDS allowance and is read
