@@ -35,7 +35,8 @@ def merges(n: int, n_experts: int, top: int, ff: int, hidden: int) -> bool:
     """Whether a step of ``n`` tokens takes a shared expert as one of ``n_experts`` + 1 of ``ff`` inner rows and ``hidden`` columns, of
     which a token chooses ``top``: two products and their starts and ends less, unless the shared expert's tiles, which has every
     token, make a round of workgroups more (2 on a compute unit in tiles of 128 rows, 3 in tiles of 64).  us, a whole
-    feed-forward, with it among them and apart: 16 of 2,048 by 2,048, 4 chosen, 1 token 49 and 57, 32 108 and 130, 64 136 and 124, 512
+    feed-forward (its pairs sorted, which up to 256 no longer are, some 7 us less on either side), with it among them and apart:
+    16 of 2,048 by 2,048, 4 chosen, 1 token 49 and 57, 32 108 and 130, 64 136 and 124, 512
     179 and 205, 700 240 and 201 (38 tiles of 128, 608 workgroups, and 32, 512), 1,024 255 and 281, 3,001 500 and 536; 8 of 1,536 by
     1,536 64 tokens 70 and 82, 2,048 186 and 170; 32 of 1,024 by 2,048 6 tokens 72 and 81, 48 117 and 114, 700 192 and 203, 1,300 252 and
     224; 4 of 4,096 by 4,096 48 tokens 160 and 142, 100 170 and 200, 400 242 and 228.  Over 24 numbers of tokens from 33 to 6,000 and
