@@ -496,23 +496,28 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_f32_ring_kernel(const float
 
 // ---------------------------------------------------------------- more rows, on the bfloat16 instructions
 // A float is the sum of three bfloat16 values exactly (24 bits are three times 8: the nearest bfloat16, the nearest of what is left, and
-// the rest), so a product of floats is the sum of nine exact products of pieces.  The six large ones are made here on
+// the rest) if its last bit is one that a bfloat16 can hold: not below 2^-133, where a float's go down to 2^-149.  So both operands are
+// cut as PIECES_UP times as large, and the sums brought down again (uncut so, rows of 2^-112, -116, -120 and -124 had errors of 2.4e-7,
+// 2.2e-6, 3.5e-5 and 5.6e-4).  A product of floats is then the sum of nine exact products of pieces.  The six large ones are made here on
 // v_mfma_f32_16x16x32_bf16, whose sums are 32-bit; the three left out are below 2^-24 of the product.  The large pieces' products have a
 // running sum of their own, the five corrections another.  That sum takes 32 products an instruction, the 32-bit
 // instruction two or four, and so rounds a sixteenth as often.
 // Bound by the multiply-adds and, where a stage's tiles are few, by their chain of loads, cuts and barriers.  us, the kernels above and
-// this one with its sums of slices: 777 rows by 10,752 x 2,048 324 and 229 (149 TFLOP/s; the 32-bit instructions reach 153 on the largest
-// products), by 2,048 x 5,376 170 and 108, by 2,048 x 2,048 73 and 52, by 3,072 x 2,048 121 and 77; 2,048 rows by 10,752 x 2,048 722 and
-// 443 (204 TFLOP/s); 64 rows 42 and 34, 59 and 25, 26 and 15, 26 and 18.  Root mean square of the error against 64 bits over that of
-// the result, in 1e-7: 2,048 columns 5.7 (rings) and 2.7 whole, 1.9 in two slices, 1.3 in four; 5,376 9.3 and 4.6, 3.2, 2.2.
-// A piece of an infinity or NaN is none of the two (and the largest floats round to an infinity): an element that comes out neither
-// finite is made again from the floats themselves.
+// this one with its sums of slices: 777 rows by 10,752 x 2,048 325 and 249 (137 TFLOP/s; the 32-bit instructions reach 153 on the largest
+// products), by 2,048 x 5,376 174 and 119, by 2,048 x 2,048 71 and 65, by 3,072 x 2,048 119 and 78; 2,048 rows by 10,752 x 2,048 728 and
+// 465 (194 TFLOP/s); 64 rows 41 and 38, 58 and 25, 25 and 15, 25 and 17.  Making the operands larger takes 2 to 3 % of it.  Root mean
+// square of the error against 64 bits over that of the result, in 1e-7: 2,048 columns 5.7 (rings) and 2.7 whole, 1.9 in two slices, 1.3
+// in four; 5,376 9.3 and 4.6, 3.2, 2.2.
+// A piece of an infinity or NaN is none of the two, and floats from 2^104 on and sums from 2^80 on leave 32 bits when they are made so much
+// larger: an element that does not come out finite is made again from the floats themselves, in 64 bits.
 // WM x WN = 2 x 2 waves make BM rows x BN columns of C.  A stage of 32 k is brought into registers a stage ahead, cut into pieces there
 // and put into LDS in the order the instruction reads its operands; two workgroups share a compute unit, and one cuts while the other
 // multiplies.
+#define PIECES_UP 0x1p24f
 struct Pieces { uint32_t u[3]; };                                 // two floats' pieces, largest first, side by side
 __device__ __forceinline__ Pieces pieces_of(float a, float b) {
     Pieces p;
+    a *= PIECES_UP, b *= PIECES_UP;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         p.u[i] = f32x2_to_bf16x2(a, b);
@@ -617,15 +622,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const float* __r
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const int n = n0 + (wn * NT + t) * 16 + 4 * g;
-            f32x4_t s = high[r][t] + low[r][t];
+            f32x4_t s = (high[r][t] + low[r][t]) * (1.0f / (PIECES_UP * PIECES_UP));
             if (m >= M || n >= N) continue;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (!(__builtin_fabsf(s[e]) < __builtin_inff()) && n + e < N) {
-                    float again = 0.f;
+                    double again = 0.0;
                     const float *pa = A + (size_t)m * lda, *pw = W + (size_t)(n + e) * ldw;
-                    for (int k = st0 * 32; k < min(st_end * 32, K); ++k) again = fmaf(pa[k], pw[k], again);
-                    s[e] = again;
+                    for (int k = st0 * 32; k < min(st_end * 32, K); ++k) again = fma((double)pa[k], (double)pw[k], again);
+                    s[e] = (float)again;
                 }
             float* dst = C + (size_t)m * ldc + n;
             if (fours && n + 4 <= N) {

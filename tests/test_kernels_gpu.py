@@ -1442,6 +1442,33 @@ def test_gemm_slices(K, tile, m, n, k, z):
     assert abs(float(got[3, n - 1] / want[3, n - 1]) - 1) <= (k + 2) * 2.0 ** -24       # (the large product outweighs the others)
 
 
+# Small floats have bits below the last one that a bfloat16 piece can hold (2^-133): from some 2^-110 on either operand's, down to the
+# numbers without an exponent, and beside them in the same row some whose pieces leave 32 bits when they are made larger.
+@pytest.mark.parametrize("tile", [(128, 128), (64, 128), (128, 64), (64, 64)])
+@pytest.mark.parametrize("power", [-100, -112, -118, -126, -140])
+@pytest.mark.parametrize("small", ["x", "w", "a row of either"])
+def test_gemm_slices_of_small_floats(K, tile, power, small):
+    m, n, k, z = 70, 136, 260, 2
+    g = torch.Generator(device=DEV).manual_seed(-power)
+    x, w = torch.randn(m, k, device=DEV, generator=g), torch.randn(n, k, device=DEV, generator=g)
+    down = lambda t: (t.double() * 2.0 ** power).float()
+    if small == "x":
+        x = down(x)
+    elif small == "w":
+        w = down(w)
+    else:
+        x[5], w[7, ::2] = down(x[5]), down(w[7, ::2])
+        x[9, 3], w[11, 4] = 2.0 ** 110, -2.0 ** 119
+    parts, plain = torch.full((z, m, n), float("nan"), device=DEV), torch.empty(m, n, device=DEV)
+    K.gemm_slices(x, w, parts, tile)
+    K.gemm_plain(x, w, plain)
+    ref, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # as above, and a product or a sum below 2^-126 is rounded to a whole number of 2^-149
+    off = (k + 2) * 2.0 ** -24 * size + (k + z) * 2.0 ** -150
+    assert bool(((parts.double().sum(0) - ref).abs() <= off).all()) and bool(((plain.double() - ref).abs() <= off).all())
+    assert float((parts.double().sum(0) - ref)[5].norm()) <= 1.1 * float((plain.double() - ref)[5].norm())
+
+
 @pytest.mark.parametrize("m,n,k", [(33, 2048, 2048), (64, 10752, 2048), (100, 512, 2048), (200, 2048, 5376), (700, 3072, 2048), (17, 2304, 9216)])
 def test_gemm_in_slices_is_as_exact_as_whole(K, m, n, k):
     """Where a product is made in slices its error against 64 bits is no larger than that of the kernels of the 32-bit instructions
