@@ -1258,19 +1258,23 @@ __global__ __launch_bounds__(256) void attn_biased_merge_kernel(const float* __r
     const float total = wave_sum(f == 0.f ? 0.f : l0 * f);
     const float inv = total > 0.f ? 1.0f / total : 0.f;
     const float weight = ms == -INFINITY ? -1.f : f;           // (a share without a key is left out whatever it holds)
-    for (int d = threadIdx.x; d < vd; d += blockDim.x) {
+    // (all lanes of a wave go round together, those past the last column too: their registers hold the shares' weights)
+    for (int d0 = 0; d0 < vd; d0 += blockDim.x) {
+        const int d = d0 + threadIdx.x;
         float acc = 0.f;
         for (int s0 = 0; s0 < splits; s0 += AHEAD) {
-            if (s0 > 0 || d >= (int)blockDim.x) ask(d, s0);
+            if (s0 > 0 || d0 > 0) ask(d, s0);
 #pragma unroll
             for (int j = 0; j < AHEAD; ++j) {
                 const float fs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), s0 + j));
                 acc = fs != -1.f && s0 + j < splits ? fmaf(x[j], fs, acc) : acc;
             }
         }
-        float y = acc * inv;
-        if (gate) y *= 1.0f / (1.0f + __expf(-bf16_to_f32(gate[(size_t)t * ldg + (size_t)h * vd + d])));
-        out[(size_t)t * ldo + (size_t)h * vd + d] = f32_to_bf16(y);
+        if (d < vd) {
+            float y = acc * inv;
+            if (gate) y *= 1.0f / (1.0f + __expf(-bf16_to_f32(gate[(size_t)t * ldg + (size_t)h * vd + d])));
+            out[(size_t)t * ldo + (size_t)h * vd + d] = f32_to_bf16(y);
+        }
     }
 }
 

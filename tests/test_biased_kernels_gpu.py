@@ -167,10 +167,10 @@ def test_a_rows_pages_shared_among_workgroups(shape, splits):
 
 
 @pytest.mark.parametrize("splits", [17, 33, 64])
-@pytest.mark.parametrize("heads, kv, hd, vd", [(8, 2, 64, 128), (4, 1, 96, 272)])
+@pytest.mark.parametrize("heads, kv, hd, vd", [(8, 2, 64, 128), (4, 1, 96, 272), (4, 1, 64, 80), (4, 1, 64, 16)])
 def test_a_rows_pages_shared_among_many_workgroups(heads, kv, hd, vd, splits):
-    """More shares than the merging kernel asks for ahead, a value row longer than its workgroup: most shares without a page, and a
-    page of its own for every one of 17."""
+    """More shares than the merging kernel asks for ahead, a value row longer than its workgroup, fewer columns in its last wave than
+    shares: most shares without a page, and a page of its own for every one of 17."""
     from agave_amd.parts import Workspace
     T = 1090
     c = Case(heads, kv, hd, vd, None, 0, "none", True, True, T=T, seed=9)
