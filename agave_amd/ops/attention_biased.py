@@ -22,9 +22,9 @@ MAX_SPLITS = 16
 
 
 def decode_splits(n_rows: int, n_kv: int, per: int, v_head_dim: int, table_width: int) -> int:
-    """How many workgroups share the pages of one (row, key head) in a step of one row a sequence: enough to have some
-    two hundred workgroups at work, never more than the longest sequence's pages give every wave one.  It depends on
-    nothing that changes from step to step, so a recorded step stays valid."""
+    """How many workgroups share the pages of one (row, key head) in a step of one row a sequence at most: enough to have
+    some two hundred workgroups at work, never more than a whole table's pages give every wave one.  It depends on
+    nothing that changes from step to step, so it sizes the buffer of their results."""
     waves = 8 if v_head_dim <= 128 else 4
     groups = max(1, n_rows * n_kv * ((per + 15) // 16))
     return max(1, min(MAX_SPLITS, 192 // groups, -(-table_width // waves)))
@@ -99,8 +99,8 @@ def attention(q: torch.Tensor, out: torch.Tensor, gate: Optional[torch.Tensor], 
     that is a multiple of 16, up to 576 and 512) run on the matrix cores, everything else (and everything with
     ``force_plain``) on the plain kernel, which reads either order.  With a ``workspace`` (something with
     ``get(name, rows, cols, dtype)``) a step of one row a sequence may share a row's pages among several workgroups,
-    whose partial results a second kernel merges (``splits``: how many; None: :func:`decode_splits`).  ``chunk`` C: a
-    token also sees only keys j with j // C == p // C.  ``softcap`` > 0: the scaled score becomes softcap * tanh(score /
+    whose partial results a second kernel merges (``splits``: how many; None: :func:`decode_splits`, and no more than there are
+    pages that a token of this step may see).  ``chunk`` C: a token also sees only keys j with j // C == p // C.  ``softcap`` > 0: the scaled score becomes softcap * tanh(score /
     softcap) before the bias is added."""
     if chunk is not None and (chunk < 1 or keep_first):
         raise ValueError("attention: a chunk has at least one position and goes without kept first positions")
@@ -136,15 +136,18 @@ def attention(q: torch.Tensor, out: torch.Tensor, gate: Optional[torch.Tensor], 
         max_rows = max(b - a for a, b in zip(step.cu[:-1], step.cu[1:]))
         one_row = 1 if (step.is_decode and step.n_tokens == step.n_seqs) else 0
         parts = None
+        most = splits
         if not one_row or workspace is None:
             splits = 1
         elif splits is None:
             # (never more shares than pages that a token of this step, or of the recorded one's kind, may see)
-            splits = min(decode_splits(n, n_kv, n_heads // n_kv, v_head_dim, width), step.page_span(window) + -(-keep_first // PAGE))
+            most = decode_splits(n, n_kv, n_heads // n_kv, v_head_dim, width)
+            splits = min(most, step.page_span(window) + -(-keep_first // PAGE))
         if not 1 <= splits <= 64:
             raise ValueError(f"attention: {splits} shares of a row (1 to 64)")
         if splits > 1:
-            parts = workspace.get("attn_biased_parts", n * n_heads * splits, v_head_dim + 2, torch.float32)
+            # (as large as for the most shares: sequences that grow move no buffer, and recorded steps stay valid)
+            parts = workspace.get("attn_biased_parts", n * n_heads * most, v_head_dim + 2, torch.float32)
         library.call(_lib(), "agave_attn_biased_mfma", ptr(q), ldq, ptr(out), ldo, ptr(gate), ldg, ptr(k_pages), ptr(v_pages),
                      ptr(table), width, ptr(base), head, n_pages, ptr(step.tok_seq), ptr(step.tok_pos), ptr(step.cu_dev), n,
                      step.n_seqs, max_rows, one_row, n_heads, n_kv, head_dim, v_head_dim, float(scale), int(window or 0),

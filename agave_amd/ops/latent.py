@@ -244,8 +244,8 @@ def decode_attention_ok(kd: int, kv_rank: int, v_head_dim: int) -> bool:
 
 
 def decode_splits(n_rows: int, n_heads: int, table_width: int) -> int:
-    """How many workgroups share a row's pages: as many as put one on every compute unit, never more than there are
-    pages.  It depends on nothing that changes from step to step, so a recorded step stays valid."""
+    """How many workgroups share a row's pages at most: as many as put one on every compute unit, never more than the table
+    has pages.  It depends on nothing that changes from step to step, so it sizes the buffers of their results."""
     groups = max(1, n_rows * ((n_heads + 15) // 16))
     return max(1, min(MAX_SPLITS, table_width, 256 // groups))
 
@@ -256,7 +256,8 @@ def decode_attention(q: torch.Tensor, v_up: torch.Tensor, out: torch.Tensor, gat
     """A decode step (one row a sequence) over cached rows in operand order: for every row and head, the softmax of ``scale *
     q.row`` over the visible rows weighs their first ``kv_rank`` elements, and ``out[t, h] = v_up[h] @ that`` (``v_up`` [heads,
     v, kv_rank]), times sigmoid(gate) where a gate is given (float32).  ``window`` W: only positions p-W+1 .. p; ``sink``:
-    exp(sink_h) joins the denominator."""
+    exp(sink_h) joins the denominator.  ``splits``: how many workgroups share a row's pages (None: :func:`decode_splits`, and no
+    more than there are pages that a token of this step may see)."""
     _dev(q, v_up, out, gate, k_pages, v_pages, table, base, sink)
     n, bf = step.n_tokens, torch.bfloat16
     if not step.is_decode or n != step.n_seqs:
@@ -270,12 +271,15 @@ def decode_attention(q: torch.Tensor, v_up: torch.Tensor, out: torch.Tensor, gat
     width = kernels._check_table(table, base, None)
     _f32vec(sink, "sink", n_heads)
     _i32(step.tok_pos, "positions", n)
+    most = splits
     if splits is None:
+        most = decode_splits(n, n_heads, width)
         # (never more shares than pages that a token of this step, or of the recorded one's kind, may see: an empty share is a row of
         # zeros to write, to read and to add; 6 rows that may see 32 pages, 42 and 32 shares: 6.3 and 6.0 us for the values, 4 rows 64 and 32: 4.8 and 4.3)
-        splits = min(decode_splits(n, n_heads, width), step.page_span(window))
-    part_o = workspace.get("latent_parts", n * n_heads * splits, kv_rank, torch.float32)
-    part_ml = workspace.get("latent_parts_ml", n * n_heads * splits, 2, torch.float32)
+        splits = min(most, step.page_span(window))
+    # (as large as for the most shares: sequences that grow move no buffer, and recorded steps stay valid)
+    part_o = workspace.get("latent_parts", n * n_heads * most, kv_rank, torch.float32)
+    part_ml = workspace.get("latent_parts_ml", n * n_heads * most, 2, torch.float32)
     library.call(_attn(), "agave_latent_decode", ptr(q), ldq, ptr(k_pages), ptr(v_pages), ptr(table), width, ptr(base), n_pages,
                  ptr(step.tok_pos), n, n_heads, kd, kv_rank, float(scale), int(window or 0), ptr(sink), splits, ptr(part_o),
                  ptr(part_ml), stream())

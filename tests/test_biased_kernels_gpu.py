@@ -180,6 +180,21 @@ def test_a_rows_pages_shared_among_many_workgroups(heads, kv, hd, vd, splits):
     close(c.run([(0, 70)] + [(t, t + 1) for t in range(70, 74)] + [(74, T - 4)] + cuts(T, T - 4, 1)[1:], torch.bfloat16), ref, torch.bfloat16, f"{splits} shares")
 
 
+def test_a_growing_sequence_moves_no_buffer():
+    """More pages, more shares of a row: their results lie in the buffer that the first shared row has made, so that steps that were
+    recorded with its address stay valid."""
+    from agave_amd.parts import Workspace
+    T = 1200
+    c = Case(8, 2, 64, 128, None, 0, "none", False, False, T=T, seed=10)
+    c.rounded(torch.bfloat16)
+    c.workspace = Workspace(torch.device(DEV))
+    cache, planner = planner_for(c.key(), dtype=torch.bfloat16)
+    planner.fixed_width = [128]
+    got = c.run([(0, 9), (9, 10), (10, 70), (70, 71), (71, 300), (300, 301), (301, T - 1), (T - 1, T)], torch.bfloat16, cache, planner, cache.alloc_slot())
+    close(got, c.plain(), torch.bfloat16, "one row after 9, 70, 300 and 1,199")
+    assert c.workspace.generation == 0 and c.workspace.allocations == 1
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_a_table_too_long_for_lds_is_read_from_memory(dtype):
     """A bias over distances up to 20,000: the table's row of a head does not fit the kernel's LDS allowance and is read

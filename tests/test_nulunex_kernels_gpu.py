@@ -276,6 +276,33 @@ def test_decode_attention_over_latent_rows(heads, kd, kv_rank, out, window, with
         assert rel(y[i], want[i]) < 1.5e-2, (before[i], rel(y[i], want[i]))
 
 
+def test_a_growing_sequence_moves_no_buffer_of_latent_attention():
+    """More pages, more shares of a row: their results lie in the buffers that the first step has made, so that steps that were recorded
+    with their addresses stay valid."""
+    from agave_amd.cache import GroupKey
+    from agave_amd.ops import attention_biased as A
+    from agave_amd.ops import latent as L
+    heads, kd, kv_rank, out, T = 16, 40, 32, 16, 1400
+    g = torch.Generator().manual_seed(3)
+    cache, planner = planner_for(GroupKey(None, 1, kd, v_head_dim=kv_rank, layout="rows_vt"), slots=1, pages=30, dtype=BF)
+    slot, ws, rows = cache.alloc_slot(), workspace(), torch.randn(T, kd, generator=g).to(BF)
+    v_up = (torch.randn(heads, out, kv_rank, generator=g) * kv_rank ** -0.5).to(BF)
+    kp, vp, packed = cache.pages_of(0)
+    planner.fixed_width, at = [64], 0
+    for n in (9, 1, 60, 1, 300, 1, T - 373, 1):
+        step = planner.plan([slot], [[0] * n], "all")
+        r, (table, base) = rows[at:at + n].to(DEV), step.tables[0]
+        A.kv_append_rows(r, r[:, :kv_rank], kp, vp, table, base, 0, step, 1, kd, kv_rank, packed)
+        if n == 1:
+            q, y = torch.randn(1, heads * kd, generator=g).to(BF), torch.empty(1, heads * out, dtype=BF, device=DEV)
+            L.decode_attention(q.to(DEV), v_up.to(DEV), y, None, kp, vp, table, base, step, heads, kd, kv_rank, kd ** -0.5, None, None, ws)
+            want = plain_decode(q.to(F64).view(heads, kd), rows.to(F64), kd ** -0.5, None, None, v_up.to(F64), None, at)
+            assert rel(y[0], want) < 1.5e-2, at
+        planner.commit(step)
+        at += n
+    assert ws.generation == 0 and ws.allocations == 2
+
+
 @pytest.mark.parametrize("splits", [1, 4, 5, 8, 9, 16, 17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize("rows, heads, vd, out", [(1, 2, 48, 10), (3, 20, 256, 40), (9, 16, 512, 128), (17, 16, 272, 200)])
 def test_latent_shares_merged_and_multiplied(rows, heads, vd, out, splits):
