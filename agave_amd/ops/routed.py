@@ -70,6 +70,20 @@ def experts_plain(x: torch.Tensor, choice: torch.Tensor, w_gate: torch.Tensor, w
                  ptr(act_rows), ptr(y), n, top, e, ff, hidden, activation, float(p0), float(p1), stream())
 
 
+def _check_pairs(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: torch.Tensor, x: torch.Tensor,
+                 shared: Optional[torch.Tensor], top: int, shared_gate: Optional[torch.Tensor]) -> int:
+    """What is added up to rows like ``x``: the pairs' rows and the shared expert's, whose stride comes back."""
+    n, hidden = x.shape
+    _f32vec(shared_gate, "shared_gate", n)
+    if shared is not None and (shared.shape != x.shape or shared.dtype != x.dtype):
+        raise ValueError("combine: the shared expert's rows must have the input's shape and dtype")
+    if y is not None and (y.dtype != torch.float32 or not y.is_contiguous() or y.shape[1] != hidden or y.shape[0] < n * top):
+        raise ValueError("combine: y must be float32 [>= N * top, hidden]")
+    _i32(choice, "choice", n * top)
+    _i32(place, "place", n * top)
+    return _rows(shared, "shared") if shared is not None else 0
+
+
 def combine(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: torch.Tensor, weight: torch.Tensor,
             x: torch.Tensor, shared: Optional[torch.Tensor], out: torch.Tensor, top: int, n_experts: int,
             shared_gate: Optional[torch.Tensor] = None) -> None:
@@ -77,20 +91,11 @@ def combine(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: to
     choice is an identity expert, e >= n_experts) + shared[t], the latter times ``sigmoid(shared_gate[t])`` where a
     float32 logit per token is given."""
     _dev(y, place, choice, weight, x, shared, out, shared_gate)
-    _f32vec(shared_gate, "shared_gate", x.shape[0])
     n, hidden = x.shape
     ldx, ldo = _rows(x, "x"), _rows(out, "out")
     if out.shape != x.shape or out.dtype != x.dtype:
         raise ValueError("combine: out must have the input's shape and dtype")
-    lds = 0
-    if shared is not None:
-        lds = _rows(shared, "shared")
-        if shared.shape != x.shape or shared.dtype != x.dtype:
-            raise ValueError("combine: the shared expert's rows must have the input's shape and dtype")
-    if y is not None and (y.dtype != torch.float32 or not y.is_contiguous() or y.shape[1] != hidden or y.shape[0] < n * top):
-        raise ValueError("combine: y must be float32 [>= N * top, hidden]")
-    _i32(choice, "choice", n * top)
-    _i32(place, "place", n * top)
+    lds = _check_pairs(y, place, choice, x, shared, top, shared_gate)
     library.call(_lib(), "agave_routed_combine", dt(x), ptr(y), ptr(place), ptr(choice), ptr(weight), ptr(x), ldx, ptr(shared),
                  lds, ptr(shared_gate) if shared is not None else None, ptr(out), ldo, n, top, n_experts, hidden, stream())
 
@@ -115,7 +120,7 @@ class RoutedRows:
         these sizes and nothing was added up yet."""
         y, place, choice, weight, x, shared, _, top, n_experts, shared_gate = self.arguments
         n, e = h.shape
-        if self._rows is not None or e % 4 or e > 16384 or out.dtype != x.dtype or h.shape != x.shape:
+        if y is None or self._rows is not None or e % 4 or e > 16384 or out.dtype != x.dtype or h.shape != x.shape:
             return False
         for t in (h, y, shared, post_gain, out, pre_gain):
             if t is not None and (t.data_ptr() % 16 or (t.dim() == 2 and (t.stride(1) != 1 or t.stride(0) % 4))):
@@ -125,13 +130,9 @@ class RoutedRows:
         _dev(h, y, place, choice, weight, shared, shared_gate, post_gain, out, pre_gain)
         _f32vec(post_gain, "post_gain", e)
         _f32vec(pre_gain, "pre_gain", e)
-        _f32vec(shared_gate, "shared_gate", n)
-        if y.dtype != torch.float32 or not y.is_contiguous() or y.shape[1] != e or (place is None and y.shape[0] < n * top):
-            raise ValueError("routed rows: y must be float32 [>= N * top, hidden]")
-        _i32(choice, "choice", n * top)
-        _i32(place, "place", n * top)
-        library.call(_lib(), "agave_routed_norm", dt(out), ptr(h), ptr(y), ptr(place), ptr(choice), ptr(weight), top, n_experts, ptr(shared),
-                     _rows(shared, "shared") if shared is not None else 0, ptr(shared_gate) if shared is not None else None, ptr(post_gain),
+        lds = _check_pairs(y, place, choice, x, shared, top, shared_gate)
+        library.call(_lib(), "agave_routed_norm", dt(out), ptr(h), ptr(y), ptr(place), ptr(choice), ptr(weight), top, n_experts, ptr(shared), lds,
+                     ptr(shared_gate) if shared is not None else None, ptr(post_gain),
                      float(post_eps), ptr(out), out.stride(0), ptr(pre_gain), float(pre_eps), n, e, stream())
         return True
 

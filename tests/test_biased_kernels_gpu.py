@@ -616,10 +616,33 @@ def test_routed_rows_into_the_norm(n, E, top, hidden, dtype, post, pre_norm, sha
         routed.combine(d(y), d(place), d(choice), d(weight), d(x), d(sh) if shared else None, summed, top, E, d(gate) if shared and gated else None)
         kernels.residual_norm(plain_h, summed, d(gain) if post else None, 1e-5, plain, d(pre) if pre_norm else None, 1e-6)
         assert float((plain_h - hd).abs().max()) <= 4e-6 * float(want_h.abs().max())
+        # (their 32-bit rows differ by that, and an element next to the middle of two may come out as the other)
+        assert bool(((plain - out).double().abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 0.0) * out.double().abs() + 8e-6 * float(want.abs().max())).all())
     assert not r.norm_into(hd[:, :hidden - 1], None, 0.0, out, d(pre), 1e-6)
     got = r.rows().cpu().double()                   # whoever cannot take the pairs' rows gets them added up, once
     assert r.rows() is spare and float((got - b).abs().max()) <= (2.0 ** -8 if dtype == torch.bfloat16 else 4e-6) * float(b.abs().max())
     assert not r.norm_into(hd, None, 0.0, out, d(pre), 1e-6)
+
+
+def test_routed_rows_are_checked_before_the_norm_reads_them(monkeypatch):
+    """The norm that adds up pairs reads the shared rows as its own type and as many rows of pairs as there are places: other types
+    and fewer rows are refused, as by the kernel that only adds them up (no kernel runs here)."""
+    from agave_amd.ops import routed
+    n, top, E, e = 3, 2, 4, 64
+    calls = []
+    monkeypatch.setattr(routed.library, "call", lambda lib, fn, *args: calls.append(fn))
+    on = dict(device=DEV)
+    h, x, out = torch.zeros(n, e, **on), torch.zeros(n, e, dtype=torch.bfloat16, **on), torch.zeros(n, e, dtype=torch.bfloat16, **on)
+    choice, place, weight, y = torch.zeros(n * top, dtype=torch.int32, **on), torch.zeros(n * top, dtype=torch.int32, **on), torch.ones(n * top, **on), torch.zeros(n * top, e, **on)
+
+    def into(y=y, place=place, shared=None, gate=None):
+        return routed.RoutedRows(y, place, choice, weight, x, shared, torch.empty_like(x), top, E, gate).norm_into(h, None, 0.0, out, None, 0.0)
+    assert into() and into(place=None) and into(shared=x.clone()) and calls == ["agave_routed_norm"] * 3
+    for wrong in (dict(shared=x.float()), dict(shared=x[:2]), dict(shared=torch.zeros(n, e + 8, dtype=torch.bfloat16, **on)), dict(y=y[:5]),
+                  dict(y=y[:5], place=None), dict(y=y.bfloat16()), dict(shared=x.clone(), gate=torch.zeros(2, **on))):
+        with pytest.raises((ValueError, TypeError)):
+            into(**wrong)
+    assert not into(y=None) and len(calls) == 3
 
 
 @pytest.mark.parametrize("n,E,top,ff,hidden", [(1, 5, 2, 1024, 2048), (6, 16, 4, 2048, 1056), (40, 3, 2, 1024, 1024), (3, 4, 4, 4096, 1024)])
