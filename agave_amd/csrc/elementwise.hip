@@ -6,6 +6,7 @@
 // Reference formulas: src/backend/kernels/cpu/norm.zig:7-40 (x * 1/sqrt(mean x^2 + eps) * g),
 // src/backend/kernels/cpu/rope.zig:11-48 (split-half pairs), src/models/gemma3.zig:884-902
 // (position scaled before the angle), src/backend/kernels/cpu/activation.zig:69-113 (tanh GELU).
+#include <climits>
 #include "common_impl.h"
 #include "gate_act.h"
 #include "qk_rope.h"
@@ -724,9 +725,9 @@ __global__ void qk_norm_rope_kv_kernel(const T* q, long ldq, const T* __restrict
 // a head (12 times the same angles at 4B sizes), and stores of single elements to places 16 bytes apart.  Here a lane holds E
 // neighbours of the row's lower half and the E they rotate with (head sizes 128 and 256, all of a head rotated or nothing), so a row
 // comes and leaves in two pieces of 2 E bytes, which is how key tiles are made up, and angles are worked out once for four heads.
-// All of a wave's rows are asked for at its start.  Values: four aligned positions lie side by side in a value tile, so the group's
-// first token stores all four where the step holds them (the next three rows, of the same sequence); a position outside of a whole
-// group is stored alone.
+// All of a wave's query or key rows are asked for at its start.  Values: four aligned positions lie side by side in a value tile, so the
+// group's first token stores all four where the step holds them (the next three rows, of the same sequence); positions outside of
+// whole groups are stored alone or as two.
 // Bound by its chain of loads up to some 700 tokens and by memory beyond.  us, above and here, 8 query and 4 key heads of 256, rows from
 // memory: 150 tokens 4.1 and 4.5, 256 4.8 and 4.6, 509 7.2 and 4.9, 2,048 17.5 and 10.0, 8,192 62.3 and 35.9 (134 MB, 3.7 TB/s).
 template <int E> struct QkPiece { uint32_t u[E / 2]; };
@@ -860,30 +861,72 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_tokens_kernel(const bf16*
     for (int o = 1; o < 4; ++o) near_ok = (ahead(near_pos, o) == near_pos + o) & (ahead(near_seq, o) == near_seq) & near_ok;
     const unsigned near_leads = (unsigned)__ballot(near_ok) & 0x7f;             // bit i: row t0 - 3 + i leads a whole group of four
     const unsigned leads = near_leads >> 3, led = (near_leads << 1 | near_leads << 2 | near_leads << 3) >> 3;
-    for (int j = 0; j < 4 && t0 + j < N; ++j) {
-        const bool leading = (leads >> j) & 1;
-        if (!leading && ((led >> j) & 1)) continue;         // the group's first token stores it
-        const int page = __builtin_amdgcn_readlane(pg, 16 * j), rj = __builtin_amdgcn_readlane(p, 16 * j) % AGAVE_PAGE, r32 = rj & 31;
-        if (page < 0) continue;
-        const int in_page = ((rj >> 5) * 64 + 16 * ((r32 & 15) >> 2)) * 8 + (r32 & 3) + ((r32 >> 4) << 2);
-        uint32_t two[E][4];
+    // a token's page of values (none: -1), and its place in a piece of them
+    auto place = [&](int j, int& page) {
+        page = __builtin_amdgcn_readlane(pg, 16 * j);
+        const int rj = __builtin_amdgcn_readlane(p, 16 * j) % AGAVE_PAGE, r32 = rj & 31;
+        return ((rj >> 5) * 64 + 16 * ((r32 & 15) >> 2)) * 8 + (r32 & 3) + ((r32 >> 4) << 2);
+    };
+    if (leads) {                                            // one of these four tokens, its group and the next three rows
+        const int j = __ffs(leads) - 1;
+        int page;
+        const int in_page = place(j, page);
+        if (page >= 0) {
+            uint32_t two[E][4];
 #pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const bf16* src = v + (size_t)(t0 + j) * ldv + (run0 + i < runs ? run0 + i : runs - 1) * 128 + lane * 2;
+            for (int i = 0; i < E; ++i) {
+                const bf16* src = v + (size_t)(t0 + j) * ldv + (run0 + i < runs ? run0 + i : runs - 1) * 128 + lane * 2;
 #pragma unroll
-            for (int o = 0; o < 4; ++o) two[i][o] = *reinterpret_cast<const uint32_t*>(src + (leading ? o : 0) * ldv);
+                for (int o = 0; o < 4; ++o) two[i][o] = *reinterpret_cast<const uint32_t*>(src + o * ldv);
+            }
+#pragma unroll
+            for (int i = 0; i < E; ++i) {
+                if (run0 + i >= runs) continue;
+                const int at = (run0 + i) * 128 + lane * 2, head = at / HD, d = at % HD;        // this lane's two elements: d, d + 1 of a head
+                bf16* dst = v_pages + ((size_t)page * nkv + head) * (size_t)(HD * AGAVE_PAGE) + ((size_t)(d >> 4) * 128 + (d & 15)) * 8 + in_page;
+                *reinterpret_cast<uint2*>(dst) = make_uint2((two[i][0] & 0xffffu) | (two[i][1] << 16), (two[i][2] & 0xffffu) | (two[i][3] << 16));
+                *reinterpret_cast<uint2*>(dst + 8) = make_uint2((two[i][0] >> 16) | (two[i][1] & 0xffff0000u), (two[i][2] >> 16) | (two[i][3] & 0xffff0000u));
+            }
         }
+    }
+    // Tokens outside of whole groups: elements 16 bytes apart, so neighbouring lanes take neighbouring ones and a store touches half the
+    // lines, and an even position takes the next one along.
+    const unsigned alone = ~(leads | led) & 0xf & ((2u << min(3, N - 1 - t0)) - 1);
+    if (!alone) return;
+    const int pos0 = p, seq0 = b;
+    uint16_t x[4][E][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if ((alone >> j) & 1) {
+#pragma unroll
+            for (int i = 0; i < E; ++i)
+#pragma unroll
+                for (int o = 0; o < 2; ++o)
+                    x[j][i][o] = reinterpret_cast<const uint16_t*>(v)[(size_t)(t0 + j) * ldv + (run0 + i < runs ? run0 + i : runs - 1) * 128 + 64 * o + lane];
+        }
+    bool taken = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (!((alone >> j) & 1)) continue;
+        if (taken) {
+            taken = false;
+            continue;
+        }
+        const int pj = __builtin_amdgcn_readlane(pos0, 16 * j);
+        if (j < 3) taken = ((alone >> j) & 2) && pj % 2 == 0 && __builtin_amdgcn_readlane(pos0, 16 * (j + 1)) == pj + 1 &&
+                           __builtin_amdgcn_readlane(seq0, 16 * (j + 1)) == __builtin_amdgcn_readlane(seq0, 16 * j);
+        int page;
+        const int in_page = place(j, page);
+        if (page < 0) continue;
 #pragma unroll
         for (int i = 0; i < E; ++i) {
             if (run0 + i >= runs) continue;
-            const int at = (run0 + i) * 128 + lane * 2, head = at / HD, d = at % HD;            // this lane's two elements: d, d + 1 of a head
-            bf16* dst = v_pages + ((size_t)page * nkv + head) * (size_t)(HD * AGAVE_PAGE) + ((size_t)(d >> 4) * 128 + (d & 15)) * 8 + in_page;
-            if (leading) {
-                *reinterpret_cast<uint2*>(dst) = make_uint2((two[i][0] & 0xffffu) | (two[i][1] << 16), (two[i][2] & 0xffffu) | (two[i][3] << 16));
-                *reinterpret_cast<uint2*>(dst + 8) = make_uint2((two[i][0] >> 16) | (two[i][1] & 0xffff0000u), (two[i][2] >> 16) | (two[i][3] & 0xffff0000u));
-            } else {
-                dst[0].x = (uint16_t)two[i][0];
-                dst[8].x = (uint16_t)(two[i][0] >> 16);
+#pragma unroll
+            for (int o = 0; o < 2; ++o) {
+                const int at = (run0 + i) * 128 + 64 * o + lane, head = at / HD, d = at % HD;
+                bf16* dst = v_pages + ((size_t)page * nkv + head) * (size_t)(HD * AGAVE_PAGE) + ((size_t)(d >> 4) * 128 + (d & 15)) * 8 + in_page;
+                if (taken) *reinterpret_cast<uint32_t*>(dst) = x[j][i][o] | (uint32_t)x[j < 3 ? j + 1 : 3][i][o] << 16;
+                else dst->x = x[j][i][o];
             }
         }
     }
@@ -913,7 +956,7 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
                                      float eps_q, float eps_k, const float* inv_freq, int rot_half, float pos_scale,
                                      const int* tok_seq, const int* tok_pos, void* k_pages, void* v_pages,
                                      const int* table, int width, const int* base, int n_pages, int N, int nh,
-                                     int nkv, int hd, int packed, hipStream_t stream) {
+                                     int nkv, int hd, int packed, int apart, hipStream_t stream) {
     AGAVE_CHECK(N >= 0 && nh >= 0 && nkv >= 0 && hd > 0, "qk_norm_rope_kv: bad sizes N=%d nh=%d nkv=%d hd=%d", N, nh, nkv, hd);
     AGAVE_CHECK(hd <= QK_HD_MAX, "qk_norm_rope_kv: head_dim %d exceeds the supported maximum %d", hd, QK_HD_MAX);
     AGAVE_CHECK(rot_half >= 0 && 2 * rot_half <= hd, "qk_norm_rope_kv: rotary_dim %d exceeds head_dim %d", 2 * rot_half, hd);
@@ -927,12 +970,23 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
     const long units = (long)N * (nh + nkv);
     if (units == 0) return 0;
     AGAVE_CHECK(units < (1L << 31) - 4, "qk_norm_rope_kv: %ld (token, head) pairs exceed what one launch takes", units);
-    // The line lies where both took the same time (256 tokens of 12 heads); below it a wave a head is the shorter chain.
+    // (token, head) pairs from which a wave takes four tokens.  Below, a wave a head is the shorter chain; with heads of 128 it has half
+    // as many elements to go through, and without values half as many stores.  Tokens outside of whole groups of four positions cost
+    // more stores here, from one compute unit for four of them: a prompt's last three with eight and more key heads, the first and
+    // last of every sequence of a batch; with fewer than eight tokens a sequence most are such.  us, that kernel and this one:
+    // 8 + 4 heads of 256, 256 tokens 4.8 and 4.7; 16 + 8, 143 tokens 5.7 and 5.9, 215 6.9 and 5.8; 1 + 1, 1,540 4.6 and 5.3, 2,350 6.0 and 5.6;
+    // 16 + 4 of 128, 171 tokens 4.2 and 4.3, 255 4.8 and 4.5; 32 + 16, 75 4.3 and 4.6, 111 5.1 and 4.7; 16 heads of 128 alone, 339 tokens 3.97 and
+    // 3.82, one head 6,151 4.1 and 4.1; sequences of 55 tokens, 8 + 4 heads of 256, 417 tokens 6.9 and 8.7, 667 9.0 and 8.1; of 21, 16 + 8,
+    // 334 tokens 9.4 and 9.5, 584 12.8 and 10.8; of 3, 8 + 4, 1,167 12.7 and 13.0.
+    long line;
+    if (nkv == 0) line = hd == 256 ? 5120 : 6656;
+    else if (apart > 0) line = N < 8L * apart ? LONG_MAX : 9216;
+    else line = hd == 256 && nkv <= 4 && nh > 1 ? 3072 : nkv <= 8 ? 4736 : 5120;
     const uintptr_t addresses = (nh ? (uintptr_t)q | (uintptr_t)q_out : 0) | (nkv ? (uintptr_t)k | (uintptr_t)v | (uintptr_t)k_pages | (uintptr_t)v_pages : 0) |
                                 (uintptr_t)q_gain | (uintptr_t)k_gain | (uintptr_t)(rot_half ? inv_freq : nullptr);
     const long strides = (nh ? ldq | ldqo : 0) | (nkv ? ldk | ldv : 0);
     if (dtype == AGAVE_BF16 && (packed || nkv == 0) && (hd == 128 || hd == 256) && (rot_half == 0 || rot_half == hd / 2) &&
-        units >= 3072 && addresses % 16 == 0 && strides % 8 == 0) {
+        units >= line && addresses % 16 == 0 && strides % 8 == 0) {
         const long waves = (long)((N + 3) / 4) * ((nh + 3) / 4 + 2 * ((nkv + 3) / 4));
         const int grid = (int)(8 * (((waves + 3) / 4 + 7) / 8));
 #define QK_TOKENS(E_)                                                                                                           \

@@ -24,6 +24,12 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages
                        most_keys=step.max_len if step.fixed_span is None else PAGE * step.fixed_span)
 
 
+def tokens_apart(step) -> int:
+    """How a step's tokens lie for the kernels that take them four positions at a time: 0 if they are one sequence's and begin at
+    a multiple of four, else of how many sequences they are."""
+    return 0 if step.n_seqs == 1 and step.pos0[0] % 4 == 0 else step.n_seqs
+
+
 def qk_attention(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.Tensor], q_rot: torch.Tensor,
                  out: torch.Tensor, q_gain, k_gain, eps_q: float, eps_k: float, inv_freq, pos_scale: float,
                  k_pages: torch.Tensor, v_pages: torch.Tensor, table: torch.Tensor, base: torch.Tensor, step,
@@ -39,6 +45,6 @@ def qk_attention(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.T
                                                v_pages, table, base, step, n_heads, n_kv, head_dim, scale, window,
                                                partials_ok=partials_ok)
     kernels.qk_norm_rope_kv(q, k, v, q_rot, q_gain, k_gain, eps_q, eps_k, inv_freq, pos_scale, step.tok_seq,
-                            step.tok_pos, k_pages, v_pages, table, base, n_heads, n_kv, head_dim, packed)
+                            step.tok_pos, k_pages, v_pages, table, base, n_heads, n_kv, head_dim, packed, tokens_apart(step))
     attention(q_rot, out, k_pages, v_pages, table, base, step, n_heads, n_kv, head_dim, scale, window, packed)
     return None

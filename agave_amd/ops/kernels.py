@@ -25,7 +25,7 @@ _SIGNATURES = {
         "agave_norm_of_sum": [_I, _P, _P, _L, _I, _L, _F, _P, _P, _F, _P, _L, _P, _F, _I, _I, _P],
         "agave_residual_layernorm": [_I, _P, _P, _L, _I, _L, _P, _P, _F, _P, _L, _P, _P, _F, _P, _I, _I, _P, _P],
         "agave_qk_norm_rope_kv": [_I, _P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _F, _F, _P, _I, _F,
-                                  _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _P],
+                                  _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P],
         "agave_geglu": [_I, _P, _L, _P, _L, _P, _L, _I, _I, _P],
         "agave_gated_act": [_I, _I, _F, _F, _P, _L, _P, _L, _P, _L, _I, _I, _P],
         "agave_unary_act": [_I, _I, _F, _F, _P, _L, _P, _L, _I, _I, _P],
@@ -274,10 +274,11 @@ def qk_norm_rope_kv(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Opt
                     eps_q: float, eps_k: float, inv_freq: Optional[torch.Tensor], pos_scale: float,
                     tok_seq: torch.Tensor, tok_pos: torch.Tensor, k_pages: Optional[torch.Tensor],
                     v_pages: Optional[torch.Tensor], table: Optional[torch.Tensor], base: Optional[torch.Tensor],
-                    n_heads: int, n_kv: int, head_dim: int, packed: bool = False) -> None:
+                    n_heads: int, n_kv: int, head_dim: int, packed: bool = False, apart: int = 0) -> None:
     """Per-head RMSNorm of q and k, rotation, q to ``q_out`` and k, v into their cache pages.
     ``k`` None: only q is processed (a layer that reads another layer's cache).  ``packed``:
-    the pages are in the matrix cores' tile order."""
+    the pages are in the matrix cores' tile order.  ``apart``: of how many sequences the tokens are (0: of one, from a position on
+    that is a multiple of four); which kernel is the faster one hangs on it, the results do not."""
     _dev(q, k, v, q_out, q_gain, k_gain, inv_freq, tok_seq, tok_pos, k_pages, v_pages, table, base)
     n = tok_pos.numel()
     _i32(tok_pos, "tok_pos")
@@ -308,7 +309,7 @@ def qk_norm_rope_kv(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Opt
     library.call(lib("elementwise"), "agave_qk_norm_rope_kv", d, ptr(q), ldq, ptr(k), ldk, ptr(v), ldv, ptr(q_out),
                  ldqo, ptr(q_gain), ptr(k_gain), eps_q, eps_k, ptr(inv_freq), rot_half, pos_scale, ptr(tok_seq),
                  ptr(tok_pos), ptr(k_pages), ptr(v_pages), ptr(table), width, ptr(base), n_pages, n, nh, nkv,
-                 head_dim, 1 if (packed and k is not None) else 0, stream())
+                 head_dim, 1 if (packed and k is not None) else 0, int(apart), stream())
 
 
 def _check_pages(k_pages: torch.Tensor, v_pages: torch.Tensor, nkv: int, hd: int, dtype: torch.dtype,

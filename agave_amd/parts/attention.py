@@ -115,7 +115,7 @@ class Attention:
             if k is not None:
                 kernels.qk_norm_rope_kv(None, k_n, v, None, None, None, 0.0, 0.0, None, 1.0, step.tok_seq,
                                         step.tok_pos, k_pages, v_pages, table, base, 0, s.n_kv_heads, s.head_dim,
-                                        packed)
+                                        packed, attn_ops.tokens_apart(step))
         attn_ops.attention(q_out, ctx_out, k_pages, v_pages, table, base, step, s.n_heads, s.n_kv_heads,
                            s.head_dim, s.scale, s.window, packed)
         return self.o.forward(ctx_out, tag="attn_o", slices_ok=True)       # the block adds it to the residual stream

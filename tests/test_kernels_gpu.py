@@ -185,6 +185,10 @@ def test_qk_norm_rope_kv(K, dtype):
     (128, 16, 4, [(5, 1), (2, 2), (63, 190)], True, True),
     (128, 6, 1, [(1, 439)], True, False),
     (128, 16, 0, [(7, 193)], True, True),                            # a layer that reads another one's cache
+    (256, 5, 3, [(62, 3), (1, 701)], False, True),                   # (above every line of the rule)
+    (128, 16, 4, [(5, 1), (2, 2), (63, 301)], True, True),
+    (128, 6, 1, [(1, 739)], True, False),
+    (128, 16, 0, [(7, 493)], True, True),
 ])
 def test_qk_norm_rope_kv_of_many_tokens(K, hd, nh, nkv, seqs, gains, rotates):
     """Steps of many tokens over pages in tile order, which take a kernel of their own: against 64-bit rows (bfloat16 rounds to
@@ -230,6 +234,41 @@ def test_qk_norm_rope_kv_of_many_tokens(K, hd, nh, nkv, seqs, gains, rotates):
     written = torch.zeros(pages, 64, dtype=torch.bool)
     written[page, row] = True
     assert float(k_rows.float().abs().sum((1, 3))[~written].sum()) == 0 == float(v_rows.float().abs().sum((1, 3))[~written].sum())
+
+
+@pytest.mark.parametrize("hd,nh,nkv", [(256, 8, 4), (256, 3, 9), (128, 5, 5), (128, 32, 16)])
+@pytest.mark.parametrize("first", [512, 513, 514, 515])
+def test_qk_norm_rope_kv_of_a_windows_pages(K, hd, nh, nkv, first):
+    """A prompt's later piece on a layer with a window: the tables begin at a page of their own, a page is not there and one is no
+    page of the pool.  Sequences of many tokens and of few, begun at every place of a group of four, ended at each, two tokens of
+    one position after the other.  The kernel of many tokens against the one of few (a token's rows differ by the order of a
+    sum and by the sine's last bits: half a unit of bfloat16's eight places each); values and untouched rows are the same."""
+    g = torch.Generator().manual_seed(hd + nh + first)
+    seqs = [(first, 389), (first + 91, 1), (130, 2), (131, 2), (133, 3), (first + 2, 5), (77, 6), (192, 7), (63, 2), (70, 601 - first % 7)]
+    tok_seq = [b for b, (_, m) in enumerate(seqs) for _ in range(m)]
+    tok_pos = [p + i for p, m in seqs for i in range(m)]
+    n, base = len(tok_pos), [max(0, p // 64 - b % 2) for b, (p, _) in enumerate(seqs)]
+    width = max((p + m - 1) // 64 + 1 - a for (p, m), a in zip(seqs, base))
+    assert n * (nh + nkv) >= 9216 and n >= 8 * len(seqs)
+    pages = len(seqs) * width
+    table = torch.randperm(pages, generator=g).to(torch.int32).view(len(seqs), width)
+    table[0, 3], table[9, 2] = -1, pages
+    on = torch.randn(n, (nh + 2 * nkv) * hd, generator=g).bfloat16().to(DEV)
+    q, k, v = on[:, :nh * hd], on[:, nh * hd:(nh + nkv) * hd], on[:, (nh + nkv) * hd:]
+    gains = [(torch.randn(hd, generator=g) * 0.1 + 1).to(DEV) for _ in range(2)]
+    inv = torch.exp(-torch.arange(hd // 2) * (26.0 / hd)).float().to(DEV)
+    got = []
+    for apart in (len(seqs), n):                    # (fewer than eight tokens a sequence: the kernel of few tokens)
+        q_out = torch.empty(n, nh * hd, dtype=torch.bfloat16, device=DEV)
+        kp, vp = torch.full((pages, nkv, 64, hd), 3.0, dtype=torch.bfloat16, device=DEV), torch.full((pages, nkv, hd, 64), 3.0, dtype=torch.bfloat16, device=DEV)
+        K.qk_norm_rope_kv(q, k, v, q_out, *gains, 1e-6, 2e-6, inv, 0.125, _i32(tok_seq), _i32(tok_pos), kp, vp, table.to(DEV), _i32(base), nh, nkv, hd, True, apart)
+        got.append((q_out.double(), kp.double(), vp))
+    (q0, k0, v0), (q1, k1, v1) = got
+    assert torch.equal(v0, v1) and torch.equal(k0 == 3.0, k1 == 3.0)
+    near = lambda a, b: bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2e-4).all())
+    assert near(q0, q1) and near(k0, k1) and float((q0 != q1).double().mean()) < 0.01 and float((k0 != k1).double().mean()) < 0.01
+    there = torch.tensor([0 <= int(table[b, p // 64 - base[b]]) < pages for b, p in zip(tok_seq, tok_pos)], device=DEV)
+    assert 0 < int(there.sum()) < n and int((v0 != 3.0).sum()) == int((v[there] != 3.0).sum())
 
 
 @pytest.mark.parametrize("pos", [0, 1, 10, 100, 1000])

@@ -50,3 +50,11 @@ def test_a_shared_expert_of_a_small_test_goes_both_ways():
     """The sizes that the GPU test of the shared expert runs."""
     from agave_amd.parts.routed_ffn import merges
     assert {merges(n, 6, 2, 1024, 1024) for n in (1, 6, 40, 130, 700, 1010)} == {True, False}
+
+
+def test_how_a_steps_tokens_lie():
+    """The kernels that take four positions at a time are told whether a step is one sequence from a multiple of four on."""
+    from types import SimpleNamespace as Step
+    from agave_amd.ops.attention import tokens_apart
+    assert tokens_apart(Step(n_seqs=1, pos0=[0])) == 0 == tokens_apart(Step(n_seqs=1, pos0=[512]))
+    assert tokens_apart(Step(n_seqs=1, pos0=[153])) == 1 and tokens_apart(Step(n_seqs=3, pos0=[0, 0, 0])) == 3
