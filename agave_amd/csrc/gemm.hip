@@ -712,27 +712,37 @@ static const SplitShape SPLIT_SHAPES[4] = {
     {64, 128, 6, {1.16, 1.18, 1.22, 1.43, 1.44, 1.55, 2.23, 2.36, 3.27, 3.95, 4.75, 6.24}},
     {128, 64, 6, {1.11, 1.10, 1.15, 1.35, 1.38, 1.50, 2.16, 2.32, 3.24, 3.74, 4.64, 6.02}},
     {64, 64, 5, {0.76, 0.78, 0.81, 0.93, 0.96, 0.99, 1.39, 1.45, 1.75, 2.21, 2.88, 3.55}}};
+// (just past a whole number of tiles a unit some have one more, which is what the others then wait for: as long as the next measured load, or
+// with more than three as the next whole number.  135 rows by 10,896 x 4,888 in tiles of 64 x 64, 2.004 a unit: 206, taken for 2 of them 149)
 static double split_stage(const SplitShape& s, double tiles_a_unit) {
-    if (tiles_a_unit <= SPLIT_TILES[0]) return s.stage[0];
+    double t = tiles_a_unit;
+    if (t > 3) t = ceil(t);
+    else if (t > 2 && t < 2.5) t = 2.5;
+    else if (t > 1 && t < 1.25) t = 1.25;
+    if (t <= SPLIT_TILES[0]) return s.stage[0];
     for (int i = 1; i < 12; ++i)
-        if (tiles_a_unit <= SPLIT_TILES[i])
-            return s.stage[i - 1] + (s.stage[i] - s.stage[i - 1]) * (tiles_a_unit - SPLIT_TILES[i - 1]) / (SPLIT_TILES[i] - SPLIT_TILES[i - 1]);
-    return s.stage[11] * tiles_a_unit / SPLIT_TILES[11];
+        if (t <= SPLIT_TILES[i]) return s.stage[i - 1] + (s.stage[i] - s.stage[i - 1]) * (t - SPLIT_TILES[i - 1]) / (SPLIT_TILES[i] - SPLIT_TILES[i - 1]);
+    return s.stage[11] * t / SPLIT_TILES[11];
 }
 struct SplitPlan { int shape, slices; double us; };
+#define SLICES_GAIN 0.92                                          // slices' time with their sum is off by up to 8 %: they have to be that much faster
 // The fastest shape, with k shared out among up to max_slices workgroups where that pays for adding up the slices (4 bytes each of
-// them and the result at 3.5 TB/s, and a launch).
+// them and the result at 3.5 TB/s, and a launch).  Large operands come at 4 TB/s (24 rows by 10,752 x 4,096 in eight slices 45.0 us).
 static SplitPlan plan_split(int M, int N, int K, int max_slices) {
     SplitPlan best = {0, 1, 1e30};
     const int stages = (K + 31) / 32;
-    for (int i = 0; i < 4; ++i) {
-        const SplitShape& s = SPLIT_SHAPES[i];
-        const double tiles = (double)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-        for (int z = 1; z <= max_slices && (z == 1 || stages / z >= 8); z *= 2) {
-            double us = s.start + 0.95 * split_stage(s, tiles * z / COMPUTE_UNITS) * ((stages + z - 1) / z);
+    const double memory = ((double)M + N) * K * 4 / 4.0e6;
+    for (int z = 1; z <= max_slices && (z == 1 || stages / z >= 8); z *= 2) {
+        const double limit = z > 1 && best.slices == 1 ? 0.95 * best.us : best.us;     // (1,200 rows by 10,752 x 4,096 587 and 604 in two)
+        SplitPlan of_z = {0, z, limit};
+        for (int i = 0; i < 4; ++i) {
+            const SplitShape& s = SPLIT_SHAPES[i];
+            const double tiles = (double)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+            double us = s.start + std::max(0.95 * split_stage(s, tiles * z / COMPUTE_UNITS) * ((stages + z - 1) / z), memory);
             if (z > 1) us += 2.0 + (z + 1.0) * M * N * 4 / 3.5e6;
-            if (us < best.us) best = {i, z, us};
+            if (us < of_z.us) of_z.shape = i, of_z.us = us;
         }
+        if (of_z.us < limit) best = of_z;
     }
     return best;
 }
@@ -745,21 +755,35 @@ static void launch_split(const SplitPlan& plan, const float* A, long lda, const 
         default: return launch_split<64, 64>(A, lda, W, ldw, C, ldc, M, N, K, plan.slices, part_stride, stream);
     }
 }
-// The plan of a product in pieces, us 0 where the 32-bit instructions take it.  The rings' times are known (see ring_rows): less than
-// theirs.  Where groups of rows or the tiles above would take it: only in slices, from 1,024 columns and 33 rows (or 4,096 and 17) on.  us, those and
-// slices: 17 rows by 3,072 x 2,048 14.1 and 15.3, 48 rows 23.8 and 17.0; 17 rows by 2,048 x 5,376 31.7 and 23.2; 400 rows by 2,048 x 2,048 42.7
-// and 37.1; 512 by 1,024 x 512 11.9 and 14.3.
+// Microseconds that the 32-bit instructions take from 17 rows on: rings as ring_rows knows them, with a start for every tile after the other
+// (by the least squares of 98 sizes' logarithms, off by 7 %: 221 rows by 31,916 x 248 45.6, 760 by 776 x 5,784 106); a round of workgroups
+// of groups of rows or of tiles at least so much a 2,048 columns (rows a power of two apart, whose columns lie on the same channels, take
+// up to a third more).
+static double whole_us(int M, int N, int K, int rows) {
+    auto rounds = [](long wgs) { return (double)((wgs + COMPUTE_UNITS - 1) / COMPUTE_UNITS); };
+    const long rows64 = ((long)M + 63) / 64, cols64 = ((long)N + TN - 1) / TN;
+    if (rows != 0) {
+        const long n = (((long)M + rows - 1) / rows * (((long)N + 127) / 128) + COMPUTE_UNITS - 1) / COMPUTE_UNITS;
+        return 2.0 + (rows == 128 ? 7.2 : 2.4) * n + 0.9 * (rows == 128 ? 130.0 * n : n <= 5 ? RING_32[n] : 35.0 * n) * K / 2048;
+    }
+    double unit;
+    if (M > SKINNY_M && rows64 * cols64 >= COMPUTE_UNITS) unit = 36.5 * rounds(rows64 * cols64);
+    else if (M > SKINNY_M && ((long)M + 31) / 32 * cols64 >= COMPUTE_UNITS) unit = 36.0;
+    else unit = (M <= 32 ? 10.0 : M <= 48 ? 15.5 : 17.5) * rounds(rows64 * (((long)N + 15) / 16));
+    return 2.3 + unit * K / 2048;
+}
+// The plan of a product in pieces, us 0 where the 32-bit instructions take it: where they are faster, to within what the times above are
+// off.  Where groups of rows or the tiles above would take it only in slices, from 1,024 columns and 33 rows (or 4,096 and 17) on.  us,
+// those and slices with their sum: 17 rows by 4,096 x 4,096 24.8 and 26.1, by 2,048 23.6 and 19.8; 33 rows by 2,048 x 1,024 11.1 and 12.6, by
+// 2,048 x 2,048 20.0 and 14.0; 64 rows by 1,024 x 1,100 13.1 and 13.5; 150 rows by 6,144 x 2,048 (rings) 42.6 and 45.8; 300 by 2,048 x 1,024 22.6 and
+// 22.8; 400 by 2,048 x 2,048 42.8 and 34.2.
 static SplitPlan split_instead(int M, int N, int K, int max_slices) {
     SplitPlan plan = {0, 1, 0};
     if (M <= 16 || (M <= 32 && K < 4096)) return plan;
     const int rows = ring_rows(M, N);
+    if (rows == 0 && (K < 1024 || max_slices == 1)) return plan;
     plan = plan_split(M, N, K, max_slices);
-    if (rows != 0) {
-        const long n = (((long)M + rows - 1) / rows * (((long)N + 127) / 128) + COMPUTE_UNITS - 1) / COMPUTE_UNITS;
-        if (plan.us >= (rows == 128 ? 130.0 * n : n <= 5 ? RING_32[n] : 35.0 * n) * K / 2048) plan.us = 0;
-    } else if (K < 1024 || plan.slices == 1) {
-        plan.us = 0;
-    }
+    if ((rows == 0 && plan.slices == 1) || plan.us >= (plan.slices > 1 ? SLICES_GAIN : 0.95) * whole_us(M, N, K, rows)) plan.us = 0;
     return plan;
 }
 
