@@ -1034,14 +1034,16 @@ __global__ __launch_bounds__(256) void routed_product_mfma_kernel(const bf16* __
 // as it takes a vote a bit of the expert's number, and a tile is then led by every sixteenth pair of an expert, tiles counted in the
 // pairs' order.  The rows of either product are the pairs themselves, and there is no sorted list to wait for, neither its kernel nor
 // two loads one after the other at the start of both products.  us, sorting and both products, and so: 17 experts of 2,048 by
-// 2,048, 5 a row, 1 row 37.1 and 35.4, 6 rows 80.2 and 72.9, 16 rows 89.6 and 82.4, 48 rows 115.9 and 109.2; 32 of 1,024 by 2,048, 4 a row,
-// 23.9 and 16.0, 54.3 and 52.9, 72.6 and 66.1, 84.8 and 79.2; 8 of 4,096 by 4,096, 2 a row, 60.1 and 44.8, 141 and 134, 150 and 141, 177 and 169;
-// 256 of 1,024 by 1,024, 8 a row, 26.2 and 18.2, 58.2 and 59.5, 141 and 126, 32 rows 228 and 200.  A thread looks at one pair, which is the
+// 2,048, 5 a row, 1 row 37.2 and 35.4, 6 rows 93.4 and 76.7, 16 rows 89.6 and 81.6, 48 rows 114 and 100; 32 of 1,024 by 2,048, 4 a row,
+// 23.6 and 15.8, 53.5 and 47.7, 71.5 and 62.4, 86.1 and 79.2; 8 of 4,096 by 4,096, 2 a row, 59.5 and 44.1, 123 and 112, 149 and 141, 176 and 154;
+// 256 of 1,024 by 1,024, 8 a row, 22.7 and 14.5, 73.3 and 65.1, 133 and 118, 32 rows 211 and 185.  A thread looks at one pair, which is the
 // limit; more pairs are sorted as before, in a time that is little of theirs.
 #define FEW_PAIRS 256
-// The expert of tile `tile` (-1: no such tile) and in mine[16], of this wave, the pairs of its rows (-1: no such row).  LDS, 16-byte
-// pieces nobody else uses until all waves are back: `counts` 4 E + 6 words, `mine` the waves' rows `stride` words apart.
-__device__ __forceinline__ int few_tile(const int* __restrict__ choice, int P, int E, int tile, int* counts, int* mine, int stride) {
+// The expert of tile `tile` (-1: no such tile) and in mine[16], of this wave, the pairs of its rows (-1: no such row).  With `runs` > 0
+// `tile` is a workgroup's number among so many runs of every tile that there is, the first runs of all tiles first, and its own run
+// comes back in `run`.  LDS, 16-byte pieces nobody else uses until all waves are back: `counts` 4 E + 6 words, `mine` the waves' rows
+// `stride` words apart.
+__device__ __forceinline__ int few_tile(const int* __restrict__ choice, int P, int E, int tile, int runs, int& run, int* counts, int* mine, int stride) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool alone = P <= 64;                                   // (every wave looks at all pairs and needs no other)
     const int pair = alone ? lane : (int)threadIdx.x;
@@ -1066,18 +1068,21 @@ __device__ __forceinline__ int few_tile(const int* __restrict__ choice, int P, i
             if (valid) rank += counts[o * E + chosen];
     }
     const unsigned long long leaders = __ballot(valid && (rank & 15) == 0);
-    int first = 0, e = -1, base = 0;
+    int first = 0, e = -1, base = 0, all = __popcll(leaders);
     if (!alone) {
         if (lane == 0) counts[4 * E + w] = __popcll(leaders);
         __syncthreads();
-        int all = 0;
+        all = 0;
         for (int o = 0; o < 4; ++o) {
             if (o == w) first = all;
             all += counts[4 * E + o];
         }
-        if (tile >= all) return -1;
-    } else if (tile >= __popcll(leaders)) {
-        return -1;
+    }
+    all = __builtin_amdgcn_readfirstlane(all);
+    if (tile >= (runs ? all * runs : all)) return -1;
+    if (runs) {
+        run = tile / all;
+        tile -= run * all;
     }
     const unsigned long long leads = __ballot(((leaders >> lane) & 1) && first + __popcll(leaders & below) == tile);
     if (leads) {
@@ -1103,11 +1108,13 @@ __device__ __forceinline__ int few_tile(const int* __restrict__ choice, int P, i
     return __builtin_amdgcn_readfirstlane(e);
 }
 
+#define FEW_BY_COLUMN 0                                           // how workgroups go through tiles and runs of blocks (see launch_routed_few);
+#define FEW_BY_TILE -1                                            // more than 0: so many runs, of the tiles that there are
 template <int KQ, bool GATED, bool CHOSEN>
 __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* __restrict__ x, long ldx, const int* __restrict__ sorted_pair,
                                                                     const int* __restrict__ tile_expert, const uint4* __restrict__ w0,
                                                                     const uint4* __restrict__ w1, void* __restrict__ out_, int top, int n_out,
-                                                                    int act, int blocks, float p0, float p1, int P, int E) {
+                                                                    int act, int blocks, float p0, float p1, int P, int E, int tiles, int order) {
     constexpr int K = KQ * 128, KB = K / 32, NS = 8;
     static_assert(KQ % NS == 0, "a step's place in the ring is known where it is written");
     constexpr int COLS = GATED ? 16 : 32;
@@ -1116,12 +1123,18 @@ __global__ __launch_bounds__(256, 2) void routed_product_few_kernel(const bf16* 
     static_assert(sizeof(ring) >= (4 * ROUTE_MAX + 6) * sizeof(int), "the experts' counts fit the ring");
     // (CHOSEN: sorted_pair holds the choices; part's first half keeps the rows' pairs until its first sums)
     int* mine = reinterpret_cast<int*>(&part[0][0][0][0]);
-    const int e = CHOSEN ? few_tile(sorted_pair, P, E, blockIdx.x, reinterpret_cast<int*>(&ring[0][0][0]), mine, 512) : tile_expert[blockIdx.x];
+    int tile = blockIdx.x, run = blockIdx.y;
+    if (CHOSEN && order == FEW_BY_TILE) {                         // (what is left of the tiles lies in the last rows of the grid)
+        const int left = (int)blockIdx.y - tiles;
+        tile = left < 0 ? (int)blockIdx.y : left * (int)gridDim.x + (int)blockIdx.x;
+        run = left < 0 ? (int)blockIdx.x : (int)gridDim.x;
+    }
+    const int e = CHOSEN ? few_tile(sorted_pair, P, E, tile, order > 0 ? order : 0, run, reinterpret_cast<int*>(&ring[0][0][0]), mine, 512) : tile_expert[tile];
     if (e < 0) return;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const int row0 = blockIdx.x * 16, NBK = n_out / 16;
-    const int b0 = blockIdx.y * blocks, b1 = min(b0 + blocks, (n_out + COLS - 1) / COLS);
+    const int row0 = blockIdx.x * 16, NBK = n_out / 16;           // (not CHOSEN)
+    const int b0 = run * blocks, b1 = min(b0 + blocks, (n_out + COLS - 1) / COLS);
     if (b0 >= b1) return;
     long r = row0 + c;
     int out_row = row0 + 4 * g + w;                               // -1: not stored
@@ -1211,10 +1224,23 @@ static bool launch_routed_few(const void* x, long ldx, const int* sorted_pair, c
     // blocks 98.9, 4 (496) 93.7; eight of 4,096 by 4,096, 12 rows, 5 and 3 (416) 178, 4 and 2 (512) 205.
     int blocks = (int)(((long)live * all + 499) / 500);
     blocks = blocks < 1 ? 1 : blocks > 16 ? 16 : blocks;
-    const dim3 grid(max_tiles, (all + blocks - 1) / blocks);
+    // CHOSEN: column by column, as sorted tiles, where all places run at once.  Beyond, tile by tile, so that the workgroups with rows are
+    // the first to start; those without look at the choices too and were among them, and with as many places for tiles as a multiple of
+    // eight a tile's runs were all on one XCD.  What is less than `blocks` of a tile comes behind all of them and fills up a second
+    // round if there is one.  With 4,096 columns, run by run of the tiles that there are.  us, sorted, column by
+    // column, and so (means of six choices): eight of 96 of 1,024 by 2,048 a row, 8 rows 119, 122, 106; eight of 65 of 1,024 by 1,024, 6 rows 56.1,
+    // 55.8, 47.9; eight of 129 of 1,024 by 2,048, 12 rows 175, 167, 155; two of 32 of 2,048 by 4,096, 16 rows 199, 193, 185.
+    const int runs = (all + blocks - 1) / blocks, whole = all / blocks;
+    if ((long)max_tiles * runs >= 1L << 31) return false;
+    int order = FEW_BY_COLUMN;
+    dim3 grid(max_tiles, runs);
+    if (CHOSEN && (long)max_tiles * runs > 512) {
+        if (K == 4096) order = runs, grid = dim3(max_tiles * runs);
+        else order = FEW_BY_TILE, grid = dim3(whole, max_tiles + (runs > whole ? (max_tiles + whole - 1) / whole : 0));
+    }
     if (grid.y > 65535) return false;
 #define FEW_GO(KQ_) routed_product_few_kernel<KQ_, GATED, CHOSEN><<<grid, 256, 0, stream>>>((const bf16*)x, ldx, sorted_pair, tile_expert, (const uint4*)w0, \
-                                                                                            (const uint4*)w1, out, top, n_out, act, blocks, p0, p1, P, E)
+                                                                                            (const uint4*)w1, out, top, n_out, act, blocks, p0, p1, P, E, max_tiles, order)
     if (K == 1024) FEW_GO(8);
     else if (K == 2048) FEW_GO(16);
     else FEW_GO(32);

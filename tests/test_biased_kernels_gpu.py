@@ -673,8 +673,19 @@ def test_routed_few_pairs_in_tile_order(n, E, top, ff, hidden):
 def test_few_pairs_find_their_rows_from_the_choices(n, top, E, chosen):
     """Without a sorted list the same rows as with one, to the bit: pairs of one wave and of four, experts of none, one, 16, 17 and all
     pairs, choices that are no expert's (negative or past the last), whose rows stay as they are."""
+    _few_pairs_against_sorted_ones(n, top, E, chosen, 1024, 2048)
+
+
+@pytest.mark.parametrize("n,top,E,chosen", [(1, 2, 9, 9), (6, 5, 17, 17), (40, 2, 17, 18)])
+@pytest.mark.parametrize("ff,hidden", [(4096, 1024), (1024, 4096)])
+def test_few_pairs_of_long_rows(n, top, E, chosen, ff, hidden):
+    """4,096 columns, whose workgroups count the tiles that there are: all at once, more than run at once, two tiles an expert."""
+    _few_pairs_against_sorted_ones(n, top, E, chosen, ff, hidden)
+
+
+def _few_pairs_against_sorted_ones(n, top, E, chosen, ff, hidden):
     from agave_amd.ops import routed
-    ff, hidden, P = 1024, 2048, n * top
+    P = n * top
     g = torch.Generator().manual_seed(P + E)
     rnd = lambda *s: (torch.randn(*s, generator=g) * s[-1] ** -0.5).bfloat16().to(DEV)
     x, w = torch.randn(n, hidden, generator=g).bfloat16().to(DEV), [routed.pack_expert_weights(rnd(*s)) for s in ((E, ff, hidden), (E, ff, hidden), (E, hidden, ff))]
