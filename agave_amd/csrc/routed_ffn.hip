@@ -669,7 +669,8 @@ __global__ void routed_norm_kernel(float* __restrict__ h, const float* __restric
 #pragma unroll
             for (int i = 0; i < 4; ++i) b[v][i] = fmaf(sg, sv[v][i], b[v][i]);
     }
-    // (rounded as the row that routed_combine leaves, so that a step's results do not depend on which of the two it takes)
+    // (rounded as the row that routed_combine leaves: whether a step takes that kernel and the norm's or this one shows in the order
+    // of the norms' sums only)
 #pragma unroll
     for (int v = 0; v < VPT; ++v)
 #pragma unroll
@@ -716,9 +717,13 @@ extern "C" int agave_routed_norm(int dtype, float* h, const float* y, const int*
                 "routed_norm: rows must be aligned to 16 bytes");
     AGAVE_CHECK(dtype == AGAVE_F32 || dtype == AGAVE_BF16, "routed_norm: unknown dtype %d", dtype);
     if (N == 0) return 0;
-    // threads as residual_norm takes them: one float4 each in steps of few tokens, two (four) in steps of many
+    // threads as residual_norm takes them: one float4 each in steps of few tokens, two (four) in steps of many.  More than eight pairs
+    // of more than 2,048 columns go in twos with few tokens, too: two batches of eight float4 and 1,024 threads wait for one another
+    // (4,096 columns of nine pairs, 64 tokens 6.9 us, so 5.0; a kernel for the sum and one for the norm 7.3).  In twos five
+    // pairs a batch are as fast as eight for six to eight pairs but for 0.4 to 0.6 us of few tokens, and faster from some 300 tokens
+    // on (5,120 columns of eight, 800 tokens 31.0 and 33.4) and for five, nine and ten pairs.
     int threads;
-    if (e <= 1024 || (N <= 64 && e <= 4096)) threads = 64 * ((e / 4 + 63) / 64);
+    if (e <= 1024 || (N <= 64 && e <= (top > 8 ? 2048 : 4096))) threads = 64 * ((e / 4 + 63) / 64);
     else {
         const int per = e / 4 <= 2048 ? 2 : 4;
         threads = 64 * ((e / 4 + per * 64 - 1) / (per * 64));

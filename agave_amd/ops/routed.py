@@ -100,6 +100,16 @@ def combine(y: Optional[torch.Tensor], place: Optional[torch.Tensor], choice: to
                  lds, ptr(shared_gate) if shared is not None else None, ptr(out), ldo, n, top, n_experts, hidden, stream())
 
 
+def norm_adds_up(n: int, top: int, hidden: int) -> bool:
+    """Whether the norm of ``n`` tokens adds up ``top`` pairs each: a workgroup takes a token's rows, so with few tokens many and wide
+    ones take longer than in the kernel that spreads them over the chip and the norm's own.  us, those two and the one kernel: 16,384
+    columns of 64 pairs, 6 tokens 17.7 and 42, of 16 10.0 and 12.9, of 7 8.9 and 9.2, of 6 8.7 and 8.2; 8,192 of 16 8.2 and 9.0, of 10
+    7.6 and 6.2; 7,168 of 12 7.3 and 7.4 (one token); 4,096 of 64 14.5 and 13.6.  48 tokens: 16,384 of 24 20.9 and 21.7, 12,288 of 24
+    19.1 and 18.2; 300 tokens 5,120 of 64 84 and 88, of 32 36.0 and 36.7.  Over 17 widths, 14 numbers of pairs, one to 800
+    tokens and both types one within these lines was slower by more than 1 % (800 tokens, 4,608 of 16: 48.4 and 50.5)."""
+    return hidden <= 4096 or top * hidden <= 84_000 or (n >= 48 and top <= 24 and top * hidden <= 300_000)
+
+
 class RoutedRows:
     """A routed feed-forward's result that is still its pairs' rows: the arguments of :func:`combine`.  The norm that takes it
     adds the pairs up itself (:meth:`norm_into`) where it can; whoever cannot asks for the rows (:meth:`rows`)."""
@@ -117,10 +127,10 @@ class RoutedRows:
     def norm_into(self, h: torch.Tensor, post_gain: Optional[torch.Tensor], post_eps: float, out: torch.Tensor,
                   pre_gain: Optional[torch.Tensor], pre_eps: float) -> bool:
         """``h += post(rows)`` and ``out = rmsnorm(h) * pre_gain`` (or the rows of ``h`` without a gain) in one kernel, if it takes
-        these sizes and nothing was added up yet."""
+        these sizes, is the faster way (:func:`norm_adds_up`) and nothing was added up yet."""
         y, place, choice, weight, x, shared, _, top, n_experts, shared_gate = self.arguments
         n, e = h.shape
-        if y is None or self._rows is not None or e % 4 or e > 16384 or out.dtype != x.dtype or h.shape != x.shape:
+        if y is None or self._rows is not None or not norm_adds_up(n, top, e) or e % 4 or e > 16384 or out.dtype != x.dtype or h.shape != x.shape:
             return False
         for t in (h, y, shared, post_gain, out, pre_gain):
             if t is not None and (t.data_ptr() % 16 or (t.dim() == 2 and (t.stride(1) != 1 or t.stride(0) % 4))):

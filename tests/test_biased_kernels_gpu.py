@@ -575,7 +575,7 @@ def test_routed_tiles_in_tile_order(n, E, top, ff, hidden, tm):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("n,E,top,hidden", [(1, 3, 1, 4), (6, 17, 5, 2048), (65, 4, 4, 2052), (3, 9, 9, 4100), (130, 8, 2, 1024), (2, 6, 3, 12292)])
+@pytest.mark.parametrize("n,E,top,hidden", [(1, 3, 1, 4), (6, 17, 5, 2048), (65, 4, 4, 2052), (3, 9, 9, 4100), (130, 8, 2, 1024), (2, 6, 3, 12292), (5, 20, 9, 2052), (64, 20, 20, 4096)])
 @pytest.mark.parametrize("post,pre_norm,shared,gated,sorted_rows", [(False, True, False, False, True), (True, False, True, True, True),
                                                                   (True, True, False, False, False), (False, False, True, False, True)])
 def test_routed_rows_into_the_norm(n, E, top, hidden, dtype, post, pre_norm, shared, gated, sorted_rows):

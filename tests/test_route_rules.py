@@ -70,3 +70,13 @@ def test_where_32_bit_products_are_shared_out_along_their_columns(m, n, k, slice
     """Only where both were measured and the slices with their sum were faster."""
     from agave_amd.ops import kernels
     assert kernels.lib("gemm").agave_gemm_slices_for(m, n, k) == slices
+
+
+@pytest.mark.parametrize("n,top,hidden,adds_up", [
+    (1, 5, 2048, True), (6, 64, 4096, True), (1, 10, 8192, True), (1, 12, 7168, False), (6, 16, 8192, False), (6, 5, 16384, True), (6, 6, 14000, True),
+    (6, 7, 16384, False), (47, 16, 12288, False), (48, 16, 12288, True), (48, 24, 16384, False), (300, 24, 12288, True), (300, 25, 5120, False),
+    (3001, 9, 16384, True)])
+def test_where_the_norm_adds_up_a_tokens_pairs(n, top, hidden, adds_up):
+    """Only where the two kernels were measured to take longer."""
+    from agave_amd.ops.routed import norm_adds_up
+    assert norm_adds_up(n, top, hidden) == adds_up
