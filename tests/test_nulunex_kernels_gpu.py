@@ -303,7 +303,7 @@ def test_a_growing_sequence_moves_no_buffer_of_latent_attention():
     assert ws.generation == 0 and ws.allocations == 2
 
 
-@pytest.mark.parametrize("splits", [1, 4, 5, 8, 9, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 5, 8, 9, 16, 17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize("rows, heads, vd, out", [(1, 2, 48, 10), (3, 20, 256, 40), (9, 16, 512, 128), (17, 16, 272, 200)])
 def test_latent_shares_merged_and_multiplied(rows, heads, vd, out, splits):
     """One to eight workgroups a (row, head), every number of shares a group of threads keeps, shares without a key.  The merged row is
