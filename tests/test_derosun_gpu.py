@@ -117,6 +117,14 @@ def test_whole_tail_and_pieces(models, name, dtype):
     assert all(g.pool.n_free == g.pool.n_pages for g in eng.cache.groups)
 
 
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_32_bit_products_in_slices(models, name, monkeypatch):
+    """What reads a product's rows adds up its slices, or gets them added up."""
+    made = U.products_in_slices(monkeypatch)
+    test_whole_tail_and_pieces(models, name, "float32")
+    assert made
+
+
 @pytest.mark.parametrize("name", ["mixed", "even"])
 def test_residual_after_every_layer(models, name):
     """The residual stream after each layer, read off the engine between its blocks."""

@@ -111,6 +111,14 @@ def test_whole_tail_and_pieces(models, name, dtype):
     assert all(g.pool.n_free == g.pool.n_pages for g in eng.cache.groups)
 
 
+@pytest.mark.parametrize("name", ["mixed", "odd", "even"])          # ("one" is too narrow for two slices)
+def test_32_bit_products_in_slices(models, name, monkeypatch):
+    """What reads a product's rows adds up its slices, or gets them added up."""
+    made = U.products_in_slices(monkeypatch)
+    test_whole_tail_and_pieces(models, name, "float32")
+    assert made
+
+
 def test_residual_after_every_layer_run(models):
     """The streams' sum after each run of a layer (a looped layer counts each time), read off the engine between its
     blocks: a block's last result is still pending when the next block starts, so it is written into a copy first."""

@@ -105,6 +105,14 @@ def test_whole_tail_and_pieces(models, name, dtype):
     assert all(g.pool.n_free == g.pool.n_pages for g in eng.cache.groups)
 
 
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_32_bit_products_in_slices(models, name, monkeypatch):
+    """What reads a product's rows adds up its slices, or gets them added up."""
+    made = U.products_in_slices(monkeypatch)
+    test_whole_tail_and_pieces(models, name, "float32")
+    assert made
+
+
 def test_streams_after_every_layer(models):
     """The residual stream after each layer, read off the engine between its blocks."""
     from agave_amd.parts.norm import add_branch

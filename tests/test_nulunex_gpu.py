@@ -104,6 +104,14 @@ def test_whole_tail_and_pieces(models, name, dtype):
     assert all(g.pool.n_free == g.pool.n_pages for g in eng.cache.groups)
 
 
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_32_bit_products_in_slices(models, name, monkeypatch):
+    """What reads a product's rows adds up its slices, or gets them added up."""
+    made = U.products_in_slices(monkeypatch)
+    test_whole_tail_and_pieces(models, name, "float32")
+    assert made
+
+
 def test_residual_after_every_layer_run(models):
     """The residual stream after each run of a layer (one that runs another layer's tensors counts as itself), read off
     the engine between its blocks."""

@@ -77,6 +77,14 @@ def test_whole_tail_and_pieces(models, name, dtype):
     assert eng.cache.slots.n_free == eng.cache.max_slots
 
 
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_32_bit_products_in_slices(models, name, monkeypatch):
+    """What reads a product's rows adds up its slices, or gets them added up."""
+    made = U.products_in_slices(monkeypatch)
+    test_whole_tail_and_pieces(models, name, "float32")
+    assert made
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_batches_of_unequal_requests_and_slots_used_again(models, dtype):
     cfg, w, folder = models("mixed")
