@@ -9,7 +9,8 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 
 // The gate's activation, by number (the feed-forward part knows the names): 0 gelu, tanh form;
 // 1 silu, x / (1 + exp(-x)); 2 gelu with the error function; 3 relu.  Another one is another case
-// here; only the tanh form also ends the matrix-core products (gemm_mfma.hip).
+// here.  A 32-bit product of a few rows ends in any of them (gemm.hip), the matrix-core products in the tanh form, silu and the clamped
+// swish in a form of their own (gemm_mfma.hip).
 #define AGAVE_GATE_ACTS 4
 #define AGAVE_GATE_SWISH_CLAMPED 6     // a gated form with two numbers of its own, known to gate_form only
 __device__ __forceinline__ float gate_act(float x, int act) {

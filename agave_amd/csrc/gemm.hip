@@ -3,7 +3,9 @@
 //
 // This is the true 32-bit path of the linear layers and the fallback for sizes the bfloat16 kernels
 // refuse.  It runs on the matrix cores' 32-bit instructions (v_mfma_f32_*: operands and sums are whole
-// floats, nothing is narrowed), which do twice the multiply-adds a clock of the vector units.
+// floats, nothing is narrowed), which do twice the multiply-adds a clock of the vector units; products of floats of 17 rows
+// and more, where that is faster (split_instead), on the bfloat16 instructions, each float as three bfloat16 pieces that
+// hold all its bits, in 32-bit sums.
 // Weights are row-major [out, in] and used as y = W x, as in the reference
 // (src/backend/backend.zig:474, 481).
 //
@@ -912,7 +914,8 @@ extern "C" int agave_gemm_slices(const float* A, long lda, const float* W, long 
     return 0;
 }
 
-// A product in a tile shape and a number of slices that the caller names.
+// A product in a tile shape and a number of slices that the caller names (the tests run every shape with it; agave_gemm_slices
+// takes the fastest).
 extern "C" int agave_gemm_slices_as(const float* A, long lda, const float* W, long ldw, float* parts, int M, int N, int K, int bm, int bn, int slices,
                                     hipStream_t stream) {
     AGAVE_CHECK(M > 0 && N > 0 && K > 0 && lda >= K && ldw >= K, "gemm_slices_as: bad sizes M=%d N=%d K=%d", M, N, K);

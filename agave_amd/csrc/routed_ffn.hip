@@ -719,7 +719,7 @@ extern "C" int agave_routed_norm(int dtype, float* h, const float* y, const int*
     if (N == 0) return 0;
     // threads as residual_norm takes them: one float4 each in steps of few tokens, two (four) in steps of many.  More than eight pairs
     // of more than 2,048 columns go in twos with few tokens, too: two batches of eight float4 and 1,024 threads wait for one another
-    // (4,096 columns of nine pairs, 64 tokens 6.9 us, so 5.0; a kernel for the sum and one for the norm 7.3).  In twos five
+    // (4,096 columns of nine pairs, 64 tokens 6.9 us, so 4.8; a kernel for the sum and one for the norm 7.3).  In twos five
     // pairs a batch are as fast as eight for six to eight pairs but for 0.4 to 0.6 us of few tokens, and faster from some 300 tokens
     // on (5,120 columns of eight, 800 tokens 31.0 and 33.4) and for five, nine and ten pairs.
     int threads;

@@ -457,7 +457,7 @@ def gemm_slices_for(a: torch.Tensor, w: torch.Tensor) -> int:
 
 def gemm_slices(a: torch.Tensor, w: torch.Tensor, parts: torch.Tensor, tile: Optional[tuple] = None) -> None:
     """``parts`` [slices, M, N] (float32) <- slices that add up to ``a @ w^T``.  ``tile``: rows and columns of the tiles, where
-    the caller names them."""
+    the caller names them (the tests do, to run every shape; the fastest otherwise)."""
     _dev(a, w, parts)
     lda, ldw = _rows(a, "a"), _rows(w, "w")
     (m, k), n, z = a.shape, w.shape[0], parts.shape[0]
