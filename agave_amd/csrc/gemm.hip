@@ -505,9 +505,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_f32_ring_kernel(const float
 // running sum of their own, the five corrections another.  That sum takes 32 products an instruction, the 32-bit
 // instruction two or four, and so rounds a sixteenth as often.
 // Bound by the multiply-adds and, where a stage's tiles are few, by their chain of loads, cuts and barriers.  us, the kernels above and
-// this one with its sums of slices: 777 rows by 10,752 x 2,048 325 and 249 (137 TFLOP/s; the 32-bit instructions reach 153 on the largest
-// products), by 2,048 x 5,376 174 and 119, by 2,048 x 2,048 71 and 65, by 3,072 x 2,048 119 and 78; 2,048 rows by 10,752 x 2,048 728 and
-// 465 (194 TFLOP/s); 64 rows 41 and 38, 58 and 25, 25 and 15, 25 and 17.  Making the operands larger takes 2 to 3 % of it.  Root mean
+// this one with its sums of slices: 777 rows by 10,752 x 2,048 325 and 232 (147 TFLOP/s; the 32-bit instructions reach 153 on the largest
+// products), by 2,048 x 5,376 174 and 110, by 2,048 x 2,048 71 and 51, by 3,072 x 2,048 119 and 76; 2,048 rows by 10,752 x 2,048 728 and
+// 456 (198 TFLOP/s); 64 rows 41 and 31, 58 and 25, 25 and 15, 25 and 17.  Making the operands larger takes 2 to 3 % of it, with up to 64
+// rows by many columns up to 8.  Root mean
 // square of the error against 64 bits over that of the result, in 1e-7: 2,048 columns 5.7 (rings) and 2.7 whole, 1.9 in two slices, 1.3
 // in four; 5,376 9.3 and 4.6, 3.2, 2.2.
 // A piece of an infinity or NaN is none of the two, and floats from 2^104 on and sums from 2^80 on leave 32 bits when they are made so much
@@ -705,15 +706,16 @@ static int ring_rows(int M, int N) {
     return (n32 <= 5 ? RING_32[n32] : 35.0 * n32) <= 130.0 * a_unit(128) ? 32 : 128;
 }
 
-// Microseconds of a product on a tile shape of gemm_f32_split_kernel, from the time of a stage of 32 k with so many tiles a compute unit
-// (2,048 columns, all operands from memory; two workgroups share a unit, up to four of the smaller tiles) and of a launch.
+// Microseconds of a product on a tile shape of gemm_f32_split_kernel: of a launch, and of a stage of 32 k with so many tiles a compute unit
+// (two workgroups share a unit, up to four of the smaller tiles).  Least squares over the times of 500 products of 33 to 6,000 rows by 512
+// to 11,000 x 512 to 11,000 in up to eight slices, from which they are 3 to 4 % off.
 struct SplitShape { int bm, bn; double start, stage[12]; };
 static const double SPLIT_TILES[12] = {0.25, 0.5, 1, 1.25, 1.5, 2, 2.5, 3, 4, 5, 6, 8};
 static const SplitShape SPLIT_SHAPES[4] = {
-    {128, 128, 8, {1.66, 1.71, 1.89, 2.32, 2.39, 2.63, 4.16, 4.25, 5.13, 7.15, 7.81, 10.52}},
-    {64, 128, 6, {1.16, 1.18, 1.22, 1.43, 1.44, 1.55, 2.23, 2.36, 3.27, 3.95, 4.75, 6.24}},
-    {128, 64, 6, {1.11, 1.10, 1.15, 1.35, 1.38, 1.50, 2.16, 2.32, 3.24, 3.74, 4.64, 6.02}},
-    {64, 64, 5, {0.76, 0.78, 0.81, 0.93, 0.96, 0.99, 1.39, 1.45, 1.75, 2.21, 2.88, 3.55}}};
+    {128, 128, 6.4, {1.63, 1.66, 1.71, 2.06, 2.11, 2.38, 4.05, 4.28, 4.59, 6.46, 7.04, 9.73}},
+    {64, 128, 5.2, {1.12, 1.12, 1.15, 1.36, 1.37, 1.48, 2.12, 2.25, 3.02, 3.48, 4.28, 5.61}},
+    {128, 64, 5.1, {1.06, 1.05, 1.09, 1.30, 1.32, 1.45, 2.03, 2.15, 2.94, 3.41, 4.18, 5.56}},
+    {64, 64, 4.4, {0.74, 0.74, 0.76, 0.87, 0.88, 0.92, 1.33, 1.39, 1.62, 2.04, 2.52, 3.20}}};
 // (just past a whole number of tiles a unit some have one more, which is what the others then wait for: as long as the next measured load, or
 // with more than three as the next whole number.  135 rows by 10,896 x 4,888 in tiles of 64 x 64, 2.004 a unit: 206, taken for 2 of them 149)
 static double split_stage(const SplitShape& s, double tiles_a_unit) {
@@ -727,24 +729,29 @@ static double split_stage(const SplitShape& s, double tiles_a_unit) {
     return s.stage[11] * t / SPLIT_TILES[11];
 }
 struct SplitPlan { int shape, slices; double us; };
-#define SLICES_GAIN 0.92                                          // slices' time with their sum is off by up to 8 %: they have to be that much faster
-// The fastest shape, with k shared out among up to max_slices workgroups where that pays for adding up the slices (4 bytes each of
-// them and the result at 3.5 TB/s, and a launch).  Large operands come at 4 TB/s (24 rows by 10,752 x 4,096 in eight slices 45.0 us).
-static SplitPlan plan_split(int M, int N, int K, int max_slices) {
-    SplitPlan best = {0, 1, 1e30};
+// The fastest shape in so many slices.  Adding them up takes a launch, and 4 bytes each of them and the result at 3.5 TB/s; large operands
+// come at 5 TB/s (33 rows by 10,240 x 4,096 in eight slices 43 us).
+static SplitPlan split_in(int M, int N, int K, int slices) {
+    SplitPlan best = {0, slices, 1e30};
+    const int stages = ((K + 31) / 32 + slices - 1) / slices;
+    const double memory = ((double)M + N) * K * 4 / 5.0e6;
+    for (int i = 0; i < 4; ++i) {
+        const SplitShape& s = SPLIT_SHAPES[i];
+        const double tiles = (double)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+        double us = s.start + std::max(split_stage(s, tiles * slices / COMPUTE_UNITS) * stages, memory);
+        if (slices > 1) us += 2.0 + (slices + 1.0) * M * N * 4 / 3.5e6;
+        if (us < best.us) best.shape = i, best.us = us;
+    }
+    return best;
+}
+// The fastest of `least` to `most` slices, powers of two, of eight stages and more; rather one than slices that are as fast (1,200 rows by
+// 10,752 x 4,096 578 and 622 in two, taken for 593 and 589).
+static SplitPlan plan_split(int M, int N, int K, int least, int most) {
+    SplitPlan best = {0, least, 1e30};
     const int stages = (K + 31) / 32;
-    const double memory = ((double)M + N) * K * 4 / 4.0e6;
-    for (int z = 1; z <= max_slices && (z == 1 || stages / z >= 8); z *= 2) {
-        const double limit = z > 1 && best.slices == 1 ? 0.95 * best.us : best.us;     // (1,200 rows by 10,752 x 4,096 587 and 604 in two)
-        SplitPlan of_z = {0, z, limit};
-        for (int i = 0; i < 4; ++i) {
-            const SplitShape& s = SPLIT_SHAPES[i];
-            const double tiles = (double)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-            double us = s.start + std::max(0.95 * split_stage(s, tiles * z / COMPUTE_UNITS) * ((stages + z - 1) / z), memory);
-            if (z > 1) us += 2.0 + (z + 1.0) * M * N * 4 / 3.5e6;
-            if (us < of_z.us) of_z.shape = i, of_z.us = us;
-        }
-        if (of_z.us < limit) best = of_z;
+    for (int z = least; z <= most && (z == 1 || stages / z >= 8); z *= 2) {
+        const SplitPlan of_z = split_in(M, N, K, z);
+        if (of_z.us < (best.slices == 1 && z > 1 ? 0.99 : 1.0) * best.us) best = of_z;
     }
     return best;
 }
@@ -759,8 +766,8 @@ static void launch_split(const SplitPlan& plan, const float* A, long lda, const 
 }
 // Microseconds that the 32-bit instructions take from 17 rows on: rings as ring_rows knows them, with a start for every tile after the other
 // (by the least squares of 98 sizes' logarithms, off by 7 %: 221 rows by 31,916 x 248 45.6, 760 by 776 x 5,784 106); a round of workgroups
-// of groups of rows or of tiles at least so much a 2,048 columns (rows a power of two apart, whose columns lie on the same channels, take
-// up to a third more).
+// of groups of rows or of tiles at least so much a 2,048 columns (1,800 times of 1,100 sizes, one in twenty of which is below it, by some 3 %;
+// rows a power of two apart, whose columns lie on the same channels, take up to a third more).
 static double whole_us(int M, int N, int K, int rows) {
     auto rounds = [](long wgs) { return (double)((wgs + COMPUTE_UNITS - 1) / COMPUTE_UNITS); };
     const long rows64 = ((long)M + 63) / 64, cols64 = ((long)N + TN - 1) / TN;
@@ -769,23 +776,25 @@ static double whole_us(int M, int N, int K, int rows) {
         return 2.0 + (rows == 128 ? 7.2 : 2.4) * n + 0.9 * (rows == 128 ? 130.0 * n : n <= 5 ? RING_32[n] : 35.0 * n) * K / 2048;
     }
     double unit;
-    if (M > SKINNY_M && rows64 * cols64 >= COMPUTE_UNITS) unit = 36.5 * rounds(rows64 * cols64);
-    else if (M > SKINNY_M && ((long)M + 31) / 32 * cols64 >= COMPUTE_UNITS) unit = 36.0;
-    else unit = (M <= 32 ? 10.0 : M <= 48 ? 15.5 : 17.5) * rounds(rows64 * (((long)N + 15) / 16));
+    if (M > SKINNY_M && rows64 * cols64 >= COMPUTE_UNITS) unit = 37.7 * rounds(rows64 * cols64);
+    else if (M > SKINNY_M && ((long)M + 31) / 32 * cols64 >= COMPUTE_UNITS) unit = 31.5;
+    else unit = (M <= 32 ? 10.3 : M <= 48 ? 16.2 : M <= 64 ? 18.0 : 19.0) * rounds(rows64 * (((long)N + 15) / 16));
     return 2.3 + unit * K / 2048;
 }
 // The plan of a product in pieces, us 0 where the 32-bit instructions take it: where they are faster, to within what the times above are
-// off.  Where groups of rows or the tiles above would take it only in slices, from 1,024 columns and 33 rows (or 4,096 and 17) on.  us,
-// those and slices with their sum: 17 rows by 4,096 x 4,096 24.8 and 26.1, by 2,048 23.6 and 19.8; 33 rows by 2,048 x 1,024 11.1 and 12.6, by
-// 2,048 x 2,048 20.0 and 14.0; 64 rows by 1,024 x 1,100 13.1 and 13.5; 150 rows by 6,144 x 2,048 (rings) 42.6 and 45.8; 300 by 2,048 x 1,024 22.6 and
-// 22.8; 400 by 2,048 x 2,048 42.8 and 34.2.
+// off.  Where groups of rows or the tiles above would take it only in slices (one is less exact than groups of rows, two and more are
+// not), from 1,024 columns and 33 rows (or 4,096 and 17) on.  Over the 1,200 sizes none is slower by more than 1 %, and they take 0.4 %
+// longer than in the fastest shape and number of slices each.  us, those and slices with their sum: 17 rows by 4,096 x 4,096 24.8 and 26.1,
+// by 2,048 23.6 and 19.8; 33 rows by 2,048 x 1,024 11.1 and 12.6, by 2,048 x 2,048 20.0 and 14.0; 64 rows by 1,024 x 1,100 13.1 and 13.5;
+// 150 rows by 6,144 x 2,048 (rings) 42.6 and 45.8; 300 by 2,048 x 1,024 22.6 and 22.8; 400 by 2,048 x 2,048 42.8 and 34.2; 1,400 by
+// 2,048 x 2,048 120 and 81.4.
 static SplitPlan split_instead(int M, int N, int K, int max_slices) {
     SplitPlan plan = {0, 1, 0};
     if (M <= 16 || (M <= 32 && K < 4096)) return plan;
     const int rows = ring_rows(M, N);
     if (rows == 0 && (K < 1024 || max_slices == 1)) return plan;
-    plan = plan_split(M, N, K, max_slices);
-    if ((rows == 0 && plan.slices == 1) || plan.us >= (plan.slices > 1 ? SLICES_GAIN : 0.95) * whole_us(M, N, K, rows)) plan.us = 0;
+    plan = plan_split(M, N, K, rows == 0 ? 2 : 1, max_slices);
+    if (plan.us >= 0.95 * whole_us(M, N, K, rows)) plan.us = 0;
     return plan;
 }
 
@@ -903,13 +912,7 @@ extern "C" int agave_gemm_slices(const float* A, long lda, const float* W, long 
                 "gemm_slices: rows of aligned fours");
     AGAVE_CHECK((long)((M + 63) / 64) * ((N + 63) / 64) < (1L << 30), "gemm_slices: M=%d x N=%d exceeds the grid limit", M, N);
     AGAVE_CHECK(slices >= 1 && slices <= 8 && slices <= (K + 31) / 32, "gemm_slices: %d slices of %d columns", slices, K);
-    SplitPlan plan = plan_split(M, N, K, 1);
-    for (int z = 2; z <= slices; z *= 2) {                        // (the shape that goes with as many slices)
-        const SplitPlan more = plan_split(M, N, K, z);
-        if (more.slices == z) plan = more;
-    }
-    plan.slices = slices;
-    launch_split(plan, A, lda, W, ldw, parts, N, M, N, K, (long)M * N, stream);
+    launch_split(split_in(M, N, K, slices), A, lda, W, ldw, parts, N, M, N, K, (long)M * N, stream);
     AGAVE_LAUNCH_CHECK("gemm_slices");
     return 0;
 }
