@@ -311,29 +311,46 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(AttnArgs a) {
 // hold without loss), and masks are applied only to units that touch the ends of the range.
 #define LAZY_LOG2 8.0f
 // FUSED: q arrives as the raw projection; the workgroup normalises and rotates its heads' queries
-// itself, and the workgroup whose range holds the token's own position does the same for the key,
-// writes key and value into their page and only then reads pages (its own stores are visible to
-// it after a workgroup barrier; no other workgroup of this launch reads that row, except those
-// of other head chunks of the same kv head, which write the same bytes themselves).
+// itself, and the workgroup whose range holds the token's own position does the same for the key and
+// writes key and value into their page (no other workgroup of this launch reads that row, except those
+// of other head chunks of the same kv head, which make the same bytes themselves).  The wave that takes that
+// position's unit asks for it like any other, whatever stands in the row by then, and puts the row into
+// its registers from LDS.
+//
+// With one wave on a SIMD, an instruction is four or five clocks of everybody's time: 600 of them are as long as a round trip to
+// memory.  So what is the same for a wave is kept in scalar registers, the first unit neither rescales nor clears anything, the
+// outputs are held transposed (a lane's are one head's: no shuffles to rescale, 16-byte pieces into LDS), and the queries are read from
+// LDS where they are used, which leaves the outputs registers that need no copies.  And a compute unit takes no more than some 45 KB of
+// loads at a time: the waves then stand at the loads they cannot issue, so the heads are normed between the keys' loads and the
+// values'.  Before, they waited for all of both first (the loads stood behind a branch).
+// (4B sizes, us a launch in a chain of all layers, before and now: one sequence of 150 keys 6.2 and 5.2, 8 of 1,024 12.5 and 10.3, 64 of 100
+// 12.3 and 9.5, of which 1.6 are a kernel's start and end; the last one's 33 MB take 5.3 of them, 6.2 TB/s.)
 template <int HDT, bool FUSED>
-__global__ __launch_bounds__(256) void attn_decode_fast_kernel(AttnArgs a, QkFuse f) {
-    constexpr int KS = HDT / 2;
-    extern __shared__ float lds[];            // [4 waves][slots][hd] outputs, then [4][16][2] (max, sum);
-                                              // FUSED: then [4][hd] floats and [16][hd] bf16 for the queries
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+__global__ __launch_bounds__(256, HDT == 16 ? 1 : (HDT == 8 ? 2 : 3)) void attn_decode_fast_kernel(AttnArgs a, QkFuse f) {
+    constexpr int KS = HDT / 2, hd = HDT * 16;
+    constexpr int PITCH = hd + 16;            // floats of a row of outputs in LDS: four heads' pieces fall into different banks
+    extern __shared__ __attribute__((aligned(16))) unsigned char dec_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
     const int G = a.nh / a.nkv;
     const int chunks = (G + 15) / 16;
     const int kvh = blockIdx.y / chunks, chunk = blockIdx.y % chunks;
     const int slots = (G - chunk * 16 < 16) ? G - chunk * 16 : 16;
     const int t = blockIdx.z, split = blockIdx.x;
+    const int head0 = kvh * G + chunk * 16;   // this chunk's first query head
+    float* const sm_o = reinterpret_cast<float*>(dec_lds);             // [4 waves][slots][PITCH] outputs
+    float* const sm_ml = sm_o + (size_t)4 * slots * PITCH;             // [4][16][2] (max, sum)
+    bf16* const q_s = reinterpret_cast<bf16*>(sm_ml + 4 * 16 * 2);     // [slots][hd] queries
+    bf16* const own_k = q_s + (size_t)slots * hd;                      // FUSED: the token's own key and value as their page has them
+    bf16* const own_v = own_k + hd;
     // the token's sequence and position are asked for first: the page ids wait for them
     const int b = a.seq_is_token ? t : a.tok_seq[t];
     const int p = a.tok_pos[t];
     // The first columns of the table row are asked for before the position is known, a column per
     // lane, and before every other vector load: loads come back in the order they left, so behind
     // the rows of q and k the page ids would wait for those, and the first keys for the page ids.
+    const int* const trow_p = a.table + (size_t)b * a.width;
     int trow = -1;
-    if (a.table_from_reach) trow = a.table[(size_t)b * a.width + (lane < a.width ? lane : 0)];
+    if (a.table_from_reach) trow = trow_p[lane < a.width ? lane : 0];
     // FUSED: the first rows of the q/k work are requested next (wave w takes query
     // head w of the chunk; the wave after the last head takes the key and value rows, in case
     // this workgroup turns out to be the one that writes them)
@@ -342,19 +359,23 @@ __global__ __launch_bounds__(256) void attn_decode_fast_kernel(AttnArgs a, QkFus
     bf16 vreg0[NV];
     const bool row0_q = FUSED && wave < slots, row0_k = FUSED && wave == slots && f.k_raw != nullptr;
     if constexpr (FUSED) {
-        constexpr int hd0 = HDT * 16;
-        // a wave without a row reads the token's first query head (and nothing uses it); no load
-        // stands under a condition, so all of them leave together
-        const bf16* src0 = row0_q ? a.q + (size_t)t * a.ldq + (size_t)(kvh * G + chunk * 16 + wave) * hd0
-                                  : (row0_k ? f.k_raw + (size_t)t * f.ldk + (size_t)kvh * hd0 : a.q + (size_t)t * a.ldq);
-        row0 = qk_row_load<bf16, NV>(src0, row0_q ? f.q_gain : f.k_gain, f.inv_freq, f.rot_half, hd0, lane);
+        // No load stands under a condition, so all of them leave together and a wait can name those it needs: where there is nothing to
+        // read (a wave without a row, no gains, no rotation), all lanes ask for one place and nothing uses it.
+        const bf16* src0 = row0_k ? f.k_raw + (size_t)t * f.ldk + (size_t)kvh * hd
+                                  : a.q + (size_t)t * a.ldq + (size_t)(head0 + (row0_q ? wave : 0)) * hd;
+        const bf16* vsrc0 = row0_k ? f.v_raw + (size_t)t * f.ldv + (size_t)kvh * hd : (const bf16*)a.k_pages;
+        const float* gain0 = row0_q ? f.q_gain : f.k_gain;
+        const bool gained = gain0 != nullptr, turned = f.rot_half > 0;
+        const float* gsrc0 = gained ? gain0 : (const float*)a.k_pages;
+        const float* fsrc0 = turned ? f.inv_freq : (const float*)a.k_pages;
 #pragma unroll
-        for (int k = 0; k < NV; ++k) vreg0[k] = bf16{0};
-        if (row0_k) {
-            const bf16* vsrc0 = f.v_raw + (size_t)t * f.ldv + (size_t)kvh * hd0;
+        for (int k = 0; k < NV; ++k) row0.xr[k] = src0[lane + 64 * k];
 #pragma unroll
-            for (int k = 0; k < NV; ++k) vreg0[k] = vsrc0[lane + 64 * k];
-        }
+        for (int k = 0; k < NV; ++k) row0.gv[k] = gsrc0[gained ? lane + 64 * k : 0];
+#pragma unroll
+        for (int k = 0; k < (NV + 1) / 2; ++k) row0.fv[k] = fsrc0[lane + 64 * k < f.rot_half ? lane + 64 * k : 0];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) vreg0[k] = vsrc0[row0_k ? lane + 64 * k : 0];
     }
     // The keys this token sees lie in half pages (units of 32 keys) u_first .. u_last.  The launch's
     // splits share them evenly, whatever the sequence's length (a run of whole pages per split would
@@ -372,173 +393,112 @@ __global__ __launch_bounds__(256) void attn_decode_fast_kernel(AttnArgs a, QkFus
     const int u0 = ua + wave;
     const int half = u0 & 1;                                       // (a wave's units are four apart: one half)
     const int n_my = u0 < ub ? (ub - u0 + 3) / 4 : 0;              // units this wave takes
-    constexpr int hd = HDT * 16;
     const float scale2 = a.scale * 1.4426950408889634f;          // scores in units of log2
+    const bool writer = FUSED && f.k_raw != nullptr && split == a.splits - 1;       // (the last split ends with u_last)
 
-    // queries of this chunk's heads: B operand of S^T = K Q^T
-    frag16 qf[KS];
-    if constexpr (!FUSED) {
-        const bool col_ok = j < slots;
-        const bf16* qrow = a.q + (size_t)t * a.ldq + (size_t)(kvh * G + chunk * 16 + j) * hd;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            if (col_ok) qf[ks].u = *reinterpret_cast<const uint4*>(qrow + 32 * ks + 8 * g);
-            else qf[ks].u = uint4{0, 0, 0, 0};
-        }
-    }
-    f32x4_t o[HDT];
-#pragma unroll
-    for (int d = 0; d < HDT; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float m_ref = -INFINITY, l = 0.f;
-
+    // Page `pi` of the sequence, -1: not there.  The ids of a row no wider than a wave wait in its lanes; of a wider one, and where the
+    // table does not start at the first page, each is a scalar load, asked for a unit ahead of its use.
+    const bool in_lanes = a.table_from_reach && a.width <= 64;
+    auto page_at = [&](int pi) -> int {           // (page ids fit 31 bits)
+        if (!a.table_from_reach) return (int)page_of(a, b, pi);
+        const int col = pi - first;
+        if (col >= a.width) return -1;
+        const int pg = in_lanes ? __builtin_amdgcn_readlane(trow, col) : __builtin_amdgcn_readfirstlane(trow_p[col]);
+        return pg < a.n_pages ? pg : -1;
+    };
     constexpr size_t k_stride = (size_t)4 * KS * 64, v_stride = (size_t)HDT * 2 * 64;   // uint4 per (page, kv head)
-    // a table wider than a wave: the ids of this wave's next pages are fetched together, ahead of
-    // any use (a lookup in the loop would stand between every two units)
-    constexpr int PG_AHEAD = 10;
-    int pg_pre[PG_AHEAD];
-    const bool wide = a.table_from_reach && a.width > 64;
-#pragma unroll
-    for (int i = 0; i < PG_AHEAD; ++i) {
-        const int col = ((u0 + 4 * i) >> 1) - first;
-        pg_pre[i] = (wide && i < n_my && col < a.width) ? a.table[(size_t)b * a.width + col] : -1;
-    }
-    auto page_id = [&](int i) -> int {           // page of this wave's i-th unit (page ids fit 31 bits)
-        const int pi = (u0 + 4 * i) >> 1;
-        int pg;
-        if (a.table_from_reach) {
-            const int col = pi - first;
-            if (!wide) {
-                pg = col < a.width ? __builtin_amdgcn_readlane(trow, col) : -1;
-            } else if (i < PG_AHEAD) {
-                pg = -1;
-#pragma unroll
-                for (int k = 0; k < PG_AHEAD; ++k)
-                    if (k == i) pg = pg_pre[k];
-            } else {
-                pg = col < a.width ? a.table[(size_t)b * a.width + col] : -1;
-            }
-            if (pg >= a.n_pages) pg = -1;
-        } else {
-            pg = (int)page_of(a, b, pi);
-        }
-        return pg;
-    };
     frag16 kb[2][KS], vb[HDT];
-    const u32x4_t* kp = nullptr;
-    const u32x4_t* vp = nullptr;
-    auto load_k = [&]() {
+    // These loads do not stand under a condition: only then can a wait name the loads it needs and leave the younger ones in flight.
+    // Where a wave has no unit, all its lanes ask for one place of the first page, and nothing uses it.  Keys outside the
+    // range are not fetched either: their lanes repeat a key's inside (their scores are masked, and 0 times its value is 0).
+    auto load_k = [&](int pg, int u) {
+        const u32x4_t* kp = (const u32x4_t*)(a.k_pages + ((size_t)(pg < 0 ? 0 : pg) * a.nkv + kvh) * k_stride) + (size_t)2 * half * KS * 64;
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < 2; ++kt) {
+            const int key0 = u * 32 + 16 * kt;
+            const int from = lo - key0 < 0 ? 0 : (lo - key0 > 15 ? 15 : lo - key0), to = p - key0 < 0 ? 0 : (p - key0 > 15 ? 15 : p - key0);
+            const unsigned at = pg < 0 ? 0 : (j < from ? from : (j > to ? to : j)) + 16 * g;
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) kb[kt][ks].r = kp[((2 * half + kt) * KS + ks) * 64 + lane];
+            for (int ks = 0; ks < KS; ++ks) kb[kt][ks].r = kp[(kt * KS + ks) * 64 + at];
+        }
     };
-    auto load_v = [&]() {
+    auto load_v = [&](int pg, int u) {
+        const u32x4_t* vp = (const u32x4_t*)(a.v_pages + ((size_t)(pg < 0 ? 0 : pg) * a.nkv + kvh) * v_stride) + (size_t)half * 64;
+        const unsigned at = pg < 0 ? 0 : (4 * g <= p - u * 32 ? lane : j);         // (a lane's keys are 4 g .. and 16 + 4 g ..)
 #pragma unroll
-        for (int d = 0; d < HDT; ++d) vb[d].r = vp[(d * 2 + half) * 64 + lane];
+        for (int d = 0; d < HDT; ++d) vb[d].r = vp[d * 2 * 64 + at];
     };
 
     // units: this wave's half of its pages, in order; the next unit's K and V are fetched while this one is used
-    int cur_page = 0;
-    int pg = n_my > 0 ? page_id(0) : -1;
-    bool have = n_my > 0 && pg >= 0;
-    if (have) {
-        kp = (const u32x4_t*)(a.k_pages + ((size_t)pg * a.nkv + kvh) * k_stride);
-        vp = (const u32x4_t*)(a.v_pages + ((size_t)pg * a.nkv + kvh) * v_stride);
-    }
-    // FUSED: the token's own key and value go into the page of position p, by the workgroup that
-    // reads it; the wave whose first page that is waits with its loads until the row is there
-    const bool writer = FUSED && f.k_raw != nullptr && split == a.splits - 1;       // (the last split ends with u_last)
-    const bool early = !(writer && u0 == u_last);
-    if (have && early) {
-        load_k();
-        load_v();
-    }
+    const int pg0 = n_my > 0 ? page_at(u0 >> 1) : -1;
+    const int wpg = writer ? page_at(last) : -1;
+    load_k(pg0, u0);
     if constexpr (FUSED) {
-        float* ybuf = lds + (size_t)4 * slots * hd + 4 * 16 * 2 + (size_t)wave * hd;
-        bf16* q_s = reinterpret_cast<bf16*>(lds + (size_t)4 * slots * hd + 4 * 16 * 2 + (size_t)4 * hd);
+        float* ybuf = sm_o + (size_t)wave * hd;                    // (where the outputs will come to stand)
         const float pf = (float)p * f.pos_scale;
         // the token's own key and value go into the page of position p, by the workgroup that reads it
         const int jobs = slots + (writer ? 1 : 0);
-        for (int job0 = 0; job0 < jobs; job0 += 4) {
-            const int job = job0 + wave;
+        auto finish = [&](int job, const QkRow<bf16, NV>& row, const bf16 (&vreg)[NV]) {
             const bool active = job < jobs, is_q = job < slots;
-            QkRow<bf16, NV> row;
-            bf16 vreg[NV];
-            if (job0 == 0) {                       // requested at the kernel's start
-                row = row0;
-#pragma unroll
-                for (int k = 0; k < NV; ++k) vreg[k] = vreg0[k];
-            } else {
-                // (a wave past the last job reads the chunk's first head; the key's job only exists with k_raw)
-                const bool k_job = active && !is_q;
-                const bf16* src = k_job ? f.k_raw + (size_t)t * f.ldk + (size_t)kvh * hd
-                                        : a.q + (size_t)t * a.ldq + (size_t)(kvh * G + chunk * 16 + (active ? job : 0)) * hd;
-                row = qk_row_load<bf16, NV>(src, is_q ? f.q_gain : f.k_gain, f.inv_freq, f.rot_half, hd, lane);
-#pragma unroll
-                for (int k = 0; k < NV; ++k) vreg[k] = bf16{0};
-                if (k_job) {
-                    const bf16* vsrc = f.v_raw + (size_t)t * f.ldv + (size_t)kvh * hd;
-#pragma unroll
-                    for (int k = 0; k < NV; ++k) vreg[k] = vsrc[lane + 64 * k];
-                }
-            }
             qk_row_finish<bf16, NV>(row, ybuf, (is_q ? f.q_gain : f.k_gain) != nullptr, is_q ? f.eps_q : f.eps_k, f.rot_half,
                                     pf, hd, lane, active);
-            if (active && is_q) {
-                for (int d = lane; d < hd; d += 64) q_s[job * hd + d] = f32_to_bf16(ybuf[d]);
-            } else if (active) {
-                long wpg;
-                if (a.table_from_reach) {
-                    const int col = last - first;
-                    wpg = col < a.width ? a.table[(size_t)b * a.width + col] : -1;
-                    if (wpg >= a.n_pages) wpg = -1;
-                } else {
-                    wpg = page_of(a, b, last);
-                }
-                if (wpg >= 0) {
-                    bf16* dk = (bf16*)(a.k_pages + ((size_t)wpg * a.nkv + kvh) * ((size_t)4 * KS * 64));
-                    bf16* dv = (bf16*)(a.v_pages + ((size_t)wpg * a.nkv + kvh) * ((size_t)HDT * 2 * 64));
-                    store_kv_row_packed_regs<bf16, NV>(dk, dv, ybuf, vreg, p % AGAVE_PAGE, hd, lane);
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        const bool col_ok = j < slots;
+            if (!active) return;
+            bf16* dst = is_q ? q_s + job * hd : own_k;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            if (col_ok) qf[ks].u = *reinterpret_cast<const uint4*>(q_s + j * hd + 32 * ks + 8 * g);
-            else qf[ks].u = uint4{0, 0, 0, 0};
+            for (int k = 0; k < NV; ++k) dst[lane + 64 * k] = f32_to_bf16(ybuf[lane + 64 * k]);
+            if (!is_q) {
+#pragma unroll
+                for (int k = 0; k < NV; ++k) own_v[lane + 64 * k] = vreg[k];
+            }
+        };
+        finish(wave, row0, vreg0);                                 // requested at the kernel's start
+        if (jobs > 4) {
+            for (int job = 4 + wave; job < jobs; job += 4) {
+                const bool is_q = job < slots;                         // (the key's job only exists with k_raw)
+                const bf16* src = is_q ? a.q + (size_t)t * a.ldq + (size_t)(head0 + job) * hd : f.k_raw + (size_t)t * f.ldk + (size_t)kvh * hd;
+                const QkRow<bf16, NV> row = qk_row_load<bf16, NV>(src, is_q ? f.q_gain : f.k_gain, f.inv_freq, f.rot_half, hd, lane);
+                const bf16* vsrc = is_q ? src : f.v_raw + (size_t)t * f.ldv + (size_t)kvh * hd;
+                bf16 vreg[NV];
+#pragma unroll
+                for (int k = 0; k < NV; ++k) vreg[k] = vsrc[lane + 64 * k];
+                finish(job, row, vreg);
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70);                    // vmcnt(0): or the loads behind would wait for it where there are no more jobs, too
         }
+    } else {
+        for (int i = threadIdx.x; i < slots * (hd / 8); i += 256)
+            reinterpret_cast<uint4*>(q_s)[i] = *reinterpret_cast<const uint4*>(a.q + (size_t)t * a.ldq + (size_t)head0 * hd + i * 8);
     }
-    if (have && !early) {
-        load_k();
-        load_v();
-    }
-    while (have) {
-        const int key0 = (u0 + 4 * cur_page) * 32;                // first key of this unit
-        // S^T for the unit's two key tiles
+    load_v(pg0, u0);
+    __syncthreads();
+
+    // B operand of S^T = K Q^T: a lane's column is a head (a column past the last head repeats it; its results are not used)
+    const bf16* const q_lane = q_s + (size_t)(j < slots ? j : slots - 1) * hd + 8 * g;
+    f32x4_t o[HDT];                                                // O^T: lane (head j, g) holds columns 16 d + 4 g ..
+    float m_ref = -INFINITY, l = 0.f;
+    auto unit = [&](int i, int next, auto first_c, auto more_c) {  // next: the page of the unit behind, if there is one (MORE)
+        constexpr bool FIRST = decltype(first_c)::value != 0, MORE = decltype(more_c)::value != 0;
+        const int u = u0 + 4 * i, key0 = u * 32;                   // first key of this unit
+        const bool own = !MORE && writer && u == u_last;           // (no unit is behind the last one)
+        // S^T for the unit's two key tiles; the own key is in the row of lane key % 16 + 16 * octet of columns
         f32x4_t st0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, st1 = st0;
+        auto scores = [&](auto own_c) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            st0 = mfma_16x16x32(kb[0][ks], qf[ks], st0);
-            st1 = mfma_16x16x32(kb[1][ks], qf[ks], st1);
-        }
-        // where the next unit lies, and its keys (the K registers are free now)
-        const int n_page = cur_page + 1;
-        bool n_have = n_page < n_my;
-        const u32x4_t* nvp = vp;
-        if (n_have) {
-            const int npg = page_id(n_page);
-            if (npg < 0) {
-                n_have = false;
-            } else {
-                kp = (const u32x4_t*)(a.k_pages + ((size_t)npg * a.nkv + kvh) * k_stride);
-                nvp = (const u32x4_t*)(a.v_pages + ((size_t)npg * a.nkv + kvh) * v_stride);
+            for (int ks = 0; ks < KS; ++ks) {
+                frag16 qf, k0 = kb[0][ks], k1 = kb[1][ks];
+                qf.u = *reinterpret_cast<const uint4*>(q_lane + 32 * ks);
+                if constexpr (decltype(own_c)::value != 0) {
+                    const uint4 row = *reinterpret_cast<const uint4*>(own_k + 32 * ks + 8 * g);
+                    if (j == (p & 31)) k0.u = row;
+                    if (j + 16 == (p & 31)) k1.u = row;
+                }
+                st0 = mfma_16x16x32(k0, qf, st0);
+                st1 = mfma_16x16x32(k1, qf, st1);
             }
-        }
-        if (n_have) load_k();
+        };
+        if (own) scores(IntC<1>{});
+        else scores(IntC<0>{});
+        if constexpr (MORE) load_k(next, u + 4);                       // (the K registers are free now)
         // scores -> probabilities against the running reference
         float s[8];
 #pragma unroll
@@ -555,19 +515,17 @@ __global__ __launch_bounds__(256) void attn_decode_fast_kernel(AttnArgs a, QkFus
             }
         }
         float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        if (__any(mx > m_ref + LAZY_LOG2)) {                       // rare after the first unit
+        mx = rows_max(mx);
+        if constexpr (FIRST) {
+            m_ref = mx;
+        } else if (__any(mx > m_ref + LAZY_LOG2)) {                // rare after the first unit
             const float m_new = fmaxf(m_ref, mx);
-            const float f = (m_ref == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_new);
-            l *= f;
-            float f4[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f4[e] = __shfl(f, 4 * g + e, 64);
+            const float r = (m_ref == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+            l *= r;
 #pragma unroll
             for (int d = 0; d < HDT; ++d)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[d][e] *= f4[e];
+                for (int e = 0; e < 4; ++e) o[d][e] *= r;
             m_ref = m_new;
         }
         const float m_use = (m_ref == -INFINITY) ? 0.f : m_ref;
@@ -580,55 +538,99 @@ __global__ __launch_bounds__(256) void attn_decode_fast_kernel(AttnArgs a, QkFus
             pf.v[e] = (__bf16)pe;
         }
         l += sum;
-        // O += P V, then the V registers are free for the next unit
+        // O^T += V^T P^T, then the V registers are free for the next unit; the own value is element key % 4 + 4 * (key / 16) of lane
+        // column % 16 + 16 * (key % 16 / 4)
+        auto values = [&](auto own_c) {
+            const int word = ((p & 3) >> 1) + ((p & 16) >> 3), shift = (p & 1) * 16;
+            // (and of the lanes that repeat another's, see load_v: what the row held before may be no number)
+            const unsigned here = g == ((p & 15) >> 2) || 4 * g > (p & 31) ? 0xffffu << shift : 0u;
+            const unsigned m0 = word == 0 ? here : 0u, m1 = word == 1 ? here : 0u, m2 = word == 2 ? here : 0u, m3 = word == 3 ? here : 0u;
 #pragma unroll
-        for (int d = 0; d < HDT; ++d) o[d] = mfma_16x16x32(pf, vb[d], o[d]);
-        vp = nvp;
-        if (n_have) load_v();
-        cur_page = n_page;
-        have = n_have;
+            for (int d = 0; d < HDT; ++d) {
+                frag16 vd = vb[d];
+                if constexpr (decltype(own_c)::value != 0) {
+                    const unsigned v = (unsigned)own_v[16 * d + j].x << shift;
+                    vd.r[0] = (vd.r[0] & ~m0) | (v & m0);
+                    vd.r[1] = (vd.r[1] & ~m1) | (v & m1);
+                    vd.r[2] = (vd.r[2] & ~m2) | (v & m2);
+                    vd.r[3] = (vd.r[3] & ~m3) | (v & m3);
+                }
+                o[d] = mfma_16x16x32(vd, pf, FIRST ? f32x4_t{0.f, 0.f, 0.f, 0.f} : o[d]);
+            }
+        };
+        if (own) values(IntC<1>{});
+        else values(IntC<0>{});
+        if constexpr (MORE) load_v(next, u + 4);
+    };
+    auto page_of_unit = [&](int i) { return i < n_my ? page_at((u0 + 4 * i) >> 1) : -1; };
+    if (pg0 >= 0) {
+        int next = page_of_unit(1);
+        if (next < 0) {
+            unit(0, next, IntC<1>{}, IntC<0>{});
+        } else {
+            unit(0, next, IntC<1>{}, IntC<1>{});
+            int i = 1;
+            for (next = page_of_unit(2); next >= 0; next = page_of_unit(++i + 1)) unit(i, next, IntC<0>{}, IntC<1>{});
+            unit(i, next, IntC<0>{}, IntC<0>{});
+        }
+    } else {
+#pragma unroll
+        for (int d = 0; d < HDT; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows_sum(l);
 
     // every wave leaves its (unnormalised) rows, references and sums in LDS
-    float* sm_o = lds;
-    float* sm_ml = lds + (size_t)4 * slots * hd;
+    if (j < slots) {
+        float* dst = sm_o + ((size_t)wave * slots + j) * PITCH + 4 * g;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int slot = 4 * g + e;
-        if (slot < slots) {
-            float* dst = sm_o + ((size_t)wave * slots + slot) * hd;
-#pragma unroll
-            for (int d = 0; d < HDT; ++d) dst[16 * d + j] = o[d][e];
-        }
+        for (int d = 0; d < HDT; ++d) *reinterpret_cast<f32x4_t*>(dst + 16 * d) = o[d];
     }
-    if (lane < 16) {
-        sm_ml[(wave * 16 + lane) * 2 + 0] = m_ref;
-        sm_ml[(wave * 16 + lane) * 2 + 1] = l;
+    if (lane < 16) *reinterpret_cast<float2*>(sm_ml + (wave * 16 + lane) * 2) = float2{m_ref, l};
+    if (FUSED && wave == 3 && wpg >= 0) {
+        bf16* dk = (bf16*)(a.k_pages + ((size_t)wpg * a.nkv + kvh) * k_stride);
+        bf16* dv = (bf16*)(a.v_pages + ((size_t)wpg * a.nkv + kvh) * v_stride);
+        bf16 vreg[NV];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) vreg[k] = own_v[lane + 64 * k];
+        store_kv_row_packed_regs<bf16, NV>(dk, dv, own_k, vreg, p % AGAVE_PAGE, hd, lane);
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < slots * hd; idx += 256) {
-        const int slot = idx / hd, d = idx % hd;
+    const bool out8 = (((uintptr_t)a.out | ((uintptr_t)a.ldo * 2)) & 7) == 0;        // (pieces of four are aligned)
+    for (int idx = threadIdx.x; idx < slots * (hd / 4); idx += 256) {
+        const int slot = idx / (hd / 4), d = idx % (hd / 4) * 4;
+        float2 ml[4];
         float mm = -INFINITY;
 #pragma unroll
-        for (int x = 0; x < 4; ++x) mm = fmaxf(mm, sm_ml[(x * 16 + slot) * 2]);
-        float acc = 0.f, ll = 0.f;
+        for (int x = 0; x < 4; ++x) {
+            ml[x] = *reinterpret_cast<const float2*>(sm_ml + (x * 16 + slot) * 2);
+            mm = fmaxf(mm, ml[x].x);
+        }
+        f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        float ll = 0.f;
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
-            const float mx = sm_ml[(x * 16 + slot) * 2];
-            if (mx != -INFINITY) {
-                const float f = __builtin_amdgcn_exp2f(mx - mm);
-                acc += sm_o[((size_t)x * slots + slot) * hd + d] * f;
-                ll += sm_ml[(x * 16 + slot) * 2 + 1] * f;
+            const f32x4_t part = *reinterpret_cast<const f32x4_t*>(sm_o + ((size_t)x * slots + slot) * PITCH + d);
+            if (ml[x].x != -INFINITY) {
+                const float r = __builtin_amdgcn_exp2f(ml[x].x - mm);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] += part[e] * r;
+                ll += ml[x].y * r;
             }
         }
-        const int head = kvh * G + chunk * 16 + slot;
+        const int head = head0 + slot;
         if (a.splits == 1) {
-            a.out[(size_t)t * a.ldo + (size_t)head * hd + d] = f32_to_bf16(ll > 0.f ? acc / ll : 0.f);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = ll > 0.f ? acc[e] / ll : 0.f;
+            bf16* dst = a.out + (size_t)t * a.ldo + (size_t)head * hd + d;
+            if (out8) {
+                *reinterpret_cast<uint2*>(dst) = uint2{f32x2_to_bf16x2(acc[0], acc[1]), f32x2_to_bf16x2(acc[2], acc[3])};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dst[e] = f32_to_bf16(acc[e]);
+            }
         } else {
             const size_t ps = ((size_t)t * a.nh + head) * a.splits + split;
-            a.part_o[ps * hd + d] = acc;
+            *reinterpret_cast<f32x4_t*>(a.part_o + ps * hd + d) = acc;
             if (d == 0) {
                 a.part_ml[ps * 2 + 0] = mm * 0.6931471805599453f;    // the combine pass works in natural logarithms
                 a.part_ml[ps * 2 + 1] = ll;
@@ -1258,8 +1260,10 @@ static int launch_decode(const AttnArgs& a, const QkFuse& f, int N, hipStream_t 
     const int G = nh / nkv;
     dim3 grid(splits, nkv * ((G + 15) / 16), N);
     const int slots = G < 16 ? G : 16;
-    size_t lds = ((size_t)4 * slots * hd + 4 * 16 * 2) * sizeof(float);
-    if (FUSED) lds += (size_t)4 * hd * sizeof(float) + (size_t)16 * hd * sizeof(bf16);
+    const bool fast = hd == 64 || hd == 128 || hd == 256;
+    size_t lds = ((size_t)4 * slots * (fast ? hd + 16 : hd) + 4 * 16 * 2) * sizeof(float);
+    if (fast) lds += (size_t)(slots + 2) * hd * sizeof(bf16);
+    AGAVE_CHECK(!fast || splits == 1 || (uintptr_t)a.part_o % 16 == 0, "attn_decode_mfma: the partial results must be 16-byte aligned");
     AGAVE_CHECK(lds <= 96 * 1024, "attn_decode_mfma: %zu bytes of LDS exceed what a workgroup may take", lds);
     if (raise_decode_lds_allowance()) return -1;
     if (FUSED) {

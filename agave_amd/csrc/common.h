@@ -117,6 +117,20 @@ __device__ __forceinline__ float wave_max(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// Every lane gets the sum (the maximum) over the four lanes 16 apart: two exchanges of rows between registers, where a shuffle is an LDS
+// instruction with its latency.
+// (Written as instructions, with the wait states they need behind a vector instruction: of the builtins' two results this compiler hands
+// out the first one twice.)
+template <typename F> __device__ __forceinline__ float over_rows(float v, F&& f) {
+    float a = v, b = v;
+    asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));       // rows 0 0 2 2 and 1 1 3 3
+    float c = f(a, b), d = c;
+    asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));       // the lower half twice and the upper half twice
+    return f(c, d);
+}
+__device__ __forceinline__ float rows_sum(float v) { return over_rows(v, [](float x, float y) { return x + y; }); }
+__device__ __forceinline__ float rows_max(float v) { return over_rows(v, [](float x, float y) { return fmaxf(x, y); }); }
+
 // Block-wide reductions for blocks of up to 1024 threads; `red` is 16 floats of LDS.
 // Every thread gets the result.  Contains barriers: call from all threads.
 __device__ __forceinline__ float block_sum(float v, float* red) {

@@ -102,14 +102,14 @@ __device__ __forceinline__ void qk_row_finish(const QkRow<T, NV>& r, float* y, b
     wave_lds_order();
 }
 
-// One wave writes a key row y[0..hd) (LDS) and a value row (in registers: vreg[k] is element
+// One wave writes a key row y[0..hd) (LDS, in 32 bits or in T) and a value row (in registers: vreg[k] is element
 // lane + 64 k) to row `row` of a page in tile
 // order: dk, dv are the page's K and V blocks of this kv head.
 //   K: tiles [row / 16][d / 32] of 64 lanes x 8: lane (row % 16) + 16 * ((d % 32) / 8), element d % 8
 //   V: tiles [d / 16][row / 32] of 64 lanes x 8: lane (d % 16) + 16 * vg, element ve, with the 32 keys
 //      of a half page in the order the score accumulators have them
-template <typename T, int NV>
-__device__ __forceinline__ void store_kv_row_packed_regs(T* dk, T* dv, const float* y, const T (&vreg)[NV], int row,
+template <typename T, int NV, typename Y>
+__device__ __forceinline__ void store_kv_row_packed_regs(T* dk, T* dv, const Y* y, const T (&vreg)[NV], int row,
                                                          int hd, int lane) {
     const int ks_n = (hd + 31) >> 5;
     const int kt = row >> 4, ki = row & 15;
@@ -120,7 +120,7 @@ __device__ __forceinline__ void store_kv_row_packed_regs(T* dk, T* dv, const flo
         const int d = lane + 64 * k;
         if (d < hd) {
             const int ks = d >> 5, g = (d & 31) >> 3, e = d & 7;
-            st(dk + ((size_t)(kt * ks_n + ks) * 64 + ki + 16 * g) * 8 + e, y[d]);
+            st(dk + ((size_t)(kt * ks_n + ks) * 64 + ki + 16 * g) * 8 + e, ld(y + d));
             const int dt = d >> 4, j = d & 15;
             dv[((size_t)(dt * 2 + s2) * 64 + j + 16 * vg) * 8 + ve] = vreg[k];
         }

@@ -1740,3 +1740,56 @@ def test_attn_decode_fused_equals_the_two_kernels(K, nh, nkv, hd, window, rot):
     A.qk_attention(q, None, None, torch.empty_like(q), out, qg, kg, 1e-5, 2e-6, inv_freq, 0.5, kp, vp, table, base,
                    step, nh, nkv, hd, scale, window, True)
     assert torch.equal(out, outs[1][0]) and torch.equal(kp, outs[1][1]) and torch.equal(vp, outs[1][2])
+
+
+# Where the decode kernel can go wrong at the token's own row: every place of it within a unit of 32 keys' registers, windows that
+# begin inside a unit, more than four jobs a workgroup, two chunks of heads, tables wider than a wave, with and without columns that
+# begin at the reach.  Until the kernel writes it, the row in the page is not a number, so whoever read it from there would be seen.
+@pytest.mark.parametrize("from_reach", [True, False])
+@pytest.mark.parametrize("nh,nkv,hd,window,lens", [
+    (8, 4, 256, None, [1, 2, 4, 5, 13, 16, 17, 18, 29, 32, 33, 49, 64, 65, 96, 128, 161, 700]),
+    (8, 4, 256, 40, [1, 16, 17, 33, 40, 41, 57, 64, 100, 129]), (5, 1, 128, None, [3, 20, 31, 95, 320]),
+    (18, 1, 64, 100, [1, 21, 32, 101, 230]), (2, 2, 256, None, [4200, 4097, 70]), (2, 1, 128, None, [4200, 33]),
+    (4, 2, 64, None, [30, 6000])])
+def test_attn_decode_fused_own_row(K, nh, nkv, hd, window, lens, from_reach):
+    from agave_amd.ops import attention_mfma as A
+    g = torch.Generator().manual_seed(hd + len(lens))
+    B, n_pages = len(lens), sum((L + 63) // 64 for L in lens) + 1
+    kp = torch.zeros(n_pages, nkv, 64, hd, dtype=torch.bfloat16, device=DEV)
+    vp = torch.zeros(n_pages, nkv, hd, 64, dtype=torch.bfloat16, device=DEV)
+    perm = torch.randperm(n_pages, generator=g).tolist()
+    full = torch.full((B, max((L + 63) // 64 for L in lens)), -1, dtype=torch.int32)
+    ks, vs, scale = [], [], 0.3 * (16 / hd) ** 0.5
+    for b, L in enumerate(lens):
+        ks.append(torch.randn(L, nkv, hd, generator=g).bfloat16())
+        vs.append(torch.randn(L, nkv, hd, generator=g).bfloat16())
+        for i in range((L + 63) // 64):
+            full[b, i] = perm.pop()
+    k_bad, v_bad = [k.clone() for k in ks], [v.clone() for v in vs]
+    for k, v in zip(k_bad, v_bad):
+        k[-1], v[-1] = float("nan"), float("nan")
+    flat = lambda xs: torch.cat(xs).reshape(-1, nkv * hd).to(DEV)
+    K.qk_norm_rope_kv(None, flat(k_bad), flat(v_bad), None, None, None, 0.0, 0.0, None, 1.0,
+                      _i32([b for b, L in enumerate(lens) for _ in range(L)]), _i32([i for L in lens for i in range(L)]), kp, vp,
+                      full.to(DEV), _i32([0] * B), 0, nkv, hd, packed=True)
+    step = _FakeStep(lens, lambda L: L - 1, window)
+    table, base = full, [0] * B
+    if from_reach:
+        step.tables_start_at_reach = True
+        base = [max(0, L - window) // 64 if window else 0 for L in lens]
+        table = torch.full_like(full, -1)
+        for b in range(B):
+            table[b, :full.shape[1] - base[b]] = full[b, base[b]:]
+    q = torch.randn(B, nh, hd, generator=g).bfloat16()
+    out = torch.full((B, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    A.decode_fused(q.reshape(B, -1).to(DEV), flat([k[-1:] for k in ks]), flat([v[-1:] for v in vs]), out, None, None, 0.0, 0.0, None, 1.0,
+                   kp, vp, table.to(DEV), _i32(base), step, nh, nkv, hd, scale, window)
+    ref = torch.cat([_last_row_attention(q[b][None].expand(L, nh, hd).double(), ks[b].double(), vs[b].double(), scale, window)
+                     for b, L in enumerate(lens)])
+    # (probabilities and results are rounded to bfloat16, half a unit of 2^-8 each; values are below 5)
+    assert torch.allclose(out.cpu().double().view(B, nh, hd), ref, atol=2e-2, rtol=1e-2)
+    want_k, want_v = torch.zeros_like(kp), torch.zeros_like(vp)
+    K.qk_norm_rope_kv(None, flat(ks), flat(vs), None, None, None, 0.0, 0.0, None, 1.0,
+                      _i32([b for b, L in enumerate(lens) for _ in range(L)]), _i32([i for L in lens for i in range(L)]), want_k, want_v,
+                      full.to(DEV), _i32([0] * B), 0, nkv, hd, packed=True)
+    assert torch.equal(kp, want_k) and torch.equal(vp, want_v)
