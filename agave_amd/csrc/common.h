@@ -133,15 +133,25 @@ __device__ __forceinline__ float rows_max(float v) { return over_rows(v, [](floa
 
 // Block-wide reductions for blocks of up to 1024 threads; `red` is 16 floats of LDS.
 // Every thread gets the result.  Contains barriers: call from all threads.
-__device__ __forceinline__ float block_sum(float v, float* red) {
+// block_sum_into: `red` must not be in use (a sum's own memory needs no barrier in front).  The waves' sums are read all at once, zeros in the
+// place of those that are not there, and added up in their order: read one by one in a loop they were a round trip to LDS each.
+__device__ __forceinline__ float block_sum_into(float v, float* red) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     v = wave_sum(v);
-    __syncthreads();
-    if (lane == 0) red[w] = v;
+    if (lane == 0 || (w == 0 && lane >= nw && lane < 16)) red[lane == 0 ? w : lane] = lane == 0 ? v : 0.f;
     __syncthreads();
     float r = 0.f;
-    for (int i = 0; i < nw; ++i) r += red[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r += red[i];
+    if (nw > 8) {
+#pragma unroll
+        for (int i = 8; i < 16; ++i) r += red[i];
+    }
     return r;
+}
+__device__ __forceinline__ float block_sum(float v, float* red) {
+    __syncthreads();
+    return block_sum_into(v, red);
 }
 __device__ __forceinline__ float block_max(float v, float* red) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;

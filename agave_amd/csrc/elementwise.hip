@@ -152,13 +152,16 @@ template <> __device__ __forceinline__ void store4<bf16>(bf16* p, float4 v) {
 // loaded is touched before everything has been asked for, so the loads travel together.
 __device__ __forceinline__ float sumsq(bool in, float4 v) { return in ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f; }
 
+// Few rows are bound by their chain of one trip to memory (0.8 us of it) and two sums over the workgroup: eight rows of 2,560 and three
+// slices 3.44 us a launch in a chain of its own, of which 1.6 are a kernel's start and end, and 3.17 since the sums read the waves' parts
+// at once and the stream is stored behind them.
 template <typename T, int VPT, int PB, bool OF_SUM>          // PB: slices asked for at a time
 __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __restrict__ branch, long ldb, int n_parts,
                                           long part_stride, const float* __restrict__ post_gain, float post_eps,
                                           T* __restrict__ out, long ldo, const float* __restrict__ pre_gain,
                                           float pre_eps, const int* __restrict__ rows, int e,
                                           const float* __restrict__ h_src, OfSum sum) {
-    __shared__ float red[16];
+    __shared__ float red[2][16];                                  // (each sum its own)
     const int i = blockIdx.x;
     const int r = rows ? rows[i] : i;
     float* hr = h + (size_t)r * e;
@@ -228,7 +231,7 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
             hv[v].w = fmaf(sum.alpha, hv[v].w, bv[v].w + bias[v].w);
             ss += sumsq(in[v], hv[v]);
         }
-        ss = block_sum(ss, red);
+        ss = block_sum_into(ss, red[0]);
         const float inv = 1.0f / sqrtf(ss / (float)e + post_eps);
 #pragma unroll
         for (int v = 0; v < VPT; ++v) {
@@ -236,7 +239,6 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
             hv[v].y *= inv * g1[v].y;
             hv[v].z *= inv * g1[v].z;
             hv[v].w *= inv * g1[v].w;
-            if (in[v]) *reinterpret_cast<float4*>(hr + col[v]) = hv[v];
         }
     } else if (branch) {
         float inv = 1.0f;
@@ -244,7 +246,7 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
             float ss = 0.f;
 #pragma unroll
             for (int v = 0; v < VPT; ++v) ss += sumsq(in[v], bv[v]);
-            ss = block_sum(ss, red);
+            ss = block_sum_into(ss, red[0]);
             inv = 1.0f / sqrtf(ss / (float)e + post_eps);
         }
 #pragma unroll
@@ -260,14 +262,17 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
                 hv[v].z += bv[v].z;
                 hv[v].w += bv[v].w;
             }
-            if (in[v]) *reinterpret_cast<float4*>(hr + col[v]) = hv[v];
         }
-    } else if (h_src) {
+    }
+    // (behind the second sum: in front of its barrier the store would be waited for)
+    auto store_h = [&]() {
+        if (!branch && !h_src) return;
 #pragma unroll
         for (int v = 0; v < VPT; ++v)
             if (in[v]) *reinterpret_cast<float4*>(hr + col[v]) = hv[v];
-    }
+    };
     if (out && !pre_gain) {                             // the rows as they are, rounded to the output's type
+        store_h();
         T* o = out + (size_t)i * ldo;
 #pragma unroll
         for (int v = 0; v < VPT; ++v)
@@ -276,7 +281,8 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
         float ss = 0.f;
 #pragma unroll
         for (int v = 0; v < VPT; ++v) ss += sumsq(in[v], hv[v]);
-        ss = block_sum(ss, red);
+        ss = block_sum_into(ss, red[1]);
+        store_h();
         const float inv = 1.0f / sqrtf(ss / (float)e + pre_eps);
         T* o = out + (size_t)i * ldo;
 #pragma unroll
@@ -286,6 +292,7 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
                                           hv[v].w * inv * g2[v].w});
         }
     }
+    if (!out) store_h();
 }
 
 template <typename T, bool OF_SUM>
