@@ -64,7 +64,10 @@ struct QkFuse {
     const float* inv_freq;
     int rot_half;
     float pos_scale;
+    int slices;          // > 0: q, k_raw and v_raw are that many 32-bit slices whose sums are the rows (and the strides count floats)
+    long slice_stride;
 };
+#define QK_MAX_SLICES 4
 
 // One wave: QT tiles of 16 query slots against the pages [page_lo, page_hi] of one sequence
 // and kv head.  Slot j of tile t has position pos[t] (per lane: the lane's column j = lane%16)
@@ -310,6 +313,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(AttnArgs a) {
 // reference stays: probabilities are bounded by 2^8, which 32-bit sums and bfloat16 operands
 // hold without loss), and masks are applied only to units that touch the ends of the range.
 #define LAZY_LOG2 8.0f
+template <bool SLICES> struct RawOf { using type = bf16; };
+template <> struct RawOf<true> { using type = float; };
 // FUSED: q arrives as the raw projection; the workgroup normalises and rotates its heads' queries
 // itself, and the workgroup whose range holds the token's own position does the same for the key and
 // writes key and value into their page (no other workgroup of this launch reads that row, except those
@@ -325,8 +330,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(AttnArgs a) {
 // values'.  Before, they waited for all of both first (the loads stood behind a branch).
 // (4B sizes, us a launch in a chain of all layers, before and now: one sequence of 150 keys 6.2 and 5.2, 8 of 1,024 12.5 and 10.3, 64 of 100
 // 12.3 and 9.5, of which 1.6 are a kernel's start and end; the last one's 33 MB take 5.3 of them, 6.2 TB/s.)
-template <int HDT, bool FUSED>
+// MODE: what q is.  0: queries ready for use; 1 (FUSED): the raw projections in bfloat16; 2: their 32-bit slices (a product of few row
+// blocks that was shared out along its columns: q/k/v of 4B sizes, 64 tokens, 10.6 us as one product and 8.0 in four slices).
+template <int HDT, int MODE>
 __global__ __launch_bounds__(256, HDT == 16 ? 1 : (HDT == 8 ? 2 : 3)) void attn_decode_fast_kernel(AttnArgs a, QkFuse f) {
+    constexpr bool FUSED = MODE != 0;
+    using Raw = typename RawOf<MODE == 2>::type;
+    constexpr int NS = MODE == 2 ? QK_MAX_SLICES : 1;
     constexpr int KS = HDT / 2, hd = HDT * 16;
     constexpr int PITCH = hd + 16;            // floats of a row of outputs in LDS: four heads' pieces fall into different banks
     extern __shared__ __attribute__((aligned(16))) unsigned char dec_lds[];
@@ -355,28 +365,32 @@ __global__ __launch_bounds__(256, HDT == 16 ? 1 : (HDT == 8 ? 2 : 3)) void attn_
     // head w of the chunk; the wave after the last head takes the key and value rows, in case
     // this workgroup turns out to be the one that writes them)
     constexpr int NV = HDT / 4;               // groups of 64 elements in a head
-    QkRow<bf16, NV> row0;
-    bf16 vreg0[NV];
+    // No load stands under a condition, so all of them leave together and a wait can name those it needs: where there is nothing to
+    // read (a wave without a row, no gains, no rotation), all lanes ask for one place and nothing uses it.
+    struct Asked { Raw x[NS][NV], v[NS][NV]; float gain[NV], freq[(NV + 1) / 2]; };
+    auto ask = [&](Asked& r, int job, bool is_k) {             // job: the query head's, unless is_k
+        const Raw* src = is_k ? (const Raw*)f.k_raw + (size_t)t * f.ldk + (size_t)kvh * hd : (const Raw*)a.q + (size_t)t * a.ldq + (size_t)(head0 + job) * hd;
+        const Raw* vsrc = is_k ? (const Raw*)f.v_raw + (size_t)t * f.ldv + (size_t)kvh * hd : (const Raw*)a.k_pages;
+        const float* gain = is_k ? f.k_gain : f.q_gain;
+        const bool gained = gain != nullptr;
+        const float* gsrc = gained ? gain : (const float*)a.k_pages;
+        const float* fsrc = f.rot_half > 0 ? f.inv_freq : (const float*)a.k_pages;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) r.x[s][k] = src[(size_t)(s < f.slices ? s : 0) * f.slice_stride + lane + 64 * k];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) r.gain[k] = gsrc[gained ? lane + 64 * k : 0];
+#pragma unroll
+        for (int k = 0; k < (NV + 1) / 2; ++k) r.freq[k] = fsrc[lane + 64 * k < f.rot_half ? lane + 64 * k : 0];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) r.v[s][k] = vsrc[is_k ? (size_t)(s < f.slices ? s : 0) * f.slice_stride + lane + 64 * k : 0];
+    };
+    Asked row0;
     const bool row0_q = FUSED && wave < slots, row0_k = FUSED && wave == slots && f.k_raw != nullptr;
-    if constexpr (FUSED) {
-        // No load stands under a condition, so all of them leave together and a wait can name those it needs: where there is nothing to
-        // read (a wave without a row, no gains, no rotation), all lanes ask for one place and nothing uses it.
-        const bf16* src0 = row0_k ? f.k_raw + (size_t)t * f.ldk + (size_t)kvh * hd
-                                  : a.q + (size_t)t * a.ldq + (size_t)(head0 + (row0_q ? wave : 0)) * hd;
-        const bf16* vsrc0 = row0_k ? f.v_raw + (size_t)t * f.ldv + (size_t)kvh * hd : (const bf16*)a.k_pages;
-        const float* gain0 = row0_q ? f.q_gain : f.k_gain;
-        const bool gained = gain0 != nullptr, turned = f.rot_half > 0;
-        const float* gsrc0 = gained ? gain0 : (const float*)a.k_pages;
-        const float* fsrc0 = turned ? f.inv_freq : (const float*)a.k_pages;
-#pragma unroll
-        for (int k = 0; k < NV; ++k) row0.xr[k] = src0[lane + 64 * k];
-#pragma unroll
-        for (int k = 0; k < NV; ++k) row0.gv[k] = gsrc0[gained ? lane + 64 * k : 0];
-#pragma unroll
-        for (int k = 0; k < (NV + 1) / 2; ++k) row0.fv[k] = fsrc0[lane + 64 * k < f.rot_half ? lane + 64 * k : 0];
-#pragma unroll
-        for (int k = 0; k < NV; ++k) vreg0[k] = vsrc0[row0_k ? lane + 64 * k : 0];
-    }
+    if constexpr (FUSED) ask(row0, row0_q ? wave : 0, row0_k);       // (a wave without a row: the first head again)
     // The keys this token sees lie in half pages (units of 32 keys) u_first .. u_last.  The launch's
     // splits share them evenly, whatever the sequence's length (a run of whole pages per split would
     // leave the last splits of a short sequence idle and the waves of a split unequal shares); a
@@ -438,9 +452,29 @@ __global__ __launch_bounds__(256, HDT == 16 ? 1 : (HDT == 8 ? 2 : 3)) void attn_
         const float pf = (float)p * f.pos_scale;
         // the token's own key and value go into the page of position p, by the workgroup that reads it
         const int jobs = slots + (writer ? 1 : 0);
-        auto finish = [&](int job, const QkRow<bf16, NV>& row, const bf16 (&vreg)[NV]) {
+        auto finish = [&](int job, const Asked& r) {
             const bool active = job < jobs, is_q = job < slots;
-            qk_row_finish<bf16, NV>(row, ybuf, (is_q ? f.q_gain : f.k_gain) != nullptr, is_q ? f.eps_q : f.eps_k, f.rot_half,
+            QkRow<Raw, NV> row;
+            bf16 vreg[NV];
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                Raw x = r.x[0][k], v = r.v[0][k];
+                if constexpr (MODE == 2) {
+#pragma unroll
+                    for (int s = 1; s < NS; ++s) {
+                        x += s < f.slices ? r.x[s][k] : 0.f;
+                        v += s < f.slices ? r.v[s][k] : 0.f;
+                    }
+                    vreg[k] = f32_to_bf16(v);
+                } else {
+                    vreg[k] = v;
+                }
+                row.xr[k] = x;
+                row.gv[k] = r.gain[k];
+            }
+#pragma unroll
+            for (int k = 0; k < (NV + 1) / 2; ++k) row.fv[k] = r.freq[k];
+            qk_row_finish<Raw, NV>(row, ybuf, (is_q ? f.q_gain : f.k_gain) != nullptr, is_q ? f.eps_q : f.eps_k, f.rot_half,
                                     pf, hd, lane, active);
             if (!active) return;
             bf16* dst = is_q ? q_s + job * hd : own_k;
@@ -451,17 +485,12 @@ __global__ __launch_bounds__(256, HDT == 16 ? 1 : (HDT == 8 ? 2 : 3)) void attn_
                 for (int k = 0; k < NV; ++k) own_v[lane + 64 * k] = vreg[k];
             }
         };
-        finish(wave, row0, vreg0);                                 // requested at the kernel's start
+        finish(wave, row0);                                        // requested at the kernel's start
         if (jobs > 4) {
-            for (int job = 4 + wave; job < jobs; job += 4) {
-                const bool is_q = job < slots;                         // (the key's job only exists with k_raw)
-                const bf16* src = is_q ? a.q + (size_t)t * a.ldq + (size_t)(head0 + job) * hd : f.k_raw + (size_t)t * f.ldk + (size_t)kvh * hd;
-                const QkRow<bf16, NV> row = qk_row_load<bf16, NV>(src, is_q ? f.q_gain : f.k_gain, f.inv_freq, f.rot_half, hd, lane);
-                const bf16* vsrc = is_q ? src : f.v_raw + (size_t)t * f.ldv + (size_t)kvh * hd;
-                bf16 vreg[NV];
-#pragma unroll
-                for (int k = 0; k < NV; ++k) vreg[k] = vsrc[lane + 64 * k];
-                finish(job, row, vreg);
+            for (int job = 4 + wave; job < jobs; job += 4) {       // (the key's job only exists with k_raw)
+                Asked row;
+                ask(row, job, job >= slots);
+                finish(job, row);
             }
             __builtin_amdgcn_s_waitcnt(0x0F70);                    // vmcnt(0): or the loads behind would wait for it where there are no more jobs, too
         }
@@ -1235,10 +1264,10 @@ static int raise_decode_lds_allowance() {
     if (raised) return 0;
     const void* fns[] = {(const void*)attn_decode_mfma_kernel<4>, (const void*)attn_decode_mfma_kernel<8>,
                          (const void*)attn_decode_mfma_kernel<16>,
-                         (const void*)attn_decode_fast_kernel<4, false>, (const void*)attn_decode_fast_kernel<8, false>,
-                         (const void*)attn_decode_fast_kernel<16, false>,
-                         (const void*)attn_decode_fast_kernel<4, true>, (const void*)attn_decode_fast_kernel<8, true>,
-                         (const void*)attn_decode_fast_kernel<16, true>};
+                         (const void*)attn_decode_fast_kernel<4, 0>, (const void*)attn_decode_fast_kernel<8, 0>,
+                         (const void*)attn_decode_fast_kernel<16, 0>,
+                         (const void*)attn_decode_fast_kernel<4, 1>, (const void*)attn_decode_fast_kernel<4, 2>, (const void*)attn_decode_fast_kernel<8, 1>, (const void*)attn_decode_fast_kernel<8, 2>,
+                         (const void*)attn_decode_fast_kernel<16, 1>, (const void*)attn_decode_fast_kernel<16, 2>};
     for (const void* fn : fns)
         AGAVE_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) == hipSuccess,
                     "attn_decode_mfma: cannot raise the LDS allowance");
@@ -1268,12 +1297,16 @@ static int launch_decode(const AttnArgs& a, const QkFuse& f, int N, hipStream_t 
     if (raise_decode_lds_allowance()) return -1;
     if (FUSED) {
         AGAVE_CHECK(hd == 64 || hd == 128 || hd == 256, "attn_decode_fused: head_dim %d is not 64, 128 or 256", hd);
-        if (hd == 64) attn_decode_fast_kernel<4, true><<<grid, 256, lds, stream>>>(a, f);
-        else if (hd == 128) attn_decode_fast_kernel<8, true><<<grid, 256, lds, stream>>>(a, f);
-        else attn_decode_fast_kernel<16, true><<<grid, 256, lds, stream>>>(a, f);
-    } else if (hd == 64) attn_decode_fast_kernel<4, false><<<grid, 256, lds, stream>>>(a, f);
-    else if (hd == 128) attn_decode_fast_kernel<8, false><<<grid, 256, lds, stream>>>(a, f);
-    else if (hd == 256) attn_decode_fast_kernel<16, false><<<grid, 256, lds, stream>>>(a, f);
+        if (f.slices > 0) {
+            if (hd == 64) attn_decode_fast_kernel<4, 2><<<grid, 256, lds, stream>>>(a, f);
+            else if (hd == 128) attn_decode_fast_kernel<8, 2><<<grid, 256, lds, stream>>>(a, f);
+            else attn_decode_fast_kernel<16, 2><<<grid, 256, lds, stream>>>(a, f);
+        } else if (hd == 64) attn_decode_fast_kernel<4, 1><<<grid, 256, lds, stream>>>(a, f);
+        else if (hd == 128) attn_decode_fast_kernel<8, 1><<<grid, 256, lds, stream>>>(a, f);
+        else attn_decode_fast_kernel<16, 1><<<grid, 256, lds, stream>>>(a, f);
+    } else if (hd == 64) attn_decode_fast_kernel<4, 0><<<grid, 256, lds, stream>>>(a, f);
+    else if (hd == 128) attn_decode_fast_kernel<8, 0><<<grid, 256, lds, stream>>>(a, f);
+    else if (hd == 256) attn_decode_fast_kernel<16, 0><<<grid, 256, lds, stream>>>(a, f);
     else if (hd <= 64) attn_decode_mfma_kernel<4><<<grid, 256, lds, stream>>>(a);
     else if (hd <= 128) attn_decode_mfma_kernel<8><<<grid, 256, lds, stream>>>(a);
     else attn_decode_mfma_kernel<16><<<grid, 256, lds, stream>>>(a);
@@ -1353,7 +1386,8 @@ extern "C" int agave_attn_decode_mfma_noalloc(const void* q, long ldq, void* out
 
 // Decode attention that first does the q/k head norm, the rotation and the cache write of each
 // sequence's new token (one token per sequence, positions tok_pos): q, k, v are the raw
-// projections; k and v null for a run that appends nothing.  leave_partials: with more than one
+// projections; k and v null for a run that appends nothing.  slices > 0: they are 32-bit, that many slices each, slice_stride elements
+// apart, whose sums are the projections.  leave_partials: with more than one
 // split, do not merge the splits' results into `out`; the caller's next kernel reads part_o and
 // part_ml itself (gemm_mfma.hip: the output projection that merges while it stages its input).
 extern "C" int agave_attn_decode_fused(const void* q, long ldq, const void* k, long ldk, const void* v, long ldv,
@@ -1363,7 +1397,7 @@ extern "C" int agave_attn_decode_fused(const void* q, long ldq, const void* k, l
                                        int width, const int* base, int n_pages, const int* tok_seq,
                                        const int* tok_pos, int N, int nh, int nkv, int hd, float scale, int window,
                                        int splits, int pages_per_split, int seq_is_token, int table_from_reach,
-                                       int leave_partials, hipStream_t stream) {
+                                       int leave_partials, int slices, long slice_stride, hipStream_t stream) {
     AttnArgs a{(const bf16*)q, ldq, (bf16*)out, ldo, part_o, part_ml, (const uint4*)k_pages, (const uint4*)v_pages,
                table, width, base, n_pages, tok_seq, tok_pos, nullptr, 0, nh, nkv, hd, scale, window, splits,
                pages_per_split, seq_is_token, table_from_reach};
@@ -1372,7 +1406,9 @@ extern "C" int agave_attn_decode_fused(const void* q, long ldq, const void* k, l
     AGAVE_CHECK((k == nullptr) == (v == nullptr), "attn_decode_fused: k and v come together");
     AGAVE_CHECK(!k || (ldk >= (long)nkv * hd && ldv >= (long)nkv * hd), "attn_decode_fused: a k or v row stride is below nkv*hd");
     AGAVE_CHECK(rot_half >= 0 && 2 * rot_half <= hd && (rot_half == 0 || inv_freq), "attn_decode_fused: bad rotation (rotary_dim %d, head_dim %d)", 2 * rot_half, hd);
-    QkFuse f{(const bf16*)k, ldk, (const bf16*)v, ldv, q_gain, k_gain, eps_q, eps_k, inv_freq, rot_half, pos_scale};
+    AGAVE_CHECK(slices >= 0 && slices <= QK_MAX_SLICES && (slices == 0 || slice_stride > 0), "attn_decode_fused: %d slices", slices);
+    AGAVE_CHECK(slices == 0 || (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 3) == 0, "attn_decode_fused: unaligned slices");
+    QkFuse f{(const bf16*)k, ldk, (const bf16*)v, ldv, q_gain, k_gain, eps_q, eps_k, inv_freq, rot_half, pos_scale, slices, slice_stride};
     return launch_decode<true>(a, f, N, stream, !leave_partials);
 }
 

@@ -6,7 +6,7 @@ from typing import Optional
 import torch
 
 from ..cache import PAGE
-from . import attention_mfma, kernels
+from . import attention_mfma, gemm_mfma, kernels
 
 
 def attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
@@ -22,6 +22,15 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages
     kernels.attn_plain(q, out, k_pages, v_pages, table, base, step.tok_seq, step.tok_pos, n_heads, n_kv, head_dim, scale, window,
                        one_token_each=one_each, span=step.page_span(window) if one_each else 1, workspace=step.workspace, most_seqs=step.most_seqs,
                        most_keys=step.max_len if step.fixed_span is None else PAGE * step.fixed_span)
+
+
+def adds_slices(n: int, qkv, head_dim: int) -> bool:
+    """Whether a decode step of ``n`` tokens hands its attention the q/k/v product (a Linear) as 32-bit slices.  From 17 tokens on: one
+    product either fills few compute units with tiles or brings all of its rows to every row block (4,096 rows of 2,560, us, one product
+    and four slices: 17 tokens 8.1 and 7.1, 32 8.8 and 7.4, 64 10.6 and 8.0; a decode step 2.52 and 2.51 ms, 2.59 and 2.55, 2.82 and 2.75).
+    With fewer tokens the plans make one product of it at these sizes."""
+    return (head_dim in attention_mfma.FUSED_HEAD_DIMS and qkv.packed is not None and 17 <= n <= gemm_mfma.SKINNY_MAX_M
+            and gemm_mfma.slices_for(n, qkv.out_features, qkv.in_features) <= attention_mfma.QK_MAX_SLICES)
 
 
 def tokens_apart(step) -> int:

@@ -12,7 +12,7 @@ kernels.register_signatures("attention_mfma", {
     "agave_attn_decode_mfma": [_P, _L, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _F, _I, _I, _I, _I,
                                _I, _P],
     "agave_attn_decode_fused": [_P, _L, _P, _L, _P, _L, _P, _P, _F, _F, _P, _I, _F, _P, _L, _P, _P, _P, _P, _P, _I, _P, _I,
-                                _P, _P, _I, _I, _I, _I, _F, _I, _I, _I, _I, _I, _I, _P],
+                                _P, _P, _I, _I, _I, _I, _F, _I, _I, _I, _I, _I, _I, _I, _L, _P],
     "agave_attn_prefill_mfma": [_P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P],
     "agave_attn_prefill_items_hw": [_I, _I],
     "agave_attn_prefill_items": [_P, _L, _P, _L, _P, _P, _P, _I, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _F, _I, _P, _I, _I,
@@ -20,6 +20,7 @@ kernels.register_signatures("attention_mfma", {
 })
 
 FUSED_HEAD_DIMS = (64, 128, 256)
+QK_MAX_SLICES = 4            # 32-bit slices of the raw projections that the decode kernel adds up
 MAX_SPLITS = 64              # what the merge inside the output product takes
 SPLITS_AT_ONCE = 12          # and what it merges with one round trip to memory (at a batch of 1, 12 splits
                              # measured as fast as 16)
@@ -213,7 +214,8 @@ def decode_fused(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.T
                  table: torch.Tensor, base: torch.Tensor, step, n_heads: int, n_kv: int, head_dim: int, scale: float,
                  window: Optional[int], partials_ok=None):
     """A decode step's attention from the raw projections: the kernel normalises and rotates q and
-    k, writes k and v into their pages (``k`` None: nothing is appended) and attends.
+    k, writes k and v into their pages (``k`` None: nothing is appended) and attends.  q, k and v may be float32
+    [slices, n, columns] with one stride between slices (at most ``QK_MAX_SLICES``), whose slices add up to the projections.
     ``partials_ok``: a function of the number of splits that says whether the caller's next kernel
     can merge the splits' partial results itself; if it says so and the step is split, they are returned as ``(part_o [n, heads, splits, head_dim], part_ml [n, heads,
     splits, 2])`` and ``out`` is left alone.  Otherwise None is returned and ``out`` is written."""
@@ -224,10 +226,16 @@ def decode_fused(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.T
                           ("out", out, n_heads * head_dim)):
         if t is None:
             continue
-        if not t.is_cuda or t.dtype != torch.bfloat16 or t.shape != (n, cols) or t.stride(1) != 1:
+        if q.dim() == 3 and name != "out":
+            if not t.is_cuda or t.dtype != torch.float32 or t.shape != (q.shape[0], n, cols) or t.stride(2) != 1 \
+                    or t.stride(0) != q.stride(0) or not 1 <= q.shape[0] <= QK_MAX_SLICES:
+                raise ValueError(f"decode_fused: {name} must be float32 [slices, {n}, {cols}] on the GPU with contiguous rows, at most "
+                                 f"{QK_MAX_SLICES} slices, as far apart as q's")
+        elif not t.is_cuda or t.dtype != torch.bfloat16 or t.shape != (n, cols) or t.stride(1) != 1:
             raise ValueError(f"decode_fused: {name} must be bfloat16 [{n}, {cols}] on the GPU with contiguous rows")
     if (k is None) != (v is None):
         raise ValueError("decode_fused: k and v come together")
+    slices, slice_stride = (q.shape[0], q.stride(0)) if q.dim() == 3 else (0, 0)
     kernels._f32vec(q_gain, "q_gain", head_dim)
     kernels._f32vec(k_gain, "k_gain", head_dim)
     rot_half = 0
@@ -235,7 +243,7 @@ def decode_fused(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.T
         rot_half = inv_freq.numel()
         kernels._f32vec(inv_freq, "inv_freq", rot_half)
     kernels._dev(q, k, v, out, q_gain, k_gain, inv_freq, k_pages, v_pages, table, base)
-    n_pages = kernels._check_pages(k_pages, v_pages, n_kv, head_dim, q.dtype, packed=True)
+    n_pages = kernels._check_pages(k_pages, v_pages, n_kv, head_dim, out.dtype, packed=True)
     width = kernels._check_table(table, base, step.tok_seq)
     span = step.page_span(window)
     chunks = -(-(n_heads // n_kv) // 16)
@@ -246,14 +254,15 @@ def decode_fused(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.T
         part_o = ws.get("attn_part_o", n * n_heads * splits, head_dim, torch.float32)
         part_ml = ws.get("attn_part_ml", n * n_heads * splits, 2, torch.float32)
     leave = bool(splits > 1 and partials_ok is not None and partials_ok(splits))
-    library.call(kernels.lib("attention_mfma"), "agave_attn_decode_fused", q.data_ptr(), q.stride(0),
-                 kernels.ptr(k), k.stride(0) if k is not None else 0, kernels.ptr(v),
-                 v.stride(0) if v is not None else 0, kernels.ptr(q_gain), kernels.ptr(k_gain), eps_q, eps_k,
+    library.call(kernels.lib("attention_mfma"), "agave_attn_decode_fused", q.data_ptr(), q.stride(-2),
+                 kernels.ptr(k), k.stride(-2) if k is not None else 0, kernels.ptr(v),
+                 v.stride(-2) if v is not None else 0, kernels.ptr(q_gain), kernels.ptr(k_gain), eps_q, eps_k,
                  kernels.ptr(inv_freq), rot_half, pos_scale, out.data_ptr(), out.stride(0), kernels.ptr(part_o),
                  kernels.ptr(part_ml), k_pages.data_ptr(), v_pages.data_ptr(), table.data_ptr(), width,
                  base.data_ptr(), n_pages, step.tok_seq.data_ptr(), step.tok_pos.data_ptr(), n, n_heads, n_kv,
                  head_dim, scale, int(window or 0), splits, per, 1 if step.n_seqs == n else 0,
-                 1 if getattr(step, "tables_start_at_reach", False) else 0, 1 if leave else 0, kernels.stream())
+                 1 if getattr(step, "tables_start_at_reach", False) else 0, 1 if leave else 0, slices, slice_stride,
+                 kernels.stream())
     if leave:
         return part_o.view(n, n_heads, splits, head_dim), part_ml.view(n, n_heads, splits, 2)
     return None

@@ -1793,3 +1793,40 @@ def test_attn_decode_fused_own_row(K, nh, nkv, hd, window, lens, from_reach):
                       _i32([b for b, L in enumerate(lens) for _ in range(L)]), _i32([i for L in lens for i in range(L)]), want_k, want_v,
                       full.to(DEV), _i32([0] * B), 0, nkv, hd, packed=True)
     assert torch.equal(kp, want_k) and torch.equal(vp, want_v)
+
+
+@pytest.mark.parametrize("slices", [1, 2, 3, 4])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 4, 256), (5, 1, 128), (18, 1, 64)])
+def test_attn_decode_fused_adds_slices_of_the_projections(K, nh, nkv, hd, slices):
+    """Raw projections as 32-bit slices leave the bits that their sum leaves in bfloat16 (whole 64ths below 2: every sum is exact in
+    both types).  The slices lie side by side, q, k and v of one product."""
+    from agave_amd.ops import attention_mfma as A
+    g = torch.Generator().manual_seed(slices)
+    lens, cols = [1, 40, 64, 200, 97], (nh + 2 * nkv) * hd
+    B, n_pages = len(lens), 12
+    table = torch.full((B, 4), -1, dtype=torch.int32)
+    perm = torch.randperm(n_pages, generator=g).tolist()
+    for b, L in enumerate(lens):
+        for i in range((L + 63) // 64):
+            table[b, i] = perm.pop()
+    parts = torch.randint(-31, 32, (slices, B, cols), generator=g).float() / 64
+    whole = parts.sum(0).bfloat16()
+    assert torch.equal(whole.float(), parts.sum(0))
+    gain = (1 + 0.2 * torch.randn(hd, generator=g)).to(DEV)
+    inv_freq = torch.exp(-torch.arange(hd // 2).float() / hd * 5).to(DEV)
+    pages = [torch.randn(n_pages, nkv, 64, hd, generator=g).bfloat16().to(DEV), torch.randn(n_pages, nkv, hd, 64, generator=g).bfloat16().to(DEV)]
+    step = _FakeStep(lens, lambda L: L - 1, None)
+    outs = []
+    for rows in (whole.to(DEV), parts.to(DEV)):
+        q, k, v = rows.split((nh * hd, nkv * hd, nkv * hd), dim=-1)
+        kp, vp = pages[0].clone(), pages[1].clone()
+        out = torch.full((B, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        A.decode_fused(q, k, v, out, gain, gain, 1e-6, 1e-6, inv_freq, 1.0, kp, vp, table.to(DEV), _i32([0] * B), step, nh, nkv, hd, 0.1, None)
+        outs.append((out, kp, vp))
+    assert torch.isfinite(outs[0][0].float()).all()
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    q5 = torch.zeros(5, B, nh * hd, device=DEV)
+    with pytest.raises(ValueError):
+        A.decode_fused(q5, None, None, outs[0][0], gain, gain, 1e-6, 1e-6, inv_freq, 1.0, kp, vp, table.to(DEV), _i32([0] * B), step, nh, nkv,
+                       hd, 0.1, None)
