@@ -39,25 +39,30 @@ __device__ __forceinline__ float lanes16_sum(float v) {
 // z-th of them in a workgroup of its own.
 // gridDim.y workgroups share a row's pages and leave (sum, maximum, unnormalised result) for attn_plain_merge_kernel: with a
 // token per sequence there are few rows and the pages one after another bound the time.
-// NT: tiles of 64 value elements (16 a wave).  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of
+// NT: tiles of 64 value elements (16 a wave).  FULL: the head is as long as they are.  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of
 // 0 must not meet a value that is not finite (a key behind a token's position may hold anything): such pages are summed element
 // by element.
 // Bound by the 32-bit products (half of them for a token of 4 rows' padding) and, with few tokens, by the loads' way from memory.
 // Measured, 16 heads on 4 key heads of 128 in 32 bits: prompts of 97, 259 and 421 tokens 63 us (a workgroup per token and head, a
 // key a thread: 943 us), 2,000 tokens 0.45 ms (16.8 ms); a token each behind as many keys 15 us (59 us), behind 4,000 keys
 // 33 us (562 us).  Errors against 64 bits are half as large (2.0 to 2.8e-7 after 4.2 to 5.5e-7).
-template <typename T, int NT, bool VEC, bool VEC_V>
+// A token each is a chain: the position, the page's id, its keys, products, sums, values, the store; 10.2 us inside, of which the queries'
+// way to LDS took 1.8, the id 1.0 and the keys behind it 4.0.  Now the first page travels while the queries are staged, all of its
+// keys at once, and rows' tokens come from a table and not from divisions: a decode step of three sequences through eight layers
+// 634 -> 610 us, prompts of 97 and 421 tokens 1.31 -> 1.26 and 2.94 -> 2.79 ms.
+template <typename T, int NT, bool VEC, bool VEC_V, bool FULL>
 __global__ __launch_bounds__(256) void attn_plain_kernel(
     const T* __restrict__ q, long ldq, T* __restrict__ out, long ldo, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ table, int width, const int* __restrict__ base,
     int n_pages, const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, int N, int nh, int nkv, int hd,
     float scale, int window, int run, float* __restrict__ part_o, float* __restrict__ part_ml) {
     constexpr int HDP = NT * 64;
+    if constexpr (FULL) hd = HDP;
     constexpr bool V_AHEAD = NT <= 4;                        // a page's values are asked for before its scores are made
     __shared__ __attribute__((aligned(16))) float Qs[ROWS][HDP + 4];
     __shared__ __attribute__((aligned(16))) float P[ROWS][AGAVE_PAGE + 4];
     __shared__ __attribute__((aligned(16))) float wmax[4][ROWS], wsum[4][ROWS];
-    __shared__ __attribute__((aligned(16))) int row_pos[ROWS], row_lo[ROWS], row_seq[ROWS];
+    __shared__ __attribute__((aligned(16))) int row_pos[ROWS], row_lo[ROWS], row_seq[ROWS], row_tok[ROWS];
 
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const int G = nh / nkv, chunks = (G + ROWS - 1) / ROWS;
@@ -77,19 +82,62 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
     const int rows = min(tokens * heads, ROWS);
     const int split = blockIdx.y, splits = gridDim.y;
 
-    if (tid < ROWS) {
-        const int t = t0 + tid / heads;
-        const bool real = tid < rows;
-        const int p = real ? tok_pos[t] : -1;
-        row_pos[tid] = p;
-        row_lo[tid] = real && window > 0 && p - window + 1 > 0 ? p - window + 1 : 0;
-        row_seq[tid] = real ? tok_seq[t] : -1;
-    }
+    // One token (a decode step): its page ids need none of the other rows', and its first page travels while the queries are staged.
+    const bool one = tokens == 1;
+    const int one_seq = tok_seq[t0], one_pos = tok_pos[t0];
+    f32x4_t x[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {                           // four elements a thread and turn
         const int row = (tid + 256 * i) / (HDP / 4), d = (tid + 256 * i) % (HDP / 4) * 4, real = min(row, rows - 1);
-        const f32x4_t x = ld4<VEC>(q + (size_t)(t0 + real / heads) * ldq + (size_t)(head0 + real % heads) * hd, d, hd);
-        *reinterpret_cast<f32x4_t*>(&Qs[row][d]) = row < rows ? x : f32x4_t{0.f, 0.f, 0.f, 0.f};
+        const int tok = one ? 0 : real / heads;
+        x[i] = ld4<VEC>(q + (size_t)(t0 + tok) * ldq + (size_t)(head0 + real - tok * heads) * hd, d, hd);
+    }
+    auto page_of = [&](int seq, int pbase, int page) -> long {
+        const int col = page - pbase;
+        const long pg = col >= 0 && col < width ? table[(size_t)seq * width + col] : -1;
+        return pg >= n_pages ? -1 : pg;
+    };
+    constexpr int KD = FULL && V_AHEAD ? HDP / 16 : 1;       // a page's keys all at once, before its values
+    f32x4_t kk[KD], vv[V_AHEAD ? NT : 1][4];
+    auto values = [&](const T* vr, f32x4_t (&v)[4], int nt) {
+        const T* row = vr + (size_t)min((4 * nt + w) * 16 + r, hd - 1) * AGAVE_PAGE;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = ld4<VEC_V>(row, 16 * j + 4 * g, AGAVE_PAGE);
+    };
+    auto ask = [&](long pg) {
+        if constexpr (KD > 1) {
+            const T* kr = k_pages + ((size_t)(pg * nkv + kvh) * AGAVE_PAGE + 16 * w + r) * hd;
+#pragma unroll
+            for (int i = 0; i < KD; ++i) kk[i] = ld4<VEC>(kr, 16 * i + 4 * g, hd);
+        }
+        if constexpr (V_AHEAD)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) values(v_pages + (size_t)(pg * nkv + kvh) * hd * AGAVE_PAGE, vv[nt], nt);
+    };
+    int asked = -1;                                          // the page that has been asked for
+    if (one) {
+        const int lo = window > 0 && one_pos - window + 1 > 0 ? one_pos - window + 1 : 0;
+        const int first = lo / AGAVE_PAGE, count = one_pos / AGAVE_PAGE - first + 1, share = (count + splits - 1) / splits;
+        const int page = first + split * share;
+        const long pg = page < first + count ? page_of(one_seq, base[one_seq], page) : -1;
+        if (pg >= 0) {
+            ask(pg);
+            asked = page;
+        }
+    }
+    if (tid < ROWS) {
+        const int tok = one ? 0 : tid / heads, at = t0 + tok;
+        const bool real = tid < rows;
+        const int p = !real ? -1 : (one ? one_pos : tok_pos[at]);
+        row_pos[tid] = p;
+        row_lo[tid] = real && window > 0 && p - window + 1 > 0 ? p - window + 1 : 0;
+        row_seq[tid] = !real ? -1 : (one ? one_seq : tok_seq[at]);
+        row_tok[tid] = tok;
+    }
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const int row = (tid + 256 * i) / (HDP / 4), d = (tid + 256 * i) % (HDP / 4) * 4;
+        *reinterpret_cast<f32x4_t*>(&Qs[row][d]) = row < rows ? x[i] : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
     __syncthreads();
 
@@ -106,10 +154,11 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
     const int4 pos4 = *reinterpret_cast<const int4*>(&row_pos[4 * g]), lo4 = *reinterpret_cast<const int4*>(&row_lo[4 * g]);
     const int pos[4] = {pos4.x, pos4.y, pos4.z, pos4.w}, low[4] = {lo4.x, lo4.y, lo4.z, lo4.w};
 
+    bool fresh = true;                                       // no page has been used yet
     for (int s0 = 0, s1; s0 < rows; s0 = s1) {               // a run of rows of one sequence
-        const int seq = row_seq[s0];
+        const int seq = one ? one_seq : row_seq[s0];
         int lo = row_lo[s0], hi = row_pos[s0];
-        for (s1 = s0 + 1; s1 < rows && row_seq[s1] == seq; ++s1) {
+        for (s1 = one ? rows : s0 + 1; s1 < rows && row_seq[s1] == seq; ++s1) {
             lo = min(lo, row_lo[s1]);
             hi = max(hi, row_pos[s1]);
         }
@@ -117,28 +166,26 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
         const int first = lo / AGAVE_PAGE, count = hi / AGAVE_PAGE - first + 1, share = (count + splits - 1) / splits;
         const int from = first + split * share, to = min(from + share, first + count), pbase = base[seq];
         for (int page = from; page < to; ++page) {
-            const int col = page - pbase;
-            const long pg = col >= 0 && col < width ? table[(size_t)seq * width + col] : -1;
-            if (pg < 0 || pg >= n_pages) continue;
+            const long pg = page_of(seq, pbase, page);
+            if (pg < 0) continue;
             const T* kr = k_pages + ((size_t)(pg * nkv + kvh) * AGAVE_PAGE + 16 * w + r) * hd;
             const T* vr = v_pages + (size_t)(pg * nkv + kvh) * hd * AGAVE_PAGE;
             const int key0 = page * AGAVE_PAGE;
-            f32x4_t vv[V_AHEAD ? NT : 1][4];
-            auto values = [&](f32x4_t (&v)[4], int nt) {
-                const T* row = vr + (size_t)min((4 * nt + w) * 16 + r, hd - 1) * AGAVE_PAGE;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) v[j] = ld4<VEC_V>(row, 16 * j + 4 * g, AGAVE_PAGE);
-            };
-            if constexpr (V_AHEAD)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) values(vv[nt], nt);
+            if (page != asked) ask(pg);
+            asked = -1;
             // scores of keys 16 w + r
             f32x4_t sum[4] = {};
-#pragma unroll 8
-            for (int d = 0; d < hd; d += 16) {
-                const f32x4_t kv = ld4<VEC>(kr, d + 4 * g, hd), qv = *reinterpret_cast<const f32x4_t*>(&Qs[r][d + 4 * g]);
+            auto scores = [&](f32x4_t kv, int d) {
+                const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(&Qs[r][d + 4 * g]);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) sum[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv[e], kv[e], sum[e], 0, 0, 0);
+            };
+            if constexpr (KD > 1) {
+#pragma unroll
+                for (int i = 0; i < KD; ++i) scores(kk[i], 16 * i);
+            } else {
+#pragma unroll 8
+                for (int d = 0; d < hd; d += 16) scores(ld4<VEC>(kr, d + 4 * g, hd), d);
             }
             f32x4_t s = (sum[0] + sum[1]) + (sum[2] + sum[3]);
             const int key = key0 + 16 * w + r;
@@ -159,7 +206,8 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
                 const int row = 4 * g + e;
                 const float m_new = fmaxf(m[e], fmaxf(fmaxf(wmax[0][row], wmax[1][row]), fmaxf(wmax[2][row], wmax[3][row])));
                 // m_new is finite whenever any key of this or an earlier page was seen
-                alpha[e] = m[e] == -INFINITY ? 0.f : expf(m[e] - m_new);
+                alpha[e] = 0.f;
+                if (!fresh) alpha[e] = m[e] == -INFINITY ? 0.f : expf(m[e] - m_new);
                 const float pr = seen[e] ? expf(s[e] - m_new) : 0.f;
                 m[e] = m_new;
                 P[row][16 * w + r] = pr;
@@ -172,6 +220,8 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
                 const int row = 4 * g + e;
                 l[e] = l[e] * alpha[e] + ((wsum[0][row] + wsum[1][row]) + (wsum[2][row] + wsum[3][row]));
             }
+            fresh = false;
+            const bool inside = key0 >= lo && key0 + AGAVE_PAGE - 1 <= hi;
             f32x4_t pf[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) pf[j] = *reinterpret_cast<const f32x4_t*>(&P[r][16 * j + 4 * g]);
@@ -179,18 +229,24 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
             for (int nt = 0; nt < NT; ++nt) {
                 if ((4 * nt + w) * 16 >= hd) continue;
                 f32x4_t late[4];
-                if constexpr (!V_AHEAD) values(late, nt);
+                if constexpr (!V_AHEAD) values(vr, late, nt);
                 f32x4_t (&v)[4] = V_AHEAD ? vv[V_AHEAD ? nt : 0] : late;
                 f32x4_t add = {};
-                bool finite = true;
+                if (!inside) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int at = key0 + 16 * j + 4 * g + e;
+                            if (at < lo || at > hi) v[j][e] = 0.f;     // (no row sees it: it may hold anything)
+                        }
+                }
+                float nothing = 0.f;                         // (0 times what is not finite is not a number)
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int at = key0 + 16 * j + 4 * g + e;
-                        if (at < lo || at > hi) v[j][e] = 0.f;         // (no row sees it: it may hold anything)
-                        finite = finite && fabsf(v[j][e]) < INFINITY;
-                    }
+                    for (int e = 0; e < 4; ++e) nothing = fmaf(v[j][e], 0.f, nothing);
+                const bool finite = nothing == 0.f;
                 if (__all(finite)) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
@@ -216,8 +272,9 @@ __global__ __launch_bounds__(256) void attn_plain_kernel(
     for (int e = 0; e < 4; ++e) {
         const int row = 4 * g + e;
         if (row >= rows) continue;
-        const size_t t = t0 + row / heads;
-        const int h = head0 + row % heads;
+        const int tok = row_tok[row];
+        const size_t t = t0 + tok;
+        const int h = head0 + row - tok * heads;
         const float inv = l[e] > 0.f ? 1.0f / l[e] : 0.f;
         const size_t part = (t * nh + h) * splits + split;
 #pragma unroll
@@ -381,9 +438,12 @@ static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages
 #undef FEW_GO
         return;
     }
-#define PLAIN_GO(VEC_, VEC_V_) attn_plain_kernel<T, NT, VEC_, VEC_V_><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, table, width, \
-        base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml)
-    if (vec) PLAIN_GO(true, true); else if (vec_v) PLAIN_GO(false, true); else PLAIN_GO(false, false);
+#define PLAIN_GO(VEC_, VEC_V_, FULL_) attn_plain_kernel<T, NT, VEC_, VEC_V_, FULL_><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, \
+        table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml)
+    if (vec && NT <= 4 && hd == NT * 64) PLAIN_GO(true, true, (NT <= 4));
+    else if (vec) PLAIN_GO(true, true, false);
+    else if (vec_v) PLAIN_GO(false, true, false);
+    else PLAIN_GO(false, false, false);
 #undef PLAIN_GO
     if (splits > 1) attn_plain_merge_kernel<T><<<N * nh, 128, 0, stream>>>(part_o, part_ml, out, ldo, nh, hd, splits);
 }

@@ -1830,3 +1830,36 @@ def test_attn_decode_fused_adds_slices_of_the_projections(K, nh, nkv, hd, slices
     with pytest.raises(ValueError):
         A.decode_fused(q5, None, None, outs[0][0], gain, gain, 1e-6, 1e-6, inv_freq, 1.0, kp, vp, table.to(DEV), _i32([0] * B), step, nh, nkv,
                        hd, 0.1, None)
+
+
+# Heads as long as the kernel's tiles: a page's keys and values are asked for at once, one token's before its queries are there.
+@pytest.mark.parametrize("nh,nkv,hd,window", [(8, 4, 64, 66), (34, 2, 64, None), (16, 4, 128, 130), (6, 6, 256, None), (4, 2, 256, 3)])
+def test_attn_plain_heads_of_whole_tiles(K, nh, nkv, hd, window):
+    for dtype in (torch.float32, torch.bfloat16):
+        test_attn_plain_rows(K, dtype, nh, nkv, hd, window)
+    if window is None:
+        for n in (90, 170):
+            test_attn_plain_values_that_are_not_finite(K, n, hd)
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256, 100])
+def test_attn_plain_pages_that_are_not_there(K, hd):
+    """Keys of pages that the table does not name count as unseen, the first, the last and one between, whoever asks for them first."""
+    from agave_amd.parts import Workspace
+    nh, nkv, ctx = 4, 2, 300
+    g = torch.Generator().manual_seed(hd)
+    kp, vp = (torch.randn(5, nkv, *shape, generator=g).to(DEV) for shape in ((64, hd), (hd, 64)))
+    q = torch.randn(3, nh * hd, generator=g).to(DEV)
+    table = torch.tensor([[-1, 1, 2, 3, 4], [0, 1, 9, 3, 4], [0, 1, 2, 3, -1]], dtype=torch.int32, device=DEV)
+    k, v = kp.cpu().double(), vp.cpu().double()
+    ref = torch.empty(3, nh, hd, dtype=torch.float64)
+    for b, gone in enumerate((0, 2, 4)):
+        seen = [i for i in range(ctx) if i // 64 != gone]
+        for h in range(nh):
+            keys = torch.stack([k[i // 64, h // 2, i % 64] for i in seen])
+            vals = torch.stack([v[i // 64, h // 2, :, i % 64] for i in seen])
+            ref[b, h] = torch.softmax(0.2 * keys @ q.cpu().double().view(3, nh, hd)[b, h], 0) @ vals
+    for more in ({}, {"span": 5, "workspace": Workspace(torch.device(DEV))}):
+        out = torch.empty_like(q)
+        K.attn_plain(q, out, kp, vp, table, _i32([0] * 3), _i32([0, 1, 2]), _i32([ctx - 1] * 3), nh, nkv, hd, 0.2, None, one_token_each=True, **more)
+        assert torch.allclose(out.cpu().double().view(3, nh, hd), ref, atol=2e-6 + 1e-7 * hd, rtol=2e-5)
