@@ -649,16 +649,20 @@ extern "C" int agave_residual_layernorm(int dtype, float* h, const void* branch,
 // NV: groups of 64 elements a head has (1, 2, 4 or 8).  Everything a wave needs is asked for at
 // its start: its row with the gains and frequencies, the value row, the position and the
 // sequence; the page id follows as soon as those two are there and travels during the arithmetic.
-template <typename T, int NV>
-__global__ void qk_norm_rope_kv_kernel(const T* q, long ldq, const T* __restrict__ k, long ldk,
-                                       const T* __restrict__ v, long ldv, T* q_out, long ldqo,
+// Raw float beside T bf16: q, k and v are `slices` 32-bit slices each, slice_stride elements apart, that add up to the rows (a product
+// of few tokens that was shared out along its columns).
+#define QK_MAX_SLICES 4
+template <typename T, int NV, typename Raw>
+__global__ void qk_norm_rope_kv_kernel(const Raw* q, long ldq, const Raw* __restrict__ k, long ldk,
+                                       const Raw* __restrict__ v, long ldv, T* q_out, long ldqo,
                                        const float* __restrict__ q_gain, const float* __restrict__ k_gain,
                                        float eps_q, float eps_k, const float* __restrict__ inv_freq,
                                        int rot_half, float pos_scale, const int* __restrict__ tok_seq,
                                        const int* __restrict__ tok_pos, T* __restrict__ k_pages,
                                        T* __restrict__ v_pages, const int* __restrict__ table, int width,
                                        const int* __restrict__ base, int n_pages, int N, int nh, int nkv, int hd,
-                                       int packed) {
+                                       int packed, int slices, long slice_stride) {
+    constexpr int MORE = sizeof(Raw) > sizeof(T) ? QK_MAX_SLICES - 1 : 0;
     __shared__ float buf[4][NV * 64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int heads = nh + nkv;
@@ -668,22 +672,31 @@ __global__ void qk_norm_rope_kv_kernel(const T* q, long ldq, const T* __restrict
     const int hh = active ? unit % heads : 0;
     const bool is_q = hh < nh;
     const int head = is_q ? hh : hh - nh;
-    const T* src = is_q ? q + (size_t)t * ldq + (size_t)head * hd : k + (size_t)t * ldk + (size_t)head * hd;
+    const Raw* src = is_q ? q + (size_t)t * ldq + (size_t)head * hd : k + (size_t)t * ldk + (size_t)head * hd;
     const float* gain = is_q ? q_gain : k_gain;
     const float eps = is_q ? eps_q : eps_k;
     float* y = buf[wave];
 
-    const QkRow<T, NV> row = qk_row_load<T, NV>(src, gain, inv_freq, rot_half, hd, lane);
-    const int p = tok_pos[t];
-    T vreg[NV];
-    int b = 0;
-    if (!is_q) {                       // a key's wave also takes the value row, and looks its page up
-        const T* sv = v + (size_t)t * ldv + (size_t)head * hd;
+    QkRow<Raw, NV> row = qk_row_load<Raw, NV>(src, gain, inv_freq, rot_half, hd, lane);
+    Raw more[MORE + 1][NV], vraw[MORE + 1][NV];
+#pragma unroll
+    for (int s = 1; s <= MORE; ++s)
 #pragma unroll
         for (int kk = 0; kk < NV; ++kk) {
             const int d = lane + 64 * kk;
-            vreg[kk] = sv[d < hd ? d : 0];
+            more[s][kk] = src[(size_t)(s < slices ? s : 0) * slice_stride + (d < hd ? d : 0)];
         }
+    const int p = tok_pos[t];
+    int b = 0;
+    if (!is_q) {                       // a key's wave also takes the value row, and looks its page up
+        const Raw* sv = v + (size_t)t * ldv + (size_t)head * hd;
+#pragma unroll
+        for (int s = 0; s <= MORE; ++s)
+#pragma unroll
+            for (int kk = 0; kk < NV; ++kk) {
+                const int d = lane + 64 * kk;
+                vraw[s][kk] = sv[(s > 0 && s < slices ? (size_t)s * slice_stride : 0) + (d < hd ? d : 0)];
+            }
         b = tok_seq[t];
     }
     int col = 0;
@@ -693,7 +706,14 @@ __global__ void qk_norm_rope_kv_kernel(const T* q, long ldq, const T* __restrict
         col = p / AGAVE_PAGE - base[b];
         if (col >= 0 && col < width) pg = table[(size_t)b * width + col];
     }
-    qk_row_finish<T, NV>(row, y, gain != nullptr, eps, rot_half, (float)p * pos_scale, hd, lane, active);
+    if constexpr (MORE > 0) {
+#pragma unroll
+        for (int s = 1; s <= MORE; ++s)
+#pragma unroll
+            for (int kk = 0; kk < NV; ++kk)
+                if (s < slices) row.xr[kk] += more[s][kk];
+    }
+    qk_row_finish<Raw, NV>(row, y, gain != nullptr, eps, rot_half, (float)p * pos_scale, hd, lane, active);
     if (!active) return;
     if (is_q) {
         T* dst = q_out + (size_t)t * ldqo + (size_t)head * hd;
@@ -705,6 +725,19 @@ __global__ void qk_norm_rope_kv_kernel(const T* q, long ldq, const T* __restrict
         return;
     }
     if (pg < 0 || pg >= n_pages) return;   // a table the host built wrongly: write nothing
+    T vreg[NV];
+#pragma unroll
+    for (int kk = 0; kk < NV; ++kk) {
+        if constexpr (MORE > 0) {
+            Raw x = vraw[0][kk];
+#pragma unroll
+            for (int s = 1; s <= MORE; ++s)
+                if (s < slices) x += vraw[s][kk];
+            st(&vreg[kk], x);
+        } else {
+            vreg[kk] = vraw[0][kk];
+        }
+    }
     if (!packed) {
         T* dk = k_pages + (((size_t)pg * nkv + head) * AGAVE_PAGE + row_in_page) * hd;
         T* dv = v_pages + ((size_t)pg * nkv + head) * hd * AGAVE_PAGE + row_in_page;
@@ -939,18 +972,18 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kv_tokens_kernel(const bf16*
     }
 }
 
-template <typename T>
+template <typename T, typename Raw>
 static void launch_qk_norm_rope_kv(int blocks, hipStream_t stream, const void* q, long ldq, const void* k, long ldk,
                                    const void* v, long ldv, void* q_out, long ldqo, const float* q_gain,
                                    const float* k_gain, float eps_q, float eps_k, const float* inv_freq, int rot_half,
                                    float pos_scale, const int* tok_seq, const int* tok_pos, void* k_pages, void* v_pages,
                                    const int* table, int width, const int* base, int n_pages, int N, int nh, int nkv,
-                                   int hd, int packed) {
+                                   int hd, int packed, int slices = 0, long slice_stride = 0) {
 #define QK_LAUNCH(NV_)                                                                                               \
-    qk_norm_rope_kv_kernel<T, NV_><<<blocks, 256, 0, stream>>>(                                                      \
-        (const T*)q, ldq, (const T*)k, ldk, (const T*)v, ldv, (T*)q_out, ldqo, q_gain, k_gain, eps_q, eps_k, inv_freq, \
+    qk_norm_rope_kv_kernel<T, NV_, Raw><<<blocks, 256, 0, stream>>>(                                                 \
+        (const Raw*)q, ldq, (const Raw*)k, ldk, (const Raw*)v, ldv, (T*)q_out, ldqo, q_gain, k_gain, eps_q, eps_k, inv_freq, \
         rot_half, pos_scale, tok_seq, tok_pos, (T*)k_pages, (T*)v_pages, table, width, base, n_pages, N, nh, nkv, hd, \
-        packed)
+        packed, slices, slice_stride)
     if (hd <= 64) QK_LAUNCH(1);
     else if (hd <= 128) QK_LAUNCH(2);
     else if (hd <= 256) QK_LAUNCH(4);
@@ -963,7 +996,7 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
                                      float eps_q, float eps_k, const float* inv_freq, int rot_half, float pos_scale,
                                      const int* tok_seq, const int* tok_pos, void* k_pages, void* v_pages,
                                      const int* table, int width, const int* base, int n_pages, int N, int nh,
-                                     int nkv, int hd, int packed, int apart, hipStream_t stream) {
+                                     int nkv, int hd, int packed, int apart, int slices, long slice_stride, hipStream_t stream) {
     AGAVE_CHECK(N >= 0 && nh >= 0 && nkv >= 0 && hd > 0, "qk_norm_rope_kv: bad sizes N=%d nh=%d nkv=%d hd=%d", N, nh, nkv, hd);
     AGAVE_CHECK(hd <= QK_HD_MAX, "qk_norm_rope_kv: head_dim %d exceeds the supported maximum %d", hd, QK_HD_MAX);
     AGAVE_CHECK(rot_half >= 0 && 2 * rot_half <= hd, "qk_norm_rope_kv: rotary_dim %d exceeds head_dim %d", 2 * rot_half, hd);
@@ -974,6 +1007,8 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
                 "qk_norm_rope_kv: bad k/v buffers or cache table");
     AGAVE_CHECK(tok_pos != nullptr, "qk_norm_rope_kv: positions are null");
     AGAVE_CHECK(!packed || (dtype == AGAVE_BF16 && hd % 16 == 0), "qk_norm_rope_kv: packed pages need bfloat16 and head_dim %% 16 == 0");
+    AGAVE_CHECK(slices >= 0 && slices <= QK_MAX_SLICES && (slices == 0 || (dtype == AGAVE_BF16 && slice_stride > 0)),
+                "qk_norm_rope_kv: %d slices (at most %d, of bfloat16 activations)", slices, QK_MAX_SLICES);
     const long units = (long)N * (nh + nkv);
     if (units == 0) return 0;
     AGAVE_CHECK(units < (1L << 31) - 4, "qk_norm_rope_kv: %ld (token, head) pairs exceed what one launch takes", units);
@@ -992,7 +1027,7 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
     const uintptr_t addresses = (nh ? (uintptr_t)q | (uintptr_t)q_out : 0) | (nkv ? (uintptr_t)k | (uintptr_t)v | (uintptr_t)k_pages | (uintptr_t)v_pages : 0) |
                                 (uintptr_t)q_gain | (uintptr_t)k_gain | (uintptr_t)(rot_half ? inv_freq : nullptr);
     const long strides = (nh ? ldq | ldqo : 0) | (nkv ? ldk | ldv : 0);
-    if (dtype == AGAVE_BF16 && (packed || nkv == 0) && (hd == 128 || hd == 256) && (rot_half == 0 || rot_half == hd / 2) &&
+    if (dtype == AGAVE_BF16 && slices == 0 && (packed || nkv == 0) && (hd == 128 || hd == 256) && (rot_half == 0 || rot_half == hd / 2) &&
         units >= line && addresses % 16 == 0 && strides % 8 == 0) {
         const long waves = (long)((N + 3) / 4) * ((nh + 3) / 4 + 2 * ((nkv + 3) / 4));
         const int grid = (int)(8 * (((waves + 3) / 4 + 7) / 8));
@@ -1007,12 +1042,16 @@ extern "C" int agave_qk_norm_rope_kv(int dtype, const void* q, long ldq, const v
         return 0;
     }
     const int blocks = (int)((units + 3) / 4);
-    if (dtype == AGAVE_F32)
-        launch_qk_norm_rope_kv<float>(blocks, stream, q, ldq, k, ldk, v, ldv, q_out, ldqo, q_gain, k_gain, eps_q, eps_k,
+    if (slices > 0)
+        launch_qk_norm_rope_kv<bf16, float>(blocks, stream, q, ldq, k, ldk, v, ldv, q_out, ldqo, q_gain, k_gain, eps_q, eps_k,
+                                            inv_freq, rot_half, pos_scale, tok_seq, tok_pos, k_pages, v_pages, table, width,
+                                            base, n_pages, N, nh, nkv, hd, packed, slices, slice_stride);
+    else if (dtype == AGAVE_F32)
+        launch_qk_norm_rope_kv<float, float>(blocks, stream, q, ldq, k, ldk, v, ldv, q_out, ldqo, q_gain, k_gain, eps_q, eps_k,
                                       inv_freq, rot_half, pos_scale, tok_seq, tok_pos, k_pages, v_pages, table, width,
                                       base, n_pages, N, nh, nkv, hd, packed);
     else if (dtype == AGAVE_BF16)
-        launch_qk_norm_rope_kv<bf16>(blocks, stream, q, ldq, k, ldk, v, ldv, q_out, ldqo, q_gain, k_gain, eps_q, eps_k,
+        launch_qk_norm_rope_kv<bf16, bf16>(blocks, stream, q, ldq, k, ldk, v, ldv, q_out, ldqo, q_gain, k_gain, eps_q, eps_k,
                                      inv_freq, rot_half, pos_scale, tok_seq, tok_pos, k_pages, v_pages, table, width,
                                      base, n_pages, N, nh, nkv, hd, packed);
     else

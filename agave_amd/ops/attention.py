@@ -24,13 +24,16 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_pages: torch.Tensor, v_pages
                        most_keys=step.max_len if step.fixed_span is None else PAGE * step.fixed_span)
 
 
-def adds_slices(n: int, qkv, head_dim: int) -> bool:
-    """Whether a decode step of ``n`` tokens hands its attention the q/k/v product (a Linear) as 32-bit slices.  From 17 tokens on: one
-    product either fills few compute units with tiles or brings all of its rows to every row block (4,096 rows of 2,560, us, one product
-    and four slices: 17 tokens 8.1 and 7.1, 32 8.8 and 7.4, 64 10.6 and 8.0; a decode step 2.52 and 2.51 ms, 2.59 and 2.55, 2.82 and 2.75).
-    With fewer tokens the plans make one product of it at these sizes."""
-    return (head_dim in attention_mfma.FUSED_HEAD_DIMS and qkv.packed is not None and 17 <= n <= gemm_mfma.SKINNY_MAX_M
-            and gemm_mfma.slices_for(n, qkv.out_features, qkv.in_features) <= attention_mfma.QK_MAX_SLICES)
+def adds_slices(step, qkv, head_dim: int) -> bool:
+    """Whether a step's q/k work is handed the q/k/v product (a Linear) as 32-bit slices.  From 17 tokens on: one product either fills few
+    compute units with tiles or brings all of its rows to every row block (4,096 rows of 2,560, us, one product and four slices: 17 tokens
+    8.1 and 7.1, 32 8.8 and 7.4, 64 10.6 and 8.0; a decode step 2.52 and 2.51 ms, 2.59 and 2.55, 2.82 and 2.75; a prompt of 20, 37 and 60 tokens
+    2.64 and 2.59, 2.74 and 2.71, 2.90 and 2.83).  With fewer tokens the plans make one product of it at these sizes.  Prompts of several
+    sequences are not recorded, and the host, which the GPU waits for there, has a little more to do with slices."""
+    n = step.n_tokens
+    return (17 <= n <= gemm_mfma.SKINNY_MAX_M and qkv.packed is not None
+            and (head_dim in attention_mfma.FUSED_HEAD_DIMS if step.is_decode else step.n_seqs == 1)
+            and gemm_mfma.slices_for(n, qkv.out_features, qkv.in_features) <= kernels.QK_MAX_SLICES)
 
 
 def tokens_apart(step) -> int:

@@ -20,7 +20,6 @@ kernels.register_signatures("attention_mfma", {
 })
 
 FUSED_HEAD_DIMS = (64, 128, 256)
-QK_MAX_SLICES = 4            # 32-bit slices of the raw projections that the decode kernel adds up
 MAX_SPLITS = 64              # what the merge inside the output product takes
 SPLITS_AT_ONCE = 12          # and what it merges with one round trip to memory (at a batch of 1, 12 splits
                              # measured as fast as 16)
@@ -215,7 +214,7 @@ def decode_fused(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.T
                  window: Optional[int], partials_ok=None):
     """A decode step's attention from the raw projections: the kernel normalises and rotates q and
     k, writes k and v into their pages (``k`` None: nothing is appended) and attends.  q, k and v may be float32
-    [slices, n, columns] with one stride between slices (at most ``QK_MAX_SLICES``), whose slices add up to the projections.
+    [slices, n, columns] with one stride between slices (at most ``kernels.QK_MAX_SLICES``), whose slices add up to the projections.
     ``partials_ok``: a function of the number of splits that says whether the caller's next kernel
     can merge the splits' partial results itself; if it says so and the step is split, they are returned as ``(part_o [n, heads, splits, head_dim], part_ml [n, heads,
     splits, 2])`` and ``out`` is left alone.  Otherwise None is returned and ``out`` is written."""
@@ -228,9 +227,9 @@ def decode_fused(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torch.T
             continue
         if q.dim() == 3 and name != "out":
             if not t.is_cuda or t.dtype != torch.float32 or t.shape != (q.shape[0], n, cols) or t.stride(2) != 1 \
-                    or t.stride(0) != q.stride(0) or not 1 <= q.shape[0] <= QK_MAX_SLICES:
+                    or t.stride(0) != q.stride(0) or not 1 <= q.shape[0] <= kernels.QK_MAX_SLICES:
                 raise ValueError(f"decode_fused: {name} must be float32 [slices, {n}, {cols}] on the GPU with contiguous rows, at most "
-                                 f"{QK_MAX_SLICES} slices, as far apart as q's")
+                                 f"{kernels.QK_MAX_SLICES} slices, as far apart as q's")
         elif not t.is_cuda or t.dtype != torch.bfloat16 or t.shape != (n, cols) or t.stride(1) != 1:
             raise ValueError(f"decode_fused: {name} must be bfloat16 [{n}, {cols}] on the GPU with contiguous rows")
     if (k is None) != (v is None):

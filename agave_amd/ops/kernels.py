@@ -25,7 +25,7 @@ _SIGNATURES = {
         "agave_norm_of_sum": [_I, _P, _P, _L, _I, _L, _F, _P, _P, _F, _P, _L, _P, _F, _I, _I, _P],
         "agave_residual_layernorm": [_I, _P, _P, _L, _I, _L, _P, _P, _F, _P, _L, _P, _P, _F, _P, _I, _I, _P, _P],
         "agave_qk_norm_rope_kv": [_I, _P, _L, _P, _L, _P, _L, _P, _L, _P, _P, _F, _F, _P, _I, _F,
-                                  _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P],
+                                  _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _L, _P],
         "agave_geglu": [_I, _P, _L, _P, _L, _P, _L, _I, _I, _P],
         "agave_gated_act": [_I, _I, _F, _F, _P, _L, _P, _L, _P, _L, _I, _I, _P],
         "agave_unary_act": [_I, _I, _F, _F, _P, _L, _P, _L, _I, _I, _P],
@@ -269,6 +269,16 @@ def residual_layernorm(h: torch.Tensor, branch: Optional[torch.Tensor], post_w: 
                  ptr(src), stream())
 
 
+def _slice_rows(t: torch.Tensor, what: str) -> int:
+    """The row stride of [slices, rows, columns]."""
+    if t.stride(2) != 1 or t.stride(1) < t.shape[2]:
+        raise ValueError(f"{what}: rows must be contiguous")
+    return t.stride(1)
+
+
+QK_MAX_SLICES = 4            # 32-bit slices of the raw projections that the kernels of few tokens add up
+
+
 def qk_norm_rope_kv(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Optional[torch.Tensor],
                     q_out: Optional[torch.Tensor], q_gain: Optional[torch.Tensor], k_gain: Optional[torch.Tensor],
                     eps_q: float, eps_k: float, inv_freq: Optional[torch.Tensor], pos_scale: float,
@@ -278,26 +288,36 @@ def qk_norm_rope_kv(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Opt
     """Per-head RMSNorm of q and k, rotation, q to ``q_out`` and k, v into their cache pages.
     ``k`` None: only q is processed (a layer that reads another layer's cache).  ``packed``:
     the pages are in the matrix cores' tile order.  ``apart``: of how many sequences the tokens are (0: of one, from a position on
-    that is a multiple of four); which kernel is the faster one hangs on it, the results do not."""
+    that is a multiple of four); which kernel is the faster one hangs on it, the results do not.  Of bfloat16 activations q, k and v may be
+    float32 [slices, n, columns] with one stride between slices (at most ``QK_MAX_SLICES``), whose slices add up to the rows."""
     _dev(q, k, v, q_out, q_gain, k_gain, inv_freq, tok_seq, tok_pos, k_pages, v_pages, table, base)
     n = tok_pos.numel()
     _i32(tok_pos, "tok_pos")
     _i32(tok_seq, "tok_seq", n)
     ref = q if q is not None else k
+    slices = slice_stride = 0
+    if ref.dim() == 3:
+        slices, slice_stride = ref.shape[0], ref.stride(0)
+        for t in (q, k, v):
+            if t is not None and (t.dim() != 3 or t.dtype != torch.float32 or t.shape[0] != slices or t.stride(0) != slice_stride
+                                  or not 1 <= slices <= QK_MAX_SLICES):
+                raise ValueError(f"q, k and v: all float32 slices, at most {QK_MAX_SLICES} and equally far apart, or none")
+        ref = q_out if q is not None else k_pages
     d = dt(ref)
     ldq = ldqo = ldk = ldv = 0
     nh = nkv = 0
+    raw = torch.float32 if slices else ref.dtype
     if q is not None:
         nh = n_heads
-        ldq, ldqo = _rows(q, "q"), _rows(q_out, "q_out")
-        if q.shape != (n, nh * head_dim) or q_out.shape != (n, nh * head_dim) or q_out.dtype != q.dtype:
+        ldq, ldqo = _rows(q, "q") if not slices else _slice_rows(q, "q"), _rows(q_out, "q_out")
+        if q.shape[-2:] != (n, nh * head_dim) or q_out.shape != (n, nh * head_dim) or q.dtype != raw or q_out.dtype != ref.dtype:
             raise ValueError(f"q and q_out must be [{n}, {nh * head_dim}] of one dtype")
         _f32vec(q_gain, "q_gain", head_dim)
     width = n_pages = 0
     if k is not None:
         nkv = n_kv
-        ldk, ldv = _rows(k, "k"), _rows(v, "v")
-        if k.shape != (n, nkv * head_dim) or v.shape != (n, nkv * head_dim) or k.dtype != ref.dtype or v.dtype != ref.dtype:
+        ldk, ldv = (_rows(k, "k"), _rows(v, "v")) if not slices else (_slice_rows(k, "k"), _slice_rows(v, "v"))
+        if k.shape[-2:] != (n, nkv * head_dim) or v.shape[-2:] != (n, nkv * head_dim) or k.dtype != raw or v.dtype != raw:
             raise ValueError(f"k and v must be [{n}, {nkv * head_dim}] of the activations' dtype")
         _f32vec(k_gain, "k_gain", head_dim)
         n_pages = _check_pages(k_pages, v_pages, nkv, head_dim, ref.dtype, packed)
@@ -309,7 +329,7 @@ def qk_norm_rope_kv(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Opt
     library.call(lib("elementwise"), "agave_qk_norm_rope_kv", d, ptr(q), ldq, ptr(k), ldk, ptr(v), ldv, ptr(q_out),
                  ldqo, ptr(q_gain), ptr(k_gain), eps_q, eps_k, ptr(inv_freq), rot_half, pos_scale, ptr(tok_seq),
                  ptr(tok_pos), ptr(k_pages), ptr(v_pages), ptr(table), width, ptr(base), n_pages, n, nh, nkv,
-                 head_dim, 1 if (packed and k is not None) else 0, int(apart), stream())
+                 head_dim, 1 if (packed and k is not None) else 0, int(apart), slices, slice_stride, stream())
 
 
 def _check_pages(k_pages: torch.Tensor, v_pages: torch.Tensor, nkv: int, hd: int, dtype: torch.dtype,

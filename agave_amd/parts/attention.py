@@ -82,10 +82,10 @@ class Attention:
         k_pages, v_pages, packed = step.cache.pages_of(memory)
         table, base = step.tables[step.cache.group_of_memory[memory]]
         fused = getattr(self.position, "fused_rotation", None)
-        # (the kernel that takes the raw projections of a decode step adds up slices of them)
-        slices_ok = packed and fused is not None and step.is_decode and attn_ops.adds_slices(n, self.qkv, s.head_dim)
+        # (the kernels that norm and rotate the raw projections of few tokens add up slices of them)
+        slices_ok = packed and fused is not None and attn_ops.adds_slices(step, self.qkv, s.head_dim)
         qkv = self.qkv.forward(x, tag="qkv", slices_ok=slices_ok)
-        q, k, v = ws.columns(qkv, self._qkv_bounds) if qkv.dim() == 2 else qkv.split((self.qd, self.kvd, self.kvd), dim=2)
+        q, k, v = ws.columns(qkv, self._qkv_bounds)
         if not writes:
             k = v = None            # a run that reads another run's cache appends nothing
         q_out = ws.get("q_rot", n, self.qd, x.dtype)

@@ -100,11 +100,11 @@ class Workspace:
         return view
 
     def columns(self, t: torch.Tensor, bounds) -> tuple:
-        """``t[:, bounds[i]:bounds[i + 1]]`` for every i, made once per tensor kept here and bounds."""
-        key = ("columns", t.data_ptr(), t.shape[0], t.stride(0), bounds)
+        """``t[..., bounds[i]:bounds[i + 1]]`` for every i, made once per tensor kept here and bounds."""
+        key = ("columns", t.data_ptr(), t.shape, t.stride(0), bounds)
         got = self._views.get(key)
         if got is None:
-            got = self._views[key] = tuple(t[:, lo:hi] for lo, hi in zip(bounds[:-1], bounds[1:]))
+            got = self._views[key] = tuple(t[..., lo:hi] for lo, hi in zip(bounds[:-1], bounds[1:]))
         return got
 
     def reserve(self, name: str, rows: int, cols: int, dtype: torch.dtype) -> None:

@@ -1826,10 +1826,23 @@ def test_attn_decode_fused_adds_slices_of_the_projections(K, nh, nkv, hd, slices
     assert torch.isfinite(outs[0][0].float()).all()
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+    # the q/k kernel of steps with several tokens a sequence, the same rows as a prompt's of one sequence
+    pos, tab = _i32(list(range(60, 60 + B))), torch.tensor([[3, 1, -1, -1]], dtype=torch.int32).to(DEV)
+    outs = []
+    for rows in (whole.to(DEV), parts.to(DEV)):
+        q, k, v = rows.split((nh * hd, nkv * hd, nkv * hd), dim=-1)
+        kp, vp, q_rot = pages[0].clone(), pages[1].clone(), torch.full((B, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+        K.qk_norm_rope_kv(q, k, v, q_rot, gain, gain, 1e-6, 1e-6, inv_freq, 1.0, _i32([0] * B), pos, kp, vp, tab, _i32([0]), nh, nkv, hd, packed=True)
+        outs.append((q_rot, kp, vp))
+    assert torch.isfinite(outs[0][0].float()).all()
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
     q5 = torch.zeros(5, B, nh * hd, device=DEV)
     with pytest.raises(ValueError):
         A.decode_fused(q5, None, None, outs[0][0], gain, gain, 1e-6, 1e-6, inv_freq, 1.0, kp, vp, table.to(DEV), _i32([0] * B), step, nh, nkv,
                        hd, 0.1, None)
+    with pytest.raises(ValueError):
+        K.qk_norm_rope_kv(q5, None, None, outs[0][0], gain, None, 1e-6, 0.0, inv_freq, 1.0, _i32([0] * B), pos, None, None, None, None, nh, 0, hd)
 
 
 # Heads as long as the kernel's tiles: a page's keys and values are asked for at once, one token's before its queries are there.
