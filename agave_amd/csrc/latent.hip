@@ -67,30 +67,86 @@ struct LatentQ {                  // the query side: a latent to be normed (head
     int heads, dim, rot_dim;
 };
 
-// One workgroup of 256 threads: the key/value row of token t
+// A row's elements tid, tid + 256, ... and their weights, asked for at once: up to ASKED of them a thread, so a longer row's others come
+// one after the other where they are used.
+#define ASKED 8
+struct NormedRow {
+    const float* x;
+    const float* weight;
+    int n;
+    float xv[ASKED], wv[ASKED];
+    __device__ __forceinline__ void ask(const float* row, const float* gain, int elements) {
+        x = row, weight = gain, n = elements;
+        const int tid = threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < ASKED; ++i)
+            if (256 * i < n) {                               // (the same for all threads; a lane past the end reads the row's start)
+                const int e = tid + 256 * i;
+                xv[i] = x[e < n ? e : 0];
+                wv[i] = weight[e < n ? e : 0];
+            }
+    }
+    // 1 / sqrt(mean of the squares + eps)
+    __device__ __forceinline__ float scale(float eps, float* red) const {
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < ASKED; ++i)
+            if (256 * i < n) ss = (int)threadIdx.x + 256 * i < n ? fmaf(xv[i], xv[i], ss) : ss;
+        for (int e = threadIdx.x + 256 * ASKED; e < n; e += 256) ss = fmaf(x[e], x[e], ss);
+        return 1.0f / sqrtf(block_sum_into(ss, red) / (float)n + eps);
+    }
+    template <typename F> __device__ __forceinline__ void each(float inv, F&& f) const {
+#pragma unroll
+        for (int i = 0; i < ASKED; ++i) {
+            const int e = threadIdx.x + 256 * i;
+            if (256 * i < n && e < n) f(e, xv[i] * inv * wv[i]);
+        }
+        for (int e = threadIdx.x + 256 * ASKED; e < n; e += 256) f(e, x[e] * inv * weight[e]);
+    }
+};
+
+// One workgroup of 256 threads: the key/value row of token t.  Bound by its trips to memory one after the other, the position, the row,
+// the page's id: the row, its weights and the pairs to be turned are asked for first and a thread turns a pair by itself (four rows of
+// 512 and 64 beside as many queries of 1,536: 6.6 -> 5.9 us).
 template <typename T>
-__device__ __forceinline__ void latent_kv_row(const LatentKv& A, const Turn& R, int t, int pos, float eps, float* red,
-                                              float (*cs)[MAX_TURNED]) {
+__device__ __forceinline__ void latent_kv_row(const LatentKv& A, const Turn& R, int t, const int* tok_pos, float eps, float* red) {
     const int tid = threadIdx.x, rank = A.rank, kd = A.rank + A.rot_dim;
+    const int pos = tok_pos[t], seq = A.k_pages ? A.tok_seq[t] : 0;
     const float* x = A.raw + (size_t)t * A.ldraw;
-    turn_table(R, pos, cs, tid, 256);
+    NormedRow row;
+    row.ask(x, A.weight, rank);
+    const bool turns = tid < R.half;                                // (at most 256 pairs)
+    const int first = rank + first_of_pair(R, tid), second = rank + second_of_pair(R, tid);
+    double freq = 0.0;
+    float u = 0.f, v = 0.f;
+    if (turns) {
+        freq = R.freq[tid];
+        u = x[first];
+        v = x[second];
+    }
     PagePlace at{-1, 0};
-    if (A.k_pages) at = place_of(pos, A.tok_seq[t], A.table, A.width, A.base, 0, A.n_pages);
-    float ss = 0.f;
-    for (int e = tid; e < rank; e += 256) ss = fmaf(x[e], x[e], ss);
-    ss = block_sum(ss, red);                                    // (its barriers complete the table too)
-    const float inv = 1.0f / sqrtf(ss / (float)rank + eps);
+    if (A.k_pages) at = place_of(pos, seq, A.table, A.width, A.base, 0, A.n_pages);
+    const float inv = row.scale(eps, red);
     const int ksl = (kd + 31) / 32;
     T* kp = (T*)A.k_pages + (size_t)at.page * (A.packed ? (size_t)AGAVE_PAGE * ksl * 32 : (size_t)AGAVE_PAGE * kd);
     T* vp = (T*)A.v_pages + (size_t)at.page * rank * AGAVE_PAGE;
-    for (int e = tid; e < kd; e += 256) {
-        const float y = e < rank ? x[e] * inv * A.weight[e] : turned_element(R, x + rank, e - rank, cs);
+    auto put = [&](int e, float y) {
         if (A.row) st((T*)A.row + (size_t)t * A.ldrow + e, y);
         if (at.page >= 0) {
             st(kp + (A.packed ? k_operand_at(at.row, e, ksl) : (size_t)at.row * kd + e), y);
             if (e < rank) st(vp + (A.packed ? v_operand_at(e, at.row) : (size_t)e * AGAVE_PAGE + at.row), y);
         }
+    };
+    row.each(inv, put);
+    if (turns) {
+        float s, c;
+        sincos_of_angle((double)pos * freq, s, c);
+        c *= R.magnitude;
+        s *= R.magnitude;
+        put(first, u * c - v * s);
+        put(second, v * c + u * s);
     }
+    for (int e = rank + 2 * R.half + tid; e < kd; e += 256) put(e, x[e]);
 }
 
 // One workgroup of 256 threads: the query rows of token t with their trailing elements turned
@@ -128,21 +184,19 @@ template <typename T>
 __global__ __launch_bounds__(256) void latent_prepare_kernel(LatentQ Q, LatentKv K, Turn R, const int* __restrict__ tok_pos, float eps) {
     __shared__ float red[16];
     __shared__ float cs[2][MAX_TURNED];
-    const int t = blockIdx.x, tid = threadIdx.x;
+    const int t = blockIdx.x;
     if (Q.raw && blockIdx.y == 0) {
         if (Q.heads) {
             latent_q_rows<float, T>(Q, R, t, tok_pos[t], cs);
             return;
         }
-        const float* x = (const float*)Q.raw + (size_t)t * Q.ldraw;
-        float ss = 0.f;
-        for (int e = tid; e < Q.rank; e += 256) ss = fmaf(x[e], x[e], ss);
-        ss = block_sum(ss, red);
-        const float inv = 1.0f / sqrtf(ss / (float)Q.rank + eps);
-        for (int e = tid; e < Q.rank; e += 256) st((T*)Q.out + (size_t)t * Q.ldout + e, x[e] * inv * Q.weight[e]);
+        NormedRow row;
+        row.ask((const float*)Q.raw + (size_t)t * Q.ldraw, Q.weight, Q.rank);
+        const float inv = row.scale(eps, red);
+        row.each(inv, [&](int e, float y) { st((T*)Q.out + (size_t)t * Q.ldout + e, y); });
         return;
     }
-    latent_kv_row<T>(K, R, t, tok_pos[t], eps, red, cs);
+    latent_kv_row<T>(K, R, t, tok_pos, eps, red);
 }
 
 static int check_turn(const char* what, const Turn& R, int rot_dim) {
@@ -361,12 +415,11 @@ __global__ __launch_bounds__(256) void heads_product_mfma_kernel(HeadsProductArg
 template <typename XT, int J>
 __global__ __launch_bounds__(256) void latent_decode_rows_kernel(HeadsProductArgs A, LatentKv K, Turn R, float eps) {
     __shared__ float red[16];
-    __shared__ float cs[2][MAX_TURNED];
     if ((int)blockIdx.y < A.heads) {
         heads_product_tile<XT, J>(A, 0, blockIdx.y, blockIdx.z);
     } else if (blockIdx.z == 0) {
         const int t = blockIdx.y - A.heads;
-        latent_kv_row<bf16>(K, R, t, A.tok_pos[t], eps, red, cs);
+        latent_kv_row<bf16>(K, R, t, A.tok_pos, eps, red);
     }
 }
 

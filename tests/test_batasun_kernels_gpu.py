@@ -66,6 +66,24 @@ def test_latent_norms_and_the_rotated_key_part(dtype, q_rank, kv_rank, rot_dim, 
     assert torch.equal(cq, cq2)
 
 
+@pytest.mark.parametrize("q_rank, kv_rank, rot_dim, rot_dims", [(255, 257, 2, 2), (2047, 256, 6, 4), (2049, 2048, 512, 512), (4100, 2300, 7, 2)])
+def test_latent_norms_of_rows_up_to_and_beyond_what_a_thread_holds(q_rank, kv_rank, rot_dim, rot_dims):
+    """One to eight elements a thread and more; no, one and 256 turned pairs, elements behind them that are not turned.  32-bit: a sum of
+    4,100 squares is off by at most some 2^-20, a turned element by its angle's 2^-23 of pi/4."""
+    from agave_amd.ops import latent as L
+    eps, pos = 3e-4, [0, 5, 4095]
+    g = torch.Generator().manual_seed(q_rank)
+    wide = torch.randn(len(pos), q_rank + kv_rank + rot_dim, generator=g) * 3
+    qw, kw = 1 + 0.3 * torch.randn(q_rank, generator=g), 1 + 0.3 * torch.randn(kv_rank, generator=g)
+    raw, w64 = wide.to(DEV), wide.to(F64)
+    cq, row = torch.empty(len(pos), q_rank, device=DEV), torch.empty(len(pos), kv_rank + rot_dim, device=DEV)
+    L.latent_prepare(Positions(pos), eps, halves(700.0, rot_dims), rot_dim, q_raw=raw[:, :q_rank], q_weight=qw.to(DEV), q_out=cq,
+                     kv_raw=raw[:, q_rank:], kv_weight=kw.to(DEV), k_row=row, kv_rank=kv_rank)
+    assert rel(cq, P.rms(w64[:, :q_rank], eps) * qw.to(F64)) < 3e-6
+    assert rel(row[:, :kv_rank], P.rms(w64[:, q_rank:q_rank + kv_rank], eps) * kw.to(F64)) < 3e-6
+    assert rel(row[:, kv_rank:], P.rotate(w64[:, q_rank + kv_rank:], pos, 700.0, rot_dims)) < 3e-6
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n, heads, K, n_out, tail, rot", [(5, 3, 16, 40, 8, 8), (40, 3, 16, 40, 8, 8), (130, 2, 24, 70, 16, 12),
                                                           (70, 5, 19, 7, 6, 4), (33, 1, 96, 128, 0, 0), (64, 4, 40, 16, 2, 2)])

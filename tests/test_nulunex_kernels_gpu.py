@@ -276,6 +276,46 @@ def test_decode_attention_over_latent_rows(heads, kd, kv_rank, out, window, with
         assert rel(y[i], want[i]) < 1.5e-2, (before[i], rel(y[i], want[i]))
 
 
+@pytest.mark.parametrize("splits", [1, 3, 64])
+@pytest.mark.parametrize("window", [None, 4200])
+def test_decode_attention_over_tables_of_more_columns_than_a_wave_has_lanes(window, splits):
+    """Sequences of one page, of 64, of 65 and of 130, with and without pages that a table does not name: the table's columns are held
+    64 at a time.  Queries, weights and the merged row are rounded to bfloat16 (2^-9 each), the result too."""
+    from agave_amd.cache import GroupKey
+    from agave_amd.ops import attention_biased as A
+    from agave_amd.ops import latent as L
+    heads, kd, kv_rank, out, before = 3, 40, 32, 16, [40, 4095, 4096, 8300]
+    g = torch.Generator().manual_seed(splits)
+    cache, planner = planner_for(GroupKey(window, 1, kd, v_head_dim=kv_rank, layout="rows_vt"), slots=4, pages=280, dtype=BF, context=9000)
+    slots, rows = [cache.alloc_slot() for _ in before], [torch.randn(n + 1, kd, generator=g).to(BF) for n in before]
+    v_up = (torch.randn(heads, out, kv_rank, generator=g) * kv_rank ** -0.5).to(BF)
+    kp, vp, packed = cache.pages_of(0)
+    for lo in range(0, 8301, 1000):
+        some = [i for i, n in enumerate(before) if n > lo]
+        part = [rows[i][lo:min(lo + 1000, before[i])] for i in some]
+        step = planner.plan([slots[i] for i in some], [[0] * len(r) for r in part], "all")
+        r, (table, base) = torch.cat(part).to(DEV), step.tables[0]
+        A.kv_append_rows(r, r[:, :kv_rank], kp, vp, table, base, 0, step, 1, kd, kv_rank, packed)
+        planner.commit(step)
+    step = planner.plan(slots, [[0]] * len(before), "all")
+    table, base = step.tables[0]
+    r = torch.stack([x[-1] for x in rows]).to(DEV)
+    A.kv_append_rows(r, r[:, :kv_rank], kp, vp, table, base, 0, step, 1, kd, kv_rank, packed)
+    q, first = torch.randn(len(before), heads * kd, generator=g).to(BF), base.cpu().tolist()
+    for gone in ((), (70, 71, 128, 129)):
+        held = table.clone()
+        for page in gone:
+            held[3, page - first[3]] = -1
+        y = torch.empty(len(before), heads * out, dtype=BF, device=DEV)
+        L.decode_attention(q.to(DEV), v_up.to(DEV), y, None, kp, vp, held, base, step, heads, kd, kv_rank, kd ** -0.5, window, None, workspace(),
+                           splits=splits)
+        for i, n in enumerate(before):
+            lo = max(0, n - window + 1) if window else 0
+            kept = torch.tensor([p for p in range(lo, n + 1) if i < 3 or p // 64 not in gone])
+            want = plain_decode(q[i].to(F64).view(heads, kd), rows[i][kept].to(F64), kd ** -0.5, None, None, v_up.to(F64), None, len(kept) - 1)
+            assert rel(y[i], want) < 1.5e-2, (n, gone)
+
+
 def test_a_growing_sequence_moves_no_buffer_of_latent_attention():
     """More pages, more shares of a row: their results lie in the buffers that the first step has made, so that steps that were recorded
     with their addresses stay valid."""
