@@ -159,6 +159,30 @@ def test_row_norm_and_rotation(dtype, H, G, d, vd, dims, scaling, normed):
     assert torch.equal(q2, q_out)
 
 
+@pytest.mark.parametrize("H, G, d, dims", [(16, 2, 128, 128), (17, 17, 128, 128), (1, 33, 130, 128), (32, 1, 140, 130), (63, 64, 128, 128), (65, 1, 128, 128)])
+@pytest.mark.parametrize("n", [1, 170, 171])
+def test_row_norm_and_rotation_at_the_edges_of_its_kernels(H, G, d, dims, n):
+    """One, two and four pairs a thread and more than are held, of queries or of keys; the most tokens with a workgroup a row and one
+    more.  32-bit: a sum of some 8,000 squares is off by at most 2^-20, a turned element by its angle's 2^-23 of pi/4."""
+    from agave_amd.ops import attention_biased as A
+    vd, eps = 24, 1e-5
+    g = torch.Generator().manual_seed(H + n)
+    wide = torch.randn(n, (H + G) * d + G * vd, generator=g) * 2
+    qw, kw = 1 + 0.3 * torch.randn(H * d, generator=g), 1 + 0.3 * torch.randn(G * d, generator=g)
+    pos, raw, w64 = torch.arange(n) * 13, wide.to(DEV), wide.to(F64)
+    freq = torch.tensor([300.0 ** (-2.0 * e / dims) for e in range(dims // 2)], dtype=F64)
+    q, kv = torch.empty(n, H * d, device=DEV), torch.empty(n, G * (d + vd), device=DEV)
+    A.row_norm_rope(raw[:, :H * d], raw[:, H * d:(H + G) * d], raw[:, (H + G) * d:], q, kv[:, :G * d], kv[:, G * d:], qw.to(DEV), kw.to(DEV), eps, eps,
+                    freq.to(DEV), 1.0, Positions(pos.tolist()), H, G, d, vd)
+    for got, x, w, heads in ((q, w64[:, :H * d], qw, H), (kv[:, :G * d], w64[:, H * d:(H + G) * d], kw, G)):
+        x = P.row_rms(x, w.to(F64), eps).view(n, heads, d)
+        angle = (pos.to(F64)[:, None] * freq)[:, None]
+        a, b = x[..., :dims // 2], x[..., dims // 2:dims]
+        want = torch.cat([a * angle.cos() - b * angle.sin(), b * angle.cos() + a * angle.sin(), x[..., dims:]], -1)
+        assert rel(got.reshape(n, heads, d), want) < 3e-6
+    assert torch.equal(kv[:, G * d:].cpu(), wide[:, (H + G) * d:])
+
+
 # ---------------------------------------------------------------- attention: chunks and a cap on the scores
 class Case:
     def __init__(self, H, G, d, vd, window, chunk, softcap, T, seed=0, big=1.0):
