@@ -150,7 +150,8 @@ template <> __device__ __forceinline__ void store4<bf16>(bf16* p, float4 v) {
 // 16-byte load into four, each in a branch of its own.  A lane past the row's end reads the
 // row's start instead; its values are left out of the sums and never stored.  Nothing that was
 // loaded is touched before everything has been asked for, so the loads travel together.
-__device__ __forceinline__ float sumsq(bool in, float4 v) { return in ? v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w : 0.f; }
+// (The fused steps are written out: left to the compiler, which of two squares is rounded hangs on the code around.)
+__device__ __forceinline__ float sumsq(bool in, float4 v) { return in ? fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.x, v.x, v.y * v.y))) : 0.f; }
 
 // Few rows are bound by their chain of one trip to memory (0.8 us of it) and two sums over the workgroup: eight rows of 2,560 and three
 // slices 3.44 us a launch in a chain of its own, of which 1.6 are a kernel's start and end, and 3.17 since the sums read the waves' parts

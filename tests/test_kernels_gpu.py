@@ -69,6 +69,52 @@ def test_residual_norm(K, dtype, e):
     K.residual_norm(h3, br.to(DEV), None, 0.0, None, None, 0.0)
     assert torch.allclose(h3.cpu().double(), h.double() + br.double(), atol=1e-6)
 
+def _inv_rms_bits(x, eps, threads, first=1):
+    """1 / rms of every row as the kernel of 16-byte loads makes it, bit by bit: a thread's four squares in fused steps behind the square of
+    the ``first`` one (x first would round another of them), its pieces added up, a wave's lanes in pairs 1, 2, 4 .. 32 apart, the waves in
+    turn.  (A fused step is made in numpy's long double: a product of 24 by 24 bits is exact there.)"""
+    n, e = x.shape
+    v = np.zeros((n, -(-e // (4 * threads)) * threads * 4), np.float32)
+    v[:, :e] = x
+    v = v.reshape(n, -1, threads, 4)
+    fma = lambda a, c: (a.astype(np.longdouble) * a + c).astype(np.float32)
+    sq = fma(v[..., 3], fma(v[..., 2], fma(v[..., 1 - first], v[..., first] * v[..., first])))
+    ss = sq[:, 0]
+    for k in range(1, sq.shape[1]):
+        ss = ss + sq[:, k]
+    ss = ss.reshape(n, threads // 64, 64)
+    while ss.shape[-1] > 1:
+        ss = ss[..., 0::2] + ss[..., 1::2]
+    total = np.zeros(n, np.float32)
+    for w in range(threads // 64):
+        total = total + ss[:, w, 0]
+    return np.float32(1) / np.sqrt(total / np.float32(e) + np.float32(eps))
+
+
+@pytest.mark.parametrize("n, e, threads", [(64, 1000, 256), (64, 2048, 512), (64, 2560, 640), (65, 2560, 320), (65, 7000, 896), (64, 16384, 1024)])
+def test_norms_add_squares_in_one_order(K, n, e, threads):
+    """A row's bits come from its elements alone, not from what else a kernel does with it: the same order of roundings in every form
+    (a row normed, a branch normed on its way into the stream, the norm of a sum), whatever the compiler fuses around it."""
+    g = torch.Generator().manual_seed(e)
+    x, gain, eps = torch.randn(n, e, generator=g) * 3, 1 + 0.3 * torch.randn(e, generator=g), 1e-5
+    inv = _inv_rms_bits(x.numpy(), eps, threads)
+    assert (inv != _inv_rms_bits(x.numpy(), eps, threads, first=0)).any()             # (the order shows in these rows)
+    inv, w = torch.from_numpy(inv)[:, None], gain.to(DEV)
+    out = torch.empty(n, e, device=DEV)
+    K.residual_norm(x.to(DEV), None, None, 0.0, out, w, eps)
+    assert torch.equal(out.cpu(), x * inv * gain)
+    for parts in (x.to(DEV), torch.stack([x, torch.zeros_like(x)]).to(DEV)):          # as a row, and as slices
+        h = torch.zeros(n, e, device=DEV)
+        K.residual_norm(h, parts, w, eps, out, w, eps)
+        assert torch.equal(h.cpu(), x * inv * gain)
+        second = torch.from_numpy(_inv_rms_bits(h.cpu().numpy(), eps, threads))[:, None]
+        assert torch.equal(out.cpu(), h.cpu() * second * gain)
+        h = torch.zeros(n, e, device=DEV)
+        K.norm_of_sum(h, parts, 1.0, None, w, eps, out, w, eps)
+        assert torch.equal(h.cpu(), x * (inv * gain))
+        second = torch.from_numpy(_inv_rms_bits(h.cpu().numpy(), eps, threads))[:, None]
+        assert torch.equal(out.cpu(), h.cpu() * second * gain)
+
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("e", [100, 2560, 20000])
