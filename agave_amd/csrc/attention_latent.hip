@@ -11,7 +11,8 @@
 //                    is multiplied.  `splits` workgroups share a sequence's pages; each leaves its reference, its sum
 //                    and its unnormalised sums over the rows.
 //                    Bound by that round trip and the chain behind it: 16 heads of 576, 4 sequences of 1,000 in 32 shares
-//                    10.9 -> 9.6 to 10.5 us, the step 0.493 -> 0.485 ms, since a share of one page reads nothing behind it.
+//                    10.9 -> 9.6 to 10.5 us, the step 0.493 -> 0.485 ms, since a share of one page reads nothing behind it
+//                    (without that branch 12.3 us for both kernels instead of 11.7).
 //   latent_values    merges the shares of a (row, head) and multiplies the merged row by the head's value matrix:
 //                    y = W_h x, times the sigmoid of a gate where there is one.  The matrix is asked for before the shares.
 //
@@ -47,7 +48,7 @@ __global__ __launch_bounds__(512) void latent_decode_kernel(LatentDecodeArgs A) 
     // what names the pages is asked for at once: the position, the table's first column's page, a table column a lane
     const int pos = A.tok_pos[b], pbase = A.base[b];
     const int* row_table = A.table + (size_t)b * A.width;
-    int column = row_table[lane < A.width ? lane : A.width - 1], column0 = 0;        // of the table's columns, 64 at a time
+    const int column = row_table[lane < A.width ? lane : A.width - 1];
     const int head = blockIdx.y * 16 + c;
     const bool valid = head < A.heads;
     const int ksl = (A.kd + 31) / 32, k0 = half ? (ksl + 1) / 2 : 0, k_end = half ? ksl : (ksl + 1) / 2;
@@ -71,16 +72,18 @@ __global__ __launch_bounds__(512) void latent_decode_kernel(LatentDecodeArgs A) 
 
     const int W = A.window, lo = W > 0 ? max(0, pos - W + 1) : 0;
     const int first = lo / AGAVE_PAGE, n_pg = pos / AGAVE_PAGE - first + 1;
-    auto page_of = [&](int idx) -> int {
+    // The page of the idx-th place in two steps: its id is asked for a page ahead of its use, by a load at one place for the whole wave
+    // (scalar: a load by the lanes is waited for with all the page's loads before it, and a sequence of more than 64 pages then asks
+    // for its second page when the first is there).  16 heads of 576, with lanes' loads and now, us: one sequence of 6,000 15.2 and 14.7,
+    // of 30,000 31.3 and 28.5, 4 of 1,000 11.8 and 11.7.
+    const auto scalar_table = (const __attribute__((address_space(4))) int*)row_table;
+    auto ask_id = [&](int idx) -> int {
         const int col = first + idx - pbase;
-        if (idx >= n_pg || col < 0 || col >= A.width) return -1;
-        if (col - column0 >= 64 || col < column0) {          // (waited for here: behind this branch nothing is asked for on either way)
-            column0 = col & ~63;
-            column = row_table[column0 + lane < A.width ? column0 + lane : A.width - 1];
-            __builtin_amdgcn_s_waitcnt(0x0F70);              // vmcnt(0)
-        }
-        const int pg = __builtin_amdgcn_readlane(column, col - column0);
-        return pg < A.n_pages ? pg : -1;
+        return scalar_table[col < 0 ? 0 : (col < A.width ? col : A.width - 1)];
+    };
+    auto page_at = [&](int idx, int id) -> int {
+        const int col = first + idx - pbase;
+        return idx >= n_pg || col < 0 || col >= A.width || id >= A.n_pages ? -1 : id;
     };
     // Loads without conditions: where a page is not there, all lanes read one place of page 0, and nothing uses it.  (A whole page 0 was
     // read behind every sequence's last, and the first page's loads waited for the queries'.)
@@ -150,7 +153,8 @@ __global__ __launch_bounds__(512) void latent_decode_kernel(LatentDecodeArgs A) 
     };
     // two sets of operands take turns; which pages there are is the same for all waves, so all of them meet at every barrier
     frag16 ka[KH], va[VW][2], kc[KH], vc[VW][2];
-    int idx = sp, pg = page_of(idx);
+    const int col0 = first + sp - pbase;
+    int idx = sp, pg = page_at(idx, col0 >= 0 && col0 < 64 ? __builtin_amdgcn_readlane(column, col0) : ask_id(idx)), id = ask_id(idx + A.splits);
     fetch(pg, ka, va);
 #pragma unroll
     for (int i = 0; i < KH; ++i)
@@ -160,12 +164,14 @@ __global__ __launch_bounds__(512) void latent_decode_kernel(LatentDecodeArgs A) 
         idx = n_pg;
     }
     while (idx < n_pg) {
-        const int next = idx + A.splits, pg_next = page_of(next);
+        const int next = idx + A.splits, pg_next = page_at(next, id);
+        id = ask_id(next + A.splits);
         fetch(pg_next, kc, vc);
         if (pg >= 0) use(idx, ka, va);
         if (next >= n_pg) break;
         idx = next + A.splits;
-        pg = page_of(idx);
+        pg = page_at(idx, id);
+        id = ask_id(idx + A.splits);
         fetch(pg, ka, va);
         if (pg_next >= 0) use(next, kc, vc);
     }

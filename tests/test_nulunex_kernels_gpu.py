@@ -279,8 +279,8 @@ def test_decode_attention_over_latent_rows(heads, kd, kv_rank, out, window, with
 @pytest.mark.parametrize("splits", [1, 3, 64])
 @pytest.mark.parametrize("window", [None, 4200])
 def test_decode_attention_over_tables_of_more_columns_than_a_wave_has_lanes(window, splits):
-    """Sequences of one page, of 64, of 65 and of 130, with and without pages that a table does not name: the table's columns are held
-    64 at a time.  Queries, weights and the merged row are rounded to bfloat16 (2^-9 each), the result too."""
+    """Sequences of one page, of 64, of 65 and of 130, with and without pages that a table does not name: a share's first page is
+    named by a lane among the first 64 columns, the others by loads of their own.  Queries, weights and the merged row are rounded to bfloat16 (2^-9 each), the result too."""
     from agave_amd.cache import GroupKey
     from agave_amd.ops import attention_biased as A
     from agave_amd.ops import latent as L
