@@ -179,12 +179,20 @@ __device__ __forceinline__ void latent_q_rows(const LatentQ& A, const Turn& R, i
     }
 }
 
+// The token of the i-th workgroup of n.  Workgroups go round the eight XCDs, each with an L2 of its own, and a value page holds 64
+// positions' elements side by side: runs of 64 tokens are kept on one XCD, or each of its L2s writes an eighth of every line.  The more rows
+// travel at a time the more that costs: rows of 2,048 beside as many queries, 8,000 tokens, bfloat16: 171 us where the
+// tokens go round and 97 (before a row's elements were all asked for at once 141 and, of 512 beside 1,536, 42.6; now 35.8 and 28.8).
+__device__ __forceinline__ int token_of_workgroup(int i, int n) {
+    return i < (n & ~511) ? (i & ~511) + ((i & 7) << 6) + ((i >> 3) & 63) : i;
+}
+
 // grid (tokens, sides): the query side first where there is one
 template <typename T>
 __global__ __launch_bounds__(256) void latent_prepare_kernel(LatentQ Q, LatentKv K, Turn R, const int* __restrict__ tok_pos, float eps) {
     __shared__ float red[16];
     __shared__ float cs[2][MAX_TURNED];
-    const int t = blockIdx.x;
+    const int t = token_of_workgroup(blockIdx.x, gridDim.x);
     if (Q.raw && blockIdx.y == 0) {
         if (Q.heads) {
             latent_q_rows<float, T>(Q, R, t, tok_pos[t], cs);

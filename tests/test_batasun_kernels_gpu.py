@@ -84,6 +84,39 @@ def test_latent_norms_of_rows_up_to_and_beyond_what_a_thread_holds(q_rank, kv_ra
     assert rel(row[:, kv_rank:], P.rotate(w64[:, q_rank + kv_rank:], pos, 700.0, rot_dims)) < 3e-6
 
 
+@pytest.mark.parametrize("n", [511, 512, 513, 1100])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_latent_rows_of_many_tokens_are_those_of_few(dtype, n):
+    """From 512 tokens on workgroups take their tokens in another order: every row, and its place in the pages, as from a step that
+    brings few tokens (the same bits)."""
+    from agave_amd.cache import GroupKey, KVCache
+    from agave_amd.engine.step import StepPlanner
+    from agave_amd.ops import latent as L
+    q_rank, kv_rank, rot, eps = 48, 32, 8, 1e-5
+    g = torch.Generator().manual_seed(n)
+    raw = torch.randn(n, q_rank + kv_rank + rot, generator=g).to(DEV)
+    qw, kw = (1 + 0.3 * torch.randn(k, generator=g).to(DEV) for k in (q_rank, kv_rank))
+    turn, key = halves(700.0, rot), GroupKey(None, 1, kv_rank + rot, v_head_dim=kv_rank, layout="rows_vt")
+    got = []
+    for most in (n, 200):
+        cache = KVCache({0: key}, {}, 1, {key: 20}, dtype, torch.device(DEV), 2048)
+        planner, slot = StepPlanner(cache, 1000, torch.device(DEV)), cache.alloc_slot()
+        kp, vp, packed = cache.pages_of(0)
+        kp.zero_(), vp.zero_()
+        cq, row = torch.empty(n, q_rank, dtype=dtype, device=DEV), torch.empty(n, kv_rank + rot, dtype=dtype, device=DEV)
+        for lo in range(0, n, most):
+            hi = min(lo + most, n)
+            step = planner.plan([slot], [[0] * (hi - lo)], "all")
+            L.latent_prepare(step, eps, turn, rot, q_raw=raw[lo:hi, :q_rank], q_weight=qw, q_out=cq[lo:hi], kv_raw=raw[lo:hi, q_rank:], kv_weight=kw,
+                             k_row=row[lo:hi], kv_rank=kv_rank, pages=L.CachePages(kp, vp, *step.tables[0], packed))
+            planner.commit(step)
+        table, base = step.tables[0]
+        pages = table[0, :-(-n // 64)].long()
+        got.append((cq, row, kp[pages], vp[pages]))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n, heads, K, n_out, tail, rot", [(5, 3, 16, 40, 8, 8), (40, 3, 16, 40, 8, 8), (130, 2, 24, 70, 16, 12),
                                                           (70, 5, 19, 7, 6, 4), (33, 1, 96, 128, 0, 0), (64, 4, 40, 16, 2, 2)])
