@@ -138,7 +138,7 @@ __device__ __forceinline__ float rows_max(float v) { return over_rows(v, [](floa
 __device__ __forceinline__ float block_sum_into(float v, float* red) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     v = wave_sum(v);
-    if (lane == 0 || (w == 0 && lane >= nw && lane < 16)) red[lane == 0 ? w : lane] = lane == 0 ? v : 0.f;
+    if (lane == w || (lane >= nw && lane < 16)) red[lane] = lane < nw ? v : 0.f;       // (every wave the zeros: one store, no branch)
     __syncthreads();
     float r = 0.f;
 #pragma unroll

@@ -222,6 +222,12 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
             }
         }
     }
+    // Where the stream is stored.  One piece a thread (few rows, or short ones): behind the second sum, in front of whose barrier the
+    // store would be waited for.  With more the card is full of rows whose stores fill its time: as soon as they are made.
+    constexpr bool LATE = VPT == 1;
+    auto store_h = [&](int v) {
+        if (in[v]) *reinterpret_cast<float4*>(hr + col[v]) = hv[v];
+    };
     if (branch && OF_SUM) {
         float ss = 0.f;
 #pragma unroll
@@ -240,6 +246,7 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
             hv[v].y *= inv * g1[v].y;
             hv[v].z *= inv * g1[v].z;
             hv[v].w *= inv * g1[v].w;
+            if (!LATE) store_h(v);
         }
     } else if (branch) {
         float inv = 1.0f;
@@ -263,17 +270,15 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
                 hv[v].z += bv[v].z;
                 hv[v].w += bv[v].w;
             }
+            if (!LATE) store_h(v);
         }
-    }
-    // (behind the second sum: in front of its barrier the store would be waited for)
-    auto store_h = [&]() {
-        if (!branch && !h_src) return;
+    } else if (!LATE && h_src) {
 #pragma unroll
-        for (int v = 0; v < VPT; ++v)
-            if (in[v]) *reinterpret_cast<float4*>(hr + col[v]) = hv[v];
-    };
+        for (int v = 0; v < VPT; ++v) store_h(v);
+    }
+    const bool stores = LATE && (OF_SUM || branch || h_src);
     if (out && !pre_gain) {                             // the rows as they are, rounded to the output's type
-        store_h();
+        if (stores) store_h(0);
         T* o = out + (size_t)i * ldo;
 #pragma unroll
         for (int v = 0; v < VPT; ++v)
@@ -283,7 +288,7 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
 #pragma unroll
         for (int v = 0; v < VPT; ++v) ss += sumsq(in[v], hv[v]);
         ss = block_sum_into(ss, red[1]);
-        store_h();
+        if (stores) store_h(0);
         const float inv = 1.0f / sqrtf(ss / (float)e + pre_eps);
         T* o = out + (size_t)i * ldo;
 #pragma unroll
@@ -293,7 +298,7 @@ __global__ void residual_norm_fast_kernel(float* __restrict__ h, const T* __rest
                                           hv[v].w * inv * g2[v].w});
         }
     }
-    if (!out) store_h();
+    if (stores && !out) store_h(0);
 }
 
 template <typename T, bool OF_SUM>
