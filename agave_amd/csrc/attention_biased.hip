@@ -337,10 +337,14 @@ __global__ __launch_bounds__(1024) void row_norm_rope_few_kernel(RowsArgs A) {
 
 template <typename T> static void row_norm_rope_on(const RowsArgs& A, int N, hipStream_t stream) {
     // Tokens whose three workgroups all find a place at once (two of sixteen waves a compute unit) and whose pairs the threads can
-    // hold: a workgroup a row, else one a token.  16 and 4 heads of 128 with norms, a row together and apart: 1 token 4.6 and 3.0 us,
-    // 64 4.9 and 3.4, 128 6.7 and 4.1, 200 6.9 and 5.7, 300 7.5 and 7.4; 8 and 2 heads of 64 with biases: 128 4.0 and 3.4, 200 4.0 and 4.7.
-    const int pairs = (A.nh > A.nkv ? A.nh : A.nkv) * A.half;
-    if (N <= 170 && pairs > 0 && pairs <= 4096) {
+    // hold: a workgroup a row, else one a token.  us, a row together and apart, 16 and 4 heads of 128 with norms: 1 token 4.6 and 3.0,
+    // 64 4.9 and 3.4, 128 7.0 and 4.4, 170 7.1 and 5.6, 200 6.9 and 5.7, 300 7.5 and 7.4; 64 and 8 heads of 128 with norms and
+    // biases (four pairs a thread): 8 7.5 and 4.2, 128 15.4 and 6.6, 170 15.8 and 8.4, 300 17.6 and 11.2.
+    // Rows of up to 256 pairs leave most of the sixteen waves idle, and keys and values beside them are slower apart as soon as a compute
+    // unit has two workgroups: 2 heads of 64 with norms, 100 4.7 and 3.9, 128 4.7 and 4.0, 129 4.7 and 4.9, 170 4.7 and 5.1 (the queries
+    // alone 3.3 and 3.1); 8 with biases, 128 4.3 and 3.7, 150 4.3 and 4.4.
+    const int pairs = (A.nh > A.nkv ? A.nh : A.nkv) * A.half, most = A.k && pairs <= 256 ? 128 : 170;
+    if (N <= most && pairs > 0 && pairs <= 4096) {
         const dim3 grid(N, A.k ? 3 : 1);
         if (pairs <= 1024) row_norm_rope_few_kernel<T, 1><<<grid, 1024, 0, stream>>>(A);
         else if (pairs <= 2048) row_norm_rope_few_kernel<T, 2><<<grid, 1024, 0, stream>>>(A);

@@ -183,6 +183,59 @@ def test_row_norm_and_rotation_at_the_edges_of_its_kernels(H, G, d, dims, n):
     assert torch.equal(kv[:, G * d:].cpu(), wide[:, (H + G) * d:])
 
 
+@pytest.mark.parametrize("normed", [True, False])
+@pytest.mark.parametrize("H, G, d, dims", [(2, 1, 64, 64), (8, 2, 64, 48), (17, 17, 128, 128), (33, 40, 128, 96), (33, 3, 128, 128)])
+@pytest.mark.parametrize("n", [1, 128, 129, 170, 171])
+def test_rows_with_biases_into_pages_at_the_edges(H, G, d, dims, n, normed):
+    """The same edges (small rows have their own line, 128 tokens) with biases, with and without norms, into pages in either order: bit
+    for bit the places that ``kv_append_rows`` gives the rows, which lie within a rounding to the output's type of 64-bit ones.  A token
+    whose page the table does not name leaves nothing."""
+    from agave_amd.cache import GroupKey, KVCache
+    from agave_amd.engine.step import StepPlanner
+    from agave_amd.ops import attention_biased as A
+    vd, eps = 32, 1e-5
+    g = torch.Generator().manual_seed(H * n)
+    raw = torch.randn(n, (H + G) * d + G * vd, generator=g) * 2
+    biases = [torch.randn(k, generator=g) for k in (H * d, G * d, G * vd)]
+    weights = [1 + 0.3 * torch.randn(k, generator=g) for k in (H * d, G * d)] if normed else [None, None]
+    dev = lambda t: t.to(DEV) if t is not None else None
+    freq = torch.tensor([300.0 ** (-2.0 * e / dims) for e in range(dims // 2)], dtype=F64)
+    q, k, v = dev(raw).split((H * d, G * d, G * vd), dim=1)
+    for dtype in (torch.bfloat16, torch.float32):
+        key = GroupKey(None, G, d, v_head_dim=vd, layout="rows_vt")
+        cache = KVCache({0: key}, {}, n, {key: 2 * n}, dtype, torch.device(DEV), 128)
+        planner, slots = StepPlanner(cache, 100000, torch.device(DEV)), [cache.alloc_slot() for _ in range(n)]
+        planner.commit(planner.plan(slots, [[0] * (40 + i % 30) for i in range(n)], "all"))       # (some tokens begin a page)
+        step = planner.plan(slots, [[0]] * n, "all")
+        kp, vp, packed = cache.pages_of(0)
+        table, base = step.tables[0]
+        table = table.clone()
+        if n > 1:
+            table[n // 2] = -1
+        made = []
+        for pages in (None, (kp, vp, table, base, 0, packed)):
+            kp.zero_(), vp.zero_()
+            q_out = torch.full((n, H * d), 9.0, dtype=dtype, device=DEV)
+            k_out, v_out = (torch.full((n, G * c), 9.0, dtype=dtype, device=DEV) if pages is None else None for c in (d, vd))
+            A.row_norm_rope(q, k, v, q_out, k_out, v_out, dev(weights[0]), dev(weights[1]), eps, eps, freq.to(DEV), 1.0, step, H, G, d, vd,
+                            pages=pages, biases=tuple(dev(b) for b in biases))
+            if pages is None:
+                rows = (k_out, v_out)
+                A.kv_append_rows(k_out, v_out, kp, vp, table, base, 0, step, G, d, vd, packed)
+            made.append((q_out, kp.clone(), vp.clone()))
+        for a, b in zip(*made):
+            assert torch.equal(a, b)
+        pos, tol = step.tok_pos.cpu().to(F64), 3e-6 if dtype == torch.float32 else 4e-3
+        for got, x, b, w, heads in ((made[0][0], q, biases[0], weights[0], H), (rows[0], k, biases[1], weights[1], G)):
+            x = x.cpu().to(F64) + b.to(F64)
+            x = (P.row_rms(x, w.to(F64), eps) if normed else x).view(n, heads, d)
+            angle = (pos[:, None] * freq)[:, None]
+            lo, hi = x[..., :dims // 2], x[..., dims // 2:dims]
+            want = torch.cat([lo * angle.cos() - hi * angle.sin(), hi * angle.cos() + lo * angle.sin(), x[..., dims:]], -1)
+            assert rel(got.reshape(n, heads, d), want) < tol
+        assert rel(rows[1], v.cpu().to(F64) + biases[2].to(F64)) < tol
+
+
 # ---------------------------------------------------------------- attention: chunks and a cap on the scores
 class Case:
     def __init__(self, H, G, d, vd, window, chunk, softcap, T, seed=0, big=1.0):
