@@ -39,7 +39,7 @@ __device__ __forceinline__ float lanes16_sum(float v) {
 // z-th of them in a workgroup of its own.
 // gridDim.y workgroups share a row's pages and leave (sum, maximum, unnormalised result) for attn_plain_merge_kernel: with a
 // token per sequence there are few rows and the pages one after another bound the time.
-// NT: tiles of 64 value elements (16 a wave).  FULL: the head is as long as they are.  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of
+// NT: tiles of 64 value elements (16 a wave).  FULL: the head is as long as they are, and a page's keys are asked for at once.  VEC, VEC_V: q and keys, and values, are aligned to four elements.  A probability of
 // 0 must not meet a value that is not finite (a key behind a token's position may hold anything): such pages are summed element
 // by element.
 // Bound by the 32-bit products (half of them for a token of 4 rows' padding) and, with few tokens, by the loads' way from memory.
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256) void attn_plain_few_keys_kernel(
 template <typename T, int NT>
 static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages, const T* v_pages, const int* table, int width,
                         const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                        int window, bool few_keys, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                        int window, bool few_keys, bool one_token_each, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
     const int chunks = (nh / nkv + ROWS - 1) / ROWS;
     const dim3 grid((N + run - 1) / run * nkv * chunks, splits, turns);
     // four elements at a time where rows are aligned to as many (a value row is a page long, so its pages' start decides)
@@ -440,7 +440,19 @@ static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages
     }
 #define PLAIN_GO(VEC_, VEC_V_, FULL_) attn_plain_kernel<T, NT, VEC_, VEC_V_, FULL_><<<grid, 256, 0, stream>>>(q, ldq, out, ldo, k_pages, v_pages, \
         table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window, run, part_o, part_ml)
-    if (vec && NT <= 4 && hd == NT * 64) PLAIN_GO(true, true, (NT <= 4));
+    // A page's keys at once beside its values cost registers: heads of 256 fit one workgroup a compute unit instead of two, of 128 in bfloat16
+    // two instead of three.  Faster at every size for shorter heads of floats; else where the others would have no work anyway,
+    // or where one token's chain bounds the time.  us, keys one after another and at once, 32-bit, heads of 256: 8 over 4, 421 tokens
+    // (212 workgroups) 67 and 51, 700 (352) 101 and 99, 800 (400) 118 and 124, 2,000 335 and 386; 16 over 8, 6,000 2,029 and 2,458;
+    // 64 tokens apart behind 1,000 keys (512) 257 and 239.  bfloat16: 8 over 4, 500 tokens (252) 70 and 65, 521 (264) 81 and 84, 2,000 334
+    // and 444; 64 apart behind 200 keys (256) 47 and 38, 128 (512) 63 and 73; heads of 128, 16 over 4, 500 tokens (500) 49 and 45, 521
+    // (524) 56 and 60, 32 over 16, 33 apart behind 1,000 keys (528) 148 and 169, 64 (1,024) 292 and 187.
+    const long wgs = (long)grid.x * splits;
+    const bool floats = sizeof(T) == 4;
+    bool full = NT <= 4 && hd == NT * 64;
+    if (NT == 4) full = full && ((floats && one_token_each) || wgs <= (floats ? 360 : COMPUTE_UNITS));
+    if (NT == 2 && !floats) full = full && (wgs <= 2 * COMPUTE_UNITS || (one_token_each && wgs > 3 * COMPUTE_UNITS));
+    if (vec && full) PLAIN_GO(true, true, (NT <= 4));
     else if (vec) PLAIN_GO(true, true, false);
     else if (vec_v) PLAIN_GO(false, true, false);
     else PLAIN_GO(false, false, false);
@@ -451,9 +463,9 @@ static void launch_rows(const T* q, long ldq, T* out, long ldo, const T* k_pages
 template <typename T>
 static void launch_type(const void* q, long ldq, void* out, long ldo, const void* k_pages, const void* v_pages, const int* table, int width,
                         const int* base, int n_pages, const int* tok_seq, const int* tok_pos, int N, int nh, int nkv, int hd, float scale,
-                        int window, bool few_keys, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
+                        int window, bool few_keys, bool one_token_each, int run, int turns, int splits, float* part_o, float* part_ml, hipStream_t stream) {
 #define ROWS_GO(NT_) launch_rows<T, NT_>((const T*)q, ldq, (T*)out, ldo, (const T*)k_pages, (const T*)v_pages, table, width, base, n_pages, \
-                                         tok_seq, tok_pos, N, nh, nkv, hd, scale, window, few_keys, run, turns, splits, part_o, part_ml, stream)
+                                         tok_seq, tok_pos, N, nh, nkv, hd, scale, window, few_keys, one_token_each, run, turns, splits, part_o, part_ml, stream)
     if (hd <= 64) ROWS_GO(1);
     else if (hd <= 128) ROWS_GO(2);
     else if (hd <= 256) ROWS_GO(4);
@@ -514,10 +526,10 @@ extern "C" int agave_attn_plain(int dtype, const void* q, long ldq, void* out, l
     const int most_turns = most_seqs < run ? most_seqs : run, turns = most_turns > 2 ? most_turns : 1;
     if (dtype == AGAVE_F32)
         launch_type<float>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
-                           few_keys, run, turns, splits, part_o, part_ml, stream);
+                           few_keys, one_token_each != 0, run, turns, splits, part_o, part_ml, stream);
     else
         launch_type<bf16>(q, ldq, out, ldo, k_pages, v_pages, table, width, base, n_pages, tok_seq, tok_pos, N, nh, nkv, hd, scale, window,
-                          few_keys, run, turns, splits, part_o, part_ml, stream);
+                          few_keys, one_token_each != 0, run, turns, splits, part_o, part_ml, stream);
     AGAVE_LAUNCH_CHECK("attn_plain");
     return 0;
 }

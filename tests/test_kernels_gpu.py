@@ -1901,6 +1901,40 @@ def test_attn_plain_heads_of_whole_tiles(K, nh, nkv, hd, window):
             test_attn_plain_values_that_are_not_finite(K, n, hd)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh,nkv,hd,n", [(8, 4, 256, 803), (6, 6, 256, 1011), (8, 4, 128, 1050)])
+def test_attn_plain_long_heads_of_many_workgroups(K, dtype, nh, nkv, hd, n):
+    """Heads of 256 (and of 128 in bfloat16), a page's keys at once (few workgroups) and one after another (many): a prompt's first rows
+    are bit for bit the same whether the rest comes with them, and a token a sequence those of the same tokens among others."""
+    few = 160
+    g = torch.Generator().manual_seed(nh)
+    pages = (n + 63) // 64
+    kp, vp = (torch.randn(pages, nkv, *shape, generator=g).to(dtype).to(DEV) for shape in ((64, hd), (hd, 64)))
+    q = torch.randn(n, nh * hd, generator=g).to(dtype).to(DEV)
+    table = torch.randperm(pages, generator=g).to(torch.int32)[None].to(DEV)
+    outs = []
+    for m in (few, n):
+        out = torch.full((m, nh * hd), float("nan"), dtype=dtype, device=DEV)
+        K.attn_plain(q[:m], out, kp, vp, table, _i32([0]), _i32([0] * m), _i32(list(range(m))), nh, nkv, hd, 0.05, None)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1][:few]) and torch.isfinite(outs[1].float()).all()
+    seqs, pos = 150, _i32([(37 * i) % (64 * pages) for i in range(150)])
+    rows = []
+    for m in (30, seqs):
+        out = torch.empty(m, nh * hd, dtype=dtype, device=DEV)
+        K.attn_plain(q[:m], out, kp, vp, table.expand(m, -1).contiguous(), _i32([0] * m), _i32(list(range(m))), pos[:m], nh, nkv, hd, 0.05, None,
+                     one_token_each=True)
+        rows.append(out)
+    assert torch.equal(rows[0], rows[1][:30])
+    k, v = kp.cpu().double()[table[0].cpu().long()], vp.cpu().double()[table[0].cpu().long()]
+    k, v = k.permute(1, 0, 2, 3).reshape(nkv, -1, hd), v.permute(1, 0, 3, 2).reshape(nkv, -1, hd)
+    tol = dict(atol=3e-5, rtol=2e-5) if dtype == torch.float32 else dict(atol=2e-2, rtol=2e-2)
+    for got, t, p in ((outs[1], n - 1, n - 1), (outs[1], 200, 200), (rows[1], 149, int(pos[149]))):
+        for h in range(nh):
+            w = torch.softmax(0.05 * k[h * nkv // nh, :p + 1] @ q[t].cpu().double().view(nh, hd)[h], 0)
+            assert torch.allclose(got[t].cpu().double().view(nh, hd)[h], w @ v[h * nkv // nh, :p + 1], **tol)
+
+
 @pytest.mark.parametrize("hd", [64, 128, 256, 100])
 def test_attn_plain_pages_that_are_not_there(K, hd):
     """Keys of pages that the table does not name count as unseen, the first, the last and one between, whoever asks for them first."""
