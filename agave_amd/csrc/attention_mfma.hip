@@ -313,6 +313,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(AttnArgs a) {
 // reference stays: probabilities are bounded by 2^8, which 32-bit sums and bfloat16 operands
 // hold without loss), and masks are applied only to units that touch the ends of the range.
 #define LAZY_LOG2 8.0f
+typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));       // four floats stored at any float's place (memory takes 16 bytes at any multiple of 4)
 template <bool SLICES> struct RawOf { using type = bf16; };
 template <> struct RawOf<true> { using type = float; };
 // FUSED: q arrives as the raw projection; the workgroup normalises and rotates its heads' queries
@@ -659,7 +660,7 @@ __global__ __launch_bounds__(256, HDT == 16 ? 1 : (HDT == 8 ? 2 : 3)) void attn_
             }
         } else {
             const size_t ps = ((size_t)t * a.nh + head) * a.splits + split;
-            *reinterpret_cast<f32x4_t*>(a.part_o + ps * hd + d) = acc;
+            *reinterpret_cast<f32x4_any_t*>(a.part_o + ps * hd + d) = acc;
             if (d == 0) {
                 a.part_ml[ps * 2 + 0] = mm * 0.6931471805599453f;    // the combine pass works in natural logarithms
                 a.part_ml[ps * 2 + 1] = ll;
@@ -1292,7 +1293,6 @@ static int launch_decode(const AttnArgs& a, const QkFuse& f, int N, hipStream_t 
     const bool fast = hd == 64 || hd == 128 || hd == 256;
     size_t lds = ((size_t)4 * slots * (fast ? hd + 16 : hd) + 4 * 16 * 2) * sizeof(float);
     if (fast) lds += (size_t)(slots + 2) * hd * sizeof(bf16);
-    AGAVE_CHECK(!fast || splits == 1 || (uintptr_t)a.part_o % 16 == 0, "attn_decode_mfma: the partial results must be 16-byte aligned");
     AGAVE_CHECK(lds <= 96 * 1024, "attn_decode_mfma: %zu bytes of LDS exceed what a workgroup may take", lds);
     if (raise_decode_lds_allowance()) return -1;
     if (FUSED) {

@@ -1841,6 +1841,37 @@ def test_attn_decode_fused_own_row(K, nh, nkv, hd, window, lens, from_reach):
     assert torch.equal(kp, want_k) and torch.equal(vp, want_v)
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 4, 256), (5, 1, 128), (18, 1, 64)])
+def test_attn_decode_takes_partial_results_at_any_float(K, nh, nkv, hd):
+    """Shares of a row that meet in memory: buffers that begin at a multiple of four bytes and not of sixteen give the same bits, from
+    raw projections and from queries ready for use."""
+    from agave_amd.ops import attention_mfma as A
+    g = torch.Generator().manual_seed(hd)
+    lens, n_pages = [700, 33], 13
+    kp = torch.randn(n_pages, nkv, 64, hd, generator=g).bfloat16().to(DEV)
+    vp = torch.randn(n_pages, nkv, hd, 64, generator=g).bfloat16().to(DEV)
+    table = torch.tensor([list(range(11)), [11] + [-1] * 10], dtype=torch.int32, device=DEV)
+    q = torch.randn(2, nh * hd, generator=g).bfloat16().to(DEV)
+    made = []
+    for off in (0, 1):
+        step, asked = _FakeStep(lens, lambda L: L - 1, None), []
+        real = step.workspace
+
+        class Shifted:
+            def get(self, name, rows, cols, dtype):
+                asked.append(name)
+                return real.get(name, rows * cols + 1, 1, dtype).view(-1)[off:off + rows * cols].view(rows, cols)
+        step.workspace = Shifted()
+        outs = [torch.full((2, nh * hd), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        A.decode_fused(q, None, None, outs[0], None, None, 0.0, 0.0, None, 1.0, kp, vp, table, _i32([0, 0]), step, nh, nkv, hd, 0.1, None)
+        A.attention(q, outs[1], kp, vp, table, _i32([0, 0]), step, nh, nkv, hd, 0.1, None)
+        assert asked.count("attn_part_o") == 2                 # (both in shares)
+        made.append(outs)
+    assert torch.isfinite(made[0][0].float()).all()
+    for a, b in zip(*made):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("slices", [1, 2, 3, 4])
 @pytest.mark.parametrize("nh,nkv,hd", [(8, 4, 256), (5, 1, 128), (18, 1, 64)])
 def test_attn_decode_fused_adds_slices_of_the_projections(K, nh, nkv, hd, slices):
