@@ -67,7 +67,6 @@ struct QkFuse {
     int slices;          // > 0: q, k_raw and v_raw are that many 32-bit slices whose sums are the rows (and the strides count floats)
     long slice_stride;
 };
-#define QK_MAX_SLICES 4
 
 // One wave: QT tiles of 16 query slots against the pages [page_lo, page_hi] of one sequence
 // and kv head.  Slot j of tile t has position pos[t] (per lane: the lane's column j = lane%16)

@@ -657,7 +657,6 @@ extern "C" int agave_residual_layernorm(int dtype, float* h, const void* branch,
 // sequence; the page id follows as soon as those two are there and travels during the arithmetic.
 // Raw float beside T bf16: q, k and v are `slices` 32-bit slices each, slice_stride elements apart, that add up to the rows (a product
 // of few tokens that was shared out along its columns).
-#define QK_MAX_SLICES 4
 template <typename T, int NV, typename Raw>
 __global__ void qk_norm_rope_kv_kernel(const Raw* q, long ldq, const Raw* __restrict__ k, long ldk,
                                        const Raw* __restrict__ v, long ldv, T* q_out, long ldqo,

@@ -5,6 +5,7 @@
 #include "common.h"
 
 #define QK_ROPE_HD_MAX 512
+#define QK_MAX_SLICES 4         // 32-bit slices of the raw projections that the kernels of few tokens add up (ops/kernels.py has the same number)
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(bf16 v) { return bf16_to_f32(v); }
 

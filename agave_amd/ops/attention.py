@@ -28,8 +28,12 @@ def adds_slices(step, qkv, head_dim: int) -> bool:
     """Whether a step's q/k work is handed the q/k/v product (a Linear) as 32-bit slices.  From 17 tokens on: one product either fills few
     compute units with tiles or brings all of its rows to every row block (4,096 rows of 2,560, us, one product and four slices: 17 tokens
     8.1 and 7.1, 32 8.8 and 7.4, 64 10.6 and 8.0; a decode step 2.52 and 2.51 ms, 2.59 and 2.55, 2.82 and 2.75; a prompt of 20, 37 and 60 tokens
-    2.64 and 2.59, 2.74 and 2.71, 2.90 and 2.83).  With fewer tokens the plans make one product of it at these sizes.  Prompts of several
-    sequences are not recorded, and the host, which the GPU waits for there, has a little more to do with slices."""
+    2.64 and 2.59, 2.74 and 2.71, 2.90 and 2.83).  Two slices pay as well, though the kernels ask for four (ms, decode steps of 17, 24, 32, 48 and 64
+    through 12 layers, one product and two slices: 8,192 rows of 3,840 1.312 1.343 1.378 1.513 1.645 and 1.315 1.340 1.370 1.496
+    1.607; 8,192 of 5,376 2.076 2.111 2.164 2.303 2.472 and 2.078 2.102 2.146 2.275 2.432; 1,536 of 1,152 48 and 64 0.657 0.725 and
+    0.659 0.720; a prompt of 60 1.568 and 1.534, 2.375 and 2.329, 0.738 and 0.730).  With fewer tokens the plans make one product of it at
+    these sizes.  Prompts of several sequences are not recorded, and the host, which the GPU waits for there, has a little more to do with
+    slices."""
     n = step.n_tokens
     return (17 <= n <= gemm_mfma.SKINNY_MAX_M and qkv.packed is not None
             and (head_dim in attention_mfma.FUSED_HEAD_DIMS if step.is_decode else step.n_seqs == 1)

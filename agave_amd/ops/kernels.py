@@ -276,7 +276,7 @@ def _slice_rows(t: torch.Tensor, what: str) -> int:
     return t.stride(1)
 
 
-QK_MAX_SLICES = 4            # 32-bit slices of the raw projections that the kernels of few tokens add up
+QK_MAX_SLICES = 4            # 32-bit slices of the raw projections that the kernels of few tokens add up (as csrc/qk_rope.h says)
 
 
 def qk_norm_rope_kv(q: Optional[torch.Tensor], k: Optional[torch.Tensor], v: Optional[torch.Tensor],

@@ -507,6 +507,49 @@ def test_wide_batches_at_a_published_size(tmp_path, n_seqs):
         close("bfloat16")(outs[i], U.plain_logits(cfg, wide, reqs[i]), f"request {i} of {n_seqs}")
 
 
+@pytest.mark.parametrize("size", ["4b", "12b"])
+def test_prompts_whose_projections_come_in_slices(tmp_path, monkeypatch, size):
+    """Prompts of one sequence around the 17 to 64 rows (with their padding to a multiple of 16) whose q/k/v product comes in slices,
+    four at the 4B sizes and two at the 12B sizes: run as they come, recorded and replayed, all alike; and a decode step of 17."""
+    from agave_amd.engine import Engine
+    from agave_amd.parts import Linear
+    sizes, _, _ = BIG_LAYERS[size]
+    cfg = dict(P.tiny_config("A"), vocab_size=1536, num_hidden_layers=2, sliding_window_pattern=2, rope_theta=1e6,
+               rope_local_base_freq=1e4, rms_norm_eps=1e-6, max_position_embeddings=4096, **dict(sizes, sliding_window=24))
+    cfg.pop("layer_types", None)
+    weights = P.random_weights(cfg, 31)
+    eng = Engine.from_folder(U.write_model(str(tmp_path / "m"), cfg, weights), dtype="bfloat16", max_slots=17, max_context=128)
+    made, real = [], Linear.forward
+
+    def forward(self, x, *args, **kw):
+        y = real(self, x, *args, **kw)
+        if kw.get("tag") == "qkv":
+            made.append((x.shape[0], y.dim(), y.shape[0]))
+        return y
+    monkeypatch.setattr(Linear, "forward", forward)
+    wide, slices = {k: v.double() for k, v in weights.items()}, {"4b": 4, "12b": 2}[size]
+    for n in (16, 17, 37, 64, 65):
+        toks = U.random_tokens(n, cfg["vocab_size"], 60 + n)
+        ref, made[:] = U.plain_logits(cfg, wide, toks)[-1:], []
+        runs = []
+        for _ in range(4):
+            slot = eng.alloc_slot()
+            runs.append(eng.step([slot], [toks], "last").float().cpu().clone())
+            eng.free_slot(slot)
+        rows = -(-n // 16) * 16
+        want = (rows, 3, slices) if 17 <= rows <= 64 else (rows, 2, rows)
+        assert made and all(m == want for m in made), (n, made)
+        close("bfloat16")(runs[0], ref, f"prompt of {n}")
+        for r in runs[1:]:
+            assert torch.equal(r, runs[0])
+    reqs = [U.random_tokens(9 + i % 3, cfg["vocab_size"], 80 + i) for i in range(17)]
+    made.clear()
+    outs = U.run_batched(eng, reqs, [8] * 17)
+    assert (17, 3, slices) in made and (8 * 17, 2, 8 * 17) in made
+    for i, (r, o) in enumerate(zip(reqs, outs)):
+        close("bfloat16")(o, U.plain_logits(cfg, wide, r), f"request {i}")
+
+
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 def test_sizes_that_fit_no_fast_kernel(tmp_path, dtype):
     """Width 100 and inner size 52 (no multiples of 8), heads of 20 (no multiple of 16), an odd

@@ -80,3 +80,27 @@ def test_where_the_norm_adds_up_a_tokens_pairs(n, top, hidden, adds_up):
     """Only where the two kernels were measured to take longer."""
     from agave_amd.ops.routed import norm_adds_up
     assert norm_adds_up(n, top, hidden) == adds_up
+
+
+def test_which_steps_hand_on_their_projections_in_slices(monkeypatch):
+    """17 to 64 tokens of a packed product in at most as many slices as the kernels add up: decode steps whose heads the one kernel
+    takes, and prompts of one sequence whatever their heads."""
+    import os
+    import re
+    from types import SimpleNamespace as Some
+    import agave_amd
+    from agave_amd.ops import attention, gemm_mfma, kernels
+    slices = {}
+    monkeypatch.setattr(gemm_mfma, "slices_for", lambda n, out, k: slices.setdefault("made", 4))
+    linear = Some(packed=object(), out_features=4096, in_features=2560)
+
+    def takes(n, seqs, head=256, of=linear):
+        return attention.adds_slices(Some(n_tokens=n, n_seqs=seqs, is_decode=seqs == n), of, head)
+    assert [n for n in (1, 16, 17, 33, 64, 65) if takes(n, n)] == [17, 33, 64] == [n for n in (16, 17, 33, 64, 65, 128) if takes(n, 1)]
+    assert not takes(40, 2) and not takes(40, 39)                    # prompts of several sequences
+    assert takes(40, 40, 64) and takes(40, 40, 128) and not takes(40, 40, 80) and takes(40, 1, 80)
+    assert not takes(40, 40, of=Some(packed=None, out_features=4096, in_features=2560))
+    slices["made"] = kernels.QK_MAX_SLICES + 1
+    assert not takes(40, 40) and not takes(40, 1)
+    with open(os.path.join(os.path.dirname(agave_amd.__file__), "csrc", "qk_rope.h")) as f:
+        assert int(re.search(r"#define QK_MAX_SLICES (\d+)", f.read()).group(1)) == kernels.QK_MAX_SLICES
