@@ -220,8 +220,8 @@ __global__ __launch_bounds__(1024) void row_norm_rope_kernel(RowsArgs A) {
 
 // The same for few tokens: three workgroups of sixteen waves a token, for q, k and v.  Bound by trips to memory one after the other (position,
 // row, place in the pages): a thread asks for its P pairs of a row, their weights and biases at once and keeps them across the sum,
-// and the sines and cosines are worked out meanwhile.  4 rows of 16 and 4 heads of 128: 4.7 -> 3.1 us;
-// 8 of 64 and 8 heads: 7.5 -> 4.2.
+// and the sines and cosines are worked out meanwhile.  4 rows of 16 and 4 heads of 128: 5.0 -> 3.4 us;
+// 4 of 64 and 8 heads: 7.7 -> 5.1.
 template <typename T, int P>
 __global__ __launch_bounds__(1024) void row_norm_rope_few_kernel(RowsArgs A) {
     __shared__ float cs[2][256];
@@ -248,9 +248,9 @@ __global__ __launch_bounds__(1024) void row_norm_rope_few_kernel(RowsArgs A) {
     const float* x = side == 0 ? A.q + (size_t)t * A.ldq : A.k + (size_t)t * A.ldk;
     const float* bias = side == 0 ? A.q_b : A.k_b;
     const float* w = side == 0 ? A.q_w : A.k_w;
-    const int heads = side == 0 ? A.nh : A.nkv, pairs = heads * half, rest = hd - 2 * half;
+    const int heads = side == 0 ? A.nh : A.nkv, pairs = heads * half, rest = hd - 2 * half, n = heads * hd;
     const double freq = A.freq[tid < half ? tid : 0];
-    float a[P], b[P], wa[P], wb[P];
+    float a[P], b[P], wa[P], wb[P], sq[2 * P];
     int at_pair[P];
 #pragma unroll
     for (int j = 0; j < P; ++j) {                                // (past the last pair: the first, not used)
@@ -259,7 +259,11 @@ __global__ __launch_bounds__(1024) void row_norm_rope_few_kernel(RowsArgs A) {
         a[j] = x[at_pair[j]];
         b[j] = x[at_pair[j] + half];
     }
+    // The squares are added up in the order of row_norm_rope_kernel's sixteen waves, of elements asked for once more (a step of up to 64
+    // tokens gives the same bits in both).
     if (w) {
+#pragma unroll
+        for (int j = 0; j < 2 * P; ++j) sq[j] = x[tid + 1024 * j < n ? tid + 1024 * j : 0];
 #pragma unroll
         for (int j = 0; j < P; ++j) {
             wa[j] = w[at_pair[j]];
@@ -271,6 +275,10 @@ __global__ __launch_bounds__(1024) void row_norm_rope_few_kernel(RowsArgs A) {
     }
     if (bias) {
         float ba[P], bb[P];
+        if (w) {
+#pragma unroll
+            for (int j = 0; j < 2 * P; ++j) sq[j] += bias[tid + 1024 * j < n ? tid + 1024 * j : 0];
+        }
 #pragma unroll
         for (int j = 0; j < P; ++j) {
             ba[j] = bias[at_pair[j]];
@@ -297,14 +305,13 @@ __global__ __launch_bounds__(1024) void row_norm_rope_few_kernel(RowsArgs A) {
     if (w) {
         float ss = 0.f;
 #pragma unroll
-        for (int j = 0; j < P; ++j)
-            if (tid + 1024 * j < pairs) ss = fmaf(a[j], a[j], fmaf(b[j], b[j], ss));
-        for (int idx = tid; idx < heads * rest; idx += 1024) {
-            int i;
-            const float v = still(idx, i);
+        for (int j = 0; j < 2 * P; ++j)
+            if (tid + 1024 * j < n) ss = fmaf(sq[j], sq[j], ss);
+        for (int i = tid + 2048 * P; i < n; i += 1024) {
+            const float v = x[i] + (bias ? bias[i] : 0.f);
             ss = fmaf(v, v, ss);
         }
-        inv = 1.0f / sqrtf(block_sum_into(ss, red) / (float)(heads * hd) + (side == 0 ? A.eps_q : A.eps_k));      // (its barrier completes the table too)
+        inv = 1.0f / sqrtf(block_sum_into(ss, red) / (float)n + (side == 0 ? A.eps_q : A.eps_k));      // (its barrier completes the table too)
     } else {
         __syncthreads();
     }
@@ -337,9 +344,9 @@ __global__ __launch_bounds__(1024) void row_norm_rope_few_kernel(RowsArgs A) {
 
 template <typename T> static void row_norm_rope_on(const RowsArgs& A, int N, hipStream_t stream) {
     // Tokens whose three workgroups all find a place at once (two of sixteen waves a compute unit) and whose pairs the threads can
-    // hold: a workgroup a row, else one a token.  us, a row together and apart, 16 and 4 heads of 128 with norms: 1 token 4.6 and 3.0,
-    // 64 4.9 and 3.4, 128 7.0 and 4.4, 170 7.1 and 5.6, 200 6.9 and 5.7, 300 7.5 and 7.4; 64 and 8 heads of 128 with norms and
-    // biases (four pairs a thread): 8 7.5 and 4.2, 128 15.4 and 6.6, 170 15.8 and 8.4, 300 17.6 and 11.2.
+    // hold: a workgroup a row, else one a token.  us, a row together and apart, 16 and 4 heads of 128 with norms: 1 token 4.9 and 3.3,
+    // 64 5.3 and 3.8, 128 7.0 and 4.5, 170 7.2 and 5.7 (300 7.5 and 7.4 before the squares were read apart); 64 and 8 heads of 128
+    // with norms and biases (four pairs a thread): 4 7.7 and 5.1, 128 15.4 and 7.3, 170 15.7 and 9.6.
     // Rows of up to 256 pairs leave most of the sixteen waves idle, and keys and values beside them are slower apart as soon as a compute
     // unit has two workgroups: 2 heads of 64 with norms, 100 4.7 and 3.9, 128 4.7 and 4.0, 129 4.7 and 4.9, 170 4.7 and 5.1 (the queries
     // alone 3.3 and 3.1); 8 with biases, 128 4.3 and 3.7, 150 4.3 and 4.4.

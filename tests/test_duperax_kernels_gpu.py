@@ -236,6 +236,41 @@ def test_rows_with_biases_into_pages_at_the_edges(H, G, d, dims, n, normed):
         assert rel(rows[1], v.cpu().to(F64) + biases[2].to(F64)) < tol
 
 
+@pytest.mark.parametrize("n", [1, 5, 64])
+@pytest.mark.parametrize("H, G, d, half, biased", [(16, 4, 128, 32, False), (3, 2, 70, 5, True), (33, 8, 128, 48, True), (80, 3, 128, 60, False)])
+def test_row_norms_of_few_tokens_add_squares_in_one_order(n, H, G, d, half, biased):
+    """Up to 64 tokens a row's root mean square is bit for bit that of sixteen waves which go round the row's elements, whichever
+    kernel takes it (80 heads have more pairs than the one of few tokens holds): seen in the elements that are not rotated."""
+    import numpy as np
+    from agave_amd.ops import attention_biased as A
+    vd, eps = 16, 1e-5
+    g = torch.Generator().manual_seed(H)
+    raw = torch.randn(n, (H + G) * d + G * vd, generator=g) * 2
+    weights = [1 + 0.3 * torch.randn(k, generator=g) for k in (H * d, G * d)]
+    biases = [torch.randn(k, generator=g) if biased else None for k in (H * d, G * d, G * vd)]
+    dev = lambda t: t.to(DEV) if t is not None else None
+    q, k, v = dev(raw).split((H * d, G * d, G * vd), dim=1)
+    q_out, k_out, v_out = torch.empty(n, H * d, device=DEV), torch.empty(n, G * d, device=DEV), torch.empty(n, G * vd, device=DEV)
+    A.row_norm_rope(q, k, v, q_out, k_out, v_out, dev(weights[0]), dev(weights[1]), eps, eps, torch.rand(half, dtype=F64, device=DEV), 1.0,
+                    Positions(list(range(n))), H, G, d, vd, biases=tuple(dev(b) for b in biases))
+    for got, x, w, b in ((q_out, q, weights[0], biases[0]), (k_out, k, weights[1], biases[1])):
+        x = x.cpu() + b if biased else x.cpu()
+        pad = np.zeros((n, -(-x.shape[1] // 1024) * 1024), np.float32)
+        pad[:, :x.shape[1]] = x.numpy()
+        ss = np.zeros((n, 1024), np.float32)
+        for piece in np.split(pad, pad.shape[1] // 1024, axis=1):                    # (a fused step, exact in long double up to its one rounding)
+            ss = (piece.astype(np.longdouble) * piece + ss).astype(np.float32)
+        ss = ss.reshape(n, 16, 64)
+        while ss.shape[-1] > 1:
+            ss = ss[..., 0::2] + ss[..., 1::2]
+        total = np.zeros(n, np.float32)
+        for i in range(16):
+            total = total + ss[:, i, 0]
+        inv = torch.from_numpy(np.float32(1) / np.sqrt(total / np.float32(x.shape[1]) + np.float32(eps)))[:, None]
+        want = (x * inv * w).view(n, -1, d)[..., 2 * half:]
+        assert torch.equal(got.cpu().view(n, -1, d)[..., 2 * half:], want)
+
+
 # ---------------------------------------------------------------- attention: chunks and a cap on the scores
 class Case:
     def __init__(self, H, G, d, vd, window, chunk, softcap, T, seed=0, big=1.0):
