@@ -329,7 +329,8 @@ template <> struct RawOf<true> { using type = float; };
 // loads at a time: the waves then stand at the loads they cannot issue, so the heads are normed between the keys' loads and the
 // values'.  Before, they waited for all of both first (the loads stood behind a branch).
 // (4B sizes, us a launch in a chain of all layers, before and now: one sequence of 150 keys 6.2 and 5.2, 8 of 1,024 12.5 and 10.3, 64 of 100
-// 12.3 and 9.5, of which 1.6 are a kernel's start and end; the last one's 33 MB take 5.3 of them, 6.2 TB/s.)
+// 12.3 and 9.5, of which 1.6 are a kernel's start and end; from the first request to the last value of the last one's 27 MB are 5.3,
+// 5.1 TB/s.)
 // MODE: what q is.  0: queries ready for use; 1 (FUSED): the raw projections in bfloat16; 2: their 32-bit slices (a product of few row
 // blocks that was shared out along its columns: q/k/v of 4B sizes, 64 tokens, 10.6 us as one product and 8.0 in four slices).
 template <int HDT, int MODE>

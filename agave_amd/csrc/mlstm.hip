@@ -88,8 +88,9 @@ template <bool VEC> __device__ __forceinline__ f32x4_t four(const float* x, int 
 // ------------------------------------------------------------------ one token a sequence
 // A column of dk elements is shared by L lanes, each with R groups of V neighbours; a wave takes 64 / L columns at a time,
 // UN times, with all of its loads under way before the first is used.  Column dv is n.  Bound by one trip to memory and the
-// chain of instructions behind it (the state of 4 sequences with 4 heads of 256 by 512 is 17 MB, read and written in some 5 us of
-// the card's rate): with the gates' logarithms in front of the loads 8.2 us, worked out behind them 6.6.
+// chain of instructions behind it: the state of 4 sequences with 4 heads of 256 by 512 is 8.4 MB, read and written 17, 2.7 us at 6.2 TB/s,
+// and a kernel's start and end 1.6; with the gates' logarithms in front of the loads 8.2 us, worked out behind them 6.6, so that
+// some 2 are still the chain's.
 template <int L, int V, int R, int UN>
 __global__ __launch_bounds__(256) void mlstm_step_kernel(MlstmArgs A, float* __restrict__ num, float* __restrict__ nq) {
     constexpr int CW = 64 / L;
